@@ -78,6 +78,11 @@ def _kernel_flags(src_dir: Path) -> list[str]:
     ] + _py_includes()
 
 
+# No HIP source is built with packed-fp32 instruction selection: some forms of v_pk_{add,mul,fma}_f32 have given
+# wrong results on this hardware.  A device-side feature, so only for sources compiled as HIP.
+HIP_FLAGS = ["-x", "hip", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+
+
 def verify_kernels(names: list[str] | None = None, jobs: int = 8) -> dict[str, str]:
     """Compile the device side of the HIP kernel sources with LLVM's machine
     verifier (``-mllvm -verify-machineinstrs``) and return {file: error} for
@@ -94,7 +99,7 @@ def verify_kernels(names: list[str] | None = None, jobs: int = 8) -> dict[str, s
     bad: dict[str, str] = {}
     with tempfile.TemporaryDirectory() as td:
         def one(s: Path):
-            cmd = [hipcc, *flags, "-x", "hip", *PER_FILE_FLAGS.get(s.name, []), "--cuda-device-only", "-c", str(s),
+            cmd = [hipcc, *flags, *HIP_FLAGS, *PER_FILE_FLAGS.get(s.name, []), "--cuda-device-only", "-c", str(s),
                    "-o", str(Path(td) / (s.name + ".o")), "-mllvm", "-verify-machineinstrs"]
             r = subprocess.run(cmd, capture_output=True, text=True)
             if r.returncode != 0:
@@ -121,8 +126,8 @@ def build_kernels(verbose: bool = False, jobs: int = 8) -> Path:
     for s in srcs:
         o = objdir / (s.name + ".o")
         objs.append(o)
-        if _stale(o, [s] + hdrs):
-            extra = ["-x", "hip"] if s.suffix == ".hip" else []
+        if _stale(o, [s, Path(__file__)] + hdrs):
+            extra = list(HIP_FLAGS) if s.suffix == ".hip" else []
             extra += PER_FILE_FLAGS.get(s.name, [])
             todo.append([hipcc, *flags, *extra, "-c", str(s), "-o", str(o)])
     with ThreadPoolExecutor(max(1, jobs)) as ex:
@@ -130,10 +135,6 @@ def build_kernels(verbose: bool = False, jobs: int = 8) -> Path:
     if todo or _stale(out, objs):
         _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(out), *map(str, objs)], verbose)
     return out
-
-
-# every HIP source of this module is built without packed-fp32 instruction selection
-MIXER_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
 def build_mixers(verbose: bool = False, jobs: int = 8) -> Path:
@@ -153,8 +154,8 @@ def build_mixers(verbose: bool = False, jobs: int = 8) -> Path:
     for s in srcs:
         o = objdir / (s.name + ".o")
         objs.append(o)
-        if _stale(o, [s] + hdrs):
-            extra = ["-x", "hip", *MIXER_FLAGS] if s.suffix == ".hip" else []
+        if _stale(o, [s, Path(__file__)] + hdrs):
+            extra = list(HIP_FLAGS) if s.suffix == ".hip" else []
             todo.append([hipcc, *flags, *extra, "-c", str(s), "-o", str(o)])
     with ThreadPoolExecutor(max(1, jobs)) as ex:
         list(ex.map(lambda c: _run(c, verbose), todo))

@@ -55,7 +55,7 @@ __device__ __forceinline__ bf16x8_t as_frag(const u16x8& v) { return __builtin_b
 //     is a scalar base (one scalar block-table load) + a per-lane constant;
 //     only the context's last tile takes the clamped per-lane path;
 //   * masking only on diagonal / ragged tiles, by select (no branches);
-//     softmax in packed fp32 (v_pk_fma), scale folded into the FMA; the row
+//     softmax with the scale folded into the FMA; the row
 //     max as two v_max3 chains; the row sum l as ones . P^T on the matrix
 //     pipe (the exact sum of the bf16 P the P.V product uses: with the
 //     deferred max, profiles/r4_prefill_attn_variants.txt).
