@@ -1,0 +1,380 @@
+// Attention of prompt rows over pages of whole 64-key tiles, for gfx950: heads of 128 columns (values of 128 or 256),
+// or one shared row of 256 columns per key that is key and value (the first 192 or all of them the value).  Every
+// score form of tile_attention.hip: causal, window (with kept first keys) and chunk masks, a tanh cap, a log-distance
+// penalty, sigmoid weights, a sink, a gate per head.  Scores, weights and sums are fp32.
+//
+// A workgroup is eight waves: HPW heads that share a key / value head times 8 / HPW blocks of 32 rows, a wave
+// per (head, block).  Products are v_mfma_f32_32x32x16_bf16, swapped (S^T = K Q^T, O^T = V^T P^T), so a query row
+// sits on a lane and the score accumulator is the second product's operand.
+//   * Tiles go from the caches to LDS by DMA (global_load_lds, 16 bytes a lane) into a double buffer; the 16-byte
+//     pieces of a row are permuted on the source side, so that both kinds of fragment reads below hit different banks.
+//   * V^T fragments are read from the row-major image by ds_read_b64_tr_b16: no value passes through registers on
+//     its way in, and where one row is key and value one image serves both products.
+//   * Weights enter the value product as one bf16, or (FINE) as the sum of two.  FINE: the running maximum moves only
+//     when a tile's exceeds it by 2^8, so the accumulators are rescaled on few tiles; a single bf16 holds a row's
+//     largest weight exactly when that weight is 1, so there the maximum follows every tile.
+//   * Wide shared rows (256 value columns): the upper half of the queries stays in LDS, the accumulators need its
+//     registers.
+// What bounds it: vector issue of the softmax beside the matrix cores at two waves a SIMD (the register file holds no
+// more), score terms most of all.  Against the register-staged, 16x16x32 forms it took over from (tile_attention.hip,
+// stream and latent prefill), 32 heads, ragged prompts of about 4000 tokens, us before -> after: two maps with values
+// of 256, window 1024 + 64: 721 -> 240; shared row 256 / 192 causal 241 -> 137 (720 TFLOP/s), 256 / 256 window 547 ->
+// 124; cap + penalty, window 1024: 315 -> 175; sigmoid 214 -> 92; plain causal, 5000 tokens: 133 -> 124, fine 160 ->
+// 145; 40 rows behind 2900 cached: 132 -> 117.
+#include <type_traits>
+
+#include "stream_attention.h"
+
+namespace {
+
+struct PromptArgs {
+  void* out;  // [T, n_qh, DV]
+  const bf16_t* q;
+  int64_t q_stride;
+  const bf16_t* kc;
+  const bf16_t* vc;
+  const int64_t* pos;
+  const int* seq;
+  const int* bt;
+  int bt_stride, bs_shift;
+  const int* tiles;  // [n, 2]: first row, rows (up to 128) of one sequence, consecutive positions
+  int subs;          // workgroups per entry of tiles
+  int n_qh, maps, group;
+  int Wk, Wv;
+  float scale;
+  int mask, size;
+  float softcap;    // 0: none
+  const float* r1;  // [n_qh], null: no distance penalty
+  const float* r2;
+  const float* hbias;  // [n_qh] (sigmoid weights only)
+  const bf16_t* gate;  // [rows, gate_stride] logits per head
+  int64_t gate_stride;
+  int keep;           // window mask: the first `keep` keys stay visible
+  const float* sink;  // [n_qh], softmax only
+};
+
+constexpr float kLog2e = 1.4426950408889634f;
+enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
+
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ __forceinline__ int piece_xor(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+// byte offset of 16-byte piece ch of row `row` in an image whose rows are RB bytes (a multiple of 256)
+template <int RB> __device__ __forceinline__ int image_off(int row, int ch) { return row * RB + 16 * (ch ^ piece_xor(row)); }
+
+// v_max3 / v_max as written: fmaxf() on matrix-core results quiets every operand first
+__device__ __forceinline__ float raw_max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float swap_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float swap_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// D: key columns, DV: value columns, SAME: the value is the first DV columns of the key's row
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW>
+__global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) {
+  constexpr int RT = 8 / HPW, ROWS = 32 * RT;
+  constexpr int KS = D / 16, NC = DV / 32, KB = 2 * D, VB = SAME ? KB : 2 * DV;  // row bytes of the images
+  constexpr int kKey = 64 * KB, kStage = kKey + (SAME ? 0 : 64 * VB);
+  constexpr int KP = 64 * KB / 8192, VP = SAME ? 0 : 64 * VB / 8192;  // 1-KB pieces per wave
+  constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
+  constexpr float kDefer = FINE ? 8.f : 0.f;  // log2 units that a score may exceed the running maximum by
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int yi = gridDim.y - 1 - blockIdx.y;  // later rows see more keys: hand them out first
+  const int ti = yi / a.subs, off = (yi - ti * a.subs) * ROWS;
+  const int n = a.tiles[2 * ti + 1] - off;
+  if (n <= 0) return;
+  const int row0 = a.tiles[2 * ti] + off;
+  const int p0 = __builtin_amdgcn_readfirstlane((int)a.pos[row0]);
+  const int* bt = a.bt + (int64_t)__builtin_amdgcn_readfirstlane(a.seq[row0]) * a.bt_stride;
+  const int per = a.group / HPW, gm = blockIdx.x / per, g = gm / a.maps;  // key head, key / value group
+  const int head = g * a.group + (blockIdx.x - gm * per) * HPW + wid % HPW;
+  const int qh = head * a.maps + (gm - g * a.maps);
+  const int rw = 32 * (wid / HPW);  // the wave's first row
+  const int hi = p0 + min(n, ROWS) - 1;
+  const int first = first_key(p0, a.mask, a.size) >> 6, last = hi >> 6;
+  const int kept = a.mask == 1 ? min((a.keep + 63) >> 6, first) : 0;  // tiles of kept keys in front of the window's
+  // rows beyond n repeat the last one and are not stored
+  const int myrow = min(rw + r, n - 1), my = p0 + myrow, mylo = first_key(my, a.mask, a.size);
+  const int wlo = p0 + min(rw, n - 1), whi = p0 + min(rw + 31, n - 1);  // the wave's first and last position
+  const int wfirst = first_key(wlo, a.mask, a.size), wlast = first_key(whi, a.mask, a.size);
+  const int keep = a.mask == 1 ? a.keep : 0;
+  bf16x8_t qf[QR];
+  bf16_t* ql = reinterpret_cast<bf16_t*>(smem + 2 * kStage) + (wid * (KS - QR) * 64 + lane) * 8;  // the lane's own pieces
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const bf16x8_t f = frag16(a.q + (int64_t)(row0 + myrow) * a.q_stride + (int64_t)qh * D + 16 * ks + 8 * h);
+    if (ks < QR) qf[ks < QR ? ks : 0] = f;
+    else *reinterpret_cast<bf16x8_t*>(ql + (ks - QR) * 512) = f;
+  }
+  // lane constants: fragment addresses (piece 16 and up of a row: + 256 bytes), DMA sources
+  int koff[8], voff_[4][2];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) koff[ks] = image_off<KB>(r, 2 * ks + h);
+  {
+    const int g16 = (lane >> 4) & 1, qq = (lane & 15) >> 2, pp = lane & 3;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      const int ch = dt * 4 + 2 * g16 + (pp >> 1);
+      voff_[dt][0] = image_off<VB>(4 * h + qq, ch) + 8 * (pp & 1);
+      voff_[dt][1] = image_off<VB>(4 * h + qq + 8, ch) + 8 * (pp & 1);
+    }
+  }
+  const bf16_t* kc = a.kc + (int64_t)gm * D;
+  const bf16_t* vc = a.vc + (int64_t)g * DV;
+  auto issue = [&](char* buf, int t) {
+    const int64_t base = tile_slot(bt, a.bs_shift, t);
+    const bf16_t *kb = kc + base * a.Wk, *vb = vc + base * a.Wv;
+    const int left = hi - (t << 6);  // rows behind the last query hold stale values: its row instead
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+      constexpr int RP = 1024 / KB, CH = KB / 16;
+      const int row = (KP * wid + k) * RP + lane / CH;
+      __builtin_amdgcn_global_load_lds(kb + (int64_t)min(row, left) * a.Wk + 8 * ((lane % CH) ^ piece_xor(row)),
+                                       (lds_void*)(buf + (KP * wid + k) * 1024), 16, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < VP; ++k) {
+      constexpr int RP = 1024 / VB, CH = VB / 16;
+      const int row = (VP * wid + k) * RP + lane / CH;
+      __builtin_amdgcn_global_load_lds(vb + (int64_t)min(row, left) * a.Wv + 8 * ((lane % CH) ^ piece_xor(row)),
+                                       (lds_void*)(buf + kKey + (VP * wid + k) * 1024), 16, 0, 0);
+    }
+  };
+  const float cap = a.softcap, inv_cap = MODE != kPlain && cap > 0.f ? 1.f / cap : 0.f;
+  const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
+  const float r1 = MODE != kPlain && a.r1 ? a.r1[qh] * 1.f : 0.f, r2 = MODE != kPlain && a.r1 ? a.r2[qh] : 0.f;
+  const float sc = terms ? 1.f : a.scale * kLog2e;  // scores to log2 units
+  const float hb = MODE == kSigmoid && a.hbias ? a.hbias[qh] * kLog2e : 0.f;
+  float m_i = -INFINITY, l_i = 0.f;
+  f32x16 O[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) O[i] = f32x16{};
+
+  auto step = [&](auto bufc, int t) {
+    const char* kb = smem + decltype(bufc)::value * kStage;
+    const char* vb = SAME ? kb : kb + kKey;
+    const int kt = t << 6;
+    const bool kept_tile = kt + 64 <= keep;  // wholly of kept keys
+    if (rw >= n || kt > whi || (kt + 63 < wfirst && kt >= keep)) return;  // nothing the wave's rows see
+    const bool live1 = kt + 32 <= whi;  // some row sees the second half
+    f32x16 s[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const char* kp = kb + koff[ks & 7] + 256 * (ks >> 3);
+      const bf16x8_t qk = ks < QR ? qf[ks < QR ? ks : 0] : frag16(ql + (ks - QR) * 512);
+      s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)kp), qk, s[0], 0, 0, 0);
+      if (live1) s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)(kp + 32 * KB)), qk, s[1], 0, 0, 0);
+    }
+    if (MODE != kPlain && terms) {  // final scores in log2 units
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          float x = s[sub][i] * a.scale;
+          // cap * tanh(x / cap): tanh(y) = 1 - 2 / (1 + e^(2 y))
+          x = cap > 0.f ? cap * kLog2e * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + fast_exp2(x * (2.f * kLog2e) * inv_cap)))
+                        : x * kLog2e;
+          if (a.r1) {
+            const int dist = my - (kt + 32 * sub + (i & 3) + 8 * (i >> 2) + 4 * h);
+            x -= r1 * __builtin_amdgcn_logf(1.f + r2 * (float)max(dist, 0));
+          }
+          s[sub][i] = x;
+        }
+    }
+    if (kt + 63 > wlo || (kt < wlast && !kept_tile)) {  // some key is not seen by some row
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int j = kt + 32 * sub + (i & 3) + 8 * (i >> 2) + 4 * h;
+          if (j > my || (j < mylo && j >= keep)) s[sub][i] = -INFINITY;
+        }
+    }
+    float mu = 0.f;
+    if constexpr (MODE != kSigmoid) {
+      float ta = fmaxf(s[0][0], s[1][0]), tb = fmaxf(s[0][1], s[1][1]);
+#pragma unroll
+      for (int i = 2; i < 16; i += 2) {
+        ta = raw_max3(ta, s[0][i], s[1][i]);
+        tb = raw_max3(tb, s[0][i + 1], s[1][i + 1]);
+      }
+      // both halves of a row see the same maximum and take the same decision
+      const float tm = swap_max(fmaxf(ta, tb)) * sc;
+      const float mn = tm > m_i + kDefer ? tm : m_i;
+      mu = mn == -INFINITY ? 0.f : mn;  // a row that has seen nothing yet
+      if (__builtin_amdgcn_ballot_w64(mn != m_i)) {
+        const float alpha = fast_exp2(m_i - mu);
+        l_i *= alpha;
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) O[i][e] *= alpha;
+      }
+      m_i = mn;
+    }
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      if (sub == 1 && !live1) break;
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        raw_u32x4 ph, pl;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float w[2];
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const float v = s[sub][8 * s2 + 2 * e + x];
+            if constexpr (MODE == kSigmoid)  // sigmoid(s + bias); an invisible key (s = -inf) weighs 0
+              w[x] = __builtin_amdgcn_rcpf(1.f + fast_exp2(-fmaf(v, sc, hb)));
+            else
+              w[x] = fast_exp2(fmaf(v, sc, -mu));
+          }
+          if constexpr (MODE != kSigmoid) l_i += w[0] + w[1];
+          ph[e] = pack_bf16x2(w[0], w[1]);
+          if constexpr (FINE) pl[e] = pack_bf16x2(w[0] - bf16lo(ph[e]), w[1] - bf16hi(ph[e]));
+        }
+#pragma unroll
+        for (int dt = 0; dt < NC; ++dt) {
+          const char* vp = vb + sub * 32 * VB + s2 * 16 * VB + 256 * (dt >> 2);
+          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[dt & 3][0]));
+          const i16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[dt & 3][1]));
+          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+          O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, ph), O[dt], 0, 0, 0);
+          if constexpr (FINE)
+            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, pl), O[dt], 0, 0, 0);
+        }
+      }
+    }
+  };
+  // tiles in order: the kept ones, then the window's
+  const int total = kept + last - first + 1;
+  auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
+  issue(smem, tile(0));
+  if (wid >= 4) __builtin_amdgcn_s_setprio(1);  // else the second wave of each SIMD loses every arbitration
+  __syncthreads();  // (waits for the DMA of the tile as well)
+  for (int i = 0; i < total; i += 2) {
+    if (i + 1 < total) issue(smem + kStage, tile(i + 1));
+    step(std::integral_constant<int, 0>{}, tile(i));
+    __syncthreads();
+    if (i + 1 < total) {
+      if (i + 2 < total) issue(smem, tile(i + 2));
+      step(std::integral_constant<int, 1>{}, tile(i + 1));
+      __syncthreads();
+    }
+  }
+
+  float inv = 1.f;
+  if constexpr (MODE != kSigmoid) {
+    float l = swap_sum(l_i);
+    if (a.sink) l += fast_exp2(a.sink[qh] * kLog2e - m_i);  // (finite: a row sees itself)
+    inv = 1.f / l;
+  }
+  if (a.gate) inv /= 1.f + __expf(-bf16_to_f32(a.gate[(int64_t)(row0 + myrow) * a.gate_stride + head]));
+  const bool ok = rw + r < n;
+  OutT* o = (OutT*)a.out + ((int64_t)(row0 + myrow) * a.n_qh + qh) * DV;
+  // lane (r, h) holds columns 8 g4 + 4 h .. + 3 of each block of 32
+#pragma unroll
+  for (int dt = 0; dt < NC; ++dt) {
+    if constexpr (sizeof(OutT) == 4) {
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        if (ok)
+          *reinterpret_cast<f32x4*>(o + dt * 32 + 8 * g4 + 4 * h) =
+              f32x4{O[dt][4 * g4] * inv, O[dt][4 * g4 + 1] * inv, O[dt][4 * g4 + 2] * inv, O[dt][4 * g4 + 3] * inv};
+    } else {  // two neighbouring groups swap halves: 16 bytes a lane
+#pragma unroll
+      for (int g4 = 0; g4 < 4; g4 += 2) {
+        const uint32_t ax = pack_bf16x2(O[dt][4 * g4] * inv, O[dt][4 * g4 + 1] * inv);
+        const uint32_t ay = pack_bf16x2(O[dt][4 * g4 + 2] * inv, O[dt][4 * g4 + 3] * inv);
+        const uint32_t bx = pack_bf16x2(O[dt][4 * g4 + 4] * inv, O[dt][4 * g4 + 5] * inv);
+        const uint32_t by = pack_bf16x2(O[dt][4 * g4 + 6] * inv, O[dt][4 * g4 + 7] * inv);
+        const auto sx = __builtin_amdgcn_permlane32_swap(ax, bx, false, false);
+        const auto sy = __builtin_amdgcn_permlane32_swap(ay, by, false, false);
+        if (ok) *reinterpret_cast<raw_u32x4*>(o + dt * 32 + 8 * g4 + 8 * h) = raw_u32x4{sx[0], sy[0], sx[1], sy[1]};
+      }
+    }
+  }
+}
+
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW>
+int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
+  PromptArgs a = a0;
+  a.subs = 128 / (32 * (8 / HPW));
+  constexpr int lds = 2 * 64 * 2 * (D + (SAME ? 0 : DV)) + (SAME && DV == 256 ? 8 * (D / 16 - 8) * 1024 : 0);
+  auto kern = prompt_attention_kernel<D, DV, SAME, MODE, FINE, OutT, HPW>;
+  static bool raised = false;  // once per instance
+  if (lds > 48 * 1024 && !raised) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 7;
+    raised = true;
+  }
+  const int step = 65535 / a.subs;
+  for (int t0 = 0; t0 < n_tiles; t0 += step) {
+    a.tiles = a0.tiles + 2 * t0;
+    const int nt = n_tiles - t0 < step ? n_tiles - t0 : step;
+    hipLaunchKernelGGL(kern, dim3(a.n_qh / HPW, nt * a.subs), dim3(512), lds, st, a);
+  }
+  DX_CHECK_LAUNCH();
+  return 0;
+}
+
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT>
+int prompt_heads(const PromptArgs& a, int n_tiles, hipStream_t st) {
+  if constexpr (SAME) {  // every head shares the row: eight heads over 32 rows meet the fewest tiles outside the mask
+    if (a.group % 8 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 8>(a, n_tiles, st);
+  }
+  if (a.group % 4 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 4>(a, n_tiles, st);
+  return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 2>(a, n_tiles, st);
+}
+
+}  // namespace
+
+extern "C" {
+
+// 1 when the kernel has an instance for the heads and the kind of result; `same`: keys and values are one cache
+int dxm_prompt_attention_ok(int d, int dv, int n_qh, int maps, int group, int bs, int same, int terms, int sigmoid,
+                            int out_f32, int fine) {
+  if (bs < 64 || (bs & (bs - 1)) || group < 1) return 0;
+  if (group % 2) return 0;
+  if (same) return d == 256 && (dv == 192 || dv == 256) && maps == 1 && group == n_qh && !terms && !sigmoid && !out_f32 && !fine;
+  if (d == 128 && dv == 256) return out_f32 && !terms && !sigmoid;
+  return d == 128 && dv == 128 && !out_f32 && !(fine && (terms || sigmoid));
+}
+
+int dxm_prompt_attention(void* out, const void* q, int64_t q_stride, const void* kc, const void* vc, const int64_t* pos,
+                         const int* seq, const int* bt, int bt_stride, int bs, const int* tiles, int n_tiles, int n_qh,
+                         int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask, int size,
+                         float softcap, const float* r1, const float* r2, int wfn, const float* hbias, const void* gate,
+                         int64_t gate_stride, int keep, const float* sink, int out_f32, int fine, hipStream_t st) {
+  if (n_tiles <= 0) return 0;
+  const bool same = kc == vc, terms = softcap > 0.f || r1;
+  if (softcap < 0.f || (r1 && !r2) || wfn < 0 || wfn > 1 || keep < 0 || (keep && mask != 1)) return 6;
+  if (!dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, same, terms, wfn, out_f32, fine)) return 2;
+  if (n_qh < 1 || maps < 1 || n_qh % maps || (n_qh / maps) % group || n_qh > 65535) return 1;
+  if (mask < 0 || mask > 2 || (mask && size < 1) || !(scale > 0.f)) return 3;
+  if (!out || !seq || !tiles || Wk % 8 || Wv % 8 || q_stride % 8 || (uintptr_t)q % 16 || (uintptr_t)kc % 16 ||
+      (uintptr_t)vc % 16 || (uintptr_t)out % 16)
+    return 4;
+  PromptArgs a{out, (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, pos, seq, bt, bt_stride,
+               __builtin_ctz((unsigned)bs), tiles, 1, n_qh, maps, group, Wk, Wv, scale, mask, size, softcap, r1, r2, hbias,
+               (const bf16_t*)gate, gate_stride, keep, sink};
+  if (same && dv == 256) return prompt_heads<256, 256, true, kPlain, false, bf16_t>(a, n_tiles, st);
+  if (same) return prompt_heads<256, 192, true, kPlain, false, bf16_t>(a, n_tiles, st);
+  if (dv == 256) return prompt_heads<128, 256, false, kPlain, true, float>(a, n_tiles, st);
+  if (wfn) return prompt_heads<128, 128, false, kSigmoid, false, bf16_t>(a, n_tiles, st);
+  if (terms) return prompt_heads<128, 128, false, kTerms, false, bf16_t>(a, n_tiles, st);
+  if (fine) return prompt_heads<128, 128, false, kPlain, true, bf16_t>(a, n_tiles, st);
+  return prompt_heads<128, 128, false, kPlain, false, bf16_t>(a, n_tiles, st);
+}
+
+}  // extern "C"

@@ -11,7 +11,8 @@
 // goes from memory straight into MFMA A fragments (a lane reads 16 bytes of its
 // key); each half's registers are refilled with the next tile as soon as they are
 // free.  Weights enter the value product as the sum of two bf16 numbers.
-// stream_prefill: eight waves per (64 or 128 prompt rows, 4 or 2 heads of a
+// stream_prefill: heads of 64 columns (prompt_attention.hip takes those of 128);
+// eight waves per (64 or 128 prompt rows, 4 or 2 heads of a
 // group), 32 rows of one head each, sharing every key tile; tiles are
 // double-buffered in LDS.  Weights enter the value product as bf16, or (FINE) as
 // the sum of two.
@@ -398,7 +399,7 @@ extern "C" {
 
 // 1 when the prompt kernel takes these heads: one map, an even number of heads per key/value head
 int dxm_stream_prefill_ok(int d, int dv, int maps, int group, int bs, int mask) {
-  return ((d == 128 && dv == 128) || (d == 64 && dv == 64)) && maps == 1 && group % 2 == 0 && bs >= 64 &&
+  return d == 64 && dv == 64 && maps == 1 && group % 2 == 0 && bs >= 64 &&
          (bs & (bs - 1)) == 0 && mask >= 0 && mask <= 2;
 }
 
@@ -419,9 +420,7 @@ int dxm_stream_prefill(void* out, const void* q, int64_t q_stride, const void* k
 #define STREAM_PREFILL(D, HPW)                                  \
   if (fine) launch_stream_prefill<D, HPW, true>(a, n_tiles, st); \
   else launch_stream_prefill<D, HPW, false>(a, n_tiles, st);
-  if (d == 128 && group % 4 == 0) { STREAM_PREFILL(128, 4) }
-  else if (d == 128) { STREAM_PREFILL(128, 2) }
-  else if (group % 4 == 0) { STREAM_PREFILL(64, 4) }
+  if (group % 4 == 0) { STREAM_PREFILL(64, 4) }
   else { STREAM_PREFILL(64, 2) }
 #undef STREAM_PREFILL
   DX_CHECK_LAUNCH();

@@ -1,0 +1,110 @@
+"""Prompt rows on csrc/mixers/prompt_attention.hip: pages of whole 64-key tiles, heads of 128 columns (values of 128 or
+256) or one shared row of 256 columns, every score form, against dense float64 arithmetic over the bf16 inputs."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from dynamo_exp_amd.ops import mixers as mx
+
+# n_qh, maps, group, d, dv, form; group 2 takes two heads a workgroup, 4 and 8 four; "shared": one row is key and value
+FORMS = {
+    "plain": (8, 1, 4, 128, 128), "plain pair": (6, 1, 2, 128, 128), "fine": (8, 1, 8, 128, 128),
+    "capped": (4, 1, 2, 128, 128), "penalty": (8, 1, 4, 128, 128), "both": (8, 1, 4, 128, 128),
+    "sigmoid": (8, 1, 4, 128, 128), "sigmoid capped": (4, 1, 2, 128, 128), "diff": (16, 2, 4, 128, 256),
+    "diff pair": (8, 2, 2, 128, 256), "shared": (16, 1, 16, 256, 192),
+    "shared wide": (8, 1, 8, 256, 256), "shared pair": (6, 1, 6, 256, 192), "gated": (8, 1, 4, 128, 128),
+}
+MASKS = [("causal", 0, 0), ("window", 70, 0), ("window", 1, 0), ("window", 100, 5), ("window", 66, 64), ("window", 40, 130),
+         ("chunk", 50, 0), ("chunk", 256, 0)]
+
+
+def dense(q, k, v, pos, scale, mask, size, keep, cap, db, sink, sig, hb):
+    """q [R, n_qh, d], k [n, n_qh, d], v [n, n_qh, dv] float64 -> [R, n_qh, dv]."""
+    s = torch.einsum("ihd,jhd->hij", q, k) * scale
+    p, j = pos[:, None], torch.arange(k.shape[0])[None, :]
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    if db is not None:
+        s = s - db[0].double()[:, None, None] * torch.log1p(db[1].double()[:, None, None] * (p - j).clamp_min(0)[None])
+    vis = (j <= p) & ((j >= mx.first_visible(p, mask, size)) | (j < keep))
+    if sig:
+        w = torch.sigmoid(s + hb.double()[:, None, None]) * vis
+    else:
+        s = s.masked_fill(~vis, float("-inf"))
+        if sink is not None:
+            s = torch.cat([s, sink.double()[:, None, None].expand(-1, s.shape[1], 1)], -1)
+        w = torch.softmax(s, -1)[..., :k.shape[0]]
+    return torch.einsum("hij,jhd->ihd", w, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size,keep", MASKS)
+@pytest.mark.parametrize("form", FORMS)
+def test_prompt_rows(form, mask, size, keep):
+    """Portions of 1, 33 and 257 rows that start at 0 and inside a cached prefix, over shuffled pages of 64 and 128
+    tokens whose unused rows hold NaN; the second sequence's last tile holds a single key."""
+    shared = form.startswith("shared")
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(11)
+    G = n_qh // maps // group
+    scale = 0.7 * d ** -0.5
+    heads = torch.arange(n_qh) // maps
+    kh, vh = heads // group * maps + torch.arange(n_qh) % maps, heads // group
+    # prefix lengths and rows: 300, 65 (one key in its last tile) and 1 keys in all
+    starts, rows = [43, 32, 0], [257, 33, 1]
+    f32 = lambda *s: torch.randn(*s)
+    kw, sig, hb, db, sink, cap, gate = {}, False, None, None, None, 0.0, None
+    if form in ("capped", "both", "sigmoid capped"):
+        cap = 2.0
+    if form in ("penalty", "both"):
+        db = (torch.rand(n_qh), torch.rand(n_qh) + 0.1)
+    if form.startswith("sigmoid"):
+        sig, hb = True, f32(n_qh) - 2.0
+    if form in ("shared", "shared wide", "plain"):
+        sink = f32(n_qh)
+    cuda = lambda t: None if t is None else t.cuda()
+    for bs in (64, 128):
+        nb = [-(-(s + r) // bs) for s, r in zip(starts, rows)]
+        perm = torch.randperm(sum(nb)).to(torch.int32)
+        table = torch.zeros(3, max(nb), dtype=torch.int32)
+        kc = torch.full((sum(nb) * bs, d if shared else G * maps * d), float("nan"), dtype=torch.bfloat16)
+        vc = kc if shared else torch.full((sum(nb) * bs, G * dv), float("nan"), dtype=torch.bfloat16)
+        want, at = [], 0
+        q = torch.randn(sum(rows), n_qh * d + 8).bfloat16()[:, :n_qh * d]  # rows wider than the heads
+        for i, (s, r) in enumerate(zip(starts, rows)):
+            n = s + r
+            table[i, :nb[i]] = perm[at:at + nb[i]]
+            at += nb[i]
+            sl = table[i].long()[torch.arange(n) // bs] * bs + torch.arange(n) % bs
+            kc[sl] = (torch.randn(n, kc.shape[1]) * 1.5).bfloat16()
+            if not shared:
+                vc[sl] = torch.randn(n, vc.shape[1]).bfloat16()
+            if shared:
+                K = kc[sl].double()[:, None].expand(n, n_qh, d)
+                V = K[:, :, :dv]
+            else:
+                K, V = kc[sl].double().view(n, -1, d)[:, kh], vc[sl].double().view(n, -1, dv)[:, vh]
+            r0 = sum(rows[:i])
+            want.append(dense(q[r0:r0 + r].double().view(r, n_qh, d), K, V, torch.arange(s, n), scale, mask, size, keep, cap,
+                              db, sink, sig, hb))
+        want = torch.cat(want)
+        if form == "gated":
+            gate = torch.randn(sum(rows), n_qh // maps + 3).bfloat16()[:, :n_qh // maps]
+            want = want * torch.sigmoid(gate.double()).repeat_interleave(maps, 1)[:, :, None]
+        pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)]).cuda()
+        seq = torch.tensor([i for i, r in enumerate(rows) for _ in range(r)], dtype=torch.int32).cuda()
+        tiles = torch.tensor([t for i in range(3) for t in mx.tile_list(sum(rows[:i]), rows[i])], dtype=torch.int32).cuda()
+        kd = kc.cuda()
+        vd = kd if shared else vc.cuda()
+        out_f32 = form.startswith("diff")
+        got = mx.attention(q.cuda(), kd, vd, pos, seq, table.cuda(), bs, n_qh, maps, group, d, dv, scale, mask, size, 1,
+                           out_f32, tiles, sum(rows), softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                           weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), head_gate=cuda(gate),
+                           keep_first=keep, sink=cuda(sink), fine_weights=form == "fine").cpu().double()
+        err = (got - want).abs()
+        # a bf16 result: its rounding (2^-9 of it) and one rounding of every weight (2^-9 of sum w |v|, |v| < 5 here
+        # and weights that sum to 1, or for sigmoid weights to their sum); fp32: two bf16 numbers per weight, 2^-17,
+        # and the hardware's exp2, logarithm and reciprocal in the scores
+        mass = want.abs().max() if sig else 5.0
+        assert float(err.max()) < (3e-4 if out_f32 else 2.0 ** -8 * (float(want.abs().max()) + float(mass))), float(err.max())
