@@ -186,38 +186,70 @@ __global__ void __launch_bounds__(64) row_attention_kernel(RowAttnArgs a) {
   }
 }
 
-// joins the per-part (max, sum, acc) of one (row, head): one wave each
-// (sigmoid weights: every part carries max 0 and sum 1, so the join is the plain sum of the
-// parts divided by their number -- `plain` undoes that division); gate: logits [rows, gs] per
-// head, the result is multiplied by their sigmoid; sink: [n_qh], exp(sink) joins the softmax denominator once
+// joins the per-part (max, sum, acc) of one (row, head): a wave each, four to a workgroup
+// (`plain`: sigmoid weights, every part with a key carries max 0 and sum 1 and the join is the plain sum); gate:
+// logits [rows, gs] per head, the result is multiplied by their sigmoid; sink: [n_qh], exp(sink) joins the softmax
+// denominator once.
+// Bound by latency, not by its bytes: lanes read the parts' (max, sum) side by side, and the parts' columns are read in
+// independent 8-byte loads.  Reading part after part, three times over, took 23 us of a 46 us layer for 33 x 32 vectors
+// of 192 columns in 16 parts; now 12.
 template <typename OutT, typename GT>
-__global__ void __launch_bounds__(64) merge_parts_kernel(OutT* __restrict__ out, const float* __restrict__ ws,
-                                                         int parts, int dv, int plain, const GT* __restrict__ gate,
-                                                         int64_t gs, int n_qh, int maps,
-                                                         const float* __restrict__ sink) {
-  const int lane = threadIdx.x;
-  const int64_t v = blockIdx.x;
-  const float* w = ws + v * parts * (int64_t)(2 + dv);
-  float post = plain ? (float)parts : 1.f;
+__global__ void __launch_bounds__(256) merge_parts_kernel(OutT* __restrict__ out, const float* __restrict__ ws,
+                                                          int64_t n_vec, int parts, int dv, int plain,
+                                                          const GT* __restrict__ gate, int64_t gs, int n_qh, int maps,
+                                                          const float* __restrict__ sink) {
+  const int lane = threadIdx.x & 63;
+  const int64_t v = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (v >= n_vec) return;
+  const int step = 2 + dv;
+  const float* w = ws + v * parts * (int64_t)step;
+  float post = 1.f;
   if (gate) {
     const int64_t row = v / n_qh;
     const int head = (int)(v - row * n_qh) / maps;
     post /= 1.f + expf(-Elem<GT>::ld(gate, row * gs + head));
   }
-  float mx = -INFINITY;
-  for (int p = 0; p < parts; ++p) mx = fmaxf(mx, w[(int64_t)p * (2 + dv)]);
-  float l = 0.f;
-  for (int p = 0; p < parts; ++p) {
-    const float* wp = w + (int64_t)p * (2 + dv);
-    if (wp[1] > 0.f) l += wp[1] * __expf(wp[0] - mx);
+  // lane p: part p (of 64 at a time); parts without a key have sum 0 and count for nothing
+  float m0 = -INFINITY, l0 = 0.f;
+  if (lane < parts) m0 = w[(int64_t)lane * step], l0 = w[(int64_t)lane * step + 1];
+  float mx = m0;
+  for (int p = lane + 64; p < parts; p += 64) mx = fmaxf(mx, w[(int64_t)p * step]);
+  mx = wave_reduce_max(mx);
+  float f0 = l0 > 0.f ? __expf(m0 - mx) : 0.f;
+  float l = l0 > 0.f ? l0 * f0 : 0.f;
+  for (int p = lane + 64; p < parts; p += 64) {
+    const float lp = w[(int64_t)p * step + 1];
+    if (lp > 0.f) l += lp * __expf(w[(int64_t)p * step] - mx);
   }
+  l = wave_reduce_sum(l);
   if (sink && !plain) l += expf(sink[v % n_qh] - mx);
-  const float inv = post / l;
+  const float inv = plain ? post : post / l;
+  // parts behind the last with a key hold nothing
+  const int n = parts > 64 ? parts : 64 - __builtin_clzll(__builtin_amdgcn_ballot_w64(l0 > 0.f) | 1);
+  auto factor = [&](int p) {  // the same in every lane
+    if (p < 64) return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f0), p));
+    const float* wp = w + (int64_t)p * step;
+    return wp[1] > 0.f ? __expf(wp[0] - mx) : 0.f;
+  };
+  if (dv % 2 == 0 && (uintptr_t)ws % 8 == 0) {
+    for (int e = 2 * lane; e < dv; e += 128) {
+      float a0 = 0.f, a1 = 0.f;
+#pragma unroll 4
+      for (int p = 0; p < n; ++p) {
+        const float2 x = *reinterpret_cast<const float2*>(w + (int64_t)p * step + 2 + e);
+        const float f = factor(p);
+        if (f > 0.f) a0 += x.x * f, a1 += x.y * f;
+      }
+      Elem<OutT>::st(out, v * dv + e, a0 * inv);
+      Elem<OutT>::st(out, v * dv + e + 1, a1 * inv);
+    }
+    return;
+  }
   for (int e = lane; e < dv; e += 64) {
     float acc = 0.f;
-    for (int p = 0; p < parts; ++p) {
-      const float* wp = w + (int64_t)p * (2 + dv);
-      if (wp[1] > 0.f) acc += wp[2 + e] * __expf(wp[0] - mx);
+    for (int p = 0; p < n; ++p) {
+      const float f = factor(p);
+      if (f > 0.f) acc += w[(int64_t)p * step + 2 + e] * f;
     }
     Elem<OutT>::st(out, v * dv + e, acc * inv);
   }
@@ -244,8 +276,8 @@ int launch_rows(const RowAttnArgs& a, int rows, hipStream_t st) {
     else if (nv <= 8) hipLaunchKernelGGL((row_attention_kernel<T, OutT, 8>), grid, dim3(64), lds, st, b);
     else hipLaunchKernelGGL((row_attention_kernel<T, OutT, 16>), grid, dim3(64), lds, st, b);
     if (a.parts > 1)
-      hipLaunchKernelGGL((merge_parts_kernel<OutT, T>), dim3((unsigned)nr * a.n_qh), dim3(64), 0, st, (OutT*)b.out, b.ws,
-                         a.parts, a.dv, a.wfn, (const T*)b.gate, a.gate_stride, a.n_qh, a.maps, a.sink);
+      hipLaunchKernelGGL((merge_parts_kernel<OutT, T>), dim3(((unsigned)nr * a.n_qh + 3) / 4), dim3(256), 0, st,
+                         (OutT*)b.out, b.ws, (int64_t)nr * a.n_qh, a.parts, a.dv, a.wfn, (const T*)b.gate, a.gate_stride, a.n_qh, a.maps, a.sink);
   }
   DX_CHECK_LAUNCH();
   return 0;
@@ -280,11 +312,11 @@ extern "C" int dxm_merge_parts(void* out, const float* ws, int64_t n_vec, int pa
   if (n_vec <= 0) return 0;
   if (parts < 1 || dv < 1 || n_vec > 0x7fffffff || n_qh < 1 || maps < 1) return 1;
   if (out_f32)
-    hipLaunchKernelGGL((merge_parts_kernel<float, bf16_t>), dim3((unsigned)n_vec), dim3(64), 0, st, (float*)out, ws,
-                       parts, dv, plain, (const bf16_t*)gate, gate_stride, n_qh, maps, sink);
+    hipLaunchKernelGGL((merge_parts_kernel<float, bf16_t>), dim3((unsigned)((n_vec + 3) / 4)), dim3(256), 0, st,
+                       (float*)out, ws, n_vec, parts, dv, plain, (const bf16_t*)gate, gate_stride, n_qh, maps, sink);
   else
-    hipLaunchKernelGGL((merge_parts_kernel<bf16_t, bf16_t>), dim3((unsigned)n_vec), dim3(64), 0, st, (bf16_t*)out, ws,
-                       parts, dv, plain, (const bf16_t*)gate, gate_stride, n_qh, maps, sink);
+    hipLaunchKernelGGL((merge_parts_kernel<bf16_t, bf16_t>), dim3((unsigned)((n_vec + 3) / 4)), dim3(256), 0, st,
+                       (bf16_t*)out, ws, n_vec, parts, dv, plain, (const bf16_t*)gate, gate_stride, n_qh, maps, sink);
   DX_CHECK_LAUNCH();
   return 0;
 }
