@@ -3,6 +3,7 @@
 // in; launches neither allocate nor synchronise, so they can be captured into
 // HIP graphs.  A launcher that rejects its arguments returns nonzero, raised
 // here.
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <pybind11/pybind11.h>
 
@@ -93,6 +94,11 @@ int dxm_latent_prefill(void*, const void*, int64_t, const void*, int, const int6
                        const int*, int, int, int, int, float, int, int, const float*, hipStream_t);
 int dxm_latent_decode(float*, const void*, int64_t, const void*, int, const int64_t*, const int*, const int*, int, int, int,
                       int, int, int, float, int, int, int, hipStream_t);
+int dxm_decode_attention_ok(int, int, int, int, int, int, int, int, int);
+int dxm_decode_attention_parts(int, int, int, int, int);
+int dxm_decode_attention(void*, float*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*,
+                         int, int, int, int, int, int, int, int, int, int, float, int, int, float, const float*, const float*,
+                         int, const float*, const void*, int64_t, int, const float*, int, int, hipStream_t);
 int dxm_merge_parts(void*, const float*, int64_t, int, int, int, const void*, int64_t, int, int, const float*, int,
                     hipStream_t);
 }
@@ -302,8 +308,19 @@ PYBIND11_MODULE(_C_mixers, m) {
                            int n_qh, int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask,
                            int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs, int keep, u sink,
                            int parts, int out_f32, u st) {
+    // pages of whole tiles and heads of 128 columns (or one shared row of 256)
+    if (scale > 0.f && qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && (q | kc | vc | out) % 16 == 0 &&
+        dxm_decode_attention_ok(d, dv, n_qh, maps, group, bs, kc == vc, cap > 0.f || r1, wfn)) {
+      parts = std::min(parts, dxm_decode_attention_parts(rows, n_qh, group, kc == vc, dv));
+      check(dxm_decode_attention(P(out), F(ws), P(q), qs, P(kc), P(vc), reinterpret_cast<const int64_t*>(pos),
+                                 reinterpret_cast<const int*>(seq), reinterpret_cast<const int*>(bt), bts, bs, rows, n_qh,
+                                 maps, group, d, dv, Wk, Wv, scale, mask, size, cap, F(r1), F(r2), wfn, F(hbias), P(gate), gs,
+                                 keep, F(sink), parts, out_f32, S(st)),
+            "decode_attention");
+      if (parts == 1) return;
+    }
     // plain heads over pages of whole tiles take the streaming kernel (same workspace)
-    if (cap == 0.f && !r1 && !wfn && !hbias && !keep && qs % 8 == 0 && (q | kc | vc) % 16 == 0 &&
+    else if (cap == 0.f && !r1 && !wfn && !hbias && !keep && qs % 8 == 0 && (q | kc | vc) % 16 == 0 &&
         dxm_stream_decode_ok(d, dv, group, bs, mask))
       check(dxm_stream_decode(F(ws), P(q), qs, P(kc), P(vc), reinterpret_cast<const int64_t*>(pos),
                               reinterpret_cast<const int*>(seq), reinterpret_cast<const int*>(bt), bts, bs, rows, n_qh,

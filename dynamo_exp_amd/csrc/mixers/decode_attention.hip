@@ -1,0 +1,477 @@
+// Attention of decode rows (one token a row) over pages of whole 32-key tiles, for gfx950: heads of 128 columns with
+// values of 128, pairs of maps with values of 256, or one shared row of 256 columns per key that is key and value (its
+// first 192 columns, or all).  Every score form of tile_attention.hip.  Scores and sums are fp32, weights enter the value
+// product as the sum of two bf16 numbers.
+//
+// A workgroup (4 waves) serves one (row, key / value group, part of the keys): up to 16 query vectors of the group (a
+// shared row: 16 QB) are the columns of 16x16x32 products.  Both maps of a two-map layer are in one workgroup, so their
+// common values are read once.  The waves take the part's tiles in turn and run on their own: a wave brings its tiles
+// into LDS of its own by DMA and waits for its own loads only, so there is no barrier until the end, where the four
+// partial results are joined in LDS.  Keys and values have a buffer each, refilled as soon as its product is done; a
+// shared row has two buffers in turn.  V^T fragments come from the row-major image by ds_read_b64_tr_b16.
+// One part: the result goes out finished; several: partials to the workspace that merge_parts joins.
+// Bound by memory at many rows and by latency at few.  Two layers in a graph with their joins, against the one-wave
+// forms it took over from (register-staged group_decode, stream_decode, latent_decode), us before -> after: two maps,
+// window 1024 + 64, 48 rows 270 -> 98 (4.4 TB/s of cache), chunk 2048 358 -> 123, 1 row 89 -> 38; shared row 256 / 192
+// causal to 4000, 33 rows 92 -> 58; cap + penalty 40 rows 174 -> 84; sigmoid 171 -> 84; plain to 4100, 48 rows 239 ->
+// 206 (5.3 TB/s), 2 rows 81 -> 32.
+#include <algorithm>
+#include <type_traits>
+
+#include "stream_attention.h"
+
+namespace {
+
+struct DecodeArgs {
+  void* out;  // [rows, n_qh, DV]
+  float* ws;  // parts > 1: [rows, n_qh, parts, 2 + DV]
+  const bf16_t* q;
+  int64_t q_stride;
+  const bf16_t* kc;
+  const bf16_t* vc;
+  const int64_t* pos;
+  const int* seq;  // null: row i is sequence i
+  const int* bt;
+  int bt_stride, bs_shift;
+  int n_qh, maps, group;
+  int Wk, Wv;
+  float scale;
+  int mask, size, parts;
+  float softcap;    // 0: none
+  const float* r1;  // [n_qh], null: no distance penalty
+  const float* r2;
+  const float* hbias;
+  const bf16_t* gate;
+  int64_t gate_stride;
+  int keep;
+  const float* sink;
+  int out_f32;
+};
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
+constexpr int kTile = 32;       // keys per tile
+constexpr float kDefer = 8.f;   // log2 units that a score may exceed the running maximum by (weights are bf16 pairs)
+enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
+
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+typedef __attribute__((address_space(3))) void lds_void;
+// metadata that no kernel in flight writes: scalar loads
+typedef const __attribute__((address_space(4))) int* scalar_int;
+
+__device__ __forceinline__ int piece_xor(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+template <int RB> __device__ __forceinline__ int image_off(int row, int ch) { return row * RB + 16 * (ch ^ piece_xor(row)); }
+// the wave's own DMA: all but the newest N instructions have landed.  (The builtin, which the compiler counts itself:
+// behind a wait it does not know it would put a full one in front of the next LDS read.)
+template <int N> __device__ __forceinline__ void dma_wait() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));  // vmcnt alone
+  asm volatile("" ::: "memory");
+}
+// every LDS read issued so far has returned: its buffer may be refilled
+__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// over the four 16-lane groups of a wave
+__device__ __forceinline__ float groups_max(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float groups_sum(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// D: key columns, DV: value columns, MAPS: maps a workgroup serves, SAME: the value is the first DV columns of the
+// key's row, QB: blocks of 16 query vectors
+template <int D, int DV, int MAPS, bool SAME, int MODE, int QB>
+__global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attention_kernel(DecodeArgs a) {
+  constexpr int KS = D / 32, NC = DV / 16, KB = 2 * D * MAPS, VB = SAME ? KB : 2 * DV;  // row bytes of the images
+  constexpr int KN = kTile * KB / 1024, VN = SAME ? KN : kTile * VB / 1024;             // DMA instructions per tile
+  constexpr int GR = MAPS == 2 ? 8 : 16;  // columns per map
+  static_assert(!SAME || (MAPS == 1 && D == 256), "one shared row");
+  // keys / values; a shared row: tiles with even / odd turn
+  __shared__ __attribute__((aligned(16))) char ka[4][kTile * KB];
+  __shared__ __attribute__((aligned(16))) char va[4][kTile * VB];
+  __shared__ float ml[2][4][QB][16];
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = blockIdx.y, part = blockIdx.z;
+  const int p = __builtin_amdgcn_readfirstlane((int)a.pos[row]);
+  const int lo = first_key(p, a.mask, a.size);
+  const int keep = a.mask == 1 ? a.keep : 0;
+  // tiles in order: those of the kept keys, then the mask's
+  const int first = lo / kTile, kept = min((keep + kTile - 1) / kTile, first), total = kept + p / kTile - first + 1;
+  // at least two tiles a wave, four of a long context: shorter parts cost more in the join than they gain
+  const int tpp = max((total + a.parts - 1) / a.parts, max(8, min(16, total / 12))), i0 = part * tpp, i1 = min(i0 + tpp, total);
+  const scalar_int bt = (scalar_int)(a.bt + (int64_t)__builtin_amdgcn_readfirstlane(a.seq ? a.seq[row] : row) * a.bt_stride);
+  // K head of the workgroup (of the first map), its key / value group
+  const int gm = SAME ? 0 : MAPS == 2 ? 2 * blockIdx.x : blockIdx.x, g = SAME ? 0 : gm / a.maps, m = gm - g * a.maps;
+  int qh[QB];
+  bool okh[QB];
+  float r1[QB], r2[QB], hb[QB];
+  bf16x8_t qf[QB][KS];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int hi_ = SAME ? (int)blockIdx.x * 16 * QB + 16 * qb + c16 : c16 % GR;
+    okh[qb] = hi_ < a.group;
+    qh[qb] = (g * a.group + (okh[qb] ? hi_ : 0)) * a.maps + (MAPS == 2 ? c16 / GR : m);
+    r1[qb] = MODE != kPlain && a.r1 ? a.r1[qh[qb]] : 0.f;
+    r2[qb] = MODE != kPlain && a.r1 ? a.r2[qh[qb]] : 0.f;
+    hb[qb] = MODE == kSigmoid && a.hbias ? a.hbias[qh[qb]] * kLog2e : 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const raw_u32x4 zero{0u, 0u, 0u, 0u};
+      qf[qb][ks] = __builtin_bit_cast(bf16x8_t, okh[qb] ? *reinterpret_cast<const raw_u32x4*>(
+          a.q + (int64_t)row * a.q_stride + (int64_t)qh[qb] * D + 32 * ks + 8 * g4) : zero);
+    }
+  }
+  // lane constants: fragment addresses (pieces 16 and up of a row: + 256 bytes)
+  int koff[4], voff_[8][2];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) koff[ks] = image_off<KB>(c16, 4 * ks + g4);
+#pragma unroll
+  for (int cb = 0; cb < 8; ++cb) {
+    const int ch = 2 * cb + ((lane & 3) >> 1), r = 4 * g4 + (c16 >> 2);
+    voff_[cb][0] = image_off<VB>(r, ch) + 8 * (lane & 1);
+    voff_[cb][1] = image_off<VB>(r + 16, ch) + 8 * (lane & 1);
+  }
+  if (i0 >= i1 && part > 0) {  // a part without a key: sum 0
+    if (w == 0 && g4 == 0)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+        if (okh[qb]) {
+          float* ws = a.ws + (((int64_t)row * a.n_qh + qh[qb]) * a.parts + part) * (2 + DV);
+          ws[0] = MODE == kSigmoid ? 0.f : -INFINITY;
+          ws[1] = 0.f;
+        }
+    return;
+  }
+  const bf16_t* kc = a.kc + (int64_t)gm * D;
+  const bf16_t* vc = a.vc + (int64_t)g * DV;
+  auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
+  // one image: rows of RB bytes; rows behind the query hold stale values, which must not meet a zero weight: its own
+  // row instead
+  auto dma = [&](auto rb, const bf16_t* src, int stride, char* dst, int t) {
+    constexpr int RB = decltype(rb)::value, CH = RB / 16, RP = 1024 / RB;
+    const int j = t * kTile;
+    const int64_t base = ((int64_t)bt[j >> a.bs_shift] << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
+    const bf16_t* s = src + base * stride;
+#pragma unroll
+    for (int k = 0; k < kTile / RP; ++k) {
+      const int r = k * RP + lane / CH;
+      __builtin_amdgcn_global_load_lds(s + (int64_t)min(r, p - j) * stride + 8 * ((lane % CH) ^ piece_xor(r)),
+                                       (lds_void*)(dst + k * 1024), 16, 0, 0);
+    }
+  };
+  auto fetch_k = [&](char* dst, int i) { dma(std::integral_constant<int, KB>{}, kc, a.Wk, dst, tile(i)); };
+  auto fetch_v = [&](char* dst, int i) { dma(std::integral_constant<int, VB>{}, vc, a.Wv, dst, tile(i)); };
+
+  const float cap = a.softcap, inv_cap = MODE != kPlain && cap > 0.f ? 1.f / cap : 0.f;
+  const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
+  const float sc = terms ? 1.f : a.scale * kLog2e;  // scores to log2 units
+  float mx[QB], lsum[QB];
+  f32x4 O[QB][NC];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    mx[qb] = -INFINITY;
+    lsum[qb] = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < NC; ++cb) O[qb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  f32x4 S[QB][2];  // scores: lane column = query vector, rows = keys 16 kb + 4 g4 + r
+  auto scores = [&](const char* K) {
+    f32x4 S1[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      S1[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) S[qb][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const char* kp = K + koff[ks & 3] + kb * 16 * KB + 256 * (ks >> 2);
+        const bf16x8_t kf = frag16((const bf16_t*)kp);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) S[qb][kb] = mma(kf, qf[qb][ks], S[qb][kb]);
+        if constexpr (MAPS == 2) S1[kb] = mma(frag16((const bf16_t*)(kp + 256)), qf[0][ks], S1[kb]);
+      }
+      if constexpr (MAPS == 2) {  // every column keeps its own map's product
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[0][kb][r] = c16 < GR ? S[0][kb][r] : S1[kb][r];
+      }
+    }
+  };
+  bf16x8_t Ph[QB], Pl[QB];
+  auto softmax = [&](int t) {
+    const int kt = t * kTile;
+    const bool edge = kt + kTile - 1 > p || (kt < lo && kt + kTile > keep);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      if (MODE != kPlain && terms) {  // final scores in log2 units
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float x = S[qb][kb][r] * a.scale;
+            // cap * tanh(x / cap): tanh(y) = 1 - 2 / (1 + e^(2 y))
+            x = cap > 0.f ? cap * kLog2e * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + fast_exp2(x * (2.f * kLog2e) * inv_cap)))
+                          : x * kLog2e;
+            if (a.r1) {
+              const int dist = p - (kt + 16 * kb + 4 * g4 + r);
+              x -= r1[qb] * __builtin_amdgcn_logf(1.f + r2[qb] * (float)max(dist, 0));
+            }
+            S[qb][kb][r] = x;
+          }
+      }
+      if (edge) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = kt + 16 * kb + 4 * g4 + r;
+            if (j > p || (j < lo && j >= keep)) S[qb][kb][r] = -INFINITY;
+          }
+      }
+      float mu = 0.f;
+      if constexpr (MODE != kSigmoid) {
+        float mloc = S[qb][0][0];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mloc = fmaxf(mloc, S[qb][kb][r]);
+        const float tm = groups_max(mloc) * sc;  // (every tile holds a visible key)
+        const float mn = tm > mx[qb] + kDefer ? tm : mx[qb];
+        mu = mn == -INFINITY ? 0.f : mn;
+        if (__any(mn != mx[qb])) {
+          const float alpha = fast_exp2(mx[qb] - mu);
+          lsum[qb] *= alpha;
+#pragma unroll
+          for (int cb = 0; cb < NC; ++cb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) O[qb][cb][r] *= alpha;
+        }
+        mx[qb] = mn;
+      }
+      raw_u32x4 ph, pl;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float wt[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const float v = S[qb][e / 2][2 * (e % 2) + x];
+          if constexpr (MODE == kSigmoid)  // an invisible key (-inf) weighs 0
+            wt[x] = __builtin_amdgcn_rcpf(1.f + fast_exp2(-fmaf(v, sc, hb[qb])));
+          else
+            wt[x] = fast_exp2(fmaf(v, sc, -mu));
+        }
+        lsum[qb] += wt[0] + wt[1];
+        ph[e] = pack_bf16x2(wt[0], wt[1]);
+        pl[e] = pack_bf16x2(wt[0] - bf16lo(ph[e]), wt[1] - bf16hi(ph[e]));
+      }
+      Ph[qb] = __builtin_bit_cast(bf16x8_t, ph);
+      Pl[qb] = __builtin_bit_cast(bf16x8_t, pl);
+    }
+  };
+  auto values = [&](const char* V) {
+#pragma unroll
+    for (int cb = 0; cb < NC; ++cb) {
+      const char* vp = V + 256 * (cb >> 3);
+      const i16x4 l4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[cb & 7][0]));
+      const i16x4 u4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[cb & 7][1]));
+      const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(l4, u4, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        O[qb][cb] = mma(vf, Ph[qb], O[qb][cb]);
+        O[qb][cb] = mma(vf, Pl[qb], O[qb][cb]);
+      }
+    }
+  };
+  char *K = ka[w], *V = va[w];
+  int i = i0 + w;
+  // (the loops hold no conditional DMA: the compiler's count of what is in flight stays exact, see dma_wait)
+  if constexpr (SAME) {
+    auto turn = [&](char* cur, int i) {
+      scores(cur);
+      softmax(tile(i));
+      values(cur);
+      lds_wait();
+    };
+    if (i < i1) fetch_k(K, i);
+    for (; i + 8 < i1; i += 8) {
+      fetch_k(V, i + 4);
+      dma_wait<KN>();
+      turn(K, i);
+      fetch_k(K, i + 8);
+      dma_wait<KN>();
+      turn(V, i + 4);
+    }
+    if (i + 4 < i1) {
+      fetch_k(V, i + 4);
+      dma_wait<KN>();
+      turn(K, i);
+      dma_wait<0>();
+      turn(V, i + 4);
+    } else if (i < i1) {
+      dma_wait<0>();
+      turn(K, i);
+    }
+  } else if (i < i1) {
+    fetch_k(K, i);
+    fetch_v(V, i);
+    for (; i + 4 < i1; i += 4) {
+      dma_wait<VN>();  // the keys; the values may still fly
+      scores(K);
+      lds_wait();
+      fetch_k(K, i + 4);
+      softmax(tile(i));
+      dma_wait<KN>();
+      values(V);
+      lds_wait();
+      fetch_v(V, i + 4);
+    }
+    dma_wait<VN>();
+    scores(K);
+    softmax(tile(i));
+    dma_wait<0>();
+    values(V);
+  }
+  // ---- join the waves
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const float l = groups_sum(lsum[qb]);
+    if (g4 == 0) {
+      ml[0][w][qb][c16] = mx[qb];
+      ml[1][w][qb][c16] = l;
+    }
+  }
+  __syncthreads();  // (also: every wave is done with its images)
+  float mt[QB], lt[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    mt[qb] = fmaxf(fmaxf(ml[0][0][qb][c16], ml[0][1][qb][c16]), fmaxf(ml[0][2][qb][c16], ml[0][3][qb][c16]));
+    if (MODE == kSigmoid) mt[qb] = 0.f;
+    lt[qb] = 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {  // a wave without a tile: sum 0, maximum -inf
+      const float l = ml[1][v][qb][c16];
+      lt[qb] += MODE == kSigmoid ? l : l > 0.f ? l * fast_exp2(ml[0][v][qb][c16] - mt[qb]) : 0.f;
+    }
+  }
+  constexpr int kSlab = QB * NC * 64;  // f32x4 of a wave
+  static_assert(4 * kSlab * 16 <= (int)(sizeof(ka) + sizeof(va)), "partial results fit the images");
+  auto slab = [&](int v) {  // waves 0, 1 in the first array, 2, 3 in the second
+    return reinterpret_cast<f32x4*>(v < 2 ? &ka[0][0] : &va[0][0]) + (v & 1) * kSlab;
+  };
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const float f = MODE == kSigmoid ? 1.f : mx[qb] == -INFINITY ? 0.f : fast_exp2(mx[qb] - mt[qb]);
+#pragma unroll
+    for (int cb = 0; cb < NC; ++cb)
+      slab(w)[(qb * NC + cb) * 64 + lane] = f32x4{O[qb][cb][0] * f, O[qb][cb][1] * f, O[qb][cb][2] * f, O[qb][cb][3] * f};
+  }
+  __syncthreads();
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    if (!okh[qb]) continue;
+    float inv = 1.f;
+    if (a.parts == 1) {
+      if constexpr (MODE != kSigmoid) {
+        float l = lt[qb];
+        if (a.sink) l += fast_exp2(a.sink[qh[qb]] * kLog2e - mt[qb]);  // (finite: a row sees itself)
+        inv = 1.f / l;
+      }
+      if (a.gate) inv /= 1.f + __expf(-bf16_to_f32(a.gate[(int64_t)row * a.gate_stride + qh[qb] / a.maps]));
+    }
+    const int64_t vrow = (int64_t)row * a.n_qh + qh[qb];
+    float* ws = a.parts == 1 ? nullptr : a.ws + (vrow * a.parts + part) * (2 + DV);
+    if (ws && w == 0 && g4 == 0) {
+      ws[0] = mt[qb] * kLn2;
+      ws[1] = MODE == kSigmoid ? 1.f : lt[qb];
+    }
+#pragma unroll
+    for (int cb = 0; cb < NC; ++cb) {
+      if ((cb & 3) != w) continue;
+      f32x4 o = slab(0)[(qb * NC + cb) * 64 + lane];
+#pragma unroll
+      for (int v = 1; v < 4; ++v) o += slab(v)[(qb * NC + cb) * 64 + lane];
+      const int c = cb * 16 + 4 * g4;
+      if (ws) {
+        *reinterpret_cast<float2*>(ws + 2 + c) = float2{o[0], o[1]};
+        *reinterpret_cast<float2*>(ws + 4 + c) = float2{o[2], o[3]};
+      } else if (a.out_f32) {
+        *reinterpret_cast<f32x4*>((float*)a.out + vrow * DV + c) = f32x4{o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+      } else {
+        *reinterpret_cast<uint2*>((bf16_t*)a.out + vrow * DV + c) = uint2{pack_bf16x2(o[0] * inv, o[1] * inv),
+                                                                          pack_bf16x2(o[2] * inv, o[3] * inv)};
+      }
+    }
+  }
+}
+
+}  // namespace
+
+extern "C" {
+
+// 1 when the kernel has an instance for the heads; `same`: keys and values are one cache
+int dxm_decode_attention_ok(int d, int dv, int n_qh, int maps, int group, int bs, int same, int terms, int sigmoid) {
+  if (bs < kTile || (bs & (bs - 1)) || group < 1) return 0;
+  if (same) return d == 256 && (dv == 192 || dv == 256) && maps == 1 && group == n_qh && !terms && !sigmoid;
+  if (d == 128 && dv == 256) return maps == 2 && group <= 8 && !terms && !sigmoid;
+  return d == 128 && dv == 128 && group <= 16;
+}
+
+// workgroups per row and part
+static int decode_units(int n_qh, int group, int same, int dv) {
+  if (same) return (n_qh + (n_qh > 16 ? 31 : 15)) / (n_qh > 16 ? 32 : 16);
+  return n_qh / group / (dv == 256 ? 2 : 1);
+}
+
+// Parts worth launching.  Values of more than 128 columns fill a CU's LDS with one workgroup: as many as fit the chip
+// at once, a second round costs more than a longer first one.  Heads of 128: two workgroups a CU, at least one each.
+int dxm_decode_attention_parts(int rows, int n_qh, int group, int same, int dv) {
+  const int units = std::max(1, rows * decode_units(n_qh, group, same, dv));
+  return std::max(1, dv > 128 ? 256 / units : (512 + units - 1) / units);
+}
+
+int dxm_decode_attention(void* out, float* ws, const void* q, int64_t q_stride, const void* kc, const void* vc,
+                         const int64_t* pos, const int* seq, const int* bt, int bt_stride, int bs, int rows, int n_qh,
+                         int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask, int size, float softcap,
+                         const float* r1, const float* r2, int wfn, const float* hbias, const void* gate,
+                         int64_t gate_stride, int keep, const float* sink, int parts, int out_f32, hipStream_t st) {
+  if (rows <= 0) return 0;
+  const bool same = kc == vc, terms = softcap > 0.f || r1;
+  if (softcap < 0.f || (r1 && !r2) || wfn < 0 || wfn > 1 || keep < 0 || (keep && mask != 1)) return 6;
+  if (!dxm_decode_attention_ok(d, dv, n_qh, maps, group, bs, same, terms, wfn)) return 2;
+  if (n_qh < 1 || maps < 1 || n_qh % maps || (n_qh / maps) % group || rows > 65535) return 1;
+  if (mask < 0 || mask > 2 || (mask && size < 1) || parts < 1 || parts > 65535 || !(scale > 0.f)) return 3;
+  if (!out || (parts > 1 && !ws) || Wk % 8 || Wv % 8 || q_stride % 8 || (uintptr_t)q % 16 || (uintptr_t)kc % 16 ||
+      (uintptr_t)vc % 16 || (uintptr_t)out % 16 || (uintptr_t)ws % 8)
+    return 4;
+  DecodeArgs a{out, ws, (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, pos, seq, bt, bt_stride,
+               __builtin_ctz((unsigned)bs), n_qh, maps, group, Wk, Wv, scale, mask, size, parts, softcap, r1, r2, hbias,
+               (const bf16_t*)gate, gate_stride, keep, sink, out_f32};
+  const dim3 grid(decode_units(n_qh, group, same, dv), rows, parts);
+#define DECODE(...) hipLaunchKernelGGL((decode_attention_kernel<__VA_ARGS__>), grid, dim3(256), 0, st, a)
+  if (same && dv == 192) {
+    if (n_qh > 16) DECODE(256, 192, 1, true, kPlain, 2);
+    else DECODE(256, 192, 1, true, kPlain, 1);
+  } else if (same) {
+    if (n_qh > 16) DECODE(256, 256, 1, true, kPlain, 2);
+    else DECODE(256, 256, 1, true, kPlain, 1);
+  } else if (dv == 256) {
+    DECODE(128, 256, 2, false, kPlain, 1);
+  } else if (wfn) {
+    DECODE(128, 128, 1, false, kSigmoid, 1);
+  } else if (terms) {
+    DECODE(128, 128, 1, false, kTerms, 1);
+  } else {
+    DECODE(128, 128, 1, false, kPlain, 1);
+  }
+#undef DECODE
+  DX_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // extern "C"

@@ -404,11 +404,10 @@ template <int D, int DV> int decode_heads(const LatentArgs& a, int rows, hipStre
 extern "C" {
 
 // 1 when the kernels take these heads: one shared row that is key and value, widths they are instantiated for,
-// pages of whole 64-key tiles; prompt rows: an even number of heads, rows of less than 256 columns
-// (prompt_attention.hip takes those)
+// pages of whole 64-key tiles (prompt_attention.hip and decode_attention.hip take rows of 256 columns); prompt rows: an
+// even number of heads
 int dxm_latent_attention_ok(int d, int dv, int n_qh, int maps, int group, int bs, int prefill) {
-  const bool width = (d == 96 && dv == 64) || (d == 160 && dv == 128) || (d == 192 && dv == 128) ||
-                     (!prefill && d == 256 && dv == 192);
+  const bool width = (d == 96 && dv == 64) || (d == 160 && dv == 128) || (d == 192 && dv == 128);
   return width && maps == 1 && group == n_qh && bs >= 64 && (bs & (bs - 1)) == 0 && (!prefill || n_qh % 2 == 0);
 }
 
@@ -435,7 +434,6 @@ int dxm_latent_decode(float* ws, const void* q, int64_t q_stride, const void* ca
   if (!ws || stride % 8 || q_stride % 8 || (uintptr_t)q % 16 || (uintptr_t)cache % 16) return 4;
   LatentArgs a{ws, (const bf16_t*)q, q_stride, (const bf16_t*)cache, stride, pos, seq, bt, bt_stride,
                __builtin_ctz((unsigned)bs), nullptr, 1, n_qh, scale * 1.4426950408889634f, mask, size, parts, nullptr};
-  if (d == 256 && dv == 192) return decode_heads<256, 192>(a, rows, st);
   LATENT_CASES(decode_heads, a, rows, st)
   return 2;
 }

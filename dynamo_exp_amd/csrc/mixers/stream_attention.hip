@@ -6,13 +6,13 @@
 //   * V is transposed on its way through registers into a swizzled LDS image
 //     whose keys lie in the order the weights' fragments have them;
 //   * masks apply to the first and the last tiles only; scores and sums are fp32.
+// Heads of 64 columns; prompt_attention.hip and decode_attention.hip take those of 128.
 // stream_decode: one wave per (decode row, K head, key part), up to 16 heads;
 // partition and workspace as in group_decode (merge_parts joins the parts).  K
 // goes from memory straight into MFMA A fragments (a lane reads 16 bytes of its
 // key); each half's registers are refilled with the next tile as soon as they are
 // free.  Weights enter the value product as the sum of two bf16 numbers.
-// stream_prefill: heads of 64 columns (prompt_attention.hip takes those of 128);
-// eight waves per (64 or 128 prompt rows, 4 or 2 heads of a
+// stream_prefill: eight waves per (64 or 128 prompt rows, 4 or 2 heads of a
 // group), 32 rows of one head each, sharing every key tile; tiles are
 // double-buffered in LDS.  Weights enter the value product as bf16, or (FINE) as
 // the sum of two.
@@ -429,7 +429,7 @@ int dxm_stream_prefill(void* out, const void* q, int64_t q_stride, const void* k
 
 // 1 when the decode kernel takes these heads: widths it is instantiated for, pages of whole 64-key tiles
 int dxm_stream_decode_ok(int d, int dv, int group, int bs, int mask) {
-  return ((d == 128 && dv == 128) || (d == 64 && dv == 64)) && group >= 1 && group <= 16 && bs >= 64 &&
+  return d == 64 && dv == 64 && group >= 1 && group <= 16 && bs >= 64 &&
          (bs & (bs - 1)) == 0 && mask >= 0 && mask <= 2;
 }
 
@@ -444,8 +444,7 @@ int dxm_stream_decode(float* ws, const void* q, int64_t q_stride, const void* kc
   StreamArgs a{(const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, ws, pos, seq, bt, bt_stride,
                __builtin_ctz((unsigned)bs), n_qh, maps, group, Wk, Wv, scale * 1.4426950408889634f, mask, size, parts};
   const dim3 grid(n_qh / group, rows, parts);
-  if (d == 128) hipLaunchKernelGGL((stream_decode_kernel<128, 128>), grid, dim3(64), 0, st, a);
-  else hipLaunchKernelGGL((stream_decode_kernel<64, 64>), grid, dim3(64), 0, st, a);
+  hipLaunchKernelGGL((stream_decode_kernel<64, 64>), grid, dim3(64), 0, st, a);
   DX_CHECK_LAUNCH();
   return 0;
 }

@@ -1,5 +1,6 @@
-"""Prompt rows on csrc/mixers/prompt_attention.hip: pages of whole 64-key tiles, heads of 128 columns (values of 128 or
-256) or one shared row of 256 columns, every score form, against dense float64 arithmetic over the bf16 inputs."""
+"""Prompt rows on csrc/mixers/prompt_attention.hip and decode rows on csrc/mixers/decode_attention.hip: pages of whole
+64-key tiles, heads of 128 columns (values of 128 or 256) or one shared row of 256 columns, every score form, against
+dense float64 arithmetic over the bf16 inputs.  The pages' unused rows hold NaN."""
 from __future__ import annotations
 
 import pytest
@@ -38,73 +39,117 @@ def dense(q, k, v, pos, scale, mask, size, keep, cap, db, sink, sig, hb):
     return torch.einsum("hij,jhd->ihd", w, v)
 
 
+
+def terms(form, n_qh):
+    """(cap, distance penalty, sigmoid weights, bias, sink) of a form."""
+    cap = 2.0 if form in ("capped", "both", "sigmoid capped") else 0.0
+    db = (torch.rand(n_qh), torch.rand(n_qh) + 0.1) if form in ("penalty", "both") else None
+    sig = form.startswith("sigmoid")
+    hb = torch.randn(n_qh) - 2.0 if sig else None
+    sink = torch.randn(n_qh) if form in ("shared", "shared wide", "plain") else None
+    return cap, db, sig, hb, sink
+
+
+def pages(form, lengths, bs):
+    """Caches of sequences of these lengths over shuffled pages: (kc, vc, table, [(K, V) float64 per query vector])."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    shared, G = form.startswith("shared"), n_qh // maps // group
+    heads = torch.arange(n_qh) // maps
+    kh, vh = heads // group * maps + torch.arange(n_qh) % maps, heads // group
+    nb = [-(-n // bs) for n in lengths]
+    perm = torch.randperm(sum(nb)).to(torch.int32)
+    table = torch.zeros(len(lengths), max(nb), dtype=torch.int32)
+    kc = torch.full((sum(nb) * bs, d if shared else G * maps * d), float("nan"), dtype=torch.bfloat16)
+    vc = kc if shared else torch.full((sum(nb) * bs, G * dv), float("nan"), dtype=torch.bfloat16)
+    at, kv = 0, []
+    for i, n in enumerate(lengths):
+        table[i, :nb[i]] = perm[at:at + nb[i]]
+        at += nb[i]
+        sl = table[i].long()[torch.arange(n) // bs] * bs + torch.arange(n) % bs
+        kc[sl] = (torch.randn(n, kc.shape[1]) * 1.5).bfloat16()
+        if shared:
+            K = kc[sl].double()[:, None].expand(n, n_qh, d)
+            kv.append((K, K[:, :, :dv]))
+        else:
+            vc[sl] = torch.randn(n, vc.shape[1]).bfloat16()
+            kv.append((kc[sl].double().view(n, -1, d)[:, kh], vc[sl].double().view(n, -1, dv)[:, vh]))
+    kd = kc.cuda()
+    return kd, kd if shared else vc.cuda(), table.cuda(), kv
+
+
+def cuda(t):
+    return None if t is None else t.cuda()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mask,size,keep", MASKS)
 @pytest.mark.parametrize("form", FORMS)
 def test_prompt_rows(form, mask, size, keep):
-    """Portions of 1, 33 and 257 rows that start at 0 and inside a cached prefix, over shuffled pages of 64 and 128
-    tokens whose unused rows hold NaN; the second sequence's last tile holds a single key."""
-    shared = form.startswith("shared")
+    """Portions of 257, 33 and 1 rows that start at 0 and inside a cached prefix; the second sequence's last tile holds a
+    single key."""
     n_qh, maps, group, d, dv = FORMS[form]
     torch.manual_seed(11)
-    G = n_qh // maps // group
     scale = 0.7 * d ** -0.5
-    heads = torch.arange(n_qh) // maps
-    kh, vh = heads // group * maps + torch.arange(n_qh) % maps, heads // group
-    # prefix lengths and rows: 300, 65 (one key in its last tile) and 1 keys in all
     starts, rows = [43, 32, 0], [257, 33, 1]
-    f32 = lambda *s: torch.randn(*s)
-    kw, sig, hb, db, sink, cap, gate = {}, False, None, None, None, 0.0, None
-    if form in ("capped", "both", "sigmoid capped"):
-        cap = 2.0
-    if form in ("penalty", "both"):
-        db = (torch.rand(n_qh), torch.rand(n_qh) + 0.1)
-    if form.startswith("sigmoid"):
-        sig, hb = True, f32(n_qh) - 2.0
-    if form in ("shared", "shared wide", "plain"):
-        sink = f32(n_qh)
-    cuda = lambda t: None if t is None else t.cuda()
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    gate = torch.randn(sum(rows), n_qh // maps + 3).bfloat16()[:, :n_qh // maps] if form == "gated" else None
     for bs in (64, 128):
-        nb = [-(-(s + r) // bs) for s, r in zip(starts, rows)]
-        perm = torch.randperm(sum(nb)).to(torch.int32)
-        table = torch.zeros(3, max(nb), dtype=torch.int32)
-        kc = torch.full((sum(nb) * bs, d if shared else G * maps * d), float("nan"), dtype=torch.bfloat16)
-        vc = kc if shared else torch.full((sum(nb) * bs, G * dv), float("nan"), dtype=torch.bfloat16)
-        want, at = [], 0
+        kd, vd, table, kv = pages(form, [s + r for s, r in zip(starts, rows)], bs)
         q = torch.randn(sum(rows), n_qh * d + 8).bfloat16()[:, :n_qh * d]  # rows wider than the heads
+        want = []
         for i, (s, r) in enumerate(zip(starts, rows)):
-            n = s + r
-            table[i, :nb[i]] = perm[at:at + nb[i]]
-            at += nb[i]
-            sl = table[i].long()[torch.arange(n) // bs] * bs + torch.arange(n) % bs
-            kc[sl] = (torch.randn(n, kc.shape[1]) * 1.5).bfloat16()
-            if not shared:
-                vc[sl] = torch.randn(n, vc.shape[1]).bfloat16()
-            if shared:
-                K = kc[sl].double()[:, None].expand(n, n_qh, d)
-                V = K[:, :, :dv]
-            else:
-                K, V = kc[sl].double().view(n, -1, d)[:, kh], vc[sl].double().view(n, -1, dv)[:, vh]
             r0 = sum(rows[:i])
-            want.append(dense(q[r0:r0 + r].double().view(r, n_qh, d), K, V, torch.arange(s, n), scale, mask, size, keep, cap,
-                              db, sink, sig, hb))
+            want.append(dense(q[r0:r0 + r].double().reshape(r, n_qh, d), *kv[i], torch.arange(s, s + r), scale, mask, size,
+                              keep, cap, db, sink, sig, hb))
         want = torch.cat(want)
-        if form == "gated":
-            gate = torch.randn(sum(rows), n_qh // maps + 3).bfloat16()[:, :n_qh // maps]
+        if gate is not None:
             want = want * torch.sigmoid(gate.double()).repeat_interleave(maps, 1)[:, :, None]
         pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)]).cuda()
         seq = torch.tensor([i for i, r in enumerate(rows) for _ in range(r)], dtype=torch.int32).cuda()
         tiles = torch.tensor([t for i in range(3) for t in mx.tile_list(sum(rows[:i]), rows[i])], dtype=torch.int32).cuda()
-        kd = kc.cuda()
-        vd = kd if shared else vc.cuda()
         out_f32 = form.startswith("diff")
-        got = mx.attention(q.cuda(), kd, vd, pos, seq, table.cuda(), bs, n_qh, maps, group, d, dv, scale, mask, size, 1,
-                           out_f32, tiles, sum(rows), softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+        got = mx.attention(q.cuda(), kd, vd, pos, seq, table, bs, n_qh, maps, group, d, dv, scale, mask, size, 1, out_f32,
+                           tiles, sum(rows), softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
                            weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), head_gate=cuda(gate),
                            keep_first=keep, sink=cuda(sink), fine_weights=form == "fine").cpu().double()
-        err = (got - want).abs()
+        err = float((got - want).abs().max())
         # a bf16 result: its rounding (2^-9 of it) and one rounding of every weight (2^-9 of sum w |v|, |v| < 5 here
         # and weights that sum to 1, or for sigmoid weights to their sum); fp32: two bf16 numbers per weight, 2^-17,
         # and the hardware's exp2, logarithm and reciprocal in the scores
-        mass = want.abs().max() if sig else 5.0
-        assert float(err.max()) < (3e-4 if out_f32 else 2.0 ** -8 * (float(want.abs().max()) + float(mass))), float(err.max())
+        top = float(want.abs().max())
+        assert err < (3e-4 if out_f32 else 2.0 ** -8 * (top + (top if sig else 5.0))), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size,keep", MASKS)
+@pytest.mark.parametrize("form", FORMS)
+def test_decode_rows(form, mask, size, keep):
+    """Contexts that end at, in front of and behind the edges of 32-key tiles and pages, in one, three and nine parts
+    (some of them, and some waves, without a key), as row i = sequence i and by sequence numbers."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(13)
+    scale = 0.7 * d ** -0.5
+    ctx = [1, 31, 32, 33, 64, 65, 300, 129]
+    B = len(ctx)
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    gate = torch.randn(B, n_qh // maps + 3).bfloat16()[:, :n_qh // maps] if form == "gated" else None
+    for bs, parts, out_f32, by_seq in ((64, 1, True, False), (128, 3, True, True), (64, 9, True, False), (64, 3, False, False),
+                                       (64, 1, False, True)):
+        kd, vd, table, kv = pages(form, ctx, bs)
+        q = torch.randn(B, n_qh * d + 8).bfloat16()[:, :n_qh * d]
+        want = torch.cat([dense(q[i:i + 1].double().reshape(1, n_qh, d), *kv[i], torch.tensor([c - 1]), scale, mask, size, keep,
+                                cap, db, sink, sig, hb) for i, c in enumerate(ctx)])
+        if gate is not None:
+            want = want * torch.sigmoid(gate.double()).repeat_interleave(maps, 1)[:, :, None]
+        pos = torch.tensor([c - 1 for c in ctx]).cuda()
+        order = torch.randperm(B) if by_seq else torch.arange(B)
+        seq = order.to(torch.int32).cuda() if by_seq else None
+        got = mx.attention(q[order].cuda(), kd, vd, pos[order.cuda()], seq, table, bs, n_qh, maps, group, d, dv, scale, mask,
+                           size, parts, out_f32, softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                           weights="sigmoid" if sig else "softmax", head_bias=cuda(hb),
+                           head_gate=None if gate is None else gate[order].cuda(), keep_first=keep,
+                           sink=cuda(sink)).cpu().double()
+        err = float((got - want[order]).abs().max())
+        # fp32: weights as two bf16 numbers, 2^-17 of sum w |v|; bf16: one rounding of the result on top
+        top = float(want.abs().max())
+        assert err < (3e-4 if not sig else 3e-4 * max(top, 1.0)) + (0.0 if out_f32 else 2.0 ** -8 * top), (bs, parts, err)
