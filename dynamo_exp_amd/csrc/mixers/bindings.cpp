@@ -39,6 +39,10 @@ int dxm_residual_step(float*, const void*, int64_t, const void*, int64_t, const 
                       const int*, int, int, const void*, int64_t, const int64_t*, int, hipStream_t);
 int dxm_act_mul(void*, const void*, int64_t, const void*, int64_t, int, int, int64_t, int, float, float, float,
                 const float*, const float*, const float*, int, int64_t, int, hipStream_t);
+int64_t dxm_delta_chunk_floats(int, int, int, int, int, int, float, int64_t, int64_t);
+int dxm_delta_chunk(float*, float*, int, float*, const void*, int64_t, const void*, int64_t, const void*, int64_t, const void*,
+                    int64_t, const void*, int64_t, const float*, const float*, float, float, const int64_t*, const int*,
+                    const int*, int, int, int, int, hipStream_t);
 int dxm_delta_rule(float*, float*, int, float*, const void*, int64_t, const void*, int64_t, const void*, int64_t, const void*,
                    int64_t, const void*, int64_t, const float*, const float*, float, float, const int64_t*, const int*,
                    const int*, int, int, int, int, int, int, hipStream_t);
@@ -195,6 +199,15 @@ PYBIND11_MODULE(_C_mixers, m) {
     check(dxm_moe_router(reinterpret_cast<int*>(idx), F(w), F(gates), P(h), hs, F(rw), n_out, T, W, F(corr), E, top,
                          n_groups, keep, score, group_max, renorm, scale, f32, S(st)),
           "moe_router");
+  });
+  m.def("delta_chunk_floats", &dxm_delta_chunk_floats);
+  m.def("delta_chunk", [](u out, u state, int n_slots, u ws, u r, int64_t rs, u k, int64_t ks, u v, int64_t vs, u a,
+                          int64_t as, u w, int64_t wst, u ab, u wb, float decay_scale, float key_eps, u pos, u seq_rows,
+                          u slots, int n_seq, int T, int H, int dv, u st) {
+    check(dxm_delta_chunk(F(out), F(state), n_slots, F(ws), P(r), rs, P(k), ks, P(v), vs, P(a), as, P(w), wst, F(ab), F(wb),
+                          decay_scale, key_eps, reinterpret_cast<const int64_t*>(pos),
+                          reinterpret_cast<const int*>(seq_rows), reinterpret_cast<const int*>(slots), n_seq, T, H, dv, S(st)),
+          "delta_chunk");
   });
   m.def("delta_rule", [](u out, u state, int n_slots, u prep, u r, int64_t rs, u k, int64_t ks, u v, int64_t vs, u a,
                          int64_t as, u w, int64_t ws, u ab, u wb, float decay_scale, float key_eps, u pos, u seq_rows,

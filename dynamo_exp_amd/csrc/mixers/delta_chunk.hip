@@ -1,0 +1,455 @@
+// The generalized delta rule (recurrent.hip) over prompt rows in chunks of 16 tokens, for gfx950; keys of 128 channels,
+// everything in true fp32 on the fp32 matrix instructions (v_mfma_f32_16x16x4_f32).
+//
+//     S_t = diag(w_t) S_(t-1) - b_t (u_t^T S_(t-1)) + k_t v_t^T,    o_t = S_t^T r_t,      b_t = a_t * u_t
+//
+// Within a chunk let P_t be the product of the decays up to token t (P_0 = 1) and S the state in front of it.  With
+//     U_t = u_t P_(t-1),  R_t = r_t P_t,  B_t = b_t / P_t,  K_t = k_t / P_t        (per channel; rows of [16, 128])
+// the removed rows X_t = u_t^T S_(t-1) solve a lower triangular system of 16 rows, and everything is linear in S and V:
+//     X = U' S + G V       U' = (I + tril(U B^T, -1))^-1 U,        G = (I + tril(U B^T, -1))^-1 tril(U K^T, -1)
+//     O = R' S + H V       R' = R - tril(R B^T) U',                H = tril(R K^T) - tril(R B^T) G
+//     S <- diag(P_16) S + K''^T V - B''^T X                        K'' = K P_16, B'' = B P_16
+// delta_form_kernel makes U', R', K'', B'', G, H and P_16 of every (chunk, head) -- no chunk needs another's -- and
+// delta_chunk_kernel runs the chunks of a sequence in order: per (sequence, head, 16 columns of S) four waves that
+// own 32 channels each, S in their accumulators.  A wave's accumulators are the second operand of its part of U' S and
+// R' S as they lie; the parts of X and O join in LDS, one barrier a chunk.
+//
+// P_t shrinks by at most exp(-16 |decay_scale|) in a chunk, so 1 / P stays far inside fp32 (the host refuses more
+// than 4).  A chunk's dependent chain is 50 matrix instructions and a barrier instead of 16 tokens' chains of lane sums.
+// Its rounding: the products of decays come from sums of logarithms in fp64, the sums run in an order that keeps them
+// small and through short chains; relative to 64 bits 1.28e-7 in o and 6.90e-8 in S where the token-by-token form has
+// 1.32e-7 and 6.91e-8 (900 to 4001 tokens; 1.9e-7 and 1.2e-7 with running products and one chain per sum).
+// A value that is not finite makes its own and the later tokens' results not finite, as token by token; zero factors
+// times it do the same to the rows in front of it in its chunk.
+// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 346 + 145 us; a
+// prompt of 600 beside 30 single tokens 1265 -> 120.  Bound by the fp32 matrix instructions (200 us of them run) beside
+// the fragments' way through L2.
+#include "recurrent.h"
+
+namespace {
+
+constexpr int kC = 16;    // tokens per chunk
+constexpr int kD = 128;   // key channels
+constexpr int kPad = 4;   // floats of padding per LDS row
+constexpr int kMat = kC * kD;
+// floats per (chunk, head): U', R' [16][128]; K''^T, B''^T [128][16]; G, H [16][16]; P_16 [128]
+constexpr int kChunkFloats = 4 * kMat + 2 * kC * kC + kD;
+
+struct FormArgs {
+  float* ws;  // [chunks, H, kChunkFloats]
+  const bf16_t *r, *k, *a, *w;
+  int64_t rs, ks, as, wst;  // row strides (elements)
+  const float *a_bias, *w_bias;
+  const int* seq_rows;
+  const int* slots;
+  float decay_scale, key_eps;
+  int n_seq, n_slots, T, H;
+};
+
+// Sequence s has the chunks seq_rows[s] / 16 + s and up: no two sequences share one.
+__device__ __forceinline__ int first_chunk(const int* seq_rows, int s) { return (seq_rows[s] >> 4) + s; }
+
+// Where token t stands in U' (row), G (row and column), H (column), K''^T and B''^T (column): instruction i of the chunk
+// kernel's sums over tokens then takes tokens 4 i .. 4 i + 3.  In the order of the tokens, later ones decayed less, the
+// partial sums stay small until the end and little is rounded away.
+__device__ __forceinline__ int place(int t) { return 4 * (t & 3) + (t >> 2); }
+
+__device__ __forceinline__ f32x4 mma1(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Barrier for what the waves exchange in LDS: __syncthreads() would also wait for every load of the next chunk.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ float sigmoid1(float z) { return 1.f / (1.f + expf(-z)); }
+
+// 2^-(hi + lo)
+__device__ __forceinline__ float exp2m(float hi, float lo) {
+  const float p = __builtin_amdgcn_exp2f(-hi);
+  return fmaf(p, -0.69314718f * lo, p);
+}
+
+__global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
+  constexpr int LD = kD + kPad;
+  // four workgroups fit a CU's LDS
+  __shared__ __attribute__((aligned(16))) float m[4][kC][LD];            // U (then U'), R, B, K
+  __shared__ __attribute__((aligned(16))) float gram[4][kC][kC + kPad];  // U B^T, U K^T (below the diagonal; then G), R B^T, R K^T
+  __shared__ __attribute__((aligned(16))) float p16[kD];
+  float(*pw)[LD] = m[3];  // minus the decays' logarithms
+  const int tid = threadIdx.x, h = blockIdx.x, ci = blockIdx.y;
+  int s = 0;
+  for (int lo = 0, hi = g.n_seq; lo < hi;) {  // the last sequence that starts at or before the chunk
+    const int mid = (lo + hi) >> 1;
+    if (first_chunk(g.seq_rows, mid) <= ci) s = mid, lo = mid + 1;
+    else hi = mid;
+  }
+  const int t0 = (ci - first_chunk(g.seq_rows, s)) * kC, r0 = g.seq_rows[s] + t0, n = g.seq_rows[s + 1] - r0;
+  const int slot = g.slots[s];
+  if (t0 < 0 || n <= 0 || g.seq_rows[s] < 0 || g.seq_rows[s + 1] > g.T || slot < 0 || slot >= g.n_slots) return;
+  // ---- a thread per token and eight channels
+  const int t = tid >> 4, c0 = (tid & 15) * 8;
+  float u[8], b[8], kk[8], rr[8];
+  if (t < n) {
+    const int64_t row = r0 + t, col = (int64_t)h * kD + c0;
+    float al[8], wl[8], ss = 0.f;
+    VecIO<bf16_t, 8>::ld(g.k + row * g.ks + col, kk);
+    VecIO<bf16_t, 8>::ld(g.r + row * g.rs + col, rr);
+    VecIO<bf16_t, 8>::ld(g.a + row * g.as + col, al);
+    VecIO<bf16_t, 8>::ld(g.w + row * g.wst + col, wl);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += kk[e] * kk[e];
+    const float inv = rsqrtf(group_sum<16>(ss) + g.key_eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float ab = g.a_bias ? g.a_bias[col + e] : 0.f, wb = g.w_bias ? g.w_bias[col + e] : 0.f;
+      u[e] = kk[e] * inv;
+      b[e] = sigmoid1(al[e] + ab) * u[e];
+      pw[t][c0 + e] = g.decay_scale * sigmoid1(wl[e] + wb);
+    }
+  } else {  // behind the sequence's end: nothing read, nothing removed, nothing added
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      u[e] = b[e] = kk[e] = rr[e] = 0.f;
+      pw[t][c0 + e] = 0.f;
+    }
+  }
+  __syncthreads();
+  // Every product of decays is 2^-(a difference of sums), its sums hi + lo: rounded once.  Products of rounded decays
+  // would drift token by token, and the form would be less exact than the one that takes the tokens in order.
+  if (tid < kD) {
+    double sum = 0;
+#pragma unroll
+    for (int i = 0; i < kC; ++i) {
+      sum = fma((double)pw[i][tid], 1.4426950408889634, sum);
+      const float hi = (float)sum;
+      m[0][i][tid] = hi;
+      m[1][i][tid] = (float)(sum - (double)hi);
+    }
+    p16[tid] = exp2m(m[0][kC - 1][tid], m[1][kC - 1][tid]);
+  }
+  __syncthreads();
+  float k2[8], b2[8];  // K'' and B''
+  f32x4 x[4][2];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int c = c0 + e;
+    const float hi = m[0][t][c], lo = m[1][t][c];
+    const float ip = exp2m(-hi, -lo), dh = m[0][kC - 1][c] - hi;
+    // (what the difference of the his rounds off, exactly)
+    const float q = exp2m(dh, ((m[0][kC - 1][c] - dh) - hi) + (m[1][kC - 1][c] - lo));
+    x[0][e >> 2][e & 3] = t ? u[e] * exp2m(m[0][t - 1][c], m[1][t - 1][c]) : u[e];
+    x[1][e >> 2][e & 3] = rr[e] * exp2m(hi, lo);
+    x[2][e >> 2][e & 3] = b[e] * ip;
+    x[3][e >> 2][e & 3] = kk[e] * ip;
+    k2[e] = kk[e] * q;
+    b2[e] = b[e] * q;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) *reinterpret_cast<f32x4*>(&m[i][t][c0 + 4 * e]) = x[i][e];
+  __syncthreads();
+  // ---- the four products of 16 x 16 over the channels, one a wave (slot g of instruction (cb, i): channel 16 cb + 4 g + i)
+  const int w = tid >> 6, lane = tid & 63, l16 = lane & 15, g4 = lane >> 4;
+  {
+    const float(*A)[LD] = m[w >> 1];
+    const float(*B)[LD] = m[2 + (w & 1)];
+    f32x4 acc[8];  // short chains: the longer the chain the more of its sum is rounded away
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int cb = 0; cb < kD / 16; ++cb) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&A[l16][16 * cb + 4 * g4]);
+      const f32x4 y = *reinterpret_cast<const f32x4*>(&B[l16][16 * cb + 4 * g4]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i + 4 * (cb & 1)] = mma1(x[i], y[i], acc[i + 4 * (cb & 1)]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += acc[i + 4];
+    acc[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tt = 4 * g4 + i;  // row tt, column l16
+      gram[w][tt][l16] = l16 < tt || (w >= 2 && l16 == tt) ? acc[0][i] : 0.f;
+    }
+  }
+  __syncthreads();
+  float* o = g.ws + ((int64_t)ci * g.H + h) * kChunkFloats;
+  // ---- K'' and B'' by channel (through the places of B and K, which are done): four tokens a thread, neighbouring
+  // threads on neighbouring pieces
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) {
+    *reinterpret_cast<f32x4*>(&m[2][t][c0 + e]) = f32x4{b2[e], b2[e + 1], b2[e + 2], b2[e + 3]};
+    *reinterpret_cast<f32x4*>(&m[3][t][c0 + e]) = f32x4{k2[e], k2[e + 1], k2[e + 2], k2[e + 3]};
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int it = tid + 256 * (k & 1), ch = it >> 2, q = it & 3;
+    const float(*src)[LD] = m[3 - (k >> 1)];
+    *reinterpret_cast<f32x4*>(o + (2 + (k >> 1)) * kMat + ch * kC + 4 * q) =
+        f32x4{src[q][ch], src[4 + q][ch], src[8 + q][ch], src[12 + q][ch]};
+  }
+  if (tid < kD) o[4 * kMat + 2 * kC * kC + tid] = p16[tid];
+  // ---- a thread per column of [U | G]: forward substitution
+  if (tid < kD + kC) {
+    const bool gcol = tid >= kD;
+    const int j = tid - kD;
+    float x[kC];
+    int row[kC];  // lane q of 16: the factor of x[q] in row i, handed out as a scalar
+#pragma unroll
+    for (int i = 0; i < kC; ++i) x[i] = gcol ? gram[1][i][j] : m[0][i][tid];
+#pragma unroll
+    for (int i = 1; i < kC; ++i) row[i] = __float_as_int(gram[0][i][l16]);
+#pragma unroll
+    for (int i = 1; i < kC; ++i)
+#pragma unroll
+      for (int q = 0; q < i; ++q) x[i] -= __int_as_float(__builtin_amdgcn_readlane(row[i], q)) * x[q];
+#pragma unroll
+    for (int i = 0; i < kC; ++i) {
+      if (gcol) {
+        gram[1][i][j] = x[i];
+        o[4 * kMat + place(i) * kC + place(j)] = x[i];
+      } else {
+        m[0][i][tid] = x[i];
+        o[place(i) * kD + tid] = x[i];
+      }
+    }
+  }
+  __syncthreads();
+  // ---- R' and H: what tril(R B^T) takes of U' and G, blocks of 16 columns by wave (slot g of instruction i: token 4 g + i)
+  const f32x4 rb = *reinterpret_cast<const f32x4*>(&gram[2][l16][4 * g4]);
+  for (int cb = w; cb <= kD / 16; cb += 4) {
+    const bool hb = cb == kD / 16;
+    f32x4 acc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = hb ? gram[3][4 * g4 + i][l16] : m[1][4 * g4 + i][16 * cb + l16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = mma1(-rb[i], hb ? gram[1][4 * g4 + i][l16] : m[0][4 * g4 + i][16 * cb + l16], acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (hb) o[4 * kMat + kC * kC + (4 * g4 + i) * kC + place(l16)] = acc[i];
+      else o[kMat + (4 * g4 + i) * kD + 16 * cb + l16] = acc[i];
+    }
+  }
+}
+
+struct ChunkArgs {
+  float* out;    // [T, H * dv]
+  float* state;  // [slots, H, dv, 128]
+  const float* ws;
+  const bf16_t* v;
+  int64_t vs;
+  const int64_t* pos;
+  const int* seq_rows;
+  const int* slots;
+  int n_seq, n_slots, T, H, dv;
+};
+
+template <int NB> struct Frags {
+  f32x4 u[2], r[2], k[2], b[2], p[2];
+  float g, h;
+  uint32_t v[NB][4];  // rows g4, 4 + g4, 8 + g4 and 12 + g4 of V; bf16 bits as loaded: a conversion here would wait for the load
+};
+
+// NB: blocks of 16 columns per workgroup
+template <int NB>
+__global__ void __launch_bounds__(256, 2) delta_chunk_kernel(ChunkArgs g) {
+  __shared__ __attribute__((aligned(16))) f32x4 px[2][4][NB][64];  // parts of X
+  __shared__ float po[2][4][NB][4][64];                             // parts of O, by accumulator register
+  const int nb = g.dv / (16 * NB);
+  // the column blocks of a (sequence, head) read the same chunks: neighbours on one XCD (blocks go out round robin)
+  const int id = blockIdx.x, sh = id / (8 * nb) * 8 + id % 8, blk = id / 8 % nb;
+  if (sh >= g.n_seq * g.H) return;
+  const int s = sh / g.H, h = sh - s * g.H;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r0 = g.seq_rows[s], n = g.seq_rows[s + 1] - r0, slot = g.slots[s];
+  if (n <= 0 || r0 < 0 || r0 + n > g.T) return;
+  const int col0 = h * g.dv + blk * 16 * NB;
+  if (slot < 0 || slot >= g.n_slots) {  // padding rows: a defined result, no state
+    for (int i = threadIdx.x; i < n * 16 * NB; i += 256)
+      g.out[(int64_t)(r0 + i / (16 * NB)) * g.H * g.dv + col0 + i % (16 * NB)] = 0.f;
+    return;
+  }
+  // S: channels 32 w + 16 cb + 4 g4 + i of column l16 of every block
+  float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv + blk * 16 * NB + l16) * kD + 32 * w + 4 * g4;
+  f32x4 S[NB][2];
+#pragma unroll
+  for (int q = 0; q < NB; ++q)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+      S[q][cb] = g.pos[r0] != 0 ? *reinterpret_cast<const f32x4*>(sp + q * 16 * kD + 16 * cb) : f32x4{0.f, 0.f, 0.f, 0.f};
+  // uniform bases and 32-bit lane offsets: the chain of a chunk has no time for 64-bit address arithmetic
+  const int64_t stride = (int64_t)g.H * kChunkFloats * 4;
+  const char* wp = (const char*)(g.ws + ((int64_t)first_chunk(g.seq_rows, s) * g.H + h) * kChunkFloats);
+  const char* vp = (const char*)(g.v + (int64_t)r0 * g.vs + col0);
+  const uint32_t row_off = 4u * (l16 * kD + 32 * w + 4 * g4), ch_off = 4u * ((32 * w + l16) * kC + 4 * g4);
+  const uint32_t p_off = 4u * (32 * w + 4 * g4), sq_off = 4u * (l16 * kC + 4 * g4 + w), vs2 = 2u * (uint32_t)g.vs;
+  const int nc = (n + kC - 1) / kC;
+  const uint32_t mine[4] = {w == 0 ? ~0u : 0u, w == 1 ? ~0u : 0u, w == 2 ? ~0u : 0u, w == 3 ? ~0u : 0u};  // the wave's quarter
+  auto load = [&](Frags<NB>& f, int c) {
+    const char *p = wp + c * stride, *vc = vp + (int64_t)c * kC * g.vs * 2;
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      f.u[cb] = *reinterpret_cast<const f32x4*>(p + row_off + 64 * cb);
+      f.r[cb] = *reinterpret_cast<const f32x4*>(p + 4 * kMat + row_off + 64 * cb);
+      f.k[cb] = *reinterpret_cast<const f32x4*>(p + 8 * kMat + ch_off + 64 * kC * cb);
+      f.b[cb] = *reinterpret_cast<const f32x4*>(p + 12 * kMat + ch_off + 64 * kC * cb);
+      f.p[cb] = *reinterpret_cast<const f32x4*>(p + 16 * kMat + 8 * kC * kC + p_off + 64 * cb);
+    }
+    f.g = *reinterpret_cast<const float*>(p + 16 * kMat + sq_off);
+    f.h = *reinterpret_cast<const float*>(p + 16 * kMat + 4 * kC * kC + sq_off);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // (the last row again behind the sequence's end)
+      const uint32_t off = (uint32_t)min(g4 + 4 * i, n - 1 - c * kC) * vs2 + 2u * l16;
+#pragma unroll
+      for (int q = 0; q < NB; ++q) f.v[q][i] = *reinterpret_cast<const bf16_t*>(vc + off + 32 * q);
+    }
+  };
+  char* op = (char*)(g.out + (int64_t)r0 * g.H * g.dv + col0);
+  const int64_t ostep = (int64_t)kC * g.H * g.dv * 4;
+  const uint32_t o_off = 4u * ((4 * g4 + w) * (uint32_t)(g.H * g.dv) + l16);
+  auto step = [&](const Frags<NB>& f, int c, Frags<NB>& next, int cn) {
+    const int buf = c & 1;
+    load(next, min(cn, nc - 1));  // (always a load, the last chunk again: the waits stay counts)
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    float v[NB][4], vw[NB];
+    f32x4 X[NB][2], O[NB][2], N[NB][2];
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[q][i] = c * kC + 4 * i + g4 < n ? bf16lo(f.v[q][i]) : 0.f;
+      vw[q] = __uint_as_float(__float_as_uint(v[q][0]) & mine[0] | __float_as_uint(v[q][1]) & mine[1] |
+                              __float_as_uint(v[q][2]) & mine[2] | __float_as_uint(v[q][3]) & mine[3]);
+      X[q][0] = X[q][1] = O[q][0] = O[q][1] = zero;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) X[q][cb] = mma1(f.u[cb][i], S[q][cb][i], X[q][cb]);
+#pragma unroll
+    for (int q = 0; q < NB; ++q) X[q][0] = mma1(f.g, vw[q], X[q][0]);  // a quarter of G V each wave, the larger part last
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          O[q][cb] = mma1(f.r[cb][i], S[q][cb][i], O[q][cb]);
+          N[q][cb] = mma1(f.k[cb][i], v[q][i], i ? N[q][cb] : zero);
+        }
+      if (i == 1)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) px[buf][w][q][lane] = X[q][0] + X[q][1];
+    }
+#pragma unroll
+    for (int q = 0; q < NB; ++q) O[q][0] = mma1(f.h, vw[q], O[q][0]);
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) po[buf][w][q][i][lane] = O[q][0][i] + O[q][1][i];
+#pragma unroll
+    for (int i = 0; i < 12 + 4 * NB; ++i) {  // a load issues while the matrix instruction in front of it runs
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // K''^T V runs while the others arrive
+    lds_barrier();  // (a buffer is written again two chunks on, when its readers have met another barrier)
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) N[q][cb][i] = fmaf(S[q][cb][i], f.p[cb][i], N[q][cb][i]);
+    f32x4 xn[NB], M[NB][2];  // (sums of their own: into diag(P) S they would be rounded at its size at every token)
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const f32x4 x0 = px[buf][0][q][lane], x1 = px[buf][1][q][lane], x2 = px[buf][2][q][lane], x3 = px[buf][3][q][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xn[q][i] = (x0[i] + x1[i]) + (x2[i] + x3[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) M[q][cb] = mma1(f.b[cb][i], xn[q][i], i ? M[q][cb] : zero);
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[q][cb][i] = N[q][cb][i] - M[q][cb][i];
+      if (c * kC + 4 * g4 + w < n)  // the wave's row of each group
+        *reinterpret_cast<float*>(op + c * ostep + o_off + 64 * q) =
+            (po[buf][0][q][w][lane] + po[buf][1][q][w][lane]) + (po[buf][2][q][w][lane] + po[buf][3][q][w][lane]);
+    }
+  };
+  Frags<NB> f0, f1, f2;  // two chunks ahead
+  load(f0, 0);
+  load(f1, min(1, nc - 1));
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): what is pending here the compiler would wait for in every turn
+  for (int c = 0; c < nc; c += 3) {
+    step(f0, c, f2, c + 2);
+    if (c + 1 < nc) step(f1, c + 1, f0, c + 3);
+    if (c + 2 < nc) step(f2, c + 2, f1, c + 4);
+  }
+#pragma unroll
+  for (int q = 0; q < NB; ++q)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) *reinterpret_cast<f32x4*>(sp + q * 16 * kD + 16 * cb) = S[q][cb];
+}
+
+}  // namespace
+
+extern "C" {
+
+// Floats of workspace of the chunked form for these rows (named by seq_rows), 0 where the token-by-token form takes them:
+// bf16 rows of at least eight tokens a sequence on average (below, most chunks are padding; a decode step has no
+// seq_rows at all), keys of 128 channels, whole blocks of 16 value columns, decays whose product over a chunk stays far
+// inside fp32, 16-byte aligned rows (`ptrs`, `strides`: those of r, k, a, w and the state's pointer, or-ed).
+int64_t dxm_delta_chunk_floats(int T_, int n_seq, int H, int dk, int dv, int f32, float decay_scale, int64_t ptrs,
+                               int64_t strides) {
+  if (f32 || dk != kD || dv % 16 || dv < 16 || ptrs % 16 || strides % 8 || !(decay_scale >= -4.f && decay_scale <= 4.f))
+    return 0;
+  const int64_t chunks = T_ / kC + (int64_t)n_seq;
+  if ((int64_t)H * dv > (1 << 26) || T_ < 8 * (int64_t)n_seq || chunks > 65535 || H > 65535 ||
+      (int64_t)n_seq * H * (dv / 16) > (1 << 30))
+    return 0;
+  return chunks * H * kChunkFloats;
+}
+
+int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void* r, int64_t rs, const void* k, int64_t ks,
+                    const void* v, int64_t vs, const void* a, int64_t as, const void* w, int64_t wst, const float* a_bias,
+                    const float* w_bias, float decay_scale, float key_eps, const int64_t* pos, const int* seq_rows,
+                    const int* slots, int n_seq, int T_, int H, int dv, hipStream_t st) {
+  if (n_seq <= 0 || T_ <= 0) return 0;
+  if (H < 1 || n_slots < 1 || !out || !state || !ws || !pos || !slots || !seq_rows) return 3;
+  const int64_t ptrs = (int64_t)(uintptr_t)r | (int64_t)(uintptr_t)k | (int64_t)(uintptr_t)a | (int64_t)(uintptr_t)w |
+                       (int64_t)(uintptr_t)state | (int64_t)(uintptr_t)ws;
+  if (!dxm_delta_chunk_floats(T_, n_seq, H, kD, dv, 0, decay_scale, ptrs, rs | ks | as | wst)) return 2;
+  FormArgs f{ws, (const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)a, (const bf16_t*)w, rs, ks, as, wst, a_bias, w_bias,
+             seq_rows, slots, decay_scale, key_eps, n_seq, n_slots, T_, H};
+  hipLaunchKernelGGL(delta_form_kernel, dim3(H, T_ / kC + n_seq), dim3(256), 0, st, f);
+  ChunkArgs c{out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
+  const int64_t heads = ((int64_t)n_seq * H + 7) / 8 * 8;
+  // Two column blocks a workgroup read a chunk once for both; one keeps more of the chip busy where there are few.
+  // Whole layer, 32 heads, us: one prompt of 3000 tokens 420 / 534 (one / two blocks), three of 4001 516 / 500, six of 5000
+  // 622 / 550
+  if (dv % 32 == 0 && heads * (dv / 16) >= 512)
+    hipLaunchKernelGGL(delta_chunk_kernel<2>, dim3((unsigned)(heads * (dv / 32))), dim3(256), 0, st, c);
+  else
+    hipLaunchKernelGGL(delta_chunk_kernel<1>, dim3((unsigned)(heads * (dv / 16))), dim3(256), 0, st, c);
+  DX_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // extern "C"

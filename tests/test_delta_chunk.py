@@ -1,0 +1,87 @@
+"""The delta rule's chunked form (csrc/mixers/delta_chunk.hip) against a float64 recurrence, and its error beside the
+token-by-token kernel's on the same inputs (which float32 copies of them take)."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from dynamo_exp_amd.ops import recurrent as rc
+
+SCALE = rc.DELTA_DECAY_SCALE
+
+
+def recurrence(r, k, v, a, w, ab, wb, S, H, dv, scale, eps=1e-6):
+    """One sequence, float64: r, k, a, w [n, H 128], v [n, H dv], S [H, 128, dv] -> (o [n, H dv], S)."""
+    n = r.shape[0]
+    r, k, a, w = (x.double() for x in (r, k, a, w))
+    wf = torch.exp(-scale * torch.sigmoid(w + wb.double())).view(n, H, 128)
+    af = torch.sigmoid(a + ab.double()).view(n, H, 128)
+    r, k, v = r.view(n, H, 128), k.view(n, H, 128), v.double().view(n, H, dv)
+    u = k * torch.rsqrt((k * k).sum(-1, keepdim=True) + eps)
+    out = torch.empty(n, H, dv, dtype=torch.float64)
+    for t in range(n):
+        us = torch.einsum("hi,hij->hj", u[t], S)
+        S = wf[t][:, :, None] * S - (af[t] * u[t])[:, :, None] * us[:, None] + k[t][:, :, None] * v[t][:, None]
+        out[t] = torch.einsum("hi,hij->hj", r[t], S)
+    return out.view(n, H * dv), S
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [[64], [15, 17, 1, 33], [64, 0, 50, 1, 1], [9, 8, 16, 31], [250]])
+@pytest.mark.parametrize("kind", ["plain", "fast decay", "slow decay", "one key", "grown"])
+@pytest.mark.parametrize("H,dv", [(2, 128), (3, 16), (1, 48)])
+def test_delta_chunks(rows, kind, H, dv):
+    """Sequences of ragged lengths (also empty ones, single tokens and a padding slot), from zero state and from a state
+    of their own; decay logits at their ends, all keys equal, and a negative decay scale (a state that grows)."""
+    torch.manual_seed(5)
+    T, n_seq, n = sum(rows), len(rows), H * 128
+    p = torch.randn(T, 3 * n + H * dv).bfloat16()
+    wl = (torch.randn(T, n) * 0.5).bfloat16()
+    scale = SCALE
+    if kind == "fast decay":
+        wl, scale = wl + 8, 4.0
+    elif kind == "slow decay":
+        wl = wl - 12
+    elif kind == "one key":
+        p[:, n:2 * n] = p[:1, n:2 * n]
+    elif kind == "grown":
+        scale = -0.25
+    ab, wb = torch.randn(n) * 0.5, torch.randn(n)
+    starts = [0 if i % 2 == 0 else 5 for i in range(n_seq)]
+    slots = torch.randperm(n_seq + 2)[:n_seq].to(torch.int32)
+    if n_seq > 2:
+        slots[2] = -1
+    state0 = torch.randn(n_seq + 2, H, dv, 128)
+    firsts = [sum(rows[:i]) for i in range(n_seq + 1)]
+    pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)])
+    want, want_state = torch.zeros(T, H * dv, dtype=torch.float64), state0.double().clone()
+    for i, (s, r) in enumerate(zip(starts, rows)):
+        if slots[i] < 0 or r == 0:
+            continue
+        x = slice(firsts[i], firsts[i + 1])
+        S = state0[slots[i]].double().transpose(1, 2) if s else torch.zeros(H, 128, dv, dtype=torch.float64)
+        want[x], S = recurrence(p[x, :n], p[x, n:2 * n], p[x, 3 * n:], p[x, 2 * n:3 * n], wl[x], ab, wb, S, H, dv, scale)
+        want_state[slots[i]] = S.transpose(1, 2)
+    errs = []
+    for dt in (torch.bfloat16, torch.float32):
+        q, w, state = p.cuda().to(dt), wl.cuda().to(dt), state0.cuda()
+        got = rc.delta_rule(q[:, :n], q[:, n:2 * n], q[:, 3 * n:], q[:, 2 * n:3 * n], w, ab.cuda(), wb.cuda(), state, pos.cuda(),
+                            torch.tensor(firsts, dtype=torch.int32).cuda(), slots.cuda(), H, 128, dv, decay_scale=scale)
+        rel = lambda x, y: float((x.cpu().double() - y).norm() / y.norm())
+        errs.append((rel(got, want), rel(state, want_state)))
+    # fp32 sums of 128 to 2000 products, each rounded to 2^-24 of it: sqrt(2000) 2^-24 = 3e-6 relative to the terms; and
+    # no further off than the token-by-token form but for a few roundings (2^-24 each)
+    for got, serial in zip(*errs):
+        assert got < 3e-6 and got < 1.25 * serial + 1e-7, errs
+
+
+@pytest.mark.gpu
+def test_delta_chunk_rule():
+    """Which rows take the chunks: bf16 prompt rows, keys of 128, whole blocks of values, a bounded decay, alignment."""
+    ok = rc._m().delta_chunk_floats
+    yes = (640, 3, 2, 128, 64, 0, SCALE, 16, 8)
+    assert ok(*yes) == (40 + 3) * 2 * (4 * 2048 + 512 + 128)
+    for i, x in ((0, 23), (3, 64), (4, 40), (5, 1), (6, 4.5), (6, math.nan), (7, 8), (8, 4)):
+        assert ok(*yes[:i], x, *yes[i + 1:]) == 0
