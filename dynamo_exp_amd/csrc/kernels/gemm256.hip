@@ -37,11 +37,18 @@
 //     phases later (one barrier before the lagging group reads them).
 //   * Grouped mode (mixture of experts): the token rows are sorted by expert
 //     (order / offsets, built on the device), an expert's run of rows is cut
-//     into 256-row tiles against that expert's weight matrix w[e] (w is
+//     into row tiles against that expert's weight matrix w[e] (w is
 //     [E, N, K]), x rows are gathered per lane (the DMA takes any row address)
-//     and y rows scattered by the same map.  The host does not know the
-//     experts' row counts: the grid walks an upper bound of row tiles and
-//     every workgroup skips the ones past the last expert.
+//     and y rows scattered by the same map.  The tiles of an expert are as many
+//     as 256 rows each need, all of one height (a multiple of 32: 312 rows are
+//     2 x 160, not 256 + 56), half of a tile's 16-row blocks in each phase; the
+//     blocks that a lower tile does not have are neither read nor multiplied.
+//     The host does not know the experts' row counts, so the workgroups count
+//     the tiles before they split them.  Bound by the weights' way from HBM up to
+//     some 300 rows per expert, above by the matrix cores.  Expert part of a
+//     layer, 16 experts of width 3584, 2 a token, model width 4096, us: 300
+//     tokens 421 -> 307 (1.41 GB of weights: 4.6 TB/s), 1000 462 -> 390, 2500
+//     667 -> 539, 4000 854 -> 754; 8 experts of 2048, width 2048, 2500: 186 -> 186.
 //   * Blocks are remapped so that each XCD walks a contiguous range of tiles
 //     (bijective for any grid size), in bands of group_m token tiles: the ~32
 //     workgroups resident on one XCD then share group_m x tiles and
@@ -89,8 +96,17 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   // ---- persistent, XCD-aware tile order: the workgroups on one XCD (blocks
   // b, b + 8, ...) walk one contiguous range of logical tiles, stride = their
   // count, so the ~32 tiles in flight on an XCD are always neighbours
-  // grouped: M is the number of sorted rows; at most this many row tiles over all experts
-  const int mtn = (M + kBM - 1) / kBM + (GRP ? gm.E : 0), ntn = N / kBN, nwg = mtn * ntn;
+  // grouped: the experts' row tiles are counted here (the host only knows a bound, and tiles that do not exist would
+  // leave the XCDs they fall to without work: they lie behind the others, and with a bound of
+  // 36 row tiles for 32 the last XCD had a ninth of the others' work)
+  int mtn = (M + kBM - 1) / kBM;
+  if constexpr (GRP) {
+    int n = 0;
+    for (int e = lane; e < gm.E; e += 64) n += (gm.offsets[e + 1] - gm.offsets[e] + kBM - 1) / kBM;
+    for (int d = 32; d; d >>= 1) n += __shfl_xor(n, d);
+    mtn = __builtin_amdgcn_readfirstlane(n);
+  }
+  const int ntn = N / kBN, nwg = mtn * ntn;
   const int G = gridDim.x, bid = blockIdx.x, xcd = bid & 7;
   const int gq = G >> 3, gr8 = G & 7;                 // workgroups on this XCD: gq (+1)
   const int per_xcd = xcd < gr8 ? gq + 1 : gq;
@@ -145,9 +161,12 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   f32x4 acc[4][8];
   bf16x8_t xf[4][2], wf[4][2];
 
+  // grouped: 16-row blocks of this tile that each wave owns, in the two phases
+  int n1 = 4, n2 = 4;
   auto read_x = [&](const char* b, int xh) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      if (GRP && j >= (xh ? n2 : n1)) break;
       const char* p = b + fx + (xh * 4 + j) * 2048;
       xf[j][0] = *reinterpret_cast<const bf16x8_t*>(p + c0);
       xf[j][1] = *reinterpret_cast<const bf16x8_t*>(p + c1);
@@ -168,6 +187,18 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   // was p2 of tile t-1), the other three parts of tile t+2 in p2; reads of
   // phase q are covered by the wait at the end of phase q-2 (stagger rule).
   auto mma2 = [&](int xh) {
+    if constexpr (GRP) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j >= (xh ? n2 : n1)) break;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc[i][xh * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i][s], xf[j][s], acc[i][xh * 4 + j], 0, 0, 0);
+      }
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -210,8 +241,7 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   // tile x 32 token tiles)
   int mt = 0, nt = 0;
   int row0 = 0, rend = 0;  // grouped: this tile's first sorted row and its expert's end
-  // false (grouped only): the row tile lies past the last expert's rows
-  auto select = [&](int lid) -> bool {
+  auto select = [&](int lid) {
     const int band = lid / (group_m * ntn), first_m = band * group_m;
     const int gsz = min(mtn - first_m, group_m), in_band = lid - band * group_m * ntn;
     mt = first_m + in_band % gsz;
@@ -225,20 +255,24 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
         if (rem < n) break;
         rem -= n;
       }
-      if (e >= gm.E) return false;
-      row0 = lo + rem * kBM;
-      rend = hi;
+      // the expert's rows in tiles of one height, in 32s
+      const int blocks = (hi - lo + 31) >> 5, tiles = (hi - lo + kBM - 1) / kBM, nj = (blocks + tiles - 1) / tiles;
+      n1 = (nj + 1) >> 1;
+      n2 = nj - n1;
+      row0 = lo + rem * 32 * nj;  // (before hi: a tile fewer would not hold the rows at 8 blocks each)
+      rend = min(row0 + 32 * nj, hi);
       xb = x;
       wb = w + ((int64_t)e * N + (int64_t)nt * kBN) * K;
 #pragma unroll
       for (int P = 0; P < 2; ++P)
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          const int r = min(row0 + prow[P][i], rend - 1);
+          const int in = prow[P][i] & 63;  // (a part's rows behind its blocks: one row for all of them)
+          const int r = in < 16 * (P ? n2 : n1) ? min(row0 + (prow[P][i] >> 7) * 16 * nj + P * 16 * n1 + in, rend - 1) : row0;
           const int src = gm.gather ? gm.order[r] / gm.top : r;
           xoff[P][i] = src * (int)ldx + goff[P][i];
         }
-      return true;
+      return;
     }
     xb = x + (int64_t)mt * kBM * ldx;
     wb = w + (int64_t)nt * kBN * K;
@@ -247,13 +281,6 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         xoff[P][i] = (min(mt * kBM + prow[P][i], M - 1) - mt * kBM) * (int)ldx + goff[P][i];
-    return true;
-  };
-  // the first tile at or after lid (in this workgroup's stride) that exists; t_end if none
-  auto next_tile = [&](int from) -> int {
-    for (int l = from; l < t_end; l += per_xcd)
-      if (select(l)) return l;
-    return t_end;
   };
   // prologue of a tile: tile 0 of K, then K-tile 1 without its x half 1 (issued in p1 of K-tile 0)
   auto prologue = [&]() {
@@ -266,8 +293,9 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     issue(3, 1, 1);
   };
 
-  int lid = next_tile(t_begin + (bid >> 3));
+  int lid = t_begin + (bid >> 3);
   if (lid >= t_end) return;
+  select(lid);
   prologue();
   for (;;) {
 #pragma unroll
@@ -288,13 +316,17 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped tail reloads landed before the buffers are refilled
 
     const int cmt = mt, cnt = nt;
-    const int tok0 = (GRP ? row0 : cmt * kBM) + wr * 128 + l15;
+    const int tok0 = (GRP ? row0 + wr * 16 * (n1 + n2) : cmt * kBM + wr * 128) + l15;
+    const int c1n = GRP ? n1 : 4, cn = GRP ? n1 + n2 : 8;  // (the next tile's select changes n1 and n2)
+    // accumulator column j: block j of phase one, block j - 4 of phase two
+    auto block = [&](int j) { return GRP ? (j < 4 ? j : c1n + j - 4) : j; };
+    auto absent = [&](int j) { return GRP && (j < 4 ? j >= c1n : c1n + j - 4 >= cn); };
     const int tok_end = GRP ? rend : M;
     // grouped + scatter: the 8 destination rows, loaded and retired like the row scales below
     int dstv[8];
     if constexpr (GRP) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) dstv[j] = gm.scatter ? gm.order[min(tok0 + 16 * j, tok_end - 1)] : tok0 + 16 * j;
+      for (int j = 0; j < 8; ++j) dstv[j] = gm.scatter ? gm.order[min(tok0 + 16 * block(j), tok_end - 1)] : tok0 + 16 * block(j);
 #pragma unroll
       for (int j = 0; j < 8; ++j) asm volatile("" ::"v"(dstv[j]));
     }
@@ -312,10 +344,10 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     }
 
     // the next tile's first K-tiles go out before this tile's stores
-    const int nlid = next_tile(lid + per_xcd);
-    const bool more = nlid < t_end;
+    lid += per_xcd;
+    const bool more = lid < t_end;
     if (more) {
-      lid = nlid;
+      select(lid);
       prologue();
     }
 
@@ -323,8 +355,8 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     if (EPI == EPI_STORE) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int tok = tok0 + 16 * j;
-        if (tok >= tok_end) continue;
+        const int tok = tok0 + 16 * block(j);
+        if (absent(j) || tok >= tok_end) continue;
         bf16_t* yr = y + (int64_t)(GRP ? dstv[j] : tok) * ldy + cnt * kBN + wc * 64 + 4 * lq;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -337,8 +369,8 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int tok = tok0 + 16 * j;
-        if (tok >= tok_end) continue;
+        const int tok = tok0 + 16 * block(j);
+        if (absent(j) || tok >= tok_end) continue;
         bf16_t* yr = y + (int64_t)(GRP ? dstv[j] : tok) * ldy + cnt * (kBN / 2) + wc * 32 + 4 * lq;
         const float sc = EPI == EPI_SILU_RS ? scv[j] : 1.f;
 #pragma unroll

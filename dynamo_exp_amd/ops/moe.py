@@ -25,6 +25,9 @@ GROUP_SCORES = {"top2": 0, "max": 1}
 # workgroup per expert and 256 columns) would leave a good part of the chip idle, half as many elsewhere
 STREAM_ROWS = 24
 STREAM_TILES = 192
+# row tiles per band of the 256-tile kernel's walk: 16 experts, 300 / 500 / 1000 / 2500 / 4000 tokens, us: 6 307 327 380 531 751,
+# 8 318 347 402 540 759, 2 319 347 391 547 803, 16 slower than 8
+GROUP_BAND = 6
 GLU_BLOCK = 32  # rows per gate / up block of weights interleaved for the fused SwiGLU epilogue
 
 
@@ -197,7 +200,7 @@ def grouped_gemm(a: torch.Tensor, w: torch.Tensor, order: torch.Tensor, offsets:
     if tile_gemm_ok(a, w):
         _native.kernels().gemm256_grouped(out.data_ptr(), out.stride(0), a.data_ptr(), a.stride(0), a.shape[0],
                                           w.data_ptr(), order.data_ptr(), offsets.data_ptr(), R, E, N, K, top,
-                                          int(gather), int(scatter), int(glu), 8, _stream())
+                                          int(gather), int(scatter), int(glu), GROUP_BAND, _stream())
         return out
     _m().grouped_gemm(out.data_ptr(), a.data_ptr(), a.stride(0), w.data_ptr(), order.data_ptr(), offsets.data_ptr(),
                       R, E, N, K, top, int(gather), int(scatter), _f32(a), _stream())
