@@ -32,7 +32,7 @@ int dx_gemm256_grouped(void*, int64_t, const void*, int64_t, int64_t, const void
                        int, int, int, int, int, int, int, hipStream_t);
 int dx_row_rrms(float*, const void*, int, int, int64_t, float, hipStream_t);
 int dx_embedding(void*, const void*, const void*, int, int, int, int64_t, hipStream_t);
-int dx_decode_attention(void*, float*, float*, const void*, int64_t, const void*, const void*, const int*, int,
+int dx_decode_attention(void*, float*, float*, const void*, int64_t, const void*, const void*, const int*, int, int,
                         const int*, int, int, int, int, int, int, float, int, float, float, hipStream_t);
 int dx_prefill_attention(void*, const void*, int64_t, const void*, const void*, const int*, int, const int*,
                          const int*, const int*, int, int, int, int, int, float, int, int, hipStream_t);
@@ -112,10 +112,10 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("embedding", [](u out, u table, u ids, int ids_i64, int tokens, int hidden, int64_t vocab, u st) {
     check(dx_embedding(P(out), P(table), P(ids), ids_i64, tokens, hidden, vocab, S(st)), "embedding");
   });
-  m.def("decode_attention", [](u out, u tmp_out, u tmp_ml, u q, int64_t qs, u kc, u vc, u bt, int bts, u ctx,
+  m.def("decode_attention", [](u out, u tmp_out, u tmp_ml, u q, int64_t qs, u kc, u vc, u bt, int bts, int btc, u ctx,
                                int batch, int hq, int hkv, int hd, int bs, int n_parts, float scale, int kv_fp8,
                                float k_scale, float v_scale, u st) {
-    check(dx_decode_attention(P(out), (float*)tmp_out, (float*)tmp_ml, P(q), qs, P(kc), P(vc), (const int*)bt, bts,
+    check(dx_decode_attention(P(out), (float*)tmp_out, (float*)tmp_ml, P(q), qs, P(kc), P(vc), (const int*)bt, bts, btc,
                               (const int*)ctx, batch, hq, hkv, hd, bs, n_parts, scale, kv_fp8, k_scale, v_scale,
                               S(st)),
           "decode_attention");

@@ -560,8 +560,8 @@ def decode_attention(q, k_cache, v_cache, block_tables, ctx_lens, scale, out, n_
     else:
         t0 = t1 = 0
     _k().decode_attention(out.data_ptr(), t0, t1, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
-                          block_tables.data_ptr(), block_tables.stride(0), ctx_lens.data_ptr(), B, Hq, Hkv, D, BS,
-                          int(n_parts), float(scale), int(_kv_fp8(k_cache)), float(kv_scales[0]), float(kv_scales[1]),
+                          block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1], ctx_lens.data_ptr(), B, Hq, Hkv,
+                          D, BS, int(n_parts), float(scale), int(_kv_fp8(k_cache)), float(kv_scales[0]), float(kv_scales[1]),
                           _stream())
     return out
 

@@ -1,0 +1,41 @@
+"""Decode attention's join of partitions and its block-table prefetch (csrc/kernels/attn_decode.hip): numbers of parts
+around the 16 rows and the 64 lanes that the join asks for at once, workspaces full of NaN, rows and workspaces with
+their elements' alignment only, and tables of fewer and of more than the 64 columns that are asked for early."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from dynamo_exp_amd import ops
+from dynamo_exp_amd.ops import reference as ref
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ctx", [[1, 17, 130], [2100, 3, 0, 1024], [20000, 129]])
+@pytest.mark.parametrize("n_parts", [2, 15, 16, 17, 64, 65, 150])
+def test_parts(ctx, n_parts):
+    torch.manual_seed(n_parts)
+    B, hq, hkv, bs = len(ctx), 8, 2, 16
+    need = [-(-c // bs) for c in ctx]
+    wide = max(need) + 5
+    table = torch.zeros(B, wide, dtype=torch.int32)
+    ids = torch.randperm(sum(need)).to(torch.int32)
+    for b, n in enumerate(need):
+        table[b, :n] = ids[sum(need[:b]):sum(need[:b]) + n]
+    kc, vc = (torch.randn(sum(need), hkv, bs, 128).bfloat16() for _ in range(2))
+    q, lens, scale = torch.randn(B, hq, 128).bfloat16(), torch.tensor(ctx, dtype=torch.int32), 1 / math.sqrt(128)
+    live = [b for b in range(B) if ctx[b]]
+    want = ref.paged_attention(q[live], kc, vc, table[live], torch.arange(len(live) + 1, dtype=torch.int32), lens[live], scale, bs)
+    bt = table.cuda()[:, :max(need)]  # rows farther apart than the columns that may be read
+    nan = float("nan")
+    out = torch.full((B * hq * 128 + 1,), nan, dtype=torch.bfloat16, device="cuda")[1:].view(B, hq, 128)
+    ws = (torch.full((B * hq * n_parts * 128 + 1,), nan, device="cuda")[1:].view(B, hq, n_parts, 128),
+          torch.full((B * hq * n_parts * 2 + 1,), nan, device="cuda")[1:].view(B, hq, n_parts, 2))
+    ops.decode_attention(q.cuda(), kc.cuda(), vc.cuda(), bt, lens.cuda(), scale, out, n_parts, workspace=ws)
+    got = out.cpu()
+    assert bool((got[[b for b in range(B) if not ctx[b]]] == 0).all())
+    # bf16 weights (2^-9 each, of values of order one) and one rounding of the result
+    err = (got[live].float() - want.float()).abs().max()
+    assert float(err) < 2 ** -7 * max(1.0, float(want.float().abs().max())), float(err)
