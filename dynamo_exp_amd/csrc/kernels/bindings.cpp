@@ -28,6 +28,8 @@ int dx_kv_dequant(const void*, const void*, void*, void*, const int*, int, const
 int dx_kv_write(const void*, const void*, int64_t, const int64_t*, void*, void*, int, int, int, int, hipStream_t);
 int dx_silu_and_mul(void*, const void*, int, int, int64_t, int64_t, int, hipStream_t);
 int dx_gemm256(void*, int64_t, const void*, int64_t, const void*, int, int, int, int, int, hipStream_t, const float*);
+int64_t dx_gemm256_add_floats(int, int, int);
+int dx_gemm256_add(void*, int64_t, const void*, int64_t, const void*, int, int, int, int, float*, hipStream_t);
 int dx_gemm256_grouped(void*, int64_t, const void*, int64_t, int64_t, const void*, const int*, const int*, int, int,
                        int, int, int, int, int, int, int, hipStream_t);
 int dx_row_rrms(float*, const void*, int, int, int64_t, float, hipStream_t);
@@ -130,6 +132,10 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("prefill_tile_tokens", &dx_prefill_tile_tokens);
   m.def("gemm256", [](u y, int64_t ldy, u x, int64_t ldx, u w, int M, int N, int K, int epi, int gm, u st, u rs) {
     check(dx_gemm256(P(y), ldy, P(x), ldx, P(w), M, N, K, epi, gm, S(st), (const float*)rs), "gemm256");
+  });
+  m.def("gemm256_add_floats", &dx_gemm256_add_floats);
+  m.def("gemm256_add", [](u y, int64_t ldy, u x, int64_t ldx, u w, int M, int N, int K, int gm, u ws, u st) {
+    check(dx_gemm256_add(P(y), ldy, P(x), ldx, P(w), M, N, K, gm, (float*)ws, S(st)), "gemm256_add");
   });
   m.def("gemm256_grouped", [](u y, int64_t ldy, u x, int64_t ldx, int64_t x_rows, u w, u order, u offsets, int R, int E,
                               int N, int K, int top, int gather, int scatter, int epi, int gm, u st) {

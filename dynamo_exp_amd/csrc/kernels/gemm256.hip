@@ -1,4 +1,4 @@
-// Large-M projection GEMM for gfx950 (prefill token counts), two epilogues:
+// Large-M projection GEMM for gfx950 (prefill token counts), three epilogues:
 //   EPI_STORE:  y[M, N]   = x[M, K] . w[N, K]^T
 //   EPI_SILU:   y[M, N/2] = silu(g) * u, where the N weight rows are the MLP's
 //               gate and up projections interleaved in blocks of 32 rows
@@ -6,6 +6,8 @@
 //               the SwiGLU of the Llama MLP fused into the gate_up GEMM, so the
 //               [M, 2F] intermediate is never written or re-read and the
 //               separate silu_and_mul launch disappears.
+//   EPI_ADD:    y[M, N]  += x[M, K] . w[N, K]^T, for a residual stream behind a
+//               long sum (the MLP's down projection)
 // bf16 in / out, fp32 accumulation (SURVEY §2.15 "SiLU-gated MLP").
 //
 // Design (CDNA4 guide §5 "256² 8-phase template", re-derived here):
@@ -49,6 +51,14 @@
 //     layer, 16 experts of width 3584, 2 a token, model width 4096, us: 300
 //     tokens 421 -> 307 (1.41 GB of weights: 4.6 TB/s), 1000 462 -> 390, 2500
 //     667 -> 539, 4000 854 -> 754; 8 experts of 2048, width 2048, 2500: 186 -> 186.
+//   * EPI_ADD with a last round that fills at most half of the CUs: its tiles are
+//     cut along K into as many pieces as there are CUs for (16 at most), the
+//     pieces' fp32 sums go through a workspace (64 MB at most) to a kernel that
+//     adds them in order.  One more round costs 230 to 320 us at K 14336, whatever
+//     it holds; a sixteenth of one costs 20 and the way through the workspace 30:
+//     4150 x 4096 520 -> 365 us, 1000 x 4096 227 -> 104.  (In a full round the
+//     clock falls to 1.45 GHz at 82 % of the matrix cores' cycles: the card's
+//     power, not the schedule, is the bound there.)
 //   * Blocks are remapped so that each XCD walks a contiguous range of tiles
 //     (bijective for any grid size), in bands of group_m token tiles: the ~32
 //     workgroups resident on one XCD then share group_m x tiles and
@@ -70,7 +80,15 @@ constexpr int kLds = 2 * kBuf;     // double buffered: 128 KB
 // EPI_SILU_RS: EPI_SILU whose input rows carry a deferred RMSNorm: g and u
 // are scaled by rs[token] (1 / rms of the row) before the activation -- the
 // norm's weight is folded into the weight columns (models/llama.py)
-enum { EPI_STORE = 0, EPI_SILU = 1, EPI_SILU_RS = 2 };
+// EPI_ADD: y += x . w^T (one rounding), the tiles of an incomplete last round split along K (Split)
+enum { EPI_STORE = 0, EPI_SILU = 1, EPI_SILU_RS = 2, EPI_ADD = 3 };
+
+// EPI_ADD: tiles 0 .. full - 1 are whole; each of the `rest` behind them is `segs` pieces of K, whose fp32 sums go to
+// part[piece * rest + tile][block (i, j) of the wave][thread] and are joined by gemm256_join_kernel.
+struct Split {
+  f32x4* part;
+  int full, rest, segs;
+};
 
 __device__ __forceinline__ float silu_f(float g) { return g / (1.f + __expf(-g)); }
 
@@ -82,11 +100,25 @@ struct GroupMap {
   int E, top, gather, scatter;
 };
 
+// four bf16 plus four sums, rounded once
+__device__ __forceinline__ uint2 add_bf16x4(uint2 a, f32x4 v) {
+  return uint2{pack_bf16x2(bf16lo(a.x) + v[0], bf16hi(a.x) + v[1]), pack_bf16x2(bf16lo(a.y) + v[2], bf16hi(a.y) + v[3])};
+}
+
+// tile lid -> (token tile, weight tile): bands of group_m token tiles across all weight tiles, token tile fastest
+__device__ __forceinline__ void tile_of(int lid, int mtn, int ntn, int group_m, int& mt, int& nt) {
+  const int band = lid / (group_m * ntn), first_m = band * group_m;
+  const int gsz = min(mtn - first_m, group_m), in_band = lid - band * group_m * ntn;
+  mt = first_m + in_band % gsz;
+  nt = in_band / gsz;
+}
+
 template <int EPI, bool GRP>
 __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, int64_t ldy,
                                                       const bf16_t* __restrict__ x, int64_t ldx,
                                                       const bf16_t* __restrict__ w, int M, int N, int K,
-                                                      int group_m, const float* __restrict__ rs, GroupMap gm) {
+                                                      int group_m, const float* __restrict__ rs, GroupMap gm,
+                                                      Split sp) {
   __shared__ __attribute__((aligned(16))) char smem[kLds];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -106,7 +138,7 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     for (int d = 32; d; d >>= 1) n += __shfl_xor(n, d);
     mtn = __builtin_amdgcn_readfirstlane(n);
   }
-  const int ntn = N / kBN, nwg = mtn * ntn;
+  const int ntn = N / kBN, nwg = EPI == EPI_ADD ? sp.full : mtn * ntn;
   const int G = gridDim.x, bid = blockIdx.x, xcd = bid & 7;
   const int gq = G >> 3, gr8 = G & 7;                 // workgroups on this XCD: gq (+1)
   const int per_xcd = xcd < gr8 ? gq + 1 : gq;
@@ -143,8 +175,9 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   const bf16_t* xb = x;
   const bf16_t* wb = w;
   int xoff[2][2];  // per tile: x part offsets (rows past M re-read row M-1)
+  int kbase = 0, nk = nkt;  // K tiles of this unit of work
   auto issue = [&](int P, int kt, int buf) {
-    kt = min(kt, nkt - 1);  // past the end: harmless reload into a buffer that is not read again
+    kt = min(kt, nk - 1) + kbase;  // past the end: harmless reload into a buffer that is not read again
     const bf16_t* src = (P < 2 ? xb : wb) + kt * kBK;
     char* dst = smem + buf * kBuf;
 #pragma unroll
@@ -234,18 +267,14 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     compute2(1, 6);
   };
 
-  // tile lid -> (token tile, weight tile): bands of group_m token tiles across
-  // all weight tiles, token tile fastest: the ~32 workgroups resident on an XCD
+  // (tile_of) the ~32 workgroups resident on an XCD
   // cover group_m x (32 / group_m) tiles (8 x 4: 12 KB of new operand bytes per
   // workgroup and K-step through the XCD's L2 instead of 33 KB for one weight
   // tile x 32 token tiles)
   int mt = 0, nt = 0;
   int row0 = 0, rend = 0;  // grouped: this tile's first sorted row and its expert's end
   auto select = [&](int lid) {
-    const int band = lid / (group_m * ntn), first_m = band * group_m;
-    const int gsz = min(mtn - first_m, group_m), in_band = lid - band * group_m * ntn;
-    mt = first_m + in_band % gsz;
-    nt = in_band / gsz;
+    tile_of(lid, mtn, ntn, group_m, mt, nt);
     if constexpr (GRP) {
       int e = 0, rem = mt, lo = 0, hi = 0;
       for (; e < gm.E; ++e) {
@@ -293,9 +322,27 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     issue(3, 1, 1);
   };
 
+  bool piece = false;  // EPI_ADD: this workgroup is at its piece of K, number `unit`
+  const int unit = (xcd < gr8 ? xcd * (gq + 1) : gr8 * (gq + 1) + (xcd - gr8) * gq) + (bid >> 3);
+  auto begin = [&](int lid) -> bool {
+    if (lid < t_end) {
+      select(lid);
+      return true;
+    }
+    if constexpr (EPI == EPI_ADD) {
+      // the workgroups of an XCD take the same piece of neighbouring tiles
+      if (piece || unit >= sp.rest * sp.segs) return false;
+      piece = true;
+      const int c = unit / sp.rest, pairs = nkt / 2;
+      kbase = pairs * c / sp.segs * 2;
+      nk = pairs * (c + 1) / sp.segs * 2 - kbase;
+      select(sp.full + unit - c * sp.rest);
+      return true;
+    }
+    return false;
+  };
   int lid = t_begin + (bid >> 3);
-  if (lid >= t_end) return;
-  select(lid);
+  if (!begin(lid)) return;
   prologue();
   for (;;) {
 #pragma unroll
@@ -308,7 +355,7 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     __builtin_amdgcn_s_barrier();
     if (wave >= 4) __builtin_amdgcn_s_barrier();  // start the lagging group one barrier late
     __builtin_amdgcn_sched_barrier(0);
-    for (int t = 0; t < nkt; t += 2) {
+    for (int t = 0; t < nk; t += 2) {
       ktile2(t, 0);
       ktile2(t + 1, 1);
     }
@@ -344,15 +391,36 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     }
 
     // the next tile's first K-tiles go out before this tile's stores
-    lid += per_xcd;
-    const bool more = lid < t_end;
-    if (more) {
-      select(lid);
-      prologue();
+    if constexpr (EPI == EPI_ADD) {
+      // (in front of the next unit's prologue: its DMA would retire before the loads of y)
+      if (piece) {
+        f32x4* o = sp.part + (int64_t)unit * (kBM * kBN / 4) + threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) o[(i * 8 + j) * 512] = acc[i][j];
+        return;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int tok = tok0 + 16 * j;
+        if (tok >= tok_end) continue;
+        bf16_t* yr = y + (int64_t)tok * ldy + cnt * kBN + wc * 64 + 4 * lq;
+        uint2 was[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) was[i] = *reinterpret_cast<const uint2*>(yr + 16 * i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(yr + 16 * i) = add_bf16x4(was[i], acc[i][j]);
+      }
     }
+    lid += per_xcd;
+    const bool more = begin(lid);
+    if (more) prologue();
 
     // ---- epilogue: acc[i][j] register r = (weight row wc*64 + 16 i + 4 lq + r, token 16 j + l15)
-    if (EPI == EPI_STORE) {
+    if (EPI == EPI_ADD) {
+      // done above
+    } else if (EPI == EPI_STORE) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int tok = tok0 + 16 * block(j);
@@ -391,6 +459,29 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   }
 }
 
+// y += the pieces of K of the tiles that EPI_ADD split.  grid (2 * 8, rest), block 256: the 16 rows j of half of the
+// tile's waves
+__global__ void __launch_bounds__(256) gemm256_join_kernel(bf16_t* __restrict__ y, int64_t ldy, int M, int N, int group_m,
+                                                           Split sp) {
+  const int j = blockIdx.x & 7, thread = (blockIdx.x >> 3) * 256 + threadIdx.x, wave = thread >> 6;
+  const int wr = wave >> 2, wc = wave & 3, l15 = thread & 15, lq = (thread & 63) >> 4;
+  int mt, nt;
+  tile_of(sp.full + blockIdx.y, (M + kBM - 1) / kBM, N / kBN, group_m, mt, nt);
+  const int tok = mt * kBM + wr * 128 + 16 * j + l15;
+  if (tok >= M) return;
+  bf16_t* yr = y + (int64_t)tok * ldy + nt * kBN + wc * 64 + 4 * lq;
+  uint2 was[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) was[i] = *reinterpret_cast<const uint2*>(yr + 16 * i);
+  f32x4 sum[4] = {};
+  const f32x4* p = sp.part + (int64_t)blockIdx.y * (kBM * kBN / 4) + j * 512 + thread;
+  for (int c = 0; c < sp.segs; ++c, p += (int64_t)sp.rest * (kBM * kBN / 4))
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += p[i * 8 * 512];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2*>(yr + 16 * i) = add_bf16x4(was[i], sum[i]);
+}
+
 // one resident workgroup per CU (128 KB of LDS): a grid of min(tiles, CUs)
 // workgroups walks all tiles
 int num_cus() {
@@ -412,7 +503,7 @@ void launch(bf16_t* y, int64_t ldy, const bf16_t* x, int64_t ldx, const bf16_t* 
   const int tiles = ((M + kBM - 1) / kBM) * (N / kBN);
   const int grid = persistent ? std::min(tiles, num_cus()) : tiles;
   hipLaunchKernelGGL((gemm256_kernel<EPI, false>), dim3(grid), dim3(512), 0, st, y, ldy, x, ldx, w, M, N, K, gm, rs,
-                     GroupMap{nullptr, nullptr, 0, 1, 0, 0});
+                     GroupMap{nullptr, nullptr, 0, 1, 0, 0}, Split{nullptr, 0, 0, 0});
 }
 
 template <int EPI>
@@ -420,7 +511,7 @@ void launch_grouped(bf16_t* y, int64_t ldy, const bf16_t* x, int64_t ldx, const 
                     hipStream_t st, const GroupMap& map) {
   const int tiles = ((R + kBM - 1) / kBM + map.E) * (N / kBN);
   hipLaunchKernelGGL((gemm256_kernel<EPI, true>), dim3(std::min(tiles, num_cus())), dim3(512), 0, st, y, ldy, x, ldx, w,
-                     R, N, K, gm, nullptr, map);
+                     R, N, K, gm, nullptr, map, Split{nullptr, 0, 0, 0});
 }
 
 }  // namespace
@@ -447,6 +538,47 @@ extern "C" int dx_gemm256(void* y, int64_t ldy, const void* x, int64_t ldx, cons
   else if (epi == EPI_SILU) launch<EPI_SILU>(Y, ldy, X, ldx, W, M, N, K, group_m, persistent, st, nullptr);
   else if (epi == EPI_SILU_RS && rs != nullptr) launch<EPI_SILU_RS>(Y, ldy, X, ldx, W, M, N, K, group_m, persistent, st, rs);
   else return 2;
+  DX_CHECK_LAUNCH();
+  return 0;
+}
+
+// How dx_gemm256_add splits its tiles: {whole tiles, the rest, pieces of K each}.  A last round that fills at most half of
+// the CUs is cut along K.
+static void add_split(int M, int N, int K, int* full, int* rest, int* segs) {
+  const int tiles = (M + kBM - 1) / kBM * (N / kBN), cus = num_cus(), left = tiles % cus;
+  *full = tiles, *rest = 0, *segs = 0;
+  if (left == 0 || 2 * left > cus) return;
+  *full = tiles - left, *rest = left, *segs = std::min(std::min(cus / left, 16), K / (2 * kBK));
+}
+
+// fp32 workspace (floats) of dx_gemm256_add
+extern "C" int64_t dx_gemm256_add_floats(int M, int N, int K) {
+  if (M < 1 || N < kBN || N % kBN || K < 2 * kBK || K % (2 * kBK)) return 0;
+  int full, rest, segs;
+  add_split(M, N, K, &full, &rest, &segs);
+  return (int64_t)rest * segs * kBM * kBN;
+}
+
+// y[M, N] += x[M, K] . w[N, K]^T, each element rounded once; ws: dx_gemm256_add_floats floats, 16-byte aligned.  Same
+// requirements as dx_gemm256.
+extern "C" int dx_gemm256_add(void* y, int64_t ldy, const void* x, int64_t ldx, const void* w, int M, int N, int K,
+                              int group_m, float* ws, hipStream_t st) {
+  if (M < 1) return 0;
+  if (group_m < 1) return 7;
+  if (N < kBN || N % kBN != 0 || K % (2 * kBK) != 0 || K < 2 * kBK) return 3;
+  if ((ldx & 7) || (ldy & 3) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(w) & 15) ||
+      (reinterpret_cast<uintptr_t>(y) & 7) || (reinterpret_cast<uintptr_t>(ws) & 15))
+    return 5;
+  if ((int64_t)N * K >= (1ll << 31) || (int64_t)kBM * ldx >= (1ll << 31)) return 6;  // 32-bit DMA offsets
+  Split sp{reinterpret_cast<f32x4*>(ws), 0, 0, 0};
+  add_split(M, N, K, &sp.full, &sp.rest, &sp.segs);
+  if (sp.rest && !ws) return 5;
+  const int grid = std::max(std::min(sp.full, num_cus()), sp.rest * sp.segs);
+  auto* Y = static_cast<bf16_t*>(y);
+  hipLaunchKernelGGL((gemm256_kernel<EPI_ADD, false>), dim3(grid), dim3(512), 0, st, Y, ldy, static_cast<const bf16_t*>(x),
+                     ldx, static_cast<const bf16_t*>(w), M, N, K, group_m, nullptr, GroupMap{nullptr, nullptr, 0, 1, 0, 0}, sp);
+  if (sp.rest)
+    hipLaunchKernelGGL(gemm256_join_kernel, dim3(16, sp.rest), dim3(256), 0, st, Y, ldy, M, N, group_m, sp);
   DX_CHECK_LAUNCH();
   return 0;
 }

@@ -606,7 +606,7 @@ class LlamaForCausalLM:
             else:
                 gu = self._mm(res, L["gate_up"])
                 a = ops.silu_and_mul((gu.float() * rs[:, None]).to(gu.dtype), blk=self.gu_blk)
-            res.addmm_(a, L["down"].t())
+            ops.linear_add_(res, a, L["down"])
         if meta.logits_idx is not None:
             if meta.logits_idx.numel() == 0:
                 return res[:0]

@@ -226,6 +226,7 @@ def silu_and_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None, blk: in
 
 # ---------------------------------------------------------------- large-M GEMM
 GEMM256_EPI_STORE, GEMM256_EPI_SILU, GEMM256_EPI_SILU_RS = 0, 1, 2
+GEMM256_ADD_BAND = 16  # token tiles per L2 band: 6151 x 4096 x 14336, us: 4 580, 8 581, 16 568, 24 590
 GEMM256_BLK = 32  # gate / up interleave of the fused SwiGLU epilogue
 
 
@@ -272,6 +273,37 @@ def gemm256(x: torch.Tensor, w: torch.Tensor, epi: int = GEMM256_EPI_STORE, out:
     _k().gemm256(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), M, N, K, epi, group_m,
                  _stream(), 0 if row_scale is None else row_scale.data_ptr())
     return out
+
+
+CUS = 256  # compute units of an MI355X
+
+
+def deep_add_tiles(M: int, N: int, K: int) -> bool:
+    """Whether y[M, N] += x w^T over a long K takes the 256-tile kernel.  It cuts an incomplete last round along K; the
+    library's choice for these shapes is uneven.  us, library / this kernel, N 4096:
+      K 14336  M 600 98 / 82, 1000 119 / 104, 1450 156 / 155, 2125 214 / 250, 3925 301 / 317, 4150 719 / 365,
+               5050 439 / 427, 5950 513 / 502, 6175 816 / 580, 7525 1010 / 626, 7750 605 / 633, 8200 1027 / 685
+      K 11008  M 600 76 / 68, 1560 127 / 128, 3000 196 / 211, 4440 632 / 309, 4920 337 / 336, 6360 643 / 449
+      K 8192   M 600 60 / 58, 1080 75 / 83, 3000 152 / 167, 4440 258 / 227, 6360 315 / 333, 7320 326 / 351
+    So: K from 10240, and either up to a third of a round (three pieces of K and more) or more than one round whose
+    last is not all but full.  (Below 384 rows nothing was gained at K 11008.)"""
+    tiles = -(-M // 256) * (N // 256)
+    left = tiles % CUS
+    return K >= 10240 and M >= 384 and (3 * tiles <= CUS or (tiles > CUS and 0 < 16 * left < 15 * CUS))
+
+
+def linear_add_(y: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """y += x @ w.T in place, the products summed in fp32 and each element rounded once."""
+    M, K = x.shape
+    N = w.shape[0]
+    if not (deep_add_tiles(M, N, K) and gemm256_ok(x, w) and y.dtype == x.dtype and y.shape == (M, N) and y.stride(1) == 1
+            and y.stride(0) % 4 == 0 and y.data_ptr() % 8 == 0):
+        return y.addmm_(x, w.t())
+    floats = _k().gemm256_add_floats(M, N, K)
+    ws = torch.empty(floats, dtype=torch.float32, device=y.device)
+    _k().gemm256_add(y.data_ptr(), y.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), M, N, K, GEMM256_ADD_BAND,
+                     ws.data_ptr() if floats else 0, _stream())
+    return y
 
 
 # ---------------------------------------------------------------- small-M GEMM

@@ -1,0 +1,63 @@
+"""y += x w^T on the 256-tile kernel (csrc/kernels/gemm256.hip): whole tiles, a last round cut along K, both together;
+and which shapes take it."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from dynamo_exp_amd import ops
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,pieces", [
+    (1, 256, 128, 1),  # one tile whose K does not divide
+    (300, 512, 256, 2), (255, 256, 1408, 11), (257, 768, 2304, 16),  # pieces of one and more pairs of K tiles
+    (1100, 4096, 512, 3), (2049, 4096, 384, 0), (4096, 4096, 256, 0),  # 80, 144 and 256 tiles
+    (4097, 4096, 640, 5), (16500, 512, 2176, 0),  # a full round and 16; 130 tiles
+    (33000, 512, 1152, 9),  # 258: the rest in the last rows
+])
+def test_add(M, N, K, pieces):
+    torch.manual_seed(M)
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * 0.1).bfloat16()
+    y0 = torch.randn(M, N + 4, device="cuda").bfloat16()
+    tiles = -(-M // 256) * (N // 256)
+    left = tiles % 256 if pieces else 0
+    floats = ops._k().gemm256_add_floats(M, N, K)
+    assert floats == left * pieces * 65536
+    outs = []
+    for _ in range(2):
+        y = y0.clone()
+        ws = torch.full((max(floats, 1),), float("nan"), device="cuda")
+        ops._k().gemm256_add(y.data_ptr(), y.stride(0), x.data_ptr(), K, w.data_ptr(), M, N, K, 16, ws.data_ptr(), ops._stream())
+        outs.append(y)
+    assert torch.equal(*outs) and torch.equal(outs[0][:, N:], y0[:, N:])
+    want = y0[:, :N].double() + x.double() @ w.double().t()
+    # one rounding to bf16 (2^-9 relative) over fp32 sums of K terms of 0.1
+    err = (outs[0][:, :N].double() - want).abs()
+    assert bool((err <= 2 ** -8 * want.abs() + 2 ** -22 * K).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [500, 1280, 1300, 4200])
+def test_linear_add(M):
+    """The op on both sides of its rule, and rows whose alignment the kernel does not take."""
+    torch.manual_seed(M)
+    N, K = 4096, 10240
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    assert ops.deep_add_tiles(M, N, K) == (M != 1300)
+    want = x.double() @ w.double().t()
+    for y in (torch.randn(M, N, device="cuda").bfloat16(), torch.randn(M * N + 1, device="cuda").bfloat16()[1:].view(M, N),
+              torch.randn(N, M, device="cuda").bfloat16().t()):
+        exact = y.double() + want
+        assert ops.linear_add_(y, x, w) is y
+        assert bool(((y.double() - exact).abs() <= 2 ** -8 * exact.abs() + 2 ** -22 * K).all())
+
+
+def test_rule_and_cpu():
+    ok = ops.deep_add_tiles
+    assert ok(600, 4096, 14336) and ok(6151, 4096, 14336) and ok(384, 4096, 10240)
+    for shape in ((383, 4096, 14336), (6151, 4096, 10112), (2000, 4096, 14336), (4096, 4096, 14336), (7936, 4096, 14336)):
+        assert not ok(*shape), shape
+    y, x, w = torch.randn(384, 256), torch.randn(384, 10240), torch.randn(256, 10240)
+    want = torch.addmm(y, x, w.t())
+    assert torch.equal(ops.linear_add_(y, x, w), want)
