@@ -21,8 +21,8 @@
 // 1.32e-7 and 6.91e-8 (900 to 4001 tokens; 1.9e-7 and 1.2e-7 with running products and one chain per sum).
 // A value that is not finite makes its own and the later tokens' results not finite, as token by token; zero factors
 // times it do the same to the rows in front of it in its chunk.
-// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 346 + 145 us; a
-// prompt of 600 beside 30 single tokens 1265 -> 120.  Bound by the fp32 matrix instructions (200 us of them run) beside
+// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us; a
+// prompt of 600 beside 30 single tokens 1265 -> 110.  Bound by the fp32 matrix instructions (200 us of them run) beside
 // the fragments' way through L2.
 #include "recurrent.h"
 
@@ -257,18 +257,32 @@ template <int NB> struct Frags {
   uint32_t v[NB][4];  // rows g4, 4 + g4, 8 + g4 and 12 + g4 of V; bf16 bits as loaded: a conversion here would wait for the load
 };
 
+// The k-th longest of up to 64 sequences (more of them even out by themselves): the workgroups go out in this order, so
+// that the longest does not start when a short one's place is free.
+__device__ __forceinline__ int by_length(const int* seq_rows, int n_seq, int k, int lane) {
+  if (n_seq > 16) return k;
+  const int len = lane < n_seq ? seq_rows[lane + 1] - seq_rows[lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < n_seq; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < n_seq && rank == k));
+}
+
 // NB: blocks of 16 columns per workgroup
 template <int NB>
-__global__ void __launch_bounds__(256, 2) delta_chunk_kernel(ChunkArgs g) {
+__global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(ChunkArgs g) {
   __shared__ __attribute__((aligned(16))) f32x4 px[2][4][NB][64];  // parts of X
   __shared__ float po[2][4][NB][4][64];                             // parts of O, by accumulator register
   const int nb = g.dv / (16 * NB);
   // the column blocks of a (sequence, head) read the same chunks: neighbours on one XCD (blocks go out round robin)
   const int id = blockIdx.x, sh = id / (8 * nb) * 8 + id % 8, blk = id / 8 % nb;
   if (sh >= g.n_seq * g.H) return;
-  const int s = sh / g.H, h = sh - s * g.H;
+  const int h = sh % g.H;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = by_length(g.seq_rows, g.n_seq, sh / g.H, lane);
   const int r0 = g.seq_rows[s], n = g.seq_rows[s + 1] - r0, slot = g.slots[s];
   if (n <= 0 || r0 < 0 || r0 + n > g.T) return;
   const int col0 = h * g.dv + blk * 16 * NB;
@@ -393,14 +407,12 @@ __global__ void __launch_bounds__(256, 2) delta_chunk_kernel(ChunkArgs g) {
             (po[buf][0][q][w][lane] + po[buf][1][q][w][lane]) + (po[buf][2][q][w][lane] + po[buf][3][q][w][lane]);
     }
   };
-  Frags<NB> f0, f1, f2;  // two chunks ahead
+  Frags<NB> f0, f1;  // (two chunks ahead: a workgroup fewer per CU, 1 to 4 % slower)
   load(f0, 0);
-  load(f1, min(1, nc - 1));
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): what is pending here the compiler would wait for in every turn
-  for (int c = 0; c < nc; c += 3) {
-    step(f0, c, f2, c + 2);
-    if (c + 1 < nc) step(f1, c + 1, f0, c + 3);
-    if (c + 2 < nc) step(f2, c + 2, f1, c + 4);
+  for (int c = 0; c < nc; c += 2) {
+    step(f0, c, f1, c + 1);
+    if (c + 1 < nc) step(f1, c + 1, f0, c + 2);
   }
 #pragma unroll
   for (int q = 0; q < NB; ++q)
@@ -441,10 +453,10 @@ int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void
   hipLaunchKernelGGL(delta_form_kernel, dim3(H, T_ / kC + n_seq), dim3(256), 0, st, f);
   ChunkArgs c{out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
   const int64_t heads = ((int64_t)n_seq * H + 7) / 8 * 8;
-  // Two column blocks a workgroup read a chunk once for both; one keeps more of the chip busy where there are few.
-  // Whole layer, 32 heads, us: one prompt of 3000 tokens 420 / 534 (one / two blocks), three of 4001 516 / 500, six of 5000
-  // 622 / 550
-  if (dv % 32 == 0 && heads * (dv / 16) >= 512)
+  // Two column blocks a workgroup read a chunk once for both, but only two of their workgroups fit a CU; one block keeps
+  // more of the chip busy until there are twice as many workgroups as fit.  Whole layer, 32 heads, us, one / two blocks:
+  // two prompts of 3000 tokens together 343 / 392, three of 4001 443 / 479, four of 3000 335 / 325, six of 5000 547 / 481
+  if (dv % 32 == 0 && heads * (dv / 16) >= 1024)
     hipLaunchKernelGGL(delta_chunk_kernel<2>, dim3((unsigned)(heads * (dv / 32))), dim3(256), 0, st, c);
   else
     hipLaunchKernelGGL(delta_chunk_kernel<1>, dim3((unsigned)(heads * (dv / 16))), dim3(256), 0, st, c);

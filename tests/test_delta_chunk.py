@@ -29,7 +29,7 @@ def recurrence(r, k, v, a, w, ab, wb, S, H, dv, scale, eps=1e-6):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [[64], [15, 17, 1, 33], [64, 0, 50, 1, 1], [9, 8, 16, 31], [250]])
+@pytest.mark.parametrize("rows", [[64], [15, 17, 1, 33], [64, 0, 50, 1, 1], [9, 8, 16, 31], [250], [9] * 18])
 @pytest.mark.parametrize("kind", ["plain", "fast decay", "slow decay", "one key", "grown"])
 @pytest.mark.parametrize("H,dv", [(2, 128), (3, 16), (1, 48)])
 def test_delta_chunks(rows, kind, H, dv):
