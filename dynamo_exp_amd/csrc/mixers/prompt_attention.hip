@@ -3,8 +3,10 @@
 // score form of tile_attention.hip: causal, window (with kept first keys) and chunk masks, a tanh cap, a log-distance
 // penalty, sigmoid weights, a sink, a gate per head.  Scores, weights and sums are fp32.
 //
-// A workgroup is eight waves: HPW heads that share a key / value head times 8 / HPW blocks of 32 rows, a wave
-// per (head, block).  Products are v_mfma_f32_32x32x16_bf16, swapped (S^T = K Q^T, O^T = V^T P^T), so a query row
+// A workgroup is four waves: HPW heads that share a key / value head times 4 / HPW blocks of 32 rows, a wave
+// per (head, block).  Two or three workgroups fit a CU and are at different places of their tiles: one's softmax runs
+// beside another's products (eight waves with one barrier went through both in step, and a last round of workgroups
+// that filled a CU each left a quarter of the card idle).  Products are v_mfma_f32_32x32x16_bf16, swapped (S^T = K Q^T, O^T = V^T P^T), so a query row
 // sits on a lane and the score accumulator is the second product's operand.
 //   * Tiles go from the caches to LDS by DMA (global_load_lds, 16 bytes a lane) into a double buffer; the 16-byte
 //     pieces of a row are permuted on the source side, so that both kinds of fragment reads below hit different banks.
@@ -15,12 +17,15 @@
 //     largest weight exactly when that weight is 1, so there the maximum follows every tile.
 //   * Wide shared rows (256 value columns): the upper half of the queries stays in LDS, the accumulators need its
 //     registers.
-// What bounds it: vector issue of the softmax beside the matrix cores at two waves a SIMD (the register file holds no
-// more), score terms most of all.  Against the register-staged, 16x16x32 forms it took over from (tile_attention.hip,
-// stream and latent prefill), 32 heads, ragged prompts of about 4000 tokens, us before -> after: two maps with values
-// of 256, window 1024 + 64: 721 -> 240; shared row 256 / 192 causal 241 -> 137 (720 TFLOP/s), 256 / 256 window 547 ->
-// 124; cap + penalty, window 1024: 315 -> 175; sigmoid 214 -> 92; plain causal, 5000 tokens: 133 -> 124, fine 160 ->
-// 145; 40 rows behind 2900 cached: 132 -> 117.
+//   * Tiles of 64 keys, or of 32 where that lets more workgroups onto a CU: rows of 256 columns, and the forms with
+//     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.
+// What bounds it: vector issue of the softmax beside the matrix cores, score terms most of all (four transcendentals a
+// score with cap and penalty).  Against the register-staged, 16x16x32 forms it took over from (tile_attention.hip,
+// stream and latent prefill), 32 heads, ragged prompts of about 4000 tokens, us: before -> with eight waves -> now: two
+// maps with values of 256 and their combine, window 1024 + 64: 776 -> 303 -> 267; shared row 256 / 192 causal 242 ->
+// 140 -> 124 (800 TFLOP/s), 256 / 256 window 546 -> 124 -> 123; cap + penalty, window 1024: 313 -> 176 -> 136; sigmoid
+// 213 -> 92 -> 86; plain causal, 5000 tokens: 132 -> 124 -> 111, fine 160 -> 148 -> 133; 40 rows behind 2900 cached:
+// 131 -> 117 -> 93.
 #include <type_traits>
 
 #include "stream_attention.h"
@@ -79,12 +84,13 @@ __device__ __forceinline__ float swap_sum(float x) {
 }
 
 // D: key columns, DV: value columns, SAME: the value is the first DV columns of the key's row
-template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW>
-__global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) {
-  constexpr int RT = 8 / HPW, ROWS = 32 * RT;
+// HPW: heads per workgroup, NW: waves, SUBS: blocks of 32 keys per tile
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS>
+__global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) prompt_attention_kernel(PromptArgs a) {
+  constexpr int RT = NW / HPW, ROWS = 32 * RT, KT = 32 * SUBS, SH = SUBS == 2 ? 6 : 5;
   constexpr int KS = D / 16, NC = DV / 32, KB = 2 * D, VB = SAME ? KB : 2 * DV;  // row bytes of the images
-  constexpr int kKey = 64 * KB, kStage = kKey + (SAME ? 0 : 64 * VB);
-  constexpr int KP = 64 * KB / 8192, VP = SAME ? 0 : 64 * VB / 8192;  // 1-KB pieces per wave
+  constexpr int kKey = KT * KB, kStage = kKey + (SAME ? 0 : KT * VB);
+  constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
   constexpr float kDefer = FINE ? 8.f : 0.f;  // log2 units that a score may exceed the running maximum by
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -102,8 +108,8 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
   const int qh = head * a.maps + (gm - g * a.maps);
   const int rw = 32 * (wid / HPW);  // the wave's first row
   const int hi = p0 + min(n, ROWS) - 1;
-  const int first = first_key(p0, a.mask, a.size) >> 6, last = hi >> 6;
-  const int kept = a.mask == 1 ? min((a.keep + 63) >> 6, first) : 0;  // tiles of kept keys in front of the window's
+  const int first = first_key(p0, a.mask, a.size) >> SH, last = hi >> SH;
+  const int kept = a.mask == 1 ? min((a.keep + KT - 1) >> SH, first) : 0;  // tiles of kept keys in front of the window's
   // rows beyond n repeat the last one and are not stored
   const int myrow = min(rw + r, n - 1), my = p0 + myrow, mylo = first_key(my, a.mask, a.size);
   const int wlo = p0 + min(rw, n - 1), whi = p0 + min(rw + 31, n - 1);  // the wave's first and last position
@@ -133,9 +139,9 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
   const bf16_t* kc = a.kc + (int64_t)gm * D;
   const bf16_t* vc = a.vc + (int64_t)g * DV;
   auto issue = [&](char* buf, int t) {
-    const int64_t base = tile_slot(bt, a.bs_shift, t);
+    const int64_t base = tile_slot(bt, a.bs_shift, (t << SH) >> 6) + ((t << SH) & 63);
     const bf16_t *kb = kc + base * a.Wk, *vb = vc + base * a.Wv;
-    const int left = hi - (t << 6);  // rows behind the last query hold stale values: its row instead
+    const int left = hi - (t << SH);  // rows behind the last query hold stale values: its row instead
 #pragma unroll
     for (int k = 0; k < KP; ++k) {
       constexpr int RP = 1024 / KB, CH = KB / 16;
@@ -151,9 +157,9 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
                                        (lds_void*)(buf + kKey + (VP * wid + k) * 1024), 16, 0, 0);
     }
   };
-  const float cap = a.softcap, inv_cap = MODE != kPlain && cap > 0.f ? 1.f / cap : 0.f;
+  const float cap = a.softcap, capl = cap * kLog2e, cape = MODE != kPlain && cap > 0.f ? a.scale * (2.f * kLog2e) / cap : 0.f;
   const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
-  const float r1 = MODE != kPlain && a.r1 ? a.r1[qh] * 1.f : 0.f, r2 = MODE != kPlain && a.r1 ? a.r2[qh] : 0.f;
+  const float r1 = MODE != kPlain && a.r1 ? a.r1[qh] : 0.f, r2 = MODE != kPlain && a.r1 ? a.r2[qh] : 0.f;
   const float sc = terms ? 1.f : a.scale * kLog2e;  // scores to log2 units
   const float hb = MODE == kSigmoid && a.hbias ? a.hbias[qh] * kLog2e : 0.f;
   float m_i = -INFINITY, l_i = 0.f;
@@ -164,37 +170,42 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
   auto step = [&](auto bufc, int t) {
     const char* kb = smem + decltype(bufc)::value * kStage;
     const char* vb = SAME ? kb : kb + kKey;
-    const int kt = t << 6;
-    const bool kept_tile = kt + 64 <= keep;  // wholly of kept keys
-    if (rw >= n || kt > whi || (kt + 63 < wfirst && kt >= keep)) return;  // nothing the wave's rows see
-    const bool live1 = kt + 32 <= whi;  // some row sees the second half
-    f32x16 s[2] = {f32x16{}, f32x16{}};
+    const int kt = t << SH;
+    const bool kept_tile = kt + KT <= keep;  // wholly of kept keys
+    if (rw >= n || kt > whi || (kt + KT - 1 < wfirst && kt >= keep)) return;  // nothing the wave's rows see
+    const bool live1 = SUBS == 2 && kt + 32 <= whi;  // some row sees the second half
+    f32x16 s[SUBS] = {};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const char* kp = kb + koff[ks & 7] + 256 * (ks >> 3);
       const bf16x8_t qk = ks < QR ? qf[ks < QR ? ks : 0] : frag16(ql + (ks - QR) * 512);
       s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)kp), qk, s[0], 0, 0, 0);
-      if (live1) s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)(kp + 32 * KB)), qk, s[1], 0, 0, 0);
+      if constexpr (SUBS == 2)
+        if (live1) s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)(kp + 32 * KB)), qk, s[1], 0, 0, 0);
     }
     if (MODE != kPlain && terms) {  // final scores in log2 units
+      if (cap > 0.f) {  // cap * tanh(x / cap): tanh(y) = 1 - 2 / (1 + e^(2 y))
 #pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
+        for (int sub = 0; sub < SUBS; ++sub)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          float x = s[sub][i] * a.scale;
-          // cap * tanh(x / cap): tanh(y) = 1 - 2 / (1 + e^(2 y))
-          x = cap > 0.f ? cap * kLog2e * (1.f - 2.f * __builtin_amdgcn_rcpf(1.f + fast_exp2(x * (2.f * kLog2e) * inv_cap)))
-                        : x * kLog2e;
-          if (a.r1) {
-            const int dist = my - (kt + 32 * sub + (i & 3) + 8 * (i >> 2) + 4 * h);
-            x -= r1 * __builtin_amdgcn_logf(1.f + r2 * (float)max(dist, 0));
-          }
-          s[sub][i] = x;
-        }
+          for (int i = 0; i < 16; ++i)
+            s[sub][i] = fmaf(-2.f * capl, __builtin_amdgcn_rcpf(1.f + fast_exp2(s[sub][i] * cape)), capl);
+      } else {
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub) s[sub] *= a.scale * kLog2e;
+      }
+      if (a.r1) {  // (keys behind the row: their argument may be anything, they are masked below)
+        const float t0 = fmaf(r2, (float)(my - kt - 4 * h), 1.f);
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            s[sub][i] = fmaf(-r1, __builtin_amdgcn_logf(fmaf(-r2, (float)(32 * sub + (i & 3) + 8 * (i >> 2)), t0)), s[sub][i]);
+      }
     }
-    if (kt + 63 > wlo || (kt < wlast && !kept_tile)) {  // some key is not seen by some row
+    if (kt + KT - 1 > wlo || (kt < wlast && !kept_tile)) {  // some key is not seen by some row
 #pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
+      for (int sub = 0; sub < SUBS; ++sub)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int j = kt + 32 * sub + (i & 3) + 8 * (i >> 2) + 4 * h;
@@ -203,11 +214,21 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
     }
     float mu = 0.f;
     if constexpr (MODE != kSigmoid) {
-      float ta = fmaxf(s[0][0], s[1][0]), tb = fmaxf(s[0][1], s[1][1]);
+      float ta, tb;
+      if constexpr (SUBS == 2) {
+        ta = fmaxf(s[0][0], s[SUBS - 1][0]), tb = fmaxf(s[0][1], s[SUBS - 1][1]);
 #pragma unroll
-      for (int i = 2; i < 16; i += 2) {
-        ta = raw_max3(ta, s[0][i], s[1][i]);
-        tb = raw_max3(tb, s[0][i + 1], s[1][i + 1]);
+        for (int i = 2; i < 16; i += 2) {
+          ta = raw_max3(ta, s[0][i], s[SUBS - 1][i]);
+          tb = raw_max3(tb, s[0][i + 1], s[SUBS - 1][i + 1]);
+        }
+      } else {
+        ta = fmaxf(s[0][0], s[0][1]), tb = fmaxf(s[0][2], s[0][3]);
+#pragma unroll
+        for (int i = 4; i < 16; i += 4) {
+          ta = raw_max3(ta, s[0][i], s[0][i + 1]);
+          tb = raw_max3(tb, s[0][i + 2], s[0][i + 3]);
+        }
       }
       // both halves of a row see the same maximum and take the same decision
       const float tm = swap_max(fmaxf(ta, tb)) * sc;
@@ -224,7 +245,7 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
       m_i = mn;
     }
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
+    for (int sub = 0; sub < SUBS; ++sub) {
       if (sub == 1 && !live1) break;
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
@@ -261,7 +282,6 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
   const int total = kept + last - first + 1;
   auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
   issue(smem, tile(0));
-  if (wid >= 4) __builtin_amdgcn_s_setprio(1);  // else the second wave of each SIMD loses every arbitration
   __syncthreads();  // (waits for the DMA of the tile as well)
   for (int i = 0; i < total; i += 2) {
     if (i + 1 < total) issue(smem + kStage, tile(i + 1));
@@ -307,12 +327,12 @@ __global__ void __launch_bounds__(512, 2) prompt_attention_kernel(PromptArgs a) 
   }
 }
 
-template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW>
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS>
 int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   PromptArgs a = a0;
-  a.subs = 128 / (32 * (8 / HPW));
-  constexpr int lds = 2 * 64 * 2 * (D + (SAME ? 0 : DV)) + (SAME && DV == 256 ? 8 * (D / 16 - 8) * 1024 : 0);
-  auto kern = prompt_attention_kernel<D, DV, SAME, MODE, FINE, OutT, HPW>;
+  a.subs = 128 / (32 * (NW / HPW));
+  constexpr int lds = 2 * 32 * SUBS * 2 * (D + (SAME ? 0 : DV)) + (SAME && DV == 256 ? NW * (D / 16 - 8) * 1024 : 0);
+  auto kern = prompt_attention_kernel<D, DV, SAME, MODE, FINE, OutT, HPW, NW, SUBS>;
   static bool raised = false;  // once per instance
   if (lds > 48 * 1024 && !raised) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 7;
@@ -322,19 +342,19 @@ int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   for (int t0 = 0; t0 < n_tiles; t0 += step) {
     a.tiles = a0.tiles + 2 * t0;
     const int nt = n_tiles - t0 < step ? n_tiles - t0 : step;
-    hipLaunchKernelGGL(kern, dim3(a.n_qh / HPW, nt * a.subs), dim3(512), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(a.n_qh / HPW, nt * a.subs), dim3(64 * NW), lds, st, a);
   }
   DX_CHECK_LAUNCH();
   return 0;
 }
 
+// (tiles of 32 / 64 keys, us: cap + penalty 158 / 173, sigmoid 85 / 91, shared row 256 / 192 of 600 rows 47 / 52, plain
+// 114 / 109, plain behind 2900 cached 107 / 94)
 template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT>
 int prompt_heads(const PromptArgs& a, int n_tiles, hipStream_t st) {
-  if constexpr (SAME) {  // every head shares the row: eight heads over 32 rows meet the fewest tiles outside the mask
-    if (a.group % 8 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 8>(a, n_tiles, st);
-  }
-  if (a.group % 4 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 4>(a, n_tiles, st);
-  return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 2>(a, n_tiles, st);
+  constexpr int SUBS = DV == 128 && MODE == kPlain ? 2 : 1;
+  if (a.group % 4 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 4, 4, SUBS>(a, n_tiles, st);
+  return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 2, 4, SUBS>(a, n_tiles, st);
 }
 
 }  // namespace
