@@ -1,9 +1,9 @@
 // Paged-KV causal prefill attention (varlen, with cached prefix) for gfx950.
 //
 // Flash-attention forward on MFMA v_mfma_f32_32x32x16_bf16:
-//   * workgroup = 8 waves; every wave owns 32 query rows of ONE query head.
-//     The waves of a workgroup share one KV head (GQA group: 4 heads x 2
-//     32-token tiles), so every K/V tile staged in LDS is reused by 8 waves;
+//   * workgroup = 8 or 4 waves; every wave owns 32 query rows of ONE query head.
+//     The waves of a workgroup share one KV head (GQA group: 4 heads x 2 or 1
+//     32-token tiles), so every K/V tile staged in LDS is reused by all of them;
 //     32-row K sub-blocks that lie entirely above a wave's causal diagonal are
 //     skipped (no MFMA, no softmax work);
 //   * K/V tiles of 64 tokens are gathered from the paged cache (block table)
@@ -40,8 +40,8 @@ __device__ __forceinline__ int tile_off(int row, int ch) { return row * 256 + 16
 __device__ __forceinline__ bf16x8_t as_frag(const u16x8& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
 // ---------------------------------------------------------------------------
-// The kernel: 8 waves (4 heads x 64 query tokens per workgroup sharing each
-// K/V tile), K/V staged by LDS-DMA (global_load_lds) into a double-buffered
+// The kernel: NW waves (8: 4 heads x 64 query tokens per workgroup sharing each
+// K/V tile; 4: 32 tokens), K/V staged by LDS-DMA (global_load_lds) into a double-buffered
 // swizzled image, with the per-tile vector work cut down -- the loop is
 // issue-bound, not MFMA-bound, at 2 waves/SIMD.  (Earlier register-staged
 // 4/8-wave, 4-wave x 2 q-block and 3-stage-DMA variants measured 322-794
@@ -93,11 +93,11 @@ __device__ __forceinline__ float halves_sum(float x) {
 
 // V: 0 = the round-3 loop (kept for A/B), 1 = round 4: deferred rescale, row
 // sum on the matrix pipe, v_max3 row max, static priority, widened epilogue.
-// (Round-4 structural variants -- 4-wave workgroups, ping-pong wave halves,
-// two tiles per barrier, a software-pipelined QK / softmax -- all measured
-// slower: profiles/r4_prefill_attn_variants.txt.)
-template <bool BS64, bool PLS, int V>
-__global__ void __launch_bounds__(512, 2) prefill_attn_v2_kernel(
+// (Ping-pong wave halves, two tiles per barrier and a software-pipelined QK /
+// softmax measured slower, as did 4-wave workgroups where there are enough of
+// 8: profiles/r4_prefill_attn_variants.txt.)
+template <bool BS64, bool PLS, int V, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ cu_seqlens_q, const int* __restrict__ ctx_lens, const int* __restrict__ work,
@@ -115,14 +115,18 @@ __global__ void __launch_bounds__(512, 2) prefill_attn_v2_kernel(
   // head's tiles for all work items.
   const int kvh = blockIdx.x / head_groups;
   const int hg = blockIdx.x % head_groups;
-  const int seq = work[2 * blockIdx.y];
-  const int tok0 = work[2 * blockIdx.y + 1];
+  const int token_tiles = NW / heads_per_wg;
+  // a work item is the rows of eight waves; its later rows see more keys and go first
+  const int item = blockIdx.y / (8 / NW), sub = 8 / NW - 1 - blockIdx.y % (8 / NW);
+  const int seq = work[2 * item];
+  const int tok0 = work[2 * item + 1] + sub * token_tiles * BQ;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int q_start = cu_seqlens_q[seq];
   const int qlen = cu_seqlens_q[seq + 1] - q_start;
   const int ctx = ctx_lens[seq];
   const int pos0 = ctx - qlen;
+  if (tok0 >= qlen) return;
   const int r = lane & 31, h = lane >> 5;
 
   const int head = kvh * G + hg * heads_per_wg + (wid % heads_per_wg);
@@ -133,7 +137,6 @@ __global__ void __launch_bounds__(512, 2) prefill_attn_v2_kernel(
   const int my_pos = causal ? pos0 + wtok0 + r : ctx - 1;
   const int wave_min_pos = causal ? pos0 + wtok0 : ctx - 1;
   const int wave_max_pos = causal ? pos0 + min(wtok0 + BQ, qlen) - 1 : ctx - 1;
-  const int token_tiles = 8 / heads_per_wg;
   const int wg_last_tok = min(tok0 + token_tiles * BQ, qlen) - 1;
   const int kv_end = causal ? min(ctx, pos0 + wg_last_tok + 1) : ctx;
   const int n_tiles = (kv_end + BKV - 1) / BKV;
@@ -161,7 +164,7 @@ __global__ void __launch_bounds__(512, 2) prefill_attn_v2_kernel(
     }
   }
   // ---- DMA slots: instruction k of this wave fills tile rows 4*(KPW*wid+k) .. +3 ----
-  constexpr int KPW = 2;  // 1-KB pieces of a 16-KB K (or V) tile per wave
+  constexpr int KPW = 16 / NW;  // 1-KB pieces of a 16-KB K (or V) tile per wave
   const int* bt = block_tables + (int64_t)seq * bt_stride;
   const int64_t head_stride = (int64_t)block_size * D;
   int src_row[KPW], src_off[KPW];
@@ -335,7 +338,7 @@ __global__ void __launch_bounds__(512, 2) prefill_attn_v2_kernel(
     if (n_tiles > 0) issue(smem, 0);
     // static priority for the second-dispatched half (guide "Two waves per
     // SIMD" item 4): without it waves 4-7 lose every arbitration
-    if (V != 0 && wid >= 4) __builtin_amdgcn_s_setprio(1);
+    if (NW == 8 && V != 0 && wid >= 4) __builtin_amdgcn_s_setprio(1);
     __syncthreads();
     for (int t = 0; t < n_tiles; t += 2) {
       step(std::integral_constant<int, 0>{}, t);
@@ -397,23 +400,33 @@ extern "C" int dx_prefill_attention(void* out, const void* q, int64_t q_stride, 
   if (n_work == 0) return 0;
   const int bs_shift = __builtin_ctz((unsigned)block_size);
   if (block_size < 4 || (1 << bs_shift) != block_size) return -3;
-  dim3 grid(n_kv_heads * (G / hpw), n_work);
+  // Workgroups of eight waves stage every K/V tile once for all of them; of four, two to a CU, out of step with each other
+  // and with half as much work in the last and the longest of them.  32 / 8 heads, us, eight / four: one prompt of 2000 61.9 /
+  // 54.8 (256 workgroups of eight), six of 3000 together 32.2 / 29.7 (392), 300 rows behind 2900 cached 92.7 / 71.0 (40),
+  // two of 5000 136.3 / 138.2 (632), three of 6151 152.4 / 151.2 (776).
+  const bool four = (int64_t)n_kv_heads * (G / hpw) * n_work < 512;
+  const dim3 grid(n_kv_heads * (G / hpw), n_work * (four ? 2 : 1));
   const float sl2e = scale * 1.4426950408889634f;
   // n_waves 92 selects the pre-round-4 loop (A/B runs: tools/attn_ab.py,
   // tools/attn_accuracy.py)
   const bool r3 = n_waves == 92;
-#define DX_PA_LAUNCH(BS, VV)                                                                                         \
-  prefill_attn_v2_kernel<BS, true, VV><<<grid, 512, 0, stream>>>((bf16_t*)out, (const bf16_t*)q, q_stride,           \
-                                                                (const bf16_t*)k_cache, (const bf16_t*)v_cache,       \
-                                                                block_tables, bt_stride, cu_seqlens_q, ctx_lens, work, \
-                                                                n_q_heads, n_kv_heads, bs_shift, hpw, sl2e, causal)
+#define DX_PA_LAUNCH(BS, VV, NW)                                                                                     \
+  prefill_attn_v2_kernel<BS, true, VV, NW><<<grid, 64 * NW, 0, stream>>>(                                            \
+      (bf16_t*)out, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,        \
+      bt_stride, cu_seqlens_q, ctx_lens, work, n_q_heads, n_kv_heads, bs_shift, hpw, sl2e, causal)
+#define DX_PA(BS, VV)                   \
+  do {                                  \
+    if (four) DX_PA_LAUNCH(BS, VV, 4);  \
+    else DX_PA_LAUNCH(BS, VV, 8);       \
+  } while (0)
   if (block_size >= 64) {
-    if (r3) DX_PA_LAUNCH(true, 0);
-    else DX_PA_LAUNCH(true, 1);
+    if (r3) DX_PA(true, 0);
+    else DX_PA(true, 1);
   } else {
-    if (r3) DX_PA_LAUNCH(false, 0);
-    else DX_PA_LAUNCH(false, 1);
+    if (r3) DX_PA(false, 0);
+    else DX_PA(false, 1);
   }
+#undef DX_PA
 #undef DX_PA_LAUNCH
   return (int)hipGetLastError();
 }
