@@ -11,21 +11,49 @@
 // Router arithmetic (sigmoid, correction, group sums, comparisons) is fp32.
 // GEMMs take bf16 (v_mfma_f32_16x16x16_bf16) or fp32 (v_mfma_f32_16x16x4_f32,
 // true fp32 products) operands and accumulate in fp32.
+#include <type_traits>
+
 #include "../kernels/common.h"
 
 namespace {
 
 // (value, index) argmax over a wave; ties go to the lower index
 __device__ __forceinline__ void wave_argmax(float& v, int& i) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, 64);
-    const int oi = __shfl_xor(i, o, 64);
+  auto take = [&](float ov, int oi) {
     if (ov > v || (ov == v && oi < i)) {
       v = ov;
       i = oi;
     }
+  };
+  auto dpp = [&](auto ctrl) {
+    constexpr int C = decltype(ctrl)::value;
+    take(__int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), C, 0xf, 0xf, false)),
+         __builtin_amdgcn_update_dpp(0, i, C, 0xf, 0xf, false));
+  };
+  dpp(std::integral_constant<int, 0xB1>{});   // quad_perm [1, 0, 3, 2]
+  dpp(std::integral_constant<int, 0x4E>{});   // quad_perm [2, 3, 0, 1]
+  dpp(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  dpp(std::integral_constant<int, 0x140>{});  // row_mirror
+  // rows of 16, then halves, change places: one of the two results is the lane's own
+  auto swapped = [&](auto pv, auto pi) {
+    v = __uint_as_float(pv[0]), i = (int)pi[0];
+    take(__uint_as_float(pv[1]), (int)pi[1]);
+  };
+  {
+    const uint32_t u = __float_as_uint(v), j = (uint32_t)i;
+    swapped(__builtin_amdgcn_permlane16_swap(u, u, false, false), __builtin_amdgcn_permlane16_swap(j, j, false, false));
   }
+  {
+    const uint32_t u = __float_as_uint(v), j = (uint32_t)i;
+    swapped(__builtin_amdgcn_permlane32_swap(u, u, false, false), __builtin_amdgcn_permlane32_swap(j, j, false, false));
+  }
+}
+
+// what one wave wrote to LDS is there for its other lanes: LDS serves a wave's accesses in order, so only the compiler
+// has to keep it
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // Expert choice of one token by one wave.  c[e] = s[e] + corr[e] are the choice scores, s = sigmoid(z)
@@ -33,7 +61,7 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
 // largest group score (the sum of their two best choice scores, or with group_max their best)
 // compete; the `top` best are written with weight s (no correction), with renorm divided by the sum of
 // the chosen s (+ 1e-20), times scale.  zt [E] (global or LDS), c [E] and gs [n_groups] LDS of the wave.
-// Every wave of the workgroup calls this together (it holds barriers); `on`: the token exists.
+// `on`: the token exists.
 struct RouteArgs {
   const float* corr;
   int E, top, n_groups, keep, score, group_max, renorm;
@@ -54,7 +82,7 @@ __device__ __forceinline__ void route_token(const RouteArgs& g, const float* zt,
   }
   auto score = [&](int e) { return g.score == 1 ? expf(zt[e] - zmax) * zinv : 1.f / (1.f + expf(-zt[e])); };
   for (int e = lane; e < E; e += 64) c[e] = score(e) + (g.corr ? g.corr[e] : 0.f);
-  __syncthreads();
+  wave_sync();
   if (g.n_groups > 1) {
     const int per = E / g.n_groups;
     for (int q = lane; q < g.n_groups; q += 64) {
@@ -70,7 +98,7 @@ __device__ __forceinline__ void route_token(const RouteArgs& g, const float* zt,
       }
       gs[q] = per > 1 && !g.group_max ? a + b : a;
     }
-    __syncthreads();
+    wave_sync();
     for (int k = 0; k < g.keep; ++k) {  // kept groups are marked +inf
       float bv = -INFINITY;
       int bi = 0x7fffffff;
@@ -82,13 +110,13 @@ __device__ __forceinline__ void route_token(const RouteArgs& g, const float* zt,
         }
       }
       wave_argmax(bv, bi);
-      __syncthreads();
+      wave_sync();
       if (lane == 0 && bi < g.n_groups) gs[bi] = INFINITY;
-      __syncthreads();
+      wave_sync();
     }
     for (int e = lane; e < E; e += 64)
       if (gs[e / per] != INFINITY) c[e] = -INFINITY;
-    __syncthreads();
+    wave_sync();
   }
   float mine = 0.f, sum = 0.f;  // renorm: lane k's chosen score (top <= 64)
   for (int k = 0; k < g.top; ++k) {
@@ -103,7 +131,7 @@ __device__ __forceinline__ void route_token(const RouteArgs& g, const float* zt,
     }
     wave_argmax(bv, bi);
     if (bi >= E) bi = 0;  // nothing left to choose (rejected on the host)
-    __syncthreads();
+    wave_sync();
     if (lane == 0) c[bi] = -INFINITY;
     const float s = score(bi);
     if (g.renorm) {
@@ -114,7 +142,7 @@ __device__ __forceinline__ void route_token(const RouteArgs& g, const float* zt,
       idx[k] = bi;
       if (!g.renorm) w[k] = s * g.scale;
     }
-    __syncthreads();
+    wave_sync();
   }
   if (g.renorm && on && lane < g.top) w[lane] = mine / (sum + 1e-20f) * g.scale;
 }
@@ -134,16 +162,16 @@ __global__ void __launch_bounds__(64 * kRouteWaves) moe_route_kernel(int* __rest
 
 // The same result for few tokens: a workgroup per token whose waves share the width, kOut outputs at a time --
 // wide rows get many waves, so that a thread has one piece of the row and all its loads are in flight together.
-template <typename T, int V, int NW>
+// 24 tokens, 16 outputs, width 4096: 13.1 -> 6.8 us (before: sums by LDS permutes, the choice by all waves with barriers).
+template <typename T, int V, int NW, int kOut>
 __global__ void __launch_bounds__(64 * NW) moe_router_rows_kernel(int* __restrict__ idx, float* __restrict__ wgt,
                                                                   float* __restrict__ gates, const T* __restrict__ h,
                                                                   int64_t hs, const float* __restrict__ w, int n_out, int W,
                                                                   RouteArgs g) {
-  constexpr int kOut = 12;
   extern __shared__ float rsm[];
   float* part = rsm;              // [NW waves][n_out]
   float* z = part + NW * n_out;   // [n_out]
-  float* scratch = z + n_out;     // [NW][E + n_groups]
+  float* scratch = z + n_out;     // [E + n_groups]
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t t = blockIdx.x;
   const T* hp = h + t * hs;
@@ -181,11 +209,30 @@ __global__ void __launch_bounds__(64 * NW) moe_router_rows_kernel(int* __restric
 #pragma unroll
         for (int i = 0; i < V; ++i) acc[j] += x[i] * q[j][i];
     }
+    // sums over the lanes, half of the outputs changing hands with a lane of the other half: lane l ends with output
+    // l % kOut, of its 16 lanes, then of all.  (In registers: the LDS permutes of sixteen waves took 5 us.)
+    auto give_and_take = [&](auto ctrl, int n) {
+      constexpr int C = decltype(ctrl)::value;
 #pragma unroll
-    for (int j = 0; j < kOut; ++j) {
-      const float s = wave_reduce_sum(acc[j]);
-      if (lane == 0 && o0 + j < n_out) part[wv * n_out + o0 + j] = s;
-    }
+      for (int j = 0; j < n; ++j) {
+        const bool up = lane & n;
+        const float give = up ? acc[j] : acc[j + n], keep = up ? acc[j + n] : acc[j];
+        acc[j] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), C, 0xf, 0xf, false));
+      }
+    };
+    if constexpr (kOut == 16) give_and_take(std::integral_constant<int, 0x140>{}, 8);  // row_mirror: lane 15 - l
+    give_and_take(std::integral_constant<int, 0x141>{}, 4);                            // row_half_mirror: 7 - l
+    give_and_take(std::integral_constant<int, 0x4E>{}, 2);                             // quad_perm: l ^ 2
+    give_and_take(std::integral_constant<int, 0xB1>{}, 1);                             // l ^ 1
+    float sum = acc[0];
+    if constexpr (kOut == 8)  // the other eight lanes of the row hold the same outputs: l ^ 8
+      sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x128, 0xf, 0xf, false));
+    const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+    sum = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
+    const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+    sum = __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
+    acc[0] = sum;
+    if (lane < kOut && o0 + lane < n_out) part[wv * n_out + o0 + lane] = acc[0];
   }
   __syncthreads();
   for (int o = tid; o < n_out; o += 64 * NW) {
@@ -196,35 +243,101 @@ __global__ void __launch_bounds__(64 * NW) moe_router_rows_kernel(int* __restric
   }
   __syncthreads();
   for (int j = tid; j < n_out - g.E; j += 64 * NW) gates[t * (n_out - g.E) + j] = 1.f / (1.f + expf(-z[g.E + j]));
-  // (every wave takes part in the choice's barriers; wave 0 writes it)
-  float* c = scratch + wv * (g.E + g.n_groups);
-  route_token(g, z, c, c + g.E, wv == 0, idx + t * g.top, wgt + t * g.top, lane);
+  if (wv == 0) route_token(g, z, scratch, scratch + g.E, true, idx + t * g.top, wgt + t * g.top, lane);
 }
 
-// order [R]: slots sorted by expert, stable; offsets [E + 1].  One workgroup:
-// counts by LDS atomics (the counts do not depend on their order), a serial
-// scan over the experts, then every wave places the slots of its experts in
-// slot order with ballots.  Choices that are no expert (identity outputs, >= E)
-// get no place: order holds offsets[E] slots.  STAGE: the choices are first
-// copied into LDS as bytes (E <= 255, R <= kPlanStage), so the placement passes
-// read no global memory.
+// order [R]: slots sorted by expert, stable; offsets [E + 1].  Choices that are no expert (identity outputs, >= E) get no
+// place: order holds offsets[E] slots.
 constexpr int kPlanThreads = 1024;
-constexpr int kPlanStage = 48 * 1024;
-template <bool STAGE>
+constexpr int kPlanExperts = 256;  // up to here a counter per wave and expert fits
+
+// One workgroup whose waves own neighbouring runs of slots.  64 slots at a time a wave finds the lanes with the same
+// choice (a ballot per bit of the number), so a lane's rank among them and the run's counts need no atomics and no pass
+// per expert; the runs' counts are summed in order of the experts and waves, then every slot knows its place.
+// 5000 slots of 16 experts 15.0 -> 7.8 us (a pass over all slots per expert, counted by LDS atomics, before).
 __global__ void __launch_bounds__(kPlanThreads) moe_plan_kernel(int* __restrict__ order, int* __restrict__ offsets,
                                                                 const int* __restrict__ idx, int R, int E) {
+  constexpr int NW = kPlanThreads / 64, kAhead = 8;
+  extern __shared__ int ism[];
+  int* cnt = ism;            // [NW][E]
+  int* base = ism + NW * E;  // [E + 1]
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int bits = 32 - __builtin_clz(E), groups = (R + 63) / 64, per = (groups + NW - 1) / NW;
+  const int g0 = min(wv * per, groups), g1 = min(g0 + per, groups);
+  for (int i = tid; i < NW * E; i += kPlanThreads) cnt[i] = 0;
+  __syncthreads();
+  int* mine = cnt + wv * E;
+  const unsigned long long before = (1ull << lane) - 1ull;
+  auto walk = [&](auto&& put) {
+    for (int c = g0; c < g1; c += kAhead) {
+      int v[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int r = (c + k) * 64 + lane;
+        v[k] = c + k < g1 && r < R ? idx[r] : E;
+      }
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        if (c + k >= g1) break;
+        const int e = v[k] >= 0 && v[k] < E ? v[k] : E;
+        unsigned long long same = ~0ull;
+        for (int b = 0; b < bits; ++b) {
+          const unsigned long long m = __builtin_amdgcn_ballot_w64((e >> b) & 1);
+          same &= (e >> b) & 1 ? m : ~m;
+        }
+        if (e < E) put((c + k) * 64 + lane, e, (int)__builtin_popcountll(same & before));
+        wave_sync();
+        if (e < E && !(same & before)) mine[e] += (int)__builtin_popcountll(same);
+        wave_sync();
+      }
+    }
+  };
+  walk([](int, int, int) {});
+  __syncthreads();
+  for (int e = tid; e < E; e += kPlanThreads) {
+    int sum = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const int n = cnt[w * E + e];
+      cnt[w * E + e] = sum;
+      sum += n;
+    }
+    base[e] = sum;
+  }
+  __syncthreads();
+  if (wv == 0) {  // exclusive sums over the experts
+    int at = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int n = e0 + lane < E ? base[e0 + lane] : 0;
+      int x = n;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+      }
+      if (e0 + lane < E) base[e0 + lane] = at + x - n;
+      at += __shfl(x, 63, 64);
+    }
+    if (lane == 0) base[E] = at;
+  }
+  __syncthreads();
+  for (int e = tid; e <= E; e += kPlanThreads) offsets[e] = base[e];
+  walk([&](int r, int e, int rank) { order[base[e] + mine[e] + rank] = r; });
+}
+
+// More experts: counts by LDS atomics (they do not depend on their order), a serial scan over the experts, then every
+// wave places the slots of its experts in slot order with ballots.
+__global__ void __launch_bounds__(kPlanThreads) moe_plan_many_kernel(int* __restrict__ order, int* __restrict__ offsets,
+                                                                     const int* __restrict__ idx, int R, int E) {
   extern __shared__ int ism[];
   int* cnt = ism;
   int* base = ism + E;
-  unsigned char* mine = reinterpret_cast<unsigned char*>(ism + 2 * E + 1);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   for (int e = tid; e < E; e += kPlanThreads) cnt[e] = 0;
   __syncthreads();
   for (int r = tid; r < R; r += kPlanThreads) {
     const int e = idx[r];
-    const bool ok = e >= 0 && e < E;
-    if (ok) atomicAdd(&cnt[e], 1);
-    if constexpr (STAGE) mine[r] = ok ? (unsigned char)e : 255;
+    if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
   if (tid == 0) {
@@ -241,9 +354,7 @@ __global__ void __launch_bounds__(kPlanThreads) moe_plan_kernel(int* __restrict_
     int at = base[e];
     for (int r0 = 0; r0 < R; r0 += 64) {
       const int r = r0 + lane;
-      bool hit;
-      if constexpr (STAGE) hit = r < R && mine[r] == e;
-      else hit = r < R && idx[r] == e;
+      const bool hit = r < R && idx[r] == e;
       const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
       if (hit) order[at + __builtin_popcountll(m & ((1ull << lane) - 1ull))] = r;
       at += __builtin_popcountll(m);
@@ -324,7 +435,8 @@ template <typename T> struct Oct {
 // then n_out - E rows of gates), true fp32 products of h as it is and w on the fp32 matrix cores
 // (v_mfma_f32_16x16x4_f32), then the choice of every token (route_token); gates[t, j] = sigmoid(z[t, E + j]).
 // A workgroup takes 16 tokens; its NW waves share the width in pieces of 32, 32 outputs per pass, and their partial
-// sums are added in LDS in wave order.
+// sums are added in LDS in wave order.  2500 tokens, 16 outputs, width 4096: 28.6 -> 17 us (pieces one after the other,
+// eight waves, products for 32 outputs); 3.4 of them the matrix instructions of 157 workgroups, the rest latency.
 template <typename T, int NW>
 __global__ void __launch_bounds__(64 * NW) moe_router_kernel(int* __restrict__ idx, float* __restrict__ wgt,
                                                              float* __restrict__ gates, const T* __restrict__ h,
@@ -351,18 +463,30 @@ __global__ void __launch_bounds__(64 * NW) moe_router_kernel(int* __restrict__ i
       on[i] = o0 + 16 * i + c16 < n_out;
       wp[i] = w + (int64_t)(on[i] ? o0 + 16 * i + c16 : 0) * W;
     }
-    for (int k0 = wv * 32 + 8 * g4; k0 - 8 * g4 < W; k0 += NW * 32) {
-      Oct<T> a;
-      Oct<float> b[2];
+    const bool both = o0 + 16 < n_out;
+    const int base = wv * 32 + 8 * g4;
+    auto load = [&](int k0, Oct<T>& a, Oct<float>(&b)[2]) {
       a.load(hp + k0, W - k0, row_on);
       b[0].load(wp[0] + k0, W - k0, on[0]);
-      b[1].load(wp[1] + k0, W - k0, on[1]);
+      if (both) b[1].load(wp[1] + k0, W - k0, on[1]);
+    };
+    auto mma = [&](const Oct<T>& a, const Oct<float>(&b)[2]) {
 #pragma unroll
       for (int s = 0; s < 8; ++s) {  // the four lane groups supply k = 8 g4 + s
         const float x = f(a.v[s]);
         C[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[0].v[s], x, C[0], 0, 0, 0);
-        C[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[1].v[s], x, C[1], 0, 0, 0);
+        if (both) C[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[1].v[s], x, C[1], 0, 0, 0);
       }
+    };
+    // four pieces on their way at once (past the width nothing is read)
+    constexpr int kAhead = 4;
+    for (int k0 = base; k0 - 8 * g4 < W; k0 += kAhead * NW * 32) {
+      Oct<T> a[kAhead];
+      Oct<float> b[kAhead][2];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) load(k0 + k * NW * 32, a[k], b[k]);
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) mma(a[k], b[k]);
     }
     __syncthreads();  // (the previous pass's sums are read)
     // C[i]: outputs o0 + 16 i + 4 g4 + r of row c16
@@ -566,11 +690,15 @@ int dxm_moe_router(int* idx, float* w, float* gates, const void* h, int64_t h_st
   const int esz = f32 ? 4 : 2;
   if (T <= 256) {
     const bool vec = W % 4 == 0 && h_stride % 4 == 0 && (uintptr_t)h % (4 * esz) == 0 && (uintptr_t)rw % 16 == 0;
-    auto lds = [&](int nw) { return ((nw + 1) * (size_t)n_out + nw * (size_t)(E + n_groups)) * sizeof(float); };
+    auto lds = [&](int nw) { return ((nw + 1) * (size_t)n_out + (size_t)(E + n_groups)) * sizeof(float); };
     const bool wide = vec && W >= 2048 && lds(16) <= 60 * 1024;
 #define ROUTER_ROWS(TY, V, NW)                                                                                        \
-  hipLaunchKernelGGL((moe_router_rows_kernel<TY, V, NW>), dim3(T), dim3(64 * NW), lds(NW), st, idx, w, gates,          \
-                     (const TY*)h, h_stride, rw, n_out, W, g);
+  if (n_out <= 8)                                                                                                     \
+    hipLaunchKernelGGL((moe_router_rows_kernel<TY, V, NW, 8>), dim3(T), dim3(64 * NW), lds(NW), st, idx, w, gates,     \
+                       (const TY*)h, h_stride, rw, n_out, W, g);                                                      \
+  else                                                                                                                \
+    hipLaunchKernelGGL((moe_router_rows_kernel<TY, V, NW, 16>), dim3(T), dim3(64 * NW), lds(NW), st, idx, w, gates,    \
+                       (const TY*)h, h_stride, rw, n_out, W, g);
     if (f32 && wide) { ROUTER_ROWS(float, 4, 16) }
     else if (f32 && vec) { ROUTER_ROWS(float, 4, 4) }
     else if (f32) { ROUTER_ROWS(float, 1, 4) }
@@ -582,8 +710,8 @@ int dxm_moe_router(int* idx, float* w, float* gates, const void* h, int64_t h_st
     return 0;
   }
   const dim3 grid((unsigned)((T + 15) / 16));
-  // few tokens: more waves share the width
-  const bool many = T <= 1024 && router_lds(16, n_out, E, n_groups) <= 60 * 1024;
+  // up to a workgroup per CU: more waves share the width
+  const bool many = T <= 4096 && router_lds(16, n_out, E, n_groups) <= 60 * 1024;
 #define ROUTER(TY, NW)                                                                                               \
   hipLaunchKernelGGL((moe_router_kernel<TY, NW>), grid, dim3(64 * NW), router_lds(NW, n_out, E, n_groups), st, idx, w, \
                      gates, (const TY*)h, h_stride, rw, n_out, T, W, g);
@@ -600,10 +728,11 @@ int dxm_moe_plan(int* order, int* offsets, const int* idx, int R, int E, hipStre
   if (E < 1 || R < 0) return 1;
   const size_t lds = (size_t)(2 * E + 1) * sizeof(int);
   if (lds > 12 * 1024) return 2;
-  if (E <= 255 && R <= kPlanStage)
-    hipLaunchKernelGGL(moe_plan_kernel<true>, dim3(1), dim3(kPlanThreads), lds + R, st, order, offsets, idx, R, E);
+  if (E <= kPlanExperts)
+    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(kPlanThreads), ((kPlanThreads / 64 + 1) * (size_t)E + 1) * sizeof(int), st,
+                       order, offsets, idx, R, E);
   else
-    hipLaunchKernelGGL(moe_plan_kernel<false>, dim3(1), dim3(kPlanThreads), lds, st, order, offsets, idx, R, E);
+    hipLaunchKernelGGL(moe_plan_many_kernel, dim3(1), dim3(kPlanThreads), lds, st, order, offsets, idx, R, E);
   DX_CHECK_LAUNCH();
   return 0;
 }
