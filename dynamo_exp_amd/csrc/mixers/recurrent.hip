@@ -2,7 +2,8 @@
 // running matrix per head), short causal convolutions over time (bias and
 // activation optional) fused with rotary positions and the paged cache write,
 // the convolution tail update, and the norms + gates that follow a recurrent
-// mixer.  (Linear recurrences without a removal term: linear_scan.hip.)
+// mixer.  (Linear recurrences without a removal term: linear_scan.hip; the delta
+// rule over bf16 prompt rows of 128-channel keys in chunks: delta_chunk.hip.)
 //
 // State lives in slots ([slots, ...] tensors); a step names the slot of each of
 // its sequences (state_slots [n_seq], -1: a padding row that touches nothing)

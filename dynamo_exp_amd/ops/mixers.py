@@ -32,7 +32,8 @@ MAX_STREAMS = 8
 # into parts shorter than ROW_MIN_PART
 ROW_TARGET_WAVES = 2048
 ROW_MIN_PART = 128
-# grouped decode kernel: one wave per workgroup, four workgroups resident per CU (LDS), so
+# grouped decode kernel (other widths than decode_attention.hip takes, which cuts parts by
+# a rule of its own): one wave per workgroup, four workgroups resident per CU (LDS), so
 # about 1024 waves fill the chip once; more parts only add merge work
 GROUP_TARGET_WAVES = 1024
 # latent decode kernel: two workgroups of four waves per CU (LDS)
