@@ -19,8 +19,8 @@
 // Its rounding: the products of decays come from sums of logarithms in fp64, the sums run in an order that keeps them
 // small and through short chains; relative to 64 bits 1.28e-7 in o and 6.90e-8 in S where the token-by-token form has
 // 1.32e-7 and 6.91e-8 (900 to 4001 tokens; 1.9e-7 and 1.2e-7 with running products and one chain per sum).
-// A value that is not finite makes its own and the later tokens' results not finite, as token by token; zero factors
-// times it do the same to the rows in front of it in its chunk.
+// A value that is not finite would reach the rows in front of it in its chunk (zero factors times it).  It also stays in
+// the state, so a workgroup that ends with such a state takes its columns again, token by token.
 // 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us; a
 // prompt of 600 beside 30 single tokens 1265 -> 110.  Bound by the fp32 matrix instructions (200 us of them run) beside
 // the fragments' way through L2.
@@ -240,6 +240,7 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
 }
 
 struct ChunkArgs {
+  FormArgs f;    // the rows themselves (in_order)
   float* out;    // [T, H * dv]
   float* state;  // [slots, H, dv, 128]
   const float* ws;
@@ -256,6 +257,53 @@ template <int NB> struct Frags {
   float g, h;
   uint32_t v[NB][4];  // rows g4, 4 + g4, 8 + g4 and 12 + g4 of V; bf16 bits as loaded: a conversion here would wait for the load
 };
+
+// NB blocks of 16 columns of a sequence of n rows, token by token and in plain loops: for values that are not finite.
+template <int NB>
+__device__ __forceinline__ void in_order(const ChunkArgs& g, float* row /* [5][128] LDS */, float* red /* [4] LDS */, int r0,
+                                                   int n, int h, int slot, int col0) {
+  constexpr int TPC = 256 / (16 * NB), CH = kD / TPC;  // threads per column, channels of each
+  const FormArgs& f = g.f;
+  const int tid = threadIdx.x, c = tid / TPC, part = tid % TPC;
+  float* sp = g.state + ((int64_t)slot * g.H * g.dv + col0 + c) * kD + part * CH;
+  float S[CH];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) S[i] = g.pos[r0] != 0 ? sp[i] : 0.f;
+  for (int t = r0; t < r0 + n; ++t) {
+    __syncthreads();
+    const int ch = tid & (kD - 1), at = h * kD + ch;
+    const float kk = bf16_to_f32(f.k[t * f.ks + at]);
+    const float ss = wave_reduce_sum(tid < kD ? kk * kk : 0.f);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    if (tid < kD) {
+      const float u = kk * rsqrtf(red[0] + red[1] + f.key_eps);
+      row[ch] = u;
+      row[kD + ch] = sigmoid1(bf16_to_f32(f.a[t * f.as + at]) + (f.a_bias ? f.a_bias[at] : 0.f)) * u;
+      row[2 * kD + ch] = expf(-f.decay_scale * sigmoid1(bf16_to_f32(f.w[t * f.wst + at]) + (f.w_bias ? f.w_bias[at] : 0.f)));
+      row[3 * kD + ch] = kk;
+      row[4 * kD + ch] = bf16_to_f32(f.r[t * f.rs + at]);
+    }
+    __syncthreads();
+    const float v = bf16_to_f32(g.v[t * g.vs + col0 + c]);
+    const float* p = row + part * CH;
+    float x = 0.f, o = 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) x += p[i] * S[i];
+#pragma unroll
+    for (int m = 1; m < TPC; m <<= 1) x += __shfl_xor(x, m, 64);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      S[i] = p[2 * kD + i] * S[i] - p[kD + i] * x + p[3 * kD + i] * v;
+      o += p[4 * kD + i] * S[i];
+    }
+#pragma unroll
+    for (int m = 1; m < TPC; m <<= 1) o += __shfl_xor(o, m, 64);
+    if (part == 0) g.out[(int64_t)t * g.H * g.dv + col0 + c] = o;
+  }
+#pragma unroll
+  for (int i = 0; i < CH; ++i) sp[i] = S[i];
+}
 
 // The k-th longest of up to 64 sequences (more of them even out by themselves): the workgroups go out in this order, so
 // that the longest does not start when a short one's place is free.
@@ -414,6 +462,17 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
     step(f0, c, f1, c + 1);
     if (c + 1 < nc) step(f1, c + 1, f0, c + 2);
   }
+  bool finite = true;
+#pragma unroll
+  for (int q = 0; q < NB; ++q)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) finite = finite && fabsf(S[q][cb][i]) < INFINITY;
+  if (__syncthreads_or(!finite)) {  // (also waits for the rows stored above)
+    in_order<NB>(g, &po[0][0][0][0][0], reinterpret_cast<float*>(&px[0][0][0][0]), r0, n, h, slot, col0);
+    return;
+  }
 #pragma unroll
   for (int q = 0; q < NB; ++q)
 #pragma unroll
@@ -451,7 +510,7 @@ int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void
   FormArgs f{ws, (const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)a, (const bf16_t*)w, rs, ks, as, wst, a_bias, w_bias,
              seq_rows, slots, decay_scale, key_eps, n_seq, n_slots, T_, H};
   hipLaunchKernelGGL(delta_form_kernel, dim3(H, T_ / kC + n_seq), dim3(256), 0, st, f);
-  ChunkArgs c{out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
+  ChunkArgs c{f, out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
   const int64_t heads = ((int64_t)n_seq * H + 7) / 8 * 8;
   // Two column blocks a workgroup read a chunk once for both, but only two of their workgroups fit a CU; one block keeps
   // more of the chip busy until there are twice as many workgroups as fit.  Whole layer, 32 heads, us, one / two blocks:

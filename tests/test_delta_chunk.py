@@ -78,6 +78,40 @@ def test_delta_chunks(rows, kind, H, dv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dv,n_seq", [(32, 2), (16, 1), (32, 40)])  # (one column block per workgroup, and two)
+@pytest.mark.parametrize("what", ["k", "v", "a", "w", "r", "state"])
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+def test_values_that_are_not_finite(dv, n_seq, what, bad):
+    """They reach what they reach token by token: their own and later rows (of a value: its column), the state, no row in
+    front of them, no other head or sequence."""
+    torch.manual_seed(3)
+    H, rows, at = 16, 70, 37
+    n, T = H * 128, 70 * n_seq
+    p, wl = torch.randn(T, 3 * n + H * dv).bfloat16(), (torch.randn(T, n) * 0.5).bfloat16()
+    state0 = torch.randn(n_seq, H, dv, 128)
+    first = {"r": 0, "k": n, "a": 2 * n, "v": 3 * n}
+    if what == "w":
+        wl[at, 130] = bad
+    elif what == "state":
+        state0[0, 1, 3, 5] = bad
+    else:
+        p[at, first[what] + (dv if what == "v" else 128) + 2] = bad  # head 1
+    ab, wb = torch.randn(n) * 0.5, torch.randn(n)
+    pos = torch.arange(5, 5 + rows).repeat(n_seq)
+    starts = (torch.arange(n_seq + 1) * rows).to(torch.int32)
+    res = []
+    for dt in (torch.bfloat16, torch.float32):  # float32 copies run token by token
+        q, w, state = p.cuda().to(dt), wl.cuda().to(dt), state0.cuda()
+        out = rc.delta_rule(q[:, :n], q[:, n:2 * n], q[:, 3 * n:], q[:, 2 * n:3 * n], w, ab.cuda(), wb.cuda(), state, pos.cuda(),
+                            starts.cuda(), torch.arange(n_seq, dtype=torch.int32).cuda(), H, 128, dv)
+        res.append((out.cpu(), state.cpu()))
+    for got, want in zip(*res):
+        ok = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), ok)
+        assert float((got[ok] - want[ok]).abs().max()) < 1e-5 * float(want[ok].abs().max())
+
+
+@pytest.mark.gpu
 def test_delta_chunk_rule():
     """Which rows take the chunks: bf16 prompt rows, keys of 128, whole blocks of values, a bounded decay, alignment."""
     ok = rc._m().delta_chunk_floats
