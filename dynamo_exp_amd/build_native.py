@@ -1,7 +1,7 @@
 """In-tree native build for dynamo_exp_amd.
 
 Two extension modules are produced next to the Python sources (so they travel
-with a ``gpurun`` snapshot and are visible to the round-end loader audit):
+with the tree to a machine that only runs them):
 
 * ``dynamo_exp_amd/_C_kernels*.so`` -- hand-written HIP kernels for gfx950
   (RMSNorm, RoPE + paged-KV write, SiLU-gate, embedding, paged attention
@@ -86,7 +86,7 @@ HIP_FLAGS = ["-x", "hip", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32
 def verify_kernels(names: list[str] | None = None, jobs: int = 8) -> dict[str, str]:
     """Compile the device side of the HIP kernel sources with LLVM's machine
     verifier (``-mllvm -verify-machineinstrs``) and return {file: error} for
-    the ones it rejects.  Round 5 met a ROCm 7.2 sub-register liveness
+    the ones it rejects.  ROCm 7.2 had a sub-register liveness
     miscompile in attn_decode.hip ("No live subrange at use": V-row registers
     reused as temporaries, wrong output in the G = 1 instance only) that the
     verifier reports at compile time; the normal build does not run it."""

@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_kernel(
   // as 4 x u32 structs, the masking branch's per-dword writes hit an LLVM
   // sub-register liveness bug (gfx950, ROCm 7.2: "No live subrange at use"
   // under -verify-machineinstrs) that reused V registers as temporaries in the
-  // G = 1 instance: half of each V vector read back as garbage (round-5 GPU
+  // G = 1 instance: half of each V vector read back as garbage (a GPU
   // dump: profiles/r5_decode_g1_miscompile.txt).  tests/test_build.py runs the
   // machine verifier over the kernel sources.
   u32x4_t kA[C::TPL][C::VPL] = {}, vA[C::TPL][C::VPL] = {};
@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_kernel(
   }
 
   // ---- merge the TPW lane groups of each wave in registers (cross-group
-  // shuffles), then the 4 waves' states through LDS.  (Round 5: merging all
+  // shuffles), then the 4 waves' states through LDS.  (Merging all
   // 4 * TPW group states through LDS took 64 KiB at G = 8 -- two workgroups
   // per CU -- and 16 LDS passes per output, a fixed per-workgroup cost that
   // short partitions, e.g. one Llama-3-70B TP4 rank's 2 KV heads, could not
@@ -773,7 +773,7 @@ extern "C" int dx_decode_attention(void* out, float* tmp_out, float* tmp_ml, con
   // K scale folds into the softmax scale, the V scale into the output; fp8
   // chunk: 16 tokens with two chunks in flight per wave (164 VGPRs, 3
   // waves/SIMD at G 4; a 32-token variant measured no better,
-  // profiles/r3_kv_fp8.txt, and was removed in round 4)
+  // profiles/r3_kv_fp8.txt, and was removed)
 #define DX_DEC(GG, LL, L8)                                                                                         \
   return kv_fp8 ? launch<GG, L8, 16, true, true>(o, tmp_out, tmp_ml, qq, q_stride, k_cache, v_cache, block_tables, \
                                                  bt_stride, ctx_lens, batch, n_kv_heads, block_size, n_parts,      \

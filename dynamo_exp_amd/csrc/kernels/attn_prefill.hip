@@ -91,7 +91,7 @@ __device__ __forceinline__ float halves_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// V: 0 = the round-3 loop (kept for A/B), 1 = round 4: deferred rescale, row
+// V: 0 = the first loop (kept for A/B), 1 = deferred rescale, row
 // sum on the matrix pipe, v_max3 row max, static priority, widened epilogue.
 // (Ping-pong wave halves, two tiles per barrier and a software-pipelined QK /
 // softmax measured slower, as did 4-wave workgroups where there are enough of
@@ -407,7 +407,7 @@ extern "C" int dx_prefill_attention(void* out, const void* q, int64_t q_stride, 
   const bool four = (int64_t)n_kv_heads * (G / hpw) * n_work < 512;
   const dim3 grid(n_kv_heads * (G / hpw), n_work * (four ? 2 : 1));
   const float sl2e = scale * 1.4426950408889634f;
-  // n_waves 92 selects the pre-round-4 loop (A/B runs: tools/attn_ab.py,
+  // n_waves 92 selects the first loop (A/B runs: tools/attn_ab.py,
   // tools/attn_accuracy.py)
   const bool r3 = n_waves == 92;
 #define DX_PA_LAUNCH(BS, VV, NW)                                                                                     \

@@ -8,7 +8,7 @@
 //               separate silu_and_mul launch disappears.
 //   EPI_ADD:    y[M, N]  += x[M, K] . w[N, K]^T, for a residual stream behind a
 //               long sum (the MLP's down projection)
-// bf16 in / out, fp32 accumulation (SURVEY §2.15 "SiLU-gated MLP").
+// bf16 in / out, fp32 accumulation.
 //
 // Design (CDNA4 guide §5 "256² 8-phase template", re-derived here):
 //   * 256 x 256 output tile per workgroup, K in 64-deep tiles, 8 waves as

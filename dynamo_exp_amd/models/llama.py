@@ -13,8 +13,7 @@ Forward pass per layer (T tokens, all bf16; one fused op per line):
 
 Tensor parallelism is Megatron style (column-parallel QKV / gate-up, row-
 parallel O / down, vocab-parallel LM head), one process per GPU.  The
-reference delegates all of this to vLLM (`lib/engines/vllm0_8/src/lib.rs:371`);
-see SURVEY.md §2.15 for the kernel inventory.
+reference delegates all of this to vLLM (`lib/engines/vllm0_8/src/lib.rs:371`).
 """
 from __future__ import annotations
 
@@ -731,7 +730,7 @@ class LlamaForCausalLM:
                 if best is not None:
                     row["best_us"], row["cfg"] = round(best[0], 2), best[1]
                     if best[0] < lib * (1 - min_gain):
-                        # numerics on the first and the last layer's weights (ADVICE r5: not layer 0 alone)
+                        # numerics on the first and the last layer's weights (not layer 0 alone)
                         for w in (ws[0], ws[-1]):
                             want = torch.matmul(x, w.t()).float()
                             got = ops.skinny_linear(x, w, best[1]).float()

@@ -46,9 +46,9 @@ __all__ = [
 
 # decode attention partitioning (decode_num_parts): aim for this many
 # workgroups per launch, never split a context into parts shorter than
-# DECODE_MIN_PART tokens.  512 since the round-5 in-wave merge cut the
+# DECODE_MIN_PART tokens.  512 since the in-wave merge cut the
 # per-workgroup epilogue: best or within 3 % of best at every batch / context /
-# head layout swept (profiles/r5_decode_wgs_sweep.txt; 2048 was the round-1
+# head layout swept (profiles/r5_decode_wgs_sweep.txt; 2048 was the first
 # optimum with the 64-state LDS merge)
 DECODE_TARGET_WGS = int(os.environ.get("DX_DECODE_WGS", "512"))
 DECODE_MIN_PART = int(os.environ.get("DX_DECODE_MIN_PART", "256"))
@@ -527,7 +527,7 @@ def quant_rows(x: torch.Tensor):
 def fp8_linear(x8: torch.Tensor, sx: torch.Tensor, w8: torch.Tensor, sw: torch.Tensor) -> torch.Tensor:
     """(x8 * sx) @ (w8 * sw)^T -> bf16 (row-wise token scales x column-wise
     channel scales; w8: [N, K] e4m3, sw: [1, N]) through hipBLASLt's fp8
-    kernels (round 5's fp8 deep-stream form was removed: its first launch
+    kernels (an fp8 deep-stream form was removed: its first launch
     faulted, cause unknown -- profiles/r5_dstream_fp8_fault.txt)."""
     if not x8.is_cuda:
         return ref.fp8_linear(x8, sx, w8, sw)
@@ -554,7 +554,7 @@ def decode_num_parts(batch: int, n_kv_heads: int, max_ctx: int) -> int:
     actual context into that many equal parts itself).  Few, long-lived
     workgroups stream HBM best (profiles/r1_decode_parts.json: balanced parts
     6.0-6.4 TB/s vs 5.0-5.8 with fixed 512-token parts; target workgroup
-    count re-swept in round 5, profiles/r5_decode_wgs_sweep.txt); small
+    count re-swept: profiles/r5_decode_wgs_sweep.txt); small
     batches get more parts so the grid still covers the 256 CUs."""
     want = -(-DECODE_TARGET_WGS // max(1, batch * n_kv_heads))
     cap = -(-max(1, max_ctx) // DECODE_MIN_PART)
@@ -662,7 +662,7 @@ def kv_dequant_scratch(k_cache, v_cache, block_tables, ctx_lens, kv_scales=(1.0,
     the prefill attention kernel, which then reads bf16 tiles unchanged.
     `scratch` = (device int32 table [nseq, max_blocks], n_blocks) from
     :func:`fp8_scratch_plan` (the model runner's packed, capped layout:
-    sum of ceil(ctx / block_size) blocks: never
+    sum of ceil(ctx / block_size) blocks -- never
     nseq x padded max_blocks); without it (direct calls in tests) the
     dense table i * max_blocks + j."""
     nseq, maxb = block_tables.shape
