@@ -23,7 +23,7 @@
 // score with cap and penalty).  Against the register-staged, 16x16x32 forms it took over from (tile_attention.hip,
 // stream and latent prefill), 32 heads, ragged prompts of about 4000 tokens, us: before -> with eight waves -> now: two
 // maps with values of 256 and their combine, window 1024 + 64: 776 -> 303 -> 267; shared row 256 / 192 causal 242 ->
-// 140 -> 124 (800 TFLOP/s), 256 / 256 window 546 -> 124 -> 123; cap + penalty, window 1024: 313 -> 176 -> 136; sigmoid
+// 140 -> 124 (800 TFLOP/s), 256 / 256 window 546 -> 124 -> 123; cap + penalty, window 1024: 313 -> 176 -> 138; sigmoid
 // 213 -> 92 -> 86; plain causal, 5000 tokens: 132 -> 124 -> 111, fine 160 -> 148 -> 133; 40 rows behind 2900 cached:
 // 131 -> 117 -> 93.
 #include <type_traits>
@@ -195,12 +195,13 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
         for (int sub = 0; sub < SUBS; ++sub) s[sub] *= a.scale * kLog2e;
       }
       if (a.r1) {  // (keys behind the row: their argument may be anything, they are masked below)
-        const float t0 = fmaf(r2, (float)(my - kt - 4 * h), 1.f);
+        // the distance first, which is exact: r2 times the lane's distance less r2 times the key's place would cancel
+        const float d0 = (float)(my - kt - 4 * h);
 #pragma unroll
         for (int sub = 0; sub < SUBS; ++sub)
 #pragma unroll
           for (int i = 0; i < 16; ++i)
-            s[sub][i] = fmaf(-r1, __builtin_amdgcn_logf(fmaf(-r2, (float)(32 * sub + (i & 3) + 8 * (i >> 2)), t0)), s[sub][i]);
+            s[sub][i] = fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, d0 - (float)(32 * sub + (i & 3) + 8 * (i >> 2)), 1.f)), s[sub][i]);
       }
     }
     if (kt + KT - 1 > wlo || (kt < wlast && !kept_tile)) {  // some key is not seen by some row

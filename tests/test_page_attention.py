@@ -153,3 +153,32 @@ def test_decode_rows(form, mask, size, keep):
         # fp32: weights as two bf16 numbers, 2^-17 of sum w |v|; bf16: one rounding of the result on top
         top = float(want.abs().max())
         assert err < (3e-4 if not sig else 3e-4 * max(top, 1.0)) + (0.0 if out_f32 else 2.0 ** -8 * top), (bs, parts, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rate", [0.1, 1.0, 100.0, 1e4, 6.3e5, 1e7, 1e12])
+@pytest.mark.parametrize("form", ["penalty", "both"])
+def test_penalty_of_any_rate(form, rate):
+    """The log-distance penalty from slow rates to ones whose product with a distance leaves no bit of the 1 beside it,
+    where a row's own key (distance 0) still pays nothing: prompt rows at every place of a key tile and a decode row."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(17)
+    scale, starts, rows = 0.7 * d ** -0.5, [43, 0, 199], [70, 97, 1]
+    cap = terms(form, n_qh)[0]
+    db = (torch.rand(n_qh) + 0.2, rate * (torch.rand(n_qh) + 0.5))
+    kd, vd, table, kv = pages(form, [s + r for s, r in zip(starts, rows)], 64)
+    q, T, Tp = torch.randn(sum(rows), n_qh * d).bfloat16(), sum(rows), sum(rows[:2])
+    want = []
+    for i, (s, r) in enumerate(zip(starts, rows)):
+        r0 = sum(rows[:i])
+        want.append(dense(q[r0:r0 + r].double().reshape(r, n_qh, d), *kv[i], torch.arange(s, s + r), scale, "window", 100, 0,
+                          cap, db, None, False, None))
+    want = torch.cat(want)
+    pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)]).cuda()
+    seq = torch.tensor([i for i, r in enumerate(rows) for _ in range(r)], dtype=torch.int32).cuda()
+    tiles = torch.tensor([t for i in range(2) for t in mx.tile_list(sum(rows[:i]), rows[i])], dtype=torch.int32).cuda()
+    got = mx.attention(q.cuda(), kd, vd, pos, seq, table, 64, n_qh, maps, group, d, dv, scale, "window", 100, 3, False, tiles, Tp,
+                       softcap=cap, dist_bias=tuple(map(cuda, db))).cpu().double()
+    # as test_prompt_rows: the result's rounding to bf16 and one rounding of every weight
+    err, top = float((got - want).abs().max()), float(want.abs().max())
+    assert err < 2.0 ** -8 * (top + 5.0), err
