@@ -9,10 +9,11 @@
 //     X = U' S + G V       U' = (I + tril(U B^T, -1))^-1 U,        G = (I + tril(U B^T, -1))^-1 tril(U K^T, -1)
 //     O = R' S + H V       R' = R - tril(R B^T) U',                H = tril(R K^T) - tril(R B^T) G
 //     S <- diag(P_16) S + K''^T V - B''^T X                        K'' = K P_16, B'' = B P_16
-// delta_form_kernel makes U', R', K'', B'', G, H and P_16 of every (chunk, head) -- no chunk needs another's -- and
-// delta_chunk_kernel runs the chunks of a sequence in order: per (sequence, head, 16 columns of S) four waves that
+// delta_form_kernel makes U', R', K'', B'', G, H and P_16 of every (chunk, head) of the sequences long enough (kLong) -- no
+// chunk needs another's -- and delta_chunk_kernel runs the chunks of a sequence in order: per (sequence, head, 16 columns of S) four waves that
 // own 32 channels each, S in their accumulators.  A wave's accumulators are the second operand of its part of U' S and
-// R' S as they lie; the parts of X and O join in LDS, one barrier a chunk.
+// R' S as they lie; the parts of X and O join in LDS, one barrier a chunk.  The other sequences run in the same launch,
+// token by token, beside the long ones' chains.
 //
 // P_t shrinks by at most exp(-16 |decay_scale|) in a chunk, so 1 / P stays far inside fp32 (the host refuses more
 // than 4).  A chunk's dependent chain is 50 matrix instructions and a barrier instead of 16 tokens' chains of lane sums.
@@ -21,14 +22,21 @@
 // 1.32e-7 and 6.91e-8 (900 to 4001 tokens; 1.9e-7 and 1.2e-7 with running products and one chain per sum).
 // A value that is not finite would reach the rows in front of it in its chunk (zero factors times it).  It also stays in
 // the state, so a workgroup that ends with such a state takes its columns again, token by token.
-// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us; a
-// prompt of 600 beside 30 single tokens 1265 -> 110.  Bound by the fp32 matrix instructions (200 us of them run) beside
-// the fragments' way through L2.
-#include "recurrent.h"
+// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us, each
+// profiled by itself (in a row, with the layer's norm of 35: 443); a prompt of 600 beside 30 single tokens 704 -> 112, the
+// layer without its norm.  Bound by the fp32 matrix instructions (200 us of them run) beside the fragments' way through L2.
+#include <algorithm>
+
+#include "delta_tokens.h"
 
 namespace {
 
 constexpr int kC = 16;    // tokens per chunk
+// A sequence with at least this many rows in the step goes in chunks, a shorter one (a decode row beside a prompt among
+// them) token by token, whatever else is in the step: what shares a step does not change a sequence's arithmetic.
+// From 32 rows on the chunks are no slower: one prompt of 32 rows 23 us either way, 63 36 token by token and 22 in chunks;
+// 16 prompts of 32 78 and 75; 600 rows beside 30 decode rows 704 all token by token, 138 all in chunks, 112 like this.
+constexpr int kLong = 32;
 constexpr int kD = 128;   // key channels
 constexpr int kPad = 4;   // floats of padding per LDS row
 constexpr int kMat = kC * kD;
@@ -46,8 +54,11 @@ struct FormArgs {
   int n_seq, n_slots, T, H;
 };
 
-// Sequence s has the chunks seq_rows[s] / 16 + s and up: no two sequences share one.
-__device__ __forceinline__ int first_chunk(const int* seq_rows, int s) { return (seq_rows[s] >> 4) + s; }
+// A long sequence s has the chunks first_chunk(s) and up.  The second term grows by one at least with every long sequence,
+// so no two share a chunk; the step's rows bound it as its sequences do.
+__device__ __forceinline__ int first_chunk(const int* seq_rows, int s) {
+  return (seq_rows[s] >> 4) + min(s, seq_rows[s] / kLong);
+}
 
 // Where token t stands in U' (row), G (row and column), H (column), K''^T and B''^T (column): instruction i of the chunk
 // kernel's sums over tokens then takes tokens 4 i .. 4 i + 3.  In the order of the tokens, later ones decayed less, the
@@ -80,7 +91,7 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
   __shared__ __attribute__((aligned(16))) float gram[4][kC][kC + kPad];  // U B^T, U K^T (below the diagonal; then G), R B^T, R K^T
   __shared__ __attribute__((aligned(16))) float p16[kD];
   float(*pw)[LD] = m[3];  // minus the decays' logarithms
-  const int tid = threadIdx.x, h = blockIdx.x, ci = blockIdx.y;
+  const int tid = threadIdx.x, h = blockIdx.x % g.H, ci = blockIdx.x / g.H;
   int s = 0;
   for (int lo = 0, hi = g.n_seq; lo < hi;) {  // the last sequence that starts at or before the chunk
     const int mid = (lo + hi) >> 1;
@@ -89,7 +100,8 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
   }
   const int t0 = (ci - first_chunk(g.seq_rows, s)) * kC, r0 = g.seq_rows[s] + t0, n = g.seq_rows[s + 1] - r0;
   const int slot = g.slots[s];
-  if (t0 < 0 || n <= 0 || g.seq_rows[s] < 0 || g.seq_rows[s + 1] > g.T || slot < 0 || slot >= g.n_slots) return;
+  if (t0 < 0 || n <= 0 || t0 + n < kLong || g.seq_rows[s] < 0 || g.seq_rows[s + 1] > g.T || slot < 0 || slot >= g.n_slots)
+    return;
   // ---- a thread per token and eight channels
   const int t = tid >> 4, c0 = (tid & 15) * 8;
   float u[8], b[8], kk[8], rr[8];
@@ -240,8 +252,8 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
 }
 
 struct ChunkArgs {
-  FormArgs f;    // the rows themselves (in_order)
-  float* out;    // [T, H * dv]
+  DeltaArgs tok;  // the same rows token by token
+  float* out;     // [T, H * dv]
   float* state;  // [slots, H, dv, 128]
   const float* ws;
   const bf16_t* v;
@@ -258,54 +270,7 @@ template <int NB> struct Frags {
   uint32_t v[NB][4];  // rows g4, 4 + g4, 8 + g4 and 12 + g4 of V; bf16 bits as loaded: a conversion here would wait for the load
 };
 
-// NB blocks of 16 columns of a sequence of n rows, token by token and in plain loops: for values that are not finite.
-template <int NB>
-__device__ __forceinline__ void in_order(const ChunkArgs& g, float* row /* [5][128] LDS */, float* red /* [4] LDS */, int r0,
-                                                   int n, int h, int slot, int col0) {
-  constexpr int TPC = 256 / (16 * NB), CH = kD / TPC;  // threads per column, channels of each
-  const FormArgs& f = g.f;
-  const int tid = threadIdx.x, c = tid / TPC, part = tid % TPC;
-  float* sp = g.state + ((int64_t)slot * g.H * g.dv + col0 + c) * kD + part * CH;
-  float S[CH];
-#pragma unroll
-  for (int i = 0; i < CH; ++i) S[i] = g.pos[r0] != 0 ? sp[i] : 0.f;
-  for (int t = r0; t < r0 + n; ++t) {
-    __syncthreads();
-    const int ch = tid & (kD - 1), at = h * kD + ch;
-    const float kk = bf16_to_f32(f.k[t * f.ks + at]);
-    const float ss = wave_reduce_sum(tid < kD ? kk * kk : 0.f);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
-    __syncthreads();
-    if (tid < kD) {
-      const float u = kk * rsqrtf(red[0] + red[1] + f.key_eps);
-      row[ch] = u;
-      row[kD + ch] = sigmoid1(bf16_to_f32(f.a[t * f.as + at]) + (f.a_bias ? f.a_bias[at] : 0.f)) * u;
-      row[2 * kD + ch] = expf(-f.decay_scale * sigmoid1(bf16_to_f32(f.w[t * f.wst + at]) + (f.w_bias ? f.w_bias[at] : 0.f)));
-      row[3 * kD + ch] = kk;
-      row[4 * kD + ch] = bf16_to_f32(f.r[t * f.rs + at]);
-    }
-    __syncthreads();
-    const float v = bf16_to_f32(g.v[t * g.vs + col0 + c]);
-    const float* p = row + part * CH;
-    float x = 0.f, o = 0.f;
-#pragma unroll
-    for (int i = 0; i < CH; ++i) x += p[i] * S[i];
-#pragma unroll
-    for (int m = 1; m < TPC; m <<= 1) x += __shfl_xor(x, m, 64);
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      S[i] = p[2 * kD + i] * S[i] - p[kD + i] * x + p[3 * kD + i] * v;
-      o += p[4 * kD + i] * S[i];
-    }
-#pragma unroll
-    for (int m = 1; m < TPC; m <<= 1) o += __shfl_xor(o, m, 64);
-    if (part == 0) g.out[(int64_t)t * g.H * g.dv + col0 + c] = o;
-  }
-#pragma unroll
-  for (int i = 0; i < CH; ++i) sp[i] = S[i];
-}
-
-// The k-th longest of up to 64 sequences (more of them even out by themselves): the workgroups go out in this order, so
+// The k-th longest of up to 16 sequences (more of them even out by themselves): the workgroups go out in this order, so
 // that the longest does not start when a short one's place is free.
 __device__ __forceinline__ int by_length(const int* seq_rows, int n_seq, int k, int lane) {
   if (n_seq > 16) return k;
@@ -318,11 +283,19 @@ __device__ __forceinline__ int by_length(const int* seq_rows, int n_seq, int k, 
   return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < n_seq && rank == k));
 }
 
-// NB: blocks of 16 columns per workgroup
-template <int NB>
+// NB: blocks of 16 columns per workgroup; CT: columns per thread of the sequences that go token by token
+template <int NB, int CT>
 __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(ChunkArgs g) {
-  __shared__ __attribute__((aligned(16))) f32x4 px[2][4][NB][64];  // parts of X
-  __shared__ float po[2][4][NB][4][64];                             // parts of O, by accumulator register
+  struct Parts {
+    __attribute__((aligned(16))) f32x4 x[2][4][NB][64];  // parts of X
+    float o[2][4][NB][4][64];                            // parts of O, by accumulator register
+  };
+  __shared__ union {
+    Parts parts;
+    DeltaLds<8, 256, CT> tok;
+  } lds;
+  auto& px = lds.parts.x;
+  auto& po = lds.parts.o;
   const int nb = g.dv / (16 * NB);
   // the column blocks of a (sequence, head) read the same chunks: neighbours on one XCD (blocks go out round robin)
   const int id = blockIdx.x, sh = id / (8 * nb) * 8 + id % 8, blk = id / 8 % nb;
@@ -337,6 +310,14 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
   if (slot < 0 || slot >= g.n_slots) {  // padding rows: a defined result, no state
     for (int i = threadIdx.x; i < n * 16 * NB; i += 256)
       g.out[(int64_t)(r0 + i / (16 * NB)) * g.H * g.dv + col0 + i % (16 * NB)] = 0.f;
+    return;
+  }
+  if (n < kLong) {
+    // CT > 1: other workgroups of every sequence and head -- they are dealt out to the chip in turn, and every fourth of
+    // them would lie in a quarter of it
+    constexpr int W = CT > 1 ? 32 * CT : 16 * NB;
+    const int c0 = (blk + sh / 8) % nb * W;
+    if (c0 < g.dv) delta_tokens<bf16_t, 8, 256, CT, true>(g.tok, lds.tok, r0, n, h, slot, c0, min(g.dv, c0 + W));
     return;
   }
   // S: channels 32 w + 16 cb + 4 g4 + i of column l16 of every block
@@ -470,7 +451,7 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
 #pragma unroll
       for (int i = 0; i < 4; ++i) finite = finite && fabsf(S[q][cb][i]) < INFINITY;
   if (__syncthreads_or(!finite)) {  // (also waits for the rows stored above)
-    in_order<NB>(g, &po[0][0][0][0][0], reinterpret_cast<float*>(&px[0][0][0][0]), r0, n, h, slot, col0);
+    delta_tokens<bf16_t, 8, 256, CT, true>(g.tok, lds.tok, r0, n, h, slot, blk * 16 * NB, (blk + 1) * 16 * NB);
     return;
   }
 #pragma unroll
@@ -483,16 +464,16 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
 
 extern "C" {
 
-// Floats of workspace of the chunked form for these rows (named by seq_rows), 0 where the token-by-token form takes them:
-// bf16 rows of at least eight tokens a sequence on average (below, most chunks are padding; a decode step has no
-// seq_rows at all), keys of 128 channels, whole blocks of 16 value columns, decays whose product over a chunk stays far
-// inside fp32, 16-byte aligned rows (`ptrs`, `strides`: those of r, k, a, w and the state's pointer, or-ed).
+// Floats of workspace of the chunked form for these rows (named by seq_rows), 0 where the token-by-token form takes all of
+// them: bf16 rows, enough for a long sequence (a decode step has no seq_rows at all), keys of 128 channels, whole blocks of
+// 16 value columns, decays whose product over a chunk stays far inside fp32, 16-byte aligned rows (`ptrs`, `strides`: those
+// of r, k, a, w and the state's pointer, or-ed).
 int64_t dxm_delta_chunk_floats(int T_, int n_seq, int H, int dk, int dv, int f32, float decay_scale, int64_t ptrs,
                                int64_t strides) {
   if (f32 || dk != kD || dv % 16 || dv < 16 || ptrs % 16 || strides % 8 || !(decay_scale >= -4.f && decay_scale <= 4.f))
     return 0;
-  const int64_t chunks = T_ / kC + (int64_t)n_seq;
-  if ((int64_t)H * dv > (1 << 26) || T_ < 8 * (int64_t)n_seq || chunks > 65535 || H > 65535 ||
+  const int64_t chunks = T_ / kC + std::min(n_seq, T_ / kLong);
+  if ((int64_t)H * dv > (1 << 26) || T_ < kLong || chunks * H > 0x7fffffff || H > 65535 ||
       (int64_t)n_seq * H * (dv / 16) > (1 << 30))
     return 0;
   return chunks * H * kChunkFloats;
@@ -509,16 +490,26 @@ int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void
   if (!dxm_delta_chunk_floats(T_, n_seq, H, kD, dv, 0, decay_scale, ptrs, rs | ks | as | wst)) return 2;
   FormArgs f{ws, (const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)a, (const bf16_t*)w, rs, ks, as, wst, a_bias, w_bias,
              seq_rows, slots, decay_scale, key_eps, n_seq, n_slots, T_, H};
-  hipLaunchKernelGGL(delta_form_kernel, dim3(H, T_ / kC + n_seq), dim3(256), 0, st, f);
-  ChunkArgs c{f, out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
+  hipLaunchKernelGGL(delta_form_kernel, dim3((unsigned)((T_ / kC + std::min(n_seq, T_ / kLong)) * H)), dim3(256), 0, st, f);
+  DeltaArgs d{};
+  d.out = out, d.state = state, d.r = r, d.k = k, d.v = v, d.rs = rs, d.ks = ks, d.vs = vs, d.pos = pos;
+  d.seq_rows = seq_rows, d.slots = slots, d.n_slots = n_slots, d.T = T_, d.H = H, d.dk = kD, d.dv = dv;
+  d.a = a, d.w = w, d.as = as, d.wst = wst, d.a_bias = a_bias, d.w_bias = w_bias;
+  d.decay_scale = decay_scale, d.key_eps = key_eps;
+  ChunkArgs c{d, out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
   const int64_t heads = ((int64_t)n_seq * H + 7) / 8 * 8;
   // Two column blocks a workgroup read a chunk once for both, but only two of their workgroups fit a CU; one block keeps
   // more of the chip busy until there are twice as many workgroups as fit.  Whole layer, 32 heads, us, one / two blocks:
   // two prompts of 3000 tokens together 343 / 392, three of 4001 443 / 479, four of 3000 335 / 325, six of 5000 547 / 481
-  if (dv % 32 == 0 && heads * (dv / 16) >= 1024)
-    hipLaunchKernelGGL(delta_chunk_kernel<2>, dim3((unsigned)(heads * (dv / 32))), dim3(256), 0, st, c);
-  else
-    hipLaunchKernelGGL(delta_chunk_kernel<1>, dim3((unsigned)(heads * (dv / 16))), dim3(256), 0, st, c);
+  // Many short sequences in tiles of four columns a thread, few in more workgroups: 64 / 16 / 4 prompts of 16 tokens, four
+  // columns 167 / 69 / 36, one 250 / 74 / 21 (in chunks, whatever their length: 168 / 63 / 24)
+  if (dv % 32 == 0 && heads * (dv / 16) >= 1024) {
+    const dim3 grid((unsigned)(heads * (dv / 32)));
+    if (heads >= 512) hipLaunchKernelGGL((delta_chunk_kernel<2, 4>), grid, dim3(256), 0, st, c);
+    else hipLaunchKernelGGL((delta_chunk_kernel<2, 1>), grid, dim3(256), 0, st, c);
+  } else {
+    hipLaunchKernelGGL((delta_chunk_kernel<1, 1>), dim3((unsigned)(heads * (dv / 16))), dim3(256), 0, st, c);
+  }
   DX_CHECK_LAUNCH();
   return 0;
 }

@@ -14,7 +14,7 @@
 // Every kernel is a template over the activation element (bf16 bits or float);
 // decays, removal rates, unit keys, the running matrix, angles and all sums are
 // fp32 whatever the element is.  Sizes are run-time arguments.
-#include "recurrent.h"
+#include "delta_tokens.h"
 
 namespace {
 
@@ -39,20 +39,7 @@ namespace {
 // chain.  Tokens are staged through LDS kTok at a time, fetched into registers
 // one block ahead (the latency hides behind the current block's recurrence).
 
-struct DeltaArgs {
-  float* out;    // [T, H * dv]
-  float* state;  // [slots, H, dv, dk]
-  const void *r, *k, *v;
-  int64_t rs, ks, vs;  // row strides (elements)
-  const float* prep;   // [T, H, 3, dk]: unit key, decay, removal rate * unit key
-  const int64_t* pos;
-  const int* seq_rows;  // null: row i is sequence i
-  const int* slots;
-  int n_slots, T, H, dk, dv;
-};
-
-// one wave per (row, head): u = k / sqrt(sum k^2 + key_eps), w = exp(-decay_scale sigmoid(wl + w_bias)),
-// a u with a = sigmoid(al + a_bias)
+// one wave per (row, head)
 template <typename T>
 __global__ void __launch_bounds__(64) delta_prep_kernel(float* __restrict__ prep, const T* __restrict__ k, int64_t ks,
                                                         const T* __restrict__ a, int64_t as, const T* __restrict__ w,
@@ -65,208 +52,37 @@ __global__ void __launch_bounds__(64) delta_prep_kernel(float* __restrict__ prep
   float ss = 0.f;
   for (int ch = lane; ch < dk; ch += 64) {
     const float x = ldf<T>(kp, ch);
-    ss += x * x;
+    ss = fmaf(x, x, ss);
   }
-  const float inv = rsqrtf(wave_reduce_sum(ss) + key_eps);
+  const float inv = delta_key_scale(ss, key_eps);
   float* o = prep + v * 3 * dk;
   for (int ch = lane; ch < dk; ch += 64) {
     const float u = ldf<T>(kp, ch) * inv;
     const float ab = a_bias ? a_bias[h * dk + ch] : 0.f, wb = w_bias ? w_bias[h * dk + ch] : 0.f;
     o[ch] = u;
-    o[dk + ch] = expf(-decay_scale * sigmoidf_(ldf<T>(w, row * ws + (int64_t)h * dk + ch) + wb));
-    o[2 * dk + ch] = sigmoidf_(ldf<T>(a, row * as + (int64_t)h * dk + ch) + ab) * u;
+    o[dk + ch] = delta_decay(ldf<T>(w, row * ws + (int64_t)h * dk + ch), wb, decay_scale);
+    o[2 * dk + ch] = delta_removal(ldf<T>(a, row * as + (int64_t)h * dk + ch), ab, u);
   }
 }
 
 template <typename T, int R, int NT, int CT>
 __global__ void __launch_bounds__(NT) delta_rule_kernel(DeltaArgs g) {
-  constexpr int kCols = CT;
-  constexpr int kGroups = NT / R;            // column tiles per workgroup
-  constexpr int kWgCols = kGroups * kCols;   // columns per workgroup
-  constexpr int kDkp = kRows * R;            // padded key width
-  constexpr int kE = (kTok * kDkp + NT - 1) / NT;  // staged elements per thread and array
-  constexpr int kEv = (kTok * kWgCols + NT - 1) / NT;
-  __shared__ __attribute__((aligned(16))) float sr[kTok][kDkp];
-  __shared__ __attribute__((aligned(16))) float sk[kTok][kDkp];
-  __shared__ __attribute__((aligned(16))) float su[kTok][kDkp];
-  __shared__ __attribute__((aligned(16))) float sw[kTok][kDkp];
-  __shared__ __attribute__((aligned(16))) float sa[kTok][kDkp];
-  __shared__ __attribute__((aligned(16))) float sv[kTok][kWgCols];
-  const int tid = threadIdx.x, part = tid % R, grp = tid / R;
-  const int s = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * kWgCols + grp * kCols;
+  __shared__ DeltaLds<R, NT, CT> lds;
+  const int s = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * (NT / R * CT);
   const int r0 = g.seq_rows ? g.seq_rows[s] : s;
   const int r1 = g.seq_rows ? g.seq_rows[s + 1] : s + 1;
   const int slot = g.slots[s];
   const int n = r1 - r0;
   if (n <= 0 || r0 < 0 || r1 > g.T) return;
   if (slot < 0 || slot >= g.n_slots) {  // padding rows: a defined result, no state
+    const int part = threadIdx.x % R, j0 = col0 + threadIdx.x / R * CT;
     if (part == 0)
       for (int t = r0; t < r1; ++t)
-        for (int c = 0; c < kCols; ++c)
+        for (int c = 0; c < CT; ++c)
           if (j0 + c < g.dv) g.out[(int64_t)t * g.H * g.dv + h * g.dv + j0 + c] = 0.f;
     return;
   }
-  // The thread's 16 rows are four quads, quad m at row (m * R + part) * 4: for one m the R lanes of a
-  // group read R consecutive 16-byte pieces of a row vector, so a wave's LDS read touches every bank once
-  // (16 consecutive rows per lane would put lanes 0, 2, 4, .. on the same banks).
-  float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv) * g.dk;  // + column * dk + row
-  const bool fresh = g.pos[r0] == 0;
-  int rq[kRows / 4];
-#pragma unroll
-  for (int m = 0; m < kRows / 4; ++m) rq[m] = (m * R + part) * 4;
-  float S[kCols][kRows];
-#pragma unroll
-  for (int c = 0; c < kCols; ++c) {
-#pragma unroll
-    for (int q = 0; q < kRows; ++q) S[c][q] = 0.f;
-    if (fresh || j0 + c >= g.dv) continue;
-    const float* spc = sp + (int64_t)(j0 + c) * g.dk;
-#pragma unroll
-    for (int m = 0; m < kRows / 4; ++m) {
-      if (g.dk % 4 == 0 && rq[m] + 4 <= g.dk) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(spc + rq[m]);
-        S[c][4 * m] = x[0], S[c][4 * m + 1] = x[1], S[c][4 * m + 2] = x[2], S[c][4 * m + 3] = x[3];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (rq[m] + e < g.dk) S[c][4 * m + e] = spc[rq[m] + e];
-      }
-    }
-  }
-  const T* pr = (const T*)g.r + (int64_t)h * g.dk;
-  const T* pk = (const T*)g.k + (int64_t)h * g.dk;
-  const float* pp = g.prep + (int64_t)h * 3 * g.dk;
-  const T* pv = (const T*)g.v + (int64_t)h * g.dv + blockIdx.z * kWgCols;
-  float fr[kE], fk[kE], fu[kE], fa[kE], fw[kE], fv[kEv];
-  auto fetch = [&](int t0) {
-#pragma unroll
-    for (int e = 0; e < kE; ++e) {
-      const int idx = tid + e * NT, tt = idx / kDkp, ch = idx % kDkp;
-      const bool ok = idx < kTok * kDkp && t0 + tt < n && ch < g.dk;
-      const int64_t row = r0 + t0 + tt;
-      const float* pq = pp + row * g.H * 3 * g.dk + ch;
-      fr[e] = ok ? ldf<T>(pr, row * g.rs + ch) : 0.f;
-      fk[e] = ok ? ldf<T>(pk, row * g.ks + ch) : 0.f;
-      fu[e] = ok ? pq[0] : 0.f;
-      fw[e] = ok ? pq[g.dk] : 0.f;
-      fa[e] = ok ? pq[2 * g.dk] : 0.f;
-    }
-#pragma unroll
-    for (int e = 0; e < kEv; ++e) {
-      const int idx = tid + e * NT, tt = idx / kWgCols, cc = idx % kWgCols;
-      const bool ok = idx < kTok * kWgCols && t0 + tt < n && blockIdx.z * kWgCols + cc < g.dv;
-      fv[e] = ok ? ldf<T>(pv, (int64_t)(r0 + t0 + tt) * g.vs + cc) : 0.f;
-    }
-  };
-  fetch(0);
-  float* outp = g.out + (int64_t)r0 * g.H * g.dv + h * g.dv + j0;
-  const bool out4 = g.dv % 4 == 0 && j0 + kCols <= g.dv;
-  for (int t0 = 0; t0 < n; t0 += kTok) {
-    __syncthreads();  // the previous block's tokens are consumed
-#pragma unroll
-    for (int e = 0; e < kE; ++e) {
-      const int idx = tid + e * NT, tt = idx / kDkp, ch = idx % kDkp;
-      if (idx < kTok * kDkp) {
-        sr[tt][ch] = fr[e];
-        sk[tt][ch] = fk[e];
-        su[tt][ch] = fu[e];
-        sw[tt][ch] = fw[e];
-        sa[tt][ch] = fa[e];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < kEv; ++e) {
-      const int idx = tid + e * NT;
-      if (idx < kTok * kWgCols) sv[idx / kWgCols][idx % kWgCols] = fv[e];
-    }
-    __syncthreads();
-    if (t0 + kTok < n) fetch(t0 + kTok);
-    const int nt = n - t0 < kTok ? n - t0 : kTok;
-    // the five row vectors of a token (unit key, decay, removal, key, read-out) and its values
-    auto load = [&](int tt, float (*b)[kRows], float* vj) {
-#pragma unroll
-      for (int q = 0; q < kRows; q += 4) {
-        *reinterpret_cast<f32x4*>(b[0] + q) = *reinterpret_cast<const f32x4*>(&su[tt][rq[q / 4]]);
-        *reinterpret_cast<f32x4*>(b[1] + q) = *reinterpret_cast<const f32x4*>(&sw[tt][rq[q / 4]]);
-        *reinterpret_cast<f32x4*>(b[2] + q) = *reinterpret_cast<const f32x4*>(&sa[tt][rq[q / 4]]);
-        *reinterpret_cast<f32x4*>(b[3] + q) = *reinterpret_cast<const f32x4*>(&sk[tt][rq[q / 4]]);
-        *reinterpret_cast<f32x4*>(b[4] + q) = *reinterpret_cast<const f32x4*>(&sr[tt][rq[q / 4]]);
-      }
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) vj[c] = sv[tt][grp * kCols + c];
-    };
-    auto step = [&](const float (*b)[kRows], const float* vj, float* o_) {
-      float us[kCols];
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) {
-        float a_ = 0.f;
-#pragma unroll
-        for (int q = 0; q < kRows; ++q) a_ += b[0][q] * S[c][q];
-        us[c] = group_sum<R>(a_);
-      }
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) {
-        float a_ = 0.f;
-#pragma unroll
-        for (int q = 0; q < kRows; ++q) {
-          S[c][q] = S[c][q] * b[1][q] - b[2][q] * us[c] + b[3][q] * vj[c];
-          a_ += b[4][q] * S[c][q];
-        }
-        o_[c] = group_sum<R>(a_);
-      }
-    };
-    auto store = [&](int tt, const float* o_) {
-      float* op = outp + (int64_t)(t0 + tt) * g.H * g.dv;
-      if constexpr (kCols == 4) {
-        if (out4) *reinterpret_cast<f32x4*>(op) = f32x4{o_[0], o_[1], o_[2], o_[3]};
-      }
-      if (kCols != 4 || !out4) {
-#pragma unroll
-        for (int c = 0; c < kCols; ++c)
-          if (j0 + c < g.dv) op[c] = o_[c];
-      }
-    };
-    if (kCols <= 2 && nt == kTok) {
-      // a whole block of the narrow tile (the wide one has no registers to spare), unrolled in one basic
-      // block: the next token's vectors are read from LDS while the current token's chain runs, and the
-      // outputs are stored once at the end
-      float b0[5][kRows], b1[5][kRows], v0[kCols], v1[kCols], ob[kTok][kCols];
-      load(0, b0, v0);
-#pragma unroll
-      for (int tt = 0; tt < kTok; tt += 2) {
-        load(tt + 1, b1, v1);
-        step(b0, v0, ob[tt]);
-        if (tt + 2 < kTok) load(tt + 2, b0, v0);
-        step(b1, v1, ob[tt + 1]);
-      }
-      if (part == 0) {
-#pragma unroll
-        for (int tt = 0; tt < kTok; ++tt) store(tt, ob[tt]);
-      }
-    } else {
-      for (int tt = 0; tt < nt; ++tt) {
-        float b0[5][kRows], v0[kCols], o_[kCols];
-        load(tt, b0, v0);
-        step(b0, v0, o_);
-        if (part == 0) store(tt, o_);
-      }
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < kCols; ++c) {
-    if (j0 + c >= g.dv) continue;
-    float* spc = sp + (int64_t)(j0 + c) * g.dk;
-#pragma unroll
-    for (int m = 0; m < kRows / 4; ++m) {
-      if (g.dk % 4 == 0 && rq[m] + 4 <= g.dk) {
-        *reinterpret_cast<f32x4*>(spc + rq[m]) = f32x4{S[c][4 * m], S[c][4 * m + 1], S[c][4 * m + 2], S[c][4 * m + 3]};
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (rq[m] + e < g.dk) spc[rq[m] + e] = S[c][4 * m + e];
-      }
-    }
-  }
+  delta_tokens<T, R, NT, CT, false>(g, lds, r0, n, h, slot, col0, g.dv);
 }
 
 // NT threads per workgroup: 64 where that covers all columns of a head, else 256.  Columns per
@@ -834,7 +650,9 @@ int dxm_delta_rule(float* out, float* state, int n_slots, float* prep, const voi
   if (!seq_rows && n_seq != T_) return 4;
   DISPATCH_T(f32, hipLaunchKernelGGL(delta_prep_kernel<T>, dim3((unsigned)(T_ * H)), dim3(64), 0, st, prep, (const T*)k,
                                      ks, (const T*)a, as, (const T*)w, ws, a_bias, w_bias, decay_scale, key_eps, H, dk));
-  DeltaArgs g{out, state, r, k, v, rs, ks, vs, prep, pos, seq_rows, slots, n_slots, T_, H, dk, dv};
+  DeltaArgs g{};
+  g.out = out, g.state = state, g.r = r, g.k = k, g.v = v, g.rs = rs, g.ks = ks, g.vs = vs, g.prep = prep;
+  g.pos = pos, g.seq_rows = seq_rows, g.slots = slots, g.n_slots = n_slots, g.T = T_, g.H = H, g.dk = dk, g.dv = dv;
   const int need = (dk + kRows - 1) / kRows;
   if (need <= 4) { DISPATCH_T(f32, (launch_delta<T, 4>(g, n_seq, st))); }
   else if (need <= 8) { DISPATCH_T(f32, (launch_delta<T, 8>(g, n_seq, st))); }

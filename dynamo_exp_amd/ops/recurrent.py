@@ -311,7 +311,8 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tenso
         o_t = S_t^T r_t
     r, k, a, w [T, H dk] and v [T, H dv] are column sections (contiguous rows,
     any row stride) of projection outputs.  Returns o [T, H dv] fp32.
-    Everything but reading the inputs is fp32."""
+    Everything but reading the inputs is fp32.  How a sequence's rows are summed
+    depends on their number alone, not on what else the step holds."""
     T = r.shape[0]
     n_seq = state_slots.numel()
     _fp32_param(a_bias, "a_bias")
@@ -348,11 +349,10 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tenso
     rows = (r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), a.data_ptr(), a.stride(0),
             w.data_ptr(), w.stride(0), _ptr(a_bias), _ptr(w_bias), float(decay_scale), float(key_eps), positions.data_ptr(),
             _ptr(seq_rows), state_slots.data_ptr(), n_seq, T, n_heads)
-    # below 64 rows both forms take what their two launches take (31 us a call of one prompt of 48, at 64 30 against 37)
-    if seq_rows is not None and T >= 64:
+    if seq_rows is not None:
         floats = _m().delta_chunk_floats(T, n_seq, n_heads, dk, dv, _f32(r), decay_scale, rows[0] | rows[2] | rows[6] | rows[8] |
                                          state.data_ptr(), rows[1] | rows[3] | rows[7] | rows[9])
-        if floats:  # prompt rows in chunks (csrc/mixers/delta_chunk.hip)
+        if floats:  # the rows of long sequences in chunks (csrc/mixers/delta_chunk.hip)
             ws = torch.empty(floats, dtype=torch.float32, device=r.device)
             _m().delta_chunk(out.data_ptr(), state.data_ptr(), state.shape[0], ws.data_ptr(), *rows, dv, _stream())
             return out

@@ -119,3 +119,41 @@ def test_delta_chunk_rule():
     assert ok(*yes) == (40 + 3) * 2 * (4 * 2048 + 512 + 128)
     for i, x in ((0, 23), (3, 64), (4, 40), (5, 1), (6, 4.5), (6, math.nan), (7, 8), (8, 4)):
         assert ok(*yes[:i], x, *yes[i + 1:]) == 0
+
+
+def run(p, wl, ab, wb, state, pos, starts, slots, H, dv, scale=SCALE):
+    """The rows [r | k | a | v] on the GPU -> outputs, with `state` updated."""
+    n = H * 128
+    return rc.delta_rule(p[:, :n], p[:, n:2 * n], p[:, 3 * n:], p[:, 2 * n:3 * n], wl, ab, wb, state, pos,
+                         None if starts is None else torch.tensor(starts, dtype=torch.int32).cuda(),
+                         torch.tensor(slots, dtype=torch.int32).cuda(), H, 128, dv, decay_scale=scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,dv,rows", [
+    (2, 128, [1, 31, 32, 200, 5, 1]), (3, 16, [70, 1, 33, 30]), (1, 48, [1, 1, 100, 33, 32, 31, 1, 80]),
+    (16, 128, [1, 32, 90, 2, 65, 0, 1, 31, 129]),  # two column blocks a workgroup
+    (8, 128, [200] + [1] * 150), (2, 32, [1] * 90 + [64]),  # more sequences than eight rows each would allow
+    (32, 128, [1] * 70 + [80])])  # (as a decode step of their own: tiles of 2 columns a thread)
+def test_a_sequence_does_not_depend_on_its_step(H, dv, rows):
+    """Every sequence's rows and state are bit for bit what they are in a step of its own."""
+    torch.manual_seed(23)
+    T, n, B = sum(rows), H * 128, len(rows)
+    p, wl = torch.randn(T, 3 * n + H * dv, device="cuda").bfloat16(), (torch.randn(T, n, device="cuda") * 0.5).bfloat16()
+    ab, wb = torch.randn(n, device="cuda") * 0.5, torch.randn(n, device="cuda")
+    firsts = [sum(rows[:i]) for i in range(B + 1)]
+    pos = torch.cat([torch.arange(7 * (i % 2), 7 * (i % 2) + r) for i, r in enumerate(rows)]).cuda()
+    state0 = torch.randn(B, H, dv, 128, device="cuda")
+    together = state0.clone()
+    out = run(p, wl, ab, wb, together, pos, firsts, list(range(B)), H, dv)
+    for i, r in enumerate(rows):
+        if r == 0:
+            assert torch.equal(together[i], state0[i])
+            continue
+        if i and r == 1 and rows[i - 1] == 1 and i % 16:  # (a few of many equal ones)
+            continue
+        x, alone = slice(firsts[i], firsts[i + 1]), state0.clone()
+        for starts in ([0, r],) if r > 1 else ([0, 1], None):  # (a decode step names no rows)
+            alone.copy_(state0)
+            got = run(p[x], wl[x], ab, wb, alone, pos[x], starts, [i], H, dv)
+            assert torch.equal(got, out[x]) and torch.equal(alone[i], together[i]), (i, r)
