@@ -15,13 +15,14 @@
 // R' S as they lie; the parts of X and O join in LDS, one barrier a chunk.  The other sequences run in the same launch,
 // token by token, beside the long ones' chains.
 //
-// P_t shrinks by at most exp(-16 |decay_scale|) in a chunk, so 1 / P stays far inside fp32 (the host refuses more
-// than 4).  A chunk's dependent chain is 50 matrix instructions and a barrier instead of 16 tokens' chains of lane sums.
+// P_t shrinks by at most exp(-16 |decay_scale|) in a chunk: 1e-7, and 1 / P 1e7, at the largest the host sends here (1), so
+// that only values within 1e7 of fp32's ends leave its range on the way.  A chunk's dependent chain is 50 matrix instructions and a barrier instead of 16 tokens' chains of lane sums.
 // Its rounding: the products of decays come from sums of logarithms in fp64, the sums run in an order that keeps them
 // small and through short chains; relative to 64 bits 1.28e-7 in o and 6.90e-8 in S where the token-by-token form has
 // 1.32e-7 and 6.91e-8 (900 to 4001 tokens; 1.9e-7 and 1.2e-7 with running products and one chain per sum).
-// A value that is not finite would reach the rows in front of it in its chunk (zero factors times it).  It also stays in
-// the state, so a workgroup that ends with such a state takes its columns again, token by token.
+// A value that is not finite, or that 1 / P makes so, would reach other rows of its chunk than its own and later ones (zero
+// factors times it).  It shows in the rows or stays in the state, and a workgroup that meets one takes its columns again,
+// token by token.
 // 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us, each
 // profiled by itself (in a row, with the layer's norm of 35: 443); a prompt of 600 beside 30 single tokens 704 -> 112, the
 // layer without its norm.  Bound by the fp32 matrix instructions (200 us of them run) beside the fragments' way through L2.
@@ -358,6 +359,7 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
   char* op = (char*)(g.out + (int64_t)r0 * g.H * g.dv + col0);
   const int64_t ostep = (int64_t)kC * g.H * g.dv * 4;
   const uint32_t o_off = 4u * ((4 * g4 + w) * (uint32_t)(g.H * g.dv) + l16);
+  bool finite = true;
   auto step = [&](const Frags<NB>& f, int c, Frags<NB>& next, int cn) {
     const int buf = c & 1;
     load(next, min(cn, nc - 1));  // (always a load, the last chunk again: the waits stay counts)
@@ -431,9 +433,11 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
       for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[q][cb][i] = N[q][cb][i] - M[q][cb][i];
-      if (c * kC + 4 * g4 + w < n)  // the wave's row of each group
-        *reinterpret_cast<float*>(op + c * ostep + o_off + 64 * q) =
-            (po[buf][0][q][w][lane] + po[buf][1][q][w][lane]) + (po[buf][2][q][w][lane] + po[buf][3][q][w][lane]);
+      if (c * kC + 4 * g4 + w < n) {  // the wave's row of each group
+        const float o = (po[buf][0][q][w][lane] + po[buf][1][q][w][lane]) + (po[buf][2][q][w][lane] + po[buf][3][q][w][lane]);
+        *reinterpret_cast<float*>(op + c * ostep + o_off + 64 * q) = o;
+        finite = finite && fabsf(o) < INFINITY;
+      }
     }
   };
   Frags<NB> f0, f1;  // (two chunks ahead: a workgroup fewer per CU, 1 to 4 % slower)
@@ -443,7 +447,6 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
     step(f0, c, f1, c + 1);
     if (c + 1 < nc) step(f1, c + 1, f0, c + 2);
   }
-  bool finite = true;
 #pragma unroll
   for (int q = 0; q < NB; ++q)
 #pragma unroll
@@ -470,7 +473,7 @@ extern "C" {
 // of r, k, a, w and the state's pointer, or-ed).
 int64_t dxm_delta_chunk_floats(int T_, int n_seq, int H, int dk, int dv, int f32, float decay_scale, int64_t ptrs,
                                int64_t strides) {
-  if (f32 || dk != kD || dv % 16 || dv < 16 || ptrs % 16 || strides % 8 || !(decay_scale >= -4.f && decay_scale <= 4.f))
+  if (f32 || dk != kD || dv % 16 || dv < 16 || ptrs % 16 || strides % 8 || !(decay_scale >= -1.f && decay_scale <= 1.f))
     return 0;
   const int64_t chunks = T_ / kC + std::min(n_seq, T_ / kLong);
   if ((int64_t)H * dv > (1 << 26) || T_ < kLong || chunks * H > 0x7fffffff || H > 65535 ||
