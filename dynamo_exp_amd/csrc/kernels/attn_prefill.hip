@@ -404,28 +404,23 @@ extern "C" int dx_prefill_attention(void* out, const void* q, int64_t q_stride, 
   // and with half as much work in the last and the longest of them.  32 / 8 heads, us, eight / four: one prompt of 2000 61.9 /
   // 54.8 (256 workgroups of eight), six of 3000 together 32.2 / 29.7 (392), 300 rows behind 2900 cached 92.7 / 71.0 (40),
   // two of 5000 136.3 / 138.2 (632), three of 6151 152.4 / 151.2 (776).
-  const bool four = (int64_t)n_kv_heads * (G / hpw) * n_work < 512;
+  // n_waves 92 selects the first loop, of eight waves (A/B runs: tools/attn_ab.py, tools/attn_accuracy.py)
+  const bool r3 = n_waves == 92;
+  const bool four = !r3 && (int64_t)n_kv_heads * (G / hpw) * n_work < 512;
   const dim3 grid(n_kv_heads * (G / hpw), n_work * (four ? 2 : 1));
   const float sl2e = scale * 1.4426950408889634f;
-  // n_waves 92 selects the first loop (A/B runs: tools/attn_ab.py,
-  // tools/attn_accuracy.py)
-  const bool r3 = n_waves == 92;
 #define DX_PA_LAUNCH(BS, VV, NW)                                                                                     \
   prefill_attn_v2_kernel<BS, true, VV, NW><<<grid, 64 * NW, 0, stream>>>(                                            \
       (bf16_t*)out, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables,        \
       bt_stride, cu_seqlens_q, ctx_lens, work, n_q_heads, n_kv_heads, bs_shift, hpw, sl2e, causal)
-#define DX_PA(BS, VV)                   \
-  do {                                  \
-    if (four) DX_PA_LAUNCH(BS, VV, 4);  \
-    else DX_PA_LAUNCH(BS, VV, 8);       \
+#define DX_PA(BS)                    \
+  do {                               \
+    if (r3) DX_PA_LAUNCH(BS, 0, 8);  \
+    else if (four) DX_PA_LAUNCH(BS, 1, 4); \
+    else DX_PA_LAUNCH(BS, 1, 8);     \
   } while (0)
-  if (block_size >= 64) {
-    if (r3) DX_PA(true, 0);
-    else DX_PA(true, 1);
-  } else {
-    if (r3) DX_PA(false, 0);
-    else DX_PA(false, 1);
-  }
+  if (block_size >= 64) DX_PA(true);
+  else DX_PA(false);
 #undef DX_PA
 #undef DX_PA_LAUNCH
   return (int)hipGetLastError();
