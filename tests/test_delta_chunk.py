@@ -78,6 +78,16 @@ def test_delta_chunks(rows, kind, H, dv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [[40, 64, 50, 33, 0, 1, 32, 70, 20], [64, 31, 33, 48, 5, 0, 40, 32, 1, 100, 17, 36, 63, 1, 34, 2],
+                                  [35, 3] * 17])
+@pytest.mark.parametrize("kind", ["plain", "slow decay", "one key", "grown"])
+def test_delta_chunks_of_many_heads(rows, kind):
+    """Workgroups of two column blocks, four of them to a head, sequences in order of their length (9 and 16) and as they
+    come (34, whose short ones take four columns a thread)."""
+    test_delta_chunks(rows, kind, 16, 128)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dv,n_seq", [(32, 2), (16, 1), (32, 40)])  # (one column block per workgroup, and two)
 @pytest.mark.parametrize("what", ["k", "v", "a", "w", "r", "state"])
 @pytest.mark.parametrize("bad", [math.nan, math.inf])

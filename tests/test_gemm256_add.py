@@ -38,6 +38,18 @@ def test_add(M, N, K, pieces):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,pieces", [
+    (6151, 4096, 256, 0),  # 400 tiles: workgroups with a second whole tile, none cut
+    (8200, 4096, 512, 4),  # 512 whole tiles, two a workgroup, then pieces of K of 16
+    (12295, 4096, 384, 3),  # 768 and 16: three whole tiles a workgroup
+])
+def test_add_after_add(M, N, K, pieces):
+    """A workgroup that adds several tiles, one after the other: a tile's loads of y and stores lie beside the next one's
+    first loads."""
+    test_add(M, N, K, pieces)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [500, 1280, 1300, 4200])
 def test_linear_add(M):
     """The op on both sides of its rule, and rows whose alignment the kernel does not take."""

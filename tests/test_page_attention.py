@@ -182,3 +182,65 @@ def test_penalty_of_any_rate(form, rate):
     # as test_prompt_rows: the result's rounding to bf16 and one rounding of every weight
     err, top = float((got - want).abs().max()), float(want.abs().max())
     assert err < 2.0 ** -8 * (top + 5.0), err
+
+
+# heads of the long contexts: shared rows for 20, 32 and 40 heads take blocks of 32 query vectors, 40 of them two workgroups
+LONG = {"plain": FORMS["plain"], "both": FORMS["both"], "sigmoid": FORMS["sigmoid"], "diff": FORMS["diff"],
+        **{f"shared {H} / {dv}": (H, 1, H, 256, dv) for H in (16, 20, 32, 40) for dv in (192, 256)}}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 1500, 0), ("window", 1000, 64), ("chunk", 2048, 0)])
+@pytest.mark.parametrize("form", LONG)
+def test_decode_rows_of_long_contexts(form, mask, size, keep):
+    """Contexts of 11 to 188 tiles in three to nine parts that hold keys, up to 21 tiles each (an even and an odd number a
+    wave), on pages of one, two and four tiles; float64 on the GPU."""
+    n_qh, maps, group, d, dv = LONG[form]
+    kind = form.split()[0]
+    torch.manual_seed(31)
+    scale, ctx = 0.7 * d ** -0.5, [700, 3500, 6000, 351]
+    G, heads, B = n_qh // maps // group, torch.arange(n_qh, device="cuda") // maps, len(ctx)
+    kh, vh = heads // group * maps + torch.arange(n_qh, device="cuda") % maps, heads // group
+    cap, db, sig, hb, sink = terms("shared" if kind == "shared" else kind, n_qh)
+    for bs, parts in ((32, 3), (64, 5), (128, 9)):
+        nb = [-(-n // bs) for n in ctx]
+        perm = torch.randperm(sum(nb), device="cuda").to(torch.int32)
+        table = torch.zeros(B, max(nb), dtype=torch.int32, device="cuda")
+        kc = torch.full((sum(nb) * bs, d if kind == "shared" else G * maps * d), float("nan"), device="cuda").bfloat16()
+        vc = kc if kind == "shared" else torch.full((sum(nb) * bs, G * dv), float("nan"), device="cuda").bfloat16()
+        q, at, want = torch.randn(B, n_qh * d, device="cuda").bfloat16(), 0, []
+        for i, n in enumerate(ctx):
+            table[i, :nb[i]] = perm[at:at + nb[i]]
+            at += nb[i]
+            j = torch.arange(n, device="cuda")
+            sl = table[i].long()[j // bs] * bs + j % bs
+            kc[sl] = (torch.randn(n, kc.shape[1], device="cuda") * 1.5).bfloat16()
+            if kind == "shared":
+                K = kc[sl].double()[:, None].expand(n, n_qh, d)
+                V = K[:, :, :dv]
+            else:
+                vc[sl] = torch.randn(n, vc.shape[1], device="cuda").bfloat16()
+                K, V = kc[sl].double().view(n, -1, d)[:, kh], vc[sl].double().view(n, -1, dv)[:, vh]
+            # (float64 scores as sums, not as a batched product)
+            s = torch.stack([K[:, h] @ q[i, h * d:(h + 1) * d].double() for h in range(n_qh)]) * scale
+            p = n - 1
+            if cap:
+                s = cap * torch.tanh(s / cap)
+            if db is not None:
+                s = s - cuda(db[0]).double()[:, None] * torch.log1p(cuda(db[1]).double()[:, None] * (p - j)[None])
+            vis = (j >= int(mx.first_visible(torch.tensor([p]), mask, size))) | (j < keep)
+            if sig:
+                w = torch.sigmoid(s + cuda(hb).double()[:, None]) * vis
+            else:
+                s = s.masked_fill(~vis, float("-inf"))
+                if sink is not None:
+                    s = torch.cat([s, cuda(sink).double()[:, None]], -1)
+                w = torch.softmax(s, -1)[:, :n]
+            want.append(torch.stack([w[h] @ V[:, h] for h in range(n_qh)]))
+        want = torch.stack(want)
+        got = mx.attention(q, kc, vc, torch.tensor([c - 1 for c in ctx]).cuda(), None, table, bs, n_qh, maps, group, d, dv, scale,
+                           mask, size, parts, True, softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                           weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), keep_first=keep, sink=cuda(sink)).double()
+        err, top = float((got - want).abs().max()), float(want.abs().max())
+        # as test_decode_rows: weights as two bf16 numbers, 2^-17 of sum w |v|
+        assert err < 3e-4 * (max(top, 1.0) if sig else 1.0), (bs, parts, err, top)
