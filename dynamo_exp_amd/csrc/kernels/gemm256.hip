@@ -56,9 +56,12 @@
 //     pieces' fp32 sums go through a workspace (64 MB at most) to a kernel that
 //     adds them in order.  One more round costs 230 to 320 us at K 14336, whatever
 //     it holds; a sixteenth of one costs 20 and the way through the workspace 30:
-//     4150 x 4096 520 -> 365 us, 1000 x 4096 227 -> 104.  (In a full round the
-//     clock falls to 1.45 GHz at 82 % of the matrix cores' cycles: the card's
-//     power, not the schedule, is the bound there.)
+//     4150 x 4096 520 -> 365 us, 1000 x 4096 227 -> 104.  (In full rounds the
+//     card's power is the bound, not the schedule: the matrix cores are busy
+//     80 % of the cycles, and the clock is 1.75 GHz where launches stand alone,
+//     1.5 in a prompt step: profiles/step_case_counters.txt.)  A row's sum is
+//     cut or not by the tile it lies in, so equal rows of a step may differ by
+//     a rounding, as they do with the library at most of these sizes.
 //   * Blocks are remapped so that each XCD walks a contiguous range of tiles
 //     (bijective for any grid size), in bands of group_m token tiles: the ~32
 //     workgroups resident on one XCD then share group_m x tiles and

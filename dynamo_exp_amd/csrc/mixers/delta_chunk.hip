@@ -25,7 +25,10 @@
 // token by token.
 // 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us, each
 // profiled by itself (in a row, with the layer's norm of 35: 443); a prompt of 600 beside 30 single tokens 704 -> 112, the
-// layer without its norm.  Bound by the fp32 matrix instructions (200 us of them run) beside the fragments' way through L2.
+// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them
+// at 5250 cycles where three workgroups share a CU, 1088 of them a wave's matrix instructions, which keep the matrix cores
+// busy 41 % of the time; the rest is waiting to issue behind the other workgroups' chains, LDS exchanges and the barrier
+// (profiles/step_case_counters.txt).
 #include <algorithm>
 
 #include "delta_tokens.h"

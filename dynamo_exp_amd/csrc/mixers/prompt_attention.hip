@@ -349,8 +349,9 @@ int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   return 0;
 }
 
-// (tiles of 32 / 64 keys, us: cap + penalty 158 / 173, sigmoid 85 / 91, shared row 256 / 192 of 600 rows 47 / 52, plain
-// 114 / 109, plain behind 2900 cached 107 / 94)
+// (tiles of 32 / 64 keys, us, launches back to back: cap + penalty 157 / 153, sigmoid 91 / 99, shared row 256 / 256
+// 128 / 182, 256 / 192 130 / 127 and of 600 rows 35.3 / 36.7, two maps 265 / 350, plain of 5000 149 / 154 and of 40 behind
+// 2900 cached 94 / 83, fine 179 / 186)
 template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT>
 int prompt_heads(const PromptArgs& a, int n_tiles, hipStream_t st) {
   constexpr int SUBS = DV == 128 && MODE == kPlain ? 2 : 1;

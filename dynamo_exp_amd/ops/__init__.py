@@ -279,14 +279,19 @@ CUS = 256  # compute units of an MI355X
 
 
 def deep_add_tiles(M: int, N: int, K: int) -> bool:
-    """Whether y[M, N] += x w^T over a long K takes the 256-tile kernel.  It cuts an incomplete last round along K; the
-    library's choice for these shapes is uneven.  us, library / this kernel, N 4096:
-      K 14336  M 600 98 / 82, 1000 119 / 104, 1450 156 / 155, 2125 214 / 250, 3925 301 / 317, 4150 719 / 365,
-               5050 439 / 427, 5950 513 / 502, 6175 816 / 580, 7525 1010 / 626, 7750 605 / 633, 8200 1027 / 685
-      K 11008  M 600 76 / 68, 1560 127 / 128, 3000 196 / 211, 4440 632 / 309, 4920 337 / 336, 6360 643 / 449
-      K 8192   M 600 60 / 58, 1080 75 / 83, 3000 152 / 167, 4440 258 / 227, 6360 315 / 333, 7320 326 / 351
-    So: K from 10240, and either up to a third of a round (three pieces of K and more) or more than one round whose
-    last is not all but full.  (Below 384 rows nothing was gained at K 11008.)"""
+    """Whether y[M, N] += x w^T over a long K takes the 256-tile kernel.  It cuts an incomplete last round along K.  The
+    library is a little faster where it chooses well and up to twice as slow where it does not, at sizes that follow no
+    rule: N 4096, K 14336, us, library / this kernel, M 600 96 / 82, 1000 112 / 103, 2050 358 / 230, 2125 202 / 223,
+    3925 299 / 311, 4150 716 / 352, 5050 424 / 420, 6151 810 / 578, 7525 1005 / 634, 7806 604 / 636, 8200 1019 / 682;
+    N 8192, K 28672, M 600 258 / 297, 2050 1284 / 723, 5050 2363 / 1599, 8192 2543 / 2554.  So the kernel is taken where
+    it loses little at worst.  Its time over the library's at 408 sizes (M 400 to 8450, N 2048 to 8192, K 10240 to 28672),
+    geometric mean and worst:
+      up to a third of a round (three pieces of K and more)   0.93  1.08
+      more than one round, the last one cut                   0.73  1.04
+      more than one round, the last one half to 15 / 16 full  0.76  1.08
+      not taken: 86 to 128 tiles 0.94 1.19, to one round 1.03 1.29, full last rounds 1.06 1.09
+    The sizes that lose more than 4 % are N 2048, K 10240 (48 to 80 tiles), M 561 of N 5120 and 6144, K 11008 at M 6035
+    and 7484, N 8192, K 14336 at 7484.  K 8192 gained nothing on average, nor did fewer than 384 rows at K 11008."""
     tiles = -(-M // 256) * (N // 256)
     left = tiles % CUS
     return K >= 10240 and M >= 384 and (3 * tiles <= CUS or (tiles > CUS and 0 < 16 * left < 15 * CUS))
