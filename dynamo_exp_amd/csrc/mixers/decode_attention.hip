@@ -59,8 +59,6 @@ typedef __attribute__((address_space(3))) void lds_void;
 // metadata that no kernel in flight writes: scalar loads
 typedef const __attribute__((address_space(4))) int* scalar_int;
 
-__device__ __forceinline__ int piece_xor(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-template <int RB> __device__ __forceinline__ int image_off(int row, int ch) { return row * RB + 16 * (ch ^ piece_xor(row)); }
 // the wave's own DMA: all but the newest N instructions have landed.  (The builtin, which the compiler counts itself:
 // behind a wait it does not know it would put a full one in front of the next LDS read.)
 template <int N> __device__ __forceinline__ void dma_wait() {

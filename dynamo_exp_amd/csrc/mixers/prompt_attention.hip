@@ -64,10 +64,6 @@ enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(3))) void lds_void;
 
-__device__ __forceinline__ int piece_xor(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-// byte offset of 16-byte piece ch of row `row` in an image whose rows are RB bytes (a multiple of 256)
-template <int RB> __device__ __forceinline__ int image_off(int row, int ch) { return row * RB + 16 * (ch ^ piece_xor(row)); }
-
 // v_max3 / v_max as written: fmaxf() on matrix-core results quiets every operand first
 __device__ __forceinline__ float raw_max3(float a, float b, float c) {
   float r;

@@ -1,5 +1,6 @@
 // Shared by the attention kernels that walk pages of whole 64-key tiles (stream_attention.hip,
-// latent_attention.hip): masks, LDS images of a tile, matrix-core fragments.
+// latent_attention.hip, and with 32-key tiles prompt_attention.hip, decode_attention.hip): masks, LDS images of a tile,
+// matrix-core fragments.
 #pragma once
 #include "recurrent.h"
 
@@ -24,6 +25,11 @@ __device__ __forceinline__ void put_v(bf16_t* Vt, const raw_u32x4* r, int kg, in
     *reinterpret_cast<uint2*>(Vt + voff(8 * ch + 2 * w + 1, pc) + hf) = od;
   }
 }
+
+// row-major images filled by DMA: byte offset of 16-byte piece ch of row `row`, rows of RB bytes (a multiple of 256); the
+// pieces are permuted by row, so that fragment reads and transposed reads both hit different banks
+__device__ __forceinline__ int piece_xor(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+template <int RB> __device__ __forceinline__ int image_off(int row, int ch) { return row * RB + 16 * (ch ^ piece_xor(row)); }
 
 __device__ __forceinline__ bf16x8_t frag16(const bf16_t* p) {
   return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const raw_u32x4*>(p));
