@@ -16,7 +16,8 @@
 // token by token, beside the long ones' chains.
 //
 // P_t shrinks by at most exp(-16 |decay_scale|) in a chunk: 1e-7, and 1 / P 1e7, at the largest the host sends here (1), so
-// that only values within 1e7 of fp32's ends leave its range on the way.  A chunk's dependent chain is 50 matrix instructions and a barrier instead of 16 tokens' chains of lane sums.
+// that only values within 1e7 of fp32's ends leave its range on the way.  A chunk's dependent chain is 50 matrix
+// instructions and a barrier instead of 16 tokens' chains of lane sums.
 // Its rounding: the products of decays come from sums of logarithms in fp64, the sums run in an order that keeps them
 // small and through short chains; relative to 64 bits 1.28e-7 in o and 6.90e-8 in S where the token-by-token form has
 // 1.32e-7 and 6.91e-8 (900 to 4001 tokens; 1.9e-7 and 1.2e-7 with running products and one chain per sum).
@@ -24,10 +25,10 @@
 // factors times it).  It shows in the rows or stays in the state, and a workgroup that meets one takes its columns again,
 // token by token.
 // 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us, each
-// profiled by itself (in a row, with the layer's norm of 35: 443); a prompt of 600 beside 30 single tokens 704 -> 112, the
-// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them
-// at 5250 cycles where three workgroups share a CU, 1088 of them a wave's matrix instructions, which keep the matrix cores
-// busy 41 % of the time; the rest is waiting to issue behind the other workgroups' chains, LDS exchanges and the barrier
+// profiled by itself (in a row, with the layer's norm of 35: 448); a prompt of 600 beside 30 single tokens 704 -> 112, the
+// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 5250 cycles where three
+// workgroups share a CU, 1088 of a wave's matrix instructions each, which keep the matrix cores busy 41 % of the time; the
+// rest is waiting to issue behind the other workgroups' chains, LDS exchanges and the barrier
 // (profiles/step_case_counters.txt).
 #include <algorithm>
 
