@@ -286,8 +286,8 @@ PYBIND11_MODULE(_C_mixers, m) {
                              int n_tiles, int n_qh, int maps, int group, int d, int dv, int Wk, int Wv, float scale,
                              int mask, int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs,
                              int keep, u sink, int out_f32, int fine, u st) {
-    // pages of whole tiles and heads of 128 columns (or one shared row of 256)
-    if (qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && (q | kc | vc | out) % 16 == 0 &&
+    // pages of whole tiles and heads of 128 columns (or one shared row of 256); a tile's bytes are counted in 31 bits
+    if (qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && Wk <= 1 << 23 && Wv <= 1 << 23 && (q | kc | vc | out) % 16 == 0 &&
         dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, kc == vc, cap > 0.f || r1, wfn, out_f32, fine))
       check(dxm_prompt_attention(P(out), P(q), qs, P(kc), P(vc), reinterpret_cast<const int64_t*>(pos),
                                  reinterpret_cast<const int*>(seq), reinterpret_cast<const int*>(bt), bts, bs,

@@ -8,8 +8,12 @@
 // beside another's products (eight waves with one barrier went through both in step, and a last round of workgroups
 // that filled a CU each left a quarter of the card idle).  Products are v_mfma_f32_32x32x16_bf16, swapped (S^T = K Q^T, O^T = V^T P^T), so a query row
 // sits on a lane and the score accumulator is the second product's operand.
-//   * Tiles go from the caches to LDS by DMA (global_load_lds, 16 bytes a lane) into a double buffer; the 16-byte
+//   * Tiles go from the caches to LDS by DMA (buffer loads, 16 bytes a lane) into a double buffer; the 16-byte
 //     pieces of a row are permuted on the source side, so that both kinds of fragment reads below hit different banks.
+//   * Fragments are asked for three or four products ahead and waited for by count.  For that the DMA may not be
+//     global_load_lds, which counts as an LDS access too and makes every wait for an LDS read one for all of them, and
+//     the transposed reads have to say what they read (read_tr16), or each waits for the DMA on its way.  With both, and
+//     every fragment read right in front of its product, the LDS's latency stood before two products of three.
 //   * V^T fragments are read from the row-major image by ds_read_b64_tr_b16: no value passes through registers on
 //     its way in, and where one row is key and value one image serves both products.
 //   * Weights enter the value product as one bf16, or (FINE) as the sum of two.  FINE: the running maximum moves only
@@ -19,13 +23,13 @@
 //     registers.
 //   * Tiles of 64 keys, or of 32 where that lets more workgroups onto a CU: rows of 256 columns, and the forms with
 //     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.
-// What bounds it: vector issue of the softmax beside the matrix cores, score terms most of all (four transcendentals a
-// score with cap and penalty).  Against the register-staged, 16x16x32 forms it took over from (tile_attention.hip,
-// stream and latent prefill), 32 heads, ragged prompts of about 4000 tokens, us: before -> with eight waves -> now: two
-// maps with values of 256 and their combine, window 1024 + 64: 776 -> 303 -> 267; shared row 256 / 192 causal 242 ->
-// 140 -> 124 (800 TFLOP/s), 256 / 256 window 546 -> 124 -> 123; cap + penalty, window 1024: 313 -> 176 -> 138; sigmoid
-// 213 -> 92 -> 86; plain causal, 5000 tokens: 132 -> 124 -> 111, fine 160 -> 148 -> 133; 40 rows behind 2900 cached:
-// 131 -> 117 -> 93.
+// What bounds it: two waves a SIMD in softmax and products in turn (two maps: the matrix cores busy 45 % of the time, 59 %
+// while both waves are there; forming a tile's scores between the weights of the one in front needs 16 registers more
+// than there are, and spills: 1.25 x slower), and vector issue, score terms most of all (four transcendentals a score
+// with cap and penalty).  32 heads, ragged prompts of about 4000 tokens, us, with fragments read one product ahead -> now: two
+// maps with values of 256, window 1024 + 64, 5003 rows: 247 -> 220; shared row 256 / 192 causal 124 -> 113 (870 TFLOP/s);
+// cap + penalty, window 1024: 138 -> 126.  (The register-staged 16x16x32 forms of tile_attention.hip, stream and latent
+// prefill, which it took over from: two maps and their combine 776, 242, 313.)
 #include <type_traits>
 
 #include "stream_attention.h"
@@ -64,6 +68,23 @@ enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(3))) void lds_void;
 
+// (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
+// DMA of the next tile, which goes to the other buffer)
+__device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
+}
+// 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
+// as well, and every wait for an LDS read become one for all of them.)
+__device__ __forceinline__ void dma16(const void* from, int bytes, int off, char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)to,
+                                           16, off, 0, 0, 0);
+}
+// every wave is done with a tile, and the DMA of the next has landed
+__device__ __forceinline__ void landed() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+}
+__device__ __forceinline__ void opaque(int& x) { asm("" : "+v"(x)); }
 // v_max3 / v_max as written: fmaxf() on matrix-core results quiets every operand first
 __device__ __forceinline__ float raw_max3(float a, float b, float c) {
   float r;
@@ -88,6 +109,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   constexpr int kKey = KT * KB, kStage = kKey + (SAME ? 0 : KT * VB);
   constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
+  constexpr int KA = MODE == kPlain ? 4 : 3, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
   constexpr float kDefer = FINE ? 8.f : 0.f;  // log2 units that a score may exceed the running maximum by
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
@@ -119,39 +141,40 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     if (ks < QR) qf[ks < QR ? ks : 0] = f;
     else *reinterpret_cast<bf16x8_t*>(ql + (ks - QR) * 512) = f;
   }
-  // lane constants: fragment addresses (piece 16 and up of a row: + 256 bytes), DMA sources
-  int koff[8], voff_[4][2];
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) koff[ks] = image_off<KB>(r, 2 * ks + h);
-  {
-    const int g16 = (lane >> 4) & 1, qq = (lane & 15) >> 2, pp = lane & 3;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      const int ch = dt * 4 + 2 * g16 + (pp >> 1);
-      voff_[dt][0] = image_off<VB>(4 * h + qq, ch) + 8 * (pp & 1);
-      voff_[dt][1] = image_off<VB>(4 * h + qq + 8, ch) + 8 * (pp & 1);
-    }
-  }
+  // Fragment addresses: step ks of the keys is an XOR with 32 ks away from the first (piece 16 and up of a row: + 256
+  // bytes), block dt of the values one with 64 dt, and the rows 8 further one with 32.
+  const int k_off = image_off<KB>(r, h);
+  const int v_off = image_off<VB>(4 * h + ((lane & 15) >> 2), 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + 8 * (lane & 1);
   const bf16_t* kc = a.kc + (int64_t)gm * D;
   const bf16_t* vc = a.vc + (int64_t)g * DV;
+  // Source of the k-th 1-KB piece of a wave, from the tile's first row.  Rows behind the last query, whose values are stale,
+  // are left out and arrive as zeros.
+  auto source = [&](auto rb, int per_wave, int k, int width) {
+    constexpr int RB = decltype(rb)::value, CH = RB / 16;
+    const int row = (per_wave * wid + k) * (1024 / RB) + lane / CH;
+    return 2 * (row * width + 8 * ((lane % CH) ^ piece_xor(row)));
+  };
+  int ksrc[KP], vsrc[VP ? VP : 1];
+#pragma unroll
+  for (int k = 0; k < KP; ++k) ksrc[k] = source(std::integral_constant<int, KB>{}, KP, k, a.Wk);
+#pragma unroll
+  for (int k = 0; k < VP; ++k) vsrc[k] = source(std::integral_constant<int, VB>{}, VP, k, a.Wv);
+  // 64 entries of the block table at a time, a lane each: a load per tile would be waited for in front of its DMA
+  int page0 = -64, pages = 0;
   auto issue = [&](char* buf, int t) {
-    const int64_t base = tile_slot(bt, a.bs_shift, (t << SH) >> 6) + ((t << SH) & 63);
-    const bf16_t *kb = kc + base * a.Wk, *vb = vc + base * a.Wv;
-    const int left = hi - (t << SH);  // rows behind the last query hold stale values: its row instead
-#pragma unroll
-    for (int k = 0; k < KP; ++k) {
-      constexpr int RP = 1024 / KB, CH = KB / 16;
-      const int row = (KP * wid + k) * RP + lane / CH;
-      __builtin_amdgcn_global_load_lds(kb + (int64_t)min(row, left) * a.Wk + 8 * ((lane % CH) ^ piece_xor(row)),
-                                       (lds_void*)(buf + (KP * wid + k) * 1024), 16, 0, 0);
+    const int j = t << SH, page = j >> a.bs_shift;
+    if (page - page0 >= 64 || page < page0) {
+      page0 = page;
+      pages = bt[min(page + lane, hi >> a.bs_shift)];
     }
+    const int64_t base = ((int64_t)__builtin_amdgcn_readlane(pages, page - page0) << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
+    const int rows = min(hi - j, KT - 1);  // whole rows in front of the last one
 #pragma unroll
-    for (int k = 0; k < VP; ++k) {
-      constexpr int RP = 1024 / VB, CH = VB / 16;
-      const int row = (VP * wid + k) * RP + lane / CH;
-      __builtin_amdgcn_global_load_lds(vb + (int64_t)min(row, left) * a.Wv + 8 * ((lane % CH) ^ piece_xor(row)),
-                                       (lds_void*)(buf + kKey + (VP * wid + k) * 1024), 16, 0, 0);
-    }
+    for (int k = 0; k < KP; ++k)
+      dma16(kc + base * a.Wk, 2 * (rows * a.Wk + D), ksrc[k], buf + (KP * wid + k) * 1024);
+#pragma unroll
+    for (int k = 0; k < VP; ++k)
+      dma16(vc + base * a.Wv, 2 * (rows * a.Wv + DV), vsrc[k], buf + kKey + (VP * wid + k) * 1024);
   };
   const float cap = a.softcap, capl = cap * kLog2e, cape = MODE != kPlain && cap > 0.f ? a.scale * (2.f * kLog2e) / cap : 0.f;
   const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
@@ -163,22 +186,47 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
 #pragma unroll
   for (int i = 0; i < NC; ++i) O[i] = f32x16{};
 
+  auto vread = [&](const char* vb, int v_at, int f) {  // columns 32 (f % NC) .. + 31 of keys 16 (f / NC) .. + 15
+    const char* vp = vb + f / NC * 16 * VB + 256 * (f % NC >> 2);
+    const i16x4 lo = read_tr16((const lds_i16x4*)(vp + (v_at ^ 64 * (f % NC & 3))));
+    const i16x4 up = read_tr16((const lds_i16x4*)(vp + 8 * VB + (v_at ^ 64 * (f % NC & 3) ^ 32)));
+    return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
   auto step = [&](auto bufc, int t) {
     const char* kb = smem + decltype(bufc)::value * kStage;
     const char* vb = SAME ? kb : kb + kKey;
     const int kt = t << SH;
     const bool kept_tile = kt + KT <= keep;  // wholly of kept keys
     if (rw >= n || kt > whi || (kt + KT - 1 < wfirst && kt >= keep)) return;  // nothing the wave's rows see
-    const bool live1 = SUBS == 2 && kt + 32 <= whi;  // some row sees the second half
     f32x16 s[SUBS] = {};
+    int k_at = k_off, v_at = v_off;
+    if constexpr (MODE != kPlain) opaque(k_at), opaque(v_at);  // (three waves a SIMD: no registers to keep them all)
+    {
+      auto kread = [&](int ks, int sub) {
+        return frag16((const bf16_t*)(kb + (k_at ^ 32 * (ks & 7)) + 256 * (ks >> 3) + sub * 32 * KB));
+      };
+      bf16x8_t kf[KA][SUBS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const char* kp = kb + koff[ks & 7] + 256 * (ks >> 3);
-      const bf16x8_t qk = ks < QR ? qf[ks < QR ? ks : 0] : frag16(ql + (ks - QR) * 512);
-      s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)kp), qk, s[0], 0, 0, 0);
-      if constexpr (SUBS == 2)
-        if (live1) s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag16((const bf16_t*)(kp + 32 * KB)), qk, s[1], 0, 0, 0);
+      for (int ks = 0; ks < KA; ++ks)
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub) kf[ks][sub] = kread(ks, sub);
+      __builtin_amdgcn_sched_group_barrier(0x100, KA * SUBS, 0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8_t qk = ks < QR ? qf[ks < QR ? ks : 0] : frag16(ql + (ks - QR) * 512);
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub) {
+          const bf16x8_t f = kf[ks % KA][sub];
+          if (ks + KA < KS) kf[ks % KA][sub] = kread(ks + KA, sub);
+          s[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, qk, s[sub], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, SUBS, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, SUBS + (QR < KS), 0);
+      }
     }
+    bf16x8_t vf[VA];
+#pragma unroll
+    for (int f = 0; f < VA; ++f) vf[f] = vread(vb, v_at, f);
     if (MODE != kPlain && terms) {  // final scores in log2 units
       if (cap > 0.f) {  // cap * tanh(x / cap): tanh(y) = 1 - 2 / (1 + e^(2 y))
 #pragma unroll
@@ -241,53 +289,55 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       }
       m_i = mn;
     }
+    // the weights of 16 keys (group f / NC of the tile) as they enter the product
+    raw_u32x4 ph[2], pl[2];
+    auto weigh = [&](int k16) {
 #pragma unroll
-    for (int sub = 0; sub < SUBS; ++sub) {
-      if (sub == 1 && !live1) break;
+      for (int e = 0; e < 4; ++e) {
+        float w[2];
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        raw_u32x4 ph, pl;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float w[2];
-#pragma unroll
-          for (int x = 0; x < 2; ++x) {
-            const float v = s[sub][8 * s2 + 2 * e + x];
-            if constexpr (MODE == kSigmoid)  // sigmoid(s + bias); an invisible key (s = -inf) weighs 0
-              w[x] = __builtin_amdgcn_rcpf(1.f + fast_exp2(-fmaf(v, sc, hb)));
-            else
-              w[x] = fast_exp2(fmaf(v, sc, -mu));
-          }
-          if constexpr (MODE != kSigmoid) l_i += w[0] + w[1];
-          ph[e] = pack_bf16x2(w[0], w[1]);
-          if constexpr (FINE) pl[e] = pack_bf16x2(w[0] - bf16lo(ph[e]), w[1] - bf16hi(ph[e]));
+        for (int x = 0; x < 2; ++x) {
+          const float v = s[k16 >> 1][8 * (k16 & 1) + 2 * e + x];
+          if constexpr (MODE == kSigmoid)  // sigmoid(s + bias); an invisible key (s = -inf) weighs 0
+            w[x] = __builtin_amdgcn_rcpf(1.f + fast_exp2(-fmaf(v, sc, hb)));
+          else
+            w[x] = fast_exp2(fmaf(v, sc, -mu));
         }
-#pragma unroll
-        for (int dt = 0; dt < NC; ++dt) {
-          const char* vp = vb + sub * 32 * VB + s2 * 16 * VB + 256 * (dt >> 2);
-          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[dt & 3][0]));
-          const i16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[dt & 3][1]));
-          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
-          O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, ph), O[dt], 0, 0, 0);
-          if constexpr (FINE)
-            O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, pl), O[dt], 0, 0, 0);
-        }
+        if constexpr (MODE != kSigmoid) l_i += w[0] + w[1];
+        ph[k16 & 1][e] = pack_bf16x2(w[0], w[1]);
+        if constexpr (FINE) pl[k16 & 1][e] = pack_bf16x2(w[0] - bf16lo(ph[k16 & 1][e]), w[1] - bf16hi(ph[k16 & 1][e]));
       }
+    };
+    constexpr int NF = 2 * SUBS * NC;  // value fragments of the tile
+    weigh(0);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const int k16 = f / NC, dt = f % NC;
+      // (blocks of rows behind one another: what the later rows' own values hold must not meet this one's zero weights)
+      if (RT > 1 && SUBS == 2 && f == NF / 2 && kt + 32 > whi) break;
+      if (dt == 0 && k16 + 1 < 2 * SUBS) weigh(k16 + 1);
+      const bf16x8_t cur = vf[f % VA];
+      if (f + VA < NF) vf[f % VA] = vread(vb, v_at, f + VA);
+      O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, __builtin_bit_cast(bf16x8_t, ph[k16 & 1]), O[dt], 0, 0, 0);
+      if constexpr (FINE)
+        O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur, __builtin_bit_cast(bf16x8_t, pl[k16 & 1]), O[dt], 0, 0, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, FINE ? 2 : 1, 0);
+      if (f + VA < NF) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
   };
   // tiles in order: the kept ones, then the window's
   const int total = kept + last - first + 1;
   auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
   issue(smem, tile(0));
-  __syncthreads();  // (waits for the DMA of the tile as well)
+  landed();
   for (int i = 0; i < total; i += 2) {
     if (i + 1 < total) issue(smem + kStage, tile(i + 1));
     step(std::integral_constant<int, 0>{}, tile(i));
-    __syncthreads();
+    landed();
     if (i + 1 < total) {
       if (i + 2 < total) issue(smem, tile(i + 2));
       step(std::integral_constant<int, 1>{}, tile(i + 1));
-      __syncthreads();
+      landed();
     }
   }
 

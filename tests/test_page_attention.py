@@ -244,3 +244,45 @@ def test_decode_rows_of_long_contexts(form, mask, size, keep):
         err, top = float((got - want).abs().max()), float(want.abs().max())
         # as test_decode_rows: weights as two bf16 numbers, 2^-17 of sum w |v|
         assert err < 3e-4 * (max(top, 1.0) if sig else 1.0), (bs, parts, err, top)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,mask,size,keep", [("plain", "causal", 0, 0), ("fine", "window", 4500, 70),
+                                                 ("diff", "window", 4300, 64), ("shared", "chunk", 4200, 0),
+                                                 ("both", "window", 130, 4100)])
+def test_prompt_rows_behind_many_pages(form, mask, size, keep):
+    """More pages than lanes of a wave, tables that are read a second time in the middle of a row's keys (and, with
+    kept keys, go back to the front)."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(5)
+    scale, start, rows, bs = 0.7 * d ** -0.5, 4470, 97, 64
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    kd, vd, table, kv = pages(form, [start + rows], bs)
+    q = torch.randn(rows, n_qh * d).bfloat16()
+    want = dense(q.double().view(rows, n_qh, d), *kv[0], torch.arange(start, start + rows), scale, mask, size, keep, cap, db,
+                 sink, sig, hb)
+    tiles = torch.tensor(mx.tile_list(0, rows), dtype=torch.int32).cuda()
+    out_f32 = form.startswith("diff")
+    got = mx.attention(q.cuda(), kd, vd, torch.arange(start, start + rows).cuda(), torch.zeros(rows, dtype=torch.int32).cuda(),
+                       table, bs, n_qh, maps, group, d, dv, scale, mask, size, 1, out_f32, tiles, rows, softcap=cap,
+                       dist_bias=None if db is None else tuple(map(cuda, db)), head_bias=cuda(hb), keep_first=keep,
+                       sink=cuda(sink), fine_weights=form == "fine").cpu().double()
+    err = float((got - want).abs().max())  # (bounds of test_prompt_rows)
+    assert err < (3e-4 if out_f32 else 2.0 ** -8 * (float(want.abs().max()) + 5.0)), err
+
+
+@pytest.mark.gpu
+def test_later_rows_values_that_are_not_finite():
+    """Two blocks of 32 rows in a workgroup and tiles of 64 keys: an infinite value of the second block's rows is none of
+    the first block's."""
+    n_qh, maps, group, d, dv = FORMS["plain pair"]
+    torch.manual_seed(6)
+    kd, vd, table, kv = pages("plain pair", [64], 64)
+    vd[int(table[0, 0]) * 64 + 40] = float("inf")
+    q = torch.randn(64, n_qh * d).bfloat16()
+    want = dense(q.double().view(64, n_qh, d), *kv[0], torch.arange(64), d ** -0.5, "causal", 0, 0, 0.0, None, None, False,
+                 None)[:32]
+    tiles = torch.tensor(mx.tile_list(0, 64), dtype=torch.int32).cuda()
+    got = mx.attention(q.cuda(), kd, vd, torch.arange(64).cuda(), torch.zeros(64, dtype=torch.int32).cuda(), table, 64, n_qh,
+                       maps, group, d, dv, d ** -0.5, "causal", 0, 1, False, tiles, 64).cpu().double()[:32]
+    assert float((got - want).abs().max()) < 2.0 ** -8 * (float(want.abs().max()) + 5.0)
