@@ -7,15 +7,23 @@
 //     32-row K sub-blocks that lie entirely above a wave's causal diagonal are
 //     skipped (no MFMA, no softmax work);
 //   * K/V tiles of 64 tokens are gathered from the paged cache (block table)
-//     by LDS-DMA (global_load_lds_dwordx4, no staging registers) into a
-//     double-buffered, XOR-swizzled LDS image (the swizzle is chosen on the
-//     source side), the next tile in flight while the current one computes;
+//     by LDS-DMA (16-byte buffer loads, no staging registers; rows past the
+//     context arrive as zeros) into a double-buffered, XOR-swizzled LDS image
+//     (the swizzle is chosen on the source side), the next tile in flight
+//     while the current one computes;
 //   * S^T = K . Q^T ("swapped" product): the query row sits on the lane, so the
 //     online softmax is lane-local (+1 cross-half exchange) and the S
 //     accumulator is directly the B operand of the P.V product
 //     O^T = V^T . P^T (guide section 3, "accumulator tile as next operand");
 //   * V^T fragments come from the same swizzled image via ds_read_b64_tr_b16
-//     (guide T10), K fragments via ds_read_b128; both conflict-free.
+//     (guide T10), K fragments via ds_read_b128; both conflict-free;
+//   * fragments are asked for four products ahead and waited for by count.
+//     With global_load_lds, which the compiler counts as an LDS access too, and
+//     transposed reads that do not say what they read, each was waited for
+//     right in front of its product (and the first of a tile's values for the
+//     next tile's DMA): 32 / 8 heads, us, then -> now: two prompts of 5000
+//     tokens together 132 -> 123, one of 2000 53.5 -> 48.6, 300 rows behind
+//     2900 cached 71 -> 65, six of 3000 with 16 / 4 heads 26.1 -> 24.4.
 //
 // Q is read straight from the fused QKV buffer (row stride q_stride) after the
 // rope kernel rotated it in place; the new tokens' K/V are already in the paged
@@ -32,16 +40,34 @@ constexpr int BKV = 64;  // kv rows per tile
 constexpr int kTileBytes = BKV * D * 2;  // 16 KiB
 
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 // byte offset of 16-B chunk `ch` (0..15) of row `row` inside a [64][128] bf16 tile
 __device__ __forceinline__ int tile_off(int row, int ch) { return row * 256 + 16 * (ch ^ swz(row)); }
 
+// (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
+// DMA of the next tile, which goes to the other buffer)
+__device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
+}
+// 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
+// as well, and every wait for an LDS read become one for all of them.)
+__device__ __forceinline__ void dma16(const void* from, int bytes, int off, char* to) {
+  typedef __attribute__((address_space(3))) void lds_void;
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)to,
+                                           16, off, 0, 0, 0);
+}
+// every wave is done with a tile, and the DMA of the next has landed
+__device__ __forceinline__ void landed() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+}
 __device__ __forceinline__ bf16x8_t as_frag(const u16x8& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
 // ---------------------------------------------------------------------------
 // The kernel: NW waves (8: 4 heads x 64 query tokens per workgroup sharing each
-// K/V tile; 4: 32 tokens), K/V staged by LDS-DMA (global_load_lds) into a double-buffered
+// K/V tile; 4: 32 tokens), K/V staged by LDS-DMA into a double-buffered
 // swizzled image, with the per-tile vector work cut down -- the loop is
 // issue-bound, not MFMA-bound, at 2 waves/SIMD.  (Earlier register-staged
 // 4/8-wave, 4-wave x 2 q-block and 3-stage-DMA variants measured 322-794
@@ -52,8 +78,8 @@ __device__ __forceinline__ bf16x8_t as_frag(const u16x8& v) { return __builtin_b
 //     depends on row bits 0..3, so +32 rows / +16 rows / the other buffer are
 //     immediate offsets): the loop is unrolled over the two buffers;
 //   * with block_size >= 64 a full tile lies in one KV block, so the DMA source
-//     is a scalar base (one scalar block-table load) + a per-lane constant;
-//     only the context's last tile takes the clamped per-lane path;
+//     is a scalar base (from 64 block-table entries in a register) + a
+//     per-lane constant;
 //   * masking only on diagonal / ragged tiles, by select (no branches);
 //     softmax with the scale folded into the FMA; the row
 //     max as two v_max3 chains; the row sum l as ones . P^T on the matrix
@@ -113,18 +139,19 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
   // a global longest-first schedule -- and consecutive workgroups land on
   // consecutive XCDs, i.e. with 8 KV-head groups each XCD's L2 serves one KV
   // head's tiles for all work items.
-  const int kvh = blockIdx.x / head_groups;
+  const int kvh = __builtin_amdgcn_readfirstlane(blockIdx.x / head_groups);
   const int hg = blockIdx.x % head_groups;
   const int token_tiles = NW / heads_per_wg;
   // a work item is the rows of eight waves; its later rows see more keys and go first
   const int item = blockIdx.y / (8 / NW), sub = 8 / NW - 1 - blockIdx.y % (8 / NW);
-  const int seq = work[2 * item];
-  const int tok0 = work[2 * item + 1] + sub * token_tiles * BQ;
+  // (the same for every lane, and known as such: a descriptor in vector registers would be read out lane by lane)
+  const int seq = __builtin_amdgcn_readfirstlane(work[2 * item]);
+  const int tok0 = __builtin_amdgcn_readfirstlane(work[2 * item + 1]) + sub * token_tiles * BQ;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int q_start = cu_seqlens_q[seq];
-  const int qlen = cu_seqlens_q[seq + 1] - q_start;
-  const int ctx = ctx_lens[seq];
+  const int q_start = __builtin_amdgcn_readfirstlane(cu_seqlens_q[seq]);
+  const int qlen = __builtin_amdgcn_readfirstlane(cu_seqlens_q[seq + 1]) - q_start;
+  const int ctx = __builtin_amdgcn_readfirstlane(ctx_lens[seq]);
   const int pos0 = ctx - qlen;
   if (tok0 >= qlen) return;
   const int r = lane & 31, h = lane >> 5;
@@ -167,37 +194,40 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
   constexpr int KPW = 16 / NW;  // 1-KB pieces of a 16-KB K (or V) tile per wave
   const int* bt = block_tables + (int64_t)seq * bt_stride;
   const int64_t head_stride = (int64_t)block_size * D;
-  int src_row[KPW], src_off[KPW];
+  int src_off[KPW];  // bytes from the tile's first row
 #pragma unroll
   for (int k = 0; k < KPW; ++k) {
     const int row = (KPW * wid + k) * 4 + (lane >> 4);
-    src_row[k] = row;
-    src_off[k] = row * D + ((lane & 15) ^ swz(row)) * 8;
+    src_off[k] = 2 * (row * D + ((lane & 15) ^ swz(row)) * 8);
   }
-  typedef __attribute__((address_space(3))) void lds_void;
-  auto dma = [&](const bf16_t* g, char* l) { __builtin_amdgcn_global_load_lds(g, (lds_void*)l, 16, 0, 0); };
-  auto issue = [&](char* kb, int j0) {
+  // 64 entries of the block table at a time, a lane each: a load per tile would be waited for in front of its DMA
+  int page0 = -64, pages = 0;
+  const int last_page = (ctx - 1) >> bs_shift;
+  auto block = [&](int j) __attribute__((always_inline)) {  // the first of 64 keys' block, or a later one of theirs
+    return __builtin_amdgcn_readlane(pages, min(j >> bs_shift, last_page) - page0);
+  };
+  auto issue = [&](char* kb, int j0) __attribute__((always_inline)) {
     char* vb = kb + kTileBytes;
-    if (BS64 && j0 + BKV <= ctx) {
-      const int blk = bt[j0 >> bs_shift];  // uniform -> scalar load
-      const int64_t base = ((int64_t)blk * n_kv_heads + kvh) * head_stride + (int64_t)(j0 & (block_size - 1)) * D;
+    if (min((j0 + BKV - 1) >> bs_shift, last_page) - page0 >= 64) {
+      page0 = j0 >> bs_shift;
+      pages = bt[min(page0 + lane, last_page)];
+    }
+    if (BS64) {  // one block; rows past the context arrive as zeros
+      const int64_t base = ((int64_t)block(j0) * n_kv_heads + kvh) * head_stride + (int64_t)(j0 & (block_size - 1)) * D;
+      const int bytes = 2 * D * min(ctx - j0, BKV);
 #pragma unroll
       for (int k = 0; k < KPW; ++k) {
-        dma(k_cache + base + src_off[k], kb + (KPW * wid + k) * 1024);
-        dma(v_cache + base + src_off[k], vb + (KPW * wid + k) * 1024);
+        dma16(k_cache + base, bytes, src_off[k], kb + (KPW * wid + k) * 1024);
+        dma16(v_cache + base, bytes, src_off[k], vb + (KPW * wid + k) * 1024);
       }
     } else {
 #pragma unroll
-      for (int k = 0; k < KPW; ++k) {
-        // rows past the context read row ctx-1 (finite); a wave's 4-row group
-        // (block_size % 4 == 0) lies in one KV block, so the block-table read is
-        // wave-uniform (a scalar load) even with the clamp
-        const int j = min(j0 + src_row[k], ctx - 1);
-        const int blk = bt[min(j0 + 4 * (KPW * wid + k), ctx - 1) >> bs_shift];
-        const int64_t o = ((int64_t)blk * n_kv_heads + kvh) * head_stride + (int64_t)(j & (block_size - 1)) * D +
-                          (src_off[k] - src_row[k] * D);
-        dma(k_cache + o, kb + (KPW * wid + k) * 1024);
-        dma(v_cache + o, vb + (KPW * wid + k) * 1024);
+      for (int k = 0; k < KPW; ++k) {  // a piece's four rows lie in one block (block_size % 4 == 0)
+        const int at = 4 * (KPW * wid + k), j = __builtin_amdgcn_readfirstlane(j0 + at);
+        const int64_t base = ((int64_t)block(j) * n_kv_heads + kvh) * head_stride + (int64_t)(j & (block_size - 1)) * D;
+        const int bytes = __builtin_amdgcn_readfirstlane(2 * D * max(min(ctx - j, 4), 0));
+        dma16(k_cache + base, bytes, src_off[k] - 2 * D * at, kb + (KPW * wid + k) * 1024);
+        dma16(v_cache + base, bytes, src_off[k] - 2 * D * at, vb + (KPW * wid + k) * 1024);
       }
     }
   };
@@ -210,26 +240,45 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
   const bf16x8_t kOnes = __builtin_bit_cast(bf16x8_t, u16x8{{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}});
   const f32x2 sc2 = {scale_log2e, scale_log2e};
 
+  constexpr int kAhead = 4;  // fragments asked for ahead of their products
+  auto vread = [&](const char* vb, int i) __attribute__((always_inline)) {  // columns 32 (i % 4) .. + 31 of keys 16 (i / 4) .. + 15
+    const i16x4 lo = read_tr16((const lds_i16x4*)(vb + i / 4 * 4096 + voff[i % 4][0]));
+    const i16x4 hi = read_tr16((const lds_i16x4*)(vb + i / 4 * 4096 + voff[i % 4][1]));
+    return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
   // segment 1 of a tile: S^T = K . Q^T, mask, online softmax -> this wave's
   // bf16 P fragments (and the O / l rescale); false: nothing of the tile is
   // at or below this wave's diagonal
-  auto qk_sm = [&](const char* kb, int t, u16x8 (&pf)[2][2], bool& live1) -> bool {
+  auto qk_sm = [&](const char* kb, int t, u16x8 (&pf)[2][2], bool& live1, bf16x8_t (&vf)[kAhead]) __attribute__((always_inline)) -> bool {
     const int j0 = t * BKV;
     live1 = j0 + 32 <= wave_max_pos;
     if (j0 > wave_max_pos) return false;
     f32x16 s0 = f32x16{}, s1 = f32x16{};
+    bf16x8_t kf[kAhead];
+    auto kread = [&](int i) __attribute__((always_inline)) { return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4*>(kb + 8192 * (i >> 3) + koff[i & 7])); };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) kf[i] = kread(i);
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      const u16x8 kf = *reinterpret_cast<const u16x8*>(kb + koff[ks]);
-      s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf), as_frag(qf[ks]), s0, 0, 0, 0);
+      const bf16x8_t f = kf[ks % kAhead];
+      kf[ks % kAhead] = kread(ks + kAhead);
+      s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, as_frag(qf[ks]), s0, 0, 0, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
     if (live1) {
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) {
-        const u16x8 kf = *reinterpret_cast<const u16x8*>(kb + 8192 + koff[ks]);
-        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf), as_frag(qf[ks]), s1, 0, 0, 0);
+        const bf16x8_t f = kf[ks % kAhead];
+        if (ks + kAhead < 8) kf[ks % kAhead] = kread(8 + ks + kAhead);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, as_frag(qf[ks]), s1, 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (ks + kAhead < 8) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
     }
+#pragma unroll
+    for (int f = 0; f < kAhead; ++f) vf[f] = vread(kb + kTileBytes, f);
     if ((j0 + BKV - 1 > wave_min_pos) || (j0 + BKV > ctx)) {  // diagonal / ragged tile
       const int lim = min(my_pos, ctx - 1) - j0 - 4 * h;  // keep kv row j0 + 4h + off <= lim + j0 + 4h
 #pragma unroll
@@ -297,49 +346,45 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
     return true;
   };
   // segment 2: O^T += V^T . P^T (+ l on the matrix pipe)
-  auto pv = [&](const char* vb, bool live1, const u16x8 (&pf)[2][2]) {
+  auto pv = [&](const char* vb, bool live1, const u16x8 (&pf)[2][2], bf16x8_t (&vf)[kAhead]) __attribute__((always_inline)) {
     // O^T[d][q] += V^T[d][kv] . P^T[kv][q]
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
-      if (sub == 1 && !live1) break;
+      if (sub == 0 || live1) {
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_i16x4*)(vb + sub * 8192 + s2 * 4096 + voff[dt][0]));
-          const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_i16x4*)(vb + sub * 8192 + s2 * 4096 + voff[dt][1]));
-          typedef short i16x8 __attribute__((ext_vector_type(8)));
-          const i16x8 vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv),
-                                                              as_frag(pf[sub][s2]), o_acc[dt], 0, 0, 0);
+        for (int i = 8 * sub; i < 8 * sub + 8; ++i) {
+          const bf16x8_t p = as_frag(pf[sub][(i >> 2) & 1]), f = vf[i % kAhead];
+          if (i + kAhead < 16) vf[i % kAhead] = vread(vb, i + kAhead);
+          o_acc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, p, o_acc[i & 3], 0, 0, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (i + kAhead < 16) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          // l += ones . P^T: the row sum of exactly the bf16 P the P.V product
+          // used (O / l stays an exact weighted mean of V rows under the
+          // deferred max), on the matrix pipe instead of 16 packed adds + a
+          // cross-half exchange on the issue-bound VALU
+          if constexpr (kMfmaSum)
+            if ((i & 3) == 3) l_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kOnes, p, l_acc, 0, 0, 0);
         }
-        // l += ones . P^T: the row sum of exactly the bf16 P the P.V product
-        // used (O / l stays an exact weighted mean of V rows under the
-        // deferred max), on the matrix pipe instead of 16 packed adds + a
-        // cross-half exchange on the issue-bound VALU
-        if constexpr (kMfmaSum)
-          l_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kOnes, as_frag(pf[sub][s2]), l_acc, 0, 0, 0);
       }
     }
   };
 
   {
-    auto step = [&](auto bufc, int t) {
+    auto step = [&](auto bufc, int t) __attribute__((always_inline)) {
       constexpr int BUF = decltype(bufc)::value;
       char* kb = smem + BUF * kBuf;
       if (t + 1 < n_tiles) issue(smem + (BUF ^ 1) * kBuf, t * BKV + BKV);
       u16x8 pf[2][2];
+      bf16x8_t vf[kAhead];
       bool live1;
-      if (qk_sm(kb, t, pf, live1)) pv(kb + kTileBytes, live1, pf);
-      __syncthreads();  // the compiler's vmcnt(0) here retires this wave's DMA of tile t+1
+      if (qk_sm(kb, t, pf, live1, vf)) pv(kb + kTileBytes, live1, pf, vf);
+      landed();
     };
     if (n_tiles > 0) issue(smem, 0);
     // static priority for the second-dispatched half (guide "Two waves per
     // SIMD" item 4): without it waves 4-7 lose every arbitration
     if (NW == 8 && V != 0 && wid >= 4) __builtin_amdgcn_s_setprio(1);
-    __syncthreads();
+    landed();
     for (int t = 0; t < n_tiles; t += 2) {
       step(std::integral_constant<int, 0>{}, t);
       if (t + 1 < n_tiles) step(std::integral_constant<int, 1>{}, t + 1);
