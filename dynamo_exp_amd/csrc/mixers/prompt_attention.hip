@@ -23,13 +23,18 @@
 //     registers.
 //   * Tiles of 64 keys, or of 32 where that lets more workgroups onto a CU: rows of 256 columns, and the forms with
 //     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.
-// What bounds it: two waves a SIMD in softmax and products in turn (two maps: the matrix cores busy 45 % of the time, 59 %
-// while both waves are there; forming a tile's scores between the weights of the one in front needs 16 registers more
-// than there are, and spills: 1.25 x slower), and vector issue, score terms most of all (four transcendentals a score
-// with cap and penalty).  32 heads, ragged prompts of about 4000 tokens, us, with fragments read one product ahead -> now: two
-// maps with values of 256, window 1024 + 64, 5003 rows: 247 -> 220; shared row 256 / 192 causal 124 -> 113 (870 TFLOP/s);
-// cap + penalty, window 1024: 138 -> 126.  (The register-staged 16x16x32 forms of tile_attention.hip, stream and latent
-// prefill, which it took over from: two maps and their combine 776, 242, 313.)
+//   * Between the products of a tile's scores the next tile's DMA goes out; all four waves' at once behind the barrier
+//     stood in each other's way.
+//   * Score terms: the tanh cap is a polynomial of degree 7 where a tile's scores are small against the cap (|x / cap| <
+//     0.36, relative error 4.3e-8; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
+//     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.
+// What bounds it: two waves a SIMD in softmax and products in turn (two maps: the matrix cores busy 45 % of the time;
+// forming a tile's scores between the weights of the one in front needs 16 registers more than there are, and spills:
+// 1.25 x slower), and a wave's issue where there are score terms.  32 heads, ragged prompts of about 4000 tokens, us,
+// with fragments read one product ahead -> now: two maps with values of 256, window 1024 + 64, 5003 rows beside 16 decode
+// rows, with the combine: 287 -> 270; shared row 256 / 192 causal 124 -> 113 (870 TFLOP/s); cap + penalty, window 1024,
+// 138 -> 99 (600 rows behind 2000 cached, window 512: 33 -> 27); sigmoid 86 -> 81.  (The register-staged 16x16x32 forms
+// of tile_attention.hip, stream and latent prefill, which it took over from: two maps and their combine 776, 242, 313.)
 #include <type_traits>
 
 #include "stream_attention.h"
@@ -63,10 +68,21 @@ struct PromptArgs {
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
-enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
+// kTable: cap and / or penalty where a row sees at most kTableKeys keys back: the penalty is a table of the distance in LDS
+enum { kPlain = 0, kTerms = 1, kSigmoid = 2, kTable = 3 };
+constexpr int kTableKeys = 1216;  // what three workgroups of a CU have room for beside their tiles
+constexpr int kTablePad = 64;     // entries for keys of a tile that a row does not see, on both sides
+
+// tanh(y) / y = sum kTanh[i] y^(2 i) for |y| <= kTanhMax, relative error 4.3e-8 (minimax, fitted in 64 bits)
+constexpr float kTanhMax = 0.36f;
+constexpr float kTanh[4] = {0.99999996f, -0.33332261f, 0.13291534f, -0.04868792f};
 
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(3))) void lds_void;
+// LDS by its own addresses: through a pointer each would be added to the array's (the front of LDS) in a vector instruction
+typedef __attribute__((address_space(3))) raw_u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) float lds_float;
+__device__ __forceinline__ bf16x8_t lds_frag(uint32_t at) { return __builtin_bit_cast(bf16x8_t, *(const lds_u32x4*)(uintptr_t)at); }
 
 // (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
 // DMA of the next tile, which goes to the other buffer)
@@ -75,8 +91,8 @@ __device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
 }
 // 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
 // as well, and every wait for an LDS read become one for all of them.)
-__device__ __forceinline__ void dma16(const void* from, int bytes, int off, char* to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)to,
+__device__ __forceinline__ void dma16(const void* from, int bytes, int off, uint32_t to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)(uintptr_t)to,
                                            16, off, 0, 0, 0);
 }
 // every wave is done with a tile, and the DMA of the next has landed
@@ -91,6 +107,13 @@ __device__ __forceinline__ float raw_max3(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+__device__ __forceinline__ float raw_max3_abs(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// a number that is the same in every lane, in a scalar register
+__device__ __forceinline__ float uniform(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
 __device__ __forceinline__ float swap_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
@@ -110,6 +133,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
   constexpr int KA = MODE == kPlain ? 4 : 3, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
+  constexpr bool kEager = MODE == kTerms || MODE == kTable;
   constexpr float kDefer = FINE ? 8.f : 0.f;  // log2 units that a score may exceed the running maximum by
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
@@ -134,17 +158,18 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   const int wfirst = first_key(wlo, a.mask, a.size), wlast = first_key(whi, a.mask, a.size);
   const int keep = a.mask == 1 ? a.keep : 0;
   bf16x8_t qf[QR];
-  bf16_t* ql = reinterpret_cast<bf16_t*>(smem + 2 * kStage) + (wid * (KS - QR) * 64 + lane) * 8;  // the lane's own pieces
+  const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)smem;
+  const uint32_t ql = base + 2 * kStage + (wid * (KS - QR) * 64 + lane) * 16;  // the lane's own pieces
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const bf16x8_t f = frag16(a.q + (int64_t)(row0 + myrow) * a.q_stride + (int64_t)qh * D + 16 * ks + 8 * h);
     if (ks < QR) qf[ks < QR ? ks : 0] = f;
-    else *reinterpret_cast<bf16x8_t*>(ql + (ks - QR) * 512) = f;
+    else *(lds_u32x4*)(uintptr_t)(ql + (ks - QR) * 1024) = __builtin_bit_cast(raw_u32x4, f);
   }
   // Fragment addresses: step ks of the keys is an XOR with 32 ks away from the first (piece 16 and up of a row: + 256
   // bytes), block dt of the values one with 64 dt, and the rows 8 further one with 32.
-  const int k_off = image_off<KB>(r, h);
-  const int v_off = image_off<VB>(4 * h + ((lane & 15) >> 2), 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + 8 * (lane & 1);
+  const int k_off = base + image_off<KB>(r, h);
+  const int v_off = base + image_off<VB>(4 * h + ((lane & 15) >> 2), 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + 8 * (lane & 1);
   const bf16_t* kc = a.kc + (int64_t)gm * D;
   const bf16_t* vc = a.vc + (int64_t)g * DV;
   // Source of the k-th 1-KB piece of a wave, from the tile's first row.  Rows behind the last query, whose values are stale,
@@ -161,24 +186,44 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   for (int k = 0; k < VP; ++k) vsrc[k] = source(std::integral_constant<int, VB>{}, VP, k, a.Wv);
   // 64 entries of the block table at a time, a lane each: a load per tile would be waited for in front of its DMA
   int page0 = -64, pages = 0;
-  auto issue = [&](char* buf, int t) {
+  // where the next tile lies: found in front of a tile's scores, its DMA goes out between their products (all four waves'
+  // at once behind the barrier stood in each other's way)
+  const bf16_t *knext = kc, *vnext = vc;
+  int kbytes = 0, vbytes = 0;
+  auto find = [&](int t) {
     const int j = t << SH, page = j >> a.bs_shift;
     if (page - page0 >= 64 || page < page0) {
       page0 = page;
       pages = bt[min(page + lane, hi >> a.bs_shift)];
     }
-    const int64_t base = ((int64_t)__builtin_amdgcn_readlane(pages, page - page0) << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
+    const uint32_t slot = ((uint32_t)__builtin_amdgcn_readlane(pages, page - page0) << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
     const int rows = min(hi - j, KT - 1);  // whole rows in front of the last one
-#pragma unroll
-    for (int k = 0; k < KP; ++k)
-      dma16(kc + base * a.Wk, 2 * (rows * a.Wk + D), ksrc[k], buf + (KP * wid + k) * 1024);
-#pragma unroll
-    for (int k = 0; k < VP; ++k)
-      dma16(vc + base * a.Wv, 2 * (rows * a.Wv + DV), vsrc[k], buf + kKey + (VP * wid + k) * 1024);
+    knext = kc + (uint64_t)slot * (uint32_t)a.Wk;
+    kbytes = 2 * (rows * a.Wk + D);
+    vnext = vc + (uint64_t)slot * (uint32_t)a.Wv;
+    vbytes = 2 * (rows * a.Wv + DV);
   };
-  const float cap = a.softcap, capl = cap * kLog2e, cape = MODE != kPlain && cap > 0.f ? a.scale * (2.f * kLog2e) / cap : 0.f;
+  auto fetch = [&](uint32_t buf, int k) {
+    if (k < KP) dma16(knext, kbytes, ksrc[k < KP ? k : 0], buf + (KP * wid + k) * 1024);
+    else dma16(vnext, vbytes, vsrc[k < KP ? 0 : k - KP], buf + kKey + (VP * wid + k - KP) * 1024);
+  };
+  constexpr int ND = KP + VP;  // DMA instructions of a wave and tile
+  const int table_len = a.size + 2 * kTablePad;  // kTable: floats per head, entry kTablePad + d is the penalty at distance d
+  const uint32_t table = base + 2 * kStage + (wid % HPW) * table_len * 4;  // of the wave's head
+  if constexpr (MODE == kTable) {  // the waves of a head share its table
+    const float p1 = a.r1[qh], p2 = a.r2[qh];
+    for (int i = lane + 64 * (wid / HPW); i < table_len; i += 64 * RT)
+      *(lds_float*)(uintptr_t)(table + 4 * i) = i >= kTablePad ? p1 * __builtin_amdgcn_logf(fmaf(p2, (float)(i - kTablePad), 1.f)) : 0.f;
+  }
+  const float cap = a.softcap, capl = uniform(cap * kLog2e);
+  const float cape = uniform(MODE != kPlain && cap > 0.f ? a.scale * (2.f * kLog2e) / cap : 0.f);
   const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
-  const float r1 = MODE != kPlain && a.r1 ? a.r1[qh] : 0.f, r2 = MODE != kPlain && a.r1 ? a.r2[qh] : 0.f;
+  // the polynomial on scores as the product leaves them, and how far it holds
+  const float y1 = terms && cap > 0.f ? a.scale / cap : 0.f, y2 = y1 * y1, near = uniform(y1 > 0.f ? kTanhMax / y1 : 0.f);
+  const float t0 = uniform(a.scale * kLog2e * kTanh[0]), t1 = uniform(a.scale * kLog2e * kTanh[1] * y2),
+              t2 = uniform(a.scale * kLog2e * kTanh[2] * y2 * y2), t3 = uniform(a.scale * kLog2e * kTanh[3] * y2 * y2 * y2);
+  const bool logs = MODE != kPlain && MODE != kTable && a.r1;
+  const float r1 = uniform(logs ? a.r1[qh] : 0.f), r2 = uniform(logs ? a.r2[qh] : 0.f);
   const float sc = terms ? 1.f : a.scale * kLog2e;  // scores to log2 units
   const float hb = MODE == kSigmoid && a.hbias ? a.hbias[qh] * kLog2e : 0.f;
   float m_i = -INFINITY, l_i = 0.f;
@@ -186,24 +231,28 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
 #pragma unroll
   for (int i = 0; i < NC; ++i) O[i] = f32x16{};
 
-  auto vread = [&](const char* vb, int v_at, int f) {  // columns 32 (f % NC) .. + 31 of keys 16 (f / NC) .. + 15
-    const char* vp = vb + f / NC * 16 * VB + 256 * (f % NC >> 2);
-    const i16x4 lo = read_tr16((const lds_i16x4*)(vp + (v_at ^ 64 * (f % NC & 3))));
-    const i16x4 up = read_tr16((const lds_i16x4*)(vp + 8 * VB + (v_at ^ 64 * (f % NC & 3) ^ 32)));
+  auto vread = [&](uint32_t vb, int v_at, int f) {  // columns 32 (f % NC) .. + 31 of keys 16 (f / NC) .. + 15
+    const uint32_t vp = vb + f / NC * 16 * VB + 256 * (f % NC >> 2);
+    const i16x4 lo = read_tr16((const lds_i16x4*)(uintptr_t)(vp + (v_at ^ 64 * (f % NC & 3))));
+    const i16x4 up = read_tr16((const lds_i16x4*)(uintptr_t)(vp + 8 * VB + (v_at ^ 64 * (f % NC & 3) ^ 32)));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
   };
   auto step = [&](auto bufc, int t) {
-    const char* kb = smem + decltype(bufc)::value * kStage;
-    const char* vb = SAME ? kb : kb + kKey;
+    constexpr uint32_t kb = decltype(bufc)::value * kStage, vb = SAME ? kb : kb + kKey;  // from the front
+    constexpr uint32_t other = (1 - decltype(bufc)::value) * kStage;                     // the next tile's
     const int kt = t << SH;
     const bool kept_tile = kt + KT <= keep;  // wholly of kept keys
-    if (rw >= n || kt > whi || (kt + KT - 1 < wfirst && kt >= keep)) return;  // nothing the wave's rows see
+    if constexpr (RT > 1) {
+#pragma unroll
+      for (int k = 0; k < ND; ++k) fetch(base + other, k);
+      if (rw >= n || kt > whi || (kt + KT - 1 < wfirst && kt >= keep)) return;  // nothing the wave's rows see
+    }
     f32x16 s[SUBS] = {};
     int k_at = k_off, v_at = v_off;
     if constexpr (MODE != kPlain) opaque(k_at), opaque(v_at);  // (three waves a SIMD: no registers to keep them all)
     {
       auto kread = [&](int ks, int sub) {
-        return frag16((const bf16_t*)(kb + (k_at ^ 32 * (ks & 7)) + 256 * (ks >> 3) + sub * 32 * KB));
+        return lds_frag((k_at ^ 32 * (ks & 7)) + (kb + 256 * (ks >> 3) + sub * 32 * KB));
       };
       bf16x8_t kf[KA][SUBS];
 #pragma unroll
@@ -213,32 +262,52 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       __builtin_amdgcn_sched_group_barrier(0x100, KA * SUBS, 0);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8_t qk = ks < QR ? qf[ks < QR ? ks : 0] : frag16(ql + (ks - QR) * 512);
+        const bf16x8_t qk = ks < QR ? qf[ks < QR ? ks : 0] : lds_frag(ql + (ks - QR) * 1024);
 #pragma unroll
         for (int sub = 0; sub < SUBS; ++sub) {
           const bf16x8_t f = kf[ks % KA][sub];
           if (ks + KA < KS) kf[ks % KA][sub] = kread(ks + KA, sub);
           s[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, qk, s[sub], 0, 0, 0);
         }
+        if (RT == 1 && ks < ND) fetch(base + other, ks);
         __builtin_amdgcn_sched_group_barrier(0x008, SUBS, 0);
+        if (RT == 1 && ks < ND) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, SUBS + (QR < KS), 0);
       }
     }
-    bf16x8_t vf[VA];
-#pragma unroll
-    for (int f = 0; f < VA; ++f) vf[f] = vread(vb, v_at, f);
     if (MODE != kPlain && terms) {  // final scores in log2 units
-      if (cap > 0.f) {  // cap * tanh(x / cap): tanh(y) = 1 - 2 / (1 + e^(2 y))
+      // penalties of the lane's keys
+      const uint32_t pen = table + 4 * (kTablePad - 31 + my - kt - 4 * h);
+      auto penalty = [&](int sub, int i) {
+        return MODE == kTable ? *(const lds_float*)(uintptr_t)(pen + 4 * (31 - (32 * sub + (i & 3) + 8 * (i >> 2)))) : 0.f;
+      };
+      if (cap > 0.f) {  // cap * tanh(x / cap)
+        float far = raw_max3_abs(s[0][0], s[0][1], s[0][2]);
+#pragma unroll
+        for (int i = 3; i < 16 * SUBS - 1; i += 2) far = raw_max3_abs(far, s[i >> 4][i & 15], s[(i + 1) >> 4][(i + 1) & 15]);
+        far = raw_max3_abs(far, far, s[SUBS - 1][15]);
+        if (__builtin_amdgcn_ballot_w64(!(far <= near)) == 0) {
+#pragma unroll
+          for (int sub = 0; sub < SUBS; ++sub)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float t = s[sub][i] * s[sub][i];
+              s[sub][i] = fmaf(s[sub][i], fmaf(t, fmaf(t, fmaf(t, t3, t2), t1), t0), -penalty(sub, i));
+            }
+        } else {  // tanh(y) = 1 - 2 / (1 + e^(2 y))
+#pragma unroll
+          for (int sub = 0; sub < SUBS; ++sub)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              s[sub][i] = fmaf(-2.f * capl, __builtin_amdgcn_rcpf(1.f + fast_exp2(s[sub][i] * cape)), capl) - penalty(sub, i);
+        }
+      } else {
 #pragma unroll
         for (int sub = 0; sub < SUBS; ++sub)
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            s[sub][i] = fmaf(-2.f * capl, __builtin_amdgcn_rcpf(1.f + fast_exp2(s[sub][i] * cape)), capl);
-      } else {
-#pragma unroll
-        for (int sub = 0; sub < SUBS; ++sub) s[sub] *= a.scale * kLog2e;
+          for (int i = 0; i < 16; ++i) s[sub][i] = fmaf(s[sub][i], a.scale * kLog2e, -penalty(sub, i));
       }
-      if (a.r1) {  // (keys behind the row: their argument may be anything, they are masked below)
+      if (logs) {  // (keys behind the row: their argument may be anything, they are masked below)
         // the distance first, which is exact: r2 times the lane's distance less r2 times the key's place would cancel
         const float d0 = (float)(my - kt - 4 * h);
 #pragma unroll
@@ -248,6 +317,9 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
             s[sub][i] = fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, d0 - (float)(32 * sub + (i & 3) + 8 * (i >> 2)), 1.f)), s[sub][i]);
       }
     }
+    bf16x8_t vf[VA];
+#pragma unroll
+    for (int f = 0; f < VA; ++f) vf[f] = vread(vb, v_at, f);
     if (kt + KT - 1 > wlo || (kt < wlast && !kept_tile)) {  // some key is not seen by some row
 #pragma unroll
       for (int sub = 0; sub < SUBS; ++sub)
@@ -310,6 +382,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     };
     constexpr int NF = 2 * SUBS * NC;  // value fragments of the tile
     weigh(0);
+    // forms whose vector work is the longer part: a wave that is at it goes first, products fill what it leaves
+    if constexpr (kEager) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const int k16 = f / NC, dt = f % NC;
@@ -324,18 +398,22 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       __builtin_amdgcn_sched_group_barrier(0x008, FINE ? 2 : 1, 0);
       if (f + VA < NF) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
+    if constexpr (kEager) __builtin_amdgcn_s_setprio(1);
   };
   // tiles in order: the kept ones, then the window's
   const int total = kept + last - first + 1;
   auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
-  issue(smem, tile(0));
+  static_assert(ND <= KS, "a DMA instruction beside a product at most");
+  find(tile(0));
+#pragma unroll
+  for (int k = 0; k < ND; ++k) fetch(base, k);
   landed();
-  for (int i = 0; i < total; i += 2) {
-    if (i + 1 < total) issue(smem + kStage, tile(i + 1));
+  for (int i = 0; i < total; i += 2) {  // (behind the last tile it is fetched again: no branch among the products)
+    find(tile(min(i + 1, total - 1)));
     step(std::integral_constant<int, 0>{}, tile(i));
     landed();
     if (i + 1 < total) {
-      if (i + 2 < total) issue(smem, tile(i + 2));
+      find(tile(min(i + 2, total - 1)));
       step(std::integral_constant<int, 1>{}, tile(i + 1));
       landed();
     }
@@ -378,11 +456,13 @@ template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW,
 int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   PromptArgs a = a0;
   a.subs = 128 / (32 * (NW / HPW));
-  constexpr int lds = 2 * 32 * SUBS * 2 * (D + (SAME ? 0 : DV)) + (SAME && DV == 256 ? NW * (D / 16 - 8) * 1024 : 0);
+  constexpr int tiles = 2 * 32 * SUBS * 2 * (D + (SAME ? 0 : DV)) + (SAME && DV == 256 ? NW * (D / 16 - 8) * 1024 : 0);
+  constexpr int most = tiles + (MODE == kTable ? HPW * (kTableKeys + 2 * kTablePad) * 4 : 0);
+  const int lds = tiles + (MODE == kTable ? HPW * (a.size + 2 * kTablePad) * 4 : 0);
   auto kern = prompt_attention_kernel<D, DV, SAME, MODE, FINE, OutT, HPW, NW, SUBS>;
   static bool raised = false;  // once per instance
-  if (lds > 48 * 1024 && !raised) {
-    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 7;
+  if (most > 48 * 1024 && !raised) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, most) != hipSuccess) return 7;
     raised = true;
   }
   const int step = 65535 / a.subs;
@@ -440,6 +520,9 @@ int dxm_prompt_attention(void* out, const void* q, int64_t q_stride, const void*
   if (same) return prompt_heads<256, 192, true, kPlain, false, bf16_t>(a, n_tiles, st);
   if (dv == 256) return prompt_heads<128, 256, false, kPlain, true, float>(a, n_tiles, st);
   if (wfn) return prompt_heads<128, 128, false, kSigmoid, false, bf16_t>(a, n_tiles, st);
+  // Every row sees keys within `size` of it.  Table / logarithms, us, window 1024, 4500 rows of 32 heads: 99 / 112; 512, 5000
+  // of 16: 41 / 46
+  if (r1 && mask && !keep && size <= kTableKeys) return prompt_heads<128, 128, false, kTable, false, bf16_t>(a, n_tiles, st);
   if (terms) return prompt_heads<128, 128, false, kTerms, false, bf16_t>(a, n_tiles, st);
   if (fine) return prompt_heads<128, 128, false, kPlain, true, bf16_t>(a, n_tiles, st);
   return prompt_heads<128, 128, false, kPlain, false, bf16_t>(a, n_tiles, st);

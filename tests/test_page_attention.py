@@ -286,3 +286,25 @@ def test_later_rows_values_that_are_not_finite():
     got = mx.attention(q.cuda(), kd, vd, torch.arange(64).cuda(), torch.zeros(64, dtype=torch.int32).cuda(), table, 64, n_qh,
                        maps, group, d, dv, d ** -0.5, "causal", 0, 1, False, tiles, 64).cpu().double()[:32]
     assert float((got - want).abs().max()) < 2.0 ** -8 * (float(want.abs().max()) + 5.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size", [("window", 1216), ("window", 1217), ("chunk", 1216), ("window", 33), ("window", 1)])
+@pytest.mark.parametrize("form,cap", [("both", 30.0), ("both", 3.0), ("penalty", 0.0), ("both pair", 12.0)])
+def test_score_terms_of_limited_distance(form, cap, mask, size):
+    """Penalties from the table of distances (up to 1216 keys back, with the first and the last entry in use) and beside
+    it; caps far above the scores (polynomial in every tile), near them (in some) and among them (in none)."""
+    n_qh, maps, group, d, dv = FORMS["plain pair" if form == "both pair" else form]
+    torch.manual_seed(7)
+    scale, start, rows, bs = 0.7 * d ** -0.5, 1190, 131, 64
+    db = (torch.rand(n_qh) * 2, torch.rand(n_qh) * 3 + 0.1)
+    kd, vd, table, kv = pages("plain pair" if form == "both pair" else form, [start + rows], bs)
+    q = torch.randn(rows, n_qh * d).bfloat16()
+    want = dense(q.double().view(rows, n_qh, d), *kv[0], torch.arange(start, start + rows), scale, mask, size, 0, cap, db, None,
+                 False, None)
+    tiles = torch.tensor(mx.tile_list(0, rows), dtype=torch.int32).cuda()
+    got = mx.attention(q.cuda(), kd, vd, torch.arange(start, start + rows).cuda(), torch.zeros(rows, dtype=torch.int32).cuda(),
+                       table, bs, n_qh, maps, group, d, dv, scale, mask, size, 1, False, tiles, rows, softcap=cap,
+                       dist_bias=tuple(map(cuda, db))).cpu().double()
+    err = float((got - want).abs().max())  # (bound of test_prompt_rows)
+    assert err < 2.0 ** -8 * (float(want.abs().max()) + 5.0), err
