@@ -211,6 +211,7 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
     if (min((j0 + BKV - 1) >> bs_shift, last_page) - page0 >= 64) {
       page0 = j0 >> bs_shift;
       pages = bt[min(page0 + lane, last_page)];
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // (here and now: behind the branch it would be waited for at every tile)
     }
     if (BS64) {  // one block; rows past the context arrive as zeros
       const int64_t base = ((int64_t)block(j0) * n_kv_heads + kvh) * head_stride + (int64_t)(j0 & (block_size - 1)) * D;

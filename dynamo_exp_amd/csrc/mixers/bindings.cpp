@@ -322,7 +322,8 @@ PYBIND11_MODULE(_C_mixers, m) {
                            int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs, int keep, u sink,
                            int parts, int out_f32, u st) {
     // pages of whole tiles and heads of 128 columns (or one shared row of 256)
-    if (scale > 0.f && qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && (q | kc | vc | out) % 16 == 0 &&
+    if (scale > 0.f && qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && Wk <= 1 << 23 && Wv <= 1 << 23 &&
+        (q | kc | vc | out) % 16 == 0 &&
         dxm_decode_attention_ok(d, dv, n_qh, maps, group, bs, kc == vc, cap > 0.f || r1, wfn)) {
       parts = std::min(parts, dxm_decode_attention_parts(rows, n_qh, group, kc == vc, dv));
       check(dxm_decode_attention(P(out), F(ws), P(q), qs, P(kc), P(vc), reinterpret_cast<const int64_t*>(pos),

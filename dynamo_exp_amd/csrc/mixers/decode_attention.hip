@@ -6,15 +6,17 @@
 // A workgroup (4 waves) serves one (row, key / value group, part of the keys): up to 16 query vectors of the group (a
 // shared row: 16 QB) are the columns of 16x16x32 products.  Both maps of a two-map layer are in one workgroup, so their
 // common values are read once.  The waves take the part's tiles in turn and run on their own: a wave brings its tiles
-// into LDS of its own by DMA and waits for its own loads only, so there is no barrier until the end, where the four
-// partial results are joined in LDS.  Keys and values have a buffer each, refilled as soon as its product is done; a
+// into LDS of its own by DMA (buffer loads: with global_load_lds no wait for an LDS read can be partial) and waits for its
+// own loads only, so there is no barrier until the end, where the four partial results are joined in LDS.  Fragments are
+// asked for six to eight ahead.  Keys and values have a buffer each, refilled as soon as its product is done; a
 // shared row has two buffers in turn.  V^T fragments come from the row-major image by ds_read_b64_tr_b16.
 // One part: the result goes out finished; several: partials to the workspace that merge_parts joins.
-// Bound by memory at many rows and by latency at few.  Two layers in a graph with their joins, against the one-wave
-// forms it took over from (register-staged group_decode, stream_decode, latent_decode), us before -> after: two maps,
-// window 1024 + 64, 48 rows 270 -> 98 (4.4 TB/s of cache), chunk 2048 358 -> 123, 1 row 89 -> 38; shared row 256 / 192
-// causal to 4000, 33 rows 92 -> 58; cap + penalty 40 rows 174 -> 84; sigmoid 171 -> 84; plain to 4100, 48 rows 239 ->
-// 206 (5.3 TB/s), 2 rows 81 -> 32.
+// Bound by memory at many rows and by latency at few (position, block table, first tile, join: 7 us of a launch with one
+// tile a wave).  Two layers in a graph with their joins, us, two maps, window 1024 + 64, 48 rows 98 (4.4 TB/s of cache);
+// shared row 256 / 192 causal to 4000, 33 rows 53 with fragments read one product ahead -> 50, to 2500, 100 rows 79 -> 73;
+// 256 / 256 window 1024, 20 rows 41 -> 38; two maps, 2 rows of 142 25.3 -> 24.2.  Parts dealt out by the rows' lengths
+// instead of equally: 33 rows the same (memory is as busy while the short rows last), 41 rows of up to 281 keys 60 -> 64.
+// (The one-wave forms it took over from, register-staged group_decode, stream_decode, latent_decode: 270 and 92.)
 #include <algorithm>
 #include <type_traits>
 
@@ -53,11 +55,9 @@ constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kTile = 32;       // keys per tile
 constexpr float kDefer = 8.f;   // log2 units that a score may exceed the running maximum by (weights are bf16 pairs)
 enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
-
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-typedef __attribute__((address_space(3))) void lds_void;
 // metadata that no kernel in flight writes: scalar loads
 typedef const __attribute__((address_space(4))) int* scalar_int;
+typedef const __attribute__((address_space(4))) int64_t* scalar_long;
 
 // the wave's own DMA: all but the newest N instructions have landed.  (The builtin, which the compiler counts itself:
 // behind a wait it does not know it would put a full one in front of the next LDS read.)
@@ -90,21 +90,22 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
   constexpr int KN = kTile * KB / 1024, VN = SAME ? KN : kTile * VB / 1024;             // DMA instructions per tile
   constexpr int GR = MAPS == 2 ? 8 : 16;  // columns per map
   static_assert(!SAME || (MAPS == 1 && D == 256), "one shared row");
-  // keys / values; a shared row: tiles with even / odd turn
-  __shared__ __attribute__((aligned(16))) char ka[4][kTile * KB];
-  __shared__ __attribute__((aligned(16))) char va[4][kTile * VB];
+  // a wave's keys and values; a shared row: its tiles with even / odd turn
+  constexpr int kImg = kTile * (KB + VB), kVal = kTile * KB;
+  __shared__ __attribute__((aligned(16))) char img[4][kImg];
   __shared__ float ml[2][4][QB][16];
   const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = blockIdx.y, part = blockIdx.z;
-  const int p = __builtin_amdgcn_readfirstlane((int)a.pos[row]);
+  const int p = (int)((scalar_long)a.pos)[row];
   const int lo = first_key(p, a.mask, a.size);
-  const int keep = a.mask == 1 ? a.keep : 0;
+  const int keep = a.mask == 1 ? a.keep : 0, keeplo = min(keep, lo);  // (kept keys in front of the window)
   // tiles in order: those of the kept keys, then the mask's
   const int first = lo / kTile, kept = min((keep + kTile - 1) / kTile, first), total = kept + p / kTile - first + 1;
   // at least two tiles a wave, four of a long context: shorter parts cost more in the join than they gain
   const int tpp = max((total + a.parts - 1) / a.parts, max(8, min(16, total / 12))), i0 = part * tpp, i1 = min(i0 + tpp, total);
-  const scalar_int bt = (scalar_int)(a.bt + (int64_t)__builtin_amdgcn_readfirstlane(a.seq ? a.seq[row] : row) * a.bt_stride);
+  const scalar_int bt = (scalar_int)(a.bt + (int64_t)(a.seq ? ((scalar_int)a.seq)[row] : row) * a.bt_stride);
+  auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
   // K head of the workgroup (of the first map), its key / value group
   const int gm = SAME ? 0 : MAPS == 2 ? 2 * blockIdx.x : blockIdx.x, g = SAME ? 0 : gm / a.maps, m = gm - g * a.maps;
   int qh[QB];
@@ -126,16 +127,6 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
           a.q + (int64_t)row * a.q_stride + (int64_t)qh[qb] * D + 32 * ks + 8 * g4) : zero);
     }
   }
-  // lane constants: fragment addresses (pieces 16 and up of a row: + 256 bytes)
-  int koff[4], voff_[8][2];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) koff[ks] = image_off<KB>(c16, 4 * ks + g4);
-#pragma unroll
-  for (int cb = 0; cb < 8; ++cb) {
-    const int ch = 2 * cb + ((lane & 3) >> 1), r = 4 * g4 + (c16 >> 2);
-    voff_[cb][0] = image_off<VB>(r, ch) + 8 * (lane & 1);
-    voff_[cb][1] = image_off<VB>(r + 16, ch) + 8 * (lane & 1);
-  }
   if (i0 >= i1 && part > 0) {  // a part without a key: sum 0
     if (w == 0 && g4 == 0)
 #pragma unroll
@@ -149,23 +140,45 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
   }
   const bf16_t* kc = a.kc + (int64_t)gm * D;
   const bf16_t* vc = a.vc + (int64_t)g * DV;
-  auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
-  // one image: rows of RB bytes; rows behind the query hold stale values, which must not meet a zero weight: its own
-  // row instead
-  auto dma = [&](auto rb, const bf16_t* src, int stride, char* dst, int t) {
-    constexpr int RB = decltype(rb)::value, CH = RB / 16, RP = 1024 / RB;
-    const int j = t * kTile;
-    const int64_t base = ((int64_t)bt[j >> a.bs_shift] << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
-    const bf16_t* s = src + base * stride;
+  const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)&img[w][0];
+  // Fragment addresses: step ks of the keys is an XOR with 64 ks away from the first (pieces 16 and up of a row: + 256
+  // bytes), block cb of the values one with 32 cb; values 16 rows further: + 16 rows.
+  uint32_t koff[4], voff_[8];
 #pragma unroll
-    for (int k = 0; k < kTile / RP; ++k) {
-      const int r = k * RP + lane / CH;
-      __builtin_amdgcn_global_load_lds(s + (int64_t)min(r, p - j) * stride + 8 * ((lane % CH) ^ piece_xor(r)),
-                                       (lds_void*)(dst + k * 1024), 16, 0, 0);
-    }
+  for (int ks = 0; ks < 4; ++ks) koff[ks] = base + image_off<KB>(c16, 4 * ks + g4);
+#pragma unroll
+  for (int cb = 0; cb < 8; ++cb)
+    voff_[cb] = base + (SAME ? 0 : kVal) + image_off<VB>(4 * g4 + (c16 >> 2), 2 * cb + ((lane & 3) >> 1)) + 8 * (lane & 1);
+  // The DMA: source of an image's k-th KB, from the tile's first row.  Rows behind the query hold stale values, which must
+  // not meet a zero weight: they lie outside the descriptor and arrive as zeros.
+  auto source = [&](auto rb, int k, int width) {
+    constexpr int CH = decltype(rb)::value / 16;
+    const int r = k * (64 / CH) + lane / CH;
+    return 2 * (r * width + 8 * ((lane % CH) ^ piece_xor(r)));
   };
-  auto fetch_k = [&](char* dst, int i) { dma(std::integral_constant<int, KB>{}, kc, a.Wk, dst, tile(i)); };
-  auto fetch_v = [&](char* dst, int i) { dma(std::integral_constant<int, VB>{}, vc, a.Wv, dst, tile(i)); };
+  int ksrc[KN], vsrc[SAME ? 1 : VN];
+#pragma unroll
+  for (int k = 0; k < KN; ++k) ksrc[k] = source(std::integral_constant<int, KB>{}, k, a.Wk);
+  if constexpr (!SAME)
+#pragma unroll
+    for (int k = 0; k < VN; ++k) vsrc[k] = source(std::integral_constant<int, VB>{}, k, a.Wv);
+  auto slot = [&](int t) __attribute__((always_inline)) {
+    const int j = t * kTile;
+    return ((uint32_t)bt[j >> a.bs_shift] << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
+  };
+  auto fetch_k = [&](uint32_t dst, int i) __attribute__((always_inline)) {
+    const int t = tile(i), rows = min(p - t * kTile, kTile - 1);  // whole rows in front of the last one
+    const bf16_t* from = kc + (uint64_t)slot(t) * (uint32_t)a.Wk;
+#pragma unroll
+    for (int k = 0; k < KN; ++k) dma16(from, 2 * rows * a.Wk + KB, ksrc[k], base + dst + k * 1024);
+  };
+  auto fetch_v = [&](int i) __attribute__((always_inline)) {
+    const int t = tile(i), rows = min(p - t * kTile, kTile - 1);
+    const bf16_t* from = vc + (uint64_t)slot(t) * (uint32_t)a.Wv;
+    if constexpr (!SAME)
+#pragma unroll
+      for (int k = 0; k < VN; ++k) dma16(from, 2 * rows * a.Wv + VB, vsrc[k], base + kVal + k * 1024);
+  };
 
   const float cap = a.softcap, inv_cap = MODE != kPlain && cap > 0.f ? 1.f / cap : 0.f;
   const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
@@ -180,29 +193,44 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
     for (int cb = 0; cb < NC; ++cb) O[qb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   f32x4 S[QB][2];  // scores: lane column = query vector, rows = keys 16 kb + 4 g4 + r
-  auto scores = [&](const char* K) {
+  constexpr int KF = 2 * KS * MAPS, KA = KF < 8 ? KF : 8;  // key fragments of a tile, of them asked for ahead
+  constexpr int VA = NC < 6 ? NC : 6;                        // value fragments asked for ahead
+  auto scores = [&](auto buf) __attribute__((always_inline)) {
+    constexpr int at = decltype(buf)::value;
+    auto kread = [&](int f) {  // fragment f: step f / (2 MAPS), 16 keys kb, map
+      const int ks = f / (2 * MAPS), kb = f / MAPS % 2, mp = f % MAPS;
+      return lds_frag(koff[ks & 3] + (at + kb * 16 * KB + 256 * (ks >> 2) + 256 * mp));
+    };
+    bf16x8_t kf[KA];
     f32x4 S1[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      S1[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < KA; ++f) kf[f] = kread(f);
+    __builtin_amdgcn_sched_group_barrier(0x100, KA, 0);
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb) S[qb][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < KF; ++f) {
+      const int ks = f / (2 * MAPS), kb = f / MAPS % 2;
+      const bf16x8_t k = kf[f % KA];
+      if (f + KA < KF) kf[f % KA] = kread(f + KA);
+      const f32x4 zero{0.f, 0.f, 0.f, 0.f};
+      if (f % MAPS == 0) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const char* kp = K + koff[ks & 3] + kb * 16 * KB + 256 * (ks >> 2);
-        const bf16x8_t kf = frag16((const bf16_t*)kp);
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) S[qb][kb] = mma(kf, qf[qb][ks], S[qb][kb]);
-        if constexpr (MAPS == 2) S1[kb] = mma(frag16((const bf16_t*)(kp + 256)), qf[0][ks], S1[kb]);
+        for (int qb = 0; qb < QB; ++qb) S[qb][kb] = mma(k, qf[qb][ks], ks ? S[qb][kb] : zero);
+        __builtin_amdgcn_sched_group_barrier(0x008, QB, 0);
+      } else {
+        S1[kb] = mma(k, qf[0][ks], ks ? S1[kb] : zero);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       }
-      if constexpr (MAPS == 2) {  // every column keeps its own map's product
+      if (f + KA < KF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    if constexpr (MAPS == 2) {  // every column keeps its own map's product
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[0][kb][r] = c16 < GR ? S[0][kb][r] : S1[kb][r];
-      }
     }
   };
   bf16x8_t Ph[QB], Pl[QB];
-  auto softmax = [&](int t) {
+  auto softmax = [&](int t) __attribute__((always_inline)) {
     const int kt = t * kTile;
     const bool edge = kt + kTile - 1 > p || (kt < lo && kt + kTile > keep);
 #pragma unroll
@@ -228,8 +256,9 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int j = kt + 16 * kb + 4 * g4 + r;
-            if (j > p || (j < lo && j >= keep)) S[qb][kb][r] = -INFINITY;
+            const int j = kt + 16 * kb + 4 * g4 + r;  // (bitwise: a compare and a select, no branches)
+            const bool seen = ((unsigned)(j - lo) <= (unsigned)(p - lo)) | (j < keeplo);
+            S[qb][kb][r] = seen ? S[qb][kb][r] : -INFINITY;
           }
       }
       float mu = 0.f;
@@ -272,68 +301,83 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
       Pl[qb] = __builtin_bit_cast(bf16x8_t, pl);
     }
   };
-  auto values = [&](const char* V) {
+  bf16x8_t vf[VA];
+  auto vread = [&](int at, int cb) __attribute__((always_inline)) {
+    const uint32_t vp = voff_[cb & 7] + (at + 256 * (cb >> 3));
+    const i16x4 l4 = read_tr16((const lds_i16x4*)(uintptr_t)vp);
+    const i16x4 u4 = read_tr16((const lds_i16x4*)(uintptr_t)(vp + 16 * VB));
+    return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(l4, u4, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto ahead = [&](auto buf) __attribute__((always_inline)) {  // the first value fragments
+#pragma unroll
+    for (int cb = 0; cb < VA; ++cb) vf[cb] = vread(decltype(buf)::value, cb);
+  };
+  auto values = [&](auto buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int cb = 0; cb < NC; ++cb) {
-      const char* vp = V + 256 * (cb >> 3);
-      const i16x4 l4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[cb & 7][0]));
-      const i16x4 u4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vp + voff_[cb & 7][1]));
-      const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(l4, u4, 0, 1, 2, 3, 4, 5, 6, 7));
+      const bf16x8_t v = vf[cb % VA];
+      if (cb + VA < NC) vf[cb % VA] = vread(decltype(buf)::value, cb + VA);
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-        O[qb][cb] = mma(vf, Ph[qb], O[qb][cb]);
-        O[qb][cb] = mma(vf, Pl[qb], O[qb][cb]);
+        O[qb][cb] = mma(v, Ph[qb], O[qb][cb]);
+        O[qb][cb] = mma(v, Pl[qb], O[qb][cb]);
       }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * QB, 0);
+      if (cb + VA < NC) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
   };
-  char *K = ka[w], *V = va[w];
+  typedef std::integral_constant<int, 0> K0;
+  typedef std::integral_constant<int, kVal> K1;  // a shared row's second image
   int i = i0 + w;
   // (the loops hold no conditional DMA: the compiler's count of what is in flight stays exact, see dma_wait)
   if constexpr (SAME) {
-    auto turn = [&](char* cur, int i) {
-      scores(cur);
+    auto turn = [&](auto buf, int i) __attribute__((always_inline)) {
+      scores(buf);
+      ahead(buf);
       softmax(tile(i));
-      values(cur);
+      values(buf);
       lds_wait();
     };
-    if (i < i1) fetch_k(K, i);
+    if (i < i1) fetch_k(0, i);
     for (; i + 8 < i1; i += 8) {
-      fetch_k(V, i + 4);
+      fetch_k(kVal, i + 4);
       dma_wait<KN>();
-      turn(K, i);
-      fetch_k(K, i + 8);
+      turn(K0{}, i);
+      fetch_k(0, i + 8);
       dma_wait<KN>();
-      turn(V, i + 4);
+      turn(K1{}, i + 4);
     }
     if (i + 4 < i1) {
-      fetch_k(V, i + 4);
+      fetch_k(kVal, i + 4);
       dma_wait<KN>();
-      turn(K, i);
+      turn(K0{}, i);
       dma_wait<0>();
-      turn(V, i + 4);
+      turn(K1{}, i + 4);
     } else if (i < i1) {
       dma_wait<0>();
-      turn(K, i);
+      turn(K0{}, i);
     }
   } else if (i < i1) {
-    fetch_k(K, i);
-    fetch_v(V, i);
+    fetch_k(0, i);
+    fetch_v(i);
     for (; i + 4 < i1; i += 4) {
       dma_wait<VN>();  // the keys; the values may still fly
-      scores(K);
+      scores(K0{});
       lds_wait();
-      fetch_k(K, i + 4);
-      softmax(tile(i));
+      fetch_k(0, i + 4);
       dma_wait<KN>();
-      values(V);
+      ahead(K0{});
+      softmax(tile(i));
+      values(K0{});
       lds_wait();
-      fetch_v(V, i + 4);
+      fetch_v(i + 4);
     }
     dma_wait<VN>();
-    scores(K);
-    softmax(tile(i));
+    scores(K0{});
     dma_wait<0>();
-    values(V);
+    ahead(K0{});
+    softmax(tile(i));
+    values(K0{});
   }
   // ---- join the waves
 #pragma unroll
@@ -358,10 +402,8 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
     }
   }
   constexpr int kSlab = QB * NC * 64;  // f32x4 of a wave
-  static_assert(4 * kSlab * 16 <= (int)(sizeof(ka) + sizeof(va)), "partial results fit the images");
-  auto slab = [&](int v) {  // waves 0, 1 in the first array, 2, 3 in the second
-    return reinterpret_cast<f32x4*>(v < 2 ? &ka[0][0] : &va[0][0]) + (v & 1) * kSlab;
-  };
+  static_assert(4 * kSlab * 16 <= (int)sizeof(img), "partial results fit the images");
+  auto slab = [&](int v) { return reinterpret_cast<f32x4*>(&img[0][0]) + v * kSlab; };
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const float f = MODE == kSigmoid ? 1.f : mx[qb] == -INFINITY ? 0.f : fast_exp2(mx[qb] - mt[qb]);

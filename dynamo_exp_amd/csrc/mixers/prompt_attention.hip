@@ -77,24 +77,6 @@ constexpr int kTablePad = 64;     // entries for keys of a tile that a row does 
 constexpr float kTanhMax = 0.36f;
 constexpr float kTanh[4] = {0.99999996f, -0.33332261f, 0.13291534f, -0.04868792f};
 
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-typedef __attribute__((address_space(3))) void lds_void;
-// LDS by its own addresses: through a pointer each would be added to the array's (the front of LDS) in a vector instruction
-typedef __attribute__((address_space(3))) raw_u32x4 lds_u32x4;
-typedef __attribute__((address_space(3))) float lds_float;
-__device__ __forceinline__ bf16x8_t lds_frag(uint32_t at) { return __builtin_bit_cast(bf16x8_t, *(const lds_u32x4*)(uintptr_t)at); }
-
-// (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
-// DMA of the next tile, which goes to the other buffer)
-__device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
-}
-// 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
-// as well, and every wait for an LDS read become one for all of them.)
-__device__ __forceinline__ void dma16(const void* from, int bytes, int off, uint32_t to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)(uintptr_t)to,
-                                           16, off, 0, 0, 0);
-}
 // every wave is done with a tile, and the DMA of the next has landed
 __device__ __forceinline__ void landed() {
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
@@ -195,6 +177,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     if (page - page0 >= 64 || page < page0) {
       page0 = page;
       pages = bt[min(page + lane, hi >> a.bs_shift)];
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // (here and now: behind the branch it would be waited for, and the DMA, at every tile)
     }
     const uint32_t slot = ((uint32_t)__builtin_amdgcn_readlane(pages, page - page0) << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
     const int rows = min(hi - j, KT - 1);  // whole rows in front of the last one
@@ -326,7 +309,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int j = kt + 32 * sub + (i & 3) + 8 * (i >> 2) + 4 * h;
-          if (j > my || (j < mylo && j >= keep)) s[sub][i] = -INFINITY;
+          const bool seen = ((unsigned)(j - mylo) <= (unsigned)(my - mylo)) | (j < min(keep, mylo));  // (bitwise: no branches)
+          s[sub][i] = seen ? s[sub][i] : -INFINITY;
         }
     }
     float mu = 0.f;

@@ -308,3 +308,26 @@ def test_score_terms_of_limited_distance(form, cap, mask, size):
                        dist_bias=tuple(map(cuda, db))).cpu().double()
     err = float((got - want).abs().max())  # (bound of test_prompt_rows)
     assert err < 2.0 ** -8 * (float(want.abs().max()) + 5.0), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size", [("causal", 0), ("chunk", 1500)])
+@pytest.mark.parametrize("form", ["shared", "plain", "diff", "sigmoid"])
+@pytest.mark.parametrize("ctx", [[4000, 33, 1, 2500, 700], [1, 3000], [300 + 61 * i for i in range(20)],
+                                 [1 + 37 * (i % 9) for i in range(64)], [65] * 65], ids=len)
+def test_decode_parts_of_unequal_rows(ctx, form, mask, size):
+    """Rows of one tile beside rows of a hundred, more parts asked for than there are tiles."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(17)
+    scale, B, bs = 0.7 * d ** -0.5, len(ctx), 64
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    kd, vd, table, kv = pages(form, ctx, bs)
+    q = torch.randn(B, n_qh * d).bfloat16()
+    want = torch.cat([dense(q[i:i + 1].double().reshape(1, n_qh, d), *kv[i], torch.tensor([c - 1]), scale, mask, size, 0, cap, db,
+                            sink, sig, hb) for i, c in enumerate(ctx)])
+    for parts in (2, 16):
+        got = mx.attention(q.cuda(), kd, vd, torch.tensor([c - 1 for c in ctx]).cuda(), None, table, bs, n_qh, maps, group, d, dv,
+                           scale, mask, size, parts, True, weights="sigmoid" if sig else "softmax", head_bias=cuda(hb),
+                           sink=cuda(sink)).cpu().double()
+        err, top = float((got - want).abs().max()), float(want.abs().max())
+        assert err < 3e-4 * (max(top, 1.0) if sig else 1.0), (parts, err)  # (bound of test_decode_rows, fp32 results)
