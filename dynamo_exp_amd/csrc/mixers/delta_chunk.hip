@@ -24,12 +24,11 @@
 // A value that is not finite, or that 1 / P makes so, would reach other rows of its chunk than its own and later ones (zero
 // factors times it).  It shows in the rows or stays in the state, and a workgroup that meets one takes its columns again,
 // token by token.
-// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 298 + 146 us, each
-// profiled by itself (in a row, with the layer's norm of 35: 448); a prompt of 600 beside 30 single tokens 704 -> 112, the
-// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 5250 cycles where three
-// workgroups share a CU, 1088 of a wave's matrix instructions each, which keep the matrix cores busy 41 % of the time; the
-// rest is waiting to issue behind the other workgroups' chains, LDS exchanges and the barrier
-// (profiles/step_case_counters.txt).
+// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 209 + 144 us, each
+// profiled by itself (in a row, with the layer's norm of 35: 362); a prompt of 600 beside 30 single tokens 704 -> 87, the
+// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 4000 cycles where three
+// workgroups share a CU, 1088 of a wave's matrix instructions each, so that the matrix cores are busy 54 % of the time (a
+// chain alone: 2400 cycles a chunk); 162 us with the loads taken out.
 #include <algorithm>
 
 #include "delta_tokens.h"
@@ -45,7 +44,11 @@ constexpr int kLong = 32;
 constexpr int kD = 128;   // key channels
 constexpr int kPad = 4;   // floats of padding per LDS row
 constexpr int kMat = kC * kD;
-// floats per (chunk, head): U', R' [16][128]; K''^T, B''^T [128][16]; G, H [16][16]; P_16 [128]
+// Floats per (chunk, head): U', R', K''^T, B''^T, G, H, P_16.  The matrices lie as the chunk kernel's lanes take them, 16
+// bytes a lane and 1 KiB an instruction in a row: U' and R' [channel / 16][channel / 4 % 4][row][channel % 4], K''^T and
+// B''^T [channel / 16][row / 4][channel % 16][row % 4], G and H [column % 4][column / 4][row].  In rows of 128 channels
+// neighbouring lanes lay 512 bytes apart, every lane a cache line of its own, and the chains waited for the vector cache's
+// tags: 298 us of the case below (163 with the loads taken out), 228 like this.
 constexpr int kChunkFloats = 4 * kMat + 2 * kC * kC + kD;
 
 struct FormArgs {
@@ -72,6 +75,25 @@ __device__ __forceinline__ int place(int t) { return 4 * (t & 3) + (t >> 2); }
 
 __device__ __forceinline__ f32x4 mma1(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Reads and writes through descriptors: a uniform base and a size for the rows of a chunk, lane offsets that stay the same
+// from chunk to chunk.  Behind the size reads are 0 and nothing is written.
+typedef __amdgpu_buffer_rsrc_t Range;
+__device__ __forceinline__ Range range(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ f32x4 get4(Range r, uint32_t off, int at) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, at, 0));
+}
+__device__ __forceinline__ float get1(Range r, uint32_t off, int at) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, at, 0));
+}
+__device__ __forceinline__ uint32_t get_half(Range r, uint32_t off, int at) {
+  return __builtin_amdgcn_raw_buffer_load_b16(r, off, at, 0);
+}
+__device__ __forceinline__ void put1(Range r, uint32_t off, int at, float x) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), r, off, at, 0);
 }
 
 // Barrier for what the waves exchange in LDS: __syncthreads() would also wait for every load of the next chunk.
@@ -207,9 +229,9 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int it = tid + 256 * (k & 1), ch = it >> 2, q = it & 3;
+    const int it = tid + 256 * (k & 1), ch = (it >> 6) * 16 + l16, q = g4;
     const float(*src)[LD] = m[3 - (k >> 1)];
-    *reinterpret_cast<f32x4*>(o + (2 + (k >> 1)) * kMat + ch * kC + 4 * q) =
+    *reinterpret_cast<f32x4*>(o + (2 + (k >> 1)) * kMat + 4 * it) =
         f32x4{src[q][ch], src[4 + q][ch], src[8 + q][ch], src[12 + q][ch]};
   }
   if (tid < kD) o[4 * kMat + 2 * kC * kC + tid] = p16[tid];
@@ -229,29 +251,31 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
       for (int q = 0; q < i; ++q) x[i] -= __int_as_float(__builtin_amdgcn_readlane(row[i], q)) * x[q];
 #pragma unroll
     for (int i = 0; i < kC; ++i) {
-      if (gcol) {
-        gram[1][i][j] = x[i];
-        o[4 * kMat + place(i) * kC + place(j)] = x[i];
-      } else {
-        m[0][i][tid] = x[i];
-        o[place(i) * kD + tid] = x[i];
-      }
+      if (gcol) gram[1][i][j] = x[i];
+      else m[0][i][tid] = x[i];
+    }
+    if (gcol) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(o + 4 * kMat + j * kC + 4 * q) = f32x4{x[q], x[4 + q], x[8 + q], x[12 + q]};
     }
   }
   __syncthreads();
+#pragma unroll
+  for (int it = tid; it < kMat / 4; it += 256)
+    *reinterpret_cast<f32x4*>(o + 4 * it) = *reinterpret_cast<const f32x4*>(&m[0][place(l16)][(it >> 6) * 16 + 4 * g4]);
   // ---- R' and H: what tril(R B^T) takes of U' and G, blocks of 16 columns by wave (slot g of instruction i: token 4 g + i)
   const f32x4 rb = *reinterpret_cast<const f32x4*>(&gram[2][l16][4 * g4]);
   for (int cb = w; cb <= kD / 16; cb += 4) {
     const bool hb = cb == kD / 16;
-    f32x4 acc;
+    f32x4 acc = *reinterpret_cast<const f32x4*>(hb ? &gram[3][l16][4 * g4] : &m[1][l16][16 * cb + 4 * g4]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = hb ? gram[3][4 * g4 + i][l16] : m[1][4 * g4 + i][16 * cb + l16];
+    for (int i = 0; i < 4; ++i) acc = mma1(hb ? gram[1][4 * g4 + i][l16] : m[0][4 * g4 + i][16 * cb + l16], -rb[i], acc);
+    if (hb) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc = mma1(-rb[i], hb ? gram[1][4 * g4 + i][l16] : m[0][4 * g4 + i][16 * cb + l16], acc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (hb) o[4 * kMat + kC * kC + (4 * g4 + i) * kC + place(l16)] = acc[i];
-      else o[kMat + (4 * g4 + i) * kD + 16 * cb + l16] = acc[i];
+      for (int i = 0; i < 4; ++i) o[4 * kMat + kC * kC + 64 * g4 + 16 * i + l16] = acc[i];
+    } else {
+      *reinterpret_cast<f32x4*>(o + kMat + 4 * (64 * cb + lane)) = acc;
     }
   }
 }
@@ -318,9 +342,9 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
     return;
   }
   if (n < kLong) {
-    // CT > 1: other workgroups of every sequence and head -- they are dealt out to the chip in turn, and every fourth of
-    // them would lie in a quarter of it
-    constexpr int W = CT > 1 ? 32 * CT : 16 * NB;
+    // as many columns as the threads take at once, and other workgroups of every sequence and head: they are dealt out to
+    // the chip in turn, and every fourth of them would lie in a quarter of it
+    constexpr int W = 32 * CT;
     const int c0 = (blk + sh / 8) % nb * W;
     if (c0 < g.dv) delta_tokens<bf16_t, 8, 256, CT, true>(g.tok, lds.tok, r0, n, h, slot, c0, min(g.dv, c0 + W));
     return;
@@ -337,35 +361,46 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
   const int64_t stride = (int64_t)g.H * kChunkFloats * 4;
   const char* wp = (const char*)(g.ws + ((int64_t)first_chunk(g.seq_rows, s) * g.H + h) * kChunkFloats);
   const char* vp = (const char*)(g.v + (int64_t)r0 * g.vs + col0);
-  const uint32_t row_off = 4u * (l16 * kD + 32 * w + 4 * g4), ch_off = 4u * ((32 * w + l16) * kC + 4 * g4);
-  const uint32_t p_off = 4u * (32 * w + 4 * g4), sq_off = 4u * (l16 * kC + 4 * g4 + w), vs2 = 2u * (uint32_t)g.vs;
+  const uint32_t f_off = 16u * (128 * w + lane), p_off = 4u * (32 * w + 4 * g4), sq_off = 4u * (64 * w + lane), vs2 = 2u * (uint32_t)g.vs;
   const int nc = (n + kC - 1) / kC;
   const uint32_t mine[4] = {w == 0 ? ~0u : 0u, w == 1 ? ~0u : 0u, w == 2 ? ~0u : 0u, w == 3 ? ~0u : 0u};  // the wave's quarter
+  uint32_t v_off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v_off[i] = (g4 + 4 * i) * vs2 + 2u * l16;
   auto load = [&](Frags<NB>& f, int c) {
-    const char *p = wp + c * stride, *vc = vp + (int64_t)c * kC * g.vs * 2;
+    const Range p = range(wp + c * stride, kChunkFloats * 4);
+    const Range vr = range(vp + (int64_t)c * kC * vs2, (uint32_t)(min(n - c * kC, kC) - 1) * vs2 + 32 * NB);
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-      f.u[cb] = *reinterpret_cast<const f32x4*>(p + row_off + 64 * cb);
-      f.r[cb] = *reinterpret_cast<const f32x4*>(p + 4 * kMat + row_off + 64 * cb);
-      f.k[cb] = *reinterpret_cast<const f32x4*>(p + 8 * kMat + ch_off + 64 * kC * cb);
-      f.b[cb] = *reinterpret_cast<const f32x4*>(p + 12 * kMat + ch_off + 64 * kC * cb);
-      f.p[cb] = *reinterpret_cast<const f32x4*>(p + 16 * kMat + 8 * kC * kC + p_off + 64 * cb);
+      f.u[cb] = get4(p, f_off, 1024 * cb);
+      f.r[cb] = get4(p, f_off, 4 * kMat + 1024 * cb);
+      f.k[cb] = get4(p, f_off, 8 * kMat + 1024 * cb);
+      f.b[cb] = get4(p, f_off, 12 * kMat + 1024 * cb);
+      f.p[cb] = get4(p, p_off, 16 * kMat + 8 * kC * kC + 64 * cb);
     }
-    f.g = *reinterpret_cast<const float*>(p + 16 * kMat + sq_off);
-    f.h = *reinterpret_cast<const float*>(p + 16 * kMat + 4 * kC * kC + sq_off);
+    f.g = get1(p, sq_off, 16 * kMat);
+    f.h = get1(p, sq_off, 16 * kMat + 4 * kC * kC);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {  // (the last row again behind the sequence's end)
-      const uint32_t off = (uint32_t)min(g4 + 4 * i, n - 1 - c * kC) * vs2 + 2u * l16;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int q = 0; q < NB; ++q) f.v[q][i] = *reinterpret_cast<const bf16_t*>(vc + off + 32 * q);
-    }
+      for (int q = 0; q < NB; ++q) f.v[q][i] = get_half(vr, v_off[i], 32 * q);
   };
   char* op = (char*)(g.out + (int64_t)r0 * g.H * g.dv + col0);
-  const int64_t ostep = (int64_t)kC * g.H * g.dv * 4;
-  const uint32_t o_off = 4u * ((4 * g4 + w) * (uint32_t)(g.H * g.dv) + l16);
+  const uint32_t out_row = 4u * (uint32_t)(g.H * g.dv), o_off = (4 * g4 + w) * out_row + 4u * l16;
   bool finite = true;
+  // The wave's row of each group of four, from the parts that the last chunk's end left
+  auto finish = [&](int c, int buf) {
+    const Range o4 = range(op + (int64_t)c * kC * out_row, (uint32_t)(min(n - c * kC, kC) - 1) * out_row + 64 * NB);
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const float o = (po[buf][0][q][w][lane] + po[buf][1][q][w][lane]) + (po[buf][2][q][w][lane] + po[buf][3][q][w][lane]);
+      put1(o4, o_off, 64 * q, o);
+      finite = finite && fabsf(o) < INFINITY;
+    }
+  };
   auto step = [&](const Frags<NB>& f, int c, Frags<NB>& next, int cn) {
     const int buf = c & 1;
+    __builtin_amdgcn_sched_barrier(0);  // (a load's first use may not move in front of the step that it is for)
     load(next, min(cn, nc - 1));  // (always a load, the last chunk again: the waits stay counts)
     const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
     float v[NB][4], vw[NB];
@@ -373,7 +408,7 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[q][i] = c * kC + 4 * i + g4 < n ? bf16lo(f.v[q][i]) : 0.f;
+      for (int i = 0; i < 4; ++i) v[q][i] = bf16lo(f.v[q][i]);
       vw[q] = __uint_as_float(__float_as_uint(v[q][0]) & mine[0] | __float_as_uint(v[q][1]) & mine[1] |
                               __float_as_uint(v[q][2]) & mine[2] | __float_as_uint(v[q][3]) & mine[3]);
       X[q][0] = X[q][1] = O[q][0] = O[q][1] = zero;
@@ -387,31 +422,33 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
 #pragma unroll
     for (int q = 0; q < NB; ++q) X[q][0] = mma1(f.g, vw[q], X[q][0]);  // a quarter of G V each wave, the larger part last
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int q = 0; q < NB; ++q) px[buf][w][q][lane] = X[q][0] + X[q][1];
+#pragma unroll
+    for (int i = 0; i < 8 * NB; ++i) {  // a load or two issue while the matrix instruction in front of them runs
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();  // (a buffer is written again two chunks on, when its readers have met another barrier)
+    f32x4 xp[NB][4];
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) xp[q][k] = px[buf][k][q][lane];
+    finish(max(c - 1, 0), 1 - buf);  // (in front of the second chunk zeros, which the first chunk's rows replace)
+    __builtin_amdgcn_sched_group_barrier(0x100, 4 * NB, 0);
+    // the products that need no other wave's part, while theirs arrive
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int q = 0; q < NB; ++q) {
-          O[q][cb] = mma1(f.r[cb][i], S[q][cb][i], O[q][cb]);
           N[q][cb] = mma1(f.k[cb][i], v[q][i], i ? N[q][cb] : zero);
+          O[q][cb] = mma1(f.r[cb][i], S[q][cb][i], O[q][cb]);
         }
-      if (i == 1)
-#pragma unroll
-        for (int q = 0; q < NB; ++q) px[buf][w][q][lane] = X[q][0] + X[q][1];
-    }
 #pragma unroll
     for (int q = 0; q < NB; ++q) O[q][0] = mma1(f.h, vw[q], O[q][0]);
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) po[buf][w][q][i][lane] = O[q][0][i] + O[q][1][i];
-#pragma unroll
-    for (int i = 0; i < 12 + 4 * NB; ++i) {  // a load issues while the matrix instruction in front of it runs
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // K''^T V runs while the others arrive
-    lds_barrier();  // (a buffer is written again two chunks on, when its readers have met another barrier)
 #pragma unroll
     for (int q = 0; q < NB; ++q)
 #pragma unroll
@@ -420,11 +457,9 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
         for (int i = 0; i < 4; ++i) N[q][cb][i] = fmaf(S[q][cb][i], f.p[cb][i], N[q][cb][i]);
     f32x4 xn[NB], M[NB][2];  // (sums of their own: into diag(P) S they would be rounded at its size at every token)
 #pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const f32x4 x0 = px[buf][0][q][lane], x1 = px[buf][1][q][lane], x2 = px[buf][2][q][lane], x3 = px[buf][3][q][lane];
+    for (int q = 0; q < NB; ++q)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) xn[q][i] = (x0[i] + x1[i]) + (x2[i] + x3[i]);
-    }
+      for (int i = 0; i < 4; ++i) xn[q][i] = (xp[q][0][i] + xp[q][1][i]) + (xp[q][2][i] + xp[q][3][i]);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -434,23 +469,26 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
 #pragma unroll
+      for (int i = 0; i < 4; ++i) po[buf][w][q][i][lane] = O[q][0][i] + O[q][1][i];  // (joined behind the next barrier)
+#pragma unroll
       for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[q][cb][i] = N[q][cb][i] - M[q][cb][i];
-      if (c * kC + 4 * g4 + w < n) {  // the wave's row of each group
-        const float o = (po[buf][0][q][w][lane] + po[buf][1][q][w][lane]) + (po[buf][2][q][w][lane] + po[buf][3][q][w][lane]);
-        *reinterpret_cast<float*>(op + c * ostep + o_off + 64 * q) = o;
-        finite = finite && fabsf(o) < INFINITY;
-      }
     }
   };
   Frags<NB> f0, f1;  // (two chunks ahead: a workgroup fewer per CU, 1 to 4 % slower)
   load(f0, 0);
+#pragma unroll
+  for (int q = 0; q < NB; ++q)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) po[1][w][q][i][lane] = 0.f;
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): what is pending here the compiler would wait for in every turn
   for (int c = 0; c < nc; c += 2) {
     step(f0, c, f1, c + 1);
     if (c + 1 < nc) step(f1, c + 1, f0, c + 2);
   }
+  lds_barrier();
+  finish(nc - 1, (nc - 1) & 1);
 #pragma unroll
   for (int q = 0; q < NB; ++q)
 #pragma unroll
@@ -480,7 +518,7 @@ int64_t dxm_delta_chunk_floats(int T_, int n_seq, int H, int dk, int dv, int f32
   if (f32 || dk != kD || dv % 16 || dv < 16 || ptrs % 16 || strides % 8 || !(decay_scale >= -1.f && decay_scale <= 1.f))
     return 0;
   const int64_t chunks = T_ / kC + std::min(n_seq, T_ / kLong);
-  if ((int64_t)H * dv > (1 << 26) || T_ < kLong || chunks * H > 0x7fffffff || H > 65535 ||
+  if ((int64_t)H * dv > (1 << 25) || T_ < kLong || chunks * H > 0x7fffffff || H > 65535 ||
       (int64_t)n_seq * H * (dv / 16) > (1 << 30))
     return 0;
   return chunks * H * kChunkFloats;
@@ -505,18 +543,16 @@ int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void
   d.decay_scale = decay_scale, d.key_eps = key_eps;
   ChunkArgs c{d, out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
   const int64_t heads = ((int64_t)n_seq * H + 7) / 8 * 8;
-  // Two column blocks a workgroup read a chunk once for both, but only two of their workgroups fit a CU; one block keeps
-  // more of the chip busy until there are twice as many workgroups as fit.  Whole layer, 32 heads, us, one / two blocks:
-  // two prompts of 3000 tokens together 343 / 392, three of 4001 443 / 479, four of 3000 335 / 325, six of 5000 547 / 481
-  // Many short sequences in tiles of four columns a thread, few in more workgroups: 64 / 16 / 4 prompts of 16 tokens, four
-  // columns 167 / 69 / 36, one 250 / 74 / 21 (in chunks, whatever their length: 168 / 63 / 24)
-  if (dv % 32 == 0 && heads * (dv / 16) >= 1024) {
-    const dim3 grid((unsigned)(heads * (dv / 32)));
-    if (heads >= 512) hipLaunchKernelGGL((delta_chunk_kernel<2, 4>), grid, dim3(256), 0, st, c);
-    else hipLaunchKernelGGL((delta_chunk_kernel<2, 1>), grid, dim3(256), 0, st, c);
-  } else {
+  // Long sequences gain nothing from two column blocks a workgroup (one / two, us, whole layer of 32 heads: three prompts of
+  // 4001 tokens together 363 / 431, four of 3000 280 / 298, six of 5000 443 / 444); short ones in great numbers do, in tiles
+  // of four columns a thread by four times fewer workgroups (32 prompts of 16 tokens 131 / 116, 64 of them 244 / 191, one of
+  // 600 beside 100 decode rows 210 / 205).  Up to about a thousand (sequence, head) there are too few of them for that: 600
+  // tokens beside 12, 30 and 48 decode rows 89 / 90, 112 / 114 and 138 / 139, 20-token prompts beside 12 46 / 63, 16 prompts
+  // of 16 tokens 64 / 65.
+  if (dv % 32 == 0 && heads >= 1024)
+    hipLaunchKernelGGL((delta_chunk_kernel<2, 4>), dim3((unsigned)(heads * (dv / 32))), dim3(256), 0, st, c);
+  else
     hipLaunchKernelGGL((delta_chunk_kernel<1, 1>), dim3((unsigned)(heads * (dv / 16))), dim3(256), 0, st, c);
-  }
   DX_CHECK_LAUNCH();
   return 0;
 }

@@ -201,3 +201,25 @@ def test_rows_of_any_size(scale, what, size):
     # (where a large row is removed again what is left has lost the same bits in both: measured 0.2 to 1.6 of each other)
     err, err_serial = (float(((x - want)[ok].norm(dim=1) / want[ok].norm(dim=1)).max()) for x in (got, serial))
     assert err < 4 * err_serial + 1e-5, (err, err_serial)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,dv,rows", [(2, 128, [33, 1, 70, 20]), (3, 16, [250]), (1, 48, [47, 32]),
+                                       (16, 32, [1] * 40 + [33, 70, 17] + [2] * 21)])  # the last: two column blocks a workgroup
+def test_value_rows_anywhere(H, dv, rows):
+    """Values in rows of an odd stride behind an odd offset, with NaN around every row and behind the last one (a chunk
+    that the sequence does not fill reads zeros there): bit for bit what packed rows give."""
+    torch.manual_seed(31)
+    T, n = sum(rows), H * 128
+    p, wl = torch.randn(T, 3 * n + H * dv, device="cuda").bfloat16(), (torch.randn(T, n, device="cuda") * 0.5).bfloat16()
+    wide = torch.full((T + 16, H * dv + 5), math.nan, dtype=torch.bfloat16, device="cuda")
+    wide[:T, 1:1 + H * dv] = p[:, 3 * n:]
+    ab, wb = torch.randn(n, device="cuda") * 0.5, torch.randn(n, device="cuda")
+    starts = torch.tensor([sum(rows[:i]) for i in range(len(rows) + 1)], dtype=torch.int32).cuda()
+    pos, slots = torch.cat([torch.arange(r) for r in rows]).cuda(), torch.arange(len(rows), dtype=torch.int32).cuda()
+    res = []
+    for v in (p[:, 3 * n:].contiguous(), wide[:T, 1:1 + H * dv]):
+        state = torch.zeros(len(rows), H, dv, 128, device="cuda")
+        res.append((rc.delta_rule(p[:, :n], p[:, n:2 * n], v, p[:, 2 * n:3 * n], wl, ab, wb, state, pos, starts, slots, H, 128,
+                                  dv), state))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1]) and bool(torch.isfinite(res[0][0]).all())
