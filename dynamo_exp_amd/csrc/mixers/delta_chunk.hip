@@ -24,8 +24,8 @@
 // A value that is not finite, or that 1 / P makes so, would reach other rows of its chunk than its own and later ones (zero
 // factors times it).  It shows in the rows or stays in the state, and a workgroup that meets one takes its columns again,
 // token by token.
-// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 209 + 144 us, each
-// profiled by itself (in a row, with the layer's norm of 35: 362); a prompt of 600 beside 30 single tokens 704 -> 87, the
+// 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 211 + 99 us, each
+// profiled by itself (in a row, with the layer's norm of 35: 323); a prompt of 600 beside 30 single tokens 704 -> 77, the
 // layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 4000 cycles where three
 // workgroups share a CU, 1088 of a wave's matrix instructions each, so that the matrix cores are busy 54 % of the time (a
 // chain alone: 2400 cycles a chunk); 162 us with the loads taken out.
@@ -103,7 +103,25 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ float sigmoid1(float z) { return 1.f / (1.f + expf(-z)); }
+// 1 / (1 + exp(-z)) with the exponential's argument in two parts and a Newton step behind the reciprocal: half the
+// instructions of 1.f / (1.f + expf(-z)), and nearer to 64 bits (largest relative error over 2^24 arguments of |z| < 1, 8 and
+// 30: 1.3e-7, 1.6e-7 and 2.1e-7; that one's 1.3e-7, 4.5e-7 and 1.4e-6).
+__device__ __forceinline__ float sigmoid1(float z) {
+  const float hi = -1.44269504f * z, lo = fmaf(-1.44269504f, z, -hi) - 1.92596300e-8f * z;
+  const float p = __builtin_amdgcn_exp2f(hi);
+  const bool in = fabsf(hi) < 126.f;
+  const float d = 1.f + (in ? fmaf(p, 0.69314718f * lo, p) : p);
+  const float q = __builtin_amdgcn_rcpf(d);
+  return in ? fmaf(fmaf(-d, q, 1.f), q, q) : q;  // (at either end, and of NaN, 1 / (1 + p) as it is)
+}
+
+// The even lane's value, in both lanes of a pair
+__device__ __forceinline__ double of_even(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_mov_dpp((int)b, 0xa0, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xa0, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
 
 // 2^-(hi + lo)
 __device__ __forceinline__ float exp2m(float hi, float lo) {
@@ -111,6 +129,9 @@ __device__ __forceinline__ float exp2m(float hi, float lo) {
   return fmaf(p, -0.69314718f * lo, p);
 }
 
+// Bound by its elementwise instructions (900 a wave with the sums in fp64, 53 matrix instructions), four workgroups a CU: 144
+// -> 99 us at 4001 tokens of 32 heads, 281 MB written.  The sums went through two of the four waves, as did the
+// substitution, one column a thread with its factors handed out lane by lane (1450 instructions in those two waves).
 __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
   constexpr int LD = kD + kPad;
   // four workgroups fit a CU's LDS
@@ -142,12 +163,19 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss += kk[e] * kk[e];
     const float inv = rsqrtf(group_sum<16>(ss) + g.key_eps);
+    const Range abr = range(g.a_bias, g.a_bias ? 4 * kD * g.H : 0), wbr = range(g.w_bias, g.w_bias ? 4 * kD * g.H : 0);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float ab = g.a_bias ? g.a_bias[col + e] : 0.f, wb = g.w_bias ? g.w_bias[col + e] : 0.f;
-      u[e] = kk[e] * inv;
-      b[e] = sigmoid1(al[e] + ab) * u[e];
-      pw[t][c0 + e] = g.decay_scale * sigmoid1(wl[e] + wb);
+    for (int q = 0; q < 2; ++q) {
+      const f32x4 ab = get4(abr, 4 * (uint32_t)col, 16 * q), wb = get4(wbr, 4 * (uint32_t)col, 16 * q);  // (0 without a bias)
+      f32x4 dec;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = 4 * q + i;
+        u[e] = kk[e] * inv;
+        b[e] = sigmoid1(al[e] + ab[i]) * u[e];
+        dec[i] = g.decay_scale * sigmoid1(wl[e] + wb[i]);
+      }
+      *reinterpret_cast<f32x4*>(&pw[t][c0 + 4 * q]) = dec;
     }
   } else {  // behind the sequence's end: nothing read, nothing removed, nothing added
 #pragma unroll
@@ -159,33 +187,46 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
   __syncthreads();
   // Every product of decays is 2^-(a difference of sums), its sums hi + lo: rounded once.  Products of rounded decays
   // would drift token by token, and the form would be less exact than the one that takes the tokens in order.
-  if (tid < kD) {
-    double sum = 0;
+  {
+    const int c = tid >> 1, first = tid & 1 ? 8 : 0;  // two threads a channel, eight tokens each
+    double sum[8];
 #pragma unroll
-    for (int i = 0; i < kC; ++i) {
-      sum = fma((double)pw[i][tid], 1.4426950408889634, sum);
-      const float hi = (float)sum;
-      m[0][i][tid] = hi;
-      m[1][i][tid] = (float)(sum - (double)hi);
+    for (int i = 0; i < 8; ++i) {
+      const double x = pw[first + i][c];
+      sum[i] = i ? fma(x, 1.4426950408889634, sum[i - 1]) : x * 1.4426950408889634;
     }
-    p16[tid] = exp2m(m[0][kC - 1][tid], m[1][kC - 1][tid]);
+    const double half = of_even(sum[7]), before = first ? half : 0.0;  // (every lane asks: one that is off answers nothing)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      sum[i] += before;
+      const float hi = (float)sum[i];
+      m[0][first + i][c] = hi;
+      m[1][first + i][c] = (float)(sum[i] - (double)hi);
+      if (i == 7 && first) p16[c] = exp2m(hi, (float)(sum[i] - (double)hi));
+    }
   }
   __syncthreads();
   float k2[8], b2[8];  // K'' and B''
   f32x4 x[4][2];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int c = c0 + e;
-    const float hi = m[0][t][c], lo = m[1][t][c];
-    const float ip = exp2m(-hi, -lo), dh = m[0][kC - 1][c] - hi;
-    // (what the difference of the his rounds off, exactly)
-    const float q = exp2m(dh, ((m[0][kC - 1][c] - dh) - hi) + (m[1][kC - 1][c] - lo));
-    x[0][e >> 2][e & 3] = t ? u[e] * exp2m(m[0][t - 1][c], m[1][t - 1][c]) : u[e];
-    x[1][e >> 2][e & 3] = rr[e] * exp2m(hi, lo);
-    x[2][e >> 2][e & 3] = b[e] * ip;
-    x[3][e >> 2][e & 3] = kk[e] * ip;
-    k2[e] = kk[e] * q;
-    b2[e] = b[e] * q;
+  for (int j = 0; j < 2; ++j) {
+    const int c = c0 + 4 * j;
+    auto at = [&](int half, int i) { return *reinterpret_cast<const f32x4*>(&m[half][i][c]); };
+    const f32x4 hi = at(0, t), lo = at(1, t), hi0 = at(0, max(t - 1, 0)), lo0 = at(1, max(t - 1, 0));
+    const f32x4 end = at(0, kC - 1), endl = at(1, kC - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = 4 * j + i;
+      const float ip = exp2m(-hi[i], -lo[i]), dh = end[i] - hi[i];
+      // (what the difference of the his rounds off, exactly)
+      const float q = exp2m(dh, ((end[i] - dh) - hi[i]) + (endl[i] - lo[i]));
+      x[0][j][i] = t ? u[e] * exp2m(hi0[i], lo0[i]) : u[e];
+      x[1][j][i] = rr[e] * exp2m(hi[i], lo[i]);
+      x[2][j][i] = b[e] * ip;
+      x[3][j][i] = kk[e] * ip;
+      k2[e] = kk[e] * q;
+      b2[e] = b[e] * q;
+    }
   }
   __syncthreads();
 #pragma unroll
@@ -235,47 +276,50 @@ __global__ void __launch_bounds__(256, 4) delta_form_kernel(FormArgs g) {
         f32x4{src[q][ch], src[4 + q][ch], src[8 + q][ch], src[12 + q][ch]};
   }
   if (tid < kD) o[4 * kMat + 2 * kC * kC + tid] = p16[tid];
-  // ---- a thread per column of [U | G]: forward substitution
-  if (tid < kD + kC) {
-    const bool gcol = tid >= kD;
-    const int j = tid - kD;
-    float x[kC];
-    int row[kC];  // lane q of 16: the factor of x[q] in row i, handed out as a scalar
+  // ---- [U | G] to [U' | G]: forward substitution by blocks of 16 columns, the waves' own to the end: blocks w and w + 4 of
+  // U, G wave 0's.  Tokens 4 p .. 4 p + 3 lie in the lanes with g4 = p, which take them from each other; the rows behind lose
+  // them in one matrix instruction, its factors below the block of four only.
+  f32x4 low[3], take;
 #pragma unroll
-    for (int i = 0; i < kC; ++i) x[i] = gcol ? gram[1][i][j] : m[0][i][tid];
+  for (int i = 0; i < 3; ++i) low[i] = *reinterpret_cast<const f32x4*>(&gram[0][4 * g4 + 1 + i][4 * g4]);
 #pragma unroll
-    for (int i = 1; i < kC; ++i) row[i] = __float_as_int(gram[0][i][l16]);
+  for (int p = 0; p < 3; ++p) take[p] = l16 > 4 * p + 3 ? -gram[0][l16][4 * p + g4] : 0.f;
+  // R' and H: what tril(R B^T) takes of U' and G (slot g of instruction i: token 4 g + i)
+  const f32x4 rb = -*reinterpret_cast<const f32x4*>(&gram[2][l16][4 * g4]);
+  auto solve = [&](float* at, int ld, f32x4 r) __attribute__((always_inline)) {  // at: the block, r: its rows of R or H
+    f32x4 y;
 #pragma unroll
-    for (int i = 1; i < kC; ++i)
+    for (int i = 0; i < 4; ++i) y[i] = at[(4 * g4 + i) * ld + l16];
 #pragma unroll
-      for (int q = 0; q < i; ++q) x[i] -= __int_as_float(__builtin_amdgcn_readlane(row[i], q)) * x[q];
+    for (int p = 0; p < 4; ++p) {
+      if (g4 == p) {
+        y[1] = fmaf(-low[0][0], y[0], y[1]);
+        y[2] = fmaf(-low[1][1], y[1], fmaf(-low[1][0], y[0], y[2]));
+        y[3] = fmaf(-low[2][2], y[2], fmaf(-low[2][1], y[1], fmaf(-low[2][0], y[0], y[3])));
 #pragma unroll
-    for (int i = 0; i < kC; ++i) {
-      if (gcol) gram[1][i][j] = x[i];
-      else m[0][i][tid] = x[i];
+        for (int i = 0; i < 4; ++i) at[(4 * p + i) * ld + l16] = y[i];
+      }
+      asm volatile("" ::: "memory");  // (a wave's LDS accesses go in order; other lanes read what this one wrote)
+      if (p < 3) y = mma1(take[p], at[(4 * p + g4) * ld + l16], y);
     }
-    if (gcol) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<f32x4*>(o + 4 * kMat + j * kC + 4 * q) = f32x4{x[q], x[4 + q], x[8 + q], x[12 + q]};
-    }
+    for (int i = 0; i < 4; ++i) r = mma1(at[(4 * g4 + i) * ld + l16], rb[i], r);
+    return r;
+  };
+#pragma unroll
+  for (int cb = w; cb < kD / 16; cb += 4) {
+    const f32x4 r = solve(&m[0][0][16 * cb], LD, *reinterpret_cast<const f32x4*>(&m[1][l16][16 * cb + 4 * g4]));
+    float* to = o + 4 * (64 * cb + lane);
+    *reinterpret_cast<f32x4*>(to) = *reinterpret_cast<const f32x4*>(&m[0][place(l16)][16 * cb + 4 * g4]);
+    *reinterpret_cast<f32x4*>(to + kMat) = r;
   }
-  __syncthreads();
+  if (w == 0) {
+    const f32x4 r = solve(&gram[1][0][0], kC + kPad, *reinterpret_cast<const f32x4*>(&gram[3][l16][4 * g4]));
+    float* to = o + 4 * kMat + 64 * g4 + l16;
 #pragma unroll
-  for (int it = tid; it < kMat / 4; it += 256)
-    *reinterpret_cast<f32x4*>(o + 4 * it) = *reinterpret_cast<const f32x4*>(&m[0][place(l16)][(it >> 6) * 16 + 4 * g4]);
-  // ---- R' and H: what tril(R B^T) takes of U' and G, blocks of 16 columns by wave (slot g of instruction i: token 4 g + i)
-  const f32x4 rb = *reinterpret_cast<const f32x4*>(&gram[2][l16][4 * g4]);
-  for (int cb = w; cb <= kD / 16; cb += 4) {
-    const bool hb = cb == kD / 16;
-    f32x4 acc = *reinterpret_cast<const f32x4*>(hb ? &gram[3][l16][4 * g4] : &m[1][l16][16 * cb + 4 * g4]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc = mma1(hb ? gram[1][4 * g4 + i][l16] : m[0][4 * g4 + i][16 * cb + l16], -rb[i], acc);
-    if (hb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[4 * kMat + kC * kC + 64 * g4 + 16 * i + l16] = acc[i];
-    } else {
-      *reinterpret_cast<f32x4*>(o + kMat + 4 * (64 * cb + lane)) = acc;
+    for (int i = 0; i < 4; ++i) {
+      to[16 * i] = gram[1][place(l16)][4 * g4 + i];
+      to[kC * kC + 16 * i] = r[i];
     }
   }
 }

@@ -223,3 +223,28 @@ def test_value_rows_anywhere(H, dv, rows):
         res.append((rc.delta_rule(p[:, :n], p[:, n:2 * n], v, p[:, 2 * n:3 * n], wl, ab, wb, state, pos, starts, slots, H, 128,
                                   dv), state))
     assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1]) and bool(torch.isfinite(res[0][0]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("z", [0.0, 20.0, 87.0, 88.5, 100.0, 3e38, math.inf])
+def test_gates_at_their_ends(z):
+    """Removal and decay gates of logits +-z, also far enough that exp() of them is 0 or infinite; and no biases at all, bit
+    for bit what biases of zero give."""
+    torch.manual_seed(37)
+    H, dv, T, n = 2, 32, 50, 256
+    p, wl = torch.randn(T, 3 * n + H * dv).bfloat16(), torch.full((T, n), z).bfloat16()
+    wl[::2] *= -1
+    p[:, 2 * n:3 * n] = wl.flip(1)
+    p[::3, 2 * n:3 * n] *= -1
+    zero, state0 = torch.zeros(n), torch.randn(1, H, dv, 128)
+    want, want_state = recurrence(p[:, :n], p[:, n:2 * n], p[:, 3 * n:], p[:, 2 * n:3 * n], wl, zero, zero,
+                                  state0[0].double().transpose(1, 2), H, dv, SCALE)
+    res = []
+    for bias in (zero.cuda(), None):
+        state = state0.cuda()
+        out = run(p.cuda(), wl.cuda(), bias, bias, state, torch.arange(5, 5 + T).cuda(), [0, T], [0], H, dv)
+        res.append((out.cpu(), state.cpu()))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    rel = lambda x, y: float((x.double() - y).norm() / y.norm())
+    # (fp32 sums of 128 to 2000 products, each rounded to 2^-24 of it: sqrt(2000) 2^-24 relative to the terms)
+    assert rel(res[0][0], want) < 3e-6 and rel(res[0][1][0], want_state.transpose(1, 2)) < 3e-6
