@@ -15,6 +15,9 @@
 // Which k a slot stands for is free as long as A and B agree: with slots {4 g +
 // 0..3, 16 + 4 g + 0..3} a pair of result tiles of S is an A operand as it lies in
 // the registers.
+#include <algorithm>
+#include <type_traits>
+
 #include "linear_scan.h"
 
 namespace {
@@ -82,14 +85,16 @@ struct Walk {
   bool fresh;
 };
 __device__ __forceinline__ bool open_walk(const ScanArgs& g, Walk& w) {
-  const int s = blockIdx.z;
+  const int z = blockIdx.z;
+  const SeqRows q = g.sorted ? by_length(g.seq_rows, g.slots, gridDim.z, z, g.min_rows)
+                             : SeqRows{g.seq_rows[z], g.seq_rows[z + 1] - g.seq_rows[z], g.slots[z], z};
   w.h = blockIdx.y;
   w.hq = w.h / g.qk_rep;
   w.col0 = blockIdx.x * kPB;
-  w.r0 = g.seq_rows[s];
-  w.n = g.seq_rows[s + 1] - w.r0;
+  w.r0 = q.r0;
+  w.n = q.n;
   if (w.n < g.min_rows || w.r0 < 0 || w.r0 + w.n > g.T) return false;
-  w.slot = g.slots[s];
+  w.slot = q.slot;
   if (w.slot < 0 || w.slot >= g.n_slots) {  // padding: zeros out, no state touched
     for (int i = threadIdx.x; i < w.n * kPB; i += blockDim.x)
       g.out[(int64_t)(w.r0 + i / kPB) * g.H * g.dv + (int64_t)w.h * g.dv + w.col0 + i % kPB] = 0.f;
@@ -106,6 +111,14 @@ __device__ __forceinline__ bool open_walk(const ScanArgs& g, Walk& w) {
 // stage a chunk's rows and form these weights, 16 token rows each (only the tiles
 // on and below the diagonal), one chunk ahead, in the other half of the
 // double-buffered LDS; the lower four form the outputs and walk the state.
+// Bound by the chain of the longest sequence's chunks, in it by the upper waves: in front of a chunk's first barrier they
+// stage the next one (rows to LDS as they lie and transposed), in front of its second one they weigh it.  Rows come
+// through descriptors (zeros behind the sequence's end instead of a branch per load), neighbouring lanes on neighbouring
+// pieces of a row, where lanes on different rows took 600 to 2000 cycles a chunk to ask for theirs; the decays are summed
+// a chunk ahead, by the wave that has least to weigh; a wave's tiles are formed side by side, as the lower waves' outputs
+// are, without branches.  Two chunks of rows ahead: more registers than there are, 173 us instead of 112.
+// 32 heads of 128 / 128, 4001 tokens in three prompts, 100 -> 81 us (with the norm behind it 139 -> 112); 128 heads of 128 /
+// 64 with a step, 152 -> 98, of which the longest sequence first 25.
 // LDS rows are cut into 16-byte pieces that an XOR with row bits moves around, so that the 16 rows a fragment
 // read touches (whichever lane groups the hardware serves together) and the staging writes (rows 4 apart) lie on
 // different banks: element offset of piece pc of row r in a [..][DK] and in a [..][64] image.
@@ -113,7 +126,7 @@ template <int DK> __device__ __forceinline__ int koff(int r, int pc) {
   if constexpr (DK == 128) return r * 128 + ((pc ^ ((r & 12) | ((r & 3) ^ (r >> 4)))) << 3);
   return r * (DK + 8) + (pc << 3);  // (narrow rows: padding)
 }
-__device__ __forceinline__ int soff(int r, int pc) { return r * 64 + ((pc ^ ((r >> 1) & 7)) << 3); }
+__device__ __forceinline__ int soff(int r, int pc) { return r * 64 + ((pc ^ ((r >> 1) & 7) ^ ((r >> 3) & 7)) << 3); }
 
 template <int DK> struct ChunkBuf {
   bf16_t q[64 * (DK == 128 ? DK : DK + 8)];  // [t][n]
@@ -134,65 +147,79 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
   Walk w;
   if (!open_walk(g, w)) return;
   const bool former = threadIdx.x >= 256;
-  const int tid = threadIdx.x & 255, wave = tid >> 6, c16 = tid & 15, g4 = (tid & 63) >> 4;
+  const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = tid & 15, g4 = (tid & 63) >> 4;
 
   if (former) {  // ---- stage the chunks' rows; form the pair weights
-    const int sq = tid & 15, oc = tid >> 4;  // token quad, channel octet
-    // the thread's first row of the chunk being fetched
-    const bf16_t* q = (const bf16_t*)g.q + (int64_t)(w.r0 + 4 * sq) * g.qs + (int64_t)w.hq * DK + 8 * oc;
-    const bf16_t* k = (const bf16_t*)g.k + (int64_t)(w.r0 + 4 * sq) * g.ks + (int64_t)w.hq * DK + 8 * oc;
-    const bf16_t* v = (const bf16_t*)g.v + (int64_t)(w.r0 + 4 * sq) * g.vs + (int64_t)w.h * g.dv + w.col0 + 8 * oc;
+    // token quad, channel octet; neighbouring threads on neighbouring octets, whole rows at a time
+    const int sq = tid / NO, oc = tid % NO;
+    const int vt = tid - 128, vq = (vt & 127) >> 3, vo = vt & 7;  // the same of v, which the upper two waves stage
+    const bf16_t* q = (const bf16_t*)g.q + (int64_t)w.r0 * g.qs + (int64_t)w.hq * DK;
+    const bf16_t* k = (const bf16_t*)g.k + (int64_t)w.r0 * g.ks + (int64_t)w.hq * DK;
+    const bf16_t* v = (const bf16_t*)g.v + (int64_t)w.r0 * g.vs + (int64_t)w.h * g.dv + w.col0;
     const float skip = g.skip ? g.skip[w.h] : 0.f, qsc = g.q_scale;
     const float fixed_l2 = MODE == kFixed ? fmaxf(log2f(g.decay[w.h]), -1e6f) : 0.f;
-    bf16_t rg = 0;  // step logit of token tid (first wave)
     const bf16_t* gl = MODE == kStep ? (const bf16_t*)g.g + (int64_t)w.r0 * g.gs + w.h : nullptr;
     const float g_bias = MODE == kStep && g.g_bias ? g.g_bias[w.h] : 0.f;
     const float rate_l2 = MODE == kStep ? -g.rate[w.h] * kLog2e : 0.f;
-    raw_u32x4 rq[4], rk[4], rv[4];
-    auto fetch = [&](int t0) {
-      const raw_u32x4 zero{0u, 0u, 0u, 0u};
+    // A chunk's rows on their way: through descriptors, which give zeros behind the sequence's end, so that no branch lies
+    // between a load and its wait, and the wait for one chunk is not one for the next.
+    struct Rows {
+      raw_u32x4 q[4], k[4], v[4];
+      uint32_t g;  // step logit of token tid (first wave)
+    };
+    const uint32_t qs2 = 2u * (uint32_t)g.qs, ks2 = 2u * (uint32_t)g.ks, vs2 = 2u * (uint32_t)g.vs, gs2 = 2u * (uint32_t)g.gs;
+    constexpr uint32_t kOff = 0x80000000u;  // behind every range
+    const uint32_t q_off = NI == 256 || tid < NI ? 4 * sq * qs2 + 16 * oc : kOff, k_off = NI == 256 || tid < NI ? 4 * sq * ks2 + 16 * oc : kOff;
+    const uint32_t v_off = vt >= 0 ? 4 * vq * vs2 + 16 * vo : kOff, g_off = tid < Q ? tid * gs2 : kOff;
+    auto fetch = [&](Rows& x, int t0) {
+      const int n = max(min(w.n - t0, Q), 0);
+      auto range = [&](const bf16_t* p, int64_t stride, int width) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(p + t0 * stride), 0, n ? 2u * (uint32_t)((n - 1) * (int)stride + width) : 0u,
+                                                 0x00020000);
+      };
+      if constexpr (MODE == kStep) x.g = __builtin_amdgcn_raw_buffer_load_b16(range(gl, g.gs, 1), g_off, 0, 0);
+      const auto qr = range(q, g.qs, DK), kr = range(k, g.ks, DK), vr = range(v, g.vs, kPB);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const bool ok = t0 + 4 * sq + i < w.n;
-        rq[i] = (NI == 256 || tid < NI) && ok ? *reinterpret_cast<const raw_u32x4*>(q + i * g.qs) : zero;
-        rk[i] = (NI == 256 || tid < NI) && ok ? *reinterpret_cast<const raw_u32x4*>(k + i * g.ks) : zero;
-        rv[i] = tid < 128 && ok ? *reinterpret_cast<const raw_u32x4*>(v + i * g.vs) : zero;
+        x.q[i] = __builtin_amdgcn_raw_buffer_load_b128(qr, q_off + i * qs2, 0, 0);
+        x.k[i] = __builtin_amdgcn_raw_buffer_load_b128(kr, k_off + i * ks2, 0, 0);
+        x.v[i] = __builtin_amdgcn_raw_buffer_load_b128(vr, v_off + i * vs2, 0, 0);
       }
-      q += Q * g.qs;
-      k += Q * g.ks;
-      v += Q * g.vs;
-      if (MODE == kStep && tid < Q && t0 + tid < w.n) rg = gl[(int64_t)(t0 + tid) * g.gs];
     };
-    auto stage = [&](ChunkBuf<DK>& b, int t0) {
+    struct Decay {
+      float L, u, w;
+    } at;
+    auto stage = [&](ChunkBuf<DK>& b, const Rows& x) {
       if (NI == 256 || tid < NI) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          *reinterpret_cast<raw_u32x4*>(b.q + koff<DK>(4 * sq + i, oc)) = rq[i];
-          *reinterpret_cast<raw_u32x4*>(ks + koff<DK>(4 * sq + i, oc)) = rk[i];
+          *reinterpret_cast<raw_u32x4*>(b.q + koff<DK>(4 * sq + i, oc)) = x.q[i];
+          *reinterpret_cast<raw_u32x4*>(ks + koff<DK>(4 * sq + i, oc)) = x.k[i];
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          *reinterpret_cast<uint2*>(b.kT + soff(8 * oc + e, sq >> 1) + 4 * (sq & 1)) = column4(rk, e);
+          *reinterpret_cast<uint2*>(b.kT + soff(8 * oc + e, sq >> 1) + 4 * (sq & 1)) = column4(x.k, e);
       }
-      if (tid < 128) {
+      if (vt >= 0) {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          *reinterpret_cast<uint2*>(b.vT + soff(8 * oc + e, sq >> 1) + 4 * (sq & 1)) = column4(rv, e);
+          *reinterpret_cast<uint2*>(b.vT + soff(8 * vo + e, vq >> 1) + 4 * (vq & 1)) = column4(x.v, e);
       }
-      if (tid < Q) {  // one wave: log decays since the chunk's start (inclusive scan)
-        const bool ok = t0 + tid < w.n;
-        float u = ok ? 1.f : 0.f, L = ok ? fixed_l2 : 0.f;
-        if (MODE == kStep && ok) {
-          u = softplusf_(bf16_to_f32(rg) + g_bias);
-          L = rate_l2 * u;
-        }
-        L = wave_scan_sum(L);
-        u *= g.k_scale;
-        b.L[tid] = L;
-        b.u[tid] = u;
-        const float Lend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, L), 63));
-        b.w[tid] = u * fast_exp2(Lend - L);
+      if (tid < Q) b.L[tid] = at.L, b.u[tid] = at.u, b.w[tid] = at.w;
+    };
+    // one wave, a chunk ahead of its rows: log decays since the chunk's start (inclusive scan)
+    auto decays = [&](const Rows& x, int t0) {
+      if (wave != 0) return;
+      const bool ok = t0 + tid < w.n;
+      float u = ok ? 1.f : 0.f, L = ok ? fixed_l2 : 0.f;
+      if (MODE == kStep) {
+        u = ok ? softplusf_(bf16_to_f32((bf16_t)x.g) + g_bias) : 0.f;
+        L = rate_l2 * u;
       }
+      L = wave_scan_sum(L);
+      u *= g.k_scale;
+      const float Lend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, L), 63));
+      at = Decay{L, u, u * fast_exp2(Lend - L)};
     };
     auto weigh = [&](ChunkBuf<DK>& b) {  // 16 query tokens per wave: (q_t . k_s) E(s, t) u_s
       const int t = 16 * wave + c16;
@@ -200,41 +227,50 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk) cq[kk] = frag8(b.q + koff<DK>(t, 4 * kk + g4));
       const float Lt = b.L[t];
-      for (int j = 0; j <= (wave | 1); ++j) {  // (an even wave's last half fragment is zero)
-        float m4[4] = {0.f, 0.f, 0.f, 0.f};
-        const int s0 = 16 * j + 4 * g4;
-        if (j <= wave) {
-          f32x4 a{0.f, 0.f, 0.f, 0.f};
+      // (its tiles together, so that one's products run behind the other's; what lies above the diagonal is masked)
+      auto tiles = [&](auto count) {
+        constexpr int NT = decltype(count)::value;
+        f32x4 a[NT];
 #pragma unroll
-          for (int kk = 0; kk < NK; ++kk) a = mfma32(frag8(ks + koff<DK>(16 * j + c16, 4 * kk + g4)), cq[kk], a);
+        for (int x = 0; x < NT; ++x) {
+          a[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kk = 0; kk < NK; ++kk) a[x] = mfma32(frag8(ks + koff<DK>(16 * x + c16, 4 * kk + g4)), cq[kk], a[x]);
+        }
+#pragma unroll
+        for (int x = 0; x < NT; ++x) {
+          const int s0 = 16 * x + 4 * g4;
           const f32x4 L4 = *reinterpret_cast<const f32x4*>(b.L + s0), u4 = *reinterpret_cast<const f32x4*>(b.u + s0);
+          float m4[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            if (s0 + r <= t) m4[r] = a[r] * fast_exp2(Lt - L4[r]) * u4[r] * qsc;
-            if (s0 + r == t) m4[r] += skip;
+            const float m = a[x][r] * fast_exp2(Lt - L4[r]) * u4[r] * qsc;
+            m4[r] = (s0 + r <= t ? m : 0.f) + (s0 + r == t ? skip : 0.f);
           }
+          uint2 hi, lo;
+          split4(m4, hi, lo);
+          *reinterpret_cast<uint2*>(b.m[0] + soff(t, s0 >> 3) + (s0 & 7)) = hi;
+          *reinterpret_cast<uint2*>(b.m[1] + soff(t, s0 >> 3) + (s0 & 7)) = lo;
         }
-        uint2 hi, lo;
-        split4(m4, hi, lo);
-        *reinterpret_cast<uint2*>(b.m[0] + soff(t, s0 >> 3) + (s0 & 7)) = hi;
-        *reinterpret_cast<uint2*>(b.m[1] + soff(t, s0 >> 3) + (s0 & 7)) = lo;
-      }
+      };
+      if (wave < 2) tiles(std::integral_constant<int, 2>{});
+      else tiles(std::integral_constant<int, 4>{});
     };
-    fetch(0);
-    stage(bufs[0], 0);
-    __syncthreads();  // chunk 0 is staged
-    fetch(Q);
-    weigh(bufs[0]);
-    for (int t0 = 0, cur = 0; t0 < w.n; t0 += Q, cur ^= 1) {
-      const bool more = t0 + Q < w.n;
-      __syncthreads();  // chunk t0 is weighed; the other half is consumed
-      if (more) stage(bufs[cur ^ 1], t0 + Q);
-      __syncthreads();  // chunk t0 + Q is staged
-      if (more) {
-        fetch(t0 + 2 * Q);
-        weigh(bufs[cur ^ 1]);
-      }
+    Rows x;
+    fetch(x, 0);
+    decays(x, 0);
+    stage(bufs[0], x);
+    lds_barrier();  // chunk 0 is staged
+    for (int t0 = 0, cur = 0;; t0 += Q, cur ^= 1) {
+      fetch(x, t0 + Q);
+      weigh(bufs[cur]);
+      decays(x, t0 + Q);
+      lds_barrier();  // chunk t0 is weighed; the other half is consumed
+      if (t0 + Q >= w.n) break;
+      stage(bufs[cur ^ 1], x);
+      lds_barrier();  // chunk t0 + Q is staged
     }
+    lds_barrier();
     return;
   }
 
@@ -245,9 +281,12 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
   for (int m = 0; m < NM; ++m) S[m] = w.fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + 16 * m);
   const float qsc = g.q_scale;
   const int p = 16 * wave + c16;
-  __syncthreads();
+  const int64_t ow = (int64_t)g.H * g.dv;
+  float* op = g.out + (int64_t)w.r0 * ow + (int64_t)w.h * g.dv + w.col0;
+  const uint32_t row_bytes = 4u * (uint32_t)ow, o_off = c16 * row_bytes + 4u * (16 * wave + 4 * g4);
+  lds_barrier();
   for (int t0 = 0, cur = 0; t0 < w.n; t0 += Q, cur ^= 1) {
-    __syncthreads();
+    lds_barrier();
     const ChunkBuf<DK>& b = bufs[cur];
     bf16x8_t xf[2], Sh[NK], Sl[NK];
 #pragma unroll
@@ -262,34 +301,44 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
       Sh[kk] = as_bf16x8(hi);
       Sl[kk] = as_bf16x8(lo);
     }
-    auto output = [&](int tt) {  // 16 tokens x the wave's 16 columns
-      if (t0 + 16 * tt >= w.n) return;
-      const int t = 16 * tt + c16;
-      f32x4 a{0.f, 0.f, 0.f, 0.f}, a1{0.f, 0.f, 0.f, 0.f};
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(op + (int64_t)t0 * ow), 0, (uint32_t)(min(w.n - t0, Q) - 1) * row_bytes + 4 * kPB, 0x00020000);
+    auto outputs = [&](auto first) {  // two tiles of 16 tokens x the wave's 16 columns; no branches between their products
+      constexpr int F = decltype(first)::value;
+      f32x4 a[2], a1[2];
 #pragma unroll
-      for (int kk = 0; kk < NK; ++kk) {
-        const bf16x8_t cf = frag4_4(b.q + koff<DK>(t, 4 * kk + (g4 >> 1)) + 4 * (g4 & 1),
-                                    b.q + koff<DK>(t, 4 * kk + 2 + (g4 >> 1)) + 4 * (g4 & 1));
-        a = mfma32(Sh[kk], cf, a);
-        a1 = mfma32(Sl[kk], cf, a1);
+      for (int x = 0; x < 2; ++x) {
+        const int t = 16 * (F + x) + c16;
+        a[x] = a1[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+          const bf16x8_t cf = frag4_4(b.q + koff<DK>(t, 4 * kk + (g4 >> 1)) + 4 * (g4 & 1),
+                                      b.q + koff<DK>(t, 4 * kk + 2 + (g4 >> 1)) + 4 * (g4 & 1));
+          a[x] = mfma32(Sh[kk], cf, a[x]);
+          a1[x] = mfma32(Sl[kk], cf, a1[x]);
+        }
       }
-      const float e = fast_exp2(b.L[t]) * qsc;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) a[r] = (a[r] + a1[r]) * e, a1[r] = 0.f;
+      for (int x = 0; x < 2; ++x) {
+        const int t = 16 * (F + x) + c16;
+        const float e = fast_exp2(b.L[t]) * qsc;
 #pragma unroll
-      for (int kk = 0; kk <= tt / 2; ++kk) {
-        a = mfma32(xf[kk], frag8(b.m[0] + soff(t, 4 * kk + g4)), a);
-        a1 = mfma32(xf[kk], frag8(b.m[1] + soff(t, 4 * kk + g4)), a1);
+        for (int r = 0; r < 4; ++r) a[x][r] = (a[x][r] + a1[x][r]) * e, a1[x][r] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk <= F / 2; ++kk) {
+          a[x] = mfma32(xf[kk], frag8(b.m[0] + soff(t, 4 * kk + g4)), a[x]);
+          a1[x] = mfma32(xf[kk], frag8(b.m[1] + soff(t, 4 * kk + g4)), a1[x]);
+        }
       }
-      if (t0 + t < w.n)
-        *reinterpret_cast<f32x4*>(g.out + ((int64_t)(w.r0 + t0 + t) * g.H + w.h) * g.dv + w.col0 + 16 * wave + 4 * g4) =
-            f32x4{a[0] + a1[0], a[1] + a1[1], a[2] + a1[2], a[3] + a1[3]};
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {  // (rows behind the sequence's end are not written)
+        const f32x4 o{a[x][0] + a1[x][0], a[x][1] + a1[x][1], a[x][2] + a1[x][2], a[x][3] + a1[x][3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(raw_u32x4, o), rows, o_off + 16 * (F + x) * row_bytes, 0, 0);
+      }
     };
-    output(0);
-    output(1);
-    __syncthreads();
-    output(2);
-    output(3);
+    outputs(std::integral_constant<int, 0>{});
+    lds_barrier();
+    outputs(std::integral_constant<int, 2>{});
     const float eq = fast_exp2(b.L[Q - 1]);
     bf16x8_t xh[2], xl[2];
 #pragma unroll
@@ -580,6 +629,9 @@ bool chunk_scan_ok(int mode, const ScanArgs& g) {
   auto al = [](const void* p) { return (uintptr_t)p % 16 == 0; };
   return (g.dk == 32 || g.dk == 64 || g.dk == 128) && g.dv % kPB == 0 && g.qs % 8 == 0 && g.ks % 8 == 0 &&
          g.vs % 8 == 0 && al(g.q) && al(g.k) && al(g.v) && al(g.state) && al(g.out) &&
+         // (a chunk's rows within 31-bit byte offsets, and rows that do not overlap: the one behind the last lies behind the range)
+         (int64_t)g.H * g.dv <= (1 << 22) && g.qs >= g.dk && g.qs <= (1 << 23) && g.ks >= g.dk && g.ks <= (1 << 23) &&
+         g.vs >= kPB && g.vs <= (1 << 23) && (mode != kStep || (g.gs >= 1 && g.gs <= (1 << 23))) &&
          (mode != kChannel || (g.gs % 8 == 0 && al(g.g) && !g.skip));
 }
 
@@ -588,8 +640,13 @@ bool chunk_scan_ok(int mode, const ScanArgs& g) {
   else if (g.dk == 64) hipLaunchKernelGGL((KERNEL(64)), grid, NT, 0, st, g);  \
   else hipLaunchKernelGGL((KERNEL(128)), grid, NT, 0, st, g);
 
-void launch_chunk_scan(int mode, const ScanArgs& g, int n_seq, hipStream_t st) {
+void launch_chunk_scan(int mode, const ScanArgs& g0, int n_seq, hipStream_t st) {
+  ScanArgs g = g0;
   const dim3 grid(g.dv / kPB, g.H, n_seq);
+  // One workgroup a CU: where sequences of 128 rows and more may be too many for one round, the longest start first (128 heads
+  // of 64 columns, prompts of 667, 1334 and 2000 rows: 152 -> 125 us); elsewhere their order is only a slower load in front
+  // (32 heads, the same prompts with the norm: 138 -> 140 us).
+  g.sorted = (int64_t)grid.x * grid.y * std::min(n_seq, g.T / 128) > 256;
 #define FIXED_K(D) chunk_scan_kernel<D, kFixed>
 #define STEP_K(D) chunk_scan_kernel<D, kStep>
 #define CHANNEL_K(D) channel_chunk_kernel<D>

@@ -96,13 +96,6 @@ __device__ __forceinline__ void put1(Range r, uint32_t off, int at, float x) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), r, off, at, 0);
 }
 
-// Barrier for what the waves exchange in LDS: __syncthreads() would also wait for every load of the next chunk.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // 1 / (1 + exp(-z)) with the exponential's argument in two parts and a Newton step behind the reciprocal: half the
 // instructions of 1.f / (1.f + expf(-z)), and nearer to 64 bits (largest relative error over 2^24 arguments of |z| < 1, 8 and
 // 30: 1.3e-7, 1.6e-7 and 2.1e-7; that one's 1.3e-7, 4.5e-7 and 1.4e-6).
@@ -343,19 +336,6 @@ template <int NB> struct Frags {
   uint32_t v[NB][4];  // rows g4, 4 + g4, 8 + g4 and 12 + g4 of V; bf16 bits as loaded: a conversion here would wait for the load
 };
 
-// The k-th longest of up to 16 sequences (more of them even out by themselves): the workgroups go out in this order, so
-// that the longest does not start when a short one's place is free.
-__device__ __forceinline__ int by_length(const int* seq_rows, int n_seq, int k, int lane) {
-  if (n_seq > 16) return k;
-  const int len = lane < n_seq ? seq_rows[lane + 1] - seq_rows[lane] : -1;
-  int rank = 0;
-  for (int j = 0; j < n_seq; ++j) {
-    const int other = __builtin_amdgcn_readlane(len, j);
-    rank += other > len || (other == len && j < lane);
-  }
-  return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < n_seq && rank == k));
-}
-
 // NB: blocks of 16 columns per workgroup; CT: columns per thread of the sequences that go token by token
 template <int NB, int CT>
 __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(ChunkArgs g) {
@@ -376,8 +356,7 @@ __global__ void __launch_bounds__(256, NB == 1 ? 3 : 2) delta_chunk_kernel(Chunk
   const int h = sh % g.H;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int s = by_length(g.seq_rows, g.n_seq, sh / g.H, lane);
-  const int r0 = g.seq_rows[s], n = g.seq_rows[s + 1] - r0, slot = g.slots[s];
+  const auto [r0, n, slot, s] = by_length(g.seq_rows, g.slots, g.n_seq, sh / g.H, 1);
   if (n <= 0 || r0 < 0 || r0 + n > g.T) return;
   const int col0 = h * g.dv + blk * 16 * NB;
   if (slot < 0 || slot >= g.n_slots) {  // padding rows: a defined result, no state

@@ -24,6 +24,7 @@ struct ScanArgs {
   const int* slots;
   int n_slots, T, H, dk, dv;
   int min_rows, max_rows;  // sequences with fewer / more rows in the step are another launch's
+  int sorted;              // chunked kernels: workgroups take the sequences by length
 };
 
 __device__ __forceinline__ float softplusf_(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }

@@ -305,7 +305,7 @@ extern "C" int dxm_linear_scan(int mode, float* out, float* state, int n_slots, 
   if (!seq_rows && n_seq != T_) return 4;
   if (qk_rep < 1 || H % qk_rep) return 5;
   ScanArgs g{out, state, q, k, v, qs, ks, vs, q_scale, k_scale, qk_rep, decay, gate, gs, g_bias, rate, skip, inv_tau,
-             pos, seq_rows, slots, n_slots, T_, H, dk, dv, 1, 0x7fffffff};
+             pos, seq_rows, slots, n_slots, T_, H, dk, dv, 1, 0x7fffffff, 0};
   // prompt portions in bf16: matrix-core chunks where the sizes fit; shorter runs of a sequence
   // (decode tokens among them) stay with the token scan
   if (!f32 && seq_rows && n_seq <= 65535 && T_ >= kChunkMinRows + n_seq - 1 && chunk_scan_ok(mode, g)) {

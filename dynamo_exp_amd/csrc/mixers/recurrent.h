@@ -2,6 +2,8 @@
 // sums over lane groups by DPP exchanges, 16-byte vector access, dispatch over
 // the activation element.
 #pragma once
+#include <climits>
+
 #include "../kernels/common.h"
 
 namespace {
@@ -35,6 +37,37 @@ template <int R> __device__ __forceinline__ float group_sum(float v) {
   if constexpr (R >= 8) v += dpp_f<0x141>(v);
   if constexpr (R >= 16) v += dpp_f<0x140>(v);
   return v;
+}
+
+// The sequence of a workgroup that is the k-th to go out: the k-th longest of those with `least` rows and more, so that the
+// longest does not start when a short one's place is free (of more than 64 sequences the k-th as they come: they even out
+// by themselves).  n = 0: there is none.  The lanes' loads are all asked for at once: where a launch is short, one that
+// waits for another is a hundredth of it.
+struct SeqRows {
+  int r0, n, slot, s;
+};
+__device__ __forceinline__ SeqRows by_length(const int* seq_rows, const int* slots, int n_seq, int k, int least) {
+  if (n_seq > 64) return SeqRows{seq_rows[k], seq_rows[k + 1] - seq_rows[k], slots[k], k};
+  const int lane = threadIdx.x & 63, at = min(lane, n_seq - 1);
+  const int r0 = seq_rows[at], end = seq_rows[at + 1], slot = slots[at];
+  const int len = lane < n_seq ? end - r0 : INT_MIN;
+  uint64_t any = __builtin_amdgcn_ballot_w64(len >= least);
+  if (__builtin_popcountll(any) <= k) return SeqRows{0, 0, 0, 0};
+  int rank = 0;
+  for (uint64_t left = any; left; left &= left - 1) {
+    const int j = __builtin_ctzll(left), other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  const int s = __builtin_ctzll(__builtin_amdgcn_ballot_w64(rank == k) & any);
+  return SeqRows{__builtin_amdgcn_readlane(r0, s), __builtin_amdgcn_readlane(len, s), __builtin_amdgcn_readlane(slot, s), s};
+}
+
+// Barrier for what the waves exchange in LDS: __syncthreads() would also wait for every load of the next chunk and
+// for the results' way to memory.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 template <typename T, int V> struct VecIO;

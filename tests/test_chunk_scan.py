@@ -1,0 +1,76 @@
+"""The chunked linear recurrences (csrc/mixers/chunk_scan.hip) against float64 recurrences, at the edges of their chunks and
+with sequences taken by length."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from dynamo_exp_amd.ops import recurrent as rc
+
+
+def recurrence(q, k, v, decay, step, S):
+    """One sequence, float64: q, k [n, H, dk], v [n, H, dv], decay [n, H, 1 or dk], step [n, H], S [H, dk, dv]."""
+    out = torch.empty(v.shape, dtype=torch.float64)
+    for t in range(q.shape[0]):
+        S = decay[t][..., None] * S + k[t][:, :, None] * (step[t][:, None] * v[t])[:, None]
+        out[t] = torch.einsum("hi,hij->hj", q[t], S)
+    return out, S
+
+
+def rel(a, b):
+    return float((a.double().cpu() - b).norm() / b.norm())
+
+
+ROWS = [[64], [63, 65], [8, 7, 129, 1, 128], [200, 9, 0, 66, 31, 8], [9] * 70]
+
+
+def scan(kind, rows, H, dk, dv):
+    torch.manual_seed(len(rows) + H)
+    T, n_seq, G = sum(rows), len(rows), 1 if kind == "ssd" else H
+    p = torch.randn(T, 2 * G * dk + H * dv + 8).bfloat16()
+    q, k, v = (x.cuda() for x in p.split([G * dk, G * dk, H * dv, 8], 1)[:3])
+    g = (torch.randn(T, H * dk if kind == "gla" else H) - 1.0).bfloat16()
+    bias, rate, skip = torch.randn(H * dk if kind == "gla" else H), torch.rand(H) * 3 + 0.1, torch.randn(H)
+    fixed = 1.0 - 2.0 ** (-3.0 - torch.arange(H) % 6)
+    first, starts = [0] + torch.tensor(rows).cumsum(0).tolist(), [0 if i % 2 else 5 for i in range(n_seq)]
+    slots = torch.randperm(n_seq + 1)[:n_seq].to(torch.int32)
+    if n_seq > 4:
+        slots[4] = -1  # padding rows
+    state0 = torch.randn(n_seq + 1, H, dv, dk)
+    pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)])
+    state, at = state0.cuda(), (pos.cuda(), torch.tensor(first, dtype=torch.int32).cuda(), slots.cuda())
+    if kind == "retention":
+        o = rc.retention(q, k, v, fixed.cuda(), dk ** -0.5, state, *at, H, dk, dv)
+    elif kind == "ssd":
+        o = rc.ssd(v, k, q, g.cuda(), bias.cuda(), rate.cuda(), skip.cuda(), state, *at, H, 1, dk, dv)
+    else:
+        o = rc.gated_linear_attention(q, k, v, g.cuda(), bias.cuda(), 16.0, dk ** -0.5, state, *at, H, dk, dv)
+    Q, K = (x.cpu().double().view(T, G, dk).expand(T, H, dk) for x in (q, k))
+    V, z, one = v.cpu().double().view(T, H, dv), g.double() + bias.double(), torch.ones(T, H, dtype=torch.float64)
+    Q, K = (Q * dk ** -0.5, K) if kind == "gla" else (Q, K * dk ** -0.5) if kind == "retention" else (Q, K)
+    step = torch.nn.functional.softplus(z) if kind == "ssd" else one
+    decay = {"retention": lambda: fixed.double() * one, "ssd": lambda: torch.exp(-rate.double() * step),
+             "gla": lambda: torch.sigmoid(z).pow(1 / 16)}[kind]().view(T, H, -1)
+    want, want_state = torch.zeros(T, H, dv, dtype=torch.float64), state0.double().clone()
+    for i in range(n_seq):
+        a, b, s = first[i], first[i + 1], int(slots[i])
+        if s < 0 or a == b:
+            continue
+        S = want_state[s].transpose(1, 2) * (starts[i] > 0)
+        want[a:b], S = recurrence(Q[a:b], K[a:b], V[a:b], decay[a:b], step[a:b], S)
+        want_state[s] = S.transpose(1, 2)
+        if kind == "ssd":
+            want[a:b] += skip.double()[:, None] * V[a:b]
+    return rel(o.view(T, H, dv), want), rel(state, want_state), o.view(T, H, dv), want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("kind,H,dk,dv", [("retention", 32, 128, 128), ("ssd", 64, 128, 64), ("gla", 32, 128, 128),
+                                          ("retention", 3, 64, 64), ("ssd", 4, 32, 128), ("gla", 5, 32, 64)])
+def test_chunks(rows, kind, H, dk, dv):
+    """Whatever carries a decay or the state has 16 bits of mantissa (a sum of two bf16), every sum is fp32: 2^-16 of the
+    results' norm."""
+    eo, es, o, want = scan(kind, rows, H, dk, dv)
+    assert eo < 2.0 ** -16 and es < 2.0 ** -16, (eo, es)
+    assert bool((o.cpu()[want.abs().sum((1, 2)) == 0] == 0).all())  # padding rows
