@@ -1,4 +1,5 @@
-"""Group norms of a wave each (gate_group_norm_wave_kernel in csrc/mixers/recurrent.hip) against float64."""
+"""Norms of groups and heads by lanes of a wave (gate_group_norm_wave_kernel and head_norm_gate_vec_kernel in
+csrc/mixers/recurrent.hip) against float64."""
 from __future__ import annotations
 
 import pytest
@@ -25,13 +26,15 @@ def test_group_norm_waves(n, groups, dtype, shift):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("gate_act", ["sigmoid", "silu"])
-@pytest.mark.parametrize("dv", [520, 1024, 2048])
-def test_wide_head_norm(dv, gate_act):
+@pytest.mark.parametrize("dv,shift", [(4, 0), (8, 0), (24, 1), (36, 1), (64, 0), (128, 1), (136, 0), (256, 0), (256, 1), (520, 0),
+                                      (1024, 0), (2048, 1)])
+def test_head_norm_by_runs(dv, shift, gate_act):
+    """Heads of whole runs of eight and of four, up to and beyond the width that lanes share; weights not on 16 bytes."""
     torch.manual_seed(dv)
     o, z, w = torch.randn(5, 2 * dv), torch.randn(5, 2 * dv).bfloat16(), torch.randn(2 * dv)
     x = o.double().view(5, 2, dv)
     x = (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-5)).flatten(1) * w.double()
     for gate in (z, None):
-        got = rc.head_norm_gate(o.cuda(), 2, w.cuda(), gate.cuda() if gate is not None else None, 1e-5, torch.bfloat16, gate_act)
+        got = rc.head_norm_gate(o.cuda(), 2, torch.cat([w[:shift], w]).cuda()[shift:], gate.cuda() if gate is not None else None, 1e-5, torch.bfloat16, gate_act)
         g = 1.0 if gate is None else torch.sigmoid(z.double()) * (z.double() if gate_act == "silu" else 1.0)
         assert torch.allclose(got.cpu().double(), x * g, rtol=2.0 ** -8, atol=1e-6)
