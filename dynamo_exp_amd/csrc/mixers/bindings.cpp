@@ -43,6 +43,7 @@ int64_t dxm_delta_chunk_floats(int, int, int, int, int, int, float, int64_t, int
 int dxm_delta_chunk(float*, float*, int, float*, const void*, int64_t, const void*, int64_t, const void*, int64_t, const void*,
                     int64_t, const void*, int64_t, const float*, const float*, float, float, const int64_t*, const int*,
                     const int*, int, int, int, int, hipStream_t);
+int64_t dxm_delta_prep_floats(int, int, int, const int*);
 int dxm_delta_rule(float*, float*, int, float*, const void*, int64_t, const void*, int64_t, const void*, int64_t, const void*,
                    int64_t, const void*, int64_t, const float*, const float*, float, float, const int64_t*, const int*,
                    const int*, int, int, int, int, int, int, hipStream_t);
@@ -209,6 +210,8 @@ PYBIND11_MODULE(_C_mixers, m) {
                           reinterpret_cast<const int*>(seq_rows), reinterpret_cast<const int*>(slots), n_seq, T, H, dv, S(st)),
           "delta_chunk");
   });
+  m.def("delta_prep_floats",
+        [](int T, int H, int dk, u seq_rows) { return dxm_delta_prep_floats(T, H, dk, reinterpret_cast<const int*>(seq_rows)); });
   m.def("delta_rule", [](u out, u state, int n_slots, u prep, u r, int64_t rs, u k, int64_t ks, u v, int64_t vs, u a,
                          int64_t as, u w, int64_t ws, u ab, u wb, float decay_scale, float key_eps, u pos, u seq_rows,
                          u slots, int n_seq, int T, int H, int dk, int dv, int f32, u st) {

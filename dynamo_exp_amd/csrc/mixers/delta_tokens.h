@@ -30,6 +30,30 @@ __device__ __forceinline__ float delta_decay(float wl, float wb, float decay_sca
 }
 __device__ __forceinline__ float delta_removal(float al, float ab, float u) { return sigmoidf_(al + ab) * u; }
 
+// One token on a thread's rows of CT columns: b is the unit key, the decay, removal rate * unit key, the key and the read-out.
+// (Its multiply-adds are written out: a row's result is the same bits in every kernel that takes it token by token.)
+template <int R, int CT>
+__device__ __forceinline__ void delta_step(float (*S)[kRows], const float (*b)[kRows], const float* vj, float* o_) {
+  float us[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    float a_ = 0.f;
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) a_ = fmaf(b[0][q], S[c][q], a_);
+    us[c] = group_sum<R>(a_);
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    float a_ = 0.f;
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      S[c][q] = fmaf(b[3][q], vj[c], fmaf(S[c][q], b[1][q], -(b[2][q] * us[c])));
+      a_ = fmaf(b[4][q], S[c][q], a_);
+    }
+    o_[c] = group_sum<R>(a_);
+  }
+}
+
 // kTok tokens' row vectors and the workgroup's values
 template <int R, int NT, int CT> struct DeltaLds {
   __attribute__((aligned(16))) float r[kTok][kRows * R], k[kTok][kRows * R], u[kTok][kRows * R], w[kTok][kRows * R],
@@ -182,26 +206,7 @@ __device__ __forceinline__ void delta_tokens(const DeltaArgs& g, DeltaLds<R, NT,
 #pragma unroll
       for (int c = 0; c < kCols; ++c) vj[c] = sv[tt][grp * kCols + c];
     };
-    auto step = [&](const float (*b)[kRows], const float* vj, float* o_) {
-      float us[kCols];
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) {
-        float a_ = 0.f;
-#pragma unroll
-        for (int q = 0; q < kRows; ++q) a_ += b[0][q] * S[c][q];
-        us[c] = group_sum<R>(a_);
-      }
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) {
-        float a_ = 0.f;
-#pragma unroll
-        for (int q = 0; q < kRows; ++q) {
-          S[c][q] = S[c][q] * b[1][q] - b[2][q] * us[c] + b[3][q] * vj[c];
-          a_ += b[4][q] * S[c][q];
-        }
-        o_[c] = group_sum<R>(a_);
-      }
-    };
+    auto step = [&](const float (*b)[kRows], const float* vj, float* o_) { delta_step<R, kCols>(S, b, vj, o_); };
     auto store = [&](int tt, const float* o_) {
       float* op = outp + (int64_t)(t0 + tt) * g.H * g.dv;
       if constexpr (kCols == 4) {

@@ -85,11 +85,99 @@ __global__ void __launch_bounds__(NT) delta_rule_kernel(DeltaArgs g) {
   delta_tokens<T, R, NT, CT, false>(g, lds, r0, n, h, slot, col0, g.dv);
 }
 
+// A decode step (row i is sequence i) of keys of 128 channels, in one launch: the row vectors are asked for in front of the
+// state and formed while it is on its way, one or two of them by each wave, with delta_prep_kernel's arithmetic.
+// Bound by memory from some 40 sequences on, by latency below.  Two layers with their norms in a graph, 32 heads of 128 columns,
+// 1 / 3 / 12 / 40 / 128 sequences, us: 25 / 30 / 49 / 114 / 278 with delta_prep_kernel in front and the kernel for runs of
+// tokens, 21 / 21 / 33 / 89 / 231 (168 MB of state a layer at 40: 4.7 TB/s with the norm) like this; that kernel forming the rows itself
+// 20 / 26 / 46 / 128 / 330, for it stages eight tokens.
+constexpr int kDeltaStepLanes = 8;
+bool delta_forms_itself(const int* seq_rows, int dk) { return !seq_rows && dk == kDeltaStepLanes * kRows; }
+
+template <typename T, int CT>
+__global__ void __launch_bounds__(256) delta_step_kernel(DeltaArgs g) {
+  constexpr int R = kDeltaStepLanes, D = R * kRows;
+  __shared__ __attribute__((aligned(16))) float row[5][D];  // unit key, decay, removal rate * unit key, key, read-out
+  const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, part = tid % R;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), j0 = (blockIdx.z * (256 / R) + tid / R) * CT;
+  const int slot = g.slots[t];
+  float* op = g.out + (int64_t)t * g.H * g.dv + h * g.dv + j0;
+  if (slot < 0 || slot >= g.n_slots) {  // a padding row: a defined result, no state
+    if (part == 0)
+      for (int c = 0; c < CT; ++c)
+        if (j0 + c < g.dv) op[c] = 0.f;
+    return;
+  }
+  // the wave's row: k for the first and the third one, the decay's or the read-out's else
+  const T* src = wave == 1 ? (const T*)g.w + t * g.wst : wave == 3 ? (const T*)g.r + t * g.rs : (const T*)g.k + t * g.ks;
+  const float* bias = wave == 1 ? g.w_bias : wave == 2 ? g.a_bias : nullptr;
+  float x[2], bv[2] = {0.f, 0.f}, al[2] = {0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int ch = h * D + lane + 64 * c;
+    x[c] = ldf<T>(src, ch);
+    if (wave == 2) al[c] = ldf<T>((const T*)g.a + t * g.as, ch);
+    if (bias) bv[c] = bias[ch];
+  }
+  float vj[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) vj[c] = j0 + c < g.dv ? ldf<T>((const T*)g.v + t * g.vs + h * g.dv, j0 + c) : 0.f;
+  // rows 4 (m R + part) .. + 3 of the state's columns, as delta_tokens holds them
+  float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv + j0) * D + 4 * part;
+  const bool fresh = g.pos[t] == 0;
+  float S[CT][kRows];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int m = 0; m < kRows / 4; ++m) {
+      const f32x4 y = fresh || j0 + c >= g.dv ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + c * D + 4 * m * R);
+      S[c][4 * m] = y[0], S[c][4 * m + 1] = y[1], S[c][4 * m + 2] = y[2], S[c][4 * m + 3] = y[3];
+    }
+  if (wave == 1) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) row[1][lane + 64 * c] = delta_decay(x[c], bv[c], g.decay_scale);
+  } else if (wave == 3) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) row[4][lane + 64 * c] = x[c];
+  } else {
+    const float inv = delta_key_scale(fmaf(x[1], x[1], x[0] * x[0]), g.key_eps);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const float u = x[c] * inv;
+      if (wave == 0) row[0][lane + 64 * c] = u, row[3][lane + 64 * c] = x[c];
+      else row[2][lane + 64 * c] = delta_removal(al[c], bv[c], u);
+    }
+  }
+  lds_barrier();
+  float b[5][kRows], o_[CT];
+#pragma unroll
+  for (int i = 0; i < 5; ++i)
+#pragma unroll
+    for (int m = 0; m < kRows / 4; ++m)
+      *reinterpret_cast<f32x4*>(b[i] + 4 * m) = *reinterpret_cast<const f32x4*>(&row[i][4 * (m * R + part)]);
+  delta_step<R, CT>(S, b, vj, o_);
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    if (j0 + c >= g.dv) continue;
+    if (part == 0) op[c] = o_[c];
+#pragma unroll
+    for (int m = 0; m < kRows / 4; ++m)
+      *reinterpret_cast<f32x4*>(sp + c * D + 4 * m * R) = f32x4{S[c][4 * m], S[c][4 * m + 1], S[c][4 * m + 2], S[c][4 * m + 3]};
+  }
+}
+
 // NT threads per workgroup: 64 where that covers all columns of a head, else 256.  Columns per
 // thread: the widest tile that still gives the launch two waves per SIMD (2048 on the chip) -- a
 // token's chain leaves a lone wave waiting most of the time -- down to one column for a few long prompts.
 template <typename T, int R, int CT>
 void launch_delta_ct(const DeltaArgs& g, int n_seq, hipStream_t st) {
+  if constexpr (R == kDeltaStepLanes) {
+    if (!g.prep) {
+      constexpr int cols = 256 / R * CT;
+      hipLaunchKernelGGL((delta_step_kernel<T, CT>), dim3(n_seq, g.H, (g.dv + cols - 1) / cols), dim3(256), 0, st, g);
+      return;
+    }
+  }
   const int need = R * ((g.dv + CT - 1) / CT);
   if constexpr (R < 16) {  // (a single wave staging 256 key channels would spill its registers)
     if (need <= 64) {
@@ -717,6 +805,11 @@ void launch_gate_group_norm(void* out, int64_t os, const float* y, const void* z
 
 extern "C" {
 
+// Floats of dxm_delta_rule's `prep`; 0: none, it may be null
+int64_t dxm_delta_prep_floats(int T_, int H, int dk, const int* seq_rows) {
+  return delta_forms_itself(seq_rows, dk) ? 0 : (int64_t)T_ * H * 3 * dk;
+}
+
 int dxm_delta_rule(float* out, float* state, int n_slots, float* prep, const void* r, int64_t rs, const void* k,
                    int64_t ks, const void* v, int64_t vs, const void* a, int64_t as, const void* w, int64_t ws,
                    const float* a_bias, const float* w_bias, float decay_scale, float key_eps, const int64_t* pos,
@@ -726,12 +819,16 @@ int dxm_delta_rule(float* out, float* state, int n_slots, float* prep, const voi
   if (H < 1 || dk < 1 || dv < 1 || n_slots < 1 || H > 65535 || n_seq > 0x7fffffff || (int64_t)T_ * H > 0x7fffffff)
     return 1;
   if (dk > kRows * 16) return 2;  // wider keys need more lanes per column than instantiated
-  if (!out || !state || !pos || !slots || !prep) return 3;
+  const bool self = delta_forms_itself(seq_rows, dk);
+  if (!out || !state || !pos || !slots || (!prep && !self)) return 3;
   if (!seq_rows && n_seq != T_) return 4;
-  DISPATCH_T(f32, hipLaunchKernelGGL(delta_prep_kernel<T>, dim3((unsigned)(T_ * H)), dim3(64), 0, st, prep, (const T*)k,
+  if (!self)
+    DISPATCH_T(f32, hipLaunchKernelGGL(delta_prep_kernel<T>, dim3((unsigned)(T_ * H)), dim3(64), 0, st, prep, (const T*)k,
                                      ks, (const T*)a, as, (const T*)w, ws, a_bias, w_bias, decay_scale, key_eps, H, dk));
   DeltaArgs g{};
-  g.out = out, g.state = state, g.r = r, g.k = k, g.v = v, g.rs = rs, g.ks = ks, g.vs = vs, g.prep = prep;
+  g.out = out, g.state = state, g.r = r, g.k = k, g.v = v, g.rs = rs, g.ks = ks, g.vs = vs, g.prep = self ? nullptr : prep;
+  g.a = a, g.w = w, g.as = as, g.wst = ws, g.a_bias = a_bias, g.w_bias = w_bias;
+  g.decay_scale = decay_scale, g.key_eps = key_eps;
   g.pos = pos, g.seq_rows = seq_rows, g.slots = slots, g.n_slots = n_slots, g.T = T_, g.H = H, g.dk = dk, g.dv = dv;
   const int need = (dk + kRows - 1) / kRows;
   if (need <= 4) { DISPATCH_T(f32, (launch_delta<T, 4>(g, n_seq, st))); }

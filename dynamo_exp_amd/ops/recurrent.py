@@ -356,8 +356,8 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tenso
             ws = torch.empty(floats, dtype=torch.float32, device=r.device)
             _m().delta_chunk(out.data_ptr(), state.data_ptr(), state.shape[0], ws.data_ptr(), *rows, dv, _stream())
             return out
-    # unit key, decay and removal rate * unit key of every row, formed by a pass of its own in front of the scan
-    prep = torch.empty((T, n_heads, 3, dk), dtype=torch.float32, device=r.device)
+    # unit key, decay and removal rate * unit key of every row, where a pass of its own forms them in front of the scan
+    prep = torch.empty(_m().delta_prep_floats(T, n_heads, dk, _ptr(seq_rows)), dtype=torch.float32, device=r.device)
     _m().delta_rule(out.data_ptr(), state.data_ptr(), state.shape[0], prep.data_ptr(), *rows, dk, dv, _f32(r), _stream())
     return out
 

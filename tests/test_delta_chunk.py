@@ -248,3 +248,58 @@ def test_gates_at_their_ends(z):
     rel = lambda x, y: float((x.double() - y).norm() / y.norm())
     # (fp32 sums of 128 to 2000 products, each rounded to 2^-24 of it: sqrt(2000) 2^-24 relative to the terms)
     assert rel(res[0][0], want) < 3e-6 and rel(res[0][1][0], want_state.transpose(1, 2)) < 3e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,H,dv", [(1, 1, 1), (3, 2, 20), (5, 3, 128), (2, 1, 200), (33, 8, 128), (70, 16, 48), (130, 32, 128)])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.bfloat16, False), (torch.float32, True)])
+def test_delta_step(n, H, dv, dtype, bias):
+    """A decode step of keys of 128 channels, one, two and four columns a thread: sequences in front of position 0 and behind,
+    a padding slot, rows at odd strides.  fp32 throughout: a sum of 128 products of size one is rounded at its partial sums,
+    of up to sqrt(128) and at most 2^-24 each, 16 in a row in a lane: 2^-21 of sqrt(128) an element (an element itself may be
+    smaller, where products cancel)."""
+    torch.manual_seed(n)
+    D = H * 128
+    p = torch.randn(n, 4 * D + H * dv + 3).to(dtype).cuda()
+    r, k, a, w = (p[:, i * D:(i + 1) * D] for i in range(4))
+    v = p[:, 4 * D + 1:4 * D + 1 + H * dv]
+    ab, wb = (torch.randn(D) * 0.5, torch.randn(D)) if bias else (None, None)
+    slots = torch.randperm(n + 2)[:n].to(torch.int32)
+    if n > 2:
+        slots[2] = -1
+    pos = torch.arange(n) % 3
+    state0 = torch.randn(n + 2, H, dv, 128)
+    state = state0.cuda()
+    dev = lambda t: None if t is None else t.cuda()  # noqa: E731
+    o = rc.delta_rule(r, k, v, a, w, dev(ab), dev(wb), state, pos.cuda(), None, slots.cuda(), H, 128, dv)
+    want, want_state = torch.zeros(n, H * dv, dtype=torch.float64), state0.double().clone()
+    zero = torch.zeros(D)
+    for i in range(n):
+        s = int(slots[i])
+        if s < 0:
+            continue
+        S = want_state[s].transpose(1, 2) * (int(pos[i]) > 0)
+        x = [t[i:i + 1].cpu() for t in (r, k, v, a, w)]
+        out, S = recurrence(*x, zero if ab is None else ab, zero if wb is None else wb, S, H, dv, SCALE)
+        want[i], want_state[s] = out[0], S.transpose(1, 2)
+    for got, ref in ((o, want), (state, want_state)):
+        assert float((got.double().cpu() - ref).norm()) < 2.0 ** -21 * max(float(ref.norm()), (128 * ref.numel()) ** 0.5)
+    if n > 2:
+        assert bool((o[2] == 0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,H", [(3, 2), (40, 16), (70, 32)])
+def test_delta_step_beside_prompt(n, H):
+    """A decode row's result and state are the same bits in a step of its own and beside a prompt."""
+    torch.manual_seed(n)
+    D, T = H * 128, n + 64
+    p = torch.randn(T, 5 * D).bfloat16().cuda()
+    ab, wb, state = torch.randn(D).cuda(), torch.randn(D).cuda(), torch.randn(n + 1, H, 128, 128).cuda()
+    both, pos = state.clone(), torch.cat([torch.arange(n) + 1, torch.arange(64)]).cuda()
+    rows = torch.tensor(list(range(n + 1)) + [T], dtype=torch.int32).cuda()
+    slots = torch.arange(n + 1, dtype=torch.int32).cuda()
+    secs = [p[:, i * D:(i + 1) * D] for i in range(5)]
+    a = rc.delta_rule(*(x[:n] for x in secs), ab, wb, state, pos[:n], None, slots[:n], H, 128, 128)
+    b = rc.delta_rule(*secs, ab, wb, both, pos, rows, slots, H, 128, 128)
+    assert torch.equal(a, b[:n]) and torch.equal(state[:n], both[:n])
