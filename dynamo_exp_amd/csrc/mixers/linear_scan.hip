@@ -120,6 +120,10 @@ __global__ void __launch_bounds__(256) scan_kernel(ScanArgs g) {
 // a group's 128-bit LDS reads of a row vector are neighbouring chunks and the state is read and
 // written as 16-byte runs.  The next block's eight tokens (q, k, decay logits of the head, v of the
 // workgroup's columns) are fetched into registers as 16-byte chunks while the current block's chain runs.
+// The first block is asked for in front of the state and staged while the state is on its way (its barriers wait for LDS
+// only), so that a decode step is one latency, not two.  Bound by memory: two layers with their other launches in a graph, us:
+// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 230 (its kernel at 64: 5.3
+// TB/s of state); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 135.
 template <typename T, int R, int MODE>
 __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
   constexpr int dk = 16 * R, cols = 256 / R, VEC = 16 / (int)sizeof(T);
@@ -146,21 +150,16 @@ __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
     return;
   }
   float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv + j) * dk;
-  const bool fresh = g.pos[r0] == 0;
-  float S[16];
-#pragma unroll
-  for (int qd = 0; qd < 4; ++qd) {
-    const f32x4 v4 = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + 4 * (r + R * qd));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) S[4 * qd + e] = v4[e];
-  }
   const float fixed = MODE == kFixed ? g.decay[h] : 0.f, skip = g.skip ? g.skip[h] : 0.f;
   const T* q = (const T*)g.q + (int64_t)hq * dk;
   const T* k = (const T*)g.k + (int64_t)hq * dk;
   const T* gl = (const T*)g.g + (int64_t)h * dk;
   const T* v = (const T*)g.v + (int64_t)h * g.dv + col0;
   raw_u32x4 pf[PER];
-  float2 step{0.f, 1.f};
+  // kStep: token tid's step logit as loaded (its terms are formed in commit(): here they would wait for the load)
+  T logit{};
+  bool stepped = false;
+  const float g_bias = MODE == kStep && g.g_bias ? g.g_bias[h] : 0.f, rate = MODE == kStep ? g.rate[h] : 0.f;
   auto fetch = [&](int t0) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -182,7 +181,8 @@ __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
       pf[i] = src ? *reinterpret_cast<const raw_u32x4*>(src) : raw_u32x4{0u, 0u, 0u, 0u};
     }
     if constexpr (MODE == kStep) {
-      if (tid < kTok && t0 + tid < r1) step = step_terms<T>(g, t0 + tid, h);
+      stepped = tid < kTok && t0 + tid < r1;
+      if (stepped) logit = ((const T*)g.g)[(int64_t)(t0 + tid) * g.gs + h];
     }
   };
   auto commit = [&]() {
@@ -214,15 +214,26 @@ __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
       }
     }
     if constexpr (MODE == kStep) {
-      if (tid < kTok) us_[tid] = step;
+      if (tid < kTok) {
+        const float u = softplusf_(ldf<T>(&logit, 0) + g_bias);
+        us_[tid] = stepped ? float2{u, expf(-rate * u)} : float2{0.f, 1.f};
+      }
     }
   };
-  fetch(r0);
+  fetch(r0);  // (in front of the state, which it does not wait for)
+  const bool fresh = g.pos[r0] == 0;
+  float S[16];
+#pragma unroll
+  for (int qd = 0; qd < 4; ++qd) {
+    const f32x4 v4 = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + 4 * (r + R * qd));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[4 * qd + e] = v4[e];
+  }
   for (int t0 = r0; t0 < r1; t0 += kTok) {
     const int nt = r1 - t0 < kTok ? r1 - t0 : kTok;
-    __syncthreads();  // the previous block's reads are done
+    lds_barrier();  // the previous block's reads are done
     commit();
-    __syncthreads();
+    lds_barrier();
     if (t0 + kTok < r1) fetch(t0 + kTok);
     for (int tt = 0; tt < nt; ++tt) {
       const float vj = vs_[tt * cols + cl];
