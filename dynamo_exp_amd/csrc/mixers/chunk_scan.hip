@@ -382,6 +382,9 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
 // The lanes of half an upper wave hold the 32 tokens of the same eight channels,
 // so the running log decays are DPP scans.  Channels and tokens are stored in the
 // order of the k-slots (slot_of32), so that every fragment is one 16-byte read.
+// Bound by the chain of the longest sequence's chunks, in it by the forming waves' elementwise work and the product waves'
+// latencies: the state's update without a branch per 16 channels 175 -> 167 us (32 heads of 128 / 128, 4001 tokens in three
+// prompts; with the norm 190 -> 183).
 template <int DK> struct ChannelBuf {
   static constexpr int KP = DK + 8, SP = 40;
   bf16_t qi[2][32 * KP];  // hi, lo of q e^L                  [t][n]
@@ -574,23 +577,28 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
       y0 = mfma32(Sh, q0l, y0);
       y1 = mfma32(Sh, q1l, y1);
     }
+    auto update = [&](auto some) {  // (where no channel is far, without a branch between the products)
+      constexpr bool kSome = decltype(some)::value;
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      // a forming wave's 16 channels: their keys are relative to the chunk's start, or (far) to its end
-      const f32x4 e4 = *reinterpret_cast<const f32x4*>(b.eq + 16 * m + 4 * g4);
-      const int o = (16 * m + c16) * SP + 8 * g4;
-      const bf16x8_t kh = frag8(b.ke[0] + o), kl = frag8(b.ke[1] + o);
-      if (far[m]) {
+      for (int m = 0; m < NM; ++m) {
+        // a forming wave's 16 channels: their keys are relative to the chunk's start, or (far) to its end
+        const f32x4 e4 = *reinterpret_cast<const f32x4*>(b.eq + 16 * m + 4 * g4);
+        const int o = (16 * m + c16) * SP + 8 * g4;
+        const bf16x8_t kh = frag8(b.ke[0] + o), kl = frag8(b.ke[1] + o);
+        if (kSome && far[m]) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[m][r] *= e4[r];
+          for (int r = 0; r < 4; ++r) S[m][r] *= e4[r];
+        }
+        S[m] = mfma32(kh, vf, S[m]);
+        S[m] = mfma32(kl, vf, S[m]);
+        if (!kSome || !far[m]) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[m][r] *= e4[r];
+        }
       }
-      S[m] = mfma32(kh, vf, S[m]);
-      S[m] = mfma32(kl, vf, S[m]);
-      if (!far[m]) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[m][r] *= e4[r];
-      }
-    }
+    };
+    if (any_far) update(std::true_type{});
+    else update(std::false_type{});
     if (any_far) {
       pair_by_pair(t0, 0, 0, a00);
       pair_by_pair(t0, 0, 1, a01);
