@@ -83,17 +83,10 @@ __device__ __forceinline__ void landed() {
   __syncthreads();
 }
 __device__ __forceinline__ void opaque(int& x) { asm("" : "+v"(x)); }
-// v_max3 / v_max as written: fmaxf() on matrix-core results quiets every operand first
-__device__ __forceinline__ float raw_max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-__device__ __forceinline__ float raw_max3_abs(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+// One v_maximum3, which hands a NaN on (fmaxf() would quiet every operand first).  The compiler's own: in front of inline
+// assembly it does not wait for the matrix product that an operand comes from.
+__device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float max3(float a, float b, float c) { return max2(max2(a, b), c); }
 // a number that is the same in every lane, in a scalar register
 __device__ __forceinline__ float uniform(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
 __device__ __forceinline__ float swap_max(float x) {
@@ -265,10 +258,10 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
         return MODE == kTable ? *(const lds_float*)(uintptr_t)(pen + 4 * (31 - (32 * sub + (i & 3) + 8 * (i >> 2)))) : 0.f;
       };
       if (cap > 0.f) {  // cap * tanh(x / cap)
-        float far = raw_max3_abs(s[0][0], s[0][1], s[0][2]);
+        float far = fabsf(s[0][0]);
 #pragma unroll
-        for (int i = 3; i < 16 * SUBS - 1; i += 2) far = raw_max3_abs(far, s[i >> 4][i & 15], s[(i + 1) >> 4][(i + 1) & 15]);
-        far = raw_max3_abs(far, far, s[SUBS - 1][15]);
+        for (int i = 1; i < 16 * SUBS - 1; i += 2) far = max3(far, fabsf(s[i >> 4][i & 15]), fabsf(s[(i + 1) >> 4][(i + 1) & 15]));
+        far = max2(far, fabsf(s[SUBS - 1][15]));
         if (__builtin_amdgcn_ballot_w64(!(far <= near)) == 0) {
 #pragma unroll
           for (int sub = 0; sub < SUBS; ++sub)
@@ -317,18 +310,18 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     if constexpr (MODE != kSigmoid) {
       float ta, tb;
       if constexpr (SUBS == 2) {
-        ta = fmaxf(s[0][0], s[SUBS - 1][0]), tb = fmaxf(s[0][1], s[SUBS - 1][1]);
+        ta = max2(s[0][0], s[SUBS - 1][0]), tb = max2(s[0][1], s[SUBS - 1][1]);
 #pragma unroll
         for (int i = 2; i < 16; i += 2) {
-          ta = raw_max3(ta, s[0][i], s[SUBS - 1][i]);
-          tb = raw_max3(tb, s[0][i + 1], s[SUBS - 1][i + 1]);
+          ta = max3(ta, s[0][i], s[SUBS - 1][i]);
+          tb = max3(tb, s[0][i + 1], s[SUBS - 1][i + 1]);
         }
       } else {
-        ta = fmaxf(s[0][0], s[0][1]), tb = fmaxf(s[0][2], s[0][3]);
+        ta = max2(s[0][0], s[0][1]), tb = max2(s[0][2], s[0][3]);
 #pragma unroll
         for (int i = 4; i < 16; i += 4) {
-          ta = raw_max3(ta, s[0][i], s[0][i + 1]);
-          tb = raw_max3(tb, s[0][i + 2], s[0][i + 3]);
+          ta = max3(ta, s[0][i], s[0][i + 1]);
+          tb = max3(tb, s[0][i + 2], s[0][i + 3]);
         }
       }
       // both halves of a row see the same maximum and take the same decision

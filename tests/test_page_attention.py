@@ -331,3 +331,30 @@ def test_decode_parts_of_unequal_rows(ctx, form, mask, size):
                            sink=cuda(sink)).cpu().double()
         err, top = float((got - want).abs().max()), float(want.abs().max())
         assert err < 3e-4 * (max(top, 1.0) if sig else 1.0), (parts, err)  # (bound of test_decode_rows, fp32 results)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size", [("window", 100), ("causal", 0)])
+@pytest.mark.parametrize("form", ["both", "both pair", "penalty", "sigmoid capped"])
+def test_scores_of_the_last_channels(form, mask, size):
+    """Scores that the last product of a row makes alone (the other channels are 0), most of them at 1 to 4 times the cap: what
+    the cap is decided by waits for that product."""
+    n_qh, maps, group, d, dv = FORMS["plain pair" if form == "both pair" else form]
+    torch.manual_seed(19)
+    scale, start, rows, bs, sig = 0.7 * d ** -0.5, 75, 131, 64, form == "sigmoid capped"
+    cap = 0.0 if form == "penalty" else 0.3
+    db = None if sig else (torch.rand(n_qh) * 2, torch.rand(n_qh) * 3 + 0.1)
+    hb = torch.randn(n_qh) - 2.0 if sig else None
+    kd, vd, table, kv = pages("plain pair" if form == "both pair" else form, [start + rows], bs)
+    last = (torch.arange(d) >= d - 16).double()
+    kd = (kd.view(-1, d) * last.bfloat16().cuda()).view(kd.shape)
+    q = (torch.randn(rows, n_qh, d) * 3 * last).bfloat16()
+    want = dense(q.double(), kv[0][0] * last, kv[0][1], torch.arange(start, start + rows), scale, mask, size, 0, cap, db, None, sig,
+                 hb)
+    tiles = torch.tensor(mx.tile_list(0, rows), dtype=torch.int32).cuda()
+    got = mx.attention(q.view(rows, -1).cuda(), kd, vd, torch.arange(start, start + rows).cuda(),
+                       torch.zeros(rows, dtype=torch.int32).cuda(), table, bs, n_qh, maps, group, d, dv, scale, mask, size, 1,
+                       False, tiles, rows, softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                       weights="sigmoid" if sig else "softmax", head_bias=cuda(hb)).cpu().double()
+    err, top = float((got - want).abs().max()), float(want.abs().max())  # (bound of test_prompt_rows)
+    assert err < 2.0 ** -8 * (top + (top if sig else 5.0)), err
