@@ -296,7 +296,9 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     bf16x8_t vf[VA];
 #pragma unroll
     for (int f = 0; f < VA; ++f) vf[f] = vread(vb, v_at, f);
-    if (kt + KT - 1 > wlo || (kt < wlast && !kept_tile)) {  // some key is not seen by some row
+    // Some key is not seen by some row.  (Bitwise: of the two ways of a || behind the scores' last product the compiler counts the
+    // longer one's instructions as waited for, and on the shorter one the scores are read too early)
+    if ((kt + KT - 1 > wlo) | ((kt < wlast) & !kept_tile)) {
 #pragma unroll
       for (int sub = 0; sub < SUBS; ++sub)
 #pragma unroll

@@ -98,7 +98,7 @@ def kernels():
 
 
 @pytest.mark.skipif(not OBJDUMP.exists(), reason="no disassembler")
-@pytest.mark.parametrize("kernel", ["prompt_attention_kernelILi128ELi128ELb0ELi[123]"])
+@pytest.mark.parametrize("kernel", ["prompt_attention_kernelILi128ELi128ELb0ELi[123]", "prompt_attention_kernel"])
 def test_products_are_waited_for(kernel):
     names = [n for n in kernels() if re.search(kernel, n)]
     assert names
