@@ -232,7 +232,8 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
   bf16x8_t Ph[QB], Pl[QB];
   auto softmax = [&](int t) __attribute__((always_inline)) {
     const int kt = t * kTile;
-    const bool edge = kt + kTile - 1 > p || (kt < lo && kt + kTile > keep);
+    // (bitwise: of the two ways of a || the compiler counts the longer one's instructions as a wait for the scores' last product)
+    const bool edge = (kt + kTile - 1 > p) | ((kt < lo) & (kt + kTile > keep));
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       if (MODE != kPlain && terms) {  // final scores in log2 units

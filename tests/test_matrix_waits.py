@@ -7,7 +7,6 @@ from __future__ import annotations
 import re
 import struct
 import subprocess
-from functools import lru_cache
 from pathlib import Path
 
 import pytest
@@ -87,7 +86,6 @@ def early(code):
     return found
 
 
-@lru_cache
 def kernels():
     package, out = Path(dynamo_exp_amd.__file__).parent, {}
     for library in sorted(package.glob("_C_kernels*.so")) + sorted(package.glob("_C_mixers*.so")):
@@ -98,11 +96,10 @@ def kernels():
 
 
 @pytest.mark.skipif(not OBJDUMP.exists(), reason="no disassembler")
-@pytest.mark.parametrize("kernel", ["prompt_attention_kernelILi128ELi128ELb0ELi[123]", "prompt_attention_kernel"])
-def test_products_are_waited_for(kernel):
-    names = [n for n in kernels() if re.search(kernel, n)]
-    assert names
-    assert {n: e for n in names if (e := early(kernels()[n]))} == {}
+def test_products_are_waited_for():
+    code = kernels()
+    assert any("prompt_attention_kernel" in n for n in code) and any("gemm256_kernel" in n for n in code)
+    assert {n: e for n, c in code.items() if (e := early(c))} == {}
 
 
 def test_the_check_itself():
