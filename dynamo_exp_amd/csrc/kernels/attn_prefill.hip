@@ -95,23 +95,6 @@ __device__ __forceinline__ float halves_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-// one v_max3_f32 / v_max_f32 as written: fmaxf() on MFMA results makes hipcc
-// quieten each operand first (a v_max_f32 x, x, x per value in IEEE mode),
-// tripling the row-max VALU work of a tile (48 instead of 16 ops per lane)
-__device__ __forceinline__ float vmax3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-__device__ __forceinline__ float vmax(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ float halves_max_raw(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 __device__ __forceinline__ float halves_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
@@ -292,14 +275,14 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
     // (!live1 implies a diagonal tile: the select above already set every
     // valid row's second half to -inf, and its P.V half is skipped below)
     float tmax;
-    if constexpr (kMfmaSum) {  // two independent v_max3 chains, no canonicalising moves
-      float ta = vmax(s0[0], s1[0]), tb = vmax(s0[1], s1[1]);
+    if constexpr (kMfmaSum) {  // two independent v_max3 chains (the file is built for scores that are no NaN: nothing is quieted first)
+      float ta = fmaxf(s0[0], s1[0]), tb = fmaxf(s0[1], s1[1]);
 #pragma unroll
       for (int i = 2; i < 16; i += 2) {
-        ta = vmax3(ta, s0[i], s1[i]);
-        tb = vmax3(tb, s0[i + 1], s1[i + 1]);
+        ta = fmaxf(fmaxf(ta, s0[i]), s1[i]);
+        tb = fmaxf(fmaxf(tb, s0[i + 1]), s1[i + 1]);
       }
-      tmax = halves_max_raw(vmax(ta, tb));
+      tmax = halves_max(fmaxf(ta, tb));
     } else {
       float ta = -INFINITY, tb = -INFINITY;
 #pragma unroll
