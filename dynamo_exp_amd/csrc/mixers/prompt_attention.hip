@@ -26,7 +26,7 @@
 //   * Between the products of a tile's scores the next tile's DMA goes out; all four waves' at once behind the barrier
 //     stood in each other's way.
 //   * Score terms: the tanh cap is a polynomial of degree 7 where a tile's scores are small against the cap (|x / cap| <
-//     0.36, relative error 4.3e-8; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
+//     0.36, relative error 2.3e-7; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
 //     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.
 // What bounds it: two waves a SIMD in softmax and products in turn (two maps: the matrix cores busy 45 % of the time;
 // forming a tile's scores between the weights of the one in front needs 16 registers more than there are, and spills:
@@ -73,8 +73,10 @@ enum { kPlain = 0, kTerms = 1, kSigmoid = 2, kTable = 3 };
 constexpr int kTableKeys = 1216;  // what three workgroups of a CU have room for beside their tiles
 constexpr int kTablePad = 64;     // entries for keys of a tile that a row does not see, on both sides
 
-// tanh(y) / y = sum kTanh[i] y^(2 i) for |y| <= kTanhMax, relative error 4.3e-8 (minimax, fitted in 64 bits)
-constexpr float kTanhMax = 0.36f;
+// tanh(y) / y = sum kTanh[i] y^(2 i) for |y| <= kTanhMax (minimax, fitted in 64 bits; relative error of these floats 6.2e-8, of
+// the scaled scores that the kernel forms with them 2.3e-7), of scores as large as kNearMax at most: beyond, their powers and
+// those of scale / cap would leave the number range
+constexpr float kTanhMax = 0.36f, kNearMax = 0x1p18f;
 constexpr float kTanh[4] = {0.99999996f, -0.33332261f, 0.13291534f, -0.04868792f};
 
 // every wave is done with a tile, and the DMA of the next has landed
@@ -195,7 +197,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   const float cape = uniform(MODE != kPlain && cap > 0.f ? a.scale * (2.f * kLog2e) / cap : 0.f);
   const bool terms = MODE != kPlain && (cap > 0.f || a.r1);
   // the polynomial on scores as the product leaves them, and how far it holds
-  const float y1 = terms && cap > 0.f ? a.scale / cap : 0.f, y2 = y1 * y1, near = uniform(y1 > 0.f ? kTanhMax / y1 : 0.f);
+  const float y1 = terms && cap > 0.f ? a.scale / cap : 0.f, y2 = y1 * y1, near = uniform(y1 > 0.f ? fminf(kTanhMax / y1, kNearMax) : 0.f);
   const float t0 = uniform(a.scale * kLog2e * kTanh[0]), t1 = uniform(a.scale * kLog2e * kTanh[1] * y2),
               t2 = uniform(a.scale * kLog2e * kTanh[2] * y2 * y2), t3 = uniform(a.scale * kLog2e * kTanh[3] * y2 * y2 * y2);
   const bool logs = MODE != kPlain && MODE != kTable && a.r1;

@@ -358,3 +358,26 @@ def test_scores_of_the_last_channels(form, mask, size):
                        weights="sigmoid" if sig else "softmax", head_bias=cuda(hb)).cpu().double()
     err, top = float((got - want).abs().max()), float(want.abs().max())  # (bound of test_prompt_rows)
     assert err < 2.0 ** -8 * (top + (top if sig else 5.0)), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cap", [1e6, 1e25, 1e38])
+@pytest.mark.parametrize("form", ["both", "both pair", "capped", "sigmoid capped"])
+def test_scores_and_caps_at_the_ends_of_the_number_range(form, cap):
+    """Scores of 1e20 below caps that are larger still (and, at 1e6, far above it): a row that sees itself alone gets its own
+    value."""
+    n_qh, maps, group, d, dv = FORMS["plain pair" if form == "both pair" else form]
+    torch.manual_seed(23)
+    rows, sig = 70, form == "sigmoid capped"
+    db = (torch.rand(n_qh), torch.rand(n_qh) + 0.1) if form.startswith("both") else None
+    kd, vd, table, kv = pages("plain pair" if form == "both pair" else form, [rows], 64)
+    tiles = torch.tensor(mx.tile_list(0, rows), dtype=torch.int32).cuda()
+    got = mx.attention(torch.full((rows, n_qh * d), 1e10).bfloat16().cuda(), torch.full_like(kd, 1e8), vd,
+                       torch.arange(rows).cuda(), torch.zeros(rows, dtype=torch.int32).cuda(), table, 64, n_qh, maps, group, d, dv,
+                       d ** -0.5, "window", 1, 1, False, tiles, rows, softcap=cap,
+                       dist_bias=None if db is None else tuple(map(cuda, db)), weights="sigmoid" if sig else "softmax",
+                       head_bias=torch.zeros(n_qh).cuda() if sig else None)
+    want = kv[0][1]
+    if sig and cap == 1e38:  # (2^-24 of the cap: the score is lost in its rounding)
+        want = want / 2
+    assert torch.equal(got.cpu().double(), want)
