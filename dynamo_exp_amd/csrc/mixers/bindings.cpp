@@ -39,7 +39,7 @@ int dxm_residual_step(float*, const void*, int64_t, const void*, int64_t, const 
                       const int*, int, int, const void*, int64_t, const int64_t*, int, hipStream_t);
 int dxm_act_mul(void*, const void*, int64_t, const void*, int64_t, int, int, int64_t, int, float, float, float,
                 const float*, const float*, const float*, int, int64_t, int, hipStream_t);
-int64_t dxm_delta_chunk_floats(int, int, int, int, int, int, float, int64_t, int64_t);
+int64_t dxm_delta_chunk_floats(int, int, int, int, int, int, float, int64_t, int64_t, int64_t);
 int dxm_delta_chunk(float*, float*, int, float*, const void*, int64_t, const void*, int64_t, const void*, int64_t, const void*,
                     int64_t, const void*, int64_t, const float*, const float*, float, float, const int64_t*, const int*,
                     const int*, int, int, int, int, hipStream_t);

@@ -535,13 +535,15 @@ extern "C" {
 // Floats of workspace of the chunked form for these rows (named by seq_rows), 0 where the token-by-token form takes all of
 // them: bf16 rows, enough for a long sequence (a decode step has no seq_rows at all), keys of 128 channels, whole blocks of
 // 16 value columns, decays whose product over a chunk stays far inside fp32, 16-byte aligned rows (`ptrs`, `strides`: those
-// of r, k, a, w and the state's pointer, or-ed).
+// of r, k, a, w and the state's pointer, or-ed), a chunk's rows of v and of the result within 32-bit byte offsets (`vs`: v's
+// row stride).
 int64_t dxm_delta_chunk_floats(int T_, int n_seq, int H, int dk, int dv, int f32, float decay_scale, int64_t ptrs,
-                               int64_t strides) {
+                               int64_t strides, int64_t vs) {
+  if (vs < 0 || vs > (1 << 27) || (int64_t)H * dv > (1 << 26)) return 0;
   if (f32 || dk != kD || dv % 16 || dv < 16 || ptrs % 16 || strides % 8 || !(decay_scale >= -1.f && decay_scale <= 1.f))
     return 0;
   const int64_t chunks = T_ / kC + std::min(n_seq, T_ / kLong);
-  if ((int64_t)H * dv > (1 << 25) || T_ < kLong || chunks * H > 0x7fffffff || H > 65535 ||
+  if (T_ < kLong || chunks * H > 0x7fffffff || H > 65535 ||
       (int64_t)n_seq * H * (dv / 16) > (1 << 30))
     return 0;
   return chunks * H * kChunkFloats;
@@ -555,7 +557,7 @@ int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void
   if (H < 1 || n_slots < 1 || !out || !state || !ws || !pos || !slots || !seq_rows) return 3;
   const int64_t ptrs = (int64_t)(uintptr_t)r | (int64_t)(uintptr_t)k | (int64_t)(uintptr_t)a | (int64_t)(uintptr_t)w |
                        (int64_t)(uintptr_t)state | (int64_t)(uintptr_t)ws;
-  if (!dxm_delta_chunk_floats(T_, n_seq, H, kD, dv, 0, decay_scale, ptrs, rs | ks | as | wst)) return 2;
+  if (!dxm_delta_chunk_floats(T_, n_seq, H, kD, dv, 0, decay_scale, ptrs, rs | ks | as | wst, vs)) return 2;
   FormArgs f{ws, (const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)a, (const bf16_t*)w, rs, ks, as, wst, a_bias, w_bias,
              seq_rows, slots, decay_scale, key_eps, n_seq, n_slots, T_, H};
   hipLaunchKernelGGL(delta_form_kernel, dim3((unsigned)((T_ / kC + std::min(n_seq, T_ / kLong)) * H)), dim3(256), 0, st, f);

@@ -349,9 +349,9 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tenso
     rows = (r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), a.data_ptr(), a.stride(0),
             w.data_ptr(), w.stride(0), _ptr(a_bias), _ptr(w_bias), float(decay_scale), float(key_eps), positions.data_ptr(),
             _ptr(seq_rows), state_slots.data_ptr(), n_seq, T, n_heads)
-    if seq_rows is not None and v.stride(0) <= 1 << 27:  # (the chunks take their rows of v by 32-bit byte offsets)
+    if seq_rows is not None:
         floats = _m().delta_chunk_floats(T, n_seq, n_heads, dk, dv, _f32(r), decay_scale, rows[0] | rows[2] | rows[6] | rows[8] |
-                                         state.data_ptr(), rows[1] | rows[3] | rows[7] | rows[9])
+                                         state.data_ptr(), rows[1] | rows[3] | rows[7] | rows[9], v.stride(0))
         if floats:  # the rows of long sequences in chunks (csrc/mixers/delta_chunk.hip)
             ws = torch.empty(floats, dtype=torch.float32, device=r.device)
             _m().delta_chunk(out.data_ptr(), state.data_ptr(), state.shape[0], ws.data_ptr(), *rows, dv, _stream())

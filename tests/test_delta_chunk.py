@@ -303,3 +303,15 @@ def test_delta_step_beside_prompt(n, H):
     a = rc.delta_rule(*(x[:n] for x in secs), ab, wb, state, pos[:n], None, slots[:n], H, 128, 128)
     b = rc.delta_rule(*secs, ab, wb, both, pos, rows, slots, H, 128, 128)
     assert torch.equal(a, b[:n]) and torch.equal(state[:n], both[:n])
+
+
+def test_rows_that_32_bit_offsets_do_not_reach():
+    """The chunked form asks for no workspace, and its launch refuses, where 16 rows of v or of the result span 4 GiB."""
+    m = rc._m()
+    for H, dv, vs, ok in ((2, 128, 256, True), (2, 128, 1 << 27, True), (2, 128, (1 << 27) + 8, False), (2, 128, 1 << 31, False),
+                          (1 << 13, 1 << 13, 1 << 26, True), (1 << 14, 1 << 13, 1 << 27, False)):
+        assert (m.delta_chunk_floats(64, 1, H, 128, dv, 0, SCALE, 0, 256, vs) > 0) == ok, (H, dv, vs)
+        if not ok:
+            with pytest.raises(RuntimeError, match="code 2"):
+                m.delta_chunk(16, 16, 1, 16, 16, 256, 16, 256, 16, vs, 16, 256, 16, 256, 0, 0, SCALE, 1e-6, 16, 16, 16, 1, 64, H,
+                              dv, 0)
