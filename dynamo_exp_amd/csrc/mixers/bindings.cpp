@@ -202,6 +202,9 @@ PYBIND11_MODULE(_C_mixers, m) {
           "moe_router");
   });
   m.def("delta_chunk_floats", &dxm_delta_chunk_floats);
+  m.def("delta_chunk_floats", [](int T, int n_seq, int H, int dk, int dv, int f32, float decay_scale, int64_t ptrs, int64_t strides) {
+    return dxm_delta_chunk_floats(T, n_seq, H, dk, dv, f32, decay_scale, ptrs, strides, 0);  // (rows of v as near as they may be)
+  });
   m.def("delta_chunk", [](u out, u state, int n_slots, u ws, u r, int64_t rs, u k, int64_t ks, u v, int64_t vs, u a,
                           int64_t as, u w, int64_t wst, u ab, u wb, float decay_scale, float key_eps, u pos, u seq_rows,
                           u slots, int n_seq, int T, int H, int dv, u st) {
