@@ -189,7 +189,16 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
     struct Decay {
       float L, u, w;
     } at;
-    auto stage = [&](ChunkBuf<DK>& b, const Rows& x) {
+    // where rows overlap (one row for all tokens, say), what lies behind the last one is in the range, and zeroed here
+    const int cut = g.ks < DK || g.vs < kPB ? w.n : INT_MAX;
+    auto stage = [&](ChunkBuf<DK>& b, Rows& x, int t0) {
+      if (t0 + Q > cut) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (t0 + 4 * sq + i >= cut) x.k[i] = raw_u32x4{0u, 0u, 0u, 0u};
+          if (t0 + 4 * vq + i >= cut) x.v[i] = raw_u32x4{0u, 0u, 0u, 0u};
+        }
+      }
       if (NI == 256 || tid < NI) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -259,7 +268,7 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
     Rows x;
     fetch(x, 0);
     decays(x, 0);
-    stage(bufs[0], x);
+    stage(bufs[0], x, 0);
     lds_barrier();  // chunk 0 is staged
     for (int t0 = 0, cur = 0;; t0 += Q, cur ^= 1) {
       fetch(x, t0 + Q);
@@ -267,7 +276,7 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
       decays(x, t0 + Q);
       lds_barrier();  // chunk t0 is weighed; the other half is consumed
       if (t0 + Q >= w.n) break;
-      stage(bufs[cur ^ 1], x);
+      stage(bufs[cur ^ 1], x, t0 + Q);
       lds_barrier();  // chunk t0 + Q is staged
     }
     lds_barrier();
@@ -637,10 +646,9 @@ bool chunk_scan_ok(int mode, const ScanArgs& g) {
   auto al = [](const void* p) { return (uintptr_t)p % 16 == 0; };
   return (g.dk == 32 || g.dk == 64 || g.dk == 128) && g.dv % kPB == 0 && g.qs % 8 == 0 && g.ks % 8 == 0 &&
          g.vs % 8 == 0 && al(g.q) && al(g.k) && al(g.v) && al(g.state) && al(g.out) &&
-         // (a chunk's rows within 31-bit byte offsets, and rows that do not overlap: the one behind the last lies behind the range)
-         (int64_t)g.H * g.dv <= (1 << 22) && g.qs >= g.dk && g.qs <= (1 << 23) && g.ks >= g.dk && g.ks <= (1 << 23) &&
-         g.vs >= kPB && g.vs <= (1 << 23) && (mode != kStep || (g.gs >= 1 && g.gs <= (1 << 23))) &&
-         (mode != kChannel || (g.gs % 8 == 0 && al(g.g) && !g.skip));
+         // (a chunk of 64 rows: inputs within 31-bit, results within 32-bit byte offsets)
+         (mode == kChannel ? g.gs % 8 == 0 && al(g.g) && !g.skip
+                           : (int64_t)g.H * g.dv <= (1 << 24) && std::max({g.qs, g.ks, g.vs, mode == kStep ? g.gs : 0}) <= (1 << 24));
 }
 
 #define CHUNK_DK(KERNEL, NT)                                                  \

@@ -74,3 +74,38 @@ def test_chunks(rows, kind, H, dk, dv):
     eo, es, o, want = scan(kind, rows, H, dk, dv)
     assert eo < 2.0 ** -16 and es < 2.0 ** -16, (eo, es)
     assert bool((o.cpu()[want.abs().sum((1, 2)) == 0] == 0).all())  # padding rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stride", [0, 8, 64])
+@pytest.mark.parametrize("kind", ["retention", "ssd", "gla"])
+def test_rows_that_overlap(kind, stride):
+    """Rows of one buffer that overlap or are all the same one (also the step's logits), the second sequence's end in the
+    middle of a chunk and an infinite key in its last row: the bits of the same rows laid out one behind the other."""
+    torch.manual_seed(3)
+    H, dk, dv, rows = 3, 128, 64, [64, 150]
+    T = sum(rows)
+
+    def row_view(width, step):
+        return torch.randn(T * max(step, 1) + width).bfloat16().cuda().as_strided((T, width), (step, 1))
+
+    q, k, v, g = row_view(H * dk, stride), row_view(H * dk, stride), row_view(H * dv, stride), row_view(H * dk, stride)
+    dt = row_view(H, stride // 8)
+    if stride:
+        k[-1, -1] = float("inf")
+    pos, first = torch.arange(T).cuda() + 1, torch.tensor([0, rows[0], T], dtype=torch.int32).cuda()
+    slots, state0 = torch.tensor([1, 0], dtype=torch.int32).cuda(), torch.randn(2, H, dv, dk).cuda()
+    bias, rate, fixed = torch.randn(H * dk).cuda(), torch.rand(H).cuda() + 0.1, 1.0 - torch.rand(H).cuda() / 8
+
+    def run(q, k, v, g, dt):
+        state = state0.clone()
+        if kind == "retention":
+            o = rc.retention(q, k, v, fixed, 0.1, state, pos, first, slots, H, dk, dv)
+        elif kind == "ssd":
+            o = rc.ssd(v, k, q, dt, bias[:H], rate, None, state, pos, first, slots, H, H, dk, dv)
+        else:
+            o = rc.gated_linear_attention(q, k, v, g, bias, 16.0, 0.1, state, pos, first, slots, H, dk, dv)
+        return o, state
+
+    for got, want in zip(run(q, k, v, g, dt), run(*(x.contiguous() for x in (q, k, v, g, dt)))):
+        torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
