@@ -779,26 +779,30 @@ __global__ void __launch_bounds__(256) gate_group_norm_wave_kernel(T* __restrict
   }
 }
 
+constexpr int kNarrowHead = 512;  // the head norms (GATE 1 and 2) have kernels of their own up to here
+
 template <typename T, int V, int GATE = 0>
 void launch_gate_group_norm(void* out, int64_t os, const float* y, const void* z, int64_t zs, const float* w, int rows,
                             int n_groups, int n, float eps, hipStream_t st) {
   if constexpr (V > 1) if ((uintptr_t)w % 16 == 0) {  // (longer groups would not fit a wave's registers)
     const int n_vec = rows * n_groups;
-    const dim3 waves((unsigned)((n_vec + 3) / 4));
+    const dim3 waves(((unsigned)n_vec + 3) / 4);
     auto run = [&](auto kern) {
       hipLaunchKernelGGL(kern, waves, dim3(256), 0, st, (T*)out, os, y, (const T*)z, zs, w, n_vec, n_groups, n, eps);
     };
-    if (n <= 64 * V) return run(gate_group_norm_wave_kernel<T, V, 1, GATE>);
-    if (n <= 128 * V) return run(gate_group_norm_wave_kernel<T, V, 2, GATE>);
+    if constexpr (GATE == 0 || 64 * V > kNarrowHead)
+      if (n <= 64 * V) return run(gate_group_norm_wave_kernel<T, V, 1, GATE>);
+    if constexpr (GATE == 0 || 128 * V > kNarrowHead)
+      if (n <= 128 * V) return run(gate_group_norm_wave_kernel<T, V, 2, GATE>);
     if (n <= 256 * V) return run(gate_group_norm_wave_kernel<T, V, 4, GATE>);
   }
   const dim3 grid((unsigned)((int64_t)rows * n_groups));
-  if (n > 64 * V)
-    hipLaunchKernelGGL((gate_group_norm_kernel<T, V, 256, GATE>), grid, dim3(256), 0, st, (T*)out, os, y, (const T*)z, zs, w,
-                       n_groups, n, eps);
-  else
-    hipLaunchKernelGGL((gate_group_norm_kernel<T, V, 64, GATE>), grid, dim3(64), 0, st, (T*)out, os, y, (const T*)z, zs, w,
-                       n_groups, n, eps);
+  auto run = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (T*)out, os, y, (const T*)z, zs, w, n_groups, n, eps);
+  };
+  if constexpr (GATE == 0 || 64 * V > kNarrowHead)
+    if (n <= 64 * V) return run(gate_group_norm_kernel<T, V, 64, GATE>, 64);
+  run(gate_group_norm_kernel<T, V, 256, GATE>, 256);
 }
 
 }  // namespace
@@ -933,8 +937,8 @@ int dxm_head_norm_gate(void* out, const float* o, const float* w, const void* ga
     return 0;
   }
   const int V = f32 ? 4 : 8;
-  if (dv > 512 && dv % V == 0 && gs % V == 0 && (uintptr_t)o % 16 == 0 && (uintptr_t)out % 16 == 0 &&
-      (uintptr_t)gate % 16 == 0) {  // a workgroup per head
+  if (dv > kNarrowHead && dv % V == 0 && gs % V == 0 && (uintptr_t)o % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+      (uintptr_t)gate % 16 == 0) {  // a wave per head (of up to 256 V elements, weights on 16 bytes) or a workgroup
     const int64_t os = (int64_t)H * dv;
     if (f32 && gate_act) launch_gate_group_norm<float, 4, 2>(out, os, o, gate, gs, w, rows, H, dv, eps, st);
     else if (f32) launch_gate_group_norm<float, 4, 1>(out, os, o, gate, gs, w, rows, H, dv, eps, st);
