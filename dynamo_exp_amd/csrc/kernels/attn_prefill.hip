@@ -39,30 +39,12 @@ constexpr int BQ = 32;   // query rows per wave
 constexpr int BKV = 64;  // kv rows per tile
 constexpr int kTileBytes = BKV * D * 2;  // 16 KiB
 
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 // byte offset of 16-B chunk `ch` (0..15) of row `row` inside a [64][128] bf16 tile
 __device__ __forceinline__ int tile_off(int row, int ch) { return row * 256 + 16 * (ch ^ swz(row)); }
 
-// (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
-// DMA of the next tile, which goes to the other buffer)
-__device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
-}
-// 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
-// as well, and every wait for an LDS read become one for all of them.)
-__device__ __forceinline__ void dma16(const void* from, int bytes, int off, char* to) {
-  typedef __attribute__((address_space(3))) void lds_void;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)to,
-                                           16, off, 0, 0, 0);
-}
-// every wave is done with a tile, and the DMA of the next has landed
-__device__ __forceinline__ void landed() {
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  __syncthreads();
-}
 __device__ __forceinline__ bf16x8_t as_frag(const u16x8& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
 // ---------------------------------------------------------------------------
@@ -201,8 +183,8 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
       const int bytes = 2 * D * min(ctx - j0, BKV);
 #pragma unroll
       for (int k = 0; k < KPW; ++k) {
-        dma16(k_cache + base, bytes, src_off[k], kb + (KPW * wid + k) * 1024);
-        dma16(v_cache + base, bytes, src_off[k], vb + (KPW * wid + k) * 1024);
+        dma16(k_cache + base, bytes, src_off[k], (lds_void*)(kb + (KPW * wid + k) * 1024));
+        dma16(v_cache + base, bytes, src_off[k], (lds_void*)(vb + (KPW * wid + k) * 1024));
       }
     } else {
 #pragma unroll
@@ -210,8 +192,8 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
         const int at = 4 * (KPW * wid + k), j = __builtin_amdgcn_readfirstlane(j0 + at);
         const int64_t base = ((int64_t)block(j) * n_kv_heads + kvh) * head_stride + (int64_t)(j & (block_size - 1)) * D;
         const int bytes = __builtin_amdgcn_readfirstlane(2 * D * max(min(ctx - j, 4), 0));
-        dma16(k_cache + base, bytes, src_off[k] - 2 * D * at, kb + (KPW * wid + k) * 1024);
-        dma16(v_cache + base, bytes, src_off[k] - 2 * D * at, vb + (KPW * wid + k) * 1024);
+        dma16(k_cache + base, bytes, src_off[k] - 2 * D * at, (lds_void*)(kb + (KPW * wid + k) * 1024));
+        dma16(v_cache + base, bytes, src_off[k] - 2 * D * at, (lds_void*)(vb + (KPW * wid + k) * 1024));
       }
     }
   };

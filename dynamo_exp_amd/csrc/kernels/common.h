@@ -48,6 +48,25 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // enough (|err| < 2^-126)
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// ---- tiles on their way to LDS by DMA, and fragments read transposed from them
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+// (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
+// DMA of the next tile, which goes to the other buffer)
+__device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
+}
+// 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
+// as well, and every wait for an LDS read become one for all of them.)
+__device__ __forceinline__ void dma16(const void* from, int bytes, int off, lds_void* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), to, 16, off, 0, 0, 0);
+}
+// every wave is done with a tile, and the DMA of the next has landed
+__device__ __forceinline__ void landed() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+}
+
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

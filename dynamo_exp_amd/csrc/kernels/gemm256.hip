@@ -73,8 +73,6 @@
 
 namespace {
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 constexpr int kBM = 256, kBN = 256, kBK = 64;
 constexpr int kTile = 256 * 128;   // one operand tile: 256 rows x 64 bf16
 constexpr int kBuf = 2 * kTile;    // x tile + w tile

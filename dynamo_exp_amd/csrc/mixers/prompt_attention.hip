@@ -79,11 +79,6 @@ constexpr int kTablePad = 64;     // entries for keys of a tile that a row does 
 constexpr float kTanhMax = 0.36f, kNearMax = 0x1p18f;
 constexpr float kTanh[4] = {0.99999996f, -0.33332261f, 0.13291534f, -0.04868792f};
 
-// every wave is done with a tile, and the DMA of the next has landed
-__device__ __forceinline__ void landed() {
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  __syncthreads();
-}
 __device__ __forceinline__ void opaque(int& x) { asm("" : "+v"(x)); }
 // One v_maximum3, which hands a NaN on (fmaxf() would quiet every operand first).  The compiler's own: in front of inline
 // assembly it does not wait for the matrix product that an operand comes from.

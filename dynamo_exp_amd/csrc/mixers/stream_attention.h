@@ -31,23 +31,13 @@ __device__ __forceinline__ void put_v(bf16_t* Vt, const raw_u32x4* r, int kg, in
 __device__ __forceinline__ int piece_xor(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 template <int RB> __device__ __forceinline__ int image_off(int row, int ch) { return row * RB + 16 * (ch ^ piece_xor(row)); }
 
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-typedef __attribute__((address_space(3))) void lds_void;
 // LDS by its own addresses: through a pointer each would be added to the array's (the front of LDS) in a vector instruction
 typedef __attribute__((address_space(3))) raw_u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) float lds_float;
 __device__ __forceinline__ bf16x8_t lds_frag(uint32_t at) { return __builtin_bit_cast(bf16x8_t, *(const lds_u32x4*)(uintptr_t)at); }
 
-// (a function of its own: the compiler then knows that the read is of what p names, and does not wait in front of it for the
-// DMA of the next tile, which goes to the other buffer)
-__device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
-}
-// 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
-// as well, and every wait for an LDS read become one for all of them.)
 __device__ __forceinline__ void dma16(const void* from, int bytes, int off, uint32_t to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), (lds_void*)(uintptr_t)to,
-                                           16, off, 0, 0, 0);
+  ::dma16(from, bytes, off, (lds_void*)(uintptr_t)to);
 }
 
 __device__ __forceinline__ bf16x8_t frag16(const bf16_t* p) {
