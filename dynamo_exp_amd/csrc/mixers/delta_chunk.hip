@@ -25,9 +25,9 @@
 // factors times it).  It shows in the rows or stays in the state, and a workgroup that meets one takes its columns again,
 // token by token.
 // 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 211 + 99 us, each
-// profiled by itself (in a row, with the layer's norm of 25: 312); a prompt of 600 beside 30 single tokens 704 -> 77, the
-// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 4000 cycles where three
-// workgroups share a CU, 1088 of a wave's matrix instructions each, so that the matrix cores are busy 54 % of the time (a
+// profiled by itself (in a row, with the layer's norm of 24: 314); a prompt of 600 beside 30 single tokens 704 -> 77, the
+// layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 3700 cycles where three
+// workgroups share a CU, 1088 of a wave's matrix instructions each, so that the matrix cores are busy 59 % of the time (a
 // chain alone: 2400 cycles a chunk); 162 us with the loads taken out.
 #include <algorithm>
 

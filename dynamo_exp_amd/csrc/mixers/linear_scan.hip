@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(256) scan_kernel(ScanArgs g) {
 // workgroup's columns) are fetched into registers as 16-byte chunks while the current block's chain runs.
 // The first block is asked for in front of the state and staged while the state is on its way (its barriers wait for LDS
 // only), so that a decode step is one latency, not two.  Bound by memory: two layers with their other launches in a graph, us:
-// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 230 (its kernel at 64: 5.3
+// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 230 (its kernel at 64: 5.2
 // TB/s of state); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 135.
 template <typename T, int R, int MODE>
 __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {

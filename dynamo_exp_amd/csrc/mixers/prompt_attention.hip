@@ -32,8 +32,8 @@
 // forming a tile's scores between the weights of the one in front needs 16 registers more than there are, and spills:
 // 1.25 x slower), and a wave's issue where there are score terms.  32 heads, ragged prompts of about 4000 tokens, us,
 // with fragments read one product ahead -> now: two maps with values of 256, window 1024 + 64, 5003 rows beside 16 decode
-// rows, with the combine: 287 -> 270; shared row 256 / 192 causal 124 -> 113 (870 TFLOP/s); cap + penalty, window 1024,
-// 138 -> 99 (600 rows behind 2000 cached, window 512: 33 -> 27); sigmoid 86 -> 81.  (The register-staged 16x16x32 forms
+// rows, with the combine: 288 -> 270; shared row 256 / 192 causal 125 -> 113 (870 TFLOP/s); cap + penalty, window 1024,
+// 138 -> 97 (600 rows behind 2000 cached, window 512: 36 -> 25); sigmoid 85 -> 78.  (The register-staged 16x16x32 forms
 // of tile_attention.hip, stream and latent prefill, which it took over from: two maps and their combine 776, 242, 313.)
 #include <type_traits>
 
@@ -496,8 +496,8 @@ int dxm_prompt_attention(void* out, const void* q, int64_t q_stride, const void*
   if (same) return prompt_heads<256, 192, true, kPlain, false, bf16_t>(a, n_tiles, st);
   if (dv == 256) return prompt_heads<128, 256, false, kPlain, true, float>(a, n_tiles, st);
   if (wfn) return prompt_heads<128, 128, false, kSigmoid, false, bf16_t>(a, n_tiles, st);
-  // Every row sees keys within `size` of it.  Table / logarithms, us, window 1024, 4500 rows of 32 heads: 99 / 112; 512, 5000
-  // of 16: 41 / 46
+  // Every row sees keys within `size` of it.  Table / logarithms, us, at 1216 / 1217 keys, 4500 rows of 32 heads 115 / 117, 5000
+  // of 16 62 / 82 (of 1024 keys, 4500 rows of 32 heads: 97)
   if (r1 && mask && !keep && size <= kTableKeys) return prompt_heads<128, 128, false, kTable, false, bf16_t>(a, n_tiles, st);
   if (terms) return prompt_heads<128, 128, false, kTerms, false, bf16_t>(a, n_tiles, st);
   if (fine) return prompt_heads<128, 128, false, kPlain, true, bf16_t>(a, n_tiles, st);
