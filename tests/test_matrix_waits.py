@@ -11,7 +11,7 @@ from pathlib import Path
 
 import pytest
 
-import dynamo_exp_amd
+from dynamo_exp_amd import _native
 
 OBJDUMP = Path("/opt/rocm/llvm/bin/llvm-objdump")
 # gfx950: passes of the matrix pipe + 4 (fp32 products: + 2); what the compiler itself leaves where nothing branches
@@ -87,9 +87,9 @@ def early(code):
 
 
 def kernels():
-    package, out = Path(dynamo_exp_amd.__file__).parent, {}
-    for library in sorted(package.glob("_C_kernels*.so")) + sorted(package.glob("_C_mixers*.so")):
-        for code in device_code(library):
+    out = {}
+    for module in (_native.kernels(), _native.mixers()):
+        for code in device_code(Path(module.__file__)):
             r = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "-"], input=code, capture_output=True, check=True)
             out |= functions(r.stdout.decode())
     return out
