@@ -31,7 +31,9 @@ __device__ __forceinline__ float delta_decay(float wl, float wb, float decay_sca
 __device__ __forceinline__ float delta_removal(float al, float ab, float u) { return sigmoidf_(al + ab) * u; }
 
 // One token on a thread's rows of CT columns: b is the unit key, the decay, removal rate * unit key, the key and the read-out.
-// (Its multiply-adds are written out: a row's result is the same bits in every kernel that takes it token by token.)
+// (Its multiply-adds are written out: a row's result is the same bits in every kernel that takes it token by token.  The sign
+// is where it leaves the state's old value in its register: with it on the product the compiler copied the tile first, 32
+// sequences of one to 27 rows, 32 heads, 50.0 us instead of 46.6.)
 template <int R, int CT>
 __device__ __forceinline__ void delta_step(float (*S)[kRows], const float (*b)[kRows], const float* vj, float* o_) {
   float us[CT];
@@ -47,7 +49,7 @@ __device__ __forceinline__ void delta_step(float (*S)[kRows], const float (*b)[k
     float a_ = 0.f;
 #pragma unroll
     for (int q = 0; q < kRows; ++q) {
-      S[c][q] = fmaf(b[3][q], vj[c], fmaf(S[c][q], b[1][q], -(b[2][q] * us[c])));
+      S[c][q] = fmaf(b[3][q], vj[c], -fmaf(-S[c][q], b[1][q], b[2][q] * us[c]));
       a_ = fmaf(b[4][q], S[c][q], a_);
     }
     o_[c] = group_sum<R>(a_);
