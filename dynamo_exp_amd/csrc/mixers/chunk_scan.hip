@@ -80,13 +80,18 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kPB = 64;  // columns of a workgroup
 
 // the workgroup's sequence: its rows and slot; false: nothing to do
+// Whole layers of 24 / 32 / 40 or 48 prompts of 3000 to 4000 tokens together, us, in order: state-space duality (128 heads) 222 /
+// 276 / 252, retention (32) 110 / 138 / 134, gated linear attention (32) 147 / 180 / 208; as they come 210 / 256 / 223, 105 /
+// 127 / 118, 147 / 172 / 186; of 17 prompts 194, 100, 137 and 188, 101, 144.
+constexpr int kInOrder = 24;
+
 struct Walk {
   int r0, n, h, hq, col0, slot;
   bool fresh;
 };
 __device__ __forceinline__ bool open_walk(const ScanArgs& g, Walk& w) {
   const int z = blockIdx.z;
-  const SeqRows q = g.sorted ? by_length(g.seq_rows, g.slots, gridDim.z, z, g.min_rows)
+  const SeqRows q = g.sorted ? by_length<false>(g.seq_rows, g.slots, gridDim.z, z, g.min_rows, kInOrder)
                              : SeqRows{g.seq_rows[z], g.seq_rows[z + 1] - g.seq_rows[z], g.slots[z], z};
   w.h = blockIdx.y;
   w.hq = w.h / g.qk_rep;
@@ -661,7 +666,7 @@ void launch_chunk_scan(int mode, const ScanArgs& g0, int n_seq, hipStream_t st) 
   const dim3 grid(g.dv / kPB, g.H, n_seq);
   // One workgroup a CU: where sequences of 128 rows and more may be too many for one round, the longest start first (128 heads
   // of 64 columns, prompts of 667, 1334 and 2000 rows: 152 -> 125 us); elsewhere their order is only a slower load in front
-  // (32 heads, the same prompts with the norm: 138 -> 140 us).
+  // (32 heads, the same prompts with the norm: 138 -> 140 us).  Up to kInOrder sequences long enough for a chunk.
   g.sorted = (int64_t)grid.x * grid.y * std::min(n_seq, g.T / 128) > 256;
 #define FIXED_K(D) chunk_scan_kernel<D, kFixed>
 #define STEP_K(D) chunk_scan_kernel<D, kStep>

@@ -77,14 +77,15 @@ def test_chunks(rows, kind, H, dk, dv):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [[130, 9, 0, 300, 130, 7, 64, 200], [300, 8, 200, 200, 129, 31, 7, 1, 0, 64], [10] * 70], ids=len)
+@pytest.mark.parametrize("rows", [[130, 9, 0, 300, 130, 7, 64, 200], [300, 8, 200, 200, 129, 31, 7, 1, 0, 64],
+                                  [16 + i % 7 * 9 for i in range(36)] + [5, 0, 300], [10] * 70], ids=len)
 @pytest.mark.parametrize("kind,H,dk,dv", [("retention", 32, 128, 128), ("ssd", 64, 128, 64), ("gla", 32, 128, 128),
                                           ("retention", 24, 32, 128)])
 def test_sequences_by_length(rows, kind, H, dk, dv):
     """More workgroups of long sequences than the chip takes at once, so that they go out by length: equal lengths, padding
     slots, runs too short for a chunk and empty ones among them, and more sequences than are put in order."""
     if (kind, H) == ("retention", 24):
-        rows = rows * 2 if len(rows) < 20 else rows + [9] * 40
+        rows = rows * 2 if len(rows) < 20 else rows + [9] * 20
     assert H * (dv // 64) * min(len(rows), sum(rows) // 128) > 256  # launch_chunk_scan's rule
     eo, es, o, want = scan(kind, rows, H, dk, dv)
     assert eo < 2.0 ** -16 and es < 2.0 ** -16, (eo, es)  # (test_chunks)
