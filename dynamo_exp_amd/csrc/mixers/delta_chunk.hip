@@ -25,7 +25,7 @@
 // factors times it).  It shows in the rows or stays in the state, and a workgroup that meets one takes its columns again,
 // token by token.
 // 4001 tokens in three prompts, 32 heads: 1287 us token by token + 85 us for its elementwise pass -> 211 + 99 us, each
-// profiled by itself (in a row, with the layer's norm of 24: 314); a prompt of 600 beside 30 single tokens 704 -> 77, the
+// profiled by itself (in a row, with the layer's norm of 24: 314); a prompt of 600 beside 30 single tokens 704 -> 89, the
 // layer without its norm.  Bound by the chain of the longest prompt's chunks: 125 of them at 3700 cycles where three
 // workgroups share a CU, 1088 of a wave's matrix instructions each, so that the matrix cores are busy 59 % of the time (a
 // chain alone: 2400 cycles a chunk); 162 us with the loads taken out.
@@ -39,7 +39,7 @@ constexpr int kC = 16;    // tokens per chunk
 // A sequence with at least this many rows in the step goes in chunks, a shorter one (a decode row beside a prompt among
 // them) token by token, whatever else is in the step: what shares a step does not change a sequence's arithmetic.
 // From 32 rows on the chunks are no slower: one prompt of 32 rows 23 us either way, 63 36 token by token and 22 in chunks;
-// 16 prompts of 32 78 and 75; 600 rows beside 30 decode rows 704 all token by token, 138 all in chunks, 112 like this.
+// 16 prompts of 32 78 and 75; 600 rows beside 30 decode rows 704 all token by token, 138 all in chunks, 102 like this.
 constexpr int kLong = 32;
 constexpr int kD = 128;   // key channels
 constexpr int kPad = 4;   // floats of padding per LDS row
@@ -571,11 +571,11 @@ int dxm_delta_chunk(float* out, float* state, int n_slots, float* ws, const void
   ChunkArgs c{d, out, state, ws, (const bf16_t*)v, vs, pos, seq_rows, slots, n_seq, n_slots, T_, H, dv};
   const int64_t heads = ((int64_t)n_seq * H + 7) / 8 * 8;
   // Long sequences gain nothing from two column blocks a workgroup (one / two, us, whole layer of 32 heads: three prompts of
-  // 4001 tokens together 363 / 431, four of 3000 280 / 298, six of 5000 443 / 444); short ones in great numbers do, in tiles
-  // of four columns a thread by four times fewer workgroups (32 prompts of 16 tokens 131 / 116, 64 of them 244 / 191, one of
-  // 600 beside 100 decode rows 210 / 205).  Up to about a thousand (sequence, head) there are too few of them for that: 600
-  // tokens beside 12, 30 and 48 decode rows 89 / 90, 112 / 114 and 138 / 139, 20-token prompts beside 12 46 / 63, 16 prompts
-  // of 16 tokens 64 / 65.
+  // 12003 tokens together 904 / 1095, four of 3000 238 / 256, six of 5000 385 / 381); short ones in great numbers do, in tiles
+  // of four columns a thread by four times fewer workgroups (32 prompts of 16 tokens 131 / 116, 64 of them 249 / 196, one of
+  // 600 beside 100 decode rows 203 / 195).  Up to about a thousand (sequence, head) there are too few of them for that: 600
+  // tokens beside 12, 30 and 48 decode rows 72 / 93, 102 / 103 and 128 / 128, three 20-token prompts beside 12 40 / 52, 16
+  // prompts of 16 tokens 64 / 66.
   if (dv % 32 == 0 && heads >= 1024)
     hipLaunchKernelGGL((delta_chunk_kernel<2, 4>), dim3((unsigned)(heads * (dv / 32))), dim3(256), 0, st, c);
   else
