@@ -59,7 +59,9 @@ def _k():
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the current device's current stream as a raw handle (the Stream object that torch.cuda.current_stream() builds
+    # for it costs 2.8 us of a launch's 13 on the host)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _chk(t: torch.Tensor, dtype=None, name="tensor"):

@@ -22,6 +22,7 @@ import math
 import torch
 
 from .. import _native
+from . import _stream
 
 MASKS = {"causal": 0, "window": 1, "chunk": 2}
 ACTS = {"relu": 0, "silu": 1, "gelu_tanh": 2, "sigmoid": 3, "relu2": 4, "tanh": 5, "swiglu_clamp": 6}
@@ -42,10 +43,6 @@ LATENT_TARGET_GROUPS = 512
 
 def _m():
     return _native.mixers()
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def _f32(t: torch.Tensor) -> int:
