@@ -87,7 +87,9 @@ int dxm_group_decode(float*, const void*, int64_t, const void*, const void*, con
 int dxm_prompt_attention_ok(int, int, int, int, int, int, int, int, int, int, int);
 int dxm_prompt_attention(void*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*, int,
                          int, const int*, int, int, int, int, int, int, int, int, float, int, int, float, const float*,
-                         const float*, int, const float*, const void*, int64_t, int, const float*, int, int, hipStream_t);
+                         const float*, int, const float*, const void*, int64_t, int, const float*, int, int, float*, int,
+                         int, hipStream_t);
+int dxm_prompt_attention_parts(int, int, int, int, int, int, int, int, int, int, int, int, int, int);
 int dxm_stream_prefill_ok(int, int, int, int, int, int);
 int dxm_stream_prefill(void*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*, int,
                        int, const int*, int, int, int, int, int, int, int, float, int, int, int, hipStream_t);
@@ -288,19 +290,25 @@ PYBIND11_MODULE(_C_mixers, m) {
     check(dxm_diff_combine(P(out), F(a), n_vec, dv, lam, post, eps, P(gate), gs, H, f32, S(st)), "diff_combine");
   });
   m.def("tile_attention_ok", &dxm_tile_attention_ok);
+  m.def("prompt_attention_parts", &dxm_prompt_attention_parts);
   m.def("tile_attention", [](u out, u q, int64_t qs, u kc, u vc, u pos, u seq, u bt, int bts, int bs, u tiles,
                              int n_tiles, int n_qh, int maps, int group, int d, int dv, int Wk, int Wv, float scale,
                              int mask, int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs,
-                             int keep, u sink, int out_f32, int fine, u st) {
+                             int keep, u sink, int out_f32, int fine, u ws, int parts, int rows, u st) {
     // pages of whole tiles and heads of 128 columns (or one shared row of 256); a tile's bytes are counted in 31 bits
     if (qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && Wk <= 1 << 23 && Wv <= 1 << 23 && (q | kc | vc | out) % 16 == 0 &&
-        dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, kc == vc, cap > 0.f || r1, wfn, out_f32, fine))
+        dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, kc == vc, cap > 0.f || r1, wfn, out_f32, fine)) {
       check(dxm_prompt_attention(P(out), P(q), qs, P(kc), P(vc), reinterpret_cast<const int64_t*>(pos),
                                  reinterpret_cast<const int*>(seq), reinterpret_cast<const int*>(bt), bts, bs,
                                  reinterpret_cast<const int*>(tiles), n_tiles, n_qh, maps, group, d, dv, Wk, Wv, scale,
                                  mask, size, cap, F(r1), F(r2), wfn, F(hbias), P(gate), gs, keep, F(sink), out_f32, fine,
-                                 S(st)),
+                                 F(ws), parts, rows, S(st)),
             "prompt_attention");
+      if (parts > 1)
+        check(dxm_merge_parts(P(out), F(ws), (int64_t)rows * n_qh, parts, dv, wfn, P(gate), gs, n_qh, maps, F(sink), out_f32,
+                              S(st)),
+              "merge_parts");
+    }
     // plain heads over pages of whole tiles take the streaming kernel
     else if (cap == 0.f && !r1 && !wfn && !hbias && !gate && !keep && !sink && !out_f32 && qs % 8 == 0 &&
         (q | kc | vc) % 16 == 0 && dxm_stream_prefill_ok(d, dv, maps, group, bs, mask))

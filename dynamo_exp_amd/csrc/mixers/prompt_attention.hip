@@ -28,6 +28,11 @@
 //   * Score terms: the tanh cap is a polynomial of degree 7 where a tile's scores are small against the cap (|x / cap| <
 //     0.36, relative error 2.3e-7; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
 //     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.
+//   * Few rows behind a long context leave most of the chip idle, and a workgroup alone on its CU takes 0.5 to 1 us for 32
+//     keys, whatever it does with them: there the keys go out in parts (dxm_prompt_attention_parts, grid z), whose sums
+//     merge_parts joins.  One prompt of 16 rows behind 2000 keys, 32 heads, us of the GPU: causal 41 -> 13, two maps in
+//     chunks of 2048 68 -> 23, shared row 256 / 192 60 -> 17, cap + penalty in a window of 1024 39 -> 14; two of 300
+//     together behind 1500: 35 -> 26, 62 -> 44, 51 -> 36, 41 -> 27.
 // What bounds it: two waves a SIMD in softmax and products in turn (two maps: the matrix cores busy 45 % of the time;
 // forming a tile's scores between the weights of the one in front needs 16 registers more than there are, and spills:
 // 1.25 x slower), and a wave's issue where there are score terms.  32 heads, ragged prompts of about 4000 tokens, us,
@@ -35,6 +40,8 @@
 // rows, with the combine: 288 -> 270; shared row 256 / 192 causal 125 -> 113 (870 TFLOP/s); cap + penalty, window 1024,
 // 138 -> 97 (600 rows behind 2000 cached, window 512: 36 -> 25); sigmoid 85 -> 78.  (The register-staged 16x16x32 forms
 // of tile_attention.hip, stream and latent prefill, which it took over from: two maps and their combine 776, 242, 313.)
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "stream_attention.h"
@@ -65,9 +72,12 @@ struct PromptArgs {
   int64_t gate_stride;
   int keep;           // window mask: the first `keep` keys stay visible
   const float* sink;  // [n_qh], softmax only
+  float* ws;          // parts > 1: [rows, n_qh, parts, 2 + DV]
+  int parts, rows;
 };
 
-constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+constexpr int kLeastTiles = 4;  // of a part, of several
 // kTable: cap and / or penalty where a row sees at most kTableKeys keys back: the penalty is a table of the distance in LDS
 enum { kPlain = 0, kTerms = 1, kSigmoid = 2, kTable = 3 };
 constexpr int kTableKeys = 1216;  // what three workgroups of a CU have room for beside their tiles
@@ -124,11 +134,19 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   const int hi = p0 + min(n, ROWS) - 1;
   const int first = first_key(p0, a.mask, a.size) >> SH, last = hi >> SH;
   const int kept = a.mask == 1 ? min((a.keep + KT - 1) >> SH, first) : 0;  // tiles of kept keys in front of the window's
+  // tiles in order: the kept ones, then the window's; of them this part's
+  const int total = kept + last - first + 1, part = blockIdx.z;
+  const int per_part = max((total + a.parts - 1) / a.parts, kLeastTiles), i0 = part * per_part, i1 = min(i0 + per_part, total);
   // rows beyond n repeat the last one and are not stored
   const int myrow = min(rw + r, n - 1), my = p0 + myrow, mylo = first_key(my, a.mask, a.size);
   const int wlo = p0 + min(rw, n - 1), whi = p0 + min(rw + 31, n - 1);  // the wave's first and last position
   const int wfirst = first_key(wlo, a.mask, a.size), wlast = first_key(whi, a.mask, a.size);
   const int keep = a.mask == 1 ? a.keep : 0;
+  float* const ws = a.ws + (((int64_t)(row0 + myrow) * a.n_qh + qh) * a.parts + part) * (2 + DV);
+  if (i0 >= i1) {  // (never the first part) no tile: sum 0
+    if (rw + r < n && row0 + myrow < a.rows && h == 0) *reinterpret_cast<float2*>(ws) = float2{MODE == kSigmoid ? 0.f : -INFINITY, 0.f};
+    return;
+  }
   bf16x8_t qf[QR];
   const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)smem;
   const uint32_t ql = base + 2 * kStage + (wid * (KS - QR) * 64 + lane) * 16;  // the lane's own pieces
@@ -376,25 +394,38 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     }
     if constexpr (kEager) __builtin_amdgcn_s_setprio(1);
   };
-  // tiles in order: the kept ones, then the window's
-  const int total = kept + last - first + 1;
   auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
   static_assert(ND <= KS, "a DMA instruction beside a product at most");
-  find(tile(0));
+  find(tile(i0));
 #pragma unroll
   for (int k = 0; k < ND; ++k) fetch(base, k);
   landed();
-  for (int i = 0; i < total; i += 2) {  // (behind the last tile it is fetched again: no branch among the products)
-    find(tile(min(i + 1, total - 1)));
+  for (int i = i0; i < i1; i += 2) {  // (behind the last tile it is fetched again: no branch among the products)
+    find(tile(min(i + 1, i1 - 1)));
     step(std::integral_constant<int, 0>{}, tile(i));
     landed();
-    if (i + 1 < total) {
-      find(tile(min(i + 2, total - 1)));
+    if (i + 1 < i1) {
+      find(tile(min(i + 2, i1 - 1)));
       step(std::integral_constant<int, 1>{}, tile(i + 1));
       landed();
     }
   }
 
+  const bool ok = rw + r < n;
+  if (a.parts > 1) {  // sums as they are: gate, sink and denominator come with the join
+    if (!ok || row0 + myrow >= a.rows) return;
+    const float l = MODE == kSigmoid ? 1.f : swap_sum(l_i);
+    if (h == 0) *reinterpret_cast<float2*>(ws) = float2{MODE == kSigmoid ? 0.f : m_i * kLn2, l};
+#pragma unroll
+    for (int dt = 0; dt < NC; ++dt)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        float* o = ws + 2 + dt * 32 + 8 * g4 + 4 * h;
+        *reinterpret_cast<float2*>(o) = float2{O[dt][4 * g4], O[dt][4 * g4 + 1]};
+        *reinterpret_cast<float2*>(o + 2) = float2{O[dt][4 * g4 + 2], O[dt][4 * g4 + 3]};
+      }
+    return;
+  }
   float inv = 1.f;
   if constexpr (MODE != kSigmoid) {
     float l = swap_sum(l_i);
@@ -402,7 +433,6 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     inv = 1.f / l;
   }
   if (a.gate) inv /= 1.f + __expf(-bf16_to_f32(a.gate[(int64_t)(row0 + myrow) * a.gate_stride + head]));
-  const bool ok = rw + r < n;
   OutT* o = (OutT*)a.out + ((int64_t)(row0 + myrow) * a.n_qh + qh) * DV;
   // lane (r, h) holds columns 8 g4 + 4 h .. + 3 of each block of 32
 #pragma unroll
@@ -445,7 +475,7 @@ int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   for (int t0 = 0; t0 < n_tiles; t0 += step) {
     a.tiles = a0.tiles + 2 * t0;
     const int nt = n_tiles - t0 < step ? n_tiles - t0 : step;
-    hipLaunchKernelGGL(kern, dim3(a.n_qh / HPW, nt * a.subs), dim3(64 * NW), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(a.n_qh / HPW, nt * a.subs, a.parts), dim3(64 * NW), lds, st, a);
   }
   DX_CHECK_LAUNCH();
   return 0;
@@ -475,23 +505,44 @@ int dxm_prompt_attention_ok(int d, int dv, int n_qh, int maps, int group, int bs
   return d == 128 && dv == 128 && !out_f32 && !(fine && (terms || sigmoid));
 }
 
+// Parts that the keys of `rows` prompt rows in n_tiles tiles are cut into, `keys` of them visible to a row's workgroup at
+// most.  A workgroup alone on its CU goes from tile to tile at the pace of its loads (0.5 to 1 us for 32 keys); one that
+// shares it takes a fifth longer, of three to a CU each takes nearly twice as long.  Against that stand the join and every
+// part's sums on their way through memory.  Terms in us, fitted to one to six prompts of 16 to 1000 rows together at 16
+// and 32 heads, behind 0 to 3000 cached keys: gains above 2 all hold there.  The rule asks for 4, which is what the second
+// launch costs on the host (it counts where steps are so small that the host is behind).
+int dxm_prompt_attention_parts(int rows, int n_tiles, int keys, int n_qh, int maps, int group, int d, int dv, int bs, int same,
+                               int terms, int sigmoid, int out_f32, int fine) {
+  if (rows < 1 || n_tiles < 1 || !dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, same, terms, sigmoid, out_f32, fine)) return 1;
+  const int tall = group % 4 ? 2 : 1, blocks = std::min(n_tiles * (4 / tall), n_tiles + rows / (32 * tall));
+  const double wgs = (double)blocks * n_qh * tall / 4, floats = (double)rows * n_qh * (2 + dv);
+  const double alone = keys / 64.0 * (sigmoid ? 1.4 : dv > 128 || terms ? 2.0 : fine ? 1.2 : 1.0);
+  double best = 4.0;
+  int parts = 1;
+  for (int p = 2; p <= 8 && (p - 1) * kLeastTiles * 32 < keys; p *= 2) {
+    const double gain = alone * (1.0 - std::max(1.0, 0.6 * std::ceil(wgs * p / 256)) / p) - 6.5 - floats * p * 1.25e-6;
+    if (gain > best) best = gain, parts = p;
+  }
+  return parts;
+}
+
 int dxm_prompt_attention(void* out, const void* q, int64_t q_stride, const void* kc, const void* vc, const int64_t* pos,
                          const int* seq, const int* bt, int bt_stride, int bs, const int* tiles, int n_tiles, int n_qh,
                          int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask, int size,
                          float softcap, const float* r1, const float* r2, int wfn, const float* hbias, const void* gate,
-                         int64_t gate_stride, int keep, const float* sink, int out_f32, int fine, hipStream_t st) {
+                         int64_t gate_stride, int keep, const float* sink, int out_f32, int fine, float* ws, int parts, int rows, hipStream_t st) {
   if (n_tiles <= 0) return 0;
   const bool same = kc == vc, terms = softcap > 0.f || r1;
   if (softcap < 0.f || (r1 && !r2) || wfn < 0 || wfn > 1 || keep < 0 || (keep && mask != 1)) return 6;
   if (!dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, same, terms, wfn, out_f32, fine)) return 2;
   if (n_qh < 1 || maps < 1 || n_qh % maps || (n_qh / maps) % group || n_qh > 65535) return 1;
-  if (mask < 0 || mask > 2 || (mask && size < 1) || !(scale > 0.f)) return 3;
-  if (!out || !seq || !tiles || Wk % 8 || Wv % 8 || q_stride % 8 || (uintptr_t)q % 16 || (uintptr_t)kc % 16 ||
+  if (mask < 0 || mask > 2 || (mask && size < 1) || !(scale > 0.f) || parts < 1 || parts > 64) return 3;
+  if (!out || (parts > 1 && (!ws || (uintptr_t)ws % 8)) || !seq || !tiles || Wk % 8 || Wv % 8 || q_stride % 8 || (uintptr_t)q % 16 || (uintptr_t)kc % 16 ||
       (uintptr_t)vc % 16 || (uintptr_t)out % 16)
     return 4;
   PromptArgs a{out, (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, pos, seq, bt, bt_stride,
                __builtin_ctz((unsigned)bs), tiles, 1, n_qh, maps, group, Wk, Wv, scale, mask, size, softcap, r1, r2, hbias,
-               (const bf16_t*)gate, gate_stride, keep, sink};
+               (const bf16_t*)gate, gate_stride, keep, sink, ws, parts, rows};
   if (same && dv == 256) return prompt_heads<256, 256, true, kPlain, false, bf16_t>(a, n_tiles, st);
   if (same) return prompt_heads<256, 192, true, kPlain, false, bf16_t>(a, n_tiles, st);
   if (dv == 256) return prompt_heads<128, 256, false, kPlain, true, float>(a, n_tiles, st);

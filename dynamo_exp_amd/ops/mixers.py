@@ -531,6 +531,8 @@ def first_visible(p: torch.Tensor, mask: str, size: int) -> torch.Tensor:
     return torch.zeros_like(p)
 
 
+# prompt rows whose keys may be cut into parts: where the rows are few and what they see is long enough
+PROMPT_PART_ROWS, PROMPT_PART_KEYS = 1024, 256
 TILE_ROWS = 128  # rows of one sequence per tile_attention workgroup
 
 
@@ -543,6 +545,16 @@ def tile_attention_ok(q: torch.Tensor, d: int, dv: int) -> bool:
     """Whether the matrix-core prefill kernel serves these rows (bf16 on the
     GPU, head widths it is instantiated for); otherwise row_attention does."""
     return q.is_cuda and q.dtype == torch.bfloat16 and bool(_m().tile_attention_ok(d, dv))
+
+
+def _prompt_parts(rows: int, n_tiles: int, keys: int, mask: str, size: int, keep: int, *form) -> int:
+    """Parts that the keys of a step's prompt rows are cut into (few rows behind a long context: their workgroups alone
+    would leave most of the chip idle); keys: the longest context at most."""
+    if mask == "window":
+        keys = min(keys, size + keep + TILE_ROWS)
+    elif mask == "chunk" and keys > size:
+        keys = keys % size if keys % size > rows else size  # (of the longest; its rows may reach back over a chunk's start)
+    return _m().prompt_attention_parts(rows, n_tiles, keys, *form)
 
 
 def attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, positions: torch.Tensor,
@@ -589,9 +601,17 @@ def attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, positions: to
     if n_tile_rows:
         if seq is None or tiles.dtype != torch.int32 or not tiles.is_contiguous():
             raise TypeError("attention: prompt-chunk rows need seq and int32 tiles")
+        pparts, pws, keys = 1, None, block_tables.shape[1] * block_size
+        if n_tile_rows <= PROMPT_PART_ROWS and keys >= PROMPT_PART_KEYS:
+            pparts = _prompt_parts(n_tile_rows, tiles.shape[0], keys, mask, size, keep_first, n_qh, maps, group, d, dv, block_size,
+                                   kc.data_ptr() == vc.data_ptr(), softcap > 0 or dist_bias is not None, WEIGHTS[weights],
+                                   out_f32, fine_weights)
+        if pparts > 1:
+            pws = torch.empty((n_tile_rows, n_qh, pparts, 2 + dv), dtype=torch.float32, device=q.device)
         _m().tile_attention(out.data_ptr(), q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(),
                             positions.data_ptr(), seq.data_ptr(), *common, tiles.data_ptr(), tiles.shape[0], *heads,
-                            _ptr(head_gate), gs, int(keep_first), _ptr(sink), int(out_f32), int(fine_weights), _stream())
+                            _ptr(head_gate), gs, int(keep_first), _ptr(sink), int(out_f32), int(fine_weights), _ptr(pws),
+                            pparts, n_tile_rows, _stream())
     n_dec = T - n_tile_rows
     if n_dec:  # decode rows: the heads of a K/V group share one wave's key tiles
         r0 = n_tile_rows

@@ -381,3 +381,46 @@ def test_scores_and_caps_at_the_ends_of_the_number_range(form, cap):
     if sig and cap == 1e38:  # (2^-24 of the cap: the score is lost in its rounding)
         want = want / 2
     assert torch.equal(got.cpu().double(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [None, 2, 3, 8])
+@pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 300, 70), ("chunk", 500, 0)])
+@pytest.mark.parametrize("form", FORMS)
+def test_prompt_rows_in_parts(monkeypatch, form, mask, size, keep, parts):
+    """Few prompt rows behind long contexts, their keys cut into parts (None: as many as the rule takes): parts without a
+    tile, rows that see nothing of a part, rows of one sequence that has a single tile."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(17)
+    scale = 0.7 * d ** -0.5
+    starts, rows, bs = [1030, 0, 491], [17, 1, 70], 64
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    gate = torch.randn(sum(rows), n_qh // maps).bfloat16() if form == "gated" else None
+    kd, vd, table, kv = pages(form, [s + r for s, r in zip(starts, rows)], bs)
+    q = torch.randn(sum(rows), n_qh * d).bfloat16()
+    want = []
+    for i, (s, r) in enumerate(zip(starts, rows)):
+        r0 = sum(rows[:i])
+        want.append(dense(q[r0:r0 + r].double().reshape(r, n_qh, d), *kv[i], torch.arange(s, s + r), scale, mask, size, keep,
+                          cap, db, sink, sig, hb))
+    want = torch.cat(want)
+    if gate is not None:
+        want = want * torch.sigmoid(gate.double()).repeat_interleave(maps, 1)[:, :, None]
+    if parts:
+        monkeypatch.setattr(mx, "_prompt_parts", lambda *a: parts)
+    else:  # the rule cuts these sizes
+        rule, seen = mx._prompt_parts, []
+        monkeypatch.setattr(mx, "_prompt_parts", lambda *a: seen.append(rule(*a)) or seen[-1])
+    pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)]).cuda()
+    seq = torch.tensor([i for i, r in enumerate(rows) for _ in range(r)], dtype=torch.int32).cuda()
+    tiles = torch.tensor([t for i in range(3) for t in mx.tile_list(sum(rows[:i]), rows[i])], dtype=torch.int32).cuda()
+    out_f32 = form.startswith("diff")
+    got = mx.attention(q.cuda(), kd, vd, pos, seq, table, bs, n_qh, maps, group, d, dv, scale, mask, size, 1, out_f32, tiles,
+                       sum(rows), softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                       weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), head_gate=cuda(gate), keep_first=keep,
+                       sink=cuda(sink), fine_weights=form == "fine").cpu().double()
+    if not parts and mask == "causal":
+        assert seen[0] > 1
+    err, top = float((got - want).abs().max()), float(want.abs().max())
+    # (as in test_prompt_rows: the parts are joined in fp32)
+    assert err < (3e-4 if out_f32 else 2.0 ** -8 * (top + (top if sig else 5.0))), err
