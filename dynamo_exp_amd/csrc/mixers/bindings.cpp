@@ -88,8 +88,8 @@ int dxm_prompt_attention_ok(int, int, int, int, int, int, int, int, int, int, in
 int dxm_prompt_attention(void*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*, int,
                          int, const int*, int, int, int, int, int, int, int, int, float, int, int, float, const float*,
                          const float*, int, const float*, const void*, int64_t, int, const float*, int, int, float*, int,
-                         int, hipStream_t);
-int dxm_prompt_attention_parts(int, int, int, int, int, int, int, int, int, int, int, int, int, int);
+                         int, int, hipStream_t);
+int dxm_prompt_attention_parts(int, int, int, int, int, int, int, int, int, int, int, int, int, int, int*);
 int dxm_stream_prefill_ok(int, int, int, int, int, int);
 int dxm_stream_prefill(void*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*, int,
                        int, const int*, int, int, int, int, int, int, int, float, int, int, int, hipStream_t);
@@ -106,8 +106,8 @@ int dxm_decode_attention_parts(int, int, int, int, int);
 int dxm_decode_attention(void*, float*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*,
                          int, int, int, int, int, int, int, int, int, int, float, int, int, float, const float*, const float*,
                          int, const float*, const void*, int64_t, int, const float*, int, int, hipStream_t);
-int dxm_merge_parts(void*, const float*, int64_t, int, int, int, const void*, int64_t, int, int, const float*, int,
-                    hipStream_t);
+int dxm_merge_parts(void*, const float*, int64_t, int, const void*, int, void*, const float*, int64_t, int, const void*, int, int,
+                    int64_t, int, int, const float*, int, hipStream_t);
 }
 
 static void check(int rc, const char* what) {
@@ -290,11 +290,19 @@ PYBIND11_MODULE(_C_mixers, m) {
     check(dxm_diff_combine(P(out), F(a), n_vec, dv, lam, post, eps, P(gate), gs, H, f32, S(st)), "diff_combine");
   });
   m.def("tile_attention_ok", &dxm_tile_attention_ok);
-  m.def("prompt_attention_parts", &dxm_prompt_attention_parts);
+  m.def("prompt_attention_parts", [](int rows, int n_tiles, int keys, int n_qh, int maps, int group, int d, int dv, int bs,
+                                     int same, int terms, int sigmoid, int out_f32, int fine) {
+    int whole;
+    const int parts = dxm_prompt_attention_parts(rows, n_tiles, keys, n_qh, maps, group, d, dv, bs, same, terms, sigmoid,
+                                                 out_f32, fine, &whole);
+    return std::make_pair(parts, whole);
+  });
   m.def("tile_attention", [](u out, u q, int64_t qs, u kc, u vc, u pos, u seq, u bt, int bts, int bs, u tiles,
                              int n_tiles, int n_qh, int maps, int group, int d, int dv, int Wk, int Wv, float scale,
                              int mask, int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs,
-                             int keep, u sink, int out_f32, int fine, u ws, int parts, int rows, u st) {
+                             int keep, u sink, int out_f32, int fine, u ws, int parts, int rows, int whole,
+                             int join, u st) {
+    // returns whether the rows' sums lie in ws and are still to be joined
     // pages of whole tiles and heads of 128 columns (or one shared row of 256); a tile's bytes are counted in 31 bits
     if (qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && Wk <= 1 << 23 && Wv <= 1 << 23 && (q | kc | vc | out) % 16 == 0 &&
         dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, kc == vc, cap > 0.f || r1, wfn, out_f32, fine)) {
@@ -302,12 +310,13 @@ PYBIND11_MODULE(_C_mixers, m) {
                                  reinterpret_cast<const int*>(seq), reinterpret_cast<const int*>(bt), bts, bs,
                                  reinterpret_cast<const int*>(tiles), n_tiles, n_qh, maps, group, d, dv, Wk, Wv, scale,
                                  mask, size, cap, F(r1), F(r2), wfn, F(hbias), P(gate), gs, keep, F(sink), out_f32, fine,
-                                 F(ws), parts, rows, S(st)),
+                                 F(ws), parts, rows, whole, S(st)),
             "prompt_attention");
-      if (parts > 1)
-        check(dxm_merge_parts(P(out), F(ws), (int64_t)rows * n_qh, parts, dv, wfn, P(gate), gs, n_qh, maps, F(sink), out_f32,
-                              S(st)),
+      if (parts > 1 && join)
+        check(dxm_merge_parts(P(out), F(ws), (int64_t)rows * n_qh, parts, P(gate), whole > 0, nullptr, nullptr, 0, 0, nullptr, dv,
+                              wfn, gs, n_qh, maps, F(sink), out_f32, S(st)),
               "merge_parts");
+      return parts > 1 && !join;
     }
     // plain heads over pages of whole tiles take the streaming kernel
     else if (cap == 0.f && !r1 && !wfn && !hbias && !gate && !keep && !sink && !out_f32 && qs % 8 == 0 &&
@@ -330,11 +339,20 @@ PYBIND11_MODULE(_C_mixers, m) {
                              reinterpret_cast<const int*>(tiles), n_tiles, n_qh, maps, group, d, dv, Wk, Wv, scale,
                              mask, size, cap, F(r1), F(r2), wfn, F(hbias), P(gate), gs, keep, F(sink), out_f32, fine, S(st)),
           "tile_attention");
+    return false;
   });
   m.def("group_decode", [](u out, u ws, u q, int64_t qs, u kc, u vc, u pos, u seq, u bt, int bts, int bs, int rows,
                            int n_qh, int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask,
                            int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs, int keep, u sink,
-                           int parts, int out_f32, u st) {
+                           int parts, int out_f32, u pre_out, u pre_ws, int pre_rows, int pre_parts, u pre_gate,
+                           int pre_whole, u st) {
+    // (pre: prompt rows in parts that are to be joined in the same launch)
+    auto join = [&](int parts) {
+      if (parts == 1 && !pre_rows) return;
+      check(dxm_merge_parts(P(pre_out), F(pre_ws), (int64_t)pre_rows * n_qh, pre_parts, P(pre_gate), pre_whole > 0, P(out), F(ws),
+                            parts == 1 ? 0 : (int64_t)rows * n_qh, parts, P(gate), dv, wfn, gs, n_qh, maps, F(sink), out_f32, S(st)),
+            "merge_parts");
+    };
     // pages of whole tiles and heads of 128 columns (or one shared row of 256)
     if (scale > 0.f && qs % 8 == 0 && Wk % 8 == 0 && Wv % 8 == 0 && Wk <= 1 << 23 && Wv <= 1 << 23 &&
         (q | kc | vc | out) % 16 == 0 &&
@@ -345,7 +363,7 @@ PYBIND11_MODULE(_C_mixers, m) {
                                  maps, group, d, dv, Wk, Wv, scale, mask, size, cap, F(r1), F(r2), wfn, F(hbias), P(gate), gs,
                                  keep, F(sink), parts, out_f32, S(st)),
             "decode_attention");
-      if (parts == 1) return;
+      return join(parts);
     }
     // plain heads over pages of whole tiles take the streaming kernel (same workspace)
     else if (cap == 0.f && !r1 && !wfn && !hbias && !keep && qs % 8 == 0 && (q | kc | vc) % 16 == 0 &&
@@ -366,8 +384,9 @@ PYBIND11_MODULE(_C_mixers, m) {
                            maps, group, d, dv, Wk, Wv, scale, mask, size, cap, F(r1), F(r2), wfn, F(hbias), keep,
                            parts, S(st)),
           "group_decode");
-    check(dxm_merge_parts(P(out), F(ws), (int64_t)rows * n_qh, parts, dv, wfn, P(gate), gs, n_qh, maps, F(sink),
-                          out_f32, S(st)),
+    // (these leave their sums in the workspace whatever the number of parts)
+    check(dxm_merge_parts(P(pre_out), F(pre_ws), (int64_t)pre_rows * n_qh, pre_parts, P(pre_gate), pre_whole > 0, P(out), F(ws),
+                          (int64_t)rows * n_qh, parts, P(gate), dv, wfn, gs, n_qh, maps, F(sink), out_f32, S(st)),
           "merge_parts");
   });
   m.def("row_attention", [](u out, u ws, u q, int64_t qs, u kc, u vc, u pos, u seq, u bt, int bts, int bs, int rows,

@@ -73,7 +73,7 @@ struct PromptArgs {
   int keep;           // window mask: the first `keep` keys stay visible
   const float* sink;  // [n_qh], softmax only
   float* ws;          // parts > 1: [rows, n_qh, parts, 2 + DV]
-  int parts, rows;
+  int parts, rows, whole;  // up to `whole` keys are not cut
 };
 
 constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
@@ -107,7 +107,9 @@ __device__ __forceinline__ float swap_sum(float x) {
 
 // D: key columns, DV: value columns, SAME: the value is the first DV columns of the key's row
 // HPW: heads per workgroup, NW: waves, SUBS: blocks of 32 keys per tile
-template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS>
+// PARTS: the keys of a workgroup that sees enough of them go out in parts (an instance of its own: the others' loop is 2 %
+// slower with what is kept for it)
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS, bool PARTS>
 __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) prompt_attention_kernel(PromptArgs a) {
   constexpr int RT = NW / HPW, ROWS = 32 * RT, KT = 32 * SUBS, SH = SUBS == 2 ? 6 : 5;
   constexpr int KS = D / 16, NC = DV / 32, KB = 2 * D, VB = SAME ? KB : 2 * DV;  // row bytes of the images
@@ -135,16 +137,18 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   const int first = first_key(p0, a.mask, a.size) >> SH, last = hi >> SH;
   const int kept = a.mask == 1 ? min((a.keep + KT - 1) >> SH, first) : 0;  // tiles of kept keys in front of the window's
   // tiles in order: the kept ones, then the window's; of them this part's
-  const int total = kept + last - first + 1, part = blockIdx.z;
-  const int per_part = max((total + a.parts - 1) / a.parts, kLeastTiles), i0 = part * per_part, i1 = min(i0 + per_part, total);
+  const int total = kept + last - first + 1, part = PARTS ? blockIdx.z : 0;
+  const bool cut = PARTS && total * KT > a.whole;
+  const int per_part = cut ? max((total + a.parts - 1) / a.parts, kLeastTiles) : total;
+  const int i0 = part * per_part, i1 = min(i0 + per_part, total);
   // rows beyond n repeat the last one and are not stored
   const int myrow = min(rw + r, n - 1), my = p0 + myrow, mylo = first_key(my, a.mask, a.size);
   const int wlo = p0 + min(rw, n - 1), whi = p0 + min(rw + 31, n - 1);  // the wave's first and last position
   const int wfirst = first_key(wlo, a.mask, a.size), wlast = first_key(whi, a.mask, a.size);
   const int keep = a.mask == 1 ? a.keep : 0;
-  float* const ws = a.ws + (((int64_t)(row0 + myrow) * a.n_qh + qh) * a.parts + part) * (2 + DV);
-  if (i0 >= i1) {  // (never the first part) no tile: sum 0
-    if (rw + r < n && row0 + myrow < a.rows && h == 0) *reinterpret_cast<float2*>(ws) = float2{MODE == kSigmoid ? 0.f : -INFINITY, 0.f};
+  float* const ws = PARTS ? a.ws + (((int64_t)(row0 + myrow) * a.n_qh + qh) * a.parts + part) * (2 + DV) : nullptr;
+  if (PARTS && i0 >= i1) {  // (never the first part) no tile: sum 0
+    if (cut && rw + r < n && row0 + myrow < a.rows && h == 0) *reinterpret_cast<float2*>(ws) = float2{MODE == kSigmoid ? 0.f : -INFINITY, 0.f};
     return;
   }
   bf16x8_t qf[QR];
@@ -412,8 +416,10 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   }
 
   const bool ok = rw + r < n;
-  if (a.parts > 1) {  // sums as they are: gate, sink and denominator come with the join
-    if (!ok || row0 + myrow >= a.rows) return;
+  const bool kept_row = PARTS && ok && row0 + myrow < a.rows;
+  if (PARTS && !cut && kept_row && h == 0) *reinterpret_cast<float2*>(ws) = float2{0.f, -1.f};  // the join's sign to leave the row
+  if (cut) {  // sums as they are: gate, sink and denominator come with the join
+    if (!kept_row) return;
     const float l = MODE == kSigmoid ? 1.f : swap_sum(l_i);
     if (h == 0) *reinterpret_cast<float2*>(ws) = float2{MODE == kSigmoid ? 0.f : m_i * kLn2, l};
 #pragma unroll
@@ -458,14 +464,14 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   }
 }
 
-template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS>
-int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS, bool PARTS>
+int launch_prompt_as(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   PromptArgs a = a0;
   a.subs = 128 / (32 * (NW / HPW));
   constexpr int tiles = 2 * 32 * SUBS * 2 * (D + (SAME ? 0 : DV)) + (SAME && DV == 256 ? NW * (D / 16 - 8) * 1024 : 0);
   constexpr int most = tiles + (MODE == kTable ? HPW * (kTableKeys + 2 * kTablePad) * 4 : 0);
   const int lds = tiles + (MODE == kTable ? HPW * (a.size + 2 * kTablePad) * 4 : 0);
-  auto kern = prompt_attention_kernel<D, DV, SAME, MODE, FINE, OutT, HPW, NW, SUBS>;
+  auto kern = prompt_attention_kernel<D, DV, SAME, MODE, FINE, OutT, HPW, NW, SUBS, PARTS>;
   static bool raised = false;  // once per instance
   if (most > 48 * 1024 && !raised) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, most) != hipSuccess) return 7;
@@ -479,6 +485,12 @@ int launch_prompt(const PromptArgs& a0, int n_tiles, hipStream_t st) {
   }
   DX_CHECK_LAUNCH();
   return 0;
+}
+
+template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT, int HPW, int NW, int SUBS>
+int launch_prompt(const PromptArgs& a, int n_tiles, hipStream_t st) {
+  return a.parts > 1 ? launch_prompt_as<D, DV, SAME, MODE, FINE, OutT, HPW, NW, SUBS, true>(a, n_tiles, st)
+                     : launch_prompt_as<D, DV, SAME, MODE, FINE, OutT, HPW, NW, SUBS, false>(a, n_tiles, st);
 }
 
 // (tiles of 32 / 64 keys, us, launches back to back: cap + penalty 157 / 153, sigmoid 91 / 99, shared row 256 / 256
@@ -506,31 +518,41 @@ int dxm_prompt_attention_ok(int d, int dv, int n_qh, int maps, int group, int bs
 }
 
 // Parts that the keys of `rows` prompt rows in n_tiles tiles are cut into, `keys` of them visible to a row's workgroup at
-// most.  A workgroup alone on its CU goes from tile to tile at the pace of its loads (0.5 to 1 us for 32 keys); one that
-// shares it takes a fifth longer, of three to a CU each takes nearly twice as long.  Against that stand the join and every
-// part's sums on their way through memory.  Terms in us, fitted to one to six prompts of 16 to 1000 rows together at 16
-// and 32 heads, behind 0 to 3000 cached keys: gains above 2 all hold there.  The rule asks for 4, which is what the second
-// launch costs on the host (it counts where steps are so small that the host is behind).
-int dxm_prompt_attention_parts(int rows, int n_tiles, int keys, int n_qh, int maps, int group, int d, int dv, int bs, int same,
-                               int terms, int sigmoid, int out_f32, int fine) {
-  if (rows < 1 || n_tiles < 1 || !dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, same, terms, sigmoid, out_f32, fine)) return 1;
+// most; *whole: a workgroup that sees no more keys than that takes them in one.  (The host knows a bound only, beside decode
+// rows of long contexts a high one.  Prompts of 60 to 300 rows with nothing cached beside 8 to 30 decode rows to 5000: 1 us
+// of 29 to 69 for the join that finds them done.)
+// A workgroup alone on its CU goes from tile to tile at the pace of its loads (0.5 to 1 us for 32 keys); one that shares it
+// takes a fifth longer, of three to a CU each takes nearly twice as long.  Against that stand the join and every part's sums
+// on their way through memory.  Terms in us, fitted to one to six prompts of 16 to 1000 rows together at 16 and 32 heads,
+// behind 0 to 3000 cached keys: gains above 2 all hold there.  The rule asks for 4, which is what the second launch costs on
+// the host (it counts where steps are so small that the host is behind).
+static int prompt_parts(int rows, int n_tiles, int keys, int n_qh, int group, int dv, bool terms, bool sigmoid, bool fine, int* whole) {
   const int tall = group % 4 ? 2 : 1, blocks = std::min(n_tiles * (4 / tall), n_tiles + rows / (32 * tall));
   const double wgs = (double)blocks * n_qh * tall / 4, floats = (double)rows * n_qh * (2 + dv);
-  const double alone = keys / 64.0 * (sigmoid ? 1.4 : dv > 128 || terms ? 2.0 : fine ? 1.2 : 1.0);
+  const double key = (sigmoid ? 1.4 : dv > 128 || terms ? 2.0 : fine ? 1.2 : 1.0) / 64;  // of a workgroup alone
   double best = 4.0;
   int parts = 1;
+  *whole = 0;
   for (int p = 2; p <= 8 && (p - 1) * kLeastTiles * 32 < keys; p *= 2) {
-    const double gain = alone * (1.0 - std::max(1.0, 0.6 * std::ceil(wgs * p / 256)) / p) - 6.5 - floats * p * 1.25e-6;
-    if (gain > best) best = gain, parts = p;
+    const double saved = key * (1.0 - std::max(1.0, 0.6 * std::ceil(wgs * p / 256)) / p), cost = 6.5 + floats * p * 1.25e-6;
+    if (saved * keys - cost > best) best = saved * keys - cost, parts = p, *whole = (int)(cost / saved);
   }
   return parts;
+}
+
+int dxm_prompt_attention_parts(int rows, int n_tiles, int keys, int n_qh, int maps, int group, int d, int dv, int bs, int same,
+                               int terms, int sigmoid, int out_f32, int fine, int* whole) {
+  *whole = 0;
+  if (rows < 1 || n_tiles < 1 || !dxm_prompt_attention_ok(d, dv, n_qh, maps, group, bs, same, terms, sigmoid, out_f32, fine)) return 1;
+  return prompt_parts(rows, n_tiles, keys, n_qh, group, dv, terms, sigmoid, fine, whole);
 }
 
 int dxm_prompt_attention(void* out, const void* q, int64_t q_stride, const void* kc, const void* vc, const int64_t* pos,
                          const int* seq, const int* bt, int bt_stride, int bs, const int* tiles, int n_tiles, int n_qh,
                          int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask, int size,
                          float softcap, const float* r1, const float* r2, int wfn, const float* hbias, const void* gate,
-                         int64_t gate_stride, int keep, const float* sink, int out_f32, int fine, float* ws, int parts, int rows, hipStream_t st) {
+                         int64_t gate_stride, int keep, const float* sink, int out_f32, int fine, float* ws, int parts,
+                         int rows, int whole, hipStream_t st) {
   if (n_tiles <= 0) return 0;
   const bool same = kc == vc, terms = softcap > 0.f || r1;
   if (softcap < 0.f || (r1 && !r2) || wfn < 0 || wfn > 1 || keep < 0 || (keep && mask != 1)) return 6;
@@ -542,7 +564,7 @@ int dxm_prompt_attention(void* out, const void* q, int64_t q_stride, const void*
     return 4;
   PromptArgs a{out, (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, pos, seq, bt, bt_stride,
                __builtin_ctz((unsigned)bs), tiles, 1, n_qh, maps, group, Wk, Wv, scale, mask, size, softcap, r1, r2, hbias,
-               (const bf16_t*)gate, gate_stride, keep, sink, ws, parts, rows};
+               (const bf16_t*)gate, gate_stride, keep, sink, ws, parts, rows, whole};
   if (same && dv == 256) return prompt_heads<256, 256, true, kPlain, false, bf16_t>(a, n_tiles, st);
   if (same) return prompt_heads<256, 192, true, kPlain, false, bf16_t>(a, n_tiles, st);
   if (dv == 256) return prompt_heads<128, 256, false, kPlain, true, float>(a, n_tiles, st);

@@ -30,6 +30,8 @@
 // (lane + 64 c) for the weighted sum, the weights broadcast by readlane.
 // `parts` > 1 splits a row's keys over blockIdx.z (long decode contexts); the
 // partial (max, sum, acc) go to a workspace and merge_parts_kernel joins them.
+#include <type_traits>
+
 #include "../kernels/common.h"
 
 namespace {
@@ -186,7 +188,19 @@ __global__ void __launch_bounds__(64) row_attention_kernel(RowAttnArgs a) {
   }
 }
 
-// joins the per-part (max, sum, acc) of one (row, head): a wave each, four to a workgroup
+// What is to be joined: n_vec vectors in `parts` parts each, the first of them row 0 of out and gate.  `some`: a vector with
+// a negative first sum is not in parts, its result is there.
+template <typename OutT, typename GT> struct PartSums {
+  OutT* out;
+  const float* ws;
+  int64_t n_vec;
+  int parts;
+  const GT* gate;
+  int some;
+};
+
+// joins the per-part (max, sum, acc) of one (row, head): a wave each, four to a workgroup; the first blocks_a workgroups those of
+// `a`, the others those of b (prompt rows and decode rows of a step, a launch of 3 us fewer)
 // (`plain`: sigmoid weights, every part with a key carries max 0 and sum 1 and the join is the plain sum); gate:
 // logits [rows, gs] per head, the result is multiplied by their sigmoid; sink: [n_qh], exp(sink) joins the softmax
 // denominator once.
@@ -194,15 +208,19 @@ __global__ void __launch_bounds__(64) row_attention_kernel(RowAttnArgs a) {
 // time, the first eight before it is known which parts count.  33 x 32 vectors of 192 columns: part after part, three
 // times over, 23 us for 16 parts; for 7 parts 7.4 with the columns behind the factors, now 4.8.
 template <typename OutT, typename GT>
-__global__ void __launch_bounds__(256) merge_parts_kernel(OutT* __restrict__ out, const float* __restrict__ ws,
-                                                          int64_t n_vec, int parts, int dv, int plain,
-                                                          const GT* __restrict__ gate, int64_t gs, int n_qh, int maps,
+__global__ void __launch_bounds__(256) merge_parts_kernel(PartSums<OutT, GT> a, PartSums<OutT, GT> b, unsigned blocks_a, int dv,
+                                                          int plain, int64_t gs, int n_qh, int maps,
                                                           const float* __restrict__ sink) {
-  const int lane = threadIdx.x & 63;
-  const int64_t v = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (v >= n_vec) return;
+  const bool second = blockIdx.x >= blocks_a;
+  OutT* __restrict__ out = second ? b.out : a.out;
+  const float* __restrict__ ws = second ? b.ws : a.ws;
+  const GT* __restrict__ gate = second ? b.gate : a.gate;
+  const int parts = second ? b.parts : a.parts, lane = threadIdx.x & 63;
+  const int64_t v = (int64_t)(blockIdx.x - (second ? blocks_a : 0)) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (v >= (second ? b.n_vec : a.n_vec)) return;
   const int step = 2 + dv;
   const float* w = ws + v * parts * (int64_t)step;
+  if ((second ? b.some : a.some) && w[1] < 0.f) return;
   // columns 2 lane, 2 lane + 1 and those 128 further of eight parts: asked for before it is known which parts count
   const bool pairs = dv % 2 == 0 && dv <= 256 && (uintptr_t)ws % 8 == 0;
   const int e0 = 2 * lane < dv ? 2 * lane : 0, e1 = 2 * lane + 128 < dv ? 2 * lane + 128 : 0;
@@ -277,6 +295,13 @@ __global__ void __launch_bounds__(256) merge_parts_kernel(OutT* __restrict__ out
   }
 }
 
+template <typename OutT, typename GT>
+void launch_merge(const PartSums<OutT, GT>& a, const PartSums<OutT, GT>& b, int dv, int plain, int64_t gs, int n_qh, int maps,
+                  const float* sink, hipStream_t st) {
+  const unsigned ba = (unsigned)((a.n_vec + 3) / 4), bb = (unsigned)((b.n_vec + 3) / 4);
+  hipLaunchKernelGGL((merge_parts_kernel<OutT, GT>), dim3(ba + bb), dim3(256), 0, st, a, b, ba, dv, plain, gs, n_qh, maps, sink);
+}
+
 template <typename T, typename OutT>
 int launch_rows(const RowAttnArgs& a, int rows, hipStream_t st) {
   const int nv = (a.dv + 63) / 64;
@@ -298,8 +323,8 @@ int launch_rows(const RowAttnArgs& a, int rows, hipStream_t st) {
     else if (nv <= 8) hipLaunchKernelGGL((row_attention_kernel<T, OutT, 8>), grid, dim3(64), lds, st, b);
     else hipLaunchKernelGGL((row_attention_kernel<T, OutT, 16>), grid, dim3(64), lds, st, b);
     if (a.parts > 1)
-      hipLaunchKernelGGL((merge_parts_kernel<OutT, T>), dim3(((unsigned)nr * a.n_qh + 3) / 4), dim3(256), 0, st,
-                         (OutT*)b.out, b.ws, (int64_t)nr * a.n_qh, a.parts, a.dv, a.wfn, (const T*)b.gate, a.gate_stride, a.n_qh, a.maps, a.sink);
+      launch_merge(PartSums<OutT, T>{(OutT*)b.out, b.ws, (int64_t)nr * a.n_qh, a.parts, (const T*)b.gate, 0}, PartSums<OutT, T>{},
+                   a.dv, a.wfn, a.gate_stride, a.n_qh, a.maps, a.sink, st);
   }
   DX_CHECK_LAUNCH();
   return 0;
@@ -327,18 +352,22 @@ extern "C" int dxm_row_attention(void* out, float* ws, const void* q, int64_t q_
 }
 
 // out [n_vec, dv] (bf16 or fp32) from per-part partials ws [n_vec, parts, 2 + dv]; n_vec = rows * n_qh;
-// plain: the parts hold sigmoid-weighted sums (max 0, sum 1 each); gate: bf16 logits [rows, gate_stride]
-extern "C" int dxm_merge_parts(void* out, const float* ws, int64_t n_vec, int parts, int dv, int plain,
-                               const void* gate, int64_t gate_stride, int n_qh, int maps, const float* sink,
-                               int out_f32, hipStream_t st) {
-  if (n_vec <= 0) return 0;
-  if (parts < 1 || dv < 1 || n_vec > 0x7fffffff || n_qh < 1 || maps < 1) return 1;
-  if (out_f32)
-    hipLaunchKernelGGL((merge_parts_kernel<float, bf16_t>), dim3((unsigned)((n_vec + 3) / 4)), dim3(256), 0, st,
-                       (float*)out, ws, n_vec, parts, dv, plain, (const bf16_t*)gate, gate_stride, n_qh, maps, sink);
-  else
-    hipLaunchKernelGGL((merge_parts_kernel<bf16_t, bf16_t>), dim3((unsigned)((n_vec + 3) / 4)), dim3(256), 0, st,
-                       (bf16_t*)out, ws, n_vec, parts, dv, plain, (const bf16_t*)gate, gate_stride, n_qh, maps, sink);
+// plain: the parts hold sigmoid-weighted sums (max 0, sum 1 each); gate: bf16 logits [rows, gate_stride].  The first set may
+// hold vectors that are not in parts (`some`, see PartSums); either set may be empty.
+extern "C" int dxm_merge_parts(void* out_a, const float* ws_a, int64_t n_a, int parts_a, const void* gate_a, int some, void* out_b,
+                               const float* ws_b, int64_t n_b, int parts_b, const void* gate_b, int dv, int plain,
+                               int64_t gate_stride, int n_qh, int maps, const float* sink, int out_f32, hipStream_t st) {
+  n_a = n_a > 0 ? n_a : 0, n_b = n_b > 0 ? n_b : 0;
+  if (n_a + n_b == 0) return 0;
+  if ((n_a && parts_a < 1) || (n_b && parts_b < 1) || dv < 1 || n_a + n_b > 0x7fffffff - 8 || n_qh < 1 || maps < 1) return 1;
+  auto both = [&](auto* as) {
+    typedef std::remove_pointer_t<decltype(as)> OutT;
+    launch_merge(PartSums<OutT, bf16_t>{(OutT*)out_a, ws_a, n_a, parts_a, (const bf16_t*)gate_a, some},
+                 PartSums<OutT, bf16_t>{(OutT*)out_b, ws_b, n_b, parts_b, (const bf16_t*)gate_b, 0}, dv, plain, gate_stride, n_qh,
+                 maps, sink, st);
+  };
+  if (out_f32) both((float*)nullptr);
+  else both((bf16_t*)nullptr);
   DX_CHECK_LAUNCH();
   return 0;
 }

@@ -547,9 +547,9 @@ def tile_attention_ok(q: torch.Tensor, d: int, dv: int) -> bool:
     return q.is_cuda and q.dtype == torch.bfloat16 and bool(_m().tile_attention_ok(d, dv))
 
 
-def _prompt_parts(rows: int, n_tiles: int, keys: int, mask: str, size: int, keep: int, *form) -> int:
+def _prompt_parts(rows: int, n_tiles: int, keys: int, mask: str, size: int, keep: int, *form) -> tuple[int, int]:
     """Parts that the keys of a step's prompt rows are cut into (few rows behind a long context: their workgroups alone
-    would leave most of the chip idle); keys: the longest context at most."""
+    would leave most of the chip idle), and up to how many keys they are not; keys: the longest context at most."""
     if mask == "window":
         keys = min(keys, size + keep + TILE_ROWS)
     elif mask == "chunk" and keys > size:
@@ -598,28 +598,30 @@ def attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, positions: to
              float(softcap), _ptr(dist_bias[0]) if dist_bias else 0, _ptr(dist_bias[1]) if dist_bias else 0,
              WEIGHTS[weights], _ptr(head_bias))
     gs = head_gate.stride(0) if head_gate is not None else 0
+    n_dec = T - n_tile_rows
+    pre = (0, 0, 0, 1, 0, 0)  # prompt rows in parts, joined in one launch with the decode rows
     if n_tile_rows:
         if seq is None or tiles.dtype != torch.int32 or not tiles.is_contiguous():
             raise TypeError("attention: prompt-chunk rows need seq and int32 tiles")
-        pparts, pws, keys = 1, None, block_tables.shape[1] * block_size
+        pparts, whole, pws, keys = 1, 0, None, block_tables.shape[1] * block_size
         if n_tile_rows <= PROMPT_PART_ROWS and keys >= PROMPT_PART_KEYS:
-            pparts = _prompt_parts(n_tile_rows, tiles.shape[0], keys, mask, size, keep_first, n_qh, maps, group, d, dv, block_size,
-                                   kc.data_ptr() == vc.data_ptr(), softcap > 0 or dist_bias is not None, WEIGHTS[weights],
-                                   out_f32, fine_weights)
+            pparts, whole = _prompt_parts(n_tile_rows, tiles.shape[0], keys, mask, size, keep_first, n_qh, maps, group, d, dv,
+                                          block_size, kc.data_ptr() == vc.data_ptr(), softcap > 0 or dist_bias is not None,
+                                          WEIGHTS[weights], out_f32, fine_weights)
         if pparts > 1:
             pws = torch.empty((n_tile_rows, n_qh, pparts, 2 + dv), dtype=torch.float32, device=q.device)
-        _m().tile_attention(out.data_ptr(), q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(),
-                            positions.data_ptr(), seq.data_ptr(), *common, tiles.data_ptr(), tiles.shape[0], *heads,
-                            _ptr(head_gate), gs, int(keep_first), _ptr(sink), int(out_f32), int(fine_weights), _ptr(pws),
-                            pparts, n_tile_rows, _stream())
-    n_dec = T - n_tile_rows
+        if _m().tile_attention(out.data_ptr(), q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(),
+                               positions.data_ptr(), seq.data_ptr(), *common, tiles.data_ptr(), tiles.shape[0], *heads,
+                               _ptr(head_gate), gs, int(keep_first), _ptr(sink), int(out_f32), int(fine_weights), _ptr(pws),
+                               pparts, n_tile_rows, whole, int(not n_dec), _stream()):
+            pre = (out.data_ptr(), pws.data_ptr(), n_tile_rows, pparts, _ptr(head_gate), whole)
     if n_dec:  # decode rows: the heads of a K/V group share one wave's key tiles
         r0 = n_tile_rows
         ws = torch.empty((n_dec, n_qh, parts, 2 + dv), dtype=torch.float32, device=q.device)
         _m().group_decode(out[r0:].data_ptr(), ws.data_ptr(), q[r0:].data_ptr(), q.stride(0), kc.data_ptr(),
                           vc.data_ptr(), positions[r0:].data_ptr(), _ptr(seq[r0:] if seq is not None else None),
                           *common, n_dec, *heads, _ptr(head_gate[r0:]) if head_gate is not None else 0, gs,
-                          int(keep_first), _ptr(sink), parts, int(out_f32), _stream())
+                          int(keep_first), _ptr(sink), parts, int(out_f32), *pre, _stream())
     return out
 
 

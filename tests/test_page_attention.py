@@ -384,12 +384,12 @@ def test_scores_and_caps_at_the_ends_of_the_number_range(form, cap):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("parts", [None, 2, 3, 8])
+@pytest.mark.parametrize("parts", [None, (2, 0), (3, 0), (8, 0), (4, 200)])
 @pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 300, 70), ("chunk", 500, 0)])
 @pytest.mark.parametrize("form", FORMS)
 def test_prompt_rows_in_parts(monkeypatch, form, mask, size, keep, parts):
     """Few prompt rows behind long contexts, their keys cut into parts (None: as many as the rule takes): parts without a
-    tile, rows that see nothing of a part, rows of one sequence that has a single tile."""
+    tile, rows that see nothing of a part, rows of one sequence that has a single tile, workgroups that stay whole."""
     n_qh, maps, group, d, dv = FORMS[form]
     torch.manual_seed(17)
     scale = 0.7 * d ** -0.5
@@ -420,7 +420,48 @@ def test_prompt_rows_in_parts(monkeypatch, form, mask, size, keep, parts):
                        weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), head_gate=cuda(gate), keep_first=keep,
                        sink=cuda(sink), fine_weights=form == "fine").cpu().double()
     if not parts and mask == "causal":
-        assert seen[0] > 1
+        assert seen[0][0] > 1
     err, top = float((got - want).abs().max()), float(want.abs().max())
     # (as in test_prompt_rows: the parts are joined in fp32)
+    assert err < (3e-4 if out_f32 else 2.0 ** -8 * (top + (top if sig else 5.0))), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("parts", [1, 5])
+@pytest.mark.parametrize("pre", [(4, 0), (3, 200), (8, 10000)])
+@pytest.mark.parametrize("form", ["plain", "gated", "sigmoid", "both", "plain pair", "diff", "shared", "fine"])
+def test_prompt_rows_in_parts_beside_decode_rows(monkeypatch, form, pre, parts, shift):
+    """One join for a step's prompt rows and its decode rows (in one part: for the prompt rows alone); prompt rows that are cut,
+    that are not, and both; a gate whose rows go on into the decode rows; queries (`shift`) whose address the kernels for whole
+    tiles do not take, so that nothing is in parts."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(19)
+    scale, bs = 0.7 * d ** -0.5, 64
+    lengths, rows = [700, 40, 1300, 5, 650], [20, 40, 1, 1, 1]
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    T, Tp = sum(rows), 60
+    gate = torch.randn(T, n_qh // maps).bfloat16() if form == "gated" else None
+    kd, vd, table, kv = pages(form, lengths, bs)
+    q = torch.randn(T, n_qh * d).bfloat16()
+    want, pos = [], []
+    for i, (n, r) in enumerate(zip(lengths, rows)):
+        r0, p = sum(rows[:i]), torch.arange(n - r, n)
+        pos.append(p)
+        want.append(dense(q[r0:r0 + r].double().reshape(r, n_qh, d), *kv[i], p, scale, "causal", 0, 0, cap, db, sink, sig, hb))
+    want = torch.cat(want)
+    if gate is not None:
+        want = want * torch.sigmoid(gate.double()).repeat_interleave(maps, 1)[:, :, None]
+    monkeypatch.setattr(mx, "_prompt_parts", lambda *a: pre)
+    seq = torch.tensor([i for i, r in enumerate(rows) for _ in range(r)], dtype=torch.int32).cuda()
+    tiles = torch.tensor(mx.tile_list(0, 20) + mx.tile_list(20, 40), dtype=torch.int32).cuda()
+    out_f32 = form.startswith("diff")
+    qd = torch.empty(T * n_qh * d + 8, dtype=torch.bfloat16, device="cuda")[4 * shift:4 * shift + T * n_qh * d].view(T, -1)
+    qd.copy_(q)
+    got = mx.attention(qd, kd, vd, torch.cat(pos).cuda(), seq, table, bs, n_qh, maps, group, d, dv, scale, "causal", 0, parts,
+                       out_f32, tiles, Tp, softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                       weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), head_gate=cuda(gate), sink=cuda(sink),
+                       fine_weights=form == "fine").cpu().double()
+    err, top = float((got - want).abs().max()), float(want.abs().max())
+    # (as in test_prompt_rows)
     assert err < (3e-4 if out_f32 else 2.0 ** -8 * (top + (top if sig else 5.0))), err
