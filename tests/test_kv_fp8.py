@@ -260,3 +260,21 @@ def test_fp8_prefill_scratch_groups_match_single_pass_gpu(cuda):
     assert got == want
     ws = [v for k, v in ops._KV_SCRATCH.items()]
     assert ws and min(w[0].shape[0] for w in ws) >= 16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,BS,D", [(1, 16, 64), (3, 16, 128), (2, 64, 128), (5, 32, 72), (8, 64, 128)])
+def test_dequant_blocks_of_every_size(H, BS, D):
+    """Blocks of less than a workgroup's piece, of whole pieces and of pieces and a rest; blocks past the context stay as they
+    are.  Widening e4m3 is exact, the scale's product is rounded once."""
+    torch.manual_seed(H * BS + D)
+    ctx, blocks, scales = [2 * BS + 1, 1, BS], 9, (0.05, 0.04)
+    k, v = (torch.randn(blocks, H, BS, D).to(torch.float8_e4m3fn) for _ in range(2))
+    bt = torch.randperm(blocks)[:9].view(3, 3).to(torch.int32)
+    table = torch.tensor([[0, 1, 2], [3, 0, 0], [4, 0, 0]], dtype=torch.int32)
+    ks, vs, _ = ops.kv_dequant_scratch(k.cuda(), v.cuda(), bt.cuda(), torch.tensor(ctx, dtype=torch.int32).cuda(), scales,
+                                       (table.cuda(), 5))
+    for got, src, sc in ((ks, k, scales[0]), (vs, v, scales[1])):
+        want = torch.cat([(src[bt[i, j].long()].float() * sc).bfloat16()[None]
+                          for i, n in enumerate((3, 1, 1)) for j in range(n)])
+        assert torch.equal(got[:5].cpu(), want)
