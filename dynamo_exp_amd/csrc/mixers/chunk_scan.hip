@@ -87,18 +87,19 @@ constexpr int kInOrder = 24;
 
 struct Walk {
   int r0, n, h, hq, col0, slot;
-  bool fresh;
+  bool fresh, tokens;  // tokens: too short for a chunk, token by token
 };
 __device__ __forceinline__ bool open_walk(const ScanArgs& g, Walk& w) {
   const int z = blockIdx.z;
-  const SeqRows q = g.sorted ? by_length<false>(g.seq_rows, g.slots, gridDim.z, z, g.min_rows, kInOrder)
+  const SeqRows q = g.sorted ? by_length<false>(g.seq_rows, g.slots, gridDim.z, z, g.min_rows, kInOrder, g.all)
                              : SeqRows{g.seq_rows[z], g.seq_rows[z + 1] - g.seq_rows[z], g.slots[z], z};
   w.h = blockIdx.y;
   w.hq = w.h / g.qk_rep;
   w.col0 = blockIdx.x * kPB;
   w.r0 = q.r0;
   w.n = q.n;
-  if (w.n < g.min_rows || w.r0 < 0 || w.r0 + w.n > g.T) return false;
+  w.tokens = w.n < g.min_rows;
+  if (w.n < (g.all ? 1 : g.min_rows) || w.r0 < 0 || w.r0 + w.n > g.T) return false;
   w.slot = q.slot;
   if (w.slot < 0 || w.slot >= g.n_slots) {  // padding: zeros out, no state touched
     for (int i = threadIdx.x; i < w.n * kPB; i += blockDim.x)
@@ -151,6 +152,12 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
   __shared__ __attribute__((aligned(16))) bf16_t ks[sizeof(bufs[0].q) / sizeof(bf16_t)];  // k [s][n]
   Walk w;
   if (!open_walk(g, w)) return;
+  if (w.tokens) {
+    typedef ScanLds<DK, MODE, kPB> Lds;
+    static_assert(sizeof(Lds) <= sizeof(bufs), "the rows of eight tokens");
+    scan_tokens<bf16_t, DK / 16, MODE, kPB, 512>(g, *reinterpret_cast<Lds*>(bufs), w.r0, w.r0 + w.n, w.h, w.hq, w.slot, w.col0);
+    return;
+  }
   const bool former = threadIdx.x >= 256;
   const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = tid & 15, g4 = (tid & 63) >> 4;
 
@@ -429,6 +436,13 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
   __shared__ __attribute__((aligned(16))) Buf bufs[2];
   Walk w;
   if (!open_walk(g, w)) return;
+  if (w.tokens) {
+    typedef ScanLds<DK, kChannel, kPB> Lds;
+    static_assert(sizeof(Lds) <= sizeof(bufs), "the rows of eight tokens");
+    scan_tokens<bf16_t, DK / 16, kChannel, kPB, kFormThreads + kProdThreads>(g, *reinterpret_cast<Lds*>(bufs), w.r0, w.r0 + w.n, w.h,
+                                                                            w.hq, w.slot, w.col0);
+    return;
+  }
   const bool former = threadIdx.x >= kProdThreads;
   const int tid = former ? threadIdx.x - kProdThreads : threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
@@ -661,17 +675,25 @@ bool chunk_scan_ok(int mode, const ScanArgs& g) {
   else if (g.dk == 64) hipLaunchKernelGGL((KERNEL(64)), grid, NT, 0, st, g);  \
   else hipLaunchKernelGGL((KERNEL(128)), grid, NT, 0, st, g);
 
-void launch_chunk_scan(int mode, const ScanArgs& g0, int n_seq, hipStream_t st) {
+bool launch_chunk_scan(int mode, const ScanArgs& g0, int n_seq, hipStream_t st) {
   ScanArgs g = g0;
   const dim3 grid(g.dv / kPB, g.H, n_seq);
   // One workgroup a CU: where sequences of 128 rows and more may be too many for one round, the longest start first (128 heads
   // of 64 columns, prompts of 667, 1334 and 2000 rows: 152 -> 125 us); elsewhere their order is only a slower load in front
   // (32 heads, the same prompts with the norm: 138 -> 140 us).  Up to kInOrder sequences long enough for a chunk.
   g.sorted = (int64_t)grid.x * grid.y * std::min(n_seq, g.T / 128) > 256;
+  // Sequences too short for a chunk go token by token in workgroups of the same launch, behind the others: most of the chip
+  // waits for the longest chain, and a launch is saved.  Whole layers, us, two launches / one: state-space duality, 600 rows beside
+  // 31 and 60 decode rows 127 / 112 and 178 / 160, 60 beside 20 67 / 66; retention, 1767 in four beside 10 58.8 / 49.1, 500 in two
+  // beside 60 79 / 64, 60 beside 100 107 / 87; gated linear attention, 2000 beside 100 209 / 159, 300 beside 30 59 / 45.  Up to what
+  // was measured.  (Heads that a step of short sequences alone would scan by the kernel for any sizes, in another order of
+  // sums, stay with it.)
+  g.all = g.dv % (4096 / g.dk) == 0 && (int64_t)grid.x * grid.y * n_seq <= 8192;
 #define FIXED_K(D) chunk_scan_kernel<D, kFixed>
 #define STEP_K(D) chunk_scan_kernel<D, kStep>
 #define CHANNEL_K(D) channel_chunk_kernel<D>
   if (mode == kFixed) { CHUNK_DK(FIXED_K, dim3(512)) }
   else if (mode == kStep) { CHUNK_DK(STEP_K, dim3(512)) }
   else { CHUNK_DK(CHANNEL_K, dim3(kFormThreads + kProdThreads)) }
+  return g.all;
 }

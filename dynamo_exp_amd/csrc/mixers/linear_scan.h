@@ -25,6 +25,7 @@ struct ScanArgs {
   int n_slots, T, H, dk, dv;
   int min_rows, max_rows;  // sequences with fewer / more rows in the step are another launch's
   int sorted;              // chunked kernels: workgroups take the sequences by length
+  int all;                 // chunked kernels: sequences of fewer rows than min_rows too, token by token
 };
 
 __device__ __forceinline__ float softplusf_(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
@@ -41,8 +42,170 @@ template <typename T> __device__ __forceinline__ float step_size(const ScanArgs&
   return softplusf_(ldf<T>((const T*)g.g, row * g.gs + h) + (g.g_bias ? g.g_bias[h] : 0.f));
 }
 
+// step size and decay of one (row, head)
+template <typename T> __device__ __forceinline__ float2 step_terms(const ScanArgs& g, int64_t row, int h) {
+  const float u = step_size<T>(g, row, h);
+  return float2{u, expf(-g.rate[h] * u)};
+}
+
+// The same for key widths dk = 16 R and 16-byte aligned operands: nothing in the token loop is
+// conditional.  Lane r of a column's group owns the four row quads 4 (r + R qd) .. + 3, qd < 4, so
+// a group's 128-bit LDS reads of a row vector are neighbouring chunks and the state is read and
+// written as 16-byte runs.  The next block's eight tokens (q, k, decay logits of the head, v of the
+// workgroup's columns) are fetched into registers as 16-byte chunks while the current block's chain runs.
+// The first block is asked for in front of the state and staged while the state is on its way (its barriers wait for LDS
+// only), and the state in front of the position that says whether it counts, so that a decode step is one latency, not three
+// (four layers of gated linear attention, 16 heads, 5 sequences 38.9 -> 37.6 us with the latter).  Bound by memory: two layers with their other launches in a graph, us:
+// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 230 (its kernel at 64: 5.2
+// TB/s of state); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 135.
+template <int DK, int MODE, int COLS> struct ScanLds {
+  __attribute__((aligned(16))) float q[kTok * DK];
+  __attribute__((aligned(16))) float k[kTok * DK];
+  __attribute__((aligned(16))) float a[MODE == kChannel ? kTok * DK : 4];
+  __attribute__((aligned(16))) float v[kTok * COLS];
+  float2 u[kTok];
+};
+
+// rows r0 .. r1 - 1 (of one sequence, whose state is in `slot`) of columns col0 .. + COLS - 1 of head h, by a workgroup of NT
+// threads, COLS R of which own columns; hq: its q / k head (a division, which the caller has done beside its loads)
+template <typename T, int R, int MODE, int COLS, int NT>
+__device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, MODE, COLS>& lds, int r0, int r1, int h, int hq, int slot,
+                                            int col0) {
+  constexpr int dk = 16 * R, cols = COLS, VEC = 16 / (int)sizeof(T);
+  constexpr int QC = dk / VEC, VC = cols / VEC;  // chunks per token row
+  constexpr int QK_CH = kTok * QC, V_CH = kTok * VC;
+  constexpr int N_ROWS = MODE == kChannel ? 3 : 2;  // row vectors of dk staged per token
+  constexpr int N_CH = N_ROWS * QK_CH + V_CH;
+  constexpr int PER = (N_CH + NT - 1) / NT;
+  float *qs_ = lds.q, *ks_ = lds.k, *as_ = lds.a, *vs_ = lds.v;
+  float2* us_ = lds.u;
+  static_assert(NT >= COLS * R, "a column's lanes");
+  const int tid = threadIdx.x, r = tid % R;
+  const bool owner = NT == COLS * R || tid < COLS * R;
+  const int cl = owner ? tid / R : 0, j = col0 + cl;
+  const int64_t ow = (int64_t)g.H * g.dv;
+  float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv + j) * dk;
+  const float fixed = MODE == kFixed ? g.decay[h] : 0.f, skip = g.skip ? g.skip[h] : 0.f;
+  const T* q = (const T*)g.q + (int64_t)hq * dk;
+  const T* k = (const T*)g.k + (int64_t)hq * dk;
+  const T* gl = (const T*)g.g + (int64_t)h * dk;
+  const T* v = (const T*)g.v + (int64_t)h * g.dv + col0;
+  raw_u32x4 pf[PER];
+  // kStep: token tid's step logit as loaded (its terms are formed in commit(): here they would wait for the load)
+  T logit{};
+  bool stepped = false;
+  const float g_bias = MODE == kStep && g.g_bias ? g.g_bias[h] : 0.f, rate = MODE == kStep ? g.rate[h] : 0.f;
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = tid + i * NT;
+      const T* src = nullptr;
+      if (c < QK_CH) {
+        const int tt = c / QC;
+        if (t0 + tt < r1) src = q + (int64_t)(t0 + tt) * g.qs + (c % QC) * VEC;
+      } else if (c < 2 * QK_CH) {
+        const int c2 = c - QK_CH, tt = c2 / QC;
+        if (t0 + tt < r1) src = k + (int64_t)(t0 + tt) * g.ks + (c2 % QC) * VEC;
+      } else if (MODE == kChannel && c < 3 * QK_CH) {
+        const int c2 = c - 2 * QK_CH, tt = c2 / QC;
+        if (t0 + tt < r1) src = gl + (int64_t)(t0 + tt) * g.gs + (c2 % QC) * VEC;
+      } else if (c < N_CH) {
+        const int c2 = c - N_ROWS * QK_CH, tt = c2 / VC;
+        if (t0 + tt < r1) src = v + (int64_t)(t0 + tt) * g.vs + (c2 % VC) * VEC;
+      }
+      pf[i] = src ? *reinterpret_cast<const raw_u32x4*>(src) : raw_u32x4{0u, 0u, 0u, 0u};
+    }
+    if constexpr (MODE == kStep) {
+      stepped = tid < kTok && t0 + tid < r1;
+      if (stepped) logit = ((const T*)g.g)[(int64_t)(t0 + tid) * g.gs + h];
+    }
+  };
+  auto commit = [&]() {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = tid + i * NT;
+      float f[VEC];
+      chunk_to_f32<T>(pf[i], f);
+      float* dst = nullptr;
+      if (c < QK_CH) {
+        dst = qs_ + c * VEC;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) f[e] *= g.q_scale;
+      } else if (c < 2 * QK_CH) {
+        dst = ks_ + (c - QK_CH) * VEC;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) f[e] *= g.k_scale;
+      } else if (MODE == kChannel && c < 3 * QK_CH) {
+        const int e0 = (c - 2 * QK_CH) * VEC, ch = h * dk + e0 % dk;
+        dst = as_ + e0;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) f[e] = channel_decay(f[e] + (g.g_bias ? g.g_bias[ch + e] : 0.f), g.inv_tau);
+      } else if (c < N_CH) {
+        dst = vs_ + (c - N_ROWS * QK_CH) * VEC;
+      }
+      if (dst) {
+#pragma unroll
+        for (int e = 0; e < VEC; e += 4) *reinterpret_cast<f32x4*>(dst + e) = f32x4{f[e], f[e + 1], f[e + 2], f[e + 3]};
+      }
+    }
+    if constexpr (MODE == kStep) {
+      if (tid < kTok) {
+        const float u = softplusf_(ldf<T>(&logit, 0) + g_bias);
+        us_[tid] = stepped ? float2{u, expf(-rate * u)} : float2{0.f, 1.f};
+      }
+    }
+  };
+  fetch(r0);  // (in front of the state, which it does not wait for)
+  // (asked for before it is known whether it counts: at position 0 the state is zero, whatever the slot held)
+  float S[16];
+#pragma unroll
+  for (int qd = 0; qd < 4; ++qd) *reinterpret_cast<f32x4*>(S + 4 * qd) = *reinterpret_cast<const f32x4*>(sp + 4 * (r + R * qd));
+  const bool fresh = g.pos[r0] == 0;
+  for (int t0 = r0; t0 < r1; t0 += kTok) {
+    const int nt = r1 - t0 < kTok ? r1 - t0 : kTok;
+    lds_barrier();  // the previous block's reads are done
+    commit();
+    lds_barrier();
+    if (fresh && t0 == r0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S[i] = 0.f;
+    }
+    if (t0 + kTok < r1) fetch(t0 + kTok);
+    for (int tt = 0; tt < nt; ++tt) {
+      const float vj = vs_[tt * cols + cl];
+      float uv = vj, dec = fixed;
+      if constexpr (MODE == kStep) {
+        const float2 u = us_[tt];
+        uv = vj * u.x;
+        dec = u.y;
+      }
+      float acc = 0.f;
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        const f32x4 kk = *reinterpret_cast<const f32x4*>(ks_ + tt * dk + 4 * (r + R * qd));
+        const f32x4 qq = *reinterpret_cast<const f32x4*>(qs_ + tt * dk + 4 * (r + R * qd));
+        f32x4 aa;
+        if constexpr (MODE == kChannel) aa = *reinterpret_cast<const f32x4*>(as_ + tt * dk + 4 * (r + R * qd));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // (written out: every instance rounds alike, whichever launch a sequence is in)
+          S[4 * qd + e] = fmaf(MODE == kChannel ? aa[e] : dec, S[4 * qd + e], kk[e] * uv);
+          acc = fmaf(qq[e], S[4 * qd + e], acc);
+        }
+      }
+      acc = group_sum<R>(acc);
+      if (r == 0 && owner) g.out[(int64_t)(t0 + tt) * ow + h * g.dv + j] = fmaf(skip, vj, acc);
+    }
+  }
+  if (!owner) return;
+#pragma unroll
+  for (int qd = 0; qd < 4; ++qd)
+    *reinterpret_cast<f32x4*>(sp + 4 * (r + R * qd)) = f32x4{S[4 * qd], S[4 * qd + 1], S[4 * qd + 2], S[4 * qd + 3]};
+}
+
 // a sequence with at least this many rows in the step goes through the chunked kernels
 constexpr int kChunkMinRows = 8;
 
 bool chunk_scan_ok(int mode, const ScanArgs& g);
-void launch_chunk_scan(int mode, const ScanArgs& g, int n_seq, hipStream_t st);
+// true: it takes the shorter sequences as well
+bool launch_chunk_scan(int mode, const ScanArgs& g, int n_seq, hipStream_t st);

@@ -20,12 +20,6 @@
 
 namespace {
 
-// step size and decay of one (row, head)
-template <typename T> __device__ __forceinline__ float2 step_terms(const ScanArgs& g, int64_t row, int h) {
-  const float u = step_size<T>(g, row, h);
-  return float2{u, expf(-g.rate[h] * u)};
-}
-
 constexpr int kMaxKey = 512;
 
 // Any sizes: rows and columns beyond dk / dv are guarded one by one.  Lane r of a column's group owns
@@ -115,154 +109,21 @@ __global__ void __launch_bounds__(256) scan_kernel(ScanArgs g) {
   }
 }
 
-// The same for key widths dk = 16 R and 16-byte aligned operands: nothing in the token loop is
-// conditional.  Lane r of a column's group owns the four row quads 4 (r + R qd) .. + 3, qd < 4, so
-// a group's 128-bit LDS reads of a row vector are neighbouring chunks and the state is read and
-// written as 16-byte runs.  The next block's eight tokens (q, k, decay logits of the head, v of the
-// workgroup's columns) are fetched into registers as 16-byte chunks while the current block's chain runs.
-// The first block is asked for in front of the state and staged while the state is on its way (its barriers wait for LDS
-// only), so that a decode step is one latency, not two.  Bound by memory: two layers with their other launches in a graph, us:
-// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 230 (its kernel at 64: 5.2
-// TB/s of state); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 135.
+// scan_tokens for every sequence of a step
 template <typename T, int R, int MODE>
 __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
-  constexpr int dk = 16 * R, cols = 256 / R, VEC = 16 / (int)sizeof(T);
-  constexpr int QC = dk / VEC, VC = cols / VEC;  // chunks per token row
-  constexpr int QK_CH = kTok * QC, V_CH = kTok * VC;
-  constexpr int N_ROWS = MODE == kChannel ? 3 : 2;  // row vectors of dk staged per token
-  constexpr int N_CH = N_ROWS * QK_CH + V_CH;
-  constexpr int PER = (N_CH + 255) / 256;
-  __shared__ __attribute__((aligned(16))) float qs_[kTok * dk];
-  __shared__ __attribute__((aligned(16))) float ks_[kTok * dk];
-  __shared__ __attribute__((aligned(16))) float as_[MODE == kChannel ? kTok * dk : 4];
-  __shared__ __attribute__((aligned(16))) float vs_[kTok * cols];
-  __shared__ float2 us_[kTok];
-  const int s = blockIdx.x, h = blockIdx.y, hq = h / g.qk_rep;
-  const int tid = threadIdx.x, cl = tid / R, r = tid % R;
-  const int col0 = blockIdx.z * cols, j = col0 + cl;
-  const int r0 = g.seq_rows ? g.seq_rows[s] : s, r1 = g.seq_rows ? g.seq_rows[s + 1] : s + 1;
-  if (r1 <= r0 || r0 < 0 || r1 > g.T || r1 - r0 > g.max_rows) return;
+  constexpr int cols = 256 / R;
+  __shared__ ScanLds<16 * R, MODE, cols> lds;
+  const int s = blockIdx.x, h = blockIdx.y, hq = h / g.qk_rep, col0 = blockIdx.z * cols;
   const int slot = g.slots[s];
-  const int64_t ow = (int64_t)g.H * g.dv;
+  const int r0 = g.seq_rows ? g.seq_rows[s] : s, r1 = g.seq_rows ? g.seq_rows[s + 1] : s + 1;
+  if ((r1 <= r0) | (r0 < 0) | (r1 > g.T) | (r1 - r0 > g.max_rows)) return;  // (bitwise: one wait for all of them)
   if (slot < 0 || slot >= g.n_slots) {  // a padding row: zeros out, no state touched
     for (int t = r0; t < r1; ++t)
-      if (r == 0) g.out[(int64_t)t * ow + h * g.dv + j] = 0.f;
+      if (threadIdx.x % R == 0) g.out[(int64_t)t * g.H * g.dv + h * g.dv + col0 + threadIdx.x / R] = 0.f;
     return;
   }
-  float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv + j) * dk;
-  const float fixed = MODE == kFixed ? g.decay[h] : 0.f, skip = g.skip ? g.skip[h] : 0.f;
-  const T* q = (const T*)g.q + (int64_t)hq * dk;
-  const T* k = (const T*)g.k + (int64_t)hq * dk;
-  const T* gl = (const T*)g.g + (int64_t)h * dk;
-  const T* v = (const T*)g.v + (int64_t)h * g.dv + col0;
-  raw_u32x4 pf[PER];
-  // kStep: token tid's step logit as loaded (its terms are formed in commit(): here they would wait for the load)
-  T logit{};
-  bool stepped = false;
-  const float g_bias = MODE == kStep && g.g_bias ? g.g_bias[h] : 0.f, rate = MODE == kStep ? g.rate[h] : 0.f;
-  auto fetch = [&](int t0) {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = tid + i * 256;
-      const T* src = nullptr;
-      if (c < QK_CH) {
-        const int tt = c / QC;
-        if (t0 + tt < r1) src = q + (int64_t)(t0 + tt) * g.qs + (c % QC) * VEC;
-      } else if (c < 2 * QK_CH) {
-        const int c2 = c - QK_CH, tt = c2 / QC;
-        if (t0 + tt < r1) src = k + (int64_t)(t0 + tt) * g.ks + (c2 % QC) * VEC;
-      } else if (MODE == kChannel && c < 3 * QK_CH) {
-        const int c2 = c - 2 * QK_CH, tt = c2 / QC;
-        if (t0 + tt < r1) src = gl + (int64_t)(t0 + tt) * g.gs + (c2 % QC) * VEC;
-      } else if (c < N_CH) {
-        const int c2 = c - N_ROWS * QK_CH, tt = c2 / VC;
-        if (t0 + tt < r1) src = v + (int64_t)(t0 + tt) * g.vs + (c2 % VC) * VEC;
-      }
-      pf[i] = src ? *reinterpret_cast<const raw_u32x4*>(src) : raw_u32x4{0u, 0u, 0u, 0u};
-    }
-    if constexpr (MODE == kStep) {
-      stepped = tid < kTok && t0 + tid < r1;
-      if (stepped) logit = ((const T*)g.g)[(int64_t)(t0 + tid) * g.gs + h];
-    }
-  };
-  auto commit = [&]() {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = tid + i * 256;
-      float f[VEC];
-      chunk_to_f32<T>(pf[i], f);
-      float* dst = nullptr;
-      if (c < QK_CH) {
-        dst = qs_ + c * VEC;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) f[e] *= g.q_scale;
-      } else if (c < 2 * QK_CH) {
-        dst = ks_ + (c - QK_CH) * VEC;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) f[e] *= g.k_scale;
-      } else if (MODE == kChannel && c < 3 * QK_CH) {
-        const int e0 = (c - 2 * QK_CH) * VEC, ch = h * dk + e0 % dk;
-        dst = as_ + e0;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) f[e] = channel_decay(f[e] + (g.g_bias ? g.g_bias[ch + e] : 0.f), g.inv_tau);
-      } else if (c < N_CH) {
-        dst = vs_ + (c - N_ROWS * QK_CH) * VEC;
-      }
-      if (dst) {
-#pragma unroll
-        for (int e = 0; e < VEC; e += 4) *reinterpret_cast<f32x4*>(dst + e) = f32x4{f[e], f[e + 1], f[e + 2], f[e + 3]};
-      }
-    }
-    if constexpr (MODE == kStep) {
-      if (tid < kTok) {
-        const float u = softplusf_(ldf<T>(&logit, 0) + g_bias);
-        us_[tid] = stepped ? float2{u, expf(-rate * u)} : float2{0.f, 1.f};
-      }
-    }
-  };
-  fetch(r0);  // (in front of the state, which it does not wait for)
-  const bool fresh = g.pos[r0] == 0;
-  float S[16];
-#pragma unroll
-  for (int qd = 0; qd < 4; ++qd) {
-    const f32x4 v4 = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + 4 * (r + R * qd));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) S[4 * qd + e] = v4[e];
-  }
-  for (int t0 = r0; t0 < r1; t0 += kTok) {
-    const int nt = r1 - t0 < kTok ? r1 - t0 : kTok;
-    lds_barrier();  // the previous block's reads are done
-    commit();
-    lds_barrier();
-    if (t0 + kTok < r1) fetch(t0 + kTok);
-    for (int tt = 0; tt < nt; ++tt) {
-      const float vj = vs_[tt * cols + cl];
-      float uv = vj, dec = fixed;
-      if constexpr (MODE == kStep) {
-        const float2 u = us_[tt];
-        uv = vj * u.x;
-        dec = u.y;
-      }
-      float acc = 0.f;
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const f32x4 kk = *reinterpret_cast<const f32x4*>(ks_ + tt * dk + 4 * (r + R * qd));
-        const f32x4 qq = *reinterpret_cast<const f32x4*>(qs_ + tt * dk + 4 * (r + R * qd));
-        f32x4 aa;
-        if constexpr (MODE == kChannel) aa = *reinterpret_cast<const f32x4*>(as_ + tt * dk + 4 * (r + R * qd));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          S[4 * qd + e] = (MODE == kChannel ? aa[e] : dec) * S[4 * qd + e] + kk[e] * uv;
-          acc += qq[e] * S[4 * qd + e];
-        }
-      }
-      acc = group_sum<R>(acc);
-      if (r == 0) g.out[(int64_t)(t0 + tt) * ow + h * g.dv + j] = acc + skip * vj;
-    }
-  }
-#pragma unroll
-  for (int qd = 0; qd < 4; ++qd)
-    *reinterpret_cast<f32x4*>(sp + 4 * (r + R * qd)) = f32x4{S[4 * qd], S[4 * qd + 1], S[4 * qd + 2], S[4 * qd + 3]};
+  scan_tokens<T, R, MODE, cols, 256>(g, lds, r0, r1, h, hq, slot, col0);
 }
 
 // whether the unconditional kernel serves the launch: dk = 16 R exactly, whole column blocks,
@@ -316,14 +177,13 @@ extern "C" int dxm_linear_scan(int mode, float* out, float* state, int n_slots, 
   if (!seq_rows && n_seq != T_) return 4;
   if (qk_rep < 1 || H % qk_rep) return 5;
   ScanArgs g{out, state, q, k, v, qs, ks, vs, q_scale, k_scale, qk_rep, decay, gate, gs, g_bias, rate, skip, inv_tau,
-             pos, seq_rows, slots, n_slots, T_, H, dk, dv, 1, 0x7fffffff, 0};
+             pos, seq_rows, slots, n_slots, T_, H, dk, dv, 1, 0x7fffffff, 0, 0};
   // prompt portions in bf16: matrix-core chunks where the sizes fit; shorter runs of a sequence
   // (decode tokens among them) stay with the token scan
   if (!f32 && seq_rows && n_seq <= 65535 && T_ >= kChunkMinRows + n_seq - 1 && chunk_scan_ok(mode, g)) {
     if ((mode == kFixed && !decay) || (mode == kStep && (!gate || !rate)) || (mode == kChannel && !gate)) return 6;
     g.min_rows = kChunkMinRows;
-    launch_chunk_scan(mode, g, n_seq, st);
-    if (n_seq == 1) {
+    if (launch_chunk_scan(mode, g, n_seq, st) || n_seq == 1) {
       DX_CHECK_LAUNCH();
       return 0;
     }

@@ -42,20 +42,27 @@ template <int R> __device__ __forceinline__ float group_sum(float v) {
 // The sequence of a workgroup that is the k-th to go out: the k-th longest of those with `least` rows and more, so that the
 // longest does not start when a short one's place is free.  Where more than `most` have as many rows, they go as they
 // come: they even out by themselves, and every wave pays for comparing their lengths (some ten instructions a length, in the
-// workgroup of a decode row more than its work).  n = 0: there is none.  The lanes' loads are all asked for at once:
+// workgroup of a decode row more than its work).  Behind them, if asked for, the `others`, as they come.  n = 0: there is none.  The lanes' loads are all asked for at once:
 // where a launch is short, one that waits for another is a hundredth of it.
 struct SeqRows {
   int r0, n, slot, s;
 };
 template <bool ALL>  // all sequences count, whatever their length
-__device__ __forceinline__ SeqRows by_length(const int* seq_rows, const int* slots, int n_seq, int k, int least, int most) {
+__device__ __forceinline__ SeqRows by_length(const int* seq_rows, const int* slots, int n_seq, int k, int least, int most,
+                                             bool others = false) {
   if (n_seq > (ALL ? most : 64)) return SeqRows{seq_rows[k], seq_rows[k + 1] - seq_rows[k], slots[k], k};
   const int lane = threadIdx.x & 63, at = min(lane, n_seq - 1);
   const int r0 = seq_rows[at], end = seq_rows[at + 1], slot = slots[at];
   const int len = lane < n_seq ? end - r0 : INT_MIN;
   const uint64_t any = __builtin_amdgcn_ballot_w64(len >= least);
   const int count = __builtin_popcountll(any);
-  if (count <= k) return SeqRows{0, 0, 0, 0};
+  if (count <= k) {  // behind them the others as they come
+    const uint64_t rest = ~any & (n_seq == 64 ? ~0ull : (1ull << n_seq) - 1);
+    if (ALL || !others || k - count >= __builtin_popcountll(rest)) return SeqRows{0, 0, 0, 0};
+    const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(rest >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)rest, 0));
+    const int s = __builtin_ctzll(__builtin_amdgcn_ballot_w64(before == k - count) & rest);
+    return SeqRows{__builtin_amdgcn_readlane(r0, s), __builtin_amdgcn_readlane(len, s), __builtin_amdgcn_readlane(slot, s), s};
+  }
   int rank = 0;
   if (!ALL && count > most) {
     rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(any >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)any, 0));

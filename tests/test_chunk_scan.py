@@ -125,3 +125,41 @@ def test_rows_that_overlap(kind, stride):
 
     for got, want in zip(run(q, k, v, g, dt), run(*(x.contiguous() for x in (q, k, v, g, dt)))):
         torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [[200, 1, 7, 3, 1, 70, 1], [9, 1], [1] * 20 + [130, 140], [1, 2, 300, 0, 5, 129, 7] * 4])
+@pytest.mark.parametrize("kind,H,dk,dv", [("retention", 32, 128, 128), ("ssd", 64, 128, 64), ("gla", 32, 128, 128),
+                                          ("retention", 2, 64, 64), ("ssd", 4, 32, 128), ("gla", 5, 64, 64), ("gla", 3, 32, 64)])
+def test_short_sequences_beside_long_ones(rows, kind, H, dk, dv):
+    """Sequences too short for a chunk, in the launch of the long ones: the same bits as in a step of their own."""
+    torch.manual_seed(len(rows) + H)
+    T, n = sum(rows), len(rows)
+    q, k, v = (torch.randn(T, H * w).bfloat16().cuda() for w in (dk, dk, dv))
+    g = (torch.randn(T, H * dk if kind == "gla" else H) - 1.0).bfloat16().cuda()
+    bias, rate, skip = torch.randn(g.shape[1]).cuda(), torch.rand(H).cuda() * 3 + 0.1, torch.randn(H).cuda()
+    fixed = (1.0 - 2.0 ** (-3.0 - torch.arange(H) % 6)).cuda()
+    state0, slots = torch.randn(n, H, dv, dk).cuda(), torch.randperm(n).to(torch.int32)
+    pos = torch.cat([torch.arange(i % 3, i % 3 + r) for i, r in enumerate(rows)])
+
+    def step(which):
+        first = [0]
+        for i in which:
+            first.append(first[-1] + rows[i])
+        at = torch.cat([torch.arange(sum(rows[:i]), sum(rows[:i + 1])) for i in which])
+        S = state0.clone()
+        here = (pos[at].cuda(), torch.tensor(first, dtype=torch.int32).cuda(), slots[list(which)].cuda(), H)
+        at = at.cuda()
+        if kind == "retention":
+            o = rc.retention(q[at], k[at], v[at], fixed, dk ** -0.5, S, *here, dk, dv)
+        elif kind == "ssd":
+            o = rc.ssd(v[at], k[at], q[at], g[at], bias, rate, skip, S, *here, H, dk, dv)
+        else:
+            o = rc.gated_linear_attention(q[at], k[at], v[at], g[at], bias, 16.0, dk ** -0.5, S, *here, dk, dv)
+        return [o[first[j]:first[j + 1]] for j in range(len(which))], S
+
+    both, S = step(range(n))
+    for i, r in enumerate(rows):
+        if 0 < r < 8:
+            alone, A = step([i])
+            assert torch.equal(both[i], alone[0]) and torch.equal(S[slots[i].item()], A[slots[i].item()]), (i, r)
