@@ -282,9 +282,7 @@ def causal_conv(x: torch.Tensor, conv_w: torch.Tensor, conv_state: torch.Tensor,
         _m().conv_run(out.data_ptr(), x.data_ptr(), x.stride(0), conv_w.data_ptr(), _ptr(bias), int(act == "silu"), taps,
                       conv_state.data_ptr(), conv_state.shape[0], positions.data_ptr(), _ptr(row_seq), _ptr(seq_rows),
                       state_slots.data_ptr(), state_slots.numel(), T, C, _f32(x), _stream())
-        if row_seq is not None:  # (a decode step's kernel has written the new state)
-            conv_state_update(x, conv_state, positions, seq_rows, state_slots)
-        return out
+        return out  # (the kernel has written the new state)
     out = conv_rope_cache(x, conv_w, conv_state, positions, torch.full_like(positions, -1), row_seq, seq_rows, state_slots,
                           1, 0, C, 0, None, None, None, bias=bias, act=act)
     conv_state_update(x, conv_state, positions, seq_rows, state_slots)
