@@ -5,17 +5,26 @@
 //     out[dst(r), :] = a[src(r), :] @ w[e]^T        src(r) = order[r] / top (gather) or r, dst(r) = order[r] (scatter) or r
 // and with glu (weights in blocks of 32 gate rows and their 32 up rows) out = silu(gate) * up, [R, N / 2].
 //
-// A workgroup (4 waves) takes 32 weight rows of one expert -- 16 gate and their 16 up rows with glu -- and
-// all rows of the expert, 32 at a time; the waves share the width in pieces of 64 and their partial
+// A workgroup (2 or 4 waves) takes 32 weight rows of one expert -- 16 gate and their 16 up rows with glu -- and
+// all rows of the expert, 64 at a time; the waves share the width in pieces of 64 and their partial
 // sums are added in LDS in wave order.  v_mfma_f32_16x16x32_bf16 with the weights as A (lane: one weight row,
 // 32 contiguous bytes of each piece: four lanes read a whole line) and the activations as B in the same
-// order, so nothing is shuffled; D pieces are in flight per wave.
+// order, so nothing is shuffled; two pieces are in flight per wave.  More in flight is slower (three pieces
+// by a tenth, eight or sixteen waves by 6 to 50 %): HBM likes the few long runs of lines better.
+//
+// Bound by HBM.  A line is read by two loads, 16 bytes of each lane's 32 at a time, so the lines have to stay:
+// as nontemporal loads (before) part of them came from memory twice.  16 experts of 3584, 24 tokens, gate-up /
+// down: 169 / 93 us -> 144 / 75, 6.3 TB/s.  A pass takes 16, 32 or 64 rows, whichever holds the rest: a pass of
+// 16 leaves out the products and loads of the second tile (24 tokens: 148 / 77 us without), one of 64 reads the
+// weights once where two of 32 read them twice (8 experts of 2048, 100 tokens: 56 / 26 us -> 39 / 23).
 #include "../kernels/common.h"
 
 namespace {
 
 typedef uint32_t gs_raw4 __attribute__((ext_vector_type(4)));
 typedef __bf16 gs_bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kMT = 4, kDepth = 2;
 
 struct StreamGemmArgs {
   bf16_t* out;
@@ -27,8 +36,8 @@ struct StreamGemmArgs {
   int N, K, top, gather, scatter;
 };
 
-// MT: 16-row activation tiles, D: pieces in flight
-template <int MT, int D, bool GLU>
+// MT: 16-row activation tiles, NW: waves, NT: the weights' lines are not kept in L2
+template <int MT, int NW, bool NT, bool GLU>
 __device__ __forceinline__ void stream_pass(const StreamGemmArgs& g, int e, int lo, int rows, int j, f32x4* red) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
   // first weight rows of the two 16-row tiles
@@ -51,18 +60,22 @@ __device__ __forceinline__ void stream_pass(const StreamGemmArgs& g, int e, int 
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int m = 0; m < MT; ++m) C[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int D = kDepth;
   gs_raw4 W[D][2][2], A[D][MT][2];
-  const int np = (g.K / 64 - wave + 3) / 4;  // this wave's pieces: wave, wave + 4, ...
+  const int np = (g.K / 64 - wave + NW - 1) / NW;  // this wave's pieces: wave, wave + NW, ...
   auto fetch = [&](int s, int p) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        W[s][t][h] = __builtin_nontemporal_load(reinterpret_cast<const gs_raw4*>(wp[t] + (int64_t)p * 256 + 8 * h));
+      for (int h = 0; h < 2; ++h) {
+        const gs_raw4* q = reinterpret_cast<const gs_raw4*>(wp[t] + (int64_t)p * (64 * NW) + 8 * h);
+        if constexpr (NT) W[s][t][h] = __builtin_nontemporal_load(q);
+        else W[s][t][h] = *q;
+      }
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) A[s][m][h] = *reinterpret_cast<const gs_raw4*>(ap[m] + (int64_t)p * 256 + 8 * h);
+      for (int h = 0; h < 2; ++h) A[s][m][h] = *reinterpret_cast<const gs_raw4*>(ap[m] + (int64_t)p * (64 * NW) + 8 * h);
   };
   auto use = [&](int s) {
 #pragma unroll
@@ -98,12 +111,12 @@ __device__ __forceinline__ void stream_pass(const StreamGemmArgs& g, int e, int 
     for (int m = 0; m < MT; ++m) red[((wave * 2 + t) * MT + m) * 64 + lane] = C[t][m];
   __syncthreads();
   constexpr int kFrags = GLU ? MT : 2 * MT;
-  for (int f = wave; f < kFrags; f += 4) {
+  for (int f = wave; f < kFrags; f += NW) {
     const int t = GLU ? 0 : f / MT, m = GLU ? f : f - t * MT;
     auto total = [&](int tt) {
       f32x4 s = red[(tt * MT + m) * 64 + lane];
 #pragma unroll
-      for (int wv = 1; wv < 4; ++wv) s += red[((wv * 2 + tt) * MT + m) * 64 + lane];
+      for (int wv = 1; wv < NW; ++wv) s += red[((wv * 2 + tt) * MT + m) * 64 + lane];
       return s;
     };
     f32x4 v = total(t);
@@ -123,13 +136,16 @@ __device__ __forceinline__ void stream_pass(const StreamGemmArgs& g, int e, int 
   __syncthreads();  // (red is free again)
 }
 
-constexpr int kMT = 2, kDepth = 2;
-template <bool GLU>
-__global__ void __launch_bounds__(256, 4) stream_grouped_gemm_kernel(StreamGemmArgs g) {
-  __shared__ __attribute__((aligned(16))) f32x4 red[4 * 2 * kMT * 64];
+template <int NW, bool NT, bool GLU>
+__global__ void __launch_bounds__(64 * NW, 2) stream_grouped_gemm_kernel(StreamGemmArgs g) {
+  __shared__ __attribute__((aligned(16))) f32x4 red[NW * 2 * kMT * 64];
   const int e = blockIdx.y, j = blockIdx.x;
   const int lo = g.offsets[e], hi = g.offsets[e + 1];
-  for (int r = lo; r < hi; r += 16 * kMT) stream_pass<kMT, kDepth, GLU>(g, e, r, min(hi - r, 16 * kMT), j, red);
+  for (int r = lo; r < hi; r += 16 * kMT) {
+    if (hi - r <= 16) stream_pass<1, NW, NT, GLU>(g, e, r, hi - r, j, red);
+    else if (hi - r <= 32) stream_pass<2, NW, NT, GLU>(g, e, r, hi - r, j, red);
+    else stream_pass<kMT, NW, NT, GLU>(g, e, r, min(hi - r, 16 * kMT), j, red);
+  }
 }
 
 }  // namespace
@@ -149,8 +165,20 @@ int dxm_stream_grouped_gemm(void* out, const void* a, int64_t a_stride, const vo
     return 2;
   const StreamGemmArgs g{(bf16_t*)out, (const bf16_t*)a, a_stride, (const bf16_t*)w, order, offsets, N, K, top, gather, scatter};
   const dim3 grid((unsigned)(N / 32), (unsigned)E);
-  if (glu) hipLaunchKernelGGL(stream_grouped_gemm_kernel<true>, grid, dim3(256), 0, st, g);
-  else hipLaunchKernelGGL(stream_grouped_gemm_kernel<false>, grid, dim3(256), 0, st, g);
+  // Two waves where four would have no more than eight pieces each: 2048 wide, 8 experts, gate-up + down, 3 / 16 / 40
+  // tokens, us: 33.2 / 45.8 / 48.5 with four, 29.0 / 44.8 / 46.2 with two; 4096 and 3584 wide, 16 experts, 6 / 24 tokens:
+  // 125.6 / 223.1 with four, 141.7 / 237.3 with two.
+  const bool two = K <= 2048;
+  // One token's experts there: of 1 / 2 / 4 layers of them the repeated step takes 33.3 / 60.7 / 125.9 us with lines not
+  // kept, 33.1 / 64.8 / 132.9 kept (before: 33.8 / 66.0 / 131); from two tokens on it is the other way round, 78.0 / 75.9
+  // for two layers and 163 / 148 for four.
+  const bool nt = two && R <= 2;
+  auto kern = nt    ? (glu ? stream_grouped_gemm_kernel<2, true, true> : stream_grouped_gemm_kernel<2, true, false>)
+              : two ? (glu ? stream_grouped_gemm_kernel<2, false, true> : stream_grouped_gemm_kernel<2, false, false>)
+                    : (glu ? stream_grouped_gemm_kernel<4, false, true> : stream_grouped_gemm_kernel<4, false, false>);
+  // LDS that is not used keeps four-wave workgroups at two a CU.  Few experts with rows are few workgroups, and the
+  // dispatcher would pile four on one CU and leave others idle: 4 experts, down (512 workgroups): 29.6 us -> 23.3.
+  hipLaunchKernelGGL(kern, grid, dim3(two ? 128 : 256), two ? 0 : 32 * 1024, st, g);
   DX_CHECK_LAUNCH();
   return 0;
 }

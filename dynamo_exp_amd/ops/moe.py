@@ -22,8 +22,13 @@ from .mixers import _f32, _fp32_param, _ptr, _stream
 ROUTER_SCORES = {"sigmoid": 0, "softmax": 1}
 GROUP_SCORES = {"top2": 0, "max": 1}
 # weight-streaming grouped GEMM: up to this many rows per expert on average where the 256-tile kernel's grid (one
-# workgroup per expert and 256 columns) would leave a good part of the chip idle, half as many elsewhere
-STREAM_ROWS = 24
+# workgroup per expert and 256 columns) would leave a good part of the chip idle; elsewhere a quarter, or three where
+# that kernel does not take the shape.  Gate-up + down, us,
+# streamed / 256-tile: 8 experts of 2048, 112 / 128 / 144 tokens (28 / 32 / 36 rows): 66 / 82, 75 / 83, 81 / 84, then 53.7 + 35.2
+# against 47.2 + 39.4 at 50 rows; 16 experts of 3584, 64 / 72 / 80 tokens (8 / 9 / 10 rows): 265 / 264, 268 / 266, 274 / 268.
+# Against the 64 x 64-tile kernel: 32 rows, 8 x [640, 1024] 8.3 / 22.5, 16 x [1408, 2048] 38 / 56; 24 and 32 rows, 8 x [14336, 4160]
+# 228 / 231 and 255 / 246
+STREAM_ROWS = 32
 STREAM_TILES = 192
 # row tiles per band of the 256-tile kernel's walk: 16 experts, 300 / 500 / 1000 / 2500 / 4000 tokens, us: 6 307 327 380 531 751,
 # 8 318 347 402 540 759, 2 319 347 391 547 803, 16 slower than 8
@@ -144,7 +149,8 @@ def stream_gemm_ok(a: torch.Tensor, w: torch.Tensor, R: int) -> bool:
     """Whether the weight-streaming kernel (csrc/mixers/grouped_stream.hip) takes
     R rows against w [E, N, K]: few rows per expert, whole pieces."""
     E, N, K = w.shape
-    most = STREAM_ROWS if not tile_gemm_ok(a, w) or E * (N // 256) < STREAM_TILES else STREAM_ROWS // 2
+    few = E * (N // 256) < STREAM_TILES
+    most = STREAM_ROWS if few else STREAM_ROWS // 4 if tile_gemm_ok(a, w) else STREAM_ROWS * 3 // 4
     return (a.is_cuda and a.dtype == torch.bfloat16 and R <= most * E and a.stride(0) % 8 == 0 and
             a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and bool(_m().stream_grouped_ok(N, K)))
 
