@@ -57,9 +57,10 @@ __device__ __forceinline__ i16x4 read_tr16(const lds_i16x4* __restrict__ p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
 }
 // 16 bytes a lane from `off` bytes behind `from` to LDS; zeros from `bytes` on.  (global_load_lds would count as an LDS access
-// as well, and every wait for an LDS read become one for all of them.)
+// as well, and every wait for an LDS read become one for all of them.)  NT 2: a nontemporal read.
+template <int NT = 0>
 __device__ __forceinline__ void dma16(const void* from, int bytes, int off, lds_void* to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), to, 16, off, 0, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)from, 0, bytes, 0x00020000), to, 16, off, 0, 0, NT);
 }
 // every wave is done with a tile, and the DMA of the next has landed
 __device__ __forceinline__ void landed() {

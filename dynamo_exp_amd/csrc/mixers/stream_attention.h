@@ -36,8 +36,9 @@ typedef __attribute__((address_space(3))) raw_u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) float lds_float;
 __device__ __forceinline__ bf16x8_t lds_frag(uint32_t at) { return __builtin_bit_cast(bf16x8_t, *(const lds_u32x4*)(uintptr_t)at); }
 
+template <int NT = 0>
 __device__ __forceinline__ void dma16(const void* from, int bytes, int off, uint32_t to) {
-  ::dma16(from, bytes, off, (lds_void*)(uintptr_t)to);
+  ::dma16<NT>(from, bytes, off, (lds_void*)(uintptr_t)to);
 }
 
 __device__ __forceinline__ bf16x8_t frag16(const bf16_t* p) {

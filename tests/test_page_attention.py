@@ -465,3 +465,30 @@ def test_prompt_rows_in_parts_beside_decode_rows(monkeypatch, form, pre, parts, 
     err, top = float((got - want).abs().max()), float(want.abs().max())
     # (as in test_prompt_rows)
     assert err < (3e-4 if out_f32 else 2.0 ** -8 * (top + (top if sig else 5.0))), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 100, 40), ("window", 1, 0), ("chunk", 192, 0)])
+@pytest.mark.parametrize("form", ["plain", "both", "sigmoid", "diff"])
+def test_decode_rows_that_read_much(form, mask, size, keep):
+    """Launches on both sides of the line beyond which cache lines are read nontemporally, with rows of both kinds in one: how
+    a line is read changes no bit, so each row is what it is in a launch of eight."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(41)
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    lengths, bs = [1000, 33, 96, 350, 1, 200], 32
+    kd, vd, table, _ = pages(form, lengths, bs)
+    for n, parts in ((600, 1), (64, 2)):
+        seq = torch.arange(n, dtype=torch.int32) % len(lengths)
+        pos = torch.tensor(lengths)[seq.long()] - 1
+        tiles = (48 << 20) // (2 * 32 * (kd.shape[1] + vd.shape[1]) * n)
+        assert 1 <= tiles < 1000 // 32  # (rows of more tiles do not keep their lines)
+        q, pos, seq = torch.randn(n, n_qh * d).bfloat16().cuda(), pos.cuda(), seq.cuda()
+
+        def run(i, j):
+            return mx.attention(q[i:j], kd, vd, pos[i:j], seq[i:j], table, bs, n_qh, maps, group, d, dv, 0.7 * d ** -0.5, mask,
+                                size, parts, True, softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
+                                weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), keep_first=keep, sink=cuda(sink))
+        got = run(0, n)
+        for i in (0, 8, n // 2, n - 8):
+            assert bool((got[i:i + 8] == run(i, i + 8)).all()), (n, i)
