@@ -56,8 +56,8 @@ template <typename T> __device__ __forceinline__ float2 step_terms(const ScanArg
 // The first block is asked for in front of the state and staged while the state is on its way (its barriers wait for LDS
 // only), and the state in front of the position that says whether it counts, so that a decode step is one latency, not three
 // (four layers of gated linear attention, 16 heads, 5 sequences 38.9 -> 37.6 us with the latter).  Bound by memory: two layers with their other launches in a graph, us:
-// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 230 (its kernel at 64: 5.2
-// TB/s of state); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 135.
+// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 60 / 204 (the latter two with
+// ONCE, 64 and 230 without); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 112 (135 without).
 template <int DK, int MODE, int COLS> struct ScanLds {
   __attribute__((aligned(16))) float q[kTok * DK];
   __attribute__((aligned(16))) float k[kTok * DK];
@@ -67,8 +67,9 @@ template <int DK, int MODE, int COLS> struct ScanLds {
 };
 
 // rows r0 .. r1 - 1 (of one sequence, whose state is in `slot`) of columns col0 .. + COLS - 1 of head h, by a workgroup of NT
-// threads, COLS R of which own columns; hq: its q / k head (a division, which the caller has done beside its loads)
-template <typename T, int R, int MODE, int COLS, int NT>
+// threads, COLS R of which own columns; hq: its q / k head (a division, which the caller has done beside its loads); ONCE: the
+// state's lines are not kept (state_once)
+template <typename T, int R, int MODE, int COLS, int NT, bool ONCE = false>
 __device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, MODE, COLS>& lds, int r0, int r1, int h, int hq, int slot,
                                             int col0) {
   constexpr int dk = 16 * R, cols = COLS, VEC = 16 / (int)sizeof(T);
@@ -159,7 +160,7 @@ __device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, M
   // (asked for before it is known whether it counts: at position 0 the state is zero, whatever the slot held)
   float S[16];
 #pragma unroll
-  for (int qd = 0; qd < 4; ++qd) *reinterpret_cast<f32x4*>(S + 4 * qd) = *reinterpret_cast<const f32x4*>(sp + 4 * (r + R * qd));
+  for (int qd = 0; qd < 4; ++qd) *reinterpret_cast<f32x4*>(S + 4 * qd) = load_state<ONCE>(sp + 4 * (r + R * qd));
   const bool fresh = g.pos[r0] == 0;
   for (int t0 = r0; t0 < r1; t0 += kTok) {
     const int nt = r1 - t0 < kTok ? r1 - t0 : kTok;
@@ -200,7 +201,7 @@ __device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, M
   if (!owner) return;
 #pragma unroll
   for (int qd = 0; qd < 4; ++qd)
-    *reinterpret_cast<f32x4*>(sp + 4 * (r + R * qd)) = f32x4{S[4 * qd], S[4 * qd + 1], S[4 * qd + 2], S[4 * qd + 3]};
+    store_state<ONCE>(sp + 4 * (r + R * qd), f32x4{S[4 * qd], S[4 * qd + 1], S[4 * qd + 2], S[4 * qd + 3]});
 }
 
 // a sequence with at least this many rows in the step goes through the chunked kernels

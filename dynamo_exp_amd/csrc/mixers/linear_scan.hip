@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256) scan_kernel(ScanArgs g) {
 }
 
 // scan_tokens for every sequence of a step
-template <typename T, int R, int MODE>
+template <typename T, int R, int MODE, bool ONCE>
 __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
   constexpr int cols = 256 / R;
   __shared__ ScanLds<16 * R, MODE, cols> lds;
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256) scan_fast_kernel(ScanArgs g) {
       if (threadIdx.x % R == 0) g.out[(int64_t)t * g.H * g.dv + h * g.dv + col0 + threadIdx.x / R] = 0.f;
     return;
   }
-  scan_tokens<T, R, MODE, cols, 256>(g, lds, r0, r1, h, hq, slot, col0);
+  scan_tokens<T, R, MODE, cols, 256, ONCE>(g, lds, r0, r1, h, hq, slot, col0);
 }
 
 // whether the unconditional kernel serves the launch: dk = 16 R exactly, whole column blocks,
@@ -141,7 +141,8 @@ template <typename T, int R, int MODE, int ROWS = kRows>
 void launch_scan(const ScanArgs& g, int n_seq, hipStream_t st) {
   if constexpr (ROWS == kRows) {
     if (scan_fast_ok<T, R, MODE>(g)) {
-      hipLaunchKernelGGL((scan_fast_kernel<T, R, MODE>), dim3(n_seq, g.H, g.dv / (256 / R)), dim3(256), 0, st, g);
+      auto kern = state_once(n_seq, g.H, g.dk, g.dv) ? scan_fast_kernel<T, R, MODE, true> : scan_fast_kernel<T, R, MODE, false>;
+      hipLaunchKernelGGL(kern, dim3(n_seq, g.H, g.dv / (256 / R)), dim3(256), 0, st, g);
       return;
     }
   }

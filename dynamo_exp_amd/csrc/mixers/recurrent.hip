@@ -91,12 +91,12 @@ __global__ void __launch_bounds__(NT) delta_rule_kernel(DeltaArgs g) {
 // state and formed while it is on its way, one or two of them by each wave, with delta_prep_kernel's arithmetic.
 // Bound by memory from some 40 sequences on, by latency below.  Two layers with their norms in a graph, 32 heads of 128 columns,
 // 1 / 3 / 12 / 40 / 128 sequences, us: 25 / 30 / 49 / 114 / 278 with delta_prep_kernel in front and the kernel for runs of
-// tokens, 21 / 21 / 33 / 89 / 231 (168 MB of state a layer at 40: 4.7 TB/s with the norm) like this; that kernel forming the rows itself
-// 20 / 26 / 46 / 128 / 330, for it stages eight tokens.
+// tokens, 21 / 21 / 33 / 89 / 231 like this; that kernel forming the rows itself 20 / 26 / 46 / 128 / 330, for it stages eight tokens.
+// With the state's lines not kept (ONCE) 40 sequences take 75 (168 MB of state a layer: 5.7 TB/s with the norm).
 constexpr int kDeltaStepLanes = 8;
 bool delta_forms_itself(const int* seq_rows, int dk) { return !seq_rows && dk == kDeltaStepLanes * kRows; }
 
-template <typename T, int CT>
+template <typename T, int CT, bool ONCE>
 __global__ void __launch_bounds__(256) delta_step_kernel(DeltaArgs g) {
   constexpr int R = kDeltaStepLanes, D = R * kRows;
   __shared__ __attribute__((aligned(16))) float row[5][D];  // unit key, decay, removal rate * unit key, key, read-out
@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaArgs g) {
   for (int c = 0; c < CT; ++c)
 #pragma unroll
     for (int m = 0; m < kRows / 4; ++m) {
-      const f32x4 y = fresh || j0 + c >= g.dv ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + c * D + 4 * m * R);
+      const f32x4 y = fresh || j0 + c >= g.dv ? f32x4{0.f, 0.f, 0.f, 0.f} : load_state<ONCE>(sp + c * D + 4 * m * R);
       S[c][4 * m] = y[0], S[c][4 * m + 1] = y[1], S[c][4 * m + 2] = y[2], S[c][4 * m + 3] = y[3];
     }
   if (wave == 1) {
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaArgs g) {
     if (part == 0) op[c] = o_[c];
 #pragma unroll
     for (int m = 0; m < kRows / 4; ++m)
-      *reinterpret_cast<f32x4*>(sp + c * D + 4 * m * R) = f32x4{S[c][4 * m], S[c][4 * m + 1], S[c][4 * m + 2], S[c][4 * m + 3]};
+      store_state<ONCE>(sp + c * D + 4 * m * R, f32x4{S[c][4 * m], S[c][4 * m + 1], S[c][4 * m + 2], S[c][4 * m + 3]});
   }
 }
 
@@ -176,7 +176,8 @@ void launch_delta_ct(const DeltaArgs& g, int n_seq, hipStream_t st) {
   if constexpr (R == kDeltaStepLanes) {
     if (!g.prep) {
       constexpr int cols = 256 / R * CT;
-      hipLaunchKernelGGL((delta_step_kernel<T, CT>), dim3(n_seq, g.H, (g.dv + cols - 1) / cols), dim3(256), 0, st, g);
+      auto kern = state_once(n_seq, g.H, g.dk, g.dv) ? delta_step_kernel<T, CT, true> : delta_step_kernel<T, CT, false>;
+      hipLaunchKernelGGL(kern, dim3(n_seq, g.H, (g.dv + cols - 1) / cols), dim3(256), 0, st, g);
       return;
     }
   }
