@@ -54,11 +54,13 @@ struct DecodeArgs {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 // A launch that reads more of the cache than this asks for it nontemporally: each line is read once, whole, and behind so many
-// the L2s (32 MB) hold none of it for the next step.  Less is kept.  Per launch, kept / not, us: two maps, window 1024 + 64,
-// 8 / 32 / 48 MB 18.3 / 19.4, 18.8 / 20.0, 21.8 / 21.7 (10 rows), 64 MB 27.8 / 26.0, 190 MB 48.7 / 43.3; plain heads,
-// 32 MB 15.6 / 16.4, 64 MB 23.4 / 21.5, 300 MB 68.4 / 60.8 (5.0 TB/s).  A shared row (one cache for all heads) gains
-// nothing: 46.9 / 48.2 and 64.9 / 62.8 for two launches of 40 and 100 rows.
-constexpr int64_t kKept = 48 << 20;
+// no cache holds much of it for the next step.  Less is kept.  Each row takes the others to be as long as itself, which a
+// window's mostly are; other rows' lengths differ, so their line lies higher.  One layer's repeated launch, kept / not, us: plain
+// heads, 51 / 85 / 128 MB 20.0 / 21.1, 26.5 / 26.9, 37.3 / 33.6; capped, window 1024, 84 / 126 / 200 MB 27.5 / 27.8, 34.4 / 31.8,
+// 50.1 / 42.8; rows in chunks of 2048, the longest 131 of 67 MB 23.5 / 26.3.  Two launches of other layers: two maps, 190 MB
+// 97.4 / 86.5; plain heads, 300 MB 137 / 122 (5.0 TB/s).  A shared row (one cache for all heads) gains nothing: 46.9 / 48.2 and
+// 64.9 / 62.8 for two launches of 40 and 100 rows.
+constexpr int64_t kKeptWindow = 96 << 20, kKept = 160 << 20;
 constexpr int kTile = 32;       // keys per tile
 constexpr float kDefer = 8.f;   // log2 units that a score may exceed the running maximum by (weights are bf16 pairs)
 enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
@@ -520,7 +522,7 @@ int dxm_decode_attention(void* out, float* ws, const void* q, int64_t q_stride, 
   // tiles a row may have at most (a window and the keys kept in front of it may each reach into two more), and of how many
   // rows still keep their lines
   const int64_t most = mask ? ((int64_t)size + keep) / kTile + 4 : (int64_t)bt_stride * bs / kTile;
-  const int64_t kept = kKept / (2 * kTile * ((int64_t)Wk + Wv) * rows);
+  const int64_t kept = (mask == 1 ? kKeptWindow : kKept) / (2 * kTile * ((int64_t)Wk + Wv) * rows);
   const bool many = most > kept;
   DecodeArgs a{out, ws, (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, pos, seq, bt, bt_stride,
                __builtin_ctz((unsigned)bs), n_qh, maps, group, Wk, Wv, scale, mask, size, parts, softcap, r1, r2, hbias,

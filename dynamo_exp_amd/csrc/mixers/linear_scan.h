@@ -56,8 +56,8 @@ template <typename T> __device__ __forceinline__ float2 step_terms(const ScanArg
 // The first block is asked for in front of the state and staged while the state is on its way (its barriers wait for LDS
 // only), and the state in front of the position that says whether it counts, so that a decode step is one latency, not three
 // (four layers of gated linear attention, 16 heads, 5 sequences 38.9 -> 37.6 us with the latter).  Bound by memory: two layers with their other launches in a graph, us:
-// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 60 / 204 (the latter two with
-// ONCE, 64 and 230 without); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 112 (135 without).
+// state-space duality, 128 heads of 64 columns, 2 / 12 / 64 sequences 32 / 70 / 239 -> 30 / 64 / 204 (the last with
+// ONCE, 230 without); gated linear attention, 32 heads of 128 columns, 12 / 64: 39 / 139 -> 38 / 112 (135 without).
 template <int DK, int MODE, int COLS> struct ScanLds {
   __attribute__((aligned(16))) float q[kTok * DK];
   __attribute__((aligned(16))) float k[kTok * DK];

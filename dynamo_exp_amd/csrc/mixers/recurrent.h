@@ -26,10 +26,7 @@ __device__ __forceinline__ float fast_sigmoid(float z) {
 }
 
 // Four neighbours of a state matrix, read and written once a step.  ONCE: nontemporally, for a decode step whose states
-// the L2s (32 MB) could not hold for the next one anyway (state_once: from 44 MB on).  Two layers with their other launches,
-// us, kept / not: retention, 16 heads, 24 / 30 / 36 / 42 / 48 / 64 MB 29.0 / 31.3, 33.5 / 37.7, 36.6 / 44.5, 44.9 / 47.2, 56.1 / 50.2,
-// 85 / 70; gated linear attention and the delta rule, 32 heads, 44 MB 57.6 / 52.0 and 51.0 / 46.2, 128 MB 134 / 112 and 128 / 107.
-// (Only read nontemporally: 128 MB 133, only written: 132.)
+// no cache could hold for the next one anyway (state_once).
 template <bool ONCE> __device__ __forceinline__ f32x4 load_state(const float* p) {
   if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
   else return *reinterpret_cast<const f32x4*>(p);
@@ -38,7 +35,11 @@ template <bool ONCE> __device__ __forceinline__ void store_state(float* p, f32x4
   if constexpr (ONCE) __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
   else *reinterpret_cast<f32x4*>(p) = v;
 }
-inline bool state_once(int n_seq, int H, int dk, int dv) { return (int64_t)n_seq * H * dk * dv * 4 >= 44 << 20; }
+// One layer's repeated step, kept / not, us: state-space duality, 128 heads, 64 / 88 / 128 MB 33.8 / 39.7, 45.2 / 49.3, 67.7 / 59.8;
+// delta rule, 32 heads, 64 / 88 / 128 MB 29.2 / 33.4, 42.2 / 41.9, 66.5 / 55.2; gated linear attention 72 / 96 / 128 MB 39.1 / 40.2,
+// 52.3 / 49.0, 69.5 / 57.4.  (Steps of several layers gain from 44 MB a layer on, up to a fifth, and one that repeats a
+// single layer loses as much there.  Only read or only written nontemporally: nothing.)
+inline bool state_once(int n_seq, int H, int dk, int dv) { return (int64_t)n_seq * H * dk * dv * 4 >= 128 << 20; }
 
 template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));

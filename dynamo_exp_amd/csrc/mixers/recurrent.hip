@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(NT) delta_rule_kernel(DeltaArgs g) {
 // Bound by memory from some 40 sequences on, by latency below.  Two layers with their norms in a graph, 32 heads of 128 columns,
 // 1 / 3 / 12 / 40 / 128 sequences, us: 25 / 30 / 49 / 114 / 278 with delta_prep_kernel in front and the kernel for runs of
 // tokens, 21 / 21 / 33 / 89 / 231 like this; that kernel forming the rows itself 20 / 26 / 46 / 128 / 330, for it stages eight tokens.
-// With the state's lines not kept (ONCE) 40 sequences take 75 (168 MB of state a layer: 5.7 TB/s with the norm).
+// With the state's lines not kept (ONCE, from 64 sequences on) 64 take 107 instead of 128.
 constexpr int kDeltaStepLanes = 8;
 bool delta_forms_itself(const int* seq_rows, int dk) { return !seq_rows && dk == kDeltaStepLanes * kRows; }
 

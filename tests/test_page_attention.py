@@ -476,13 +476,13 @@ def test_decode_rows_that_read_much(form, mask, size, keep):
     n_qh, maps, group, d, dv = FORMS[form]
     torch.manual_seed(41)
     cap, db, sig, hb, sink = terms(form, n_qh)
-    lengths, bs = [1000, 33, 96, 350, 1, 200], 32
+    lengths, bs = [2000, 33, 96, 350, 1, 200], 32
     kd, vd, table, _ = pages(form, lengths, bs)
-    for n, parts in ((600, 1), (64, 2)):
+    for n, parts in ((600, 1), (64 if form == "diff" else 100, 2)):
         seq = torch.arange(n, dtype=torch.int32) % len(lengths)
         pos = torch.tensor(lengths)[seq.long()] - 1
-        tiles = (48 << 20) // (2 * 32 * (kd.shape[1] + vd.shape[1]) * n)
-        assert 1 <= tiles < 1000 // 32  # (rows of more tiles do not keep their lines)
+        tiles = ((96 if mask == "window" else 160) << 20) // (2 * 32 * (kd.shape[1] + vd.shape[1]) * n)
+        assert 1 <= tiles < 2000 // 32  # (rows of more tiles do not keep their lines)
         q, pos, seq = torch.randn(n, n_qh * d).bfloat16().cuda(), pos.cuda(), seq.cuda()
 
         def run(i, j):
