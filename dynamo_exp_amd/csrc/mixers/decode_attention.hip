@@ -422,9 +422,9 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
       if (MODE == kSigmoid) mt[qb] = 0.f;
       lt[qb] = 0.f;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {  // a wave without a tile: sum 0, maximum -inf
+      for (int v = 0; v < 4; ++v) {  // a wave without a tile: sum 0, maximum -inf (a NaN stays one)
         const float l = ml[1][v][qb][c16];
-        lt[qb] += MODE == kSigmoid ? l : l > 0.f ? l * fast_exp2(ml[0][v][qb][c16] - mt[qb]) : 0.f;
+        lt[qb] += MODE == kSigmoid ? l : l != 0.f ? l * fast_exp2(ml[0][v][qb][c16] - mt[qb]) : 0.f;
       }
     }
     constexpr int kSlab = QB * NC * 64;  // f32x4 of a wave

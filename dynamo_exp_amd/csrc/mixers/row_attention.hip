@@ -240,27 +240,30 @@ __global__ void __launch_bounds__(256) merge_parts_kernel(PartSums<OutT, GT> a, 
     const int head = (int)(v - row * n_qh) / maps;
     post /= 1.f + expf(-Elem<GT>::ld(gate, row * gs + head));
   }
-  // lane p: part p (of 64 at a time); parts without a key have sum 0 and count for nothing
+  // lane p: part p (of 64 at a time); parts without a key have sum 0 and count for nothing (those alone: a part that saw a NaN
+  // has a NaN for its sum, which makes the row one)
   float m0 = -INFINITY, l0 = 0.f;
   if (lane < parts) m0 = w[(int64_t)lane * step], l0 = w[(int64_t)lane * step + 1];
   float mx = m0;
   for (int p = lane + 64; p < parts; p += 64) mx = fmaxf(mx, w[(int64_t)p * step]);
   mx = wave_reduce_max(mx);
-  float f0 = l0 > 0.f ? __expf(m0 - mx) : 0.f;
-  float l = l0 > 0.f ? l0 * f0 : 0.f;
+  float f0 = l0 != 0.f ? __expf(m0 - mx) : 0.f;
+  float l = l0 != 0.f ? l0 * f0 : 0.f;
   for (int p = lane + 64; p < parts; p += 64) {
     const float lp = w[(int64_t)p * step + 1];
-    if (lp > 0.f) l += lp * __expf(w[(int64_t)p * step] - mx);
+    if (lp != 0.f) l += lp * __expf(w[(int64_t)p * step] - mx);
   }
   l = wave_reduce_sum(l);
   if (sink && !plain) l += expf(sink[v % n_qh] - mx);
   const float inv = plain ? post : post / l;
   // parts behind the last with a key hold nothing
-  const int n = parts > 64 ? parts : 64 - __builtin_clzll(__builtin_amdgcn_ballot_w64(l0 > 0.f) | 1);
+  const uint64_t keys = __builtin_amdgcn_ballot_w64(l0 != 0.f);
+  const int n = parts > 64 ? parts : 64 - __builtin_clzll(keys | 1);
+  auto counts = [&](int p) { return p < 64 ? (keys >> p & 1) != 0 : w[(int64_t)p * step + 1] != 0.f; };
   auto factor = [&](int p) {  // the same in every lane
     if (p < 64) return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f0), p));
     const float* wp = w + (int64_t)p * step;
-    return wp[1] > 0.f ? __expf(wp[0] - mx) : 0.f;
+    return __expf(wp[0] - mx);
   };
   if (pairs) {
     float2 a0 = {0.f, 0.f}, a1 = {0.f, 0.f};
@@ -268,8 +271,8 @@ __global__ void __launch_bounds__(256) merge_parts_kernel(PartSums<OutT, GT> a, 
       if (p0) columns(p0, n - 1);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const float f = p0 + k < n ? factor(p0 + k) : 0.f;
-        if (f > 0.f) {  // (what a part without a key left there may be anything)
+        if (p0 + k < n && counts(p0 + k)) {  // (what a part without a key left there may be anything)
+          const float f = factor(p0 + k);
           a0.x += x0[k].x * f, a0.y += x0[k].y * f;
           a1.x += x1[k].x * f, a1.y += x1[k].y * f;
         }
@@ -287,10 +290,8 @@ __global__ void __launch_bounds__(256) merge_parts_kernel(PartSums<OutT, GT> a, 
   }
   for (int e = lane; e < dv; e += 64) {
     float acc = 0.f;
-    for (int p = 0; p < n; ++p) {
-      const float f = factor(p);
-      if (f > 0.f) acc += w[(int64_t)p * step + 2 + e] * f;
-    }
+    for (int p = 0; p < n; ++p)
+      if (counts(p)) acc += w[(int64_t)p * step + 2 + e] * factor(p);
     Elem<OutT>::st(out, v * dv + e, acc * inv);
   }
 }

@@ -468,6 +468,51 @@ def test_prompt_rows_in_parts_beside_decode_rows(monkeypatch, form, pre, parts, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("pre,parts", [((1, 0), 1), ((2, 0), 2), ((8, 0), 16), ((4, 200), 5)])
+@pytest.mark.parametrize("at", [3, 500, 1035])
+@pytest.mark.parametrize("mask,size", [("causal", 0), ("window", 900)])
+@pytest.mark.parametrize("form", ["plain", "fine", "both", "sigmoid", "diff", "shared"])
+def test_rows_that_see_a_nan(monkeypatch, form, mask, size, at, pre, parts):
+    """A key that holds a NaN, in the first, a middle and the last part of the contexts of prompt and decode rows, and query
+    vectors that do: the rows and heads that see it are NaN however the keys are cut, with a sink and without, and no others."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(47)
+    scale, bs = 0.7 * d ** -0.5, 64
+    lengths, rows, Tp = [1047, 531, 1047, 650], [17, 40, 1, 1], 57
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    kd, vd, table, kv = pages(form, lengths, bs)
+    col = 200 if form == "shared" else 5  # (of a shared row: a column that is no value's)
+    for i in (0, 2):
+        kd[int(table[i, at // bs]) * bs + at % bs, col] = float("nan")
+    q, q_nan = torch.randn(sum(rows), n_qh, d).bfloat16(), torch.zeros(sum(rows), n_qh, dtype=torch.bool)
+    q_nan[20, 1] = q_nan[-1, 1] = True
+    heads = torch.arange(n_qh) // maps
+    hit = ((heads // group == 0) & (torch.arange(n_qh) % maps == 0)) | (form == "shared")  # heads of the key with the NaN
+    want, pos = [], []
+    for i, (n, r) in enumerate(zip(lengths, rows)):
+        p = torch.arange(n - r, n)
+        pos.append(p)
+        w = dense(q[sum(rows[:i]):sum(rows[:i + 1])].double(), *kv[i], p, scale, mask, size, 0, cap, db, sink, sig, hb)
+        if i in (0, 2):
+            w[((p >= at) & (mx.first_visible(p, mask, size) <= at))[:, None] & hit] = float("nan")
+        want.append(w)
+    want = torch.cat(want)
+    want[q_nan] = float("nan")
+    q[q_nan] = float("nan")
+    monkeypatch.setattr(mx, "_prompt_parts", lambda *a: pre)
+    seq = torch.tensor([i for i, r in enumerate(rows) for _ in range(r)], dtype=torch.int32).cuda()
+    tiles = torch.tensor(mx.tile_list(0, 17) + mx.tile_list(17, 40), dtype=torch.int32).cuda()
+    got = mx.attention(q.view(sum(rows), -1).cuda(), kd, vd, torch.cat(pos).cuda(), seq, table, bs, n_qh, maps, group, d, dv, scale,
+                       mask, size, parts, form == "diff", tiles, Tp, softcap=cap,
+                       dist_bias=None if db is None else tuple(map(cuda, db)), weights="sigmoid" if sig else "softmax",
+                       head_bias=cuda(hb), sink=cuda(sink), fine_weights=form == "fine").cpu().double()
+    assert torch.equal(got.isnan(), want.isnan())
+    err, top = float((got - want).nan_to_num().abs().max()), float(want.nan_to_num().abs().max())
+    # (as in test_prompt_rows)
+    assert err < (3e-4 if form == "diff" else 2.0 ** -8 * (top + (top if sig else 5.0))), err
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 100, 40), ("window", 1, 0), ("chunk", 192, 0)])
 @pytest.mark.parametrize("form", ["plain", "both", "sigmoid", "diff"])
 def test_decode_rows_that_read_much(form, mask, size, keep):
