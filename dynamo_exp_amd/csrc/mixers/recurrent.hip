@@ -449,14 +449,20 @@ __global__ void __launch_bounds__(128) conv_run_kernel(ConvArgs g, T* __restrict
   };
   if constexpr (R > 1 && M > 0) {
     if ((int)blockIdx.y >= runs) {  // ---- a sequence's first rows and its tail
-      const int s = seq0 + blockIdx.y - runs, slot = g.slots[s], r0 = g.seq_rows[s], n = g.seq_rows[s + 1] - r0;
-      if (n <= 0 || r0 < 0 || r0 + n > g.T) return;
+      const int s = seq0 + blockIdx.y - runs, slot = g.slots[s], r0 = g.seq_rows[s], r1 = g.seq_rows[s + 1];
+      if (r0 < 0 || r0 >= g.T) return;
+      // whose a row is, row_seq says; a sequence without rows, or with some that the step does not hold, keeps its tail
+      const bool moves = r1 > r0 && r1 <= g.T;
+      const int n = moves ? r1 - r0 : 1;
       const bool live = slot >= 0 && slot < g.n_slots;
       T* tl = tail + (int64_t)(live ? slot : 0) * M * C + c;
       raw_u32x4 in[M], was[M], last[M];  // the first rows, the old tail, the last rows
+      bool its[M];
 #pragma unroll
       for (int m = 0; m < M; ++m) {
-        in[m] = *reinterpret_cast<const raw_u32x4*>(x + (int64_t)(r0 + min(m, n - 1)) * g.xs);
+        const int t = min(r0 + m, g.T - 1);
+        its[m] = (r0 + m < g.T) & (g.row_seq[t] == s);
+        in[m] = *reinterpret_cast<const raw_u32x4*>(x + (int64_t)t * g.xs);
         was[m] = live ? *reinterpret_cast<const raw_u32x4*>(tl + (int64_t)m * C) : raw_u32x4{0u, 0u, 0u, 0u};
         last[m] = *reinterpret_cast<const raw_u32x4*>(x + (int64_t)(r0 + max(n - M + m, 0)) * g.xs);
       }
@@ -469,8 +475,8 @@ __global__ void __launch_bounds__(128) conv_run_kernel(ConvArgs g, T* __restrict
       }
 #pragma unroll
       for (int m = 0; m < M; ++m)
-        if (m < n) conv(in[m], live, out + (int64_t)(r0 + m) * C);
-      if (!live) return;
+        if (r0 + m < g.T) conv(in[m], live, its[m] ? out + (int64_t)(r0 + m) * C : nullptr);
+      if (!live || !moves) return;
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         raw_u32x4 v = last[m];
