@@ -28,8 +28,13 @@ GROUP_SCORES = {"top2": 0, "max": 1}
 # against 47.2 + 39.4 at 50 rows; 16 experts of 3584, 64 / 72 / 80 tokens (8 / 9 / 10 rows): 265 / 264, 268 / 266, 274 / 268.
 # Against the 64 x 64-tile kernel: 32 rows, 8 x [640, 1024] 8.3 / 22.5, 16 x [1408, 2048] 38 / 56; 24 and 32 rows, 8 x [14336, 4160]
 # 228 / 231 and 255 / 246
+# The average says nothing of the largest expert, whose weights go through once for every 64 rows: against the 256-tile kernel
+# the last quarter of the rows is taken only where an expert that half of the tokens choose (two each) still fits one pass, or
+# where that kernel's grid is smaller still (STREAM_FEW).  28 rows per expert, even / half of the tokens choose one: 16 x [2048, 1024],
+# four each, 20.2 / 22.5 streamed, 20.7 / 20.4 tiled; 16 x [2048, 1536], two each, 32.6 / 42.2, 32.3 / 35.3; 32 x [1024, 1024],
+# four each, 20.8 / 27.5, 22.3 / 22.1; 16 x [1024, 1024], four each, 12.2 / 15.2, 16.8 / 17.2; 8 x [4096, 2048] 39.4 / 43.2, 41.8 / 42.3
 STREAM_ROWS = 32
-STREAM_TILES = 192
+STREAM_TILES, STREAM_FEW, STREAM_ONE_PASS = 192, 64, 256
 # row tiles per band of the 256-tile kernel's walk: 16 experts, 300 / 500 / 1000 / 2500 / 4000 tokens, us: 6 307 327 380 531 751,
 # 8 318 347 402 540 759, 2 319 347 391 547 803, 16 slower than 8
 GROUP_BAND = 6
@@ -149,8 +154,12 @@ def stream_gemm_ok(a: torch.Tensor, w: torch.Tensor, R: int) -> bool:
     """Whether the weight-streaming kernel (csrc/mixers/grouped_stream.hip) takes
     R rows against w [E, N, K]: few rows per expert, whole pieces."""
     E, N, K = w.shape
-    few = E * (N // 256) < STREAM_TILES
-    most = STREAM_ROWS if few else STREAM_ROWS // 4 if tile_gemm_ok(a, w) else STREAM_ROWS * 3 // 4
+    tiles, fits = E * (N // 256), tile_gemm_ok(a, w)
+    most = STREAM_ROWS * 3 // 4
+    if tiles < STREAM_TILES and (not fits or tiles <= STREAM_FEW or R <= STREAM_ONE_PASS):
+        most = STREAM_ROWS
+    elif tiles >= STREAM_TILES and fits:
+        most = STREAM_ROWS // 4
     return (a.is_cuda and a.dtype == torch.bfloat16 and R <= most * E and a.stride(0) % 8 == 0 and
             a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and bool(_m().stream_grouped_ok(N, K)))
 

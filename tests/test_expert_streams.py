@@ -41,3 +41,14 @@ def test_rows_it_is_taken_for(E, N, K, most):
     w = torch.empty(1, device="cuda", dtype=torch.bfloat16).expand(E, N, K)
     for R, ok in ((most * E, True), (most * E + 1, False)):
         assert moe.stream_gemm_ok(torch.empty(R, K, device="cuda", dtype=torch.bfloat16), w, R) is ok
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,N,K,rows", [(16, 2048, 1024, 384), (16, 1024, 1024, 512), (32, 1024, 512, 768), (10, 3072, 1536, 256),
+                                        (16, 1408, 2048, 512), (16, 2048, 1088, 512)])
+def test_rows_it_is_taken_for_however_they_are_routed(E, N, K, rows):
+    """Against the 256-tile kernel more than 24 rows per expert only up to 256 in all or where that kernel's grid is small: beyond,
+    an expert that half of the tokens choose holds several passes.  (The last two that kernel does not take.)"""
+    w = torch.empty(1, device="cuda", dtype=torch.bfloat16).expand(E, N, K)
+    for R, ok in ((rows, True), (rows + 1, False)):
+        assert moe.stream_gemm_ok(torch.empty(R, K, device="cuda", dtype=torch.bfloat16), w, R) is ok
