@@ -24,7 +24,7 @@ int dxm_depth_mix(float*, float*, int64_t, int, const float*, const int64_t*, in
                   const void*, int64_t, const float*, int, int, hipStream_t);
 int dxm_linear_scan(int, float*, float*, int, const void*, int64_t, const void*, int64_t, const void*, int64_t, float,
                     float, int, const float*, const void*, int64_t, const float*, const float*, const float*, float,
-                    const int64_t*, const int*, const int*, int, int, int, int, int, int, hipStream_t);
+                    const int64_t*, const int*, const int*, int, int, int, int, int, int, int, hipStream_t);
 int dxm_norm_rope_cache(void*, int64_t, const int64_t*, const int64_t*, int, int, int, int, int, const float*,
                         const float*, float, const float*, int, void*, void*, int, int, int, hipStream_t);
 int dxm_gate_group_norm(void*, int64_t, const float*, const void*, int64_t, const float*, int, int, int, float, int,
@@ -46,7 +46,7 @@ int dxm_delta_chunk(float*, float*, int, float*, const void*, int64_t, const voi
 int64_t dxm_delta_prep_floats(int, int, int, const int*);
 int dxm_delta_rule(float*, float*, int, float*, const void*, int64_t, const void*, int64_t, const void*, int64_t, const void*,
                    int64_t, const void*, int64_t, const float*, const float*, float, float, const int64_t*, const int*,
-                   const int*, int, int, int, int, int, int, hipStream_t);
+                   const int*, int, int, int, int, int, int, int, hipStream_t);
 int dxm_conv_rope_cache(void*, const void*, int64_t, const float*, const float*, int, int, const void*, int, const int64_t*,
                         const int64_t*, const int*, const int*, const int*, int, int, int, int, int, int, const float*,
                         int, void*, void*, int, hipStream_t);
@@ -105,7 +105,7 @@ int dxm_decode_attention_ok(int, int, int, int, int, int, int, int, int);
 int dxm_decode_attention_parts(int, int, int, int, int);
 int dxm_decode_attention(void*, float*, const void*, int64_t, const void*, const void*, const int64_t*, const int*, const int*,
                          int, int, int, int, int, int, int, int, int, int, float, int, int, float, const float*, const float*,
-                         int, const float*, const void*, int64_t, int, const float*, int, int, hipStream_t);
+                         int, const float*, const void*, int64_t, int, const float*, int, int, int, hipStream_t);
 int dxm_merge_parts(void*, const float*, int64_t, int, const void*, int, void*, const float*, int64_t, int, const void*, int, int,
                     int64_t, int, int, const float*, int, hipStream_t);
 }
@@ -144,11 +144,11 @@ PYBIND11_MODULE(_C_mixers, m) {
   m.def("linear_scan", [](int mode, u out, u state, int n_slots, u q, int64_t qs, u k, int64_t ks, u v, int64_t vs,
                           float q_scale, float k_scale, int qk_rep, u decay, u gate, int64_t gs, u g_bias, u rate,
                           u skip, float inv_tau, u pos, u seq_rows, u slots, int n_seq, int T, int H, int dk, int dv,
-                          int f32, u st) {
+                          int f32, int layers, u st) {
     check(dxm_linear_scan(mode, F(out), F(state), n_slots, P(q), qs, P(k), ks, P(v), vs, q_scale, k_scale, qk_rep,
                           F(decay), P(gate), gs, F(g_bias), F(rate), F(skip), inv_tau,
                           reinterpret_cast<const int64_t*>(pos), reinterpret_cast<const int*>(seq_rows),
-                          reinterpret_cast<const int*>(slots), n_seq, T, H, dk, dv, f32, S(st)),
+                          reinterpret_cast<const int*>(slots), n_seq, T, H, dk, dv, f32, layers, S(st)),
           "linear_scan");
   });
   m.def("norm_rope_cache", [](u x, int64_t xs, u pos, u slots, int rows, int n_q, int n_k, int d, int v_w, u qw, u kw,
@@ -219,11 +219,11 @@ PYBIND11_MODULE(_C_mixers, m) {
         [](int T, int H, int dk, u seq_rows) { return dxm_delta_prep_floats(T, H, dk, reinterpret_cast<const int*>(seq_rows)); });
   m.def("delta_rule", [](u out, u state, int n_slots, u prep, u r, int64_t rs, u k, int64_t ks, u v, int64_t vs, u a,
                          int64_t as, u w, int64_t ws, u ab, u wb, float decay_scale, float key_eps, u pos, u seq_rows,
-                         u slots, int n_seq, int T, int H, int dk, int dv, int f32, u st) {
+                         u slots, int n_seq, int T, int H, int dk, int dv, int f32, int layers, u st) {
     check(dxm_delta_rule(F(out), F(state), n_slots, F(prep), P(r), rs, P(k), ks, P(v), vs, P(a), as, P(w), ws, F(ab), F(wb),
                          decay_scale, key_eps, reinterpret_cast<const int64_t*>(pos),
                          reinterpret_cast<const int*>(seq_rows), reinterpret_cast<const int*>(slots), n_seq, T, H, dk,
-                         dv, f32, S(st)),
+                         dv, f32, layers, S(st)),
           "delta_rule");
   });
   m.def("conv_rope_cache", [](u q, u x, int64_t xs, u cw, u cb, int silu, int taps, u tail, int n_slots, u pos, u kv_slots, u row_seq,
@@ -345,7 +345,7 @@ PYBIND11_MODULE(_C_mixers, m) {
                            int n_qh, int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask,
                            int size, float cap, u r1, u r2, int wfn, u hbias, u gate, int64_t gs, int keep, u sink,
                            int parts, int out_f32, u pre_out, u pre_ws, int pre_rows, int pre_parts, u pre_gate,
-                           int pre_whole, u st) {
+                           int pre_whole, int layers, u st) {
     // (pre: prompt rows in parts that are to be joined in the same launch)
     auto join = [&](int parts) {
       if (parts == 1 && !pre_rows) return;
@@ -361,7 +361,7 @@ PYBIND11_MODULE(_C_mixers, m) {
       check(dxm_decode_attention(P(out), F(ws), P(q), qs, P(kc), P(vc), reinterpret_cast<const int64_t*>(pos),
                                  reinterpret_cast<const int*>(seq), reinterpret_cast<const int*>(bt), bts, bs, rows, n_qh,
                                  maps, group, d, dv, Wk, Wv, scale, mask, size, cap, F(r1), F(r2), wfn, F(hbias), P(gate), gs,
-                                 keep, F(sink), parts, out_f32, S(st)),
+                                 keep, F(sink), parts, out_f32, layers, S(st)),
             "decode_attention");
       return join(parts);
     }

@@ -53,14 +53,16 @@ struct DecodeArgs {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-// A launch that reads more of the cache than this asks for it nontemporally: each line is read once, whole, and behind so many
-// no cache holds much of it for the next step.  Less is kept.  Each row takes the others to be as long as itself, which a
-// window's mostly are; other rows' lengths differ, so their line lies higher.  One layer's repeated launch, kept / not, us: plain
-// heads, 51 / 85 / 128 MB 20.0 / 21.1, 26.5 / 26.9, 37.3 / 33.6; capped, window 1024, 84 / 126 / 200 MB 27.5 / 27.8, 34.4 / 31.8,
-// 50.1 / 42.8; rows in chunks of 2048, the longest 131 of 67 MB 23.5 / 26.3.  Two launches of other layers: two maps, 190 MB
-// 97.4 / 86.5; plain heads, 300 MB 137 / 122 (5.0 TB/s).  A shared row (one cache for all heads) gains nothing: 46.9 / 48.2 and
-// 64.9 / 62.8 for two launches of 40 and 100 rows.
-constexpr int64_t kKeptWindow = 96 << 20, kKept = 160 << 20;
+// A launch that reads more of the cache than this asks for it nontemporally: each line is read once, whole, and behind so
+// many no cache holds much of it for the next step.  Less is kept.  Of a single layer that is repeated: each row takes the
+// others to be as long as itself, which a window's mostly are; other rows' lengths differ, so their line lies higher.  One
+// layer's repeated launch, kept / not, us: plain heads, 51 / 85 / 128 MB 20.0 / 21.1, 26.5 / 26.9, 37.3 / 33.6; capped,
+// window 1024, 84 / 126 / 200 MB 27.5 / 27.8, 34.4 / 31.8, 50.1 / 42.8; rows in chunks of 2048, the longest 131 of 67 MB
+// 23.5 / 26.3.  Two launches of other layers: two maps, 190 MB 97.4 / 86.5; plain heads, 300 MB 137 / 122 (5.0 TB/s).  In a
+// step of several layers nothing of one is left when it comes round again: eight layers, a layer, two maps, 62 / 89 MB 24.9
+// / 23.8, 28.6 / 27.3; capped, 64 / 85 MB 20.5 / 18.7, 26.3 / 24.1; plain heads, 65 / 120 MB 16.9 / 16.5, 24.7 / 22.8.  A
+// shared row (one cache for all heads) gains nothing: 46.9 / 48.2 and 64.9 / 62.8 for two launches of 40 and 100 rows.
+constexpr int64_t kKeptWindow = 96 << 20, kKept = 160 << 20, kKeptLayers = 48 << 20;
 constexpr int kTile = 32;       // keys per tile
 constexpr float kDefer = 8.f;   // log2 units that a score may exceed the running maximum by (weights are bf16 pairs)
 enum { kPlain = 0, kTerms = 1, kSigmoid = 2 };
@@ -509,7 +511,7 @@ int dxm_decode_attention(void* out, float* ws, const void* q, int64_t q_stride, 
                          const int64_t* pos, const int* seq, const int* bt, int bt_stride, int bs, int rows, int n_qh,
                          int maps, int group, int d, int dv, int Wk, int Wv, float scale, int mask, int size, float softcap,
                          const float* r1, const float* r2, int wfn, const float* hbias, const void* gate,
-                         int64_t gate_stride, int keep, const float* sink, int parts, int out_f32, hipStream_t st) {
+                         int64_t gate_stride, int keep, const float* sink, int parts, int out_f32, int layers, hipStream_t st) {
   if (rows <= 0) return 0;
   const bool same = kc == vc, terms = softcap > 0.f || r1;
   if (softcap < 0.f || (r1 && !r2) || wfn < 0 || wfn > 1 || keep < 0 || (keep && mask != 1)) return 6;
@@ -522,7 +524,7 @@ int dxm_decode_attention(void* out, float* ws, const void* q, int64_t q_stride, 
   // tiles a row may have at most (a window and the keys kept in front of it may each reach into two more), and of how many
   // rows still keep their lines
   const int64_t most = mask ? ((int64_t)size + keep) / kTile + 4 : (int64_t)bt_stride * bs / kTile;
-  const int64_t kept = (mask == 1 ? kKeptWindow : kKept) / (2 * kTile * ((int64_t)Wk + Wv) * rows);
+  const int64_t kept = (layers > 1 ? kKeptLayers : mask == 1 ? kKeptWindow : kKept) / (2 * kTile * ((int64_t)Wk + Wv) * rows);
   const bool many = most > kept;
   DecodeArgs a{out, ws, (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, pos, seq, bt, bt_stride,
                __builtin_ctz((unsigned)bs), n_qh, maps, group, Wk, Wv, scale, mask, size, parts, softcap, r1, r2, hbias,

@@ -20,6 +20,7 @@ struct DeltaArgs {
   int64_t as, wst;
   const float *a_bias, *w_bias;
   float decay_scale, key_eps;
+  int layers;  // of the step (state_once)
 };
 
 // u = k / sqrt(sum k^2 + key_eps), w = exp(-decay_scale sigmoid(wl + w_bias)), a u with a = sigmoid(al + a_bias); a wave

@@ -26,6 +26,7 @@ struct ScanArgs {
   int min_rows, max_rows;  // sequences with fewer / more rows in the step are another launch's
   int sorted;              // chunked kernels: workgroups take the sequences by length
   int all;                 // chunked kernels: sequences of fewer rows than min_rows too, token by token
+  int layers;              // of the step (state_once)
 };
 
 __device__ __forceinline__ float softplusf_(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }

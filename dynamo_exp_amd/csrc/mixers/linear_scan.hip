@@ -141,7 +141,7 @@ template <typename T, int R, int MODE, int ROWS = kRows>
 void launch_scan(const ScanArgs& g, int n_seq, hipStream_t st) {
   if constexpr (ROWS == kRows) {
     if (scan_fast_ok<T, R, MODE>(g)) {
-      auto kern = state_once(n_seq, g.H, g.dk, g.dv) ? scan_fast_kernel<T, R, MODE, true> : scan_fast_kernel<T, R, MODE, false>;
+      auto kern = state_once(n_seq, g.H, g.dk, g.dv, g.layers) ? scan_fast_kernel<T, R, MODE, true> : scan_fast_kernel<T, R, MODE, false>;
       hipLaunchKernelGGL(kern, dim3(n_seq, g.H, g.dv / (256 / R)), dim3(256), 0, st, g);
       return;
     }
@@ -170,7 +170,8 @@ extern "C" int dxm_linear_scan(int mode, float* out, float* state, int n_slots, 
                                int64_t ks, const void* v, int64_t vs, float q_scale, float k_scale, int qk_rep,
                                const float* decay, const void* gate, int64_t gs, const float* g_bias, const float* rate,
                                const float* skip, float inv_tau, const int64_t* pos, const int* seq_rows,
-                               const int* slots, int n_seq, int T_, int H, int dk, int dv, int f32, hipStream_t st) {
+                               const int* slots, int n_seq, int T_, int H, int dk, int dv, int f32, int layers,
+                               hipStream_t st) {
   if (n_seq <= 0 || T_ <= 0) return 0;
   if (H < 1 || dk < 1 || dv < 1 || n_slots < 1 || H > 65535 || (int64_t)T_ * H * dv > 0x7fffffffffffLL) return 1;
   if (dk > kMaxKey) return 2;  // wider keys need more rows per lane than instantiated
@@ -178,7 +179,7 @@ extern "C" int dxm_linear_scan(int mode, float* out, float* state, int n_slots, 
   if (!seq_rows && n_seq != T_) return 4;
   if (qk_rep < 1 || H % qk_rep) return 5;
   ScanArgs g{out, state, q, k, v, qs, ks, vs, q_scale, k_scale, qk_rep, decay, gate, gs, g_bias, rate, skip, inv_tau,
-             pos, seq_rows, slots, n_slots, T_, H, dk, dv, 1, 0x7fffffff, 0, 0};
+             pos, seq_rows, slots, n_slots, T_, H, dk, dv, 1, 0x7fffffff, 0, 0, layers};
   // prompt portions in bf16: matrix-core chunks where the sizes fit; shorter runs of a sequence
   // (decode tokens among them) stay with the token scan
   if (!f32 && seq_rows && n_seq <= 65535 && T_ >= kChunkMinRows + n_seq - 1 && chunk_scan_ok(mode, g)) {

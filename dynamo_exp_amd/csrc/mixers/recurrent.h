@@ -37,9 +37,13 @@ template <bool ONCE> __device__ __forceinline__ void store_state(float* p, f32x4
 }
 // One layer's repeated step, kept / not, us: state-space duality, 128 heads, 64 / 88 / 128 MB 33.8 / 39.7, 45.2 / 49.3, 67.7 / 59.8;
 // delta rule, 32 heads, 64 / 88 / 128 MB 29.2 / 33.4, 42.2 / 41.9, 66.5 / 55.2; gated linear attention 72 / 96 / 128 MB 39.1 / 40.2,
-// 52.3 / 49.0, 69.5 / 57.4.  (Steps of several layers gain from 44 MB a layer on, up to a fifth, and one that repeats a
-// single layer loses as much there.  Only read or only written nontemporally: nothing.)
-inline bool state_once(int n_seq, int H, int dk, int dv) { return (int64_t)n_seq * H * dk * dv * 4 >= 128 << 20; }
+// 52.3 / 49.0, 69.5 / 57.4.  Behind the states of other layers nothing of this one's is left when its next step comes, and
+// the line lies lower.  Eight layers with their other launches, a layer, kept / not, us: state-space duality 46 / 67 / 101 MB
+// 30.8 / 27.1, 40.7 / 36.1, 53.7 / 46.9; delta rule 46 / 84 / 126 MB 29.4 / 22.7, 43.0 / 36.2, 59.9 / 50.5; gated linear attention
+// 50 / 84 MB 30.4 / 26.5, 44.6 / 39.9; 24 layers of the smallest the same.  (Only read or only written nontemporally: nothing.)
+inline bool state_once(int n_seq, int H, int dk, int dv, int layers) {
+  return (int64_t)n_seq * H * dk * dv * 4 >= (layers > 1 ? 44 : 128) << 20;
+}
 
 template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));

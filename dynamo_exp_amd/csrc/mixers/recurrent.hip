@@ -91,8 +91,8 @@ __global__ void __launch_bounds__(NT) delta_rule_kernel(DeltaArgs g) {
 // state and formed while it is on its way, one or two of them by each wave, with delta_prep_kernel's arithmetic.
 // Bound by memory from some 40 sequences on, by latency below.  Two layers with their norms in a graph, 32 heads of 128 columns,
 // 1 / 3 / 12 / 40 / 128 sequences, us: 25 / 30 / 49 / 114 / 278 with delta_prep_kernel in front and the kernel for runs of
-// tokens, 21 / 21 / 33 / 89 / 231 like this; that kernel forming the rows itself 20 / 26 / 46 / 128 / 330, for it stages eight tokens.
-// With the state's lines not kept (ONCE, from 64 sequences on) 64 take 107 instead of 128.
+// tokens, 21 / 21 / 33 / 89 / 231 like this with the lines kept; that kernel forming the rows itself 20 / 26 / 46 / 128 / 330, for it
+// stages eight tokens.  With the state's lines not kept (ONCE: state_once) 64 take 107 instead of 128.
 constexpr int kDeltaStepLanes = 8;
 bool delta_forms_itself(const int* seq_rows, int dk) { return !seq_rows && dk == kDeltaStepLanes * kRows; }
 
@@ -176,7 +176,7 @@ void launch_delta_ct(const DeltaArgs& g, int n_seq, hipStream_t st) {
   if constexpr (R == kDeltaStepLanes) {
     if (!g.prep) {
       constexpr int cols = 256 / R * CT;
-      auto kern = state_once(n_seq, g.H, g.dk, g.dv) ? delta_step_kernel<T, CT, true> : delta_step_kernel<T, CT, false>;
+      auto kern = state_once(n_seq, g.H, g.dk, g.dv, g.layers) ? delta_step_kernel<T, CT, true> : delta_step_kernel<T, CT, false>;
       hipLaunchKernelGGL(kern, dim3(n_seq, g.H, (g.dv + cols - 1) / cols), dim3(256), 0, st, g);
       return;
     }
@@ -879,7 +879,7 @@ int64_t dxm_delta_prep_floats(int T_, int H, int dk, const int* seq_rows) {
 int dxm_delta_rule(float* out, float* state, int n_slots, float* prep, const void* r, int64_t rs, const void* k,
                    int64_t ks, const void* v, int64_t vs, const void* a, int64_t as, const void* w, int64_t ws,
                    const float* a_bias, const float* w_bias, float decay_scale, float key_eps, const int64_t* pos,
-                   const int* seq_rows, const int* slots, int n_seq, int T_, int H, int dk, int dv, int f32,
+                   const int* seq_rows, const int* slots, int n_seq, int T_, int H, int dk, int dv, int f32, int layers,
                    hipStream_t st) {
   if (n_seq <= 0 || T_ <= 0) return 0;
   if (H < 1 || dk < 1 || dv < 1 || n_slots < 1 || H > 65535 || n_seq > 0x7fffffff || (int64_t)T_ * H > 0x7fffffff)
@@ -894,7 +894,7 @@ int dxm_delta_rule(float* out, float* state, int n_slots, float* prep, const voi
   DeltaArgs g{};
   g.out = out, g.state = state, g.r = r, g.k = k, g.v = v, g.rs = rs, g.ks = ks, g.vs = vs, g.prep = self ? nullptr : prep;
   g.a = a, g.w = w, g.as = as, g.wst = ws, g.a_bias = a_bias, g.w_bias = w_bias;
-  g.decay_scale = decay_scale, g.key_eps = key_eps;
+  g.decay_scale = decay_scale, g.key_eps = key_eps, g.layers = layers;
   g.pos = pos, g.seq_rows = seq_rows, g.slots = slots, g.n_slots = n_slots, g.T = T_, g.H = H, g.dk = dk, g.dv = dv;
   const int need = (dk + kRows - 1) / kRows;
   if (need <= 4) { DISPATCH_T(f32, (launch_delta<T, 4>(g, n_seq, st))); }

@@ -295,7 +295,7 @@ class BekulixForCausalLM:
             mx.headprep_cache(p, pos, slots, H, G, d, H * d, L["qn"], L["kn"], eps,
                               (qt["coef"], qt["every"]) if qt else None, kc, vc, v_mode=1)
             a = mx.attention(p, kc, vc, pos, seq, tables, bs, H, 1, H // G, d, d, m["scale"], "causal", 0,
-                             self._parts(T, H, "causal", 0, meta, H // G), False, *tl)
+                             self._parts(T, H, "causal", 0, meta, H // G), False, *tl, layers=len(self.layers))
             return torch.matmul(a.view(T, H * d), L["w_o"].t())
         if L["type"] == "latent_attention":
             r, dv = m["kv_rank"], m["vdim"]
@@ -315,7 +315,7 @@ class BekulixForCausalLM:
         mx.headprep_cache(p, pos, slots, 0, 2 * G, d, qw, None, None, eps, None, kc, vc, v_mode=2, v_off=qw + kw,
                           v_w=G * dv)
         a = mx.attention(p, kc, vc, pos, seq, tables, bs, 2 * H, 2, H // G, d, dv, m["scale"], mask, size,
-                         self._parts(T, 2 * H, mask, size, meta, H // G), True, *tl)
+                         self._parts(T, 2 * H, mask, size, meta, H // G), True, *tl, layers=len(self.layers))
         o = mx.diff_combine(a.view(T, H, 2, dv), L["lam"], 1.0 - float(m["diff"]), eps, self.dtype)
         return torch.matmul(o, L["w_o"].t())
 

@@ -300,7 +300,7 @@ class BolinexForCausalLM:
         tl = (meta.row_tiles, meta.num_prefill_tokens) if meta.is_prefill else (None, 0)
         a = mx.attention(p, kc, vc, meta.positions, seq, tables, bs, H, 1, H // G, d, dv, m["scale"],
                          "window" if size else "causal", size, self._parts(T, H, H // G, size, meta), False, *tl,
-                         softcap=float(m.get("softcap") or 0.0), dist_bias=L["bias"])
+                         softcap=float(m.get("softcap") or 0.0), dist_bias=L["bias"], layers=len(self.layers))
         a = mx.act_mul(p[:, g_off:g_off + H * dv], a.view(T, H * dv), "sigmoid")
         return self._mm(a, L["w_o"])
 

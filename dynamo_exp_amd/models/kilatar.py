@@ -303,7 +303,8 @@ class KilatarForCausalLM(StatefulLayeredModel):
                              meta.row_seq if meta.is_prefill else None, meta.seq_rows, meta.state_slots, bias=L["conv_b"],
                              act="silu")
         y = rc.ssd(xbc[:, :inner], xbc[:, inner:inner + G * N], xbc[:, inner + G * N:], p[:, t0:t0 + Hs], L["dt_bias"],
-                   L["rate"], L["skip"], state, meta.positions, meta.seq_rows, meta.state_slots, Hs, G, N, P)
+                   L["rate"], L["skip"], state, meta.positions, meta.seq_rows, meta.state_slots, Hs, G, N, P,
+                   layers=len(self.layers))
         rc.gate_group_norm(y, p[:, :inner], L["gn"], m["norm_groups"], self.cfg.rms_norm_eps, self.dtype, out=o)
 
     def _parallel(self, L: dict, p: torch.Tensor, meta: AttnMeta, kc, vc, state, seq, tables) -> dict:
@@ -319,9 +320,10 @@ class KilatarForCausalLM(StatefulLayeredModel):
         size = int((a.get("mask") or {}).get("size") or 0)
         tl = (meta.row_tiles, meta.num_prefill_tokens) if meta.is_prefill else (None, 0)
         y = mx.attention(p, kc, vc, meta.positions, seq, tables, meta.block_size, H, 1, H // G, d, dv, a["scale"],
-                         "chunk" if size else "causal", size, self._parts(T, H, H // G, size, meta), False, *tl)
+                         "chunk" if size else "causal", size, self._parts(T, H, H // G, size, meta), False, *tl,
+                         layers=len(self.layers))
         o = rc.retention(p[:, r0:r0 + n], p[:, r0 + n:r0 + 2 * n], p[:, r0 + 2 * n:r0 + 2 * n + nv], L["decay"], 1.0, state,
-                         meta.positions, meta.seq_rows, meta.state_slots, Hr, dk, dvr)
+                         meta.positions, meta.seq_rows, meta.state_slots, Hr, dk, dvr, layers=len(self.layers))
         g0 = r0 + 2 * n + nv
         o = rc.head_norm_gate(o, 1, L["hn"], p[:, g0:g0 + nv], self.cfg.rms_norm_eps, self.dtype)  # all heads together
         return dict(c=self._mm(y.view(T, H * dv), L["w_lo"]), c_w=L["lw"], d=self._mm(o, L["w_ro"]), d_w=L["rw"])

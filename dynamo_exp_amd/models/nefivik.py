@@ -349,7 +349,7 @@ class NefivikForCausalLM:
         p = self._mm(h, L["w_in"])  # [r | k | v | g | a | rg1 | w1]
         wl = self._mm(mx.act_mul(p[:, 5 * n + W:5 * n + W + L["lora"]], None, "tanh"), L["w_w2"])
         o = rc.delta_rule(p[:, :n], p[:, n:2 * n], p[:, 2 * n:3 * n], p[:, 4 * n:5 * n], wl, L["a_b"], L["w0"], state,
-                          meta.positions, meta.seq_rows, meta.state_slots, H, d, d)
+                          meta.positions, meta.seq_rows, meta.state_slots, H, d, d, layers=len(self.layers))
         o = rc.head_norm_gate(o, H, L["hnorm"], p[:, 3 * n:4 * n], self.cfg.rms_norm_eps, self.dtype)
         return self._mm(o, L["w_o"]), p[:, 5 * n:5 * n + W]
 
@@ -367,7 +367,7 @@ class NefivikForCausalLM:
         tl = (meta.row_tiles, meta.num_prefill_tokens) if meta.is_prefill else (None, 0)
         a = mx.attention(q, kc, vc, meta.positions, seq, tables, bs, H, 1, H // G, d, dv, m["scale"],
                          "window" if size else "causal", size, self._parts(T, H, H // G, size, meta), False, *tl,
-                         weights="sigmoid", head_bias=L["pb"], head_gate=p[:, C + W:C + W + H])
+                         weights="sigmoid", head_bias=L["pb"], head_gate=p[:, C + W:C + W + H], layers=len(self.layers))
         return self._mm(a.view(T, H * dv), L["w_o"]), p[:, C:C + W]
 
     def _ff(self, L: dict, h: torch.Tensor) -> torch.Tensor:

@@ -231,13 +231,15 @@ class PovuraxForCausalLM(StatefulLayeredModel):
                            kc, vc)
         tl = (meta.row_tiles, meta.num_prefill_tokens) if meta.is_prefill else (None, 0)
         y = mx.attention(p, kc, vc, meta.positions, seq, tables, bs, H, 1, H // G, d, dv, a["scale"], "causal", 0,
-                         self._parts(T, H, H // G, 0, meta), False, *tl, fine_weights=True)
+                         self._parts(T, H, H // G, 0, meta), False, *tl, fine_weights=True,
+                         layers=len(self.layers))
         mx.act_mul(p[:, g0:z0], y.view(T, nv), "sigmoid", out=o[:, :nv], scale=L["left_scale"])
         # right: state-space mixer
         xbc = rc.causal_conv(p[:, c0:c0 + C], L["conv_w"], tail, meta.positions, meta.row_seq if meta.is_prefill else None,
                              meta.seq_rows, meta.state_slots, bias=L["conv_b"], act="silu")
         y = rc.ssd(xbc[:, :inner], xbc[:, inner:inner + Gs * N], xbc[:, inner + Gs * N:], p[:, c0 + C:c0 + C + Hs],
-                   L["dt_bias"], L["rate"], L["skip"], state, meta.positions, meta.seq_rows, meta.state_slots, Hs, Gs, N, P)
+                   L["dt_bias"], L["rate"], L["skip"], state, meta.positions, meta.seq_rows, meta.state_slots, Hs, Gs, N, P,
+                   layers=len(self.layers))
         rc.gate_group_norm(y, p[:, z0:c0], L["gn"], b["norm_groups"], eps, self.dtype, out=o[:, nv:])
         return self._mm(o, L["w_o"])
 
@@ -249,7 +251,7 @@ class PovuraxForCausalLM(StatefulLayeredModel):
         g0 = 2 * n + nv
         z = self._mm(p[:, g0 + nv:g0 + nv + L["lora"]], L["w_a2"])
         o = rc.gated_linear_attention(p[:, :n], p[:, n:2 * n], p[:, 2 * n:g0], z, L["a_b"], float(m["tau"]), d ** -0.5, state,
-                                      meta.positions, meta.seq_rows, meta.state_slots, H, d, dv)
+                                      meta.positions, meta.seq_rows, meta.state_slots, H, d, dv, layers=len(self.layers))
         o = rc.head_norm_gate(o, H, L["hnorm"], p[:, g0:g0 + nv], self.cfg.rms_norm_eps, self.dtype, gate_act="silu")
         return self._mm(o, L["w_o"])
 

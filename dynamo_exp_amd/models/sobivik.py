@@ -386,7 +386,8 @@ class SobivikForCausalLM:
         mask, size, keep = self._mask(m)
         tl = (meta.row_tiles, meta.num_prefill_tokens) if meta.is_prefill else (None, 0)
         a = mx.attention(p, kc, vc, meta.positions, seq, tables, bs, 2 * H, 2, H // G, d, dv, m["scale"], mask, size,
-                         self._parts(T, 2 * H, H // G, size + keep if size else 0, meta), True, *tl, keep_first=keep)
+                         self._parts(T, 2 * H, H // G, size + keep if size else 0, meta), True, *tl, keep_first=keep,
+                         layers=len(self.layers))
         g0 = nq + nk + G * dv
         o = mx.diff_combine(a.view(T, H, 2, dv), L["lam"], 1.0 - float(m["diff"]), self.cfg.rms_norm_eps, self.dtype,
                             head_gate=p[:, g0:g0 + H])
@@ -398,7 +399,7 @@ class SobivikForCausalLM:
         n, nv = H * d, H * dv
         p = self._mm(h, L["w_in"])  # [q | k | v | g]
         o = rc.retention(p[:, :n], p[:, n:2 * n], p[:, 2 * n:2 * n + nv], L["decay"], d ** -0.5, state, meta.positions,
-                         meta.seq_rows, meta.state_slots, H, d, dv)
+                         meta.seq_rows, meta.state_slots, H, d, dv, layers=len(self.layers))
         o = rc.head_norm_gate(o, H, None, p[:, 2 * n + nv:2 * n + 2 * nv], self.cfg.rms_norm_eps, self.dtype,
                               gate_act="silu")
         return self._mm(o, L["w_o"])

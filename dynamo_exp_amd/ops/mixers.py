@@ -563,14 +563,16 @@ def attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, positions: to
               out_f32: bool = False, tiles: torch.Tensor | None = None, n_tile_rows: int = 0, softcap: float = 0.0,
               dist_bias: tuple[torch.Tensor, torch.Tensor] | None = None, weights: str = "softmax",
               head_bias: torch.Tensor | None = None, head_gate: torch.Tensor | None = None, keep_first: int = 0,
-              sink: torch.Tensor | None = None, fine_weights: bool = False) -> torch.Tensor:
+              sink: torch.Tensor | None = None, fine_weights: bool = False, layers: int = 1) -> torch.Tensor:
     """Attention of one step's rows: the first n_tile_rows rows (prompt chunks,
     cut into `tiles` [n, 2] = first row, row count) on the matrix-core prefill
     kernel where it applies, all other rows (decode tokens; every row when it
     does not apply) on the row kernel.  Same arguments and result as
     row_attention.  fine_weights: prompt rows' softmax weights enter the product with the
     values as the sum of two bf16 numbers also where the result is bf16 (decode rows'
-    always do)."""
+    always do).  layers: how many layers the step goes through before it comes back to
+    these caches (with several, less of them is still in a cache of the chip's; only how
+    decode rows' lines are read depends on it)."""
     T = q.shape[0]
     if not tile_attention_ok(q, d, dv) or not scale > 0:  # the matrix-core kernels fold a positive scale
         return row_attention(q, kc, vc, positions, seq, block_tables, block_size, n_qh, maps, group, d, dv, scale,
@@ -622,7 +624,7 @@ def attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, positions: to
                           q.data_ptr() + r0 * q.stride(0) * q.element_size(), q.stride(0), kc.data_ptr(), vc.data_ptr(),
                           positions.data_ptr() + r0 * 8 * positions.stride(0), seq.data_ptr() + r0 * 4 * seq.stride(0) if seq is not None else 0,
                           *common, n_dec, *heads, head_gate.data_ptr() + r0 * gs * head_gate.element_size() if head_gate is not None else 0,
-                          gs, int(keep_first), _ptr(sink), parts, int(out_f32), *pre, _stream())
+                          gs, int(keep_first), _ptr(sink), parts, int(out_f32), *pre, layers, _stream())
     return out
 
 

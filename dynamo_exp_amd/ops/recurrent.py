@@ -296,7 +296,7 @@ DELTA_DECAY_SCALE = math.exp(-0.5)
 def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                a_bias: torch.Tensor | None, w_bias: torch.Tensor | None, state: torch.Tensor, positions: torch.Tensor,
                seq_rows: torch.Tensor | None, state_slots: torch.Tensor, n_heads: int, dk: int, dv: int,
-               decay_scale: float = DELTA_DECAY_SCALE, key_eps: float = 1e-6) -> torch.Tensor:
+               decay_scale: float = DELTA_DECAY_SCALE, key_eps: float = 1e-6, layers: int = 1) -> torch.Tensor:
     """The generalized delta rule over the rows of a step, per sequence and head
     from the sequence's state S [dk, dv] (fp32; stored column by column,
     state [slots, H, dv, dk] with state[s, h, j, i] = S[i, j], so that the
@@ -310,7 +310,9 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tenso
     r, k, a, w [T, H dk] and v [T, H dv] are column sections (contiguous rows,
     any row stride) of projection outputs.  Returns o [T, H dv] fp32.
     Everything but reading the inputs is fp32.  How a sequence's rows are summed
-    depends on their number alone, not on what else the step holds."""
+    depends on their number alone, not on what else the step holds.  layers: how many
+    layers the step goes through before it comes back to this state (with several, less
+    of it is still in a cache of the chip's; only how it is read depends on that)."""
     T = r.shape[0]
     n_seq = state_slots.numel()
     _fp32_param(a_bias, "a_bias")
@@ -356,7 +358,7 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tenso
             return out
     # unit key, decay and removal rate * unit key of every row, where a pass of its own forms them in front of the scan
     prep = torch.empty(_m().delta_prep_floats(T, n_heads, dk, _ptr(seq_rows)), dtype=torch.float32, device=r.device)
-    _m().delta_rule(out.data_ptr(), state.data_ptr(), state.shape[0], prep.data_ptr(), *rows, dk, dv, _f32(r), _stream())
+    _m().delta_rule(out.data_ptr(), state.data_ptr(), state.shape[0], prep.data_ptr(), *rows, dk, dv, _f32(r), layers, _stream())
     return out
 
 
@@ -365,7 +367,7 @@ SCAN_MODES = {"fixed": 0, "step": 1, "channel": 2}
 
 def _linear_scan(mode: str, q, k, v, state, positions, seq_rows, state_slots, n_heads: int, dk: int, dv: int,
                  q_scale: float = 1.0, k_scale: float = 1.0, qk_heads: int | None = None, decay=None, gate=None,
-                 g_bias=None, rate=None, skip=None, tau: float = 1.0) -> torch.Tensor:
+                 g_bias=None, rate=None, skip=None, tau: float = 1.0, layers: int = 1) -> torch.Tensor:
     """S_t = D_t S_(t-1) + (k_scale k_t) (u_t v_t)^T,  o_t = S_t^T (q_scale q_t) + skip[h] v_t, with D_t and
     u_t by mode (csrc/mixers/linear_scan.hip); head h reads q / k head h // (n_heads / qk_heads)."""
     T, H, n_seq = q.shape[0], n_heads, state_slots.numel()
@@ -419,13 +421,13 @@ def _linear_scan(mode: str, q, k, v, state, positions, seq_rows, state_slots, n_
                      k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), float(q_scale), float(k_scale), H // G,
                      _ptr(decay), _ptr(gate), gate.stride(0) if gate is not None else 0, _ptr(g_bias), _ptr(rate),
                      _ptr(skip), 1.0 / float(tau), positions.data_ptr(), _ptr(seq_rows), state_slots.data_ptr(), n_seq, T,
-                     H, dk, dv, _f32(q), _stream())
+                     H, dk, dv, _f32(q), layers, _stream())
     return out
 
 
 def retention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, k_scale: float,
               state: torch.Tensor, positions: torch.Tensor, seq_rows: torch.Tensor | None, state_slots: torch.Tensor,
-              n_heads: int, dk: int, dv: int) -> torch.Tensor:
+              n_heads: int, dk: int, dv: int, layers: int = 1) -> torch.Tensor:
     """Retention (linear attention with a fixed decay per head, no softmax and
     no denominator) over the rows of a step, per sequence and head from the
     sequence's state S [dk, dv] (fp32; stored column by column, state
@@ -433,38 +435,39 @@ def retention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Te
         S_t = decay[h] S_(t-1) + (k_scale k_t) v_t^T,     o_t = S_t^T q_t.
     q, k [T, H dk] and v [T, H dv] are column sections (contiguous rows, any
     row stride) of projection outputs; decay fp32 [H].  Returns o [T, H dv]
-    fp32.  Everything but reading the inputs is fp32."""
+    fp32.  Everything but reading the inputs is fp32.  layers: as for delta_rule."""
     return _linear_scan("fixed", q, k, v, state, positions, seq_rows, state_slots, n_heads, dk, dv, k_scale=k_scale,
-                        decay=decay)
+                        decay=decay, layers=layers)
 
 
 def ssd(x: torch.Tensor, B: torch.Tensor, C: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor | None,
         rate: torch.Tensor, skip: torch.Tensor | None, state: torch.Tensor, positions: torch.Tensor,
         seq_rows: torch.Tensor | None, state_slots: torch.Tensor, n_heads: int, n_groups: int, N: int,
-        P: int) -> torch.Tensor:
+        P: int, layers: int = 1) -> torch.Tensor:
     """State-space duality (Mamba-2's recurrence) over the rows of a step, per
     sequence and head from the sequence's state S [N, P] (fp32, stored as for
     retention: [slots, H, P, N]; updated in place), with the step size
     u_t = softplus(dt_t + dt_bias[h]):
         S_t = exp(-rate[h] u_t) S_(t-1) + u_t B_t x_t^T,     y_t = S_t^T C_t + skip[h] x_t.
     x [T, H P]; B, C [T, n_groups N] shared by H / n_groups heads each; dt [T, H]
-    -- column sections, any row stride.  Returns y [T, H P] fp32."""
+    -- column sections, any row stride.  Returns y [T, H P] fp32.  layers: as for delta_rule."""
     return _linear_scan("step", C, B, x, state, positions, seq_rows, state_slots, n_heads, N, P, qk_heads=n_groups,
-                        gate=dt, g_bias=dt_bias, rate=rate, skip=skip)
+                        gate=dt, g_bias=dt_bias, rate=rate, skip=skip, layers=layers)
 
 
 def gated_linear_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor,
                            z_bias: torch.Tensor | None, tau: float, q_scale: float, state: torch.Tensor,
                            positions: torch.Tensor, seq_rows: torch.Tensor | None, state_slots: torch.Tensor,
-                           n_heads: int, dk: int, dv: int) -> torch.Tensor:
+                           n_heads: int, dk: int, dv: int, layers: int = 1) -> torch.Tensor:
     """Gated linear attention over the rows of a step, per sequence and head
     from the sequence's state S [dk, dv] (fp32, stored as for retention; updated
     in place), with a decay per key channel and token, alpha_t =
     sigmoid(z_t + z_bias)^(1 / tau):
         S_t = diag(alpha_t) S_(t-1) + k_t v_t^T,     o_t = S_t^T (q_scale q_t).
-    q, k, z [T, H dk] and v [T, H dv] are column sections.  Returns o [T, H dv] fp32."""
+    q, k, z [T, H dk] and v [T, H dv] are column sections.  Returns o [T, H dv] fp32.
+    layers: as for delta_rule."""
     return _linear_scan("channel", q, k, v, state, positions, seq_rows, state_slots, n_heads, dk, dv, q_scale=q_scale,
-                        gate=z, g_bias=z_bias, tau=tau)
+                        gate=z, g_bias=z_bias, tau=tau, layers=layers)
 
 
 GATE_ACTS = {"sigmoid": 0, "silu": 1}

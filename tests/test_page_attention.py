@@ -537,3 +537,25 @@ def test_decode_rows_that_read_much(form, mask, size, keep):
         got = run(0, n)
         for i in (0, 8, n // 2, n - 8):
             assert bool((got[i:i + 8] == run(i, i + 8)).all()), (n, i)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 1000, 40), ("chunk", 1500, 0)])
+@pytest.mark.parametrize("form", ["plain", "capped", "sigmoid", "diff", "shared"])
+def test_decode_rows_of_a_step_of_several_layers(form, mask, size, keep):
+    """Rows on both sides of the line that holds where a step goes through several layers (48 MB), below one layer's."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(43)
+    cap, db, sig, hb, sink = terms(form, n_qh)
+    lengths, bs = [2000, 33, 96, 1350, 1, 700], 32
+    kd, vd, table, _ = pages(form, lengths, bs)
+    for n in (30 if form == "diff" else 60, 3):
+        seq = torch.arange(n, dtype=torch.int32) % len(lengths)
+        pos = torch.tensor(lengths)[seq.long()] - 1
+        q, pos, seq = torch.randn(n, n_qh * d).bfloat16().cuda(), pos.cuda(), seq.cuda()
+
+        def run(**kw):
+            return mx.attention(q, kd, vd, pos, seq, table, bs, n_qh, maps, group, d, dv, 0.7 * d ** -0.5, mask, size, 2, True,
+                                softcap=cap, weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), keep_first=keep,
+                                sink=cuda(sink), **kw)
+        assert bool((run(layers=24) == run()).all()), n
