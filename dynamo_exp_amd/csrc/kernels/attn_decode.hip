@@ -115,7 +115,7 @@ __device__ __forceinline__ void finish_workgroup(const float* so, const float* s
       sl_sum += f * sl[s2 * G + h];
     }
     const int qh = kvh * G + h;
-    const float val = sl_sum > 0.f ? so_sum / sl_sum * out_scale : 0.f;
+    const float val = sl_sum != 0.f ? so_sum / sl_sum * out_scale : 0.f;  // (no key: 0; a NaN stays one)
     if (single) {
       out[((int64_t)b * n_q_heads + qh) * D + d] = f32_to_bf16(val);
     } else {
@@ -708,7 +708,7 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
   if (grp) return;
   num += other[threadIdx.x];
   u32x2_a2 pk = {0u, 0u};
-  if (den > 0.f) pk = u32x2_a2{pack_bf16x2(num[0] / den, num[1] / den), pack_bf16x2(num[2] / den, num[3] / den)};
+  if (den != 0.f) pk = u32x2_a2{pack_bf16x2(num[0] / den, num[1] / den), pack_bf16x2(num[2] / den, num[3] / den)};
   *reinterpret_cast<u32x2_a2*>(o) = pk;
 }
 

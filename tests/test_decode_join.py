@@ -39,3 +39,24 @@ def test_parts(ctx, n_parts):
     # bf16 weights (2^-9 each, of values of order one) and one rounding of the result
     err = (got[live].float() - want.float()).abs().max()
     assert float(err) < 2 ** -7 * max(1.0, float(want.float().abs().max())), float(err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at", [0, 700, 1999])
+@pytest.mark.parametrize("n_parts", [1, 2, 16, 70])
+@pytest.mark.parametrize("mfma", ["0", "1"])
+def test_rows_that_see_a_nan(monkeypatch, mfma, n_parts, at):
+    """A key that holds a NaN, in the first, a middle and the last part: the query heads of its key head are NaN, not 0."""
+    monkeypatch.setenv("DX_DECODE_MFMA", mfma)
+    torch.manual_seed(n_parts)
+    hq, hkv, bs, lens = 8, 2, 16, torch.tensor([2000, 300], dtype=torch.int32)
+    table = torch.arange(2 * 125, dtype=torch.int32).view(2, 125)
+    kc, vc = (torch.randn(250, hkv, bs, 128).bfloat16() for _ in range(2))
+    q, scale = torch.randn(2, hq, 128).bfloat16(), 1 / math.sqrt(128)
+    want = ref.paged_attention(q, kc, vc, table, torch.arange(3, dtype=torch.int32), lens, scale, bs)
+    kc[at // bs, 1, at % bs, 3] = float("nan")
+    out = torch.empty(2, hq, 128, dtype=torch.bfloat16, device="cuda")
+    got = ops.decode_attention(q.cuda(), kc.cuda(), vc.cuda(), table.cuda(), lens.cuda(), scale, out, n_parts).cpu()
+    assert bool(got[0, 4:].isnan().all())
+    for g, w in ((got[0, :4], want[0, :4]), (got[1], want[1])):  # (bound of test_parts)
+        assert float((g.float() - w.float()).abs().max()) < 2 ** -7 * max(1.0, float(want.float().abs().max()))
