@@ -92,6 +92,22 @@ def test_sequences_by_length(rows, kind, H, dk, dv):
     assert bool((o.cpu()[want.abs().sum((1, 2)) == 0] == 0).all())
 
 
+MANY = [n for i in range(26) for n in (33 + i % 7 * 9, (1, 0, 3, 7)[i % 4])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [MANY, MANY + [1, 2] * 6, MANY + [1, 2] * 6 + [200]], ids=len)
+@pytest.mark.parametrize("kind,H,dk,dv", [("retention", 32, 128, 128), ("ssd", 64, 128, 64), ("gla", 32, 128, 128),
+                                          ("retention", 24, 32, 128)])
+def test_short_sequences_behind_many(rows, kind, H, dk, dv):
+    """Short sequences in the launch of more long ones than are put in order, of 64 in all and of more than a wave compares:
+    each goes through once (one left out, or taken twice, is a hundredth of the results)."""
+    assert H * (dv // 64) * min(len(rows), sum(rows) // 128) > 256 and H * (dv // 64) * len(rows) <= 8192  # launch_chunk_scan's rules
+    eo, es, o, want = scan(kind, rows, H, dk, dv)
+    assert eo < 2.0 ** -16 and es < 2.0 ** -16, (eo, es)  # (test_chunks)
+    assert bool((o.cpu()[want.abs().sum((1, 2)) == 0] == 0).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("stride", [0, 8, 64])
 @pytest.mark.parametrize("kind", ["retention", "ssd", "gla"])

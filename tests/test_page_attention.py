@@ -383,9 +383,34 @@ def test_scores_and_caps_at_the_ends_of_the_number_range(form, cap):
     assert torch.equal(got.cpu().double(), want)
 
 
+CUT_AT_500 = ("capped", "penalty", "both", "diff pair", "shared wide", "shared pair")
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_rule_of_prompt_parts(form):
+    """The keys that a row sees decide, not the context: a window's and those behind the start of a chunk, of which rows that reach
+    back over it see a whole one; many rows are not cut."""
+    n_qh, maps, group, d, dv = FORMS[form]
+
+    def cut(rows, tiles, keys, mask="causal", size=0, keep=0, heads=n_qh):
+        return mx._prompt_parts(rows, tiles, keys, mask, size, keep, heads, maps, heads // maps if form.startswith("shared") else group,
+                                d, dv, 64, form.startswith("shared"), form in ("capped", "penalty", "both", "sigmoid capped"),
+                                int(form.startswith("sigmoid")), form.startswith("diff"), form == "fine")[0] > 1
+
+    assert cut(88, 3, 1088) and not cut(16, 1, 128) and not cut(1024, 8, 100000, heads=64 * n_qh)
+    for size in (900, 2000):
+        assert cut(88, 3, 100000, "window", size, 70)
+    assert cut(88, 3, 100000, "window", 300, 70) == (form in CUT_AT_500) == cut(88, 3, 498)
+    assert not cut(16, 1, 100000, "window", 100)
+    for keys, seen in ((999, True), (1000, True), (1001, True), (1016, True), (1017, False), (1100, False), (1990, True), (2000, True),
+                       (2016, True), (2017, False)):
+        assert cut(16, 1, keys, "chunk", 1000) == seen, keys
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("parts", [None, (2, 0), (3, 0), (8, 0), (4, 200)])
-@pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 300, 70), ("chunk", 500, 0)])
+@pytest.mark.parametrize("mask,size,keep", [("causal", 0, 0), ("window", 300, 70), ("chunk", 500, 0), ("window", 900, 70),
+                                            ("chunk", 1000, 0)])
 @pytest.mark.parametrize("form", FORMS)
 def test_prompt_rows_in_parts(monkeypatch, form, mask, size, keep, parts):
     """Few prompt rows behind long contexts, their keys cut into parts (None: as many as the rule takes): parts without a
@@ -408,7 +433,7 @@ def test_prompt_rows_in_parts(monkeypatch, form, mask, size, keep, parts):
         want = want * torch.sigmoid(gate.double()).repeat_interleave(maps, 1)[:, :, None]
     if parts:
         monkeypatch.setattr(mx, "_prompt_parts", lambda *a: parts)
-    else:  # the rule cuts these sizes
+    else:
         rule, seen = mx._prompt_parts, []
         monkeypatch.setattr(mx, "_prompt_parts", lambda *a: seen.append(rule(*a)) or seen[-1])
     pos = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows)]).cuda()
@@ -419,8 +444,8 @@ def test_prompt_rows_in_parts(monkeypatch, form, mask, size, keep, parts):
                        sum(rows), softcap=cap, dist_bias=None if db is None else tuple(map(cuda, db)),
                        weights="sigmoid" if sig else "softmax", head_bias=cuda(hb), head_gate=cuda(gate), keep_first=keep,
                        sink=cuda(sink), fine_weights=form == "fine").cpu().double()
-    if not parts and mask == "causal":
-        assert seen[0][0] > 1
+    if not parts:  # (the rule: 500 keys are cut only where a key takes longest)
+        assert (seen[0][0] > 1) == (mask == "causal" or size > 500 or form in CUT_AT_500)
     err, top = float((got - want).abs().max()), float(want.abs().max())
     # (as in test_prompt_rows: the parts are joined in fp32)
     assert err < (3e-4 if out_f32 else 2.0 ** -8 * (top + (top if sig else 5.0))), err
