@@ -13,7 +13,7 @@
 // by a tenth, eight or sixteen waves by 6 to 50 %): HBM likes the few long runs of lines better.
 //
 // Bound by HBM.  A line is read by two loads, 16 bytes of each lane's 32 at a time, so the lines have to stay:
-// as nontemporal loads (before) part of them came from memory twice.  16 experts of 3584, 24 tokens, gate-up /
+// as nontemporal loads (before, and for steps of one or two rows) part of them come from memory twice.  16 experts of 3584, 24 tokens, gate-up /
 // down: 169 / 93 us -> 144 / 75, 6.3 TB/s.  A pass takes 16, 32 or 64 rows, whichever holds the rest: a pass of
 // 16 leaves out the products and loads of the second tile (24 tokens: 148 / 77 us without), one of 64 reads the
 // weights once where two of 32 read them twice (8 experts of 2048, 100 tokens: 56 / 26 us -> 39 / 23).
@@ -167,11 +167,14 @@ int dxm_stream_grouped_gemm(void* out, const void* a, int64_t a_stride, const vo
   const dim3 grid((unsigned)(N / 32), (unsigned)E);
   // Two waves where four would have no more than eight pieces each: 2048 wide, 8 experts, gate-up + down, 3 / 16 / 40
   // tokens, us: 33.2 / 45.8 / 48.5 with four, 29.0 / 44.8 / 46.2 with two; 4096 and 3584 wide, 16 experts, 6 / 24 tokens:
-  // 125.6 / 223.1 with four, 141.7 / 237.3 with two.
+  // 125.6 / 223.1 with four, 141.7 / 237.3 with two.  Between them, 16 experts as wide as the model, two layers, 2 / 6 / 24 / 60
+  // tokens: 2304 80 / 143 / 204 / 222 with four, 86 / 146 / 209 / 223 with two; 2560 76 / 140 / 242 / 264, 95 / 158 / 262 / 283.
   const bool two = K <= 2048;
-  // One token's experts there: of 1 / 2 / 4 layers of them the repeated step takes 33.3 / 60.7 / 125.9 us with lines not
-  // kept, 33.1 / 64.8 / 132.9 kept (before: 33.8 / 66.0 / 131); from two tokens on it is the other way round, 78.0 / 75.9
-  // for two layers and 163 / 148 for four.
+  // Of one or two rows in all little comes through the caches, and what a step of many layers reads is not there the next time:
+  // 24 layers of 8 experts of 2048 (nothing of 0.4 to 1.2 GB is left), a layer, kept / not, us, one row 21.7 / 20.4, two (one
+  // token's at two each) 25.0 / 24.3, two tokens' at one each 24.9 / 24.6, four 31.4 / 34.3 (two tokens') and 33.3 / 37.1 (one
+  // token's); experts of 1792 20.9 / 19.6, 25.0 / 25.5, 24.6 / 25.1, 30.3 / 34.0 and 32.2 / 36.7.  (Steps that fit the last cache lose:
+  // eight layers of 2048, one row 17.7 / 20.8, two 25.1 / 24.2.)
   const bool nt = two && R <= 2;
   auto kern = nt    ? (glu ? stream_grouped_gemm_kernel<2, true, true> : stream_grouped_gemm_kernel<2, true, false>)
               : two ? (glu ? stream_grouped_gemm_kernel<2, false, true> : stream_grouped_gemm_kernel<2, false, false>)
