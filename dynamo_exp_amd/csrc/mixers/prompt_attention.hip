@@ -21,13 +21,16 @@
 //     largest weight exactly when that weight is 1, so there the maximum follows every tile.
 //   * Wide shared rows (256 value columns): the upper half of the queries stays in LDS, the accumulators need its
 //     registers.
-//   * Tiles of 64 keys, or of 32 where that lets more workgroups onto a CU: rows of 256 columns, and the forms with
-//     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.
+//   * Tiles of 64 keys, or of 32 where that lets more workgroups onto a CU: values of 256 columns, and the forms with
+//     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.  (Most tiles hold a
+//     new maximum for one of a wave's 32 rows, and every one costs a multiplication of each accumulator: half as many of them
+//     is what shared rows of 192 value columns gain from 64 keys.)
 //   * Between the products of a tile's scores the next tile's DMA goes out; all four waves' at once behind the barrier
 //     stood in each other's way.
-//   * Score terms: the tanh cap is a polynomial of degree 7 where a tile's scores are small against the cap (|x / cap| <
-//     0.36, relative error 2.3e-7; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
-//     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.
+//   * Score terms: the tanh cap is a polynomial of degree 5 or 7 where a tile's scores are small against the cap (|x / cap| <
+//     0.17 or 0.36, relative error 2.3e-7; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
+//     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.  With the table a
+//     row's newest keys come first: new maxima (64 multiplications a tile, of some 270 instructions) end with them.
 //   * Few rows behind a long context leave most of the chip idle, and a workgroup alone on its CU takes 0.5 to 1 us for 32
 //     keys, whatever it does with them: there the keys go out in parts (dxm_prompt_attention_parts, grid z), whose sums
 //     merge_parts joins.  One prompt of 16 rows behind 2000 keys, 32 heads, us of the GPU: causal 41 -> 13, two maps in
@@ -36,9 +39,11 @@
 // What bounds it: two waves a SIMD in softmax and products in turn (two maps: the matrix cores busy 45 % of the time;
 // forming a tile's scores between the weights of the one in front needs 16 registers more than there are, and spills:
 // 1.25 x slower), and a wave's issue where there are score terms.  32 heads, ragged prompts of about 4000 tokens, us,
-// with fragments read one product ahead -> now: two maps with values of 256, window 1024 + 64, 5003 rows beside 16 decode
-// rows, with the combine: 288 -> 270; shared row 256 / 192 causal 125 -> 113 (870 TFLOP/s); cap + penalty, window 1024,
-// 138 -> 97 (600 rows behind 2000 cached, window 512: 36 -> 25); sigmoid 85 -> 78.  (The register-staged 16x16x32 forms
+// before -> now: two maps with values of 256, window 1024 + 64, 5003 rows beside 16 decode rows, with the combine: 288 -> 270;
+// shared row 256 / 192 causal, tiles of 32 keys -> 64, 4203 rows 111 -> 101 (970 TFLOP/s), 600 rows 25.3 -> 21.8, window 1024,
+// 1500 rows 47 -> 43; cap + penalty, window 1024, keys in order and degree 7 -> the newest first and degree 5, 4500 rows 95 -> 87,
+// 3000 of 16 heads 47 -> 43, 600 rows behind 2000 cached, window 512, 26.6 -> 24.9 (its error against 64 bits 1.95e-3 -> 1.96e-3);
+// sigmoid 85 -> 78.  (The register-staged 16x16x32 forms
 // of tile_attention.hip, stream and latent prefill, which it took over from: two maps and their combine 776, 242, 313.)
 #include <algorithm>
 #include <cmath>
@@ -81,6 +86,7 @@ constexpr int kLeastTiles = 4;  // of a part, of several
 // kTable: cap and / or penalty where a row sees at most kTableKeys keys back: the penalty is a table of the distance in LDS
 enum { kPlain = 0, kTerms = 1, kSigmoid = 2, kTable = 3 };
 constexpr int kTableKeys = 1216;  // what three workgroups of a CU have room for beside their tiles
+constexpr int kExact = 8;         // tiles of a row's newest keys whose largest weight is exactly 1
 constexpr int kTablePad = 64;     // entries for keys of a tile that a row does not see, on both sides
 
 // tanh(y) / y = sum kTanh[i] y^(2 i) for |y| <= kTanhMax (minimax, fitted in 64 bits; relative error of these floats 6.2e-8, of
@@ -88,12 +94,20 @@ constexpr int kTablePad = 64;     // entries for keys of a tile that a row does 
 // those of scale / cap would leave the number range
 constexpr float kTanhMax = 0.36f, kNearMax = 0x1p18f;
 constexpr float kTanh[4] = {0.99999996f, -0.33332261f, 0.13291534f, -0.04868792f};
+// the same for |y| <= kTanhMin, to 6.2e-8 with a term less
+constexpr float kTanhMin = 0.17f, kTanhFew[3] = {0.99999994f, -0.33330771f, 0.13098775f};
 
 __device__ __forceinline__ void opaque(int& x) { asm("" : "+v"(x)); }
 // One v_maximum3, which hands a NaN on (fmaxf() would quiet every operand first).  The compiler's own: in front of inline
 // assembly it does not wait for the matrix product that an operand comes from.
 __device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 __device__ __forceinline__ float max3(float a, float b, float c) { return max2(max2(a, b), c); }
+// x + the two bf16 of w
+__device__ __forceinline__ float sum_of_pair(uint32_t w, float x) {
+  uint32_t ones = 0x3f803f80u;  // (in a register: of some constants the encoding takes only one half)
+  asm("" : "+s"(ones));
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, ones), x, false);
+}
 // a number that is the same in every lane, in a scalar register
 __device__ __forceinline__ float uniform(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
 __device__ __forceinline__ float swap_max(float x) {
@@ -116,9 +130,12 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   constexpr int kKey = KT * KB, kStage = kKey + (SAME ? 0 : KT * VB);
   constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
-  constexpr int KA = MODE == kPlain ? 4 : 3, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
+  constexpr int KA = MODE != kPlain ? 3 : SAME && SUBS == 2 ? (PARTS ? 2 : 3) : 4, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
   constexpr bool kEager = MODE == kTerms || MODE == kTable;
-  constexpr float kDefer = FINE ? 8.f : 0.f;  // log2 units that a score may exceed the running maximum by
+  // A penalty that grows with the distance: the newest keys first, whose scores are a row's largest.  Behind them the maximum
+  // hardly moves, and from kExact tiles on it stays where it is for scores that exceed it a little (their weights, over 1, are
+  // then rounded like any other, and summed as rounded).
+  constexpr bool kBack = MODE == kTable;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -187,8 +204,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   auto find = [&](int t) {
     const int j = t << SH, page = j >> a.bs_shift;
     if (page - page0 >= 64 || page < page0) {
-      page0 = page;
-      pages = bt[min(page + lane, hi >> a.bs_shift)];
+      page0 = kBack ? max(page - 63, 0) : page;
+      pages = bt[min(page0 + lane, hi >> a.bs_shift)];
       __builtin_amdgcn_s_waitcnt(0x0f70);  // (here and now: behind the branch it would be waited for, and the DMA, at every tile)
     }
     const uint32_t slot = ((uint32_t)__builtin_amdgcn_readlane(pages, page - page0) << a.bs_shift) + (j & ((1 << a.bs_shift) - 1));
@@ -217,6 +234,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   const float y1 = terms && cap > 0.f ? a.scale / cap : 0.f, y2 = y1 * y1, near = uniform(y1 > 0.f ? fminf(kTanhMax / y1, kNearMax) : 0.f);
   const float t0 = uniform(a.scale * kLog2e * kTanh[0]), t1 = uniform(a.scale * kLog2e * kTanh[1] * y2),
               t2 = uniform(a.scale * kLog2e * kTanh[2] * y2 * y2), t3 = uniform(a.scale * kLog2e * kTanh[3] * y2 * y2 * y2);
+  const float nearer = near * (kTanhMin / kTanhMax), u0 = uniform(a.scale * kLog2e * kTanhFew[0]),
+              u1 = uniform(a.scale * kLog2e * kTanhFew[1] * y2), u2 = uniform(a.scale * kLog2e * kTanhFew[2] * y2 * y2);
   const bool logs = MODE != kPlain && MODE != kTable && a.r1;
   const float r1 = uniform(logs ? a.r1[qh] : 0.f), r2 = uniform(logs ? a.r2[qh] : 0.f);
   const float sc = terms ? 1.f : a.scale * kLog2e;  // scores to log2 units
@@ -232,7 +251,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     const i16x4 up = read_tr16((const lds_i16x4*)(uintptr_t)(vp + 8 * VB + (v_at ^ 64 * (f % NC & 3) ^ 32)));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  auto step = [&](auto bufc, int t) {
+  auto step = [&](auto bufc, int t, float defer) {
     constexpr uint32_t kb = decltype(bufc)::value * kStage, vb = SAME ? kb : kb + kKey;  // from the front
     constexpr uint32_t other = (1 - decltype(bufc)::value) * kStage;                     // the next tile's
     const int kt = t << SH;
@@ -281,7 +300,15 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
 #pragma unroll
         for (int i = 1; i < 16 * SUBS - 1; i += 2) far = max3(far, fabsf(s[i >> 4][i & 15]), fabsf(s[(i + 1) >> 4][(i + 1) & 15]));
         far = max2(far, fabsf(s[SUBS - 1][15]));
-        if (__builtin_amdgcn_ballot_w64(!(far <= near)) == 0) {
+        if (__builtin_amdgcn_ballot_w64(!(far <= nearer)) == 0) {
+#pragma unroll
+          for (int sub = 0; sub < SUBS; ++sub)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float t = s[sub][i] * s[sub][i];
+              s[sub][i] = fmaf(s[sub][i], fmaf(t, fmaf(t, u2, u1), u0), -penalty(sub, i));
+            }
+        } else if (__builtin_amdgcn_ballot_w64(!(far <= near)) == 0) {
 #pragma unroll
           for (int sub = 0; sub < SUBS; ++sub)
 #pragma unroll
@@ -347,7 +374,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       }
       // both halves of a row see the same maximum and take the same decision
       const float tm = swap_max(fmaxf(ta, tb)) * sc;
-      const float mn = tm > m_i + kDefer ? tm : m_i;
+      const float mn = tm > m_i + defer ? tm : m_i;
       mu = mn == -INFINITY ? 0.f : mn;  // a row that has seen nothing yet
       if (__builtin_amdgcn_ballot_w64(mn != m_i)) {
         const float alpha = fast_exp2(m_i - mu);
@@ -373,8 +400,9 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
           else
             w[x] = fast_exp2(fmaf(v, sc, -mu));
         }
-        if constexpr (MODE != kSigmoid) l_i += w[0] + w[1];
+        if constexpr (MODE != kSigmoid && !kBack) l_i += w[0] + w[1];
         ph[k16 & 1][e] = pack_bf16x2(w[0], w[1]);
+        if constexpr (kBack) l_i = sum_of_pair(ph[k16 & 1][e], l_i);
         if constexpr (FINE) pl[k16 & 1][e] = pack_bf16x2(w[0] - bf16lo(ph[k16 & 1][e]), w[1] - bf16hi(ph[k16 & 1][e]));
       }
     };
@@ -398,7 +426,12 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     }
     if constexpr (kEager) __builtin_amdgcn_s_setprio(1);
   };
-  auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
+  auto tile = [&](int i) {
+    if constexpr (kBack) return first + i0 + i1 - 1 - i;  // (this form has no kept keys)
+    return i < kept ? i : first + i - kept;
+  };
+  // log2 units that a score may exceed the running maximum by
+  auto defer = [&](int i) { return FINE || (kBack && i - i0 >= kExact) ? 8.f : 0.f; };
   static_assert(ND <= KS, "a DMA instruction beside a product at most");
   find(tile(i0));
 #pragma unroll
@@ -406,11 +439,11 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   landed();
   for (int i = i0; i < i1; i += 2) {  // (behind the last tile it is fetched again: no branch among the products)
     find(tile(min(i + 1, i1 - 1)));
-    step(std::integral_constant<int, 0>{}, tile(i));
+    step(std::integral_constant<int, 0>{}, tile(i), defer(i));
     landed();
     if (i + 1 < i1) {
       find(tile(min(i + 2, i1 - 1)));
-      step(std::integral_constant<int, 1>{}, tile(i + 1));
+      step(std::integral_constant<int, 1>{}, tile(i + 1), defer(i + 1));
       landed();
     }
   }
@@ -494,11 +527,11 @@ int launch_prompt(const PromptArgs& a, int n_tiles, hipStream_t st) {
 }
 
 // (tiles of 32 / 64 keys, us, launches back to back: cap + penalty 157 / 153, sigmoid 91 / 99, shared row 256 / 256
-// 128 / 182, 256 / 192 130 / 127 and of 600 rows 35.3 / 36.7, two maps 265 / 350, plain of 5000 149 / 154 and of 40 behind
+// 128 / 182, 256 / 192 causal 120 / 113, 600 rows 24.5 / 22.0, 40 behind 2900 cached 24.4 / 22.3, two maps 265 / 350, plain of 5000 149 / 154 and of 40 behind
 // 2900 cached 94 / 83, fine 179 / 186)
 template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT>
 int prompt_heads(const PromptArgs& a, int n_tiles, hipStream_t st) {
-  constexpr int SUBS = DV == 128 && MODE == kPlain ? 2 : 1;
+  constexpr int SUBS = (DV == 128 && MODE == kPlain) || DV == 192 ? 2 : 1;
   if (a.group % 4 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 4, 4, SUBS>(a, n_tiles, st);
   return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 2, 4, SUBS>(a, n_tiles, st);
 }

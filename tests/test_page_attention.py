@@ -311,6 +311,31 @@ def test_score_terms_of_limited_distance(form, cap, mask, size):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form,cap", [("both", 30.0), ("both", 50.0), ("penalty", 0.0)])
+@pytest.mark.parametrize("old", [(), (100,), (100, 250, 640), (3, 4, 870)])
+def test_penalty_rows_whose_old_keys_count(form, cap, old):
+    """The newest keys come first: maxima among the first tiles, behind them (by less and by more than the maximum waits for),
+    in the last one; scores on both sides of what each polynomial of the cap takes."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(13)
+    scale, start, rows, bs, size = 0.7 * d ** -0.5, 900, 40, 64, 1000
+    db = (torch.rand(n_qh), torch.rand(n_qh) + 0.1)
+    kd, vd, table, kv = pages(form, [start + rows], bs)
+    for i, j in enumerate(old):  # (powers of two: the keys stay bf16)
+        kd[int(table[0, j // bs]) * bs + j % bs] *= 4 << i % 2
+        kv[0][0][j] *= 4 << i % 2
+    q = torch.randn(rows, n_qh * d).bfloat16()
+    want = dense(q.double().view(rows, n_qh, d), *kv[0], torch.arange(start, start + rows), scale, "window", size, 0, cap, db,
+                 None, False, None)
+    tiles = torch.tensor(mx.tile_list(0, rows), dtype=torch.int32).cuda()
+    got = mx.attention(q.cuda(), kd, vd, torch.arange(start, start + rows).cuda(), torch.zeros(rows, dtype=torch.int32).cuda(),
+                       table, bs, n_qh, maps, group, d, dv, scale, "window", size, 1, False, tiles, rows, softcap=cap,
+                       dist_bias=tuple(map(cuda, db))).cpu().double()
+    # (bound of test_prompt_rows: weights over their own sum as rounded are 2^-9 off in each, 2^-8 of |v| < 5 together)
+    assert float((got - want).abs().max()) < 2.0 ** -8 * (float(want.abs().max()) + 5.0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mask,size", [("causal", 0), ("chunk", 1500)])
 @pytest.mark.parametrize("form", ["shared", "plain", "diff", "sigmoid"])
 @pytest.mark.parametrize("ctx", [[4000, 33, 1, 2500, 700], [1, 3000], [300 + 61 * i for i in range(20)],
