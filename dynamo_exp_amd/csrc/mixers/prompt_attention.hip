@@ -131,7 +131,13 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
   constexpr int KA = MODE != kPlain ? 3 : SAME && SUBS == 2 ? (PARTS ? 2 : 3) : 4, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
-  constexpr bool kEager = MODE == kTerms || MODE == kTable;
+  // What a wave does at raised priority, where two or three share a SIMD.  Score terms and pairs of maps: everything but the
+  // value products, which fill what the others' vector work leaves; shared rows, whose products are the longer part: the value
+  // products; sigmoid weights: both products.  us, without / with (5003 rows of two maps beside 16, 3000 in chunks of 2048; 4203
+  // causal 256 / 192, 4935 of a window 256 / 256; 3000 sigmoid): 272 / 270, 130 / 125; 107 / 102, 156 / 150; 55.7 / 52.7.  Plain
+  // heads lose 2 to 5 % with each of them.
+  enum { kNothing, kVectors, kValues, kProducts };
+  constexpr int kRaised = SAME ? kValues : MODE == kSigmoid ? kProducts : MODE != kPlain || DV == 256 ? kVectors : kNothing;
   // A penalty that grows with the distance: the newest keys first, whose scores are a row's largest.  Behind them the maximum
   // hardly moves, and from kExact tiles on it stays where it is for scores that exceed it a little (their weights, over 1, are
   // then rounded like any other, and summed as rounded).
@@ -289,6 +295,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
         __builtin_amdgcn_sched_group_barrier(0x100, SUBS + (QR < KS), 0);
       }
     }
+    if constexpr (kRaised == kProducts) __builtin_amdgcn_s_setprio(0);
     if (MODE != kPlain && terms) {  // final scores in log2 units
       // penalties of the lane's keys
       const uint32_t pen = table + 4 * (kTablePad - 31 + my - kt - 4 * h);
@@ -374,7 +381,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       }
       // both halves of a row see the same maximum and take the same decision
       const float tm = swap_max(fmaxf(ta, tb)) * sc;
-      const float mn = tm > m_i + defer ? tm : m_i;
+      const float mn = tm > (FINE || kBack ? m_i + defer : m_i) ? tm : m_i;
       mu = mn == -INFINITY ? 0.f : mn;  // a row that has seen nothing yet
       if (__builtin_amdgcn_ballot_w64(mn != m_i)) {
         const float alpha = fast_exp2(m_i - mu);
@@ -408,8 +415,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     };
     constexpr int NF = 2 * SUBS * NC;  // value fragments of the tile
     weigh(0);
-    // forms whose vector work is the longer part: a wave that is at it goes first, products fill what it leaves
-    if constexpr (kEager) __builtin_amdgcn_s_setprio(0);
+    if constexpr (kRaised != kNothing) __builtin_amdgcn_s_setprio(kRaised == kVectors ? 0 : 1);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const int k16 = f / NC, dt = f % NC;
@@ -424,7 +430,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       __builtin_amdgcn_sched_group_barrier(0x008, FINE ? 2 : 1, 0);
       if (f + VA < NF) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    if constexpr (kEager) __builtin_amdgcn_s_setprio(1);
+    if constexpr (kRaised == kVectors) __builtin_amdgcn_s_setprio(1);
+    if constexpr (kRaised == kValues) __builtin_amdgcn_s_setprio(0);
   };
   auto tile = [&](int i) {
     if constexpr (kBack) return first + i0 + i1 - 1 - i;  // (this form has no kept keys)
