@@ -83,7 +83,7 @@ __device__ __forceinline__ float halves_sum(float x) {
 }
 
 // V: 0 = the first loop (kept for A/B), 1 = deferred rescale, row
-// sum on the matrix pipe, v_max3 row max, static priority, widened epilogue.
+// sum on the matrix pipe, v_max3 row max, raised priority (step), widened epilogue.
 // (Ping-pong wave halves, two tiles per barrier and a software-pipelined QK /
 // softmax measured slower, as did 4-wave workgroups where there are enough of
 // 8: profiles/r4_prefill_attn_variants.txt.)
@@ -336,6 +336,9 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
   };
 
   {
+    // Two waves of one workgroup share a SIMD: scores and softmax at raised priority, the value products fill what they leave.
+    // (Three of 2000 together 141 -> 137 us with waves 4-7 raised throughout before.  Two workgroups of four waves lose 4 to 6 %.)
+    constexpr bool kRaised = NW == 8 && V != 0;
     auto step = [&](auto bufc, int t) __attribute__((always_inline)) {
       constexpr int BUF = decltype(bufc)::value;
       char* kb = smem + BUF * kBuf;
@@ -343,13 +346,14 @@ __global__ void __launch_bounds__(64 * NW, 2) prefill_attn_v2_kernel(
       u16x8 pf[2][2];
       bf16x8_t vf[kAhead];
       bool live1;
-      if (qk_sm(kb, t, pf, live1, vf)) pv(kb + kTileBytes, live1, pf, vf);
+      if (qk_sm(kb, t, pf, live1, vf)) {
+        if constexpr (kRaised) __builtin_amdgcn_s_setprio(0);
+        pv(kb + kTileBytes, live1, pf, vf);
+        if constexpr (kRaised) __builtin_amdgcn_s_setprio(1);
+      }
       landed();
     };
     if (n_tiles > 0) issue(smem, 0);
-    // static priority for the second-dispatched half (guide "Two waves per
-    // SIMD" item 4): without it waves 4-7 lose every arbitration
-    if (NW == 8 && V != 0 && wid >= 4) __builtin_amdgcn_s_setprio(1);
     landed();
     for (int t = 0; t < n_tiles; t += 2) {
       step(std::integral_constant<int, 0>{}, t);
