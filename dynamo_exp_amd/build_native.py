@@ -59,9 +59,13 @@ def _headers(d: Path) -> list[Path]:
     return sorted(d.glob("*.h"))
 
 
-# attention: scores are finite or -inf by construction, so fmax needs no NaN
-# quieting (IEEE mode off: v_max3 without a v_mul canonicalize per score)
-PER_FILE_FLAGS = {"attn_prefill.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
+# attn_prefill: scores are finite or -inf by construction, so fmax needs no NaN
+# quieting (IEEE mode off: v_max3 without a v_mul canonicalize per score).
+# decode_attention: one wave a SIMD has registers of both kinds; without the
+# option all matrix products' accumulators are of the second kind, and those
+# of shared rows were copied to and fro in every tile (600 instructions of 1770).
+PER_FILE_FLAGS = {"attn_prefill.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
+                  "decode_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _kernel_flags(src_dir: Path) -> list[str]:
@@ -156,6 +160,7 @@ def build_mixers(verbose: bool = False, jobs: int = 8) -> Path:
         objs.append(o)
         if _stale(o, [s, Path(__file__)] + hdrs):
             extra = list(HIP_FLAGS) if s.suffix == ".hip" else []
+            extra += PER_FILE_FLAGS.get(s.name, [])
             todo.append([hipcc, *flags, *extra, "-c", str(s), "-o", str(o)])
     with ThreadPoolExecutor(max(1, jobs)) as ex:
         list(ex.map(lambda c: _run(c, verbose), todo))

@@ -12,9 +12,11 @@
 // shared row has two buffers in turn.  V^T fragments come from the row-major image by ds_read_b64_tr_b16.
 // One part: the result goes out finished; several: partials to the workspace that merge_parts joins.
 // Bound by memory at many rows and by latency at few (position, block table, first tile, join: 7 us of a launch with one
-// tile a wave).  Two layers in a graph with their joins, us, two maps, window 1024 + 64, 48 rows 98 -> 86.5 nontemporally;
-// shared row 256 / 192 causal to 4000, 33 rows 53 with fragments read one product ahead -> 50, to 2500, 100 rows 79 -> 73;
-// 256 / 256 window 1024, 20 rows 41 -> 38; two maps, 2 rows of 142 25.3 -> 24.2.  Parts dealt out by the rows' lengths
+// tile a wave).  Two layers in a graph with their joins, us: two maps, window 1024 + 64, 48 rows 98 -> 86 nontemporally -> 84.5,
+// shared row 256 / 192 causal to 4000, 33 rows 53 with fragments read one product ahead -> 49.5 -> 44.5, to 2500, 100 rows 79 ->
+// 70.5 -> 63; 256 / 256 window 1024, 20 rows 41 -> 37.4 -> 33.8; two maps, 2 rows of 142 25.3 -> 24.2 (the last step each time:
+// accumulators that are not copied between the two kinds of registers, a build option; the join's reads all at once instead of
+// column block by column block, 3400 cycles before; both blocks of query vectors through the softmax side by side).  Parts dealt out by the rows' lengths
 // instead of equally: 33 rows the same (memory is as busy while the short rows last), 41 rows of up to 281 keys 60 -> 64.
 // (The one-wave forms it took over from, register-staged group_decode, stream_decode, latent_decode: 270 and 92.)
 #include <algorithm>
@@ -276,7 +278,13 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
               S[qb][kb][r] = seen ? S[qb][kb][r] : -INFINITY;
             }
         }
-        float mu = 0.f;
+      }
+      // (all blocks of query vectors behind one branch: with one for each their chains ran one after the other)
+      float mu[QB], mn[QB];
+      bool moved = false;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        mu[qb] = 0.f;
         if constexpr (MODE != kSigmoid) {
           float mloc = S[qb][0][0];
 #pragma unroll
@@ -284,18 +292,25 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
 #pragma unroll
             for (int r = 0; r < 4; ++r) mloc = fmaxf(mloc, S[qb][kb][r]);
           const float tm = groups_max(mloc) * sc;  // (every tile holds a visible key)
-          const float mn = tm > mx[qb] + kDefer ? tm : mx[qb];
-          mu = mn == -INFINITY ? 0.f : mn;
-          if (__any(mn != mx[qb])) {
-            const float alpha = fast_exp2(mx[qb] - mu);
-            lsum[qb] *= alpha;
-#pragma unroll
-            for (int cb = 0; cb < NC; ++cb)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) O[qb][cb][r] *= alpha;
-          }
-          mx[qb] = mn;
+          mn[qb] = tm > mx[qb] + kDefer ? tm : mx[qb];
+          mu[qb] = mn[qb] == -INFINITY ? 0.f : mn[qb];
+          moved |= mn[qb] != mx[qb];
         }
+      }
+      if (MODE != kSigmoid && __any(moved)) {
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+          const float alpha = fast_exp2(mx[qb] - mu[qb]);
+          lsum[qb] *= alpha;
+#pragma unroll
+          for (int cb = 0; cb < NC; ++cb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) O[qb][cb][r] *= alpha;
+          mx[qb] = mn[qb];
+        }
+      }
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
         raw_u32x4 ph, pl;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -306,7 +321,7 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
             if constexpr (MODE == kSigmoid)  // an invisible key (-inf) weighs 0
               wt[x] = __builtin_amdgcn_rcpf(1.f + fast_exp2(-fmaf(v, sc, hb[qb])));
             else
-              wt[x] = fast_exp2(fmaf(v, sc, -mu));
+              wt[x] = fast_exp2(fmaf(v, sc, -mu[qb]));
           }
           lsum[qb] += wt[0] + wt[1];
           ph[e] = pack_bf16x2(wt[0], wt[1]);
@@ -440,6 +455,18 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
         slab(w)[(qb * NC + cb) * 64 + lane] = f32x4{O[qb][cb][0] * f, O[qb][cb][1] * f, O[qb][cb][2] * f, O[qb][cb][3] * f};
     }
     __syncthreads();
+    // the wave's blocks of 16 columns, every fourth: all reads on their way together
+    constexpr int CW = NC / 4;
+    f32x4 o[QB][CW];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int j = 0; j < CW; ++j) {
+        const int at = (qb * NC + 4 * j + w) * 64 + lane;
+        o[qb][j] = slab(0)[at];
+#pragma unroll
+        for (int v = 1; v < 4; ++v) o[qb][j] += slab(v)[at];
+      }
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       if (!okh[qb]) continue;
@@ -459,20 +486,17 @@ __global__ void __launch_bounds__(256, SAME || MAPS == 2 ? 1 : 2) decode_attenti
         ws[1] = MODE == kSigmoid ? 1.f : lt[qb];
       }
 #pragma unroll
-      for (int cb = 0; cb < NC; ++cb) {
-        if ((cb & 3) != w) continue;
-        f32x4 o = slab(0)[(qb * NC + cb) * 64 + lane];
-#pragma unroll
-        for (int v = 1; v < 4; ++v) o += slab(v)[(qb * NC + cb) * 64 + lane];
-        const int c = cb * 16 + 4 * g4;
+      for (int j = 0; j < CW; ++j) {
+        const f32x4 x = o[qb][j];
+        const int c = (4 * j + w) * 16 + 4 * g4;
         if (ws) {
-          *reinterpret_cast<float2*>(ws + 2 + c) = float2{o[0], o[1]};
-          *reinterpret_cast<float2*>(ws + 4 + c) = float2{o[2], o[3]};
+          *reinterpret_cast<float2*>(ws + 2 + c) = float2{x[0], x[1]};
+          *reinterpret_cast<float2*>(ws + 4 + c) = float2{x[2], x[3]};
         } else if (a.out_f32) {
-          *reinterpret_cast<f32x4*>((float*)a.out + vrow * DV + c) = f32x4{o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+          *reinterpret_cast<f32x4*>((float*)a.out + vrow * DV + c) = f32x4{x[0] * inv, x[1] * inv, x[2] * inv, x[3] * inv};
         } else {
-          *reinterpret_cast<uint2*>((bf16_t*)a.out + vrow * DV + c) = uint2{pack_bf16x2(o[0] * inv, o[1] * inv),
-                                                                            pack_bf16x2(o[2] * inv, o[3] * inv)};
+          *reinterpret_cast<uint2*>((bf16_t*)a.out + vrow * DV + c) = uint2{pack_bf16x2(x[0] * inv, x[1] * inv),
+                                                                            pack_bf16x2(x[2] * inv, x[3] * inv)};
         }
       }
     }
