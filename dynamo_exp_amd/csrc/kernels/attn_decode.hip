@@ -80,9 +80,15 @@ __device__ __forceinline__ float group_sum(float v) {
 }
 
 // tokens per partition when a context of ctx tokens is split into n balanced
-// parts, rounded up to `align` (the workgroup's 4-wave chunk stride)
+// parts, rounded up to `align` (the workgroup's 4-wave chunk stride), or to
+// half or a quarter of it where a part is no longer: a CU takes 55 cycles for
+// a KB of K or V however its lanes lie, so a part of 128 tokens holds its CU
+// for 3500 while most of the chip has none.  Eight layers in a graph, one
+// sequence of 700 tokens 71 -> 64 us; four layers, one of 150 36.4 -> 33.7,
+// two of 500 44.6 -> 36.6, four of 700 45.6 -> 40.0, 32 / 8 heads.
 __device__ __forceinline__ int balanced_part(int ctx, int n, int align) {
   const int per = (ctx + n - 1) / n;
+  align = per <= align / 4 ? align / 4 : per <= align / 2 ? align / 2 : align;
   return (per + align - 1) / align * align;
 }
 
@@ -435,6 +441,14 @@ __device__ __forceinline__ int vimg_off(int row, int ch) {  // byte offset of 16
   return row * 256 + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
+// over the four 16-lane groups of a wave, by exchanges in registers
+template <typename F> __device__ __forceinline__ float over_groups(float x, F f) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4_t;
 
 template <int G, bool NT, bool F8>
@@ -595,8 +609,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
       for (int j = 0; j < 8; ++j) t[j] = cb + 8 * g + j >= p1 ? -INFINITY : t[j];
     }
     float cmax = fmaxf(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])), fmaxf(fmaxf(t[4], t[5]), fmaxf(t[6], t[7])));
-    cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
-    cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+    cmax = over_groups(cmax, [](float x, float y) { return fmaxf(x, y); });
     const float m_new = cmax > m_i + kRescale ? cmax : m_i;
     const float alpha = fast_exp2(m_i - m_new);
     m_i = m_new;
@@ -631,8 +644,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
 
   // wave state -> LDS: lane (g, r < G) holds dims 16 db + 4 g + i of head r;
   // l is this lane's share of the head's row sum (its 8 tokens per chunk)
-  float l_tot = l_i + __shfl_xor(l_i, 16, 64);
-  l_tot += __shfl_xor(l_tot, 32, 64);
+  const float l_tot = over_groups(l_i, [](float x, float y) { return x + y; });
   if (r < G) {
 #pragma unroll
     for (int db = 0; db < 8; ++db)
@@ -652,10 +664,11 @@ typedef float f32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef unsigned int u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 
 // merge flash-decoding partitions: grid (Hq, B), block D threads.  Latency-bound (a head's parts are a few KB): the
-// context, the parts' (m, l) and the first 16 parts' rows are all asked for at once, whether the parts exist or not, and
+// context, the parts' (m, l) and the first 4 AHEAD parts' rows are all asked for at once, whether the parts exist or not, and
 // four groups of 32 lanes x 4 columns sum every fourth part.  In a captured step, a layer's attention at 32 / 8 heads, us,
 // part by part with one column a thread before: one sequence of 700 tokens 10.5 -> 9.3, of 4000 19.6 -> 11.1, four of
 // 1500 15.7 -> 12.5.
+template <int AHEAD>
 __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ out, const float* __restrict__ tmp_out,
                                                           const float* __restrict__ tmp_ml,
                                                           const int* __restrict__ ctx_lens, int n_parts, int align) {
@@ -666,9 +679,9 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
   const f32x2_a4* ml = reinterpret_cast<const f32x2_a4*>(tmp_ml) + row0;
   const float* rows = tmp_out + row0 * D + col;
   const f32x2_a4 first = ml[min(lane, n_parts - 1)];
-  f32x4 x[4];
+  f32x4 x[AHEAD];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const f32x4_a4*>(rows + (int64_t)min(grp + 4 * k, n_parts - 1) * D);
+  for (int k = 0; k < AHEAD; ++k) x[k] = *reinterpret_cast<const f32x4_a4*>(rows + (int64_t)min(grp + 4 * k, n_parts - 1) * D);
   const int ctx = ctx_lens[b];
   bf16_t* o = out + ((int64_t)b * nqh + qh) * D + col;
   if (ctx <= 0) {  // a graph bucket's padding row (context 0): no partition wrote it
@@ -688,11 +701,11 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
   for (int d = 32; d; d >>= 1) den += __shfl_xor(den, d, 64);
   f32x4 num = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < AHEAD; ++k) {
     const float w = __shfl(w0, grp + 4 * k, 64);
     if (grp + 4 * k < np) num += w * x[k];  // (a part that does not exist may hold anything)
   }
-  for (int p0 = 16; p0 < np; p0 += 16)
+  for (int p0 = 4 * AHEAD; p0 < np; p0 += 16)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int p = p0 + grp + 4 * k, q = min(p, np - 1);
@@ -710,6 +723,15 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
   u32x2_a2 pk = {0u, 0u};
   if (den != 0.f) pk = u32x2_a2{pack_bf16x2(num[0] / den, num[1] / den), pack_bf16x2(num[2] / den, num[3] / den)};
   *reinterpret_cast<u32x2_a2*>(o) = pk;
+}
+
+// (with few parts the rows that are not there only cost time: 44 sequences of 76 tokens in two parts, three layers 41.5 us
+// asking for 16, 43.0 for 32)
+void join(bf16_t* out, const float* tmp_out, const float* tmp_ml, const int* ctx, int n_q_heads, int batch, int n_parts, int align,
+          hipStream_t st) {
+  const dim3 grid(n_q_heads, batch);
+  if (n_parts > 16) decode_reduce_kernel<8><<<grid, D, 0, st>>>(out, tmp_out, tmp_ml, ctx, n_parts, align);
+  else decode_reduce_kernel<4><<<grid, D, 0, st>>>(out, tmp_out, tmp_ml, ctx, n_parts, align);
 }
 
 template <int G, int LPT, int CH, bool NT, bool F8>
@@ -730,8 +752,7 @@ int launch(bf16_t* out, float* tmp_out, float* tmp_ml, const bf16_t* q, int64_t 
                                                                      bt_stride, ctx, n_kv_heads, block_size,
                                                                      scale * 1.4426950408889634f, out_scale);
   if (n_parts > 1) {
-    dim3 g2(n_kv_heads * G, batch);
-    decode_reduce_kernel<<<g2, D, 0, st>>>(out, tmp_out, tmp_ml, ctx, n_parts, 4 * CH);
+    join(out, tmp_out, tmp_ml, ctx, n_kv_heads * G, batch, n_parts, 4 * CH, st);
   }
   return (int)hipGetLastError();
 }
@@ -746,8 +767,7 @@ int launch_mfma(bf16_t* out, float* tmp_out, float* tmp_ml, const bf16_t* q, int
                                                                 bt_stride, bt_cols, ctx, n_kv_heads, block_size,
                                                                 scale * 1.4426950408889634f, out_scale);
   if (n_parts > 1) {
-    dim3 g2(n_kv_heads * G, batch);
-    decode_reduce_kernel<<<g2, D, 0, st>>>(out, tmp_out, tmp_ml, ctx, n_parts, 4 * MCH);
+    join(out, tmp_out, tmp_ml, ctx, n_kv_heads * G, batch, n_parts, 4 * MCH, st);
   }
   return (int)hipGetLastError();
 }

@@ -60,3 +60,27 @@ def test_rows_that_see_a_nan(monkeypatch, mfma, n_parts, at):
     assert bool(got[0, 4:].isnan().all())
     for g, w in ((got[0, :4], want[0, :4]), (got[1], want[1])):  # (bound of test_parts)
         assert float((g.float() - w.float()).abs().max()) < 2 ** -7 * max(1.0, float(want.float().abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_parts", [3, 17, 33])
+@pytest.mark.parametrize("mfma,bs", [("1", 16), ("1", 48), ("1", 64), ("0", 64)])
+def test_part_lengths(monkeypatch, mfma, bs, n_parts):
+    """Shares of a context around a quarter, a half and the whole of a workgroup's stride, so around the lengths at which
+    parts get coarser; blocks of one, of a ragged number and of a whole number of a wave's 32 tokens."""
+    monkeypatch.setenv("DX_DECODE_MFMA", mfma)
+    torch.manual_seed(n_parts)
+    hq, hkv = 8, 2
+    ctx = [n_parts * k + e for k in (16, 32, 64, 128) for e in (-1, 0, 1)]
+    need = [-(-c // bs) for c in ctx]
+    table = torch.zeros(len(ctx), max(need), dtype=torch.int32)
+    ids = torch.randperm(sum(need)).to(torch.int32)
+    for b, n in enumerate(need):
+        table[b, :n] = ids[sum(need[:b]):sum(need[:b]) + n]
+    kc, vc = (torch.randn(sum(need), hkv, bs, 128).bfloat16() for _ in range(2))
+    q, lens, scale = torch.randn(len(ctx), hq, 128).bfloat16(), torch.tensor(ctx, dtype=torch.int32), 1 / math.sqrt(128)
+    want = ref.paged_attention(q, kc, vc, table, torch.arange(len(ctx) + 1, dtype=torch.int32), lens, scale, bs)
+    out = torch.empty(len(ctx), hq, 128, dtype=torch.bfloat16, device="cuda")
+    got = ops.decode_attention(q.cuda(), kc.cuda(), vc.cuda(), table.cuda(), lens.cuda(), scale, out, n_parts).cpu()
+    err = (got.float() - want.float()).abs().max()  # (bound of test_parts)
+    assert float(err) < 2 ** -7 * max(1.0, float(want.float().abs().max())), float(err)
