@@ -56,7 +56,12 @@
 //     pieces' fp32 sums go through a workspace (64 MB at most) to a kernel that
 //     adds them in order.  One more round costs 230 to 320 us at K 14336, whatever
 //     it holds; a sixteenth of one costs 20 and the way through the workspace 30:
-//     4150 x 4096 520 -> 365 us, 1000 x 4096 227 -> 104.  (In full rounds the
+//     4150 x 4096 520 -> 365 us, 1000 x 4096 227 -> 104.  Where it fills somewhat more,
+//     half as many tiles as there are CUs go out in two pieces each and the others in
+//     as many as fit beside each other (512 pieces, 134 MB): a round is cut to half of
+//     one and a quarter or less.  6151 x 4096 609 -> 589 us, 6400 602 -> 569, 6900 618 ->
+//     600, 7100 628 -> 621, 12400 x 2048 614 -> 548, 2500 x 8192 of K 28672 838 -> 813.
+//     (In full rounds the
 //     card's power is the bound, not the schedule: the matrix cores are busy
 //     80 % of the cycles, and the clock is 1.75 GHz where launches stand alone,
 //     1.5 in a prompt step: profiles/step_case_counters.txt.)  A row's sum is
@@ -84,12 +89,14 @@ constexpr int kLds = 2 * kBuf;     // double buffered: 128 KB
 // EPI_ADD: y += x . w^T (one rounding), the tiles of an incomplete last round split along K (Split)
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_SILU_RS = 2, EPI_ADD = 3 };
 
-// EPI_ADD: tiles 0 .. full - 1 are whole; each of the `rest` behind them is `segs` pieces of K, whose fp32 sums go to
-// part[piece * rest + tile][block (i, j) of the wave][thread] and are joined by gemm256_join_kernel.
+// EPI_ADD: tiles 0 .. full - 1 are whole; each of the rest[0] behind them is segs[0] pieces of K, and each of the rest[1]
+// behind those segs[1].  Their fp32 sums go to part[piece * rest + tile][block (i, j) of the wave][thread] (the second kind's
+// behind all of the first one's) and are joined by gemm256_join_kernel.
 struct Split {
   f32x4* part;
-  int full, rest, segs;
+  int full, rest[2], segs[2];
 };
+constexpr int kSavedK = 3072;  // part of K that two kinds of pieces have to save (K 10240, 144 tiles: 417 -> 412 us, 160: 420 -> 418)
 
 __device__ __forceinline__ float silu_f(float g) { return g / (1.f + __expf(-g)); }
 
@@ -323,7 +330,7 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     issue(3, 1, 1);
   };
 
-  bool piece = false;  // EPI_ADD: this workgroup is at its piece of K, number `unit`
+  int pieces = 0, slot = 0;  // EPI_ADD: kinds of pieces of K that this workgroup has come to (it takes number `unit` of each)
   const int unit = (xcd < gr8 ? xcd * (gq + 1) : gr8 * (gq + 1) + (xcd - gr8) * gq) + (bid >> 3);
   auto begin = [&](int lid) -> bool {
     if (lid < t_end) {
@@ -332,12 +339,16 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     }
     if constexpr (EPI == EPI_ADD) {
       // the workgroups of an XCD take the same piece of neighbouring tiles
-      if (piece || unit >= sp.rest * sp.segs) return false;
-      piece = true;
-      const int c = unit / sp.rest, pairs = nkt / 2;
-      kbase = pairs * c / sp.segs * 2;
-      nk = pairs * (c + 1) / sp.segs * 2 - kbase;
-      select(sp.full + unit - c * sp.rest);
+      const int first = sp.rest[0] * sp.segs[0];
+      if (pieces == 0 && unit >= first) ++pieces;
+      if (pieces == 2 || (pieces == 1 && unit >= sp.rest[1] * sp.segs[1])) return false;
+      const int rest = pieces ? sp.rest[1] : sp.rest[0], segs = pieces ? sp.segs[1] : sp.segs[0];
+      const int c = unit / rest, pairs = nkt / 2;
+      kbase = pairs * c / segs * 2;
+      nk = pairs * (c + 1) / segs * 2 - kbase;
+      select(sp.full + (pieces ? sp.rest[0] : 0) + unit - c * rest);
+      slot = (pieces ? first : 0) + unit;
+      ++pieces;
       return true;
     }
     return false;
@@ -394,18 +405,18 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
     // the next tile's first K-tiles go out before this tile's stores
     if constexpr (EPI == EPI_ADD) {
       // (in front of the next unit's prologue: its DMA would retire before the loads of y)
+      const bool piece = pieces > 0;
       if (piece) {
-        f32x4* o = sp.part + (int64_t)unit * (kBM * kBN / 4) + threadIdx.x;
+        f32x4* o = sp.part + (int64_t)slot * (kBM * kBN / 4) + threadIdx.x;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int j = 0; j < 8; ++j) o[(i * 8 + j) * 512] = acc[i][j];
-        return;
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int tok = tok0 + 16 * j;
-        if (tok >= tok_end) continue;
+        if (piece || tok >= tok_end) continue;
         bf16_t* yr = y + (int64_t)tok * ldy + cnt * kBN + wc * 64 + 4 * lq;
         uint2 was[4];
 #pragma unroll
@@ -460,7 +471,7 @@ __global__ void __launch_bounds__(512) gemm256_kernel(bf16_t* __restrict__ y, in
   }
 }
 
-// y += the pieces of K of the tiles that EPI_ADD split.  grid (2 * 8, rest), block 256: the 16 rows j of half of the
+// y += the pieces of K of the tiles that EPI_ADD split.  grid (2 * 8, tiles), block 256: the 16 rows j of half of the
 // tile's waves
 __global__ void __launch_bounds__(256) gemm256_join_kernel(bf16_t* __restrict__ y, int64_t ldy, int M, int N, int group_m,
                                                            Split sp) {
@@ -475,8 +486,9 @@ __global__ void __launch_bounds__(256) gemm256_join_kernel(bf16_t* __restrict__ 
 #pragma unroll
   for (int i = 0; i < 4; ++i) was[i] = *reinterpret_cast<const uint2*>(yr + 16 * i);
   f32x4 sum[4] = {};
-  const f32x4* p = sp.part + (int64_t)blockIdx.y * (kBM * kBN / 4) + j * 512 + thread;
-  for (int c = 0; c < sp.segs; ++c, p += (int64_t)sp.rest * (kBM * kBN / 4))
+  const int kind = (int)blockIdx.y >= sp.rest[0], rest = kind ? sp.rest[1] : sp.rest[0], segs = kind ? sp.segs[1] : sp.segs[0];
+  const f32x4* p = sp.part + ((int64_t)(kind ? sp.rest[0] * (sp.segs[0] - 1) : 0) + blockIdx.y) * (kBM * kBN / 4) + j * 512 + thread;
+  for (int c = 0; c < segs; ++c, p += (int64_t)rest * (kBM * kBN / 4))
 #pragma unroll
     for (int i = 0; i < 4; ++i) sum[i] += p[i * 8 * 512];
 #pragma unroll
@@ -504,7 +516,7 @@ void launch(bf16_t* y, int64_t ldy, const bf16_t* x, int64_t ldx, const bf16_t* 
   const int tiles = ((M + kBM - 1) / kBM) * (N / kBN);
   const int grid = persistent ? std::min(tiles, num_cus()) : tiles;
   hipLaunchKernelGGL((gemm256_kernel<EPI, false>), dim3(grid), dim3(512), 0, st, y, ldy, x, ldx, w, M, N, K, gm, rs,
-                     GroupMap{nullptr, nullptr, 0, 1, 0, 0}, Split{nullptr, 0, 0, 0});
+                     GroupMap{nullptr, nullptr, 0, 1, 0, 0}, Split{});
 }
 
 template <int EPI>
@@ -512,7 +524,7 @@ void launch_grouped(bf16_t* y, int64_t ldy, const bf16_t* x, int64_t ldx, const 
                     hipStream_t st, const GroupMap& map) {
   const int tiles = ((R + kBM - 1) / kBM + map.E) * (N / kBN);
   hipLaunchKernelGGL((gemm256_kernel<EPI, true>), dim3(std::min(tiles, num_cus())), dim3(512), 0, st, y, ldy, x, ldx, w,
-                     R, N, K, gm, nullptr, map, Split{nullptr, 0, 0, 0});
+                     R, N, K, gm, nullptr, map, Split{});
 }
 
 }  // namespace
@@ -543,21 +555,27 @@ extern "C" int dx_gemm256(void* y, int64_t ldy, const void* x, int64_t ldx, cons
   return 0;
 }
 
-// How dx_gemm256_add splits its tiles: {whole tiles, the rest, pieces of K each}.  A last round that fills at most half of
-// the CUs is cut along K.
-static void add_split(int M, int N, int K, int* full, int* rest, int* segs) {
-  const int tiles = (M + kBM - 1) / kBM * (N / kBN), cus = num_cus(), left = tiles % cus;
-  *full = tiles, *rest = 0, *segs = 0;
-  if (left == 0 || 2 * left > cus) return;
-  *full = tiles - left, *rest = left, *segs = std::min(std::min(cus / left, 16), K / (2 * kBK));
+// How dx_gemm256_add splits its tiles.  A last round that fills at most half of the CUs is cut along K into as many pieces
+// as there are CUs for.  A fuller one: half as many tiles as CUs in two pieces each, then what is left like that, where the
+// part of a round that this saves, 1 - 1 / 2 - 1 / pieces, is longer than the way of 512 pieces through the workspace.
+static Split add_split(int M, int N, int K) {
+  const int tiles = (M + kBM - 1) / kBM * (N / kBN), cus = num_cus(), left = tiles % cus, half = cus / 2;
+  auto pieces = [&](int n) { return std::min(std::min(cus / n, 16), K / (2 * kBK)); };
+  Split sp{nullptr, tiles, {0, 0}, {0, 0}};
+  if (left == 0) return sp;
+  if (2 * left <= cus) {
+    sp.full = tiles - left, sp.rest[0] = left, sp.segs[0] = pieces(left);
+  } else if (const int n = pieces(left - half); n > 2 && (int64_t)(n - 2) * K >= 2 * kSavedK * n) {
+    sp.full = tiles - left, sp.rest[0] = half, sp.segs[0] = 2, sp.rest[1] = left - half, sp.segs[1] = n;
+  }
+  return sp;
 }
 
 // fp32 workspace (floats) of dx_gemm256_add
 extern "C" int64_t dx_gemm256_add_floats(int M, int N, int K) {
   if (M < 1 || N < kBN || N % kBN || K < 2 * kBK || K % (2 * kBK)) return 0;
-  int full, rest, segs;
-  add_split(M, N, K, &full, &rest, &segs);
-  return (int64_t)rest * segs * kBM * kBN;
+  const Split sp = add_split(M, N, K);
+  return (int64_t)(sp.rest[0] * sp.segs[0] + sp.rest[1] * sp.segs[1]) * kBM * kBN;
 }
 
 // y[M, N] += x[M, K] . w[N, K]^T, each element rounded once; ws: dx_gemm256_add_floats floats, 16-byte aligned.  Same
@@ -571,15 +589,15 @@ extern "C" int dx_gemm256_add(void* y, int64_t ldy, const void* x, int64_t ldx, 
       (reinterpret_cast<uintptr_t>(y) & 7) || (reinterpret_cast<uintptr_t>(ws) & 15))
     return 5;
   if ((int64_t)N * K >= (1ll << 31) || (int64_t)kBM * ldx >= (1ll << 31)) return 6;  // 32-bit DMA offsets
-  Split sp{reinterpret_cast<f32x4*>(ws), 0, 0, 0};
-  add_split(M, N, K, &sp.full, &sp.rest, &sp.segs);
-  if (sp.rest && !ws) return 5;
-  const int grid = std::max(std::min(sp.full, num_cus()), sp.rest * sp.segs);
+  Split sp = add_split(M, N, K);
+  sp.part = reinterpret_cast<f32x4*>(ws);
+  if (sp.rest[0] && !ws) return 5;
+  const int grid = std::max({std::min(sp.full, num_cus()), sp.rest[0] * sp.segs[0], sp.rest[1] * sp.segs[1]});
   auto* Y = static_cast<bf16_t*>(y);
   hipLaunchKernelGGL((gemm256_kernel<EPI_ADD, false>), dim3(grid), dim3(512), 0, st, Y, ldy, static_cast<const bf16_t*>(x),
                      ldx, static_cast<const bf16_t*>(w), M, N, K, group_m, nullptr, GroupMap{nullptr, nullptr, 0, 1, 0, 0}, sp);
-  if (sp.rest)
-    hipLaunchKernelGGL(gemm256_join_kernel, dim3(16, sp.rest), dim3(256), 0, st, Y, ldy, M, N, group_m, sp);
+  if (sp.rest[0])
+    hipLaunchKernelGGL(gemm256_join_kernel, dim3(16, sp.rest[0] + sp.rest[1]), dim3(256), 0, st, Y, ldy, M, N, group_m, sp);
   DX_CHECK_LAUNCH();
   return 0;
 }

@@ -50,6 +50,32 @@ def test_add_after_add(M, N, K, pieces):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,left,pieces", [
+    (2100, 4096, 7168, 16, 16),  # no whole tile
+    (6151, 4096, 7296, 16, 16),  # a round in front; 57 pairs of K tiles in 16 pieces
+    (16500, 512, 7168, 2, 16),  # a workgroup without a second piece
+    (22728, 512, 10240, 50, 5),
+])
+def test_add_two_kinds(M, N, K, left, pieces):
+    """A last round of more than half of the CUs: 128 tiles in two pieces of K, the others in more."""
+    torch.manual_seed(M)
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    y0 = torch.randn(M, N + 4, device="cuda").bfloat16()
+    floats = ops._k().gemm256_add_floats(M, N, K)
+    assert floats == (128 * 2 + left * pieces) * 65536
+    outs = []
+    for _ in range(2):
+        y = y0.clone()
+        ws = torch.full((floats,), float("nan"), device="cuda")
+        ops._k().gemm256_add(y.data_ptr(), y.stride(0), x.data_ptr(), K, w.data_ptr(), M, N, K, 16, ws.data_ptr(), ops._stream())
+        outs.append(y)
+    assert torch.equal(*outs) and torch.equal(outs[0][:, N:], y0[:, N:])
+    want = torch.addmm(y0[:, :N].double(), x.double(), w.double().t())
+    # as above
+    assert bool(((outs[0][:, :N].double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -22 * K).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [500, 1280, 1300, 4200])
 def test_linear_add(M):
     """The op on both sides of its rule, and rows whose alignment the kernel does not take."""
