@@ -454,6 +454,15 @@ __global__ void __launch_bounds__(kThreads) decode_attn_kernel(
 // contiguous dims: dim block 4g + s), V before the LDS store (the image and
 // the transposed reads stay bf16); half the bytes per token.
 // The epilogue and the flash-decoding partitions are the VALU kernel's.
+// A wave's last chunk goes apart from its loop, whose loads then lie in no
+// branch: behind one the compiler did not know how many are on their way, and
+// the wait for a chunk's V rows was one for the next chunk's K rows too, a whole
+// latency in every chunk.  32 / 8 heads, layers in a graph, us: bf16, four of 40
+// sequences of 3000 tokens 256 -> 229 (5.0 -> 5.6 TB/s), two of 96 of 3150 278 ->
+// 256, eight of one of 700 61.5 -> 58.5; e4m3, two of 96 of 3150 153 -> 149, of 75
+// of 500 37 -> 35; 64 / 8 heads, bf16, two of 48 of 3000 149 -> 137.  Two
+// workgroups a CU, which is what the registers give: bounded to the 168 of three,
+// 40 of 3000 254, 38 of 5000 171 -> 197.
 constexpr int MCH = 32;  // tokens per wave chunk
 
 __device__ __forceinline__ int vimg_off(int row, int ch) {  // byte offset of 16-B chunk ch of row in a wave's image
@@ -579,15 +588,10 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
     }
   };
 
-  int c = wid;
-  if (c < n_chunks) {
-    load_k(c);
-    load_v(c);
-  }
-  for (; c < n_chunks; c += 4) {
-    const bool more = c + 4 < n_chunks;  // wave-uniform
+  auto step = [&](auto more_, int c) {
+    constexpr bool more = decltype(more_)::value;  // the wave has another chunk behind this one
     const int cb = p0 + c * MCH;
-    const bool partial = cb + MCH > p1;
+    const bool partial = !more && cb + MCH > p1;  // (the part's last chunk)
     // S = K . Q^T, two 16-token row blocks
     f32x4 sacc[2];
 #pragma unroll
@@ -598,7 +602,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
         sacc[bb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kfrag(bb, s2), __builtin_bit_cast(bf16x8_t, qf[s2]),
                                                            sacc[bb], 0, 0, 0);
     }
-    if (more) load_k(c + 4);
+    if constexpr (more) load_k(c + 4);
     // V rows of this chunk -> the wave's LDS image (rows past the context zeroed:
     // their P is 0, but stale cache bytes may be NaN)
     if (partial) {
@@ -614,7 +618,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
         *reinterpret_cast<u32x4_t*>(vimg + vimg_off(4 * k + g, r)) = vr[k];
       }
     }
-    if (more) load_v(c + 4);
+    if constexpr (more) load_v(c + 4);
     // softmax: lane (g, r) holds tokens 8g + j (j = 4 bb + i) of head r
     float t[8];
 #pragma unroll
@@ -655,6 +659,13 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
       const i16x8 vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pfrag, oacc[db], 0, 0, 0);
     }
+  };
+  int c = wid;
+  if (c < n_chunks) {
+    load_k(c);
+    load_v(c);
+    for (; c + 4 < n_chunks; c += 4) step(std::true_type{}, c);
+    step(std::false_type{}, c);
   }
 
   // wave state -> LDS: lane (g, r < G) holds dims 16 db + 4 g + i of head r;
