@@ -429,7 +429,7 @@ __global__ void __launch_bounds__(kThreads) decode_attn_kernel(
 // 16 q / 2 kv heads, or 70B at TP1) it is issue-bound at 3.3-3.8 TB/s.  Here
 // both products run on the matrix pipe and the VALU only does the softmax:
 //   * a wave takes 32-token chunks (every 4th); the G heads are the 16 columns
-//     of v_mfma_f32_16x16x32_bf16 (padded with zero Q rows);
+//     of v_mfma_f32_16x16x32_bf16 (the last head's again behind them);
 //   * S = K . Q^T as two 16-token row blocks: K is the A operand straight from
 //     global memory (lane = token row, 4 lanes x 64 contiguous bytes per row
 //     per load), Q the B operand (dims permuted identically: k-step s, lane
@@ -510,11 +510,8 @@ __global__ void __launch_bounds__(kThreads) decode_attn_mfma_kernel(
   auto dblk = [&](int s) { return F8 ? 4 * g + s : 4 * s + g; };
   u32x4_t qf[4];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    qf[s] = u32x4_t{0u, 0u, 0u, 0u};
-    if (r < G)
-      qf[s] = *reinterpret_cast<const u32x4_t*>(q + (int64_t)b * q_stride + (int64_t)(kvh * G + r) * D + 8 * dblk(s));
-  }
+  for (int s = 0; s < 4; ++s)  // (columns behind the heads hold the last one's, and go nowhere: a branch here was a latency for each s)
+    qf[s] = *reinterpret_cast<const u32x4_t*>(q + (int64_t)b * q_stride + (int64_t)(kvh * G + min(r, G - 1)) * D + 8 * dblk(s));
   const int part_size = balanced_part(ctx, n_parts, 4 * MCH);
   const int p0 = pid * part_size;
   if (p0 >= ctx) return;
@@ -713,13 +710,11 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
   const int np = min((ctx + part_size - 1) / part_size, n_parts);
   float M = lane < np ? first.x : -1e30f;
   for (int p = lane + 64; p < np; p += 64) M = fmaxf(M, ml[p].x);
-#pragma unroll
-  for (int d = 32; d; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
+  M = wave_reduce_max(M);
   const float w0 = lane < np ? exp2f(first.x - M) * first.y : 0.f;
   float den = w0;
   for (int p = lane + 64; p < np; p += 64) den += exp2f(ml[p].x - M) * ml[p].y;
-#pragma unroll
-  for (int d = 32; d; d >>= 1) den += __shfl_xor(den, d, 64);
+  den = wave_reduce_sum(den);
   f32x4 num = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < AHEAD; ++k) {
@@ -736,7 +731,7 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
       if (p < np) num += w * y;
     }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) num[i] += __shfl_xor(num[i], 32, 64);
+  for (int i = 0; i < 4; ++i) num[i] = over_halves(num[i], [](float x, float y) { return x + y; });
   if (grp == 2) other[threadIdx.x & 31] = num;
   __syncthreads();
   if (grp) return;

@@ -68,15 +68,29 @@ __device__ __forceinline__ void landed() {
   __syncthreads();
 }
 
+// over a wave, every lane with the lane 32, 16, 8, 4, 2 and 1 from it, by exchanges in registers (all lanes on): the six LDS
+// permutes of __shfl_xor took some 700 cycles, a part of every small kernel's time (a launch of 3 to 5 us)
+template <int CTRL> __device__ __forceinline__ float row_dpp(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, false));
+}
+template <typename F> __device__ __forceinline__ float over_halves(float v, F f) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <typename F> __device__ __forceinline__ float over_wave(float v, F f) {
+  v = over_halves(v, f);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = f(v, row_dpp<0x128>(v));  // row_ror:8
+  v = f(v, row_dpp<0x124>(v));  // row_ror:4 (4 or 12 lanes on, which hold the same by now)
+  v = f(v, row_dpp<0x4E>(v));   // quad_perm
+  return f(v, row_dpp<0xB1>(v));
+}
 __device__ __forceinline__ float wave_reduce_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return over_wave(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_reduce_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return over_wave(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide sum for blockDim.x <= 1024 (16 waves). `red` must hold >= 16 floats.

@@ -233,6 +233,9 @@ __global__ void __launch_bounds__(256) merge_parts_kernel(PartSums<OutT, GT> a, 
       x1[k] = dv > 128 ? *reinterpret_cast<const float2*>(wp + e1) : float2{0.f, 0.f};
     }
   };
+  // lane p: part p (of 64 at a time; asked for in front of the columns, so that its factor is formed while they come)
+  const float* mine = w + (int64_t)min(lane, parts - 1) * step;
+  const float m1 = mine[0], l1 = mine[1];
   if (pairs) columns(0, parts - 1);
   float post = 1.f;
   if (gate) {
@@ -240,10 +243,9 @@ __global__ void __launch_bounds__(256) merge_parts_kernel(PartSums<OutT, GT> a, 
     const int head = (int)(v - row * n_qh) / maps;
     post /= 1.f + expf(-Elem<GT>::ld(gate, row * gs + head));
   }
-  // lane p: part p (of 64 at a time); parts without a key have sum 0 and count for nothing (those alone: a part that saw a NaN
-  // has a NaN for its sum, which makes the row one)
-  float m0 = -INFINITY, l0 = 0.f;
-  if (lane < parts) m0 = w[(int64_t)lane * step], l0 = w[(int64_t)lane * step + 1];
+  // parts without a key have sum 0 and count for nothing (those alone: a part that saw a NaN has a NaN for its sum, which makes
+  // the row one)
+  const float m0 = lane < parts ? m1 : -INFINITY, l0 = lane < parts ? l1 : 0.f;
   float mx = m0;
   for (int p = lane + 64; p < parts; p += 64) mx = fmaxf(mx, w[(int64_t)p * step]);
   mx = wave_reduce_max(mx);
