@@ -504,13 +504,18 @@ __global__ void __launch_bounds__(128) conv_run_kernel(ConvArgs g, T* __restrict
     live = slot >= 0 && slot < g.n_slots && r0 >= 0 && r0 <= t;
     if (M == 0 || !live) return;
     const T* tl = tail + (int64_t)slot * M * C + c;
-    const int64_t p = g.pos[t];
+    raw_u32x4 was[M > 0 ? M : 1];
 #pragma unroll
     for (int m = 0; m < M; ++m) {  // h[m]: the input at position p - M + m
-      const int back = M - m, rel = t - r0 - back;  // its row in this step's run of the sequence
+      const int rel = t - r0 - (M - m);  // its row in this step's run of the sequence
+      was[m] = *reinterpret_cast<const raw_u32x4*>(rel >= 0 ? x + (int64_t)(r0 + rel) * g.xs : R == 1 ? tl + (int64_t)(rel + M) * C : x + (int64_t)t * g.xs);
+    }
+    const int64_t p = g.pos[t];
 #pragma unroll
-      for (int e = 0; e < V; ++e) h[m][e] = 0.f;
-      if (p >= back && (R == 1 || rel >= 0)) VecIO<T, V>::ld(rel >= 0 ? x + (int64_t)(r0 + rel) * g.xs : tl + (int64_t)(rel + M) * C, h[m]);
+    for (int m = 0; m < M; ++m) {  // (asked for whether they count or not: behind a branch they came one after the other)
+      const int back = M - m;
+      if (!(p >= back && (R == 1 || t - r0 - back >= 0))) was[m] = raw_u32x4{0u, 0u, 0u, 0u};
+      chunk_to_f32<T>(was[m], h[m]);
     }
   };
   enter(t0);
