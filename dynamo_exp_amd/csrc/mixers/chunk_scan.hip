@@ -300,6 +300,7 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
   f32x4 S[NM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) S[m] = w.fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + 16 * m);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): here once, not in every turn, where it would be one for the last turn's stores
   const float qsc = g.q_scale;
   const int p = 16 * wave + c16;
   const int64_t ow = (int64_t)g.H * g.dv;
@@ -405,7 +406,8 @@ __global__ void __launch_bounds__(512, 2) chunk_scan_kernel(ScanArgs g) {
 // order of the k-slots (slot_of32), so that every fragment is one 16-byte read.
 // Bound by the chain of the longest sequence's chunks, in it by the forming waves' elementwise work and the product waves'
 // latencies: the state's update without a branch per 16 channels 175 -> 167 us (32 heads of 128 / 128, 4001 tokens in three
-// prompts; with the norm 190 -> 183).
+// prompts; with the norm 190 -> 183); rows asked for together, and no wait for loads or stores at the chunks' barriers, with
+// the norm 175 -> 173, one prompt of 4000 317 -> 313, six of 5000 together 150 -> 148.
 template <int DK> struct ChannelBuf {
   static constexpr int KP = DK + 8, SP = 40;
   bf16_t qi[2][32 * KP];  // hi, lo of q e^L                  [t][n]
@@ -464,14 +466,18 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
     for (int e = 0; e < 8; ++e) bias[e] = zb && has_k ? zb[8 * oc + e] : 0.f;
     raw_u32x4 rq, rk, rz, rv;
     bool live = false;
+    // (through descriptors, zeros where there is nothing: behind branches the four came one after the other)
     auto fetch = [&](int t0) {
-      const raw_u32x4 zero{0u, 0u, 0u, 0u};
-      const int64_t t = t0 + tok;
-      live = t < w.n;
-      rz = live && has_k ? *reinterpret_cast<const raw_u32x4*>(z + t * g.gs + 8 * oc) : zero;
-      rq = live && has_k ? *reinterpret_cast<const raw_u32x4*>(q + t * g.qs + 8 * oc) : zero;
-      rk = live && has_k ? *reinterpret_cast<const raw_u32x4*>(k + t * g.ks + 8 * oc) : zero;
-      rv = live && has_v ? *reinterpret_cast<const raw_u32x4*>(v + t * g.vs + 8 * ov) : zero;
+      live = t0 + tok < w.n;
+      auto row = [&](const bf16_t* p, int64_t stride, int col, bool has) {
+        const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)(p + t0 * stride), 0, 0x80000000u, 0x00020000);
+        return __builtin_bit_cast(raw_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+            r, live && has ? 2u * (uint32_t)(tok * (int)stride + col) : 0x80000000u, 0, 0));
+      };
+      rz = row(z, g.gs, 8 * oc, has_k);
+      rq = row(q, g.qs, 8 * oc, has_k);
+      rk = row(k, g.ks, 8 * oc, has_k);
+      rv = row(v, g.vs, 8 * ov, has_v);
     };
     auto form = [&](Buf& b) {
       bool far = false;
@@ -532,7 +538,7 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
     form(bufs[0]);
     fetch(Q);
     for (int t0 = 0, cur = 0; t0 < w.n; t0 += Q, cur ^= 1) {
-      __syncthreads();  // chunk t0 is formed; the other half is consumed
+      lds_barrier();  // chunk t0 is formed; the other half is consumed
       if (t0 + Q < w.n) {
         form(bufs[cur ^ 1]);
         fetch(t0 + 2 * Q);
@@ -547,6 +553,7 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
   f32x4 S[NM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) S[m] = w.fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + 16 * m);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): here once, not in every turn, where it would be one for the last turn's stores
   auto pair_by_pair = [&](int t0, int st, int tt, f32x4& a) {  // a[r] = sum_n q_t k_s E(s, t), s = 16 st + 4 g4 + r, t = 16 tt + c16
     a = f32x4{0.f, 0.f, 0.f, 0.f};
     const int tl = 16 * tt + c16, s_lo = 16 * st + 4 * g4;
@@ -567,7 +574,7 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
     }
   };
   for (int t0 = 0, cur = 0; t0 < w.n; t0 += Q, cur ^= 1) {
-    __syncthreads();  // this chunk is formed
+    lds_barrier();  // this chunk is formed
     const Buf& b = bufs[cur];
     int far[8], any_far = 0;
 #pragma unroll
@@ -666,8 +673,8 @@ bool chunk_scan_ok(int mode, const ScanArgs& g) {
   return (g.dk == 32 || g.dk == 64 || g.dk == 128) && g.dv % kPB == 0 && g.qs % 8 == 0 && g.ks % 8 == 0 &&
          g.vs % 8 == 0 && al(g.q) && al(g.k) && al(g.v) && al(g.state) && al(g.out) &&
          // (a chunk of 64 rows: inputs within 31-bit, results within 32-bit byte offsets)
-         (mode == kChannel ? g.gs % 8 == 0 && al(g.g) && !g.skip
-                           : (int64_t)g.H * g.dv <= (1 << 24) && std::max({g.qs, g.ks, g.vs, mode == kStep ? g.gs : 0}) <= (1 << 24));
+         std::max({g.qs, g.ks, g.vs, mode == kFixed ? 0 : g.gs}) <= (1 << 24) &&
+         (mode == kChannel ? g.gs % 8 == 0 && al(g.g) && !g.skip : (int64_t)g.H * g.dv <= (1 << 24));
 }
 
 #define CHUNK_DK(KERNEL, NT)                                                  \
