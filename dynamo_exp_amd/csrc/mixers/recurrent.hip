@@ -92,7 +92,9 @@ __global__ void __launch_bounds__(NT) delta_rule_kernel(DeltaArgs g) {
 // Bound by memory from some 40 sequences on, by latency below.  Two layers with their norms in a graph, 32 heads of 128 columns,
 // 1 / 3 / 12 / 40 / 128 sequences, us: 25 / 30 / 49 / 114 / 278 with delta_prep_kernel in front and the kernel for runs of
 // tokens, 21 / 21 / 33 / 89 / 231 like this with the lines kept; that kernel forming the rows itself 20 / 26 / 46 / 128 / 330, for it
-// stages eight tokens.  With the state's lines not kept (ONCE: state_once) 64 take 107 instead of 128.
+// stages eight tokens.  With the state's lines not kept (ONCE: state_once) 64 take 107 instead of 128.  With everything asked
+// for together, layers with their norms, four of 4 sequences 38.6 -> 36.3, of 16 69.7 -> 64.5, two of 40 65.5 -> 61.9, of 64
+// 104 -> 101, three of 30 of 16 heads 50.9 -> 46.2; 128 unchanged.
 constexpr int kDeltaStepLanes = 8;
 bool delta_forms_itself(const int* seq_rows, int dk) { return !seq_rows && dk == kDeltaStepLanes * kRows; }
 
@@ -112,29 +114,38 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaArgs g) {
   }
   // the wave's row: k for the first and the third one, the decay's or the read-out's else
   const T* src = wave == 1 ? (const T*)g.w + t * g.wst : wave == 3 ? (const T*)g.r + t * g.rs : (const T*)g.k + t * g.ks;
+  const T* src2 = wave == 2 ? (const T*)g.a + t * g.as : src;
   const float* bias = wave == 1 ? g.w_bias : wave == 2 ? g.a_bias : nullptr;
-  float x[2], bv[2] = {0.f, 0.f}, al[2] = {0.f, 0.f};
+  const float* some = bias ? bias : g.state;  // (as long as a row of biases at least)
+  // Everything is asked for together, whether it counts or not (a column behind the last one is the last one again, and goes
+  // nowhere): behind a branch each load was waited for before the next one went out, five latencies in a row.
+  float x[2], bv[2], al[2], vj[CT];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     const int ch = h * D + lane + 64 * c;
     x[c] = ldf<T>(src, ch);
-    if (wave == 2) al[c] = ldf<T>((const T*)g.a + t * g.as, ch);
-    if (bias) bv[c] = bias[ch];
+    al[c] = ldf<T>(src2, ch);
+    bv[c] = some[ch];
   }
-  float vj[CT];
 #pragma unroll
-  for (int c = 0; c < CT; ++c) vj[c] = j0 + c < g.dv ? ldf<T>((const T*)g.v + t * g.vs + h * g.dv, j0 + c) : 0.f;
+  for (int c = 0; c < CT; ++c) vj[c] = ldf<T>((const T*)g.v + t * g.vs + h * g.dv, min(j0 + c, g.dv - 1));
   // rows 4 (m R + part) .. + 3 of the state's columns, as delta_tokens holds them
   float* sp = g.state + (((int64_t)slot * g.H + h) * g.dv + j0) * D + 4 * part;
+  f32x4 y[CT][kRows / 4];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int m = 0; m < kRows / 4; ++m) y[c][m] = load_state<ONCE>(sp + (min(j0 + c, g.dv - 1) - j0) * D + 4 * m * R);
   const bool fresh = g.pos[t] == 0;
   float S[CT][kRows];
 #pragma unroll
   for (int c = 0; c < CT; ++c)
 #pragma unroll
-    for (int m = 0; m < kRows / 4; ++m) {
-      const f32x4 y = fresh || j0 + c >= g.dv ? f32x4{0.f, 0.f, 0.f, 0.f} : load_state<ONCE>(sp + c * D + 4 * m * R);
-      S[c][4 * m] = y[0], S[c][4 * m + 1] = y[1], S[c][4 * m + 2] = y[2], S[c][4 * m + 3] = y[3];
-    }
+    for (int m = 0; m < kRows / 4; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[c][4 * m + i] = fresh ? 0.f : y[c][m][i];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) bv[c] = bias ? bv[c] : 0.f;
   if (wave == 1) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) row[1][lane + 64 * c] = delta_decay(x[c], bv[c], g.decay_scale);
