@@ -77,20 +77,24 @@ template <typename F> __device__ __forceinline__ float over_halves(float v, F f)
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-template <typename F> __device__ __forceinline__ float over_wave(float v, F f) {
-  v = over_halves(v, f);
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+// (N: aligned groups of so many lanes, 16 or more)
+template <int N, typename F> __device__ __forceinline__ float over_lanes(float v, F f) {
+  static_assert(N == 16 || N == 32 || N == 64, "whole rows of lanes");
+  if constexpr (N == 64) v = over_halves(v, f);
+  if constexpr (N >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
   v = f(v, row_dpp<0x128>(v));  // row_ror:8
   v = f(v, row_dpp<0x124>(v));  // row_ror:4 (4 or 12 lanes on, which hold the same by now)
   v = f(v, row_dpp<0x4E>(v));   // quad_perm
   return f(v, row_dpp<0xB1>(v));
 }
 __device__ __forceinline__ float wave_reduce_sum(float v) {
-  return over_wave(v, [](float a, float b) { return a + b; });
+  return over_lanes<64>(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_reduce_max(float v) {
-  return over_wave(v, [](float a, float b) { return fmaxf(a, b); });
+  return over_lanes<64>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide sum for blockDim.x <= 1024 (16 waves). `red` must hold >= 16 floats.

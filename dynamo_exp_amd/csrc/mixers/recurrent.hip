@@ -667,6 +667,8 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // whe
 // elements each, so a wave works on 64 / LPH heads.  Bound by memory, and by the latency of loads behind one another: the
 // weights' are asked for in front of the sum like the others.  4001 rows of 32 heads of 128 with weights and a gate, us: 36.8
 // with the weights behind the sum, 30.9 in front, 24.9 (5.3 TB/s) in runs of eight bf16; heads of 256 67.0, 55.3, 43.7.
+// Decode steps, four layers of retention of 4 sequences with the sum by LDS permutes and the row by a division in 64 bits 34.9
+// us, now 34.2, of one 27.2 and 26.4.
 template <typename T, int LPH, int E>
 __global__ void __launch_bounds__(256) head_norm_gate_vec_kernel(T* __restrict__ out, const float* __restrict__ o,
                                                                  const float* __restrict__ w, const T* __restrict__ gate,
@@ -676,7 +678,8 @@ __global__ void __launch_bounds__(256) head_norm_gate_vec_kernel(T* __restrict__
   const int e = (threadIdx.x % LPH) * E;
   if (v >= n_vec) return;  // (whole lane groups)
   const bool on = e < dv;
-  const int64_t row = v / H;
+  // (in 32 bits where the numbers are: a division in 64 is some 150 instructions in front of the gate's loads)
+  const int64_t row = n_vec <= 0xffffffffll ? (int64_t)((uint32_t)v / (uint32_t)H) : v / H;
   const int c = (int)(v - row * H) * dv + e;  // column of the row
   float x[E] = {}, z[E] = {}, u[E];
 #pragma unroll
@@ -703,8 +706,12 @@ __global__ void __launch_bounds__(256) head_norm_gate_vec_kernel(T* __restrict__
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < E; ++i) ss += x[i] * x[i];
+  if constexpr (LPH >= 16) {
+    ss = over_lanes<LPH>(ss, [](float a, float b) { return a + b; });
+  } else {
 #pragma unroll
-  for (int m = LPH / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    for (int m = LPH / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  }
   const float inv = rsqrtf(ss / (float)dv + eps);
   if (!on) return;
   float y[E];
