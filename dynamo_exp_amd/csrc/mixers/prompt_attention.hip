@@ -29,8 +29,9 @@
 //     stood in each other's way.
 //   * Score terms: the tanh cap is a polynomial of degree 5 or 7 where a tile's scores are small against the cap (|x / cap| <
 //     0.17 or 0.36, relative error 2.3e-7; exp2 and reciprocal elsewhere), and where a row sees at most 1216 keys back the
-//     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.  With the table a
-//     row's newest keys come first: new maxima (64 multiplications a tile, of some 270 instructions) end with them.
+//     log-distance penalty is a table of the distance in LDS: of four transcendentals a score one is left.  The keys
+//     stay in order: with the newest first the maximum soon stands and 4500 rows of a window of 1024 take 91 us rather than 98,
+//     but the largest weight of most tiles is no longer 1, and the error against 64 bits grows by 0.5 to 2 %.
 //   * Few rows behind a long context leave most of the chip idle, and a workgroup alone on its CU takes 0.5 to 1 us for 32
 //     keys, whatever it does with them: there the keys go out in parts (dxm_prompt_attention_parts, grid z), whose sums
 //     merge_parts joins.  One prompt of 16 rows behind 2000 keys, 32 heads, us of the GPU: causal 41 -> 13, two maps in
@@ -41,8 +42,8 @@
 // 1.25 x slower), and a wave's issue where there are score terms.  32 heads, ragged prompts of about 4000 tokens, us,
 // before -> now: two maps with values of 256, window 1024 + 64, 5003 rows beside 16 decode rows, with the combine: 288 -> 270;
 // shared row 256 / 192 causal, tiles of 32 keys -> 64, 4203 rows 111 -> 101 (970 TFLOP/s), 600 rows 25.3 -> 21.8, window 1024,
-// 1500 rows 47 -> 43; cap + penalty, window 1024, keys in order and degree 7 -> the newest first and degree 5, 4500 rows 95 -> 87,
-// 3000 of 16 heads 47 -> 43, 600 rows behind 2000 cached, window 512, 26.6 -> 24.9 (its error against 64 bits 1.95e-3 -> 1.96e-3);
+// 1500 rows 47 -> 43; cap + penalty, window 1024, degree 7 -> 5, 4500 rows 99 -> 97, 3000 of
+// 16 heads 52.1 -> 50.5, 600 rows behind 2000 cached, window 512, 25.6 -> 25.3 (its error against 64 bits unchanged);
 // sigmoid 85 -> 78.  (The register-staged 16x16x32 forms
 // of tile_attention.hip, stream and latent prefill, which it took over from: two maps and their combine 776, 242, 313.)
 #include <algorithm>
@@ -86,7 +87,6 @@ constexpr int kLeastTiles = 4;  // of a part, of several
 // kTable: cap and / or penalty where a row sees at most kTableKeys keys back: the penalty is a table of the distance in LDS
 enum { kPlain = 0, kTerms = 1, kSigmoid = 2, kTable = 3 };
 constexpr int kTableKeys = 1216;  // what three workgroups of a CU have room for beside their tiles
-constexpr int kExact = 8;         // tiles of a row's newest keys whose largest weight is exactly 1
 constexpr int kTablePad = 64;     // entries for keys of a tile that a row does not see, on both sides
 
 // tanh(y) / y = sum kTanh[i] y^(2 i) for |y| <= kTanhMax (minimax, fitted in 64 bits; relative error of these floats 6.2e-8, of
@@ -102,12 +102,6 @@ __device__ __forceinline__ void opaque(int& x) { asm("" : "+v"(x)); }
 // assembly it does not wait for the matrix product that an operand comes from.
 __device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 __device__ __forceinline__ float max3(float a, float b, float c) { return max2(max2(a, b), c); }
-// x + the two bf16 of w
-__device__ __forceinline__ float sum_of_pair(uint32_t w, float x) {
-  uint32_t ones = 0x3f803f80u;  // (in a register: of some constants the encoding takes only one half)
-  asm("" : "+s"(ones));
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, ones), x, false);
-}
 // a number that is the same in every lane, in a scalar register
 __device__ __forceinline__ float uniform(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
 __device__ __forceinline__ float swap_max(float x) {
@@ -138,10 +132,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   // heads lose 2 to 5 % with each of them.
   enum { kNothing, kVectors, kValues, kProducts };
   constexpr int kRaised = SAME ? kValues : MODE == kSigmoid ? kProducts : MODE != kPlain || DV == 256 ? kVectors : kNothing;
-  // A penalty that grows with the distance: the newest keys first, whose scores are a row's largest.  Behind them the maximum
-  // hardly moves, and from kExact tiles on it stays where it is for scores that exceed it a little (their weights, over 1, are
-  // then rounded like any other, and summed as rounded).
-  constexpr bool kBack = MODE == kTable;
+  constexpr float kDefer = 8.f;  // pairs of products: log2 units that a score may exceed the running maximum by
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -210,7 +201,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   auto find = [&](int t) {
     const int j = t << SH, page = j >> a.bs_shift;
     if (page - page0 >= 64 || page < page0) {
-      page0 = kBack ? max(page - 63, 0) : page;
+      page0 = page;
       pages = bt[min(page0 + lane, hi >> a.bs_shift)];
       __builtin_amdgcn_s_waitcnt(0x0f70);  // (here and now: behind the branch it would be waited for, and the DMA, at every tile)
     }
@@ -257,7 +248,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     const i16x4 up = read_tr16((const lds_i16x4*)(uintptr_t)(vp + 8 * VB + (v_at ^ 64 * (f % NC & 3) ^ 32)));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  auto step = [&](auto bufc, int t, float defer) {
+  auto step = [&](auto bufc, int t) {
     constexpr uint32_t kb = decltype(bufc)::value * kStage, vb = SAME ? kb : kb + kKey;  // from the front
     constexpr uint32_t other = (1 - decltype(bufc)::value) * kStage;                     // the next tile's
     const int kt = t << SH;
@@ -381,7 +372,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       }
       // both halves of a row see the same maximum and take the same decision
       const float tm = swap_max(fmaxf(ta, tb)) * sc;
-      const float mn = tm > (FINE || kBack ? m_i + defer : m_i) ? tm : m_i;
+      const float mn = tm > (FINE ? m_i + kDefer : m_i) ? tm : m_i;
       mu = mn == -INFINITY ? 0.f : mn;  // a row that has seen nothing yet
       if (__builtin_amdgcn_ballot_w64(mn != m_i)) {
         const float alpha = fast_exp2(m_i - mu);
@@ -407,9 +398,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
           else
             w[x] = fast_exp2(fmaf(v, sc, -mu));
         }
-        if constexpr (MODE != kSigmoid && !kBack) l_i += w[0] + w[1];
+        if constexpr (MODE != kSigmoid) l_i += w[0] + w[1];
         ph[k16 & 1][e] = pack_bf16x2(w[0], w[1]);
-        if constexpr (kBack) l_i = sum_of_pair(ph[k16 & 1][e], l_i);
         if constexpr (FINE) pl[k16 & 1][e] = pack_bf16x2(w[0] - bf16lo(ph[k16 & 1][e]), w[1] - bf16hi(ph[k16 & 1][e]));
       }
     };
@@ -434,11 +424,8 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     if constexpr (kRaised == kValues) __builtin_amdgcn_s_setprio(0);
   };
   auto tile = [&](int i) {
-    if constexpr (kBack) return first + i0 + i1 - 1 - i;  // (this form has no kept keys)
     return i < kept ? i : first + i - kept;
   };
-  // log2 units that a score may exceed the running maximum by
-  auto defer = [&](int i) { return FINE || (kBack && i - i0 >= kExact) ? 8.f : 0.f; };
   static_assert(ND <= KS, "a DMA instruction beside a product at most");
   find(tile(i0));
 #pragma unroll
@@ -446,11 +433,11 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   landed();
   for (int i = i0; i < i1; i += 2) {  // (behind the last tile it is fetched again: no branch among the products)
     find(tile(min(i + 1, i1 - 1)));
-    step(std::integral_constant<int, 0>{}, tile(i), defer(i));
+    step(std::integral_constant<int, 0>{}, tile(i));
     landed();
     if (i + 1 < i1) {
       find(tile(min(i + 2, i1 - 1)));
-      step(std::integral_constant<int, 1>{}, tile(i + 1), defer(i + 1));
+      step(std::integral_constant<int, 1>{}, tile(i + 1));
       landed();
     }
   }

@@ -314,8 +314,7 @@ def test_score_terms_of_limited_distance(form, cap, mask, size):
 @pytest.mark.parametrize("form,cap", [("both", 30.0), ("both", 50.0), ("penalty", 0.0)])
 @pytest.mark.parametrize("old", [(), (100,), (100, 250, 640), (3, 4, 870)])
 def test_penalty_rows_whose_old_keys_count(form, cap, old):
-    """The newest keys come first: maxima among the first tiles, behind them (by less and by more than the maximum waits for),
-    in the last one; scores on both sides of what each polynomial of the cap takes."""
+    """Maxima among the first tiles, behind them and in the last one; scores on both sides of what each polynomial of the cap takes."""
     n_qh, maps, group, d, dv = FORMS[form]
     torch.manual_seed(13)
     scale, start, rows, bs, size = 0.7 * d ** -0.5, 900, 40, 64, 1000
@@ -331,7 +330,7 @@ def test_penalty_rows_whose_old_keys_count(form, cap, old):
     got = mx.attention(q.cuda(), kd, vd, torch.arange(start, start + rows).cuda(), torch.zeros(rows, dtype=torch.int32).cuda(),
                        table, bs, n_qh, maps, group, d, dv, scale, "window", size, 1, False, tiles, rows, softcap=cap,
                        dist_bias=tuple(map(cuda, db))).cpu().double()
-    # (bound of test_prompt_rows: weights over their own sum as rounded are 2^-9 off in each, 2^-8 of |v| < 5 together)
+    # (bound of test_prompt_rows)
     assert float((got - want).abs().max()) < 2.0 ** -8 * (float(want.abs().max()) + 5.0)
 
 
