@@ -22,9 +22,10 @@
 //   * Wide shared rows (256 value columns): the upper half of the queries stays in LDS, the accumulators need its
 //     registers.
 //   * Tiles of 64 keys, or of 32 where that lets more workgroups onto a CU: values of 256 columns, and the forms with
-//     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.  (Most tiles hold a
-//     new maximum for one of a wave's 32 rows, and every one costs a multiplication of each accumulator: half as many of them
-//     is what shared rows of 192 value columns gain from 64 keys.)
+//     score terms or sigmoid weights, whose vector work hides behind three waves a SIMD rather than two.  Shared rows of 192
+//     value columns take 32 for their exactness: with 64 they are 8 % faster (half as many tiles raise a maximum, which
+//     costs a multiplication of each accumulator: 4203 rows 107.5 -> 98.8 us, 600 23.8 -> 21.7), but half as many hold a weight
+//     that is 1, and the error against 64 bits grows by 0.5 % (1.919e-3 -> 1.927e-3, 1.928e-3 -> 1.938e-3).
 //   * Between the products of a tile's scores the next tile's DMA goes out; all four waves' at once behind the barrier
 //     stood in each other's way.
 //   * Score terms: the tanh cap is a polynomial of degree 5 or 7 where a tile's scores are small against the cap (|x / cap| <
@@ -41,8 +42,7 @@
 // forming a tile's scores between the weights of the one in front needs 16 registers more than there are, and spills:
 // 1.25 x slower), and a wave's issue where there are score terms.  32 heads, ragged prompts of about 4000 tokens, us,
 // before -> now: two maps with values of 256, window 1024 + 64, 5003 rows beside 16 decode rows, with the combine: 288 -> 270;
-// shared row 256 / 192 causal, tiles of 32 keys -> 64, 4203 rows 111 -> 101 (970 TFLOP/s), 600 rows 25.3 -> 21.8, window 1024,
-// 1500 rows 47 -> 43; cap + penalty, window 1024, degree 7 -> 5, 4500 rows 99 -> 97, 3000 of
+// shared row 256 / 192 causal 125 -> 113 (870 TFLOP/s); cap + penalty, window 1024, degree 7 -> 5, 4500 rows 99 -> 97, 3000 of
 // 16 heads 52.1 -> 50.5, 600 rows behind 2000 cached, window 512, 25.6 -> 25.3 (its error against 64 bits unchanged);
 // sigmoid 85 -> 78.  (The register-staged 16x16x32 forms
 // of tile_attention.hip, stream and latent prefill, which it took over from: two maps and their combine 776, 242, 313.)
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   constexpr int kKey = KT * KB, kStage = kKey + (SAME ? 0 : KT * VB);
   constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
-  constexpr int KA = MODE != kPlain ? 3 : SAME && SUBS == 2 ? (PARTS ? 2 : 3) : 4, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
+  constexpr int KA = MODE == kPlain ? 4 : 3, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
   // What a wave does at raised priority, where two or three share a SIMD.  Score terms and pairs of maps: everything but the
   // value products, which fill what the others' vector work leaves; shared rows, whose products are the longer part: the value
   // products; sigmoid weights: both products.  us, without / with (5003 rows of two maps beside 16, 3000 in chunks of 2048; 4203
@@ -423,9 +423,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     if constexpr (kRaised == kVectors) __builtin_amdgcn_s_setprio(1);
     if constexpr (kRaised == kValues) __builtin_amdgcn_s_setprio(0);
   };
-  auto tile = [&](int i) {
-    return i < kept ? i : first + i - kept;
-  };
+  auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
   static_assert(ND <= KS, "a DMA instruction beside a product at most");
   find(tile(i0));
 #pragma unroll
@@ -521,11 +519,11 @@ int launch_prompt(const PromptArgs& a, int n_tiles, hipStream_t st) {
 }
 
 // (tiles of 32 / 64 keys, us, launches back to back: cap + penalty 157 / 153, sigmoid 91 / 99, shared row 256 / 256
-// 128 / 182, 256 / 192 causal 120 / 113, 600 rows 24.5 / 22.0, 40 behind 2900 cached 24.4 / 22.3, two maps 265 / 350, plain of 5000 149 / 154 and of 40 behind
+// 128 / 182, 256 / 192 causal 120 / 113 and of 600 rows 24.5 / 22.0 (less exact: above), two maps 265 / 350, plain of 5000 149 / 154 and of 40 behind
 // 2900 cached 94 / 83, fine 179 / 186)
 template <int D, int DV, bool SAME, int MODE, bool FINE, typename OutT>
 int prompt_heads(const PromptArgs& a, int n_tiles, hipStream_t st) {
-  constexpr int SUBS = (DV == 128 && MODE == kPlain) || DV == 192 ? 2 : 1;
+  constexpr int SUBS = DV == 128 && MODE == kPlain ? 2 : 1;
   if (a.group % 4 == 0) return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 4, 4, SUBS>(a, n_tiles, st);
   return launch_prompt<D, DV, SAME, MODE, FINE, OutT, 2, 4, SUBS>(a, n_tiles, st);
 }

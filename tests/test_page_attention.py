@@ -335,6 +335,37 @@ def test_penalty_rows_whose_old_keys_count(form, cap, old):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [600, 1501])
+@pytest.mark.parametrize("form,keys", [("shared", 32), ("shared wide", 32), ("plain", 64)])
+def test_rounding_of_the_weights(form, keys, rows):
+    """A weight that enters its product as one bf16 is rounded relative to the maximum so far, so a row's largest weight in a
+    tile that raises it is exactly 1: with tiles of more keys there are fewer of those.  The distance from exact sums is
+    that of weights rounded tile by tile."""
+    n_qh, maps, group, d, dv = FORMS[form]
+    torch.manual_seed(17)
+    scale = d ** -0.5
+    kd, vd, table, ((K, V),) = pages(form, [rows], 64)
+    q = torch.randn(rows, n_qh * d).bfloat16().cuda()
+    tiles = torch.tensor(mx.tile_list(0, rows), dtype=torch.int32).cuda()
+    pos = torch.arange(rows).cuda()
+    got = mx.attention(q, kd, vd, pos, torch.zeros(rows, dtype=torch.int32).cuda(), table, 64, n_qh, maps, group, d, dv, scale,
+                       "causal", 0, 1, False, tiles, rows).double().view(rows, n_qh, dv).transpose(0, 1)
+    Q, K, V = (t.transpose(0, 1).contiguous() for t in (q.double().view(rows, n_qh, d), K.cuda(), V.cuda()))
+    S = ((Q @ K.transpose(1, 2).contiguous()) * scale).masked_fill(pos[None, None] > pos[None, :, None], float("-inf"))
+    want = torch.softmax(S, -1) @ V
+    m = torch.full((n_qh, rows, 1), float("-inf"), dtype=torch.float64, device="cuda")
+    l, O = torch.zeros_like(m), torch.zeros_like(want)
+    for at in range(0, rows, keys):
+        s = S[:, :, at:at + keys]
+        new = torch.maximum(m, s.amax(-1, keepdim=True))
+        w, fade = torch.exp(s - new), torch.exp(m - new)
+        l, O, m = l * fade + w.sum(-1, keepdim=True), O * fade + w.bfloat16().double() @ V[:, at:at + keys].contiguous(), new
+    far = lambda x: float((x - want).norm() / want.norm())
+    # (twice as many keys a tile: 0.5 % more; the kernel's own sums and exponentials are in 32 bits, 2^-14 of a rounding to bf16)
+    assert far(got) <= 1.002 * far((O / l).bfloat16().double()), (far(got), far((O / l).bfloat16().double()))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mask,size", [("causal", 0), ("chunk", 1500)])
 @pytest.mark.parametrize("form", ["shared", "plain", "diff", "sigmoid"])
 @pytest.mark.parametrize("ctx", [[4000, 33, 1, 2500, 700], [1, 3000], [300 + 61 * i for i in range(20)],
