@@ -125,13 +125,12 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   constexpr int KP = KT * KB / 1024 / NW, VP = SAME ? 0 : KT * VB / 1024 / NW;  // 1-KB pieces per wave
   constexpr int QR = SAME && DV == 256 ? 8 : KS;                      // query fragments in registers
   constexpr int KA = MODE == kPlain ? 4 : 3, VA = FINE ? 3 : MODE == kPlain ? 4 : 2;  // fragments asked for ahead of their products
-  // What a wave does at raised priority, where two or three share a SIMD.  Score terms and pairs of maps: everything but the
-  // value products, which fill what the others' vector work leaves; shared rows, whose products are the longer part: the value
-  // products; sigmoid weights: both products.  us, without / with (5003 rows of two maps beside 16, 3000 in chunks of 2048; 4203
-  // causal 256 / 192, 4935 of a window 256 / 256; 3000 sigmoid): 272 / 270, 130 / 125; 107 / 102, 156 / 150; 55.7 / 52.7.  Plain
-  // heads lose 2 to 5 % with each of them.
-  enum { kNothing, kVectors, kValues, kProducts };
-  constexpr int kRaised = SAME ? kValues : MODE == kSigmoid ? kProducts : MODE != kPlain || DV == 256 ? kVectors : kNothing;
+  // Forms whose vector work is the longer part: a wave that is at it goes first, products fill what it leaves.  Not for the
+  // others: raised value products of shared rows, vector work of two maps, products of sigmoid weights are 2 to 9 % faster at
+  // some sizes and 2 to 5 % slower at others, and neither rows nor workgroups tell which.  us, without / with:
+  // 256 / 192 causal, 3000 rows of 32 heads 136 / 126, 2500 in two prompts 63.6 / 66.7, 4000 of 16 heads 132 / 140; two maps, 4000
+  // rows in chunks 180 / 175, 3000 in three prompts 99 / 103; sigmoid, 3000 rows 54.9 / 51.9, 2500 of 16 heads 28.2 / 29.4.
+  constexpr bool kEager = MODE == kTerms || MODE == kTable;
   constexpr float kDefer = 8.f;  // pairs of products: log2 units that a score may exceed the running maximum by
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
@@ -286,7 +285,6 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
         __builtin_amdgcn_sched_group_barrier(0x100, SUBS + (QR < KS), 0);
       }
     }
-    if constexpr (kRaised == kProducts) __builtin_amdgcn_s_setprio(0);
     if (MODE != kPlain && terms) {  // final scores in log2 units
       // penalties of the lane's keys
       const uint32_t pen = table + 4 * (kTablePad - 31 + my - kt - 4 * h);
@@ -405,7 +403,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
     };
     constexpr int NF = 2 * SUBS * NC;  // value fragments of the tile
     weigh(0);
-    if constexpr (kRaised != kNothing) __builtin_amdgcn_s_setprio(kRaised == kVectors ? 0 : 1);
+    if constexpr (kEager) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const int k16 = f / NC, dt = f % NC;
@@ -420,8 +418,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
       __builtin_amdgcn_sched_group_barrier(0x008, FINE ? 2 : 1, 0);
       if (f + VA < NF) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    if constexpr (kRaised == kVectors) __builtin_amdgcn_s_setprio(1);
-    if constexpr (kRaised == kValues) __builtin_amdgcn_s_setprio(0);
+    if constexpr (kEager) __builtin_amdgcn_s_setprio(1);
   };
   auto tile = [&](int i) { return i < kept ? i : first + i - kept; };
   static_assert(ND <= KS, "a DMA instruction beside a product at most");
