@@ -53,14 +53,15 @@
 //     667 -> 539, 4000 854 -> 754; 8 experts of 2048, width 2048, 2500: 186 -> 186.
 //   * EPI_ADD with a last round that fills at most half of the CUs: its tiles are
 //     cut along K into as many pieces as there are CUs for (16 at most), the
-//     pieces' fp32 sums go through a workspace (64 MB at most) to a kernel that
+//     pieces' fp32 sums go through a workspace (256 pieces, 67 MB at most) to a kernel that
 //     adds them in order.  One more round costs 230 to 320 us at K 14336, whatever
 //     it holds; a sixteenth of one costs 20 and the way through the workspace 30:
 //     4150 x 4096 520 -> 365 us, 1000 x 4096 227 -> 104.  Where it fills somewhat more,
 //     half as many tiles as there are CUs go out in two pieces each and the others in
-//     as many as fit beside each other (512 pieces, 134 MB): a round is cut to half of
-//     one and a quarter or less.  6151 x 4096 609 -> 589 us, 6400 602 -> 569, 6900 618 ->
-//     600, 7100 628 -> 621, 12400 x 2048 614 -> 548, 2500 x 8192 of K 28672 838 -> 813.
+//     as many as fit beside each other, three at least (512 pieces, 134 MB at most), if K
+//     is long enough for that (kWorth): a round is cut to half of one and a third or less.
+//     K 14336: 6151 x 4096 575 -> 534 us, 6500 583 -> 554, 6800 598 -> 579, 12492 x 2048
+//     606 -> 530; K 28672: 3100 x 8192 1132 -> 1055.
 //     (In full rounds the
 //     card's power is the bound, not the schedule: the matrix cores are busy
 //     80 % of the cycles, and the clock is 1.75 GHz where launches stand alone,
@@ -96,7 +97,12 @@ struct Split {
   f32x4* part;
   int full, rest[2], segs[2];
 };
-constexpr int kSavedK = 3072;  // part of K that two kinds of pieces have to save (K 10240, 144 tiles: 417 -> 412 us, 160: 420 -> 418)
+// Two kinds of pieces: the least K times the part of K that they save.  The pieces' way to
+// the workspace and back is 134 MB each way whatever K is.  6151 / 6500 / 6800 / 7100 / 7300 x 4096 (16, 8, 5, 4, 3 pieces of the second kind), time over that of whole
+// tiles: K 10240 1.05 1.02 1.04 1.04 1.06, 11520 1.00 1.01 1.03 1.04 1.03, 12288 0.98 0.99 1.00 1.00 1.02, 14336 0.93 0.95 0.97
+// 0.99 1.00, 18432 0.91 0.94 0.95 0.97 0.99, 28672 0.89 0.92 0.93 0.96 0.98; 3100 / 3500 x 8192 (8, 4) K 12288 1.01 1.04, 14336
+// 0.98 1.02, 28672 0.93 0.98; N 2048 gains from K 10240 on.  What loses anywhere lies below 59e6 (K 16384, 4 pieces: 67e6, 0.97).
+constexpr int64_t kWorth = 60000000;
 
 __device__ __forceinline__ float silu_f(float g) { return g / (1.f + __expf(-g)); }
 
@@ -556,8 +562,8 @@ extern "C" int dx_gemm256(void* y, int64_t ldy, const void* x, int64_t ldx, cons
 }
 
 // How dx_gemm256_add splits its tiles.  A last round that fills at most half of the CUs is cut along K into as many pieces
-// as there are CUs for.  A fuller one: half as many tiles as CUs in two pieces each, then what is left like that, where the
-// part of a round that this saves, 1 - 1 / 2 - 1 / pieces, is longer than the way of 512 pieces through the workspace.
+// as there are CUs for.  A fuller one: half as many tiles as CUs in two pieces each, then what is left like that, where this
+// saves enough of K, (1 - 1 / 2 - 1 / pieces) K, for the way of 512 pieces through the workspace (kWorth).
 static Split add_split(int M, int N, int K) {
   const int tiles = (M + kBM - 1) / kBM * (N / kBN), cus = num_cus(), left = tiles % cus, half = cus / 2;
   auto pieces = [&](int n) { return std::min(std::min(cus / n, 16), K / (2 * kBK)); };
@@ -565,7 +571,7 @@ static Split add_split(int M, int N, int K) {
   if (left == 0) return sp;
   if (2 * left <= cus) {
     sp.full = tiles - left, sp.rest[0] = left, sp.segs[0] = pieces(left);
-  } else if (const int n = pieces(left - half); n > 2 && (int64_t)(n - 2) * K >= 2 * kSavedK * n) {
+  } else if (const int n = pieces(left - half); n > 2 && (int64_t)K * K * (n - 2) >= 2 * kWorth * n) {
     sp.full = tiles - left, sp.rest[0] = half, sp.segs[0] = 2, sp.rest[1] = left - half, sp.segs[1] = n;
   }
   return sp;

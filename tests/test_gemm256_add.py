@@ -51,10 +51,10 @@ def test_add_after_add(M, N, K, pieces):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,left,pieces", [
-    (2100, 4096, 7168, 16, 16),  # no whole tile
-    (6151, 4096, 7296, 16, 16),  # a round in front; 57 pairs of K tiles in 16 pieces
-    (16500, 512, 7168, 2, 16),  # a workgroup without a second piece
-    (22728, 512, 10240, 50, 5),
+    (2100, 4096, 13312, 16, 16),  # no whole tile
+    (6151, 4096, 13440, 16, 16),  # a round in front; 105 pairs of K tiles in 16 pieces
+    (16500, 512, 13312, 2, 16),  # a workgroup without a second piece
+    (22728, 512, 14336, 50, 5), (7100, 4096, 16384, 64, 4), (5800, 5120, 25600, 76, 3),
 ])
 def test_add_two_kinds(M, N, K, left, pieces):
     """A last round of more than half of the CUs: 128 tiles in two pieces of K, the others in more."""
@@ -89,6 +89,18 @@ def test_linear_add(M):
         exact = y.double() + want
         assert ops.linear_add_(y, x, w) is y
         assert bool(((y.double() - exact).abs() <= 2 ** -8 * exact.abs() + 2 ** -22 * K).all())
+
+
+@pytest.mark.parametrize("M,N,K,left,pieces", [
+    # (no pieces: whole tiles are faster there, or two pieces all that fit)
+    (6151, 4096, 10240, 16, 0), (6151, 4096, 11008, 16, 0), (6500, 4096, 11520, 32, 0), (6800, 4096, 12288, 48, 0),
+    (7100, 4096, 12288, 64, 0), (3500, 8192, 14336, 64, 0), (7300, 4096, 16384, 80, 0), (7525, 4096, 28672, 96, 0),
+    (6151, 4096, 12288, 16, 16), (6500, 4096, 13312, 32, 8), (6800, 4096, 14336, 48, 5), (7100, 4096, 16384, 64, 4),
+    (3100, 8192, 28672, 32, 8), (7300, 4096, 28672, 80, 3),
+])
+def test_rule_of_two_kinds(M, N, K, left, pieces):
+    assert -(-M // 256) * (N // 256) % 256 == 128 + left
+    assert ops._k().gemm256_add_floats(M, N, K) == (128 * 2 + left * pieces if pieces else 0) * 65536
 
 
 def test_rule_and_cpu():
