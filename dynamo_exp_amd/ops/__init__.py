@@ -283,17 +283,19 @@ CUS = 256  # compute units of an MI355X
 def deep_add_tiles(M: int, N: int, K: int) -> bool:
     """Whether y[M, N] += x w^T over a long K takes the 256-tile kernel.  It cuts an incomplete last round along K.  The
     library is a little faster where it chooses well and up to twice as slow where it does not, at sizes that follow no
-    rule: N 4096, K 14336, us, library / this kernel, M 600 96 / 82, 1000 112 / 103, 2050 358 / 230, 2125 202 / 223,
-    3925 299 / 311, 4150 716 / 352, 5050 424 / 420, 6151 810 / 578, 7525 1005 / 634, 7806 604 / 636, 8200 1019 / 682;
-    N 8192, K 28672, M 600 258 / 297, 2050 1284 / 723, 5050 2363 / 1599, 8192 2543 / 2554.  So the kernel is taken where
-    it loses little at worst.  Its time over the library's at 408 sizes (M 400 to 8450, N 2048 to 8192, K 10240 to 28672),
+    rule: N 4096, K 14336, us, library / this kernel, M 600 93 / 80, 1000 112 / 100, 2050 365 / 224, 2125 208 / 223,
+    3925 298 / 316, 4150 733 / 363, 5050 443 / 427, 6151 822 / 541, 7525 1017 / 633, 7806 608 / 648, 8200 1038 / 672;
+    N 8192, K 28672, M 600 266 / 296, 2050 1289 / 731, 5050 2369 / 1631, 8192 2575 / 2597.  So the kernel is taken where
+    it loses little at worst.  Its time over the library's at 440 sizes (M 400 to 8450, N 2048 to 8192, K 10240 to 28672),
     geometric mean and worst:
-      up to a third of a round (three pieces of K and more)   0.93  1.08
-      more than one round, the last one cut                   0.73  1.04
-      more than one round, the last one half to 15 / 16 full  0.76  1.08
-      not taken: 86 to 128 tiles 0.94 1.19, to one round 1.03 1.29, full last rounds 1.06 1.09
-    The sizes that lose more than 4 % are N 2048, K 10240 (48 to 80 tiles), M 561 of N 5120 and 6144, K 11008 at M 6035
-    and 7484, N 8192, K 14336 at 7484.  K 8192 gained nothing on average, nor did fewer than 384 rows at K 11008."""
+      up to a third of a round (three pieces of K and more)   0.80  1.16
+      more than one round, the last one cut                   0.74  1.05
+      more than one round, the last one half to 15 / 16 full  0.78  1.09 (cut into two kinds of pieces 0.68  0.84)
+      not taken: 86 to 128 tiles 0.90 1.21, to one round 1.00 1.29 (cut into two kinds of pieces 0.85 1.09), full last
+      rounds 1.03 1.10
+    The sizes that lose more than 6 % are 418 x 2048, 568 x 5120, 556 and 606 x 6144, 7475 and 7649 x 4096 of K 10240,
+    5900 to 6016 x 5120 and 3603 x 8192 of K 11008.  K 8192 gained nothing on average, nor did fewer than 384 rows at
+    K 11008."""
     tiles = -(-M // 256) * (N // 256)
     left = tiles % CUS
     return K >= 10240 and M >= 384 and (3 * tiles <= CUS or (tiles > CUS and 0 < 16 * left < 15 * CUS))
