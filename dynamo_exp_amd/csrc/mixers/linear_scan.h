@@ -93,7 +93,9 @@ __device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, M
   const T* gl = (const T*)g.g + (int64_t)h * dk;
   const T* v = (const T*)g.v + (int64_t)h * g.dv + col0;
   raw_u32x4 pf[PER];
-  float zb[MODE == kChannel ? PER : 1][VEC];
+  // kChannel: a thread's chunks Z0 .. Z1 - 1 may be decays, and have biases
+  constexpr int Z0 = 2 * QK_CH / NT, Z1 = (3 * QK_CH + NT - 1) / NT;
+  float zb[MODE == kChannel ? Z1 - Z0 : 1][VEC] = {};
   // kStep: token tid's step logit as loaded (its terms are formed in commit(): here they would wait for the load)
   T logit{};
   bool stepped = false;
@@ -141,7 +143,7 @@ __device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, M
       } else if (MODE == kChannel && c < 3 * QK_CH) {
         dst = as_ + (c - 2 * QK_CH) * VEC;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) f[e] = channel_decay(f[e] + (g.g_bias ? zb[i][e] : 0.f), g.inv_tau);
+        for (int e = 0; e < VEC; ++e) f[e] = channel_decay(f[e] + zb[i >= Z0 && i < Z1 ? i - Z0 : 0][e], g.inv_tau);
       } else if (c < N_CH) {
         dst = vs_ + (c - N_ROWS * QK_CH) * VEC;
       }
@@ -160,17 +162,21 @@ __device__ __forceinline__ void scan_tokens(const ScanArgs& g, ScanLds<16 * R, M
   fetch(r0);  // (in front of the state, which it does not wait for)
   // The biases of the thread's decays, the same for every token.  (Asked for where the rows go to LDS they were a latency more:
   // decode steps with their norms in a graph, 32 heads of 128 columns, four layers of 4 / 16 sequences 39.3 -> 37.6, 78 -> 67
-  // us, two of 40 71 -> 64.)
+  // us, two of 40 71 -> 64.  Only by the waves that hold decays, and where there are biases: asked for by all, with the state for
+  // missing ones, three layers without biases of 8 sequences 28.6 -> 27.3 us, of 400 of 64 / 64 columns 264 -> 257, with them
+  // 264 -> 257 and of 8 of 128 / 128 28.7 -> 27.8; 256 / 128 columns, 64 prompts of 30 rows without 549 -> 533.)
   if constexpr (MODE == kChannel) {
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-    const float* from = (g.g_bias ? g.g_bias : g.state) + h * dk;
+    const float* from = g.g_bias + h * dk;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c2 = tid + i * NT - 2 * QK_CH, ch = c2 >= 0 && c2 < QK_CH ? c2 % QC * VEC : 0;
+    for (int i = Z0; i < Z1; ++i) {
+      const int c2 = tid + i * NT - 2 * QK_CH;
+      if (g.g_bias && c2 >= 0 && c2 < QK_CH) {
 #pragma unroll
-      for (int e = 0; e < VEC; e += 4) {
-        const f32x4 b = *reinterpret_cast<const f32x4_a4*>(from + ch + e);
-        zb[i][e] = b[0], zb[i][e + 1] = b[1], zb[i][e + 2] = b[2], zb[i][e + 3] = b[3];
+        for (int e = 0; e < VEC; e += 4) {
+          const f32x4 b = *reinterpret_cast<const f32x4_a4*>(from + c2 % QC * VEC + e);
+          zb[i - Z0][e] = b[0], zb[i - Z0][e + 1] = b[1], zb[i - Z0][e + 2] = b[2], zb[i - Z0][e + 3] = b[3];
+        }
       }
     }
   }
