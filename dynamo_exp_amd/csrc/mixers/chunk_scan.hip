@@ -420,6 +420,8 @@ template <int DK> struct ChannelBuf {
 
 constexpr float kFarLog2 = 96.f;  // log2 of the largest e^-L used as a factor
 constexpr int kFormThreads = 512, kProdThreads = 256;
+// elements between rows: a chunk's inputs (64 rows) lie within 31-bit, its results within 32-bit byte offsets
+constexpr int64_t kNearRows = 1 << 24;
 
 // place of element i of a run of 32: group g's slots are {4 g .. + 3, 16 + 4 g .. + 3}
 __device__ __forceinline__ int slot_of32(int i) { return 8 * ((i >> 2) & 3) + 4 * (i >> 4) + (i & 3); }
@@ -430,7 +432,8 @@ __device__ __forceinline__ float channel_log2(float z, float inv_tau) {
   return -(fmaxf(-y, 0.f) + __builtin_amdgcn_logf(1.f + fast_exp2(-fabsf(y)))) * inv_tau;
 }
 
-template <int DK>
+// WIDE: rows further apart than kNearRows elements
+template <int DK, bool WIDE>
 __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_kernel(ScanArgs g) {
   using Buf = ChannelBuf<DK>;
   constexpr int Q = 32, KP = Buf::KP, SP = Buf::SP, NM = DK / 16, NK = DK / 32;
@@ -470,6 +473,7 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
     auto fetch = [&](int t0) {
       live = t0 + tok < w.n;
       auto row = [&](const bf16_t* p, int64_t stride, int col, bool has) {
+        if constexpr (WIDE) return live && has ? *reinterpret_cast<const raw_u32x4*>(p + (t0 + tok) * stride + col) : raw_u32x4{0u, 0u, 0u, 0u};
         const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)(p + t0 * stride), 0, 0x80000000u, 0x00020000);
         return __builtin_bit_cast(raw_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
             r, live && has ? 2u * (uint32_t)(tok * (int)stride + col) : 0x80000000u, 0, 0));
@@ -667,14 +671,14 @@ __global__ void __launch_bounds__(kFormThreads + kProdThreads, 3) channel_chunk_
 
 }  // namespace
 
+static bool near_rows(int mode, const ScanArgs& g) { return std::max({g.qs, g.ks, g.vs, mode == kFixed ? 0 : g.gs}) <= kNearRows; }
+
 // sizes and alignment the chunked kernels take (bf16 rows as 16-byte runs, whole column blocks)
 bool chunk_scan_ok(int mode, const ScanArgs& g) {
   auto al = [](const void* p) { return (uintptr_t)p % 16 == 0; };
   return (g.dk == 32 || g.dk == 64 || g.dk == 128) && g.dv % kPB == 0 && g.qs % 8 == 0 && g.ks % 8 == 0 &&
          g.vs % 8 == 0 && al(g.q) && al(g.k) && al(g.v) && al(g.state) && al(g.out) &&
-         // (a chunk of 64 rows: inputs within 31-bit, results within 32-bit byte offsets)
-         std::max({g.qs, g.ks, g.vs, mode == kFixed ? 0 : g.gs}) <= (1 << 24) &&
-         (mode == kChannel ? g.gs % 8 == 0 && al(g.g) && !g.skip : (int64_t)g.H * g.dv <= (1 << 24));
+         (mode == kChannel ? g.gs % 8 == 0 && al(g.g) && !g.skip : (int64_t)g.H * g.dv <= kNearRows && near_rows(mode, g));
 }
 
 #define CHUNK_DK(KERNEL, NT)                                                  \
@@ -698,9 +702,11 @@ bool launch_chunk_scan(int mode, const ScanArgs& g0, int n_seq, hipStream_t st) 
   g.all = g.dv % (4096 / g.dk) == 0 && (int64_t)grid.x * grid.y * n_seq <= 8192;
 #define FIXED_K(D) chunk_scan_kernel<D, kFixed>
 #define STEP_K(D) chunk_scan_kernel<D, kStep>
-#define CHANNEL_K(D) channel_chunk_kernel<D>
+#define CHANNEL_K(D) channel_chunk_kernel<D, false>
+#define CHANNEL_WIDE_K(D) channel_chunk_kernel<D, true>
   if (mode == kFixed) { CHUNK_DK(FIXED_K, dim3(512)) }
   else if (mode == kStep) { CHUNK_DK(STEP_K, dim3(512)) }
-  else { CHUNK_DK(CHANNEL_K, dim3(kFormThreads + kProdThreads)) }
+  else if (near_rows(mode, g)) { CHUNK_DK(CHANNEL_K, dim3(kFormThreads + kProdThreads)) }
+  else { CHUNK_DK(CHANNEL_WIDE_K, dim3(kFormThreads + kProdThreads)) }
   return g.all;
 }

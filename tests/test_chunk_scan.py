@@ -179,3 +179,25 @@ def test_short_sequences_beside_long_ones(rows, kind, H, dk, dv):
         if 0 < r < 8:
             alone, A = step([i])
             assert torch.equal(both[i], alone[0]) and torch.equal(S[slots[i].item()], A[slots[i].item()]), (i, r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stride", [1 << 24, (1 << 24) + 8])
+@pytest.mark.parametrize("dk", [32, 128])
+def test_rows_far_apart(dk, stride):
+    """Rows on both sides of what 32-bit offsets inside a chunk reach: the same bits as rows that lie together."""
+    torch.manual_seed(dk)
+    H, dv, rows = 2, 64, [41, 9]
+    T, n = sum(rows), 2 * dk
+    x = torch.randn(T, 3 * n + H * dv, device="cuda").bfloat16()
+    far = torch.empty((T - 1) * stride + x.shape[1], dtype=x.dtype, device="cuda").as_strided(x.shape, (stride, 1))
+    far.copy_(x)
+    first, pos = torch.tensor([0, *rows]).cumsum(0).to(torch.int32).cuda(), torch.cat([torch.arange(r) for r in rows]).cuda()
+    slots, bias = torch.tensor([1, 0], dtype=torch.int32).cuda(), torch.randn(n, device="cuda")
+    got = []
+    for p in (x, far):
+        state = torch.zeros(2, H, dv, dk, device="cuda")
+        got.append((rc.gated_linear_attention(p[:, :n], p[:, n:2 * n], p[:, 3 * n:], p[:, 2 * n:3 * n], bias, 16.0, dk ** -0.5, state,
+                                              pos, first, slots, H, dk, dv), state))
+    assert float(got[0][0].abs().sum()) > 0
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
