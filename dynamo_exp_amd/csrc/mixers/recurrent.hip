@@ -514,6 +514,15 @@ __global__ void __launch_bounds__(128) conv_run_kernel(ConvArgs g, T* __restrict
     r0 = known ? (g.seq_rows ? g.seq_rows[s] : t) : t;
     live = slot >= 0 && slot < g.n_slots && r0 >= 0 && r0 <= t;
     if (M == 0 || !live) return;
+    // (nothing of the run lies in front of its first row: asking all the same, prompts of 500 and 300 rows beside 40 decode rows,
+    // three layers of 10240 / 2176 / 1000 channels, took 50.4 / 29.4 / 25.1 us for 44.6 / 26.2 / 20.6)
+    if (R > 1 && t == r0) {
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int e = 0; e < V; ++e) h[m][e] = 0.f;
+      return;
+    }
     const T* tl = tail + (int64_t)slot * M * C + c;
     raw_u32x4 was[M > 0 ? M : 1];
 #pragma unroll
