@@ -3,6 +3,10 @@
 dense float64 arithmetic over the bf16 inputs.  The pages' unused rows hold NaN."""
 from __future__ import annotations
 
+import re
+from pathlib import Path
+
+import numpy as np
 import pytest
 import torch
 
@@ -332,6 +336,31 @@ def test_penalty_rows_whose_old_keys_count(form, cap, old):
                        dist_bias=tuple(map(cuda, db))).cpu().double()
     # (bound of test_prompt_rows)
     assert float((got - want).abs().max()) < 2.0 ** -8 * (float(want.abs().max()) + 5.0)
+
+
+@pytest.mark.parametrize("name,limit", [("kTanh", "kTanhMax"), ("kTanhFew", "kTanhMin")])
+def test_polynomials_of_the_cap(name, limit):
+    """tanh(y) / y as the kernel's coefficients give it over the range that each polynomial is taken for.  (The bounds of the
+    results above could not tell: 1e-4 of a score is far below the rounding of a weight.)"""
+    text = (Path(mx.__file__).parents[1] / "csrc" / "mixers" / "prompt_attention.hip").read_text()
+    coef = [float(np.float32(x)) for x in re.search(rf"\b{name}\[\d\] = {{(.*?)}}", text)[1].replace("f", "").split(",")]
+    top = float(re.search(rf"\b{limit} = ([\d.]+)f", text)[1])
+    y = np.linspace(1e-6, top, 200001)
+    exact = np.tanh(y) / y
+    far = lambda c: np.abs(sum(a * y ** (2 * i) for i, a in enumerate(c)) / exact - 1).max()
+    assert far(coef) < 6.3e-8, far(coef)
+    # evaluated as the kernel does, in 32 bits: 2^-24 each for the leading coefficient times the scale, the sum and the product
+    # (the other terms are 4 % of it at most)
+    f = np.float32
+    for s in (0.05, 1.0, 37.0):  # score = s y
+        x, y2 = (s * y).astype(f), f(f(1 / s) * f(1 / s))
+        c = [f(f(s) * f(a)) for a in coef]  # (scale and cap: the polynomial of x, times the cap)
+        u = [f(c[i] * f(f(1 / s) * f(y2 ** i))) for i in range(len(c))]
+        t, r = x * x, np.full_like(x, u[-1])
+        for a in u[-2::-1]:
+            r = (t.astype(np.float64) * r + a).astype(f)
+        got = (x * r).astype(np.float64) / s
+        assert np.abs(got / np.tanh(x.astype(np.float64) / s) - 1).max() < 6.3e-8 + 3 * 2.0 ** -24
 
 
 @pytest.mark.gpu
