@@ -88,7 +88,8 @@ HIP_FLAGS = ["-x", "hip", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32
 
 
 def verify_kernels(names: list[str] | None = None, jobs: int = 8) -> dict[str, str]:
-    """Compile the device side of the HIP kernel sources with LLVM's machine
+    """Compile the device side of the HIP sources in csrc/kernels, and of the
+    mixers with code generation options of their own, with LLVM's machine
     verifier (``-mllvm -verify-machineinstrs``) and return {file: error} for
     the ones it rejects.  ROCm 7.2 had a sub-register liveness
     miscompile in attn_decode.hip ("No live subrange at use": V-row registers
@@ -96,13 +97,13 @@ def verify_kernels(names: list[str] | None = None, jobs: int = 8) -> dict[str, s
     verifier reports at compile time; the normal build does not run it."""
     import tempfile
 
-    src_dir = CSRC / "kernels"
-    srcs = [s for s in sorted(src_dir.glob("*.hip")) if names is None or s.name in names]
+    srcs = sorted((CSRC / "kernels").glob("*.hip")) + [s for s in sorted((CSRC / "mixers").glob("*.hip")) if s.name in PER_FILE_FLAGS]
+    srcs = [s for s in srcs if names is None or s.name in names]
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    flags = [f for f in _kernel_flags(src_dir) if f != "-fPIC"]
     bad: dict[str, str] = {}
     with tempfile.TemporaryDirectory() as td:
         def one(s: Path):
+            flags = [f for f in _kernel_flags(s.parent) if f != "-fPIC"]
             cmd = [hipcc, *flags, *HIP_FLAGS, *PER_FILE_FLAGS.get(s.name, []), "--cuda-device-only", "-c", str(s),
                    "-o", str(Path(td) / (s.name + ".o")), "-mllvm", "-verify-machineinstrs"]
             r = subprocess.run(cmd, capture_output=True, text=True)
