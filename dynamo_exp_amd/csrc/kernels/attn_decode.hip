@@ -469,13 +469,8 @@ __device__ __forceinline__ int vimg_off(int row, int ch) {  // byte offset of 16
   return row * 256 + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
-// over the four 16-lane groups of a wave, by exchanges in registers
-template <typename F> __device__ __forceinline__ float over_groups(float x, F f) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
+// over the four 16-lane groups of a wave
+template <typename F> __device__ __forceinline__ float over_groups(float x, F f) { return over_row_pairs(over_halves(x, f), f); }
 
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4_t;
 
@@ -731,7 +726,7 @@ __global__ void __launch_bounds__(D) decode_reduce_kernel(bf16_t* __restrict__ o
       if (p < np) num += w * y;
     }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) num[i] = over_halves(num[i], [](float x, float y) { return x + y; });
+  for (int i = 0; i < 4; ++i) num[i] = halves_sum(num[i]);
   if (grp == 2) other[threadIdx.x & 31] = num;
   __syncthreads();
   if (grp) return;

@@ -70,18 +70,8 @@ __device__ __forceinline__ bf16x8_t as_frag(const u16x8& v) { return __builtin_b
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr float kRescaleLog2 = 8.0f;  // deferred-max threshold (log2 units)
 
-// max / sum of a lane's value and the value of the lane 32 apart: on gfx950 one
-// v_permlane32_swap (VALU) instead of a ds_bpermute round trip through LDS in
-// the softmax's dependent chain
-__device__ __forceinline__ float halves_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float halves_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
+// PLS: max / sum over the two halves of a wave by one v_permlane32_swap (halves_max, halves_sum: VALU) instead of a
+// ds_bpermute round trip through LDS in the softmax's dependent chain
 // V: 0 = the first loop (kept for A/B), 1 = deferred rescale, row
 // sum on the matrix pipe, v_max3 row max, raised priority (step), widened epilogue.
 // (Ping-pong wave halves, two tiles per barrier and a software-pipelined QK /

@@ -77,14 +77,21 @@ template <typename F> __device__ __forceinline__ float over_halves(float v, F f)
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+template <typename F> __device__ __forceinline__ float over_row_pairs(float v, F f) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float halves_max(float v) {
+  return over_halves(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float halves_sum(float v) {
+  return over_halves(v, [](float a, float b) { return a + b; });
+}
 // (N: aligned groups of so many lanes, 16 or more)
 template <int N, typename F> __device__ __forceinline__ float over_lanes(float v, F f) {
   static_assert(N == 16 || N == 32 || N == 64, "whole rows of lanes");
   if constexpr (N == 64) v = over_halves(v, f);
-  if constexpr (N >= 32) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  }
+  if constexpr (N >= 32) v = over_row_pairs(v, f);
   v = f(v, row_dpp<0x128>(v));  // row_ror:8
   v = f(v, row_dpp<0x124>(v));  // row_ror:4 (4 or 12 lanes on, which hold the same by now)
   v = f(v, row_dpp<0x4E>(v));   // quad_perm

@@ -104,14 +104,6 @@ __device__ __forceinline__ float max2(float a, float b) { return __builtin_eleme
 __device__ __forceinline__ float max3(float a, float b, float c) { return max2(max2(a, b), c); }
 // a number that is the same in every lane, in a scalar register
 __device__ __forceinline__ float uniform(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
-__device__ __forceinline__ float swap_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float swap_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 // D: key columns, DV: value columns, SAME: the value is the first DV columns of the key's row
 // HPW: heads per workgroup, NW: waves, SUBS: blocks of 32 keys per tile
@@ -369,7 +361,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
         }
       }
       // both halves of a row see the same maximum and take the same decision
-      const float tm = swap_max(fmaxf(ta, tb)) * sc;
+      const float tm = halves_max(fmaxf(ta, tb)) * sc;
       const float mn = tm > (FINE ? m_i + kDefer : m_i) ? tm : m_i;
       mu = mn == -INFINITY ? 0.f : mn;  // a row that has seen nothing yet
       if (__builtin_amdgcn_ballot_w64(mn != m_i)) {
@@ -442,7 +434,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   if (PARTS && !cut && kept_row && h == 0) *reinterpret_cast<float2*>(ws) = float2{0.f, -1.f};  // the join's sign to leave the row
   if (cut) {  // sums as they are: gate, sink and denominator come with the join
     if (!kept_row) return;
-    const float l = MODE == kSigmoid ? 1.f : swap_sum(l_i);
+    const float l = MODE == kSigmoid ? 1.f : halves_sum(l_i);
     if (h == 0) *reinterpret_cast<float2*>(ws) = float2{MODE == kSigmoid ? 0.f : m_i * kLn2, l};
 #pragma unroll
     for (int dt = 0; dt < NC; ++dt)
@@ -456,7 +448,7 @@ __global__ void __launch_bounds__(64 * NW, SUBS == 1 && DV == 128 ? 3 : 2) promp
   }
   float inv = 1.f;
   if constexpr (MODE != kSigmoid) {
-    float l = swap_sum(l_i);
+    float l = halves_sum(l_i);
     if (a.sink) l += fast_exp2(a.sink[qh] * kLog2e - m_i);  // (finite: a row sees itself)
     inv = 1.f / l;
   }
