@@ -459,9 +459,9 @@ __global__ void __launch_bounds__(kThreads) decode_attn_kernel(
 // the wait for a chunk's V rows was one for the next chunk's K rows too, a whole
 // latency in every chunk.  32 / 8 heads, layers in a graph, us: bf16, four of 40
 // sequences of 3000 tokens 256 -> 229 (5.0 -> 5.6 TB/s), two of 96 of 3150 278 ->
-// 256, eight of one of 700 61.5 -> 58.5; e4m3, two of 96 of 3150 153 -> 149, of 75
-// of 500 37 -> 35; 64 / 8 heads, bf16, two of 48 of 3000 149 -> 137.  Two
-// workgroups a CU, which is what the registers give: bounded to the 168 of three,
+// 256, eight of one of 700 61.5 -> 58.5; e4m3, two of 75 of 500 37 -> 35 (of 96 of
+// 3150 within what two runs differ by); 64 / 8 heads, bf16, two of 48 of 3000 149 -> 137.
+// Two workgroups a CU, which is what the registers give: bounded to the 168 of three,
 // 40 of 3000 254, 38 of 5000 171 -> 197.
 constexpr int MCH = 32;  // tokens per wave chunk
 
