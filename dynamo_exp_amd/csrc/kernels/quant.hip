@@ -103,20 +103,24 @@ __global__ void __launch_bounds__(TPB) rmsnorm_quant_kernel(uint8_t* __restrict_
       for (int k = 0; k < 8; ++k) ss += v[i][k] * v[i][k];
     }
   }
+  const u16x8* wr = reinterpret_cast<const u16x8*>(w);
+  u16x8 g[kMaxVec];
+  if constexpr (kExact)  // in front of the sum, which they do not wait for
+#pragma unroll
+    for (int i = 0; i < kMaxVec; ++i) g[i] = wr[threadIdx.x + i * TPB];
   ss = block_reduce_sum(ss, red);
   const float inv = rsqrtf(ss / (float)hidden + eps);
-  const u16x8* wr = reinterpret_cast<const u16x8*>(w);
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < kMaxVec; ++i) {
     const int vi = threadIdx.x + i * TPB;
     if (kExact || vi < nvec) {
-      u16x8 g = wr[vi];
+      if constexpr (!kExact) g[i] = wr[vi];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         // round through bf16 like the bf16 path's normalised output
-        v[i][2 * k] = bf16lo(pack_bf16x2(v[i][2 * k] * inv * bf16lo(g.w[k]), 0.f));
-        v[i][2 * k + 1] = bf16lo(pack_bf16x2(v[i][2 * k + 1] * inv * bf16hi(g.w[k]), 0.f));
+        v[i][2 * k] = bf16lo(pack_bf16x2(v[i][2 * k] * inv * bf16lo(g[i].w[k]), 0.f));
+        v[i][2 * k + 1] = bf16lo(pack_bf16x2(v[i][2 * k + 1] * inv * bf16hi(g[i].w[k]), 0.f));
         amax = fmaxf(amax, fmaxf(fabsf(v[i][2 * k]), fabsf(v[i][2 * k + 1])));
       }
     }
