@@ -53,19 +53,26 @@ __global__ void __launch_bounds__(kThreads) rmsnorm_kernel(bf16_t* out, const bf
       for (int k = 0; k < 8; ++k) ss += v[i][k] * v[i][k];
     }
   }
+  const u16x8* wr = reinterpret_cast<const u16x8*>(w);
+  u16x8 g[kMaxVec];
+  // in front of the sum, which they do not wait for: 2000 / 8192 / 16000 rows of 4096 8.0 / 25.2 / 47.0 -> 7.6 / 24.5 / 46.0 us a
+  // launch (with an addition, 2000 rows 9.9 -> 10.4, others -2 to 3 %)
+  constexpr bool kEarly = kExact && !kAdd;
+  if constexpr (kEarly)
+#pragma unroll
+    for (int i = 0; i < kMaxVec; ++i) g[i] = wr[threadIdx.x + i * kThreads];
   ss = block_reduce_sum(ss, red);
   const float inv = rsqrtf(ss / (float)hidden + eps);
-  const u16x8* wr = reinterpret_cast<const u16x8*>(w);
   u16x8* orow = reinterpret_cast<u16x8*>(out + row * out_stride);
 #pragma unroll
   for (int i = 0; i < kMaxVec; ++i) {
     const int vi = threadIdx.x + i * kThreads;
     if (kExact || vi < nvec) {
-      u16x8 g = wr[vi];
+      if constexpr (!kEarly) g[i] = wr[vi];
       u16x8 o;
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        o.w[k] = pack_bf16x2(v[i][2 * k] * inv * bf16lo(g.w[k]), v[i][2 * k + 1] * inv * bf16hi(g.w[k]));
+        o.w[k] = pack_bf16x2(v[i][2 * k] * inv * bf16lo(g[i].w[k]), v[i][2 * k + 1] * inv * bf16hi(g[i].w[k]));
       orow[vi] = o;
     }
   }
